@@ -6,6 +6,7 @@ module raises.
 """
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -162,22 +163,48 @@ def device_check():
     return buf.value.decode()
 
 
-def _stream_ptr(stream=None):
+# torch's dtypes and the raw stream lookup, filled in at the first use.  A launch of the kernel layer takes the host 1 to 3
+# us; torch.cuda.current_stream() alone took 3 (it builds a Stream object), the raw handle takes 0.2.
+_TORCH_DTYPE, _BZ_DTYPE = {}, {}
+_current_device = _raw_stream = None
+
+
+def _bind_torch():
+    global _current_device, _raw_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    _TORCH_DTYPE.update({F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16, I8: torch.int8, I32: torch.int32,
+                         I64: torch.int64})
+    _BZ_DTYPE.update({t: d for d, t in _TORCH_DTYPE.items()})
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    _current_device = torch.cuda.current_device
+    if _raw_stream is None:  # a torch without the raw lookup
+        _raw_stream = lambda device: torch.cuda.current_stream(device).cuda_stream  # noqa: E731
+
+
+def _stream_ptr(stream=None):
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        _bind_torch()
+    return _raw_stream(_current_device())
 
 
 def torch_dtype(dt):
-    import torch
-    return {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16, I8: torch.int8, I32: torch.int32,
-            I64: torch.int64}[dt]
+    if not _TORCH_DTYPE:
+        _bind_torch()
+    return _TORCH_DTYPE[dt]
 
 
 def bz_dtype(t):
-    import torch
-    return {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16, torch.int8: I8, torch.int32: I32,
-            torch.int64: I64}[t]
+    if not _BZ_DTYPE:
+        _bind_torch()
+    return _BZ_DTYPE[t]
+
+
+# The descriptors of the per-call entry points, filled in one go: thirty ctypes attribute assignments took 4 us of a call.
+_FC_DESC = struct.Struct("@7P3q9i3fi3P2q4iq2P")
+_BGEMM_DESC = struct.Struct("@3P3q7i2f")
+assert _FC_DESC.size == C.sizeof(FcDesc) and _BGEMM_DESC.size <= C.sizeof(BgemmDesc)
 
 
 # ----------------------------------------------------------------------------------- tables
@@ -376,40 +403,38 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
     """head: dict(w=packed [n2, ldw] weight of a second layer with n2 <= 8 outputs, bias=fp32 [n2] or None, act=ACT_NONE |
     ACT_SIGMOID | ACT_SOFTMAX, out=tensor [m, n2]) computed in the same launch; then returns (out, head out), and
     store_out=False skips storing the first layer's output (out is returned as None)."""
-    import torch
-    m = a.shape[0]
-    n = w_packed.shape[0]
+    m, n = a.shape[0], w_packed.shape[0]
+    dt = bz_dtype(a.dtype)
     if out is None:
-        out = torch.empty((m, n), dtype=torch_dtype(out_dtype or bz_dtype(a.dtype)), device=a.device)
-    d = FcDesc()
-    d.a, d.w, d.y = a.data_ptr(), w_packed.data_ptr(), out.data_ptr()
-    d.lda, d.ldw, d.ldy = a.stride(0), w_packed.stride(0), out.stride(0)
-    d.m, d.n, d.k = m, n, k
-    d.in_dtype, d.out_dtype = bz_dtype(a.dtype), bz_dtype(out.dtype)
+        import torch
+        out = torch.empty((m, n), dtype=torch_dtype(out_dtype or dt), device=a.device)
     assert w_packed.dtype == a.dtype
+    bias_ptr = bias_rows = 0
     if bias is not None:
-        assert bias.dtype == torch.float32
-        d.bias = bias.data_ptr()
-        d.bias_rows = 1 if bias.numel() == n else m
-    d.act = act
-    ps = list(act_params) + [None] * 3
-    for name, p in zip(("act_p0", "act_p1", "act_p2"), ps):
-        if p is not None:
-            assert p.dtype == torch.float32
-            setattr(d, name, p.data_ptr())
-    d.act_size = ps[0].numel() if ps[0] is not None else 0
-    d.dice_nosqrt = int(dice_nosqrt)
-    d.alpha, d.beta, d.act_alpha = alpha, beta, act_alpha
+        assert bz_dtype(bias.dtype) == F32
+        bias_ptr, bias_rows = bias.data_ptr(), 1 if bias.numel() == n else m
+    p = [0, 0, 0]
+    for i, t in enumerate(act_params[:3]):
+        if t is not None:
+            assert bz_dtype(t.dtype) == F32
+            p[i] = t.data_ptr()
+    act_size = act_params[0].numel() if act_params and act_params[0] is not None else 0
+    y = out.data_ptr()
+    hw_ptr = hb_ptr = hy_ptr = h_ldw = h_ldy = h_n = h_act = h_dt = 0
     if head is not None:
-        hw, hy = head["w"], head["out"]
+        hw, hb, hy = head["w"], head.get("bias"), head["out"]
         assert hw.dtype == a.dtype and hy.shape[0] == m
-        d.head_w, d.head_y, d.head_ldw, d.head_ldy = hw.data_ptr(), hy.data_ptr(), hw.stride(0), hy.stride(0)
-        d.head_n, d.head_act, d.head_out_dtype = hw.shape[0], head.get("act", ACT_NONE), bz_dtype(hy.dtype)
-        if head.get("bias") is not None:
-            assert head["bias"].dtype == torch.float32
-            d.head_bias = head["bias"].data_ptr()
+        hw_ptr, hy_ptr, h_ldw, h_ldy = hw.data_ptr(), hy.data_ptr(), hw.stride(0), hy.stride(0)
+        h_n, h_act, h_dt = hw.shape[0], head.get("act", ACT_NONE), bz_dtype(hy.dtype)
+        if hb is not None:
+            assert bz_dtype(hb.dtype) == F32
+            hb_ptr = hb.data_ptr()
         if not store_out:
-            d.y = None
+            y = 0
+    d = FcDesc()
+    _FC_DESC.pack_into(d, 0, a.data_ptr(), w_packed.data_ptr(), bias_ptr, y, p[0], p[1], p[2], a.stride(0), w_packed.stride(0),
+                       out.stride(0), m, n, k, dt, bz_dtype(out.dtype), bias_rows, act, act_size, int(dice_nosqrt), alpha, beta,
+                       act_alpha, 0, hw_ptr, hb_ptr, hy_ptr, h_ldw, h_ldy, h_n, h_act, h_dt, 0, 0, 0, 0)
     check(lib().bz_fc_fused(C.byref(d), _stream_ptr(stream)))
     if head is not None:
         return (out if store_out else None), head["out"]
@@ -419,12 +444,8 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
 def gemm_strided_batched(a, b, c, m, n, k, batch, stride_a, stride_b, stride_c, trans_a=False, trans_b=False, alpha=1.0,
                          beta=0.0, stream=None):
     d = BgemmDesc()
-    d.a, d.b, d.c = a.data_ptr(), b.data_ptr(), c.data_ptr()
-    d.stride_a, d.stride_b, d.stride_c = stride_a, stride_b, stride_c
-    d.trans_a, d.trans_b = int(trans_a), int(trans_b)
-    d.m, d.n, d.k, d.batch = m, n, k, batch
-    d.dtype = bz_dtype(a.dtype)
-    d.alpha, d.beta = alpha, beta
+    _BGEMM_DESC.pack_into(d, 0, a.data_ptr(), b.data_ptr(), c.data_ptr(), stride_a, stride_b, stride_c, int(trans_a), int(trans_b),
+                          m, n, k, batch, bz_dtype(a.dtype), alpha, beta)
     check(lib().bz_gemm_strided_batched(C.byref(d), _stream_ptr(stream)))
     return c
 
