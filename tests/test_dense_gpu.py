@@ -275,6 +275,30 @@ def _bgemm(bz, A, B, M, N, K, batch, sa, sb, ta, tb, dtype, C0=None, alpha=1.0, 
     return c.to(torch.float32).cpu().numpy()
 
 
+@pytest.mark.parametrize("dtype_name", ["f32", "f16"])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 1, 1, 1), (5, 1, 7, 65), (6, 32, 32, 64), (5, 33, 31, 65), (3, 17, 5, 83), (2, 65, 63, 129),
+                                         (2, 3, 130, 33), (4, 64, 64, 40)])
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_bgemm_tile_edges(bz, dtype_name, batch, M, N, K, ta, tb):
+    """edges of the 32- and 64-wide tiles and of the 128-byte pieces of K, operands starting off 16-byte boundaries, C scaled in"""
+    import torch
+    print("case bgemm %s b=%d %dx%dx%d ta=%d tb=%d" % (dtype_name, batch, M, N, K, ta, tb), flush=True)
+    dtype = {"f32": torch.float32, "f16": torch.float16}[dtype_name]
+    rng = np.random.default_rng(M * 1000 + N * 10 + K)
+    A, B, C0 = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(dtype) for s in
+                ((batch, K, M) if ta else (batch, M, K), (batch, N, K) if tb else (batch, K, N), (batch, M, N)))
+    a, b, c = (torch.cat([t.new_zeros(1), t.reshape(-1)]).cuda()[1:] for t in (A, B, C0))
+    bz.gemm_strided_batched(a, b, c, M, N, K, batch, M * K, K * N, M * N, ta, tb, 0.5, -2.0)
+    torch.cuda.synchronize()
+    want = 0.5 * np.matmul(A.double().numpy().transpose(0, 2, 1) if ta else A.double().numpy(),
+                           B.double().numpy().transpose(0, 2, 1) if tb else B.double().numpy()) - 2.0 * C0.double().numpy()
+    got = c.double().cpu().numpy().reshape(batch, M, N)
+    tol = 1e-5 if dtype_name == "f32" else 2e-3
+    assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want)
+    np.testing.assert_allclose(got, want, rtol=20 * tol, atol=20 * tol)
+
+
 @pytest.mark.parametrize("name", ["matmul_net_v1_cpu", "fused_parallel_matmul_net_v1_cpu", "fused_parallel_matmul_net_v2_cpu",
                                   "fused_parallel_matmul_net_v3_cpu"])
 def test_reference_matmul_kats_on_gpu(bz, kats, name):

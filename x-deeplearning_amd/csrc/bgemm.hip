@@ -5,15 +5,14 @@
 // blaze/math/broadcast.h:157-222), FusedParallelGemm (fused_parallel_gemm_op.h:96-129) and
 // FusedParallelMatMul / BatchedBroadcastGemm_NxN (blaze/math/broadcast.h:267-381).
 //
-// On this path the matrices are tiny (the DIN attention sum is 1xT . TxD with T<=50, D=54):
-// the work is one pass over B, i.e. memory bound.  One wavefront owns one batch item; its
-// lanes own output elements (m,n) with n fastest, so reads of a non-transposed B row and
-// writes of C are contiguous; A values are wave-uniform broadcasts.  fp32 accumulate in
-// ascending k.
+// Two kernels.  A row times a matrix (M = 1, B stored [K, N]: the DIN attention sum, 1xT . TxD) is one pass over B with
+// nothing to reuse: bz_bgemm_row_kernel.  Everything else is a contraction whose operands are used M or N times, on the
+// matrix cores: bz_bgemm_mfma_kernel.  fp32 accumulate in both.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
 #include "bz_common.h"
+#include "fc_common.h"
 
 namespace {
 
@@ -38,59 +37,260 @@ __device__ __forceinline__ void st<__half>(__half* p, float v) {
   *p = __float2half_rn(v);
 }
 
-// One wave per batch item, one lane per output element; K is walked in steps of kUnroll with all loads of a step
-// issued before the first multiply-add (the products are still added in ascending k, so the sum is the plain loop's).
-constexpr int kUnroll = 16;
+// One wave per batch item, one lane per output column; K is walked in steps of kUnroll with all loads of a step issued
+// before the first multiply-add.  The products are added in ascending k, the order bz_weighted_pool_kernel keeps as well.
+constexpr int kUnroll = 32;
 
-template <typename T, bool TA, bool TB>
-__global__ __launch_bounds__(256) void bz_bgemm_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C,
-                                                       int64_t sa, int64_t sb, int64_t sc, int M, int N, int K, int batch,
-                                                       float alpha, float beta) {
+template <typename T>
+__global__ __launch_bounds__(256) void bz_bgemm_row_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C,
+                                                           int64_t sa, int64_t sb, int64_t sc, int N, int K, int batch, float alpha,
+                                                           float beta) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * 4 + wave;
   if (item >= batch) return;
-  const T* a = A + sa * item;
+  const T* a = A + sa * item;  // (a single row: [1, K] and [K, 1] are the same memory)
   const T* b = B + sb * item;
   T* c = C + sc * item;
-  const int lda = TA ? M : K, ldb = TB ? K : N;
-  for (int e = lane; e < M * N; e += 64) {
-    const int m = e / N, n = e - m * N;
-    const T* ap = TA ? a + m : a + (int64_t)m * lda;  // element k: ap[k * (TA ? lda : 1)]
-    const T* bp = TB ? b + (int64_t)n * ldb : b + n;  // element k: bp[k * (TB ? 1 : ldb)]
-    const int64_t as = TA ? lda : 1, bs = TB ? 1 : ldb;
+  for (int n = lane; n < N; n += 64) {
     float acc = 0.f;
     for (int k0 = 0; k0 < K; k0 += kUnroll) {
       float av[kUnroll], bv[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const int k = k0 + u < K ? k0 + u : K - 1;  // clamped address; the product is skipped below
-        av[u] = ld<T>(ap + k * as);
-        bv[u] = ld<T>(bp + k * bs);
+        av[u] = ld<T>(a + k);
+        bv[u] = ld<T>(b + (int64_t)k * N + n);
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u)
         if (k0 + u < K) acc = fmaf(av[u], bv[u], acc);
     }
     float v = alpha * acc;
-    if (beta != 0.f) v += beta * ld<T>(c + e);  // beta == 0: C is not read (BLAS rule)
-    st<T>(c + e, v);
+    if (beta != 0.f) v += beta * ld<T>(c + n);  // beta == 0: C is not read (BLAS rule)
+    st<T>(c + n, v);
   }
 }
 
-template <typename T>
-void launch_bgemm(const bz_bgemm_desc& d, int grid, hipStream_t s) {
-#define BZ_BGEMM(TA, TB)                                                                                                     \
-  hipLaunchKernelGGL((bz_bgemm_kernel<T, TA, TB>), dim3(grid), dim3(256), 0, s, (const T*)d.a, (const T*)d.b, (T*)d.c, d.stride_a, \
-                     d.stride_b, d.stride_c, d.m, d.n, d.k, d.batch, d.alpha, d.beta)
-  if (d.trans_a && d.trans_b)
-    BZ_BGEMM(true, true);
-  else if (d.trans_a)
-    BZ_BGEMM(true, false);
-  else if (d.trans_b)
-    BZ_BGEMM(false, true);
-  else
-    BZ_BGEMM(false, false);
+// ---------------------------------------------------------------------------------------------
+// matrix-core kernel
+// ---------------------------------------------------------------------------------------------
+// The matrices are small (tens of rows and columns) and there are many: the work is one pass over A, B and C, and an
+// item's operands fit LDS whole.  A workgroup of four waves owns G items (G = 1: a C tile of 64 x 64, a wave per 32 x 32
+// block; G = 4: items of at most 32 x 32, a wave each), stages K in pieces of 128 bytes a row -- both operands K contiguous,
+// rows padded by 16 bytes so that the fragment reads (16 bytes a lane) spread over the banks -- and stores C straight from
+// the accumulators (a store instruction covers 32 neighbouring columns of two rows).  The next piece of K is loaded into
+// registers while the present one is multiplied.
+// An operand stored K contiguous is read 16 bytes a lane wherever its rows start (an item's matrix is contiguous, so most
+// rows start on 2 bytes; the memory system takes such loads), the few chunks that would reach past the operand's last
+// element by elements.  An operand stored the other way round is read 16 bytes a lane along its rows with neighbouring
+// lanes on neighbouring k, so that the transposing LDS writes of a wave are contiguous.
+// 1024 x [50,54]x[54,50] fp16 (16 MB, 3.3 us at the copy's rate): a lane per output element with scalar loads took 184 us.
+constexpr int kRowB = 128;            // bytes of K staged per row
+constexpr int kPitch = kRowB + 16;    // LDS pitch of a staged row
+
+template <int DT>
+struct Elem;
+template <>
+struct Elem<BZ_F16> {
+  typedef __half T;
+};
+template <>
+struct Elem<BZ_F32> {
+  typedef float T;
+};
+
+// 16 bytes from any element-aligned address
+__device__ __forceinline__ uint4 load16(const char* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// 16 bytes of which only the first `n` elements count (n <= 0: none): the rest come back as zeros.  `end`: one past the
+// operand's last byte.
+template <int ES>
+__device__ __forceinline__ uint4 load_part(const char* p, int n, const char* end) {
+  constexpr int CH = 16 / ES;
+  uint4 v = make_uint4(0, 0, 0, 0);
+  if (n <= 0) return v;
+  if (p + 16 <= end) {
+    v = load16(p);
+  } else {
+    uint32_t w[4] = {0, 0, 0, 0};
+    for (int i = 0; i < CH; ++i)
+      if (i < n) {
+        if constexpr (ES == 4)
+          w[i] = *(const uint32_t*)(p + 4 * i);
+        else
+          w[i / 2] |= (uint32_t) * (const unsigned short*)(p + 2 * i) << (16 * (i & 1));
+      }
+    v = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  if (n < CH) {
+    uint32_t* w = (uint32_t*)&v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (ES == 4)
+        w[j] = j < n ? w[j] : 0u;
+      else
+        w[j] = 2 * j + 1 < n ? w[j] : (2 * j < n ? w[j] & 0xffffu : 0u);
+    }
+  }
+  return v;
+}
+
+// one operand's tile: ROWS rows (of M or N) by kRowB bytes of K, NT threads.  KC: the operand is stored K contiguous.
+template <int DT, int ROWS, int NT, bool KC>
+struct Stage {
+  static constexpr int ES = bz::fc::In<DT>::kSize;
+  static constexpr int CH = 16 / ES;                // elements per chunk
+  static constexpr int BK = kRowB / ES;             // K per piece
+  static constexpr int CHUNKS = ROWS * kRowB / 16;  // per piece
+  static constexpr int PER = CHUNKS / NT;
+  static_assert(CHUNKS % NT == 0, "tile");
+  uint4 r[PER];
+  // base: the item's matrix; ld: its row length; rows r0 .. of `rows`, k0 .. of K
+  __device__ __forceinline__ void load(const char* base, const char* end, int t, int r0, int rows, int k0, int K) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int q = t + i * NT;
+      if constexpr (KC) {
+        const int row = r0 + q / (kRowB / 16), k = k0 + (q % (kRowB / 16)) * CH;
+        r[i] = load_part<ES>(base + ((int64_t)row * K + k) * ES, row < rows ? K - k : 0, end);
+      } else {
+        const int k = k0 + q % BK, row = r0 + (q / BK) * CH;
+        r[i] = load_part<ES>(base + ((int64_t)k * rows + row) * ES, k < K ? rows - row : 0, end);
+      }
+    }
+  }
+  __device__ __forceinline__ void store(char* lds, int t) const {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int q = t + i * NT;
+      if constexpr (KC) {
+        *(uint4*)(lds + (q / (kRowB / 16)) * kPitch + (q % (kRowB / 16)) * 16) = r[i];
+      } else {
+        const uint32_t w[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
+        char* p = lds + (q / BK) * CH * kPitch + (q % BK) * ES;
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+          if constexpr (ES == 4)
+            *(uint32_t*)(p + e * kPitch) = w[e];
+          else
+            *(unsigned short*)(p + e * kPitch) = (unsigned short)(w[e / 2] >> (16 * (e & 1)));
+        }
+      }
+    }
+  }
+};
+
+template <int DT, bool TA, bool TB, int G>
+__global__ __launch_bounds__(256) void bz_bgemm_mfma_kernel(const char* __restrict__ A, const char* __restrict__ B,
+                                                            typename Elem<DT>::T* __restrict__ C, int64_t sa, int64_t sb, int64_t sc,
+                                                            int M, int N, int K, int batch, int tiles_m, int tiles_n, int total_wg,
+                                                            int wg_per_xcd, float alpha, float beta) {
+  typedef typename Elem<DT>::T T;
+  typedef bz::fc::In<DT> IN;
+  constexpr int ES = IN::kSize;
+  constexpr int BK = kRowB / ES;
+  constexpr int TILE = G == 1 ? 64 : 32, NT = 256 / G;
+  __shared__ __attribute__((aligned(16))) char lds[G][2 * TILE * kPitch];
+  // the tiles of an item share its operands: neighbouring workgroups of one XCD (workgroups are dealt round robin)
+  const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
+  if (v >= total_wg) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tile = v % (tiles_m * tiles_n);
+  const int mine = v / (tiles_m * tiles_n) * G + (G == 1 ? 0 : wave);
+  const bool live = mine < batch;
+  const int64_t item = live ? mine : batch - 1;  // (a wave without an item of its own meets the barriers and stores nothing)
+  const int t = G == 1 ? threadIdx.x : lane;
+  const int m0 = tile / tiles_n * TILE, n0 = tile % tiles_n * TILE;
+  const char* a = A + item * sa * ES;
+  const char* b = B + item * sb * ES;
+  const char* a_end = a + (int64_t)M * K * ES;
+  const char* b_end = b + (int64_t)N * K * ES;
+  char* la = lds[G == 1 ? 0 : wave];
+  char* lb = la + TILE * kPitch;
+  Stage<DT, TILE, NT, !TA> ga;
+  Stage<DT, TILE, NT, TB> gb;
+  ga.load(a, a_end, t, m0, M, 0, K);
+  gb.load(b, b_end, t, n0, N, 0, K);
+  bz::fc::floatx16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const int wm = G == 1 ? (wave >> 1) * 32 : 0, wn = G == 1 ? (wave & 1) * 32 : 0;
+  const char* fa = la + (wm + (lane & 31)) * kPitch + (lane >> 5) * 16;
+  const char* fb = lb + (wn + (lane & 31)) * kPitch + (lane >> 5) * 16;
+  // a block wholly outside C leaves the matrix cores to the other workgroups of the CU (fp32 5x150x64: half of the blocks)
+  const bool works = m0 + wm < M && n0 + wn < N;
+  for (int k0 = 0; k0 < K; k0 += BK) {
+    ga.store(la, t);
+    gb.store(lb, t);
+    __syncthreads();
+    if (k0 + BK < K) {
+      ga.load(a, a_end, t, m0, M, k0 + BK, K);
+      gb.load(b, b_end, t, n0, N, k0 + BK, K);
+    }
+    const int steps = works ? (min(K - k0, BK) + IN::kStepK - 1) / IN::kStepK : 0;
+#pragma unroll
+    for (int ks = 0; ks < BK / IN::kStepK; ++ks)
+      if (ks < steps) IN::mma(*(const uint4*)(fa + ks * 32), *(const uint4*)(fb + ks * 32), acc);
+    __syncthreads();
+  }
+  // a lane owns column n and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4 of its block
+  const int n = n0 + wn + (lane & 31);
+  if (!live || n >= N) return;
+  T* c = C + item * sc + n;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int m = m0 + wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+    if (m < M) {
+      float x = alpha * acc[r];
+      if (beta != 0.f) x += beta * ld<T>(c + (int64_t)m * N);  // beta == 0: C is not read (BLAS rule)
+      st<T>(c + (int64_t)m * N, x);
+    }
+  }
+}
+
+template <int DT>
+int launch_bgemm(const bz_bgemm_desc& d, hipStream_t s) {
+  typedef typename Elem<DT>::T T;
+  // A single row on a matrix stored [K, N] reads every element of B once: no tile, no transposition.
+  if (d.m == 1 && !d.trans_b) {
+    const int grid = (d.batch + 3) / 4;
+    hipLaunchKernelGGL((bz_bgemm_row_kernel<T>), dim3(grid), dim3(256), 0, s, (const T*)d.a, (const T*)d.b, (T*)d.c, d.stride_a,
+                       d.stride_b, d.stride_c, d.n, d.k, d.batch, d.alpha, d.beta);
+    BZ_LAUNCH_OK("bz_bgemm_row_kernel");
+    return BZ_OK;
+  }
+  const bool small = d.m <= 32 && d.n <= 32;
+  const int tile = small ? 32 : 64;
+  const int64_t tiles_m = (d.m + tile - 1) / tile, tiles_n = (d.n + tile - 1) / tile;
+  const int64_t total = small ? (d.batch + 3) / 4 : tiles_m * tiles_n * d.batch;
+  BZ_REQUIRE(total < (1ll << 30), "bz_gemm_strided_batched: m=%d n=%d batch=%d make too many tiles", d.m, d.n, d.batch);
+  const int per_xcd = (int)((total + bz::kNumXcd - 1) / bz::kNumXcd);
+#define BZ_BGEMM(TA, TB, G)                                                                                                        \
+  hipLaunchKernelGGL((bz_bgemm_mfma_kernel<DT, TA, TB, G>), dim3(per_xcd * bz::kNumXcd), dim3(256), 0, s, (const char*)d.a,        \
+                     (const char*)d.b, (T*)d.c, d.stride_a, d.stride_b, d.stride_c, d.m, d.n, d.k, d.batch, (int)tiles_m,          \
+                     (int)tiles_n, (int)total, per_xcd, d.alpha, d.beta)
+#define BZ_BGEMM_G(TA, TB) \
+  if (small)               \
+    BZ_BGEMM(TA, TB, 4);   \
+  else                     \
+    BZ_BGEMM(TA, TB, 1)
+  if (d.trans_a && d.trans_b) {
+    BZ_BGEMM_G(true, true);
+  } else if (d.trans_a) {
+    BZ_BGEMM_G(true, false);
+  } else if (d.trans_b) {
+    BZ_BGEMM_G(false, true);
+  } else {
+    BZ_BGEMM_G(false, false);
+  }
+#undef BZ_BGEMM_G
 #undef BZ_BGEMM
+  BZ_LAUNCH_OK("bz_bgemm_mfma_kernel");
+  return BZ_OK;
 }
 
 // One wave per batch item, lanes over the channels.  Both sums walk t in ascending order, the weighted one with the
@@ -195,14 +395,8 @@ extern "C" int bz_gemm_strided_batched(const bz_bgemm_desc* desc, bz_stream_t st
   BZ_REQUIRE(d.stride_c >= (int64_t)d.m * d.n || d.batch <= 1, "bz_gemm_strided_batched: outputs overlap (stride_c=%lld)",
              (long long)d.stride_c);
   if (d.batch == 0) return BZ_OK;
-  const int grid = (d.batch + 3) / 4;
   hipStream_t s = bz::as_stream(stream);
-  if (d.dtype == BZ_F32)
-    launch_bgemm<float>(d, grid, s);
-  else if (d.dtype == BZ_F16)
-    launch_bgemm<__half>(d, grid, s);
-  else
-    return bz::fail(BZ_ENOTSUP, "bz_gemm_strided_batched: unsupported dtype %d", d.dtype);
-  BZ_LAUNCH_OK("bz_bgemm_kernel");
-  return BZ_OK;
+  if (d.dtype == BZ_F32) return launch_bgemm<BZ_F32>(d, s);
+  if (d.dtype == BZ_F16) return launch_bgemm<BZ_F16>(d, s);
+  return bz::fail(BZ_ENOTSUP, "bz_gemm_strided_batched: unsupported dtype %d", d.dtype);
 }
