@@ -66,6 +66,20 @@ BZ_API int bz_device_check(char* name, size_t cap);
  */
 BZ_API int bz_spin(int64_t microseconds, bz_stream_t stream);
 
+/*
+ * Copies from device-readable memory (pinned host memory as a rule) in one launch: a contiguous range of `bytes` (16-byte
+ * aligned, a multiple of 16; 0 = none) and up to BZ_FEED_MAX_ROWS pieces whose rows are a pitch apart at either end.
+ * Stands in for the copies of the reference's Feed (blaze/api/cpp_api/predictor_impl.cc:110-138).
+ */
+#define BZ_FEED_MAX_ROWS 8
+typedef struct bz_feed_rows {
+  const void* src;
+  void* dst;
+  int64_t rows, row_bytes;
+  int64_t src_pitch, dst_pitch; /* bytes between rows, at least row_bytes */
+} bz_feed_rows;
+BZ_API int bz_feed(const void* src, void* dst, int64_t bytes, const bz_feed_rows* rows, int n_rows, bz_stream_t stream);
+
 /* ------------------------------------------------------------------------- */
 /* Embedding                                                                  */
 /* ------------------------------------------------------------------------- */

@@ -1,0 +1,55 @@
+"""bz_feed: a contiguous range and strided pieces out of pinned host memory, against the bytes themselves."""
+import ctypes as C
+
+import pytest
+import torch
+
+import blaze_hip as bz
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("range_bytes,pieces", [
+    (0, [(1, 1, 1, 1)]),                                      # the smallest piece
+    (16, []),
+    (16384 * 3 + 16, [(300, 26, 26, 890)]),                   # a workgroup's edge, odd rows in a wide tensor
+    (1 << 20, [(2048, 128, 128, 1792), (7, 3, 5, 11)]),       # 16-byte units and single bytes in one launch
+    (0, [(5, 8, 8, 24), (1025, 4, 4, 12), (0, 4, 4, 4), (513, 2, 2, 2), (1, 16384, 16384, 16384), (3, 48, 64, 80), (2, 12, 12, 12),
+         (9, 1, 1, 2)]),                                      # every unit, an empty piece, as many pieces as a launch takes
+])
+def test_feed(range_bytes, pieces):
+    gen = torch.Generator().manual_seed(range_bytes + len(pieces))
+
+    def rand(n):
+        return torch.randint(256, (max(n, 1), ), generator=gen, dtype=torch.uint8)
+
+    src = rand(range_bytes).pin_memory()
+    dst = torch.full((max(range_bytes, 1) + 16, ), 7, dtype=torch.uint8, device="cuda")
+    rows = (bz.FeedRows * max(len(pieces), 1))()
+    keep = []
+    for i, (n, w, sp, dp) in enumerate(pieces):
+        s = rand(n * sp).pin_memory()
+        d = torch.full((n * dp + 16, ), 9, dtype=torch.uint8, device="cuda")
+        keep.append((s, d))
+        rows[i].src, rows[i].dst, rows[i].rows, rows[i].row_bytes, rows[i].src_pitch, rows[i].dst_pitch = s.data_ptr(), d.data_ptr(), n, w, sp, dp
+    bz.check(bz.lib().bz_feed(src.data_ptr(), dst.data_ptr(), range_bytes, rows, len(pieces), bz._stream_ptr()))
+    got = dst.cpu()
+    assert torch.equal(got[:range_bytes], src[:range_bytes]) and bool((got[range_bytes:] == 7).all())
+    for (n, w, sp, dp), (s, d) in zip(pieces, keep):
+        want = torch.full((n * dp + 16, ), 9, dtype=torch.uint8)
+        for r in range(n):
+            want[r * dp:r * dp + w] = s[r * sp:r * sp + w]
+        assert torch.equal(d.cpu(), want), (n, w, sp, dp)
+
+
+def test_feed_refuses():
+    rows = (bz.FeedRows * 9)()
+    buf = torch.zeros(64, dtype=torch.uint8).pin_memory()
+    call = bz.lib().bz_feed
+    p = buf.data_ptr()
+    assert call(p, p, 24, rows, 0, None) == bz.EINVAL      # no multiple of 16 bytes
+    assert call(p + 4, p, 16, rows, 0, None) == bz.EINVAL  # misaligned
+    assert call(None, None, 0, rows, 9, None) == bz.EINVAL
+    rows[0] = bz.FeedRows(p, p, 2, 8, 4, 8)                # rows that overlap
+    assert call(None, None, 0, rows, 1, None) == bz.EINVAL
+    assert C.sizeof(bz.FeedRows) == 48

@@ -151,9 +151,13 @@ void* Net::StreamOfLastLaunch() {
 
 bool Net::Run() {
   if (!Launch()) return false;
+  Wait();
+  return true;
+}
+
+void Net::Wait() {
   // all operators run on stream 0 of this thread: waiting for that stream waits for the net (simple_net.cc:27-32)
   if (!operators_.empty()) operators_.back()->WaitStream();
-  return true;
 }
 
 std::string Net::DumpProfile() const {

@@ -66,6 +66,9 @@ class Net {
   // that stream (null when the net has no device operator).  Run = Launch + waiting for the stream.
   bool Launch();
   void* StreamOfLastLaunch();
+  // waits as Run does, and the stream that it waits for (null when the last operator is a host one: nothing is waited for)
+  void Wait();
+  void* WaitedStream() { return operators_.empty() ? nullptr : operators_.back()->DeviceStream(); }
   const std::vector<std::string>& external_input() const { return external_input_; }
   const std::vector<std::string>& external_output() const { return external_output_; }
   Blob* external_input_blob(const std::string& name) const;

@@ -3,6 +3,7 @@
 #include <algorithm>
 
 #include "blaze/qed_store.h"
+#include "blaze_hip.h"
 
 namespace blaze {
 
@@ -16,7 +17,10 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
     cpu.set_device_type(kCPU);
     output_cpu_.push_back(std::make_shared<Blob>(cpu));
     output_cpu_.back()->set_data_type((DataType)b->data_type());
+    output_next_.push_back(std::make_shared<Blob>(cpu));
   }
+  output_wanted_.assign(output_cpu_.size(), false);
+  output_ahead_.assign(output_cpu_.size(), false);
   for (const auto& name : net_->external_input()) {
     Blob* b = net_->external_input_blob(name);
     BLAZE_CONDITION_THROW(b != nullptr, "external_input: ", name, " is not in external_input_blob");
@@ -73,6 +77,20 @@ bool Predictor::ReshapeInput(size_t idx, const std::vector<size_t>& shape) {
   return true;
 }
 
+namespace {
+// rows of a 2-D input that lives inside a Concat's output, from a dense staging copy
+bz_feed_rows StridedRows(Blob* blob, const void* staged) {
+  const int64_t es = (int64_t)DataTypeSize(blob->data_type()), w = (int64_t)blob->shape()[1] * es;
+  bz_feed_rows r;
+  r.src = staged;
+  r.dst = blob->data();
+  r.rows = (int64_t)blob->shape()[0];
+  r.row_bytes = r.src_pitch = w;
+  r.dst_pitch = (int64_t)blob->pitch() * es;
+  return r;
+}
+}  // namespace
+
 bool Predictor::Feed(const char* name, const void* data, size_t len) {
   const int idx = InputName2Idx(name);
   if (idx < 0) {
@@ -116,8 +134,11 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
       stage->Reshape(blob->shape());
       memcpy(stage->data(), data, need);
       if (blob->pitch() != 0) {  // the input lives inside a Concat's output: rows are `pitch` elements apart
-        const size_t es = DataTypeSize(blob->data_type()), w = blob->shape()[1] * es;
-        HIP_CHECK(hipMemcpy2DAsync(blob->data(), blob->pitch() * es, stage->data(), w, w, blob->shape()[0], hipMemcpyHostToDevice, st));
+        const bz_feed_rows r = StridedRows(blob, stage->data());
+        if (IsPinnedHost(stage->data()))
+          BZ_CHECK(bz_feed(nullptr, nullptr, 0, &r, 1, st));
+        else  // (staging the runtime could not pin: a kernel cannot read it)
+          HIP_CHECK(hipMemcpy2DAsync(r.dst, r.dst_pitch, r.src, r.src_pitch, r.row_bytes, r.rows, hipMemcpyHostToDevice, st));
       } else if (need > 0) {
         HIP_CHECK(hipMemcpyAsync(blob->data(), stage->data(), need, hipMemcpyHostToDevice, st));
       }
@@ -132,6 +153,14 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
   return true;
 }
 
+// A request is moved in as many even parts as it has whole megabytes (at least one), each launched as soon as it is
+// staged.  Staging runs at 58 GB/s and the kernel at 47, so the transfer hides under the staging but for the last part and
+// the difference; a launch costs the host 2.9 us, the time of 160 KB, so that 1 MB in four parts was 5 us slower than in
+// one.  (The copy engine moves 57 GB/s, but each copy costs 10 us until what follows it on the stream may start: 5 MB in
+// ten parts arrived 230 us after the first byte was staged, in one part behind the whole staging 210, through five
+// launches of the kernel 162.)
+constexpr size_t kFeedPart = 1 << 20;
+
 bool Predictor::FeedMany(int count, const char* const* names, const void* const* data, const size_t* lens) {
   try {
     struct Item {
@@ -139,7 +168,8 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       int arg;
       size_t offset;
     };
-    std::vector<Item> in_arena;
+    // plain inputs first, in one range that lands as it is staged; inputs that live inside a Concat's output behind them
+    std::vector<Item> in_arena, strided;
     size_t total = 0;
     const DeviceOption* dev = nullptr;
     for (int i = 0; i < count; ++i) {
@@ -154,15 +184,28 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
         LOG_ERROR("The len=%zu need size=%zu blob->size()=%zu", lens[i], need, (size_t)blob->size());
         return false;
       }
-      if (blob->device_type() != kHIP || blob->pitch() != 0) {
+      if (blob->device_type() != kHIP) {
         if (!Feed((size_t)idx, data[i], lens[i])) return false;
         continue;
       }
       dev = &blob->device_option();
+      if (blob->pitch() != 0) {
+        auto same = std::find_if(strided.begin(), strided.end(), [&](const Item& it) { return it.idx == idx; });
+        if (same != strided.end())
+          same->arg = i;  // named twice: the last one counts, and two pieces of one launch must not share a target
+        else
+          strided.push_back({idx, i, 0});
+        continue;
+      }
       in_arena.push_back({idx, i, total});
       total += (need + 255) / 256 * 256;  // every slice 256-byte aligned
     }
-    if (in_arena.empty()) return true;
+    if (dev == nullptr) return true;
+    const size_t plain = total;
+    for (Item& it : strided) {
+      it.offset = total;
+      total += (lens[it.arg] + 255) / 256 * 256;
+    }
     HIPContext ctx(*dev);
     ctx.Activate();
     hipStream_t st = ctx.hip_stream();
@@ -183,9 +226,39 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       HIP_CHECK(hipMalloc((void**)&arena_dev_, cap));
       arena_cap_ = cap;
     }
-    for (const Item& it : in_arena) memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
-    HIP_CHECK(hipMemcpyAsync(arena_dev_, arena_host_, total, hipMemcpyHostToDevice, st));
-    HIP_CHECK(hipEventRecord(feed_done_, st));
+    // from the first launch on the arena is being read: whatever happens next, it is waited for before it is written again
+    try {
+      const size_t parts = std::max<size_t>(plain / kFeedPart, 1), part = (plain / parts / 256 + 1) * 256;
+      bz_feed_rows rows[BZ_FEED_MAX_ROWS];
+      size_t moved = 0;
+      int n = 0;
+      auto launch = [&](size_t upto) {
+        BZ_CHECK(bz_feed(arena_host_ + moved, arena_dev_ + moved, (int64_t)(upto - moved), rows, n, st));
+        moved = upto;
+        n = 0;
+      };
+      for (const Item& it : strided) {
+        if (n == BZ_FEED_MAX_ROWS) launch(moved);
+        memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
+        rows[n++] = StridedRows(external_input_blob_[it.idx], arena_host_ + it.offset);
+      }
+      for (const Item& it : in_arena)
+        for (size_t at = 0; at < lens[it.arg];) {
+          // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte)
+          const size_t len = std::min(lens[it.arg] - at, moved + part - (it.offset + at));
+          memcpy(arena_host_ + it.offset + at, (const char*)data[it.arg] + at, len);
+          at += len;
+          if (it.offset + at == moved + part) launch(it.offset + at);
+        }
+      if (plain > moved || n > 0) launch(plain);
+      HIP_CHECK(hipEventRecord(feed_done_, st));
+      any_feed_pending_ = true;
+    } catch (...) {
+      (void)hipStreamSynchronize(st);  // no event stands behind what was launched
+      any_feed_pending_ = false;
+      throw;
+    }
+    for (const Item& it : strided) feed_pending_[it.idx] = true;
     for (const Item& it : in_arena) {
       Blob* blob = external_input_blob_[it.idx];
       // (also when the slice did not move: this records the slice's new size and clears "unplaced")
@@ -193,7 +266,6 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       blob->RefReshape(shape, arena_dev_ + it.offset, /*arena_view=*/true);
       feed_pending_[it.idx] = true;
     }
-    any_feed_pending_ = true;
   } catch (std::exception& e) {
     LOG_ERROR("feed failed: %s", e.what());
     last_error_for_thread() = e.what();
@@ -232,6 +304,7 @@ bool Predictor::ForwardLaunch() {
         break;
       }
     }
+    output_ahead_.assign(output_ahead_.size(), false);
     if (!net_->Launch()) return false;
     launched_on_ = net_->StreamOfLastLaunch();
     if (launched_on_ != nullptr) {
@@ -287,7 +360,10 @@ bool Predictor::Forward(const PredictorCallback&& cb) {
         break;
       }
     }
-    if (!net_->Run()) return false;
+    output_ahead_.assign(output_ahead_.size(), false);
+    if (!net_->Launch()) return false;
+    QueueOutputs();
+    net_->Wait();
     if (any_feed_pending_) {  // Run waited for the stream, which had waited for the transfers
       std::fill(feed_pending_.begin(), feed_pending_.end(), false);
       any_feed_pending_ = false;
@@ -299,6 +375,38 @@ bool Predictor::Forward(const PredictorCallback&& cb) {
     last_error_for_thread() = e.what();
     return false;
   }
+}
+
+// Outputs that were read after the last Forward are copied to the host behind this one, under the same wait: a copy asked
+// for by Output alone is another launch and another wait, 16 us of a 58 us request.  Small ones only, by a kernel that
+// writes the pinned copy over the link (the copy engine's hand-over would cost more than it moves); larger ones are
+// copied by Output.  Into a second buffer: the one Output handed out stays as it is until the next Output.
+void Predictor::QueueOutputs() {
+  constexpr size_t kMax = 64 << 10;
+  hipStream_t st = (hipStream_t)net_->WaitedStream();
+  bz_feed_rows rows[BZ_FEED_MAX_ROWS];
+  int n = 0;
+  for (size_t i = 0; i < external_output_blob_.size() && n < BZ_FEED_MAX_ROWS; ++i) {
+    const bool wanted = output_wanted_[i];
+    output_wanted_[i] = false;
+    Blob* blob = external_output_blob_[i];
+    const size_t bytes = blob->size() * DataTypeSize(blob->data_type());
+    if (!wanted || st == nullptr || blob->device_type() != kHIP || blob->pitch() != 0 || blob->data() == nullptr || bytes == 0 || bytes > kMax)
+      continue;
+    Blob* next = output_next_[i].get();
+    next->set_data_type((DataType)blob->data_type());
+    next->Reshape(blob->shape());
+    if (!IsPinnedHost(next->data())) continue;
+    rows[n].src = blob->data();
+    rows[n].dst = next->data();
+    rows[n].rows = 1;
+    rows[n].row_bytes = rows[n].src_pitch = rows[n].dst_pitch = (int64_t)bytes;
+    ++n;
+    output_ahead_[i] = true;
+  }
+  if (n == 0) return;
+  const int rc = bz_feed(nullptr, nullptr, 0, rows, n, st);
+  if (rc != 0) output_ahead_.assign(output_ahead_.size(), false);  // Output copies by itself
 }
 
 bool Predictor::Output(const char* name, void** data, size_t* len) {
@@ -321,11 +429,17 @@ bool Predictor::Output(size_t idx, void** data, size_t* len) {
       *data = blob->data();
     } else {
       std::shared_ptr<Blob>& cpu = output_cpu_[idx];
-      cpu->set_data_type((DataType)blob->data_type());
-      cpu->Reshape(blob->shape());
-      HIPContext ctx(blob->device_option());
-      ctx.Activate();
-      CopyBytes(cpu->data(), kCPU, blob->data(), kHIP, bytes, ctx.hip_stream());
+      output_wanted_[idx] = true;
+      if (output_ahead_[idx]) {  // (a second Output of the same pass copies again)
+        cpu.swap(output_next_[idx]);
+        output_ahead_[idx] = false;
+      } else {
+        cpu->set_data_type((DataType)blob->data_type());
+        cpu->Reshape(blob->shape());
+        HIPContext ctx(blob->device_option());
+        ctx.Activate();
+        CopyBytes(cpu->data(), kCPU, blob->data(), kHIP, bytes, ctx.hip_stream());
+      }
       *data = cpu->data();
     }
   } catch (std::exception& e) {

@@ -38,10 +38,10 @@ class Predictor {
   // copies len bytes in; len must equal size * sizeof(dtype) (predictor_impl.cc:110-138)
   bool Feed(const char* name, const void* data, size_t len);
   bool Feed(size_t idx, const void* data, size_t len);
-  // extension: feed `count` inputs at once.  Inputs that are plain device tensors travel in ONE transfer: they are
-  // staged side by side in a pinned arena, copied to a device arena of the same layout, and the input blobs become
-  // views of their slices (a model with 26 feature groups has 79 inputs; one queued copy instead of 79).  Other
-  // inputs (host tensors, inputs living inside a Concat's output) are fed one by one.
+  // extension: feed `count` inputs at once.  The device inputs are staged side by side in a pinned arena
+  // and cross together: plain ones into a device arena of the same layout, whose slices the input blobs become views of,
+  // those that live inside a Concat's output straight into their rows (a model with 26 feature groups has 79 inputs; one
+  // launch, or a few while the rest is being staged, instead of 79 copies).  Host tensors are fed one by one.
   bool FeedMany(int count, const char* const* names, const void* const* data, const size_t* lens);
   size_t InputSize() const { return external_input_blob_.size(); }
   int InputDataType(const char* name) const;
@@ -85,6 +85,10 @@ class Predictor {
   std::vector<Blob*> external_input_blob_, external_output_blob_;
   std::unordered_map<std::string, int> input_index_, output_index_;
   std::vector<std::shared_ptr<Blob>> output_cpu_;
+  std::vector<std::shared_ptr<Blob>> output_next_;  // what Forward copied ahead of Output (QueueOutputs)
+  std::vector<bool> output_wanted_;                 // read since the last Forward
+  std::vector<bool> output_ahead_;                  // output_next_ holds the last Forward's result
+  void QueueOutputs();
   // pinned staging of fed inputs: Feed copies the caller's bytes here and queues the transfer on the thread's
   // stream; Forward runs behind it on the same stream.  feed_pending_[i]: input i's staging is still being read.
   std::vector<std::shared_ptr<Blob>> input_cpu_;

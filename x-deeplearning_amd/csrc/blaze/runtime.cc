@@ -63,6 +63,11 @@ void Free(void* ptr, int device_type, int) {
   }
 }
 
+bool IsPinnedHost(const void* ptr) {
+  std::lock_guard<std::mutex> lock(g_pinned_mu);
+  return PinnedSet().count(const_cast<void*>(ptr)) != 0;
+}
+
 void HIPContext::Activate() const {
   static thread_local int current = -1;
   if (current != device_id_) {

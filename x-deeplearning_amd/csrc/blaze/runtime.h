@@ -20,6 +20,8 @@ namespace blaze {
 // (hipHostMalloc) whenever a device is usable, so Feed / Output copies run at full PCIe rate; plain malloc otherwise.
 void* Alloc(size_t bytes, int device_type, int device_id);
 void Free(void* ptr, int device_type, int device_id);
+// whether `ptr` is a block of Alloc's that kernels can read and write (kCPU memory that could be pinned)
+bool IsPinnedHost(const void* ptr);
 // number of device / pinned-host allocations the host layer has made in this process (Alloc above plus the feed
 // arenas and the Embedding operator's slot and offset buffers): lets a serving loop check that its steady state
 // allocates nothing
