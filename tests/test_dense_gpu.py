@@ -148,6 +148,24 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + N * 3 + K)
 
 
+# Few 32x32 tiles (512 of fp32, 256 of 2-byte operands) go to the kernel whose eight waves share K in units of 128 bytes;
+# rows that start on no 16 bytes, beyond that, to the staged tiles with loads at any element.
+@pytest.mark.parametrize("in_name,out_name", [("f32", "f32"), ("f16", "f16"), ("bf16", "f32")])
+@pytest.mark.parametrize("M,N,K,act,kw", [
+    (1, 9, 1, "none", {}), (33, 40, 3, "prelu", {}), (31, 64, 31, "dice", {}),   # a partial unit only
+    (32, 32, 64, "relu", {}), (65, 33, 65, "dice", {}),                          # whole units and one element
+    (7, 100, 2075, "sigmoid", {}), (96, 70, 1023, "prelu", {"full_bias": True}),  # units a wave, ragged; a bias a row
+    (40, 24, 513, "none", {"alpha": 0.5, "beta": 2.0}),
+    (512, 512, 96, "prelu", {}), (513, 512, 96, "prelu", {}),                     # the last size of 256 tiles, the first beyond
+    (1024, 512, 77, "dice", {}), (1025, 512, 77, "dice", {}),                     # 512
+    (3000, 200, 5, "relu", {}), (2100, 300, 9, "none", {"full_bias": True}),      # staged: K about a chunk
+    (4100, 1000, 73, "prelu", {}), (8200, 1000, 201, "dice", {}), (33000, 80, 215, "dice", {}),  # 64x128, 128x128, 128x96
+])
+def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, act, kw):
+    print("case any %s M=%d N=%d K=%d act=%s %r" % (in_name, M, N, K, act, kw), flush=True)
+    _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + 5 * N + K, **kw)
+
+
 # Large 2-byte layers go to the streaming kernel (256x128 tiles, loader waves, operands straight into LDS) once
 # ceil(M/256) * ceil(N/128) >= 200, K is a multiple of 64 and at least 512, and the output takes 16-byte stores.
 @pytest.mark.parametrize("in_name", ["f16", "bf16"])

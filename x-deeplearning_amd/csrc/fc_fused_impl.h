@@ -40,43 +40,50 @@ namespace {
 
 using namespace bz::fc;
 
-// one 16-byte chunk of a K-contiguous operand row; zero beyond K; element-wise when unaligned
+// one 16-byte chunk of a K-contiguous operand row that may start anywhere; a chunk that reaches beyond K is read by
+// elements and zero there
 template <int DT>
-__device__ __forceinline__ uint4 load_chunk(const char* base, int64_t row, int64_t ld, int k, int K, bool vec_ok) {
+__device__ __forceinline__ uint4 load_chunk(const char* base, int64_t row, int64_t ld, int k, int K) {
   constexpr int ES = In<DT>::kSize;
   constexpr int CH = In<DT>::kChunk;
-  uint4 out = make_uint4(0, 0, 0, 0);
-  if (k >= K) return out;
   const char* p = base + (row * ld + k) * ES;
-  if (vec_ok && k + CH <= K) return *(const uint4*)p;
-  if constexpr (ES == 2) {
-    if (((uintptr_t)p & 3) == 0) {
-      // rows that start on 4 bytes (an even row length, e.g. a Concat of 3 x 54 columns): pairs of elements
-      uint32_t d[4];
+  uint4 out = make_uint4(0, 0, 0, 0);
+  if (k + CH <= K) {
+    __builtin_memcpy(&out, p, 16);
+  } else if (k < K) {
+    uint32_t e[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        d[i] = 0u;
-        if (k + 2 * i + 1 < K)
-          d[i] = *(const uint32_t*)(p + 4 * i);
-        else if (k + 2 * i < K)
-          d[i] = *(const unsigned short*)(p + 4 * i);
+    for (int i = 0; i < CH - 1; ++i)
+      if (k + i < K) {
+        if constexpr (ES == 2)
+          e[i / 2] |= (uint32_t) * (const unsigned short*)(p + 2 * i) << (16 * (i & 1));
+        else
+          e[i] = *(const uint32_t*)(p + 4 * i);
       }
-      return make_uint4(d[0], d[1], d[2], d[3]);
-    }
-    unsigned short e[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) e[i] = (k + i < K) ? *(const unsigned short*)(p + 2 * i) : (unsigned short)0;
-    out.x = e[0] | ((uint32_t)e[1] << 16);
-    out.y = e[2] | ((uint32_t)e[3] << 16);
-    out.z = e[4] | ((uint32_t)e[5] << 16);
-    out.w = e[6] | ((uint32_t)e[7] << 16);
-  } else {
-    uint32_t e[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) e[i] = (k + i < K) ? *(const uint32_t*)(p + 4 * i) : 0u;
     out = make_uint4(e[0], e[1], e[2], e[3]);
   }
   return out;
+}
+
+// The same without a branch, for K of at least a chunk: the chunk is read from where it lies wholly inside the row, and
+// shift_chunk drops the elements before k (and brings zeros in behind) when it is put into LDS.  The memory system takes
+// 16-byte loads at any element; by elements and with one K tile in flight, 4096 x 3071 -> 1024 fp16 took 159 us and
+// 600 x 900 -> 512 16.4.
+template <int DT>
+__device__ __forceinline__ uint4 load_chunk_anywhere(const char* base, int64_t row, int64_t ld, int k, int K) {
+  uint4 out;
+  __builtin_memcpy(&out, base + (row * ld + min(k, K - In<DT>::kChunk)) * In<DT>::kSize, 16);
+  return out;
+}
+// `n` elements out at the front, zeros in at the back (n >= the chunk: all zeros)
+template <int DT>
+__device__ __forceinline__ uint4 shift_chunk(uint4 v, int n) {
+  const int b = n * In<DT>::kSize;
+  if (b & 4) v = make_uint4(v.y, v.z, v.w, 0u);
+  if (b & 8) v = make_uint4(v.z, v.w, 0u, 0u);
+  if (b & 2) v = make_uint4(v.x >> 16 | v.y << 16, v.y >> 16 | v.z << 16, v.z >> 16 | v.w << 16, v.w >> 16);
+  if (b >= 16) v = make_uint4(0, 0, 0, 0);
+  return v;
 }
 
 // The same for operands whose rows are 16-byte aligned and K a multiple of the chunk (a chunk is either wholly inside
@@ -141,8 +148,8 @@ struct HeadArgs {
 template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD>
 __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                   OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
-                                                                  int64_t ldw, int64_t ldy, bool vec_a, bool vec_w,
-                                                                  bool vec_y, int tiles_m, Epilogue ep, HeadArgs head) {
+                                                                  int64_t ldw, int64_t ldy, bool vec_y, int tiles_m, Epilogue ep,
+                                                                  HeadArgs head) {
   using T = In<DT>;
   constexpr int NT = WM * WN * 64;
   constexpr int ES = T::kSize;
@@ -186,7 +193,7 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
         const int r = q / CPR, ch = q % CPR;
         int m = m0 + r;
         m = m < M ? m : M - 1;
-        ra[set][i] = !ALIGNED ? load_chunk<DT>(A, m, lda, k0 + ch * T::kChunk, K, vec_a)
+        ra[set][i] = !ALIGNED ? load_chunk_anywhere<DT>(A, m, lda, k0 + ch * T::kChunk, K)
                      : CLAMPED ? load_chunk_clamped<DT>(A, m, lda, k0 + ch * T::kChunk, K)
                             : load_chunk_aligned<DT>(A, m, lda, k0 + ch * T::kChunk, K);
       }
@@ -198,14 +205,15 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
         const int r = q / CPR, ch = q % CPR;
         int n = n0 + r;
         n = n < N ? n : N - 1;
-        rw[set][i] = !ALIGNED ? load_chunk<DT>(W, n, ldw, k0 + ch * T::kChunk, K, vec_w)
+        rw[set][i] = !ALIGNED ? load_chunk_anywhere<DT>(W, n, ldw, k0 + ch * T::kChunk, K)
                      : CLAMPED ? load_chunk_clamped<DT>(W, n, ldw, k0 + ch * T::kChunk, K)
                             : load_chunk_aligned<DT>(W, n, ldw, k0 + ch * T::kChunk, K);
       }
     }
   };
-  // registers -> LDS (chunks beyond K already arrived as zeros, except from the clamped loader)
-  auto masked = [&](uint4 v, int k) {
+  // registers -> LDS (chunks beyond K already arrived as zeros, except from the clamped loaders)
+  auto masked = [&](uint4 v, int k, bool inside) {
+    if (!ALIGNED && !inside) return shift_chunk<DT>(v, k - min(k, K - T::kChunk));
     if (ALIGNED && CLAMPED) {
       const uint32_t keep = k < K ? 0xffffffffu : 0u;
       v.x &= keep;
@@ -216,17 +224,18 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
     return v;
   };
   auto lstore = [&](int set, int buf, int k0) {
+    const bool inside = k0 + BK <= K;
 #pragma unroll
     for (int i = 0; i < A_PER; ++i) {
       const int q = tid + i * NT;
       if (A_CHUNKS % NT == 0 || q < A_CHUNKS)
-        *(uint4*)&lds[buf][(q / CPR) * PITCH + (q % CPR) * 16] = masked(ra[set][i], k0 + (q % CPR) * T::kChunk);
+        *(uint4*)&lds[buf][(q / CPR) * PITCH + (q % CPR) * 16] = masked(ra[set][i], k0 + (q % CPR) * T::kChunk, inside);
     }
 #pragma unroll
     for (int i = 0; i < W_PER; ++i) {
       const int q = tid + i * NT;
       if (W_CHUNKS % NT == 0 || q < W_CHUNKS)
-        *(uint4*)&lds[buf][(BM + q / CPR) * PITCH + (q % CPR) * 16] = masked(rw[set][i], k0 + (q % CPR) * T::kChunk);
+        *(uint4*)&lds[buf][(BM + q / CPR) * PITCH + (q % CPR) * 16] = masked(rw[set][i], k0 + (q % CPR) * T::kChunk, inside);
     }
   };
 
@@ -754,13 +763,116 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 #undef BZ_PIN_PHASE
 
 // ---------------------------------------------------------------------------------------------
+// split kernel: few tiles, or rows that start on no 16 bytes
+// ---------------------------------------------------------------------------------------------
+// A workgroup owns a 32 x 32 tile of C and its eight waves share the K range: unit u (128 bytes of every row) is
+// wave u % 8's.  A wave loads its units straight into MFMA fragments, the next unit's loads in flight while the present
+// one is multiplied; nothing goes through LDS and no wave waits for another before the partial tiles are added up.
+//  - Few tiles leave the chip idle and the chain of K tiles sets the time: eight waves walk it in an eighth of the steps.
+//  - A lane's 16 bytes may start anywhere (a row pitch of 445 fp16 elements): the memory system takes such loads, and
+//    the lines they share are L1 hits.
+// It is bound by the path into a CU (a load instruction touches 32 lines for 1 KB), which is why it stops at few tiles, why
+// the compiler's choice to keep few loads in flight and many waves resident is left alone (all of two units' loads pinned
+// ahead of the multiplications: 5 to 30 % slower), and why wider tiles a workgroup
+// (64 x 64: 32 x 2075 -> 768 fp32 47 us against 17) do not pay.
+constexpr int kSplitWaves = 8, kSplitUnit = 128;
+
+template <int DT, typename OutT>
+__global__ __launch_bounds__(kSplitWaves * 64, 2) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
+                                                                          OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
+                                                                          int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
+  using T = In<DT>;
+  constexpr int ES = T::kSize, NW = kSplitWaves, STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
+  constexpr int PITCH = 33;
+  __shared__ float red[NW / 2][32 * PITCH];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = (int)(blockIdx.x % tiles_m) * 32, n0 = (int)(blockIdx.x / tiles_m) * 32;
+  const int frow = lane & 31, fhalf = lane >> 5;
+  const int am = min(m0 + frow, M - 1), wn = min(n0 + frow, N - 1);
+  const char* pa = A + (int64_t)am * lda * ES + fhalf * 16;
+  const char* pw = W + (int64_t)wn * ldw * ES + fhalf * 16;
+  floatx16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+
+  struct Unit {
+    uint4 a[STEPS], w[STEPS];
+  };
+  auto mma = [&](const Unit& x) {
+#pragma unroll
+    for (int ks = 0; ks < STEPS; ++ks) T::mma(x.a[ks], x.w[ks], acc);
+  };
+  const int whole = (int)((int64_t)K * ES / kSplitUnit);
+  // (no branch round the loads of a unit that does not exist: the last whole one is read again)
+  auto load = [&](Unit& x, int u) {
+    const int64_t off = (int64_t)min(u, whole - 1) * kSplitUnit;
+#pragma unroll
+    for (int ks = 0; ks < STEPS; ++ks) {
+      __builtin_memcpy(&x.a[ks], pa + off + ks * 32, 16);
+      __builtin_memcpy(&x.w[ks], pw + off + ks * 32, 16);
+    }
+  };
+  if (wave < whole) {
+    Unit x, y;
+    load(x, wave);
+    for (int u = wave; u < whole; u += 2 * NW) {
+      load(y, u + NW);
+      mma(x);
+      if (u + NW >= whole) break;
+      load(x, u + 2 * NW);
+      mma(y);
+    }
+  }
+  if ((int64_t)whole * kSplitUnit < (int64_t)K * ES && wave == whole % NW) {
+    const int k0 = whole * (kSplitUnit / ES);
+#pragma unroll
+    for (int ks = 0; ks < STEPS; ++ks)
+      if (k0 + ks * T::kStepK < K) {
+        const int k = k0 + ks * T::kStepK + fhalf * T::kChunk;
+        if (K >= T::kChunk) {
+          const int drop = k - min(k, K - T::kChunk);
+          T::mma(shift_chunk<DT>(load_chunk_anywhere<DT>(A, am, lda, k, K), drop),
+                 shift_chunk<DT>(load_chunk_anywhere<DT>(W, wn, ldw, k, K), drop), acc);
+        } else {
+          T::mma(load_chunk<DT>(A, am, lda, k, K), load_chunk<DT>(W, wn, ldw, k, K), acc);
+        }
+      }
+  }
+  // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper four waves hand theirs to the
+  // lower four, which add their own at the same places
+  float* mine = red[wave % (NW / 2)] + 4 * fhalf * PITCH + frow;
+  if (wave >= NW / 2) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mine[(8 * (r >> 2) + (r & 3)) * PITCH] = acc[r];
+  }
+  __syncthreads();
+  if (wave < NW / 2) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mine[(8 * (r >> 2) + (r & 3)) * PITCH] += acc[r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 32 * 32 / (NW * 64); ++e) {
+    const int q = tid + e * NW * 64, ml = q / 32, nl = q % 32;
+    const int m = m0 + ml, n = n0 + nl;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW / 2; ++w) v += red[w][ml * PITCH + nl];
+    if (m < M && n < N) {
+      const float b = ep.bias_rows == 0 ? 0.f : ep.bias[ep.bias_rows == 1 ? n : full_bias_index(ep, m, n, M, N)];
+      store_out<OutT>(Y + out_index(ep, m, n, ldy), apply_act(fmaf(ep.alpha, v, ep.beta * b), n, ep));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // skinny kernel: N <= 8
 // ---------------------------------------------------------------------------------------------
 template <int DT, typename OutT>
 __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                            OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
-                                                           int64_t ldw, int64_t ldy, bool vec_a, bool vec_w, int lpr,
-                                                           Epilogue ep) {
+                                                           int64_t ldw, int64_t ldy, int lpr, Epilogue ep) {
   constexpr int CH = In<DT>::kChunk;
   const int tid = threadIdx.x;
   const int g = tid / lpr, l = tid - g * lpr;
@@ -786,12 +898,12 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
     for (int n = 0; n < kSkinnyMaxN; ++n) acc[n] = 0.f;
     for (int c = l; c < nchunks; c += lpr) {
       float a[CH];
-      chunk_to_float<DT>(load_chunk<DT>(A, m, lda, c * CH, K, vec_a), a);
+      chunk_to_float<DT>(load_chunk<DT>(A, m, lda, c * CH, K), a);
 #pragma unroll
       for (int n = 0; n < kSkinnyMaxN; ++n) {
         if (n < N) {
           float w[CH];
-          chunk_to_float<DT>(load_chunk<DT>(W, n, ldw, c * CH, K, vec_w), w);
+          chunk_to_float<DT>(load_chunk<DT>(W, n, ldw, c * CH, K), w);
 #pragma unroll
           for (int i = 0; i < CH; ++i) acc[n] = fmaf(a[i], w[i], acc[n]);
         }
@@ -845,7 +957,7 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
 
 
 template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false>
-int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
+int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
   // output rows 16-byte aligned and N a whole number of 16-byte chunks: coalesced stores through LDS
   // (with split outputs every slice must start on a chunk boundary as well)
@@ -864,9 +976,18 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w,
     head.out_dtype = d.head_out_dtype;
   }
   hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD>), dim3(tiles_m * tiles_n), dim3(WM * WN * 64), 0,
-                     st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_a, vec_w, vec_y,
-                     tiles_m, ep, head);
+                     st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
+  return BZ_OK;
+}
+
+
+template <int DT, typename OutT>
+int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+  const int tiles_m = (d.m + 31) / 32, tiles_n = (d.n + 31) / 32;
+  hipLaunchKernelGGL((bz_fc_split_kernel<DT, OutT>), dim3(tiles_m * tiles_n), dim3(kSplitWaves * 64), 0, st, (const char*)d.a,
+                     (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, tiles_m, ep);
+  BZ_LAUNCH_OK("bz_fc_split_kernel");
   return BZ_OK;
 }
 
@@ -900,30 +1021,55 @@ template <int DT, typename OutT>
 int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   if (d.n <= 64) {
-    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, true>(d, ep, true, true, st);
-    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true>(d, ep, true, true, st);
+    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, true>(d, ep, st);
+    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true>(d, ep, st);
   }
-  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, true>(d, ep, true, true, st);
+  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, true>(d, ep, st);
   // eight waves: with one workgroup per 32 rows only M / 32 CUs work, and each has 288 KB of operands to pull in
   // (two K tiles in flight: with eight waves taking turns that hides the loads, and it is faster than four both alone,
   // 10.5 against 11.3 us on config 2's 512 -> 256 -> 2, and next to other kernels)
-  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, true>(d, ep, true, true, st);
+  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, true>(d, ep, st);
+}
+
+// The tiles of the staged kernel that both kinds of rows take (ALIGNED: every row starts on 16 bytes and K is a whole
+// number of chunks)
+template <int DT, typename OutT, bool ALIGNED>
+int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+  constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
+  const int64_t wg128 = (int64_t)((d.m + 127) / 128) * ((d.n + 127) / 128);
+  const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
+  const int64_t wg64x128 = (int64_t)((d.m + 63) / 64) * ((d.n + 127) / 128);
+  // tall and narrow (the attention MLP over batch x history rows): one 96-wide tile reads A once
+  if (d.n > 64 && d.n <= 96 && (d.m + 127) / 128 >= 256)
+    return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, ALIGNED>(d, ep, st);
+  if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
+  if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  if (wg64 >= 256) {
+    // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
+    // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
+    // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.
+    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  }
+  return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
 }
 
 template <int DT, typename OutT>
 int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
-  const int64_t wg128 = (int64_t)((d.m + 127) / 128) * ((d.n + 127) / 128);
-  const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
-  // rows 16-byte aligned and K a whole number of chunks: branch-free loads, several tiles in flight
+  // rows 16-byte aligned and K a whole number of chunks
   const bool aligned = vec_a && vec_w && d.k % In<DT>::kChunk == 0;
-  if (!aligned) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, false>(d, ep, vec_a, vec_w, st);
+  // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Up to 512 32x32 tiles of fp32
+  // (1024 x 896 -> 512: 17.6 us against the staged tile's 23.2; 2048 x 512 -> 256 10.9 and 15.1; 2048 x 896 -> 512, 1024
+  // tiles, 33 and 24) and 256 of 2-byte operands, which the path into a CU feeds at half the fp32 rate a multiplication
+  // (256 x 3000 -> 512: 10.5 and 17.4; 512 x 600 -> 512 6.4 and 7.1; 1024 x 1000 -> 512, 512 tiles, 10.5 and 8.5).
+  const int64_t wg32 = (int64_t)((d.m + 31) / 32) * ((d.n + 31) / 32);
+  if (d.k < In<DT>::kChunk || wg32 <= (In<DT>::kSize == 4 ? 512 : 256)) return launch_split<DT, OutT>(d, ep, st);
+  if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
   // Largest first, and never a tile much wider than N.  128x256 with eight waves and three K tiles in flight fills the
   // chip once it has a workgroup per CU (its fp32 output tile would not fit the operand buffers it is staged in, so
   // 2-byte outputs only); below that, 128x128; then 64x128 while that still gives two workgroups per CU; then the
   // latency-bound small tiles.
   const int64_t wg128x256 = (int64_t)((d.m + 127) / 128) * ((d.n + 255) / 256);
-  const int64_t wg64x128 = (int64_t)((d.m + 63) / 64) * ((d.n + 127) / 128);
   if constexpr (sizeof(OutT) == 2 && In<DT>::kSize == 2) {
     // the streaming kernel once its 256x128 tiles keep most CUs busy and K is deep enough to pay for filling its ring
     // (8192 x 12800 -> 1024 bf16: 192 against 238 us; 4096^3: 128 against 139 us)
@@ -939,25 +1085,14 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
     // (256x256 once even that fills the chip: 4096^3 bf16 987 against 885 TFLOP/s; with fp32 operands these two tiles
     // do not fit the registers)
     const int64_t wg256 = (int64_t)((d.m + 255) / 256) * ((d.n + 255) / 256);
-    if (wg256 >= 256 && d.bias_rows <= 1) return launch_mfma<DT, OutT, 256, 256, BK, 4, 2, 2, true>(d, ep, vec_a, vec_w, st);
-    if (d.n > 128 && wg128x256 >= 256) return launch_mfma<DT, OutT, 128, 256, BK, 2, 4, 3, true>(d, ep, vec_a, vec_w, st);
+    if (wg256 >= 256 && d.bias_rows <= 1) return launch_mfma<DT, OutT, 256, 256, BK, 4, 2, 2, true>(d, ep, st);
+    if (d.n > 128 && wg128x256 >= 256) return launch_mfma<DT, OutT, 128, 256, BK, 2, 4, 3, true>(d, ep, st);
   }
-  // tall and narrow (the attention MLP over batch x history rows): one 96-wide tile reads A once
-  if (d.n > 64 && d.n <= 96 && (d.m + 127) / 128 >= 256)
-    return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, true>(d, ep, vec_a, vec_w, st);
-  if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, true>(d, ep, vec_a, vec_w, st);
-  if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, true>(d, ep, vec_a, vec_w, st);
-  if (wg64 >= 256) {
-    // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
-    // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
-    // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.
-    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true>(d, ep, vec_a, vec_w, st);
-  }
-  return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true>(d, ep, vec_a, vec_w, st);
+  return dispatch_mid<DT, OutT, true>(d, ep, st);
 }
 
 template <int DT, typename OutT>
-int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
+int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int nchunks = (d.k + In<DT>::kChunk - 1) / In<DT>::kChunk;
   int lpr = 1;
   while (lpr < nchunks && lpr < 64) lpr <<= 1;
@@ -965,7 +1100,7 @@ int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool ve
   int64_t grid = ((int64_t)d.m + rows_per_wg - 1) / rows_per_wg;
   if (grid > 256 * 32) grid = 256 * 32;
   hipLaunchKernelGGL((bz_fc_skinny_kernel<DT, OutT>), dim3((int)grid), dim3(256), 0, st, (const char*)d.a,
-                     (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_a, vec_w, lpr, ep);
+                     (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
   BZ_LAUNCH_OK("bz_fc_skinny_kernel");
   return BZ_OK;
 }
@@ -975,12 +1110,12 @@ int dispatch_out(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w
   const bool skinny = d.n <= kSkinnyMaxN;
   switch (d.out_dtype) {
     case BZ_F32:
-      return skinny ? dispatch_skinny<DT, float>(d, ep, vec_a, vec_w, st) : dispatch_tiles<DT, float>(d, ep, vec_a, vec_w, st);
+      return skinny ? dispatch_skinny<DT, float>(d, ep, st) : dispatch_tiles<DT, float>(d, ep, vec_a, vec_w, st);
     case BZ_F16:
-      return skinny ? dispatch_skinny<DT, __half>(d, ep, vec_a, vec_w, st)
+      return skinny ? dispatch_skinny<DT, __half>(d, ep, st)
                     : dispatch_tiles<DT, __half>(d, ep, vec_a, vec_w, st);
     case BZ_BF16:
-      return skinny ? dispatch_skinny<DT, __hip_bfloat16>(d, ep, vec_a, vec_w, st)
+      return skinny ? dispatch_skinny<DT, __hip_bfloat16>(d, ep, st)
                     : dispatch_tiles<DT, __hip_bfloat16>(d, ep, vec_a, vec_w, st);
     default:
       return bz::fail(BZ_EINVAL, "bz_fc_fused: unsupported out dtype %d", d.out_dtype);
