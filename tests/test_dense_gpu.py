@@ -148,7 +148,7 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + N * 3 + K)
 
 
-# Few 32x32 tiles (512 of fp32, 256 of 2-byte operands) go to the kernel whose eight waves share K in units of 128 bytes;
+# Up to 512 32x32 tiles go to the kernel whose eight waves share K in units of 128 bytes;
 # rows that start on no 16 bytes, beyond that, to the staged tiles with loads at any element.
 @pytest.mark.parametrize("in_name,out_name", [("f32", "f32"), ("f16", "f16"), ("bf16", "f32")])
 @pytest.mark.parametrize("M,N,K,act,kw", [
@@ -156,8 +156,7 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     (32, 32, 64, "relu", {}), (65, 33, 65, "dice", {}),                          # whole units and one element
     (7, 100, 2075, "sigmoid", {}), (96, 70, 1023, "prelu", {"full_bias": True}),  # units a wave, ragged; a bias a row
     (40, 24, 513, "none", {"alpha": 0.5, "beta": 2.0}),
-    (512, 512, 96, "prelu", {}), (513, 512, 96, "prelu", {}),                     # the last size of 256 tiles, the first beyond
-    (1024, 512, 77, "dice", {}), (1025, 512, 77, "dice", {}),                     # 512
+    (1024, 512, 77, "dice", {}), (1025, 512, 77, "dice", {}),                     # 512 tiles, and one row of tiles more
     (3000, 200, 5, "relu", {}), (2100, 300, 9, "none", {"full_bias": True}),      # staged: K about a chunk
     (4100, 1000, 73, "prelu", {}), (8200, 1000, 201, "dice", {}), (33000, 80, 215, "dice", {}),  # 64x128, 128x128, 128x96
 ])
@@ -191,6 +190,10 @@ def test_fc_streaming_kernel(bz, oracle, in_name, M, N, K, act, kw):
     (17000, 80, 40, 1, "dice", "none"),        # the same with enough rows for the 64x64 tile
     (513, 128, 128, 8, "relu", "sigmoid"),     # widest head
     (100, 64, 16, 3, "none", "softmax"),
+    (4096, 96, 256, 2, "relu", "sigmoid"),     # fp32: the last size of sixteen rows a workgroup, and the first beyond
+    (4097, 96, 256, 2, "relu", "sigmoid"),
+    (17, 8, 224, 5, "none", "none"),           # a part of one unit of K, seven column blocks on sixteen waves, a single row left
+    (1, 1104, 72, 1, "prelu", "sigmoid"),      # units shared by five parts, K ending inside one
 ])
 def test_fc_with_skinny_head_in_one_launch(bz, oracle, in_name, M, K, N, N2, act, hact):
     """Layer + skinny head in one launch against the same two layers as two launches.  The one-launch form uses a tile

@@ -14,6 +14,7 @@ namespace fc {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr float kDiceEps = 1e-8f;  // blaze/operator/common_helper.h:90
 
@@ -151,6 +152,10 @@ struct In<BZ_F16> {
   static __device__ __forceinline__ void mma(const uint4& a, const uint4& b, floatx16& acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const half8*)&a, *(const half8*)&b, acc, 0, 0, 0);
   }
+  // 16x16 block, K of 64 bytes: lane l holds row l % 16, bytes 16 * (l / 16) ..; result: column l % 16, rows 4 * (l / 16) ..
+  static __device__ __forceinline__ void mma16(const uint4& a, const uint4& b, floatx4& acc) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(*(const half8*)&a, *(const half8*)&b, acc, 0, 0, 0);
+  }
 };
 template <>
 struct In<BZ_BF16> {
@@ -159,6 +164,9 @@ struct In<BZ_BF16> {
   static constexpr int kStepK = 16;
   static __device__ __forceinline__ void mma(const uint4& a, const uint4& b, floatx16& acc) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)&a, *(const bf16x8*)&b, acc, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void mma16(const uint4& a, const uint4& b, floatx4& acc) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)&a, *(const bf16x8*)&b, acc, 0, 0, 0);
   }
 };
 template <>
@@ -173,6 +181,13 @@ struct In<BZ_F32> {
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
+  }
+  // (instruction i multiplies element i of the four lane groups: again one permutation of k for both operands)
+  static __device__ __forceinline__ void mma16(const uint4& a, const uint4& b, floatx4& acc) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
   }
 };
 

@@ -142,6 +142,47 @@ struct HeadArgs {
   int n, act, out_dtype;
 };
 
+// the head's outputs of row m from its dot products: bias, activation, store
+__device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const float (&dot)[kSkinnyMaxN]) {
+  float v[kSkinnyMaxN];
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < head.n) ? dot[j] + (head.bias ? head.bias[j] : 0.f) : 0.f;
+  if (head.act == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
+    float mx = v[0];
+#pragma unroll
+    for (int j = 1; j < kSkinnyMaxN; ++j)
+      if (j < head.n) mx = v[j] > mx ? v[j] : mx;
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j)
+      if (j < head.n) {
+        v[j] = expf(v[j] - mx);
+        sum += v[j];
+      }
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j)
+      if (j < head.n) v[j] = v[j] / sum;
+  } else if (head.act == BZ_ACT_SIGMOID) {
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j) {
+      const float t = expf(v[j]);
+      v[j] = t / (1.f + t);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j) {
+    if (j < head.n) {
+      const int64_t at = (int64_t)m * head.ldy + j;
+      if (head.out_dtype == BZ_F32)
+        store_out<float>((float*)head.y + at, v[j]);
+      else if (head.out_dtype == BZ_F16)
+        store_out<__half>((__half*)head.y + at, v[j]);
+      else
+        store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // tiled MFMA kernel
 // ---------------------------------------------------------------------------------------------
@@ -491,45 +532,7 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
 #pragma unroll
       for (int j = 0; j < kSkinnyMaxN; ++j) hacc[j] += __shfl_xor(hacc[j], d, 64);
     }
-    if (hl == 0 && m < M) {
-      float v[kSkinnyMaxN];
-#pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < head.n) ? hacc[j] + (head.bias ? head.bias[j] : 0.f) : 0.f;
-      if (head.act == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
-        float mx = v[0];
-#pragma unroll
-        for (int j = 1; j < kSkinnyMaxN; ++j)
-          if (j < head.n) mx = v[j] > mx ? v[j] : mx;
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < kSkinnyMaxN; ++j)
-          if (j < head.n) {
-            v[j] = expf(v[j] - mx);
-            sum += v[j];
-          }
-#pragma unroll
-        for (int j = 0; j < kSkinnyMaxN; ++j)
-          if (j < head.n) v[j] = v[j] / sum;
-      } else if (head.act == BZ_ACT_SIGMOID) {
-#pragma unroll
-        for (int j = 0; j < kSkinnyMaxN; ++j) {
-          const float t = expf(v[j]);
-          v[j] = t / (1.f + t);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) {
-        if (j < head.n) {
-          const int64_t at = (int64_t)m * head.ldy + j;
-          if (head.out_dtype == BZ_F32)
-            store_out<float>((float*)head.y + at, v[j]);
-          else if (head.out_dtype == BZ_F16)
-            store_out<__half>((__half*)head.y + at, v[j]);
-          else
-            store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
-        }
-      }
-    }
+    if (hl == 0 && m < M) head_finish(head, m, hacc);
   }
 }
 
@@ -766,90 +769,108 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 // split kernel: few tiles, or rows that start on no 16 bytes
 // ---------------------------------------------------------------------------------------------
 // A workgroup owns a 32 x 32 tile of C and its eight waves share the K range: unit u (128 bytes of every row) is
-// wave u % 8's.  A wave loads its units straight into MFMA fragments, the next unit's loads in flight while the present
-// one is multiplied; nothing goes through LDS and no wave waits for another before the partial tiles are added up.
+// wave u % 8's.  A wave works for itself: it loads a unit with eight lanes on a row, turns it in LDS of its own into MFMA
+// fragments, the next unit's loads in flight meanwhile, and meets the others only when the partial tiles are added up.
 //  - Few tiles leave the chip idle and the chain of K tiles sets the time: eight waves walk it in an eighth of the steps.
 //  - A lane's 16 bytes may start anywhere (a row pitch of 445 fp16 elements): the memory system takes such loads, and
 //    the lines they share are L1 hits.
-// It is bound by the path into a CU (a load instruction touches 32 lines for 1 KB), which is why it stops at few tiles, why
-// the compiler's choice to keep few loads in flight and many waves resident is left alone (all of two units' loads pinned
-// ahead of the multiplications: 5 to 30 % slower), and why wider tiles a workgroup
-// (64 x 64: 32 x 2075 -> 768 fp32 47 us against 17) do not pay.
-constexpr int kSplitWaves = 8, kSplitUnit = 128;
+// Loaded straight into fragments a group of 16 lanes touches 16 lines, and the path into the CU takes a line a clock:
+// 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile); 32 x 2075 -> 768 fp32 17.0, 14.4 (51.7).
+constexpr int kSplitWaves = 8, kSplitUnit = 128, kSplitPitch = kSplitUnit + 16;
+
+// One wave's 8 * P rows of an operand, a unit of K at a time: global memory -> registers (lane: row l / 8 of each pass,
+// chunk l % 8) -> LDS rows kSplitPitch apart.
+template <int DT, int P>
+struct SplitRows {
+  static constexpr int ES = In<DT>::kSize, CH = In<DT>::kChunk;
+  const char* p[P];
+  uint4 r[P];
+  __device__ __forceinline__ void init(const char* base, int64_t ld, int row0, int rows, int lane) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) p[i] = base + (int64_t)min(row0 + i * 8 + (lane >> 3), rows - 1) * ld * ES;
+  }
+  // a whole unit
+  __device__ __forceinline__ void load(int u, int lane) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) __builtin_memcpy(&r[i], p[i] + (int64_t)u * kSplitUnit + (lane & 7) * 16, 16);
+  }
+  // the unit that K ends in: zeros beyond K
+  __device__ __forceinline__ void load_last(int u, int K, int lane) {
+    const int k = u * (kSplitUnit / ES) + (lane & 7) * CH;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      if (K >= CH)
+        r[i] = shift_chunk<DT>(load_chunk_anywhere<DT>(p[i], 0, 0, k, K), k - min(k, K - CH));
+      else
+        r[i] = load_chunk<DT>(p[i], 0, 0, k, K);
+    }
+  }
+  __device__ __forceinline__ void store(char* lds, int lane) const {
+#pragma unroll
+    for (int i = 0; i < P; ++i) *(uint4*)(lds + (i * 8 + (lane >> 3)) * kSplitPitch + (lane & 7) * 16) = r[i];
+  }
+};
 
 template <int DT, typename OutT>
-__global__ __launch_bounds__(kSplitWaves * 64, 2) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
+__global__ __launch_bounds__(kSplitWaves * 64, 4) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                           OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                           int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
   using T = In<DT>;
-  constexpr int ES = T::kSize, NW = kSplitWaves, STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
+  constexpr int NW = kSplitWaves, STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
   constexpr int PITCH = 33;
-  __shared__ float red[NW / 2][32 * PITCH];
+  __shared__ __attribute__((aligned(16))) char lds[NW][64 * kSplitPitch];
+  static_assert(32 * PITCH * 4 <= 64 * kSplitPitch, "a partial tile fits where its wave's operands were");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = (int)(blockIdx.x % tiles_m) * 32, n0 = (int)(blockIdx.x / tiles_m) * 32;
   const int frow = lane & 31, fhalf = lane >> 5;
-  const int am = min(m0 + frow, M - 1), wn = min(n0 + frow, N - 1);
-  const char* pa = A + (int64_t)am * lda * ES + fhalf * 16;
-  const char* pw = W + (int64_t)wn * ldw * ES + fhalf * 16;
+  char* la = lds[wave];
+  char* lw = la + 32 * kSplitPitch;
+  SplitRows<DT, 4> ra, rw;
+  ra.init(A, lda, m0, M, lane);
+  rw.init(W, ldw, n0, N, lane);
   floatx16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-
-  struct Unit {
-    uint4 a[STEPS], w[STEPS];
-  };
-  auto mma = [&](const Unit& x) {
-#pragma unroll
-    for (int ks = 0; ks < STEPS; ++ks) T::mma(x.a[ks], x.w[ks], acc);
-  };
-  const int whole = (int)((int64_t)K * ES / kSplitUnit);
-  // (no branch round the loads of a unit that does not exist: the last whole one is read again)
-  auto load = [&](Unit& x, int u) {
-    const int64_t off = (int64_t)min(u, whole - 1) * kSplitUnit;
-#pragma unroll
-    for (int ks = 0; ks < STEPS; ++ks) {
-      __builtin_memcpy(&x.a[ks], pa + off + ks * 32, 16);
-      __builtin_memcpy(&x.w[ks], pw + off + ks * 32, 16);
+  const int whole = (int)((int64_t)K * T::kSize / kSplitUnit), units = (int)(((int64_t)K * T::kSize + kSplitUnit - 1) / kSplitUnit);
+  auto load = [&](int u) {
+    if (u < whole) {
+      ra.load(u, lane);
+      rw.load(u, lane);
+    } else if (u < units) {
+      ra.load_last(u, K, lane);
+      rw.load_last(u, K, lane);
     }
   };
-  if (wave < whole) {
-    Unit x, y;
-    load(x, wave);
-    for (int u = wave; u < whole; u += 2 * NW) {
-      load(y, u + NW);
-      mma(x);
-      if (u + NW >= whole) break;
-      load(x, u + 2 * NW);
-      mma(y);
-    }
-  }
-  if ((int64_t)whole * kSplitUnit < (int64_t)K * ES && wave == whole % NW) {
-    const int k0 = whole * (kSplitUnit / ES);
+  load(wave);
+  for (int u = wave; u < units; u += NW) {
+    // (a wave's own LDS operations keep their order: nobody to wait for)
+    ra.store(la, lane);
+    rw.store(lw, lane);
+    __builtin_amdgcn_wave_barrier();
+    load(u + NW);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < STEPS; ++ks)
-      if (k0 + ks * T::kStepK < K) {
-        const int k = k0 + ks * T::kStepK + fhalf * T::kChunk;
-        if (K >= T::kChunk) {
-          const int drop = k - min(k, K - T::kChunk);
-          T::mma(shift_chunk<DT>(load_chunk_anywhere<DT>(A, am, lda, k, K), drop),
-                 shift_chunk<DT>(load_chunk_anywhere<DT>(W, wn, ldw, k, K), drop), acc);
-        } else {
-          T::mma(load_chunk<DT>(A, am, lda, k, K), load_chunk<DT>(W, wn, ldw, k, K), acc);
-        }
-      }
+      T::mma(*(const uint4*)(la + frow * kSplitPitch + fhalf * 16 + ks * 32),
+             *(const uint4*)(lw + frow * kSplitPitch + fhalf * 16 + ks * 32), acc);
+    __builtin_amdgcn_wave_barrier();
   }
-  // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper four waves hand theirs to the
-  // lower four, which add their own at the same places
-  float* mine = red[wave % (NW / 2)] + 4 * fhalf * PITCH + frow;
+  // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper four waves leave theirs where
+  // their operands were, the lower four add their own
+  float* mine = (float*)lds[wave] + 4 * fhalf * PITCH + frow;
   if (wave >= NW / 2) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) mine[(8 * (r >> 2) + (r & 3)) * PITCH] = acc[r];
   }
   __syncthreads();
   if (wave < NW / 2) {
+    const float* other = (const float*)lds[wave + NW / 2] + 4 * fhalf * PITCH + frow;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mine[(8 * (r >> 2) + (r & 3)) * PITCH] += acc[r];
+    for (int r = 0; r < 16; ++r) {
+      const int at = (8 * (r >> 2) + (r & 3)) * PITCH;
+      mine[at] = acc[r] + other[at];
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -858,12 +879,131 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void bz_fc_split_kernel(const 
     const int m = m0 + ml, n = n0 + nl;
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW / 2; ++w) v += red[w][ml * PITCH + nl];
+    for (int w = 0; w < NW / 2; ++w) v += ((const float*)lds[w])[ml * PITCH + nl];
     if (m < M && n < N) {
       const float b = ep.bias_rows == 0 ? 0.f : ep.bias[ep.bias_rows == 1 ? n : full_bias_index(ep, m, n, M, N)];
       store_out<OutT>(Y + out_index(ep, m, n, ldy), apply_act(fmaf(ep.alpha, v, ep.beta * b), n, ep));
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// split kernel with the skinny head
+// ---------------------------------------------------------------------------------------------
+// A layer with a head keeps whole rows in one workgroup, so M sets how many CUs work: 16 rows a workgroup where the staged
+// tile takes 32, and sixteen waves that share its columns (32 each) and, for N below 256, K, each working for itself as in
+// the split kernel above.  After the partial blocks are added up, wave r
+// owns row r: its lanes hold the row's outputs in registers, and the head is a dot product within the wave.
+constexpr int kHeadWaves = 16;
+
+template <int DT, typename OutT>
+__global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const char* __restrict__ A, const char* __restrict__ W,
+                                                                           OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
+                                                                           int64_t ldw, int64_t ldy, Epilogue ep, HeadArgs head) {
+  using T = In<DT>;
+  static_assert(sizeof(OutT) == T::kSize, "the head reads the tile with the operand type");
+  constexpr int ES = T::kSize, STEPS = kSplitUnit / 64, COLS = 256 / 64;
+  constexpr int kHeadStage = 48 * kSplitPitch;
+  __shared__ __attribute__((aligned(16))) char lds[kHeadWaves * kHeadStage];
+  static_assert(16 * 33 * 4 <= kHeadStage, "the partial blocks fit");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.x * 16;
+  // the row's columns of this lane: their parameters and the head's weights, asked for first
+  float cb[COLS], q0[COLS], q1[COLS], q2[COLS];
+  OutT hw[kSkinnyMaxN][COLS];
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    const int n = min(lane + 64 * c, N - 1);
+    cb[c] = ep.bias_rows == 1 ? ep.bias[n] : 0.f;
+    q0[c] = q1[c] = q2[c] = 0.f;
+    if (ep.act == BZ_ACT_PRELU) q0[c] = ep.p0[ep.act_size == 1 ? 0 : n];
+    if (ep.act == BZ_ACT_DICE) {
+      q0[c] = ep.p0[n];
+      q1[c] = ep.p1[n];
+      q2[c] = ep.p2[n];
+    }
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j)
+      if (j < head.n) hw[j][c] = ((const OutT*)head.w)[j * head.ldw + n];
+  }
+  const int nb = (N + 31) / 32, parts = kHeadWaves / nb, pitch = nb * 32 + 1;
+  const int part = wave / nb, block = wave - part * nb;
+  const int frow = lane & 15, fq = lane >> 4;
+  floatx4 acc[2];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) acc[0][r] = acc[1][r] = 0.f;
+  if (part < parts) {
+    char* la = lds + wave * kHeadStage;
+    char* lw = la + 16 * kSplitPitch;
+    SplitRows<DT, 2> ra;
+    SplitRows<DT, 4> rw;
+    ra.init(A, lda, m0, M, lane);
+    rw.init(W, ldw, block * 32, N, lane);
+    const int64_t kbytes = (int64_t)K * ES;
+    const int whole = (int)(kbytes / kSplitUnit), units = (int)((kbytes + kSplitUnit - 1) / kSplitUnit);
+    auto load = [&](int u) {
+      if (u < whole) {
+        ra.load(u, lane);
+        rw.load(u, lane);
+      } else if (u < units) {
+        ra.load_last(u, K, lane);
+        rw.load_last(u, K, lane);
+      }
+    };
+    load(part);
+    for (int u = part; u < units; u += parts) {
+      ra.store(la, lane);
+      rw.store(lw, lane);
+      __builtin_amdgcn_wave_barrier();
+      load(u + parts);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        const uint4 a = *(const uint4*)(la + frow * kSplitPitch + s * 64 + fq * 16);
+        T::mma16(a, *(const uint4*)(lw + frow * kSplitPitch + s * 64 + fq * 16), acc[0]);
+        T::mma16(a, *(const uint4*)(lw + (16 + frow) * kSplitPitch + s * 64 + fq * 16), acc[1]);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  __syncthreads();  // the operands' LDS becomes the partial blocks'
+  float* red = (float*)lds;
+  if (part < parts) {
+    float* mine = red + (part * 16 + 4 * fq) * pitch + block * 32 + frow;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      mine[r * pitch] = acc[0][r];
+      mine[r * pitch + 16] = acc[1][r];
+    }
+  }
+  __syncthreads();
+  const int m = m0 + wave;
+  if (m >= M) return;
+  float dot[kSkinnyMaxN];
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j) dot[j] = 0.f;
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    const int n = lane + 64 * c;
+    if (n < N) {
+      float v = 0.f;
+      for (int p = 0; p < parts; ++p) v += red[(p * 16 + wave) * pitch + n];
+      OutT y;
+      store_out<OutT>(&y, apply_act_regs(fmaf(ep.alpha, v, ep.beta * cb[c]), ep, q0[c], q1[c], q2[c]));
+      if (Y != nullptr) Y[(int64_t)m * ldy + n] = y;
+#pragma unroll
+      for (int j = 0; j < kSkinnyMaxN; ++j)
+        if (j < head.n) dot[j] = fmaf((float)y, (float)hw[j][c], dot[j]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j)
+    if (j < head.n) {
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) dot[j] += __shfl_xor(dot[j], d, 64);
+    }
+  if (lane == 0) head_finish(head, m, dot);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -956,6 +1096,19 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
 }
 
 
+inline HeadArgs head_args(const bz_fc_desc& d) {
+  HeadArgs head;
+  head.w = (const char*)d.head_w;
+  head.bias = d.head_bias;
+  head.y = d.head_y;
+  head.ldw = d.head_ldw;
+  head.ldy = d.head_ldy;
+  head.n = d.head_n;
+  head.act = d.head_act;
+  head.out_dtype = d.head_out_dtype;
+  return head;
+}
+
 template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false>
 int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
@@ -964,17 +1117,7 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const bool vec_y = d.y != nullptr && ((uintptr_t)d.y % 16 == 0) && ((d.ldy * (int64_t)sizeof(OutT)) % 16 == 0) &&
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
-  HeadArgs head = {};
-  if (HEAD) {
-    head.w = (const char*)d.head_w;
-    head.bias = d.head_bias;
-    head.y = d.head_y;
-    head.ldw = d.head_ldw;
-    head.ldy = d.head_ldy;
-    head.n = d.head_n;
-    head.act = d.head_act;
-    head.out_dtype = d.head_out_dtype;
-  }
+  const HeadArgs head = HEAD ? head_args(d) : HeadArgs{};
   hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD>), dim3(tiles_m * tiles_n), dim3(WM * WN * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
@@ -1020,6 +1163,17 @@ int launch_stream(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 template <int DT, typename OutT>
 int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
+  // fp32 is bound by the matrix cores of the CUs that work: 16 rows a workgroup up to 4096 rows (2048 x 512 -> 256 19.2 us
+  // against 25.2, 4096 x 1024 -> 128 19.4 and 30.7, 201 x 200 -> 80 7.8 and 10.3; 8192 rows 35.7 and 26.4).  2-byte layers
+  // are not (2048 x 512 -> 256 fp16 10.2 and 9.0).
+  if constexpr (DT == BZ_F32) {
+    if (d.m <= 4096) {
+      hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
+                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d));
+      BZ_LAUNCH_OK("bz_fc_split_head_kernel");
+      return BZ_OK;
+    }
+  }
   if (d.n <= 64) {
     if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, true>(d, ep, st);
     return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true>(d, ep, st);
@@ -1058,12 +1212,11 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   // rows 16-byte aligned and K a whole number of chunks
   const bool aligned = vec_a && vec_w && d.k % In<DT>::kChunk == 0;
-  // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Up to 512 32x32 tiles of fp32
-  // (1024 x 896 -> 512: 17.6 us against the staged tile's 23.2; 2048 x 512 -> 256 10.9 and 15.1; 2048 x 896 -> 512, 1024
-  // tiles, 33 and 24) and 256 of 2-byte operands, which the path into a CU feeds at half the fp32 rate a multiplication
-  // (256 x 3000 -> 512: 10.5 and 17.4; 512 x 600 -> 512 6.4 and 7.1; 1024 x 1000 -> 512, 512 tiles, 10.5 and 8.5).
+  // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Up to 512 32x32 tiles
+  // (fp32 1024 x 896 -> 512 15.4 us against the staged tile's 23.2, fp16 1024 x 1000 -> 512 7.5 and 8.4; with 1024 tiles
+  // fp32 2048 x 896 -> 512 29 and 24, fp16 9.5 and 8.8).
   const int64_t wg32 = (int64_t)((d.m + 31) / 32) * ((d.n + 31) / 32);
-  if (d.k < In<DT>::kChunk || wg32 <= (In<DT>::kSize == 4 ? 512 : 256)) return launch_split<DT, OutT>(d, ep, st);
+  if (d.k < In<DT>::kChunk || wg32 <= 512) return launch_split<DT, OutT>(d, ep, st);
   if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
   // Largest first, and never a tile much wider than N.  128x256 with eight waves and three K tiles in flight fills the
   // chip once it has a workgroup per CU (its fp32 output tile would not fit the operand buffers it is staged in, so
