@@ -186,13 +186,14 @@ __device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const f
 // ---------------------------------------------------------------------------------------------
 // tiled MFMA kernel
 // ---------------------------------------------------------------------------------------------
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD>
-__global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
+// WK: groups of WM x WN waves that share each K tile between them and add up at the end
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD, int WK>
+__global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                   OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                   int64_t ldw, int64_t ldy, bool vec_y, int tiles_m, Epilogue ep,
                                                                   HeadArgs head) {
   using T = In<DT>;
-  constexpr int NT = WM * WN * 64;
+  constexpr int NT = WM * WN * WK * 64;
   constexpr int ES = T::kSize;
   constexpr int ROWB = BK * ES;        // bytes of one tile row
   constexpr int PITCH = ROWB + 16;     // padded LDS pitch
@@ -214,7 +215,8 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
+  const int wk = WK == 1 ? 0 : wave / (WM * WN), wmn = WK == 1 ? wave : wave % (WM * WN);
+  const int wm = wmn / WN, wn = wmn % WN;
   // consecutive workgroups walk down M within one N panel: the W panel stays hot in L2
   const int tile_m = blockIdx.x % tiles_m, tile_n = blockIdx.x / tiles_m;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
 
   // with a single 32x32 block per wave, back-to-back MFMAs into one accumulator would each wait for the
   // previous result; alternate K steps between two accumulators and add them at the end
-  constexpr int KACC = (TM * TN == 1 && BK / T::kStepK >= 2) ? 2 : 1;
+  constexpr int KACC = (TM * TN == 1 && BK / T::kStepK / WK >= 2) ? 2 : 1;
   floatx16 acc[KACC][TM][TN];
 #pragma unroll
   for (int a = 0; a < KACC; ++a)
@@ -339,13 +341,14 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
   // (not the 256x256 tile: with 128 accumulator registers a wave has no room for a second set of fragments; measured on
   // the other tiles: 128x256 245 -> 238 us on 8192x12800x1024, 64x64 9.6 -> 9.2 us on config 2's first layer)
   constexpr bool PIPE = !HEAD && BM * BN >= 64 * 64 && BM * BN < 256 * 256;
-  constexpr int KS = BK / T::kStepK;
+  constexpr int KS = BK / T::kStepK / WK;  // sub-steps of a K tile that are this wave's
+  static_assert(WK == 1 || PIPE, "K is shared in the pipelined loop");
   if constexpr (PIPE) {
     static_assert(KS % 2 == 0, "fragment double buffer needs an even number of sub-steps");
     uint4 fa[2][TM], fw[2][TN];
     auto fread = [&](int slot, int buf, int ks) {
-      const char* la = &lds[buf][(wm * WTM + frag_row) * PITCH + frag_half * 16];
-      const char* lw = &lds[buf][(BM + wn * WTN + frag_row) * PITCH + frag_half * 16];
+      const char* la = &lds[buf][(wm * WTM + frag_row) * PITCH + frag_half * 16 + wk * (KS * 32)];
+      const char* lw = &lds[buf][(BM + wn * WTN + frag_row) * PITCH + frag_half * 16 + wk * (KS * 32)];
 #pragma unroll
       for (int i = 0; i < TM; ++i) fa[slot][i] = *(const uint4*)(la + i * 32 * PITCH + ks * 32);
 #pragma unroll
@@ -412,6 +415,28 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[0][i][j][r] += acc[KACC - 1][i][j][r];
   }
+  // the other groups' partial tiles, through LDS behind the output tile's place: group 0 goes on with the sum
+  if constexpr (WK > 1) {
+    static_assert(WK == 2 && !HEAD && BM * (BN * (int)sizeof(OutT) + 16) + BM * (BN + 1) * 4 <= (int)sizeof(lds), "room for the partial tile");
+    float* part = (float*)(&lds[0][0] + BM * (BN * (int)sizeof(OutT) + 16)) + (wm * WTM + 4 * frag_half) * (BN + 1) + wn * WTN + frag_row;
+    if (wk == 1) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) part[(i * 32 + 8 * (r >> 2) + (r & 3)) * (BN + 1) + j * 32] = acc[0][i][j][r];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[0][i][j][r] += part[(i * 32 + 8 * (r >> 2) + (r & 3)) * (BN + 1) + j * 32];
+    }
+  }
   // epilogue: lane owns column n, rows 8*(r/4) + 4*(lane/32) + r%4 of each 32x32 block.  The activated tile
   // goes through LDS (free after the K loop) so that global stores are 16 bytes per lane along rows.
   constexpr int OS = (int)sizeof(OutT);
@@ -464,7 +489,9 @@ __global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __r
       }
     }
   };
-  switch (ep.act) {
+  switch (WK > 1 && wk != 0 ? -1 : ep.act) {
+    case -1:
+      break;
     case BZ_ACT_PRELU:
       epilogue(std::integral_constant<int, BZ_ACT_PRELU>());
       break;
@@ -915,6 +942,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const int n = min(lane + 64 * c, N - 1);
+    const OutT* w2 = (const OutT*)head.w + n;
     cb[c] = ep.bias_rows == 1 ? ep.bias[n] : 0.f;
     q0[c] = q1[c] = q2[c] = 0.f;
     if (ep.act == BZ_ACT_PRELU) q0[c] = ep.p0[ep.act_size == 1 ? 0 : n];
@@ -925,7 +953,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
     }
 #pragma unroll
     for (int j = 0; j < kSkinnyMaxN; ++j)
-      if (j < head.n) hw[j][c] = ((const OutT*)head.w)[j * head.ldw + n];
+      if (j < head.n) hw[j][c] = w2[j * head.ldw];
   }
   const int nb = (N + 31) / 32, parts = kHeadWaves / nb, pitch = nb * 32 + 1;
   const int part = wave / nb, block = wave - part * nb;
@@ -1109,7 +1137,7 @@ inline HeadArgs head_args(const bz_fc_desc& d) {
   return head;
 }
 
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false>
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false, int WK = 1>
 int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
   // output rows 16-byte aligned and N a whole number of 16-byte chunks: coalesced stores through LDS
@@ -1118,7 +1146,7 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
   const HeadArgs head = HEAD ? head_args(d) : HeadArgs{};
-  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD>), dim3(tiles_m * tiles_n), dim3(WM * WN * 64), 0,
+  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
   return BZ_OK;
@@ -1198,10 +1226,17 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
     return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, ALIGNED>(d, ep, st);
   if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
   if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  // fp32: eight waves, two to a SIMD, that share each K tile.  Its MFMAs are long, and with one wave a SIMD nothing runs
+  // while that wave reads fragments or waits at the barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way (at 8192 rows the
+  // matrix cores set the time, 64 us, either way).
+  if constexpr (DT == BZ_F32) {
+    if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
+  }
   if (wg64 >= 256) {
     // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
     // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
-    // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.
+    // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
+    // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
     return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
   }
   return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
