@@ -1225,8 +1225,17 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   // tall and narrow (the attention MLP over batch x history rows): one 96-wide tile reads A once
   if (d.n > 64 && d.n <= 96 && (d.m + 127) / 128 >= 256)
     return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, ALIGNED>(d, ep, st);
-  if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
-  if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  // 2-byte operands: eight waves on a 128- or 64-row tile of 128 columns with two K tiles in flight, once they give half
+  // the CUs a workgroup of the former or all of them one of the latter (fp16, against four waves on 64x128 or 64x64:
+  // 8192 x 1024 -> 512 17.2 us and 20.2, 4096 x 896 -> 1024 13.4 and 17.9, 3000 x 1024 -> 768, 144 tiles, 12.9 and 17.2;
+  // 4096 x 2048 -> 512, 128 tiles, 22.8 and 20.7, on 64 rows 17.9)
+  if constexpr (In<DT>::kSize == 2) {
+    if (d.n > 64 && wg128 >= 140) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
+    if (d.n > 64 && wg64x128 >= 256) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
+  } else {
+    if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
+    if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  }
   // fp32: eight waves, two to a SIMD, that share each K tile.  Its MFMAs are long, and with one wave a SIMD nothing runs
   // while that wave reads fragments or waits at the barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way (at 8192 rows the
   // matrix cores set the time, 64 us, either way).
