@@ -294,7 +294,7 @@ int launch_bgemm(const bz_bgemm_desc& d, hipStream_t s) {
 }
 
 // One wave per batch item, lanes over the channels.  Both sums walk t in ascending order, the weighted one with the
-// fused multiply-add bz_bgemm_kernel uses for C = A^T * B, the plain one with separate adds like bz_reduce_sum_kernel,
+// fused multiply-add bz_bgemm_row_kernel uses for C = A^T * B, the plain one with separate adds like bz_reduce_sum_kernel,
 // and the weight is rounded to the tensor type first, as the Mul operator would have stored it: the results are the
 // three operators' results bit for bit.
 // (a history of 50 in one round of loads: with one wave per item and four waves per CU the kernel is a chain of
