@@ -104,6 +104,7 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
     LOG_ERROR("The idx=%zu exceed size=%zu", idx, external_input_blob_.size());
     return false;
   }
+  output_ahead_.assign(output_ahead_.size(), false);  // (an input may itself be an output)
   Blob* blob = external_input_blob_[idx];
   const size_t need = blob->size() * DataTypeSize(blob->data_type());
   if (len != need) {
@@ -162,6 +163,7 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
 constexpr size_t kFeedPart = 1 << 20;
 
 bool Predictor::FeedMany(int count, const char* const* names, const void* const* data, const size_t* lens) {
+  output_ahead_.assign(output_ahead_.size(), false);
   try {
     struct Item {
       int idx;
