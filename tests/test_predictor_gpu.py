@@ -842,3 +842,45 @@ def test_store_get_with_host_pointers(pb, oracle, out_dtype, with_keys):
     ids, seg, vals = case(20, 5)
     with pytest.raises(pb.BlazeError):
         pm.store_get("t", ids, seg, vals, dim, [(oracle.SUM, 0, 0, np.zeros((20, 4), np.float32), 0)])  # stride < dim
+
+
+def _in_place_net(pb):
+    """x -> Sigmoid -> x: the input is the output"""
+    nb = pb.NetBuilder("in_place", device_type=1)
+    nb.external_input("x", 1)
+    nb.op("Sigmoid", ["x"], ["x"])
+    nb.external_output("x", 1)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    return pm
+
+
+def _sigmoid(x):
+    return 1.0 / (1.0 + np.exp(-x.astype(np.float64)))
+
+
+def test_output_after_an_in_place_input_was_reshaped(pb):
+    """Forward copies an output that was read before ahead of the next Output; an input that is that output may be
+    reshaped in between, and Output then answers for the new shape: the tensor's own memory, not the copy of the old
+    size.  A shape beyond the fed slice is refused, as Forward refuses it."""
+    rng = np.random.default_rng(3)
+    pm = _in_place_net(pb)
+    p = pm.create_predictor(1, 0)
+    big, small = rng.standard_normal((8, 32)).astype(np.float32), rng.standard_normal((2, 32)).astype(np.float32)
+    p.feed("x", big)
+    p.forward()
+    np.testing.assert_allclose(p.output_asnumpy("x"), _sigmoid(big), rtol=1e-5)
+    want = _sigmoid(big)
+    for step in range(3):  # from the second pass on the output has been copied ahead
+        p.feed("x", small + step)
+        p.forward()
+        if step < 2:
+            np.testing.assert_allclose(p.output_asnumpy("x"), _sigmoid(small + step), rtol=1e-5)
+    want[:2] = _sigmoid(small + 2)
+    p.reshape_input("x", big.shape)
+    np.testing.assert_allclose(p.output_asnumpy("x"), want, rtol=1e-5)  # the last small pass, behind it what the large one left
+    p.feed_many(p.feed_batch([("x", big)]))
+    p.forward()
+    p.reshape_input("x", (1000, 1000))
+    with pytest.raises(pb.BlazeError, match="Output x failed"):
+        p.output_asnumpy("x")

@@ -68,6 +68,7 @@ bool Predictor::ReshapeInput(size_t idx, const std::vector<size_t>& shape) {
     LOG_ERROR("The idx=%zu exceed size=%zu", idx, external_input_blob_.size());
     return false;
   }
+  output_ahead_.assign(output_ahead_.size(), false);  // (an input may itself be an output, of another size from here on)
   try {
     external_input_blob_[idx]->Reshape(shape);
   } catch (std::exception& e) {
@@ -425,6 +426,10 @@ bool Predictor::Output(size_t idx, void** data, size_t* len) {
     return false;
   }
   Blob* blob = external_output_blob_[idx];
+  if (blob->unplaced()) {
+    LOG_ERROR("output %s is an input that was reshaped beyond its fed size and has not been fed since", net_->external_output()[idx].c_str());
+    return false;
+  }
   const size_t bytes = blob->size() * DataTypeSize(blob->data_type());
   try {
     if (blob->device_type() == kCPU) {
