@@ -884,3 +884,55 @@ def test_output_after_an_in_place_input_was_reshaped(pb):
     p.reshape_input("x", (1000, 1000))
     with pytest.raises(pb.BlazeError, match="Output x failed"):
         p.output_asnumpy("x")
+
+
+class _DeviceArray:
+    def __init__(self, ptr, shape):
+        self.__cuda_array_interface__ = dict(shape=shape, typestr="<f4", data=(ptr, False), version=3, strides=None)
+
+
+@pytest.mark.parametrize("through", ["output", "in-place input", "input under a Reshape"])
+@pytest.mark.parametrize("when", ["before the first pass", "after a copy ahead"])
+def test_output_sees_what_was_written_through_a_device_address(pb, through, when):
+    """Output returns the tensor as it is when Output is called, also where the caller changed it in place after Forward
+    through an address from output_device_ptr or input_device_ptr -- on every pass, whether the address was taken
+    before the first pass or after Forward had already copied an output ahead."""
+    import torch
+    nb = pb.NetBuilder("addr", device_type=1)
+    nb.external_input("x", 1)
+    if through == "in-place input":
+        nb.op("Sigmoid", ["x"], ["x"])
+        out = "x"
+    elif through == "input under a Reshape":
+        nb.constant("shape", np.array([16, 4], np.int32))
+        nb.op("Reshape", ["x", "shape"], ["y"])
+        out = "y"
+    else:
+        nb.op("Sigmoid", ["x"], ["y"])
+        out = "y"
+    nb.external_output(out, 1)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    x = np.random.default_rng(4).standard_normal((4, 16)).astype(np.float32)
+
+    def address():
+        return p.output_device_ptr(out) if through == "output" else p.input_device_ptr("x")
+
+    p.feed("x", x)
+    p.forward()
+    if when == "after a copy ahead":
+        for _ in range(2):
+            p.output_asnumpy(out)
+            p.forward()
+    for step in range(4):
+        view = torch.as_tensor(_DeviceArray(address(), x.shape), device="cuda")
+        view.fill_(float(step))
+        torch.cuda.synchronize()
+        got = p.output_asnumpy(out)
+        assert got.size == x.size and (got == step).all(), (step, got.reshape(-1)[:4])
+        p.forward()
+        if through == "output":
+            np.testing.assert_allclose(p.output_asnumpy(out), _sigmoid(x), rtol=1e-5)
+        elif through == "in-place input":
+            np.testing.assert_allclose(p.output_asnumpy(out), _sigmoid(np.full_like(x, step)), rtol=1e-5)

@@ -380,10 +380,27 @@ bool Predictor::Forward(const PredictorCallback&& cb) {
   }
 }
 
+namespace {
+// whether two blobs share memory (an output may be an input, or a Reshape's view of one)
+bool Overlap(Blob* a, Blob* b) {
+  auto range = [](Blob* x, uintptr_t* from, uintptr_t* to) {
+    const size_t es = DataTypeSize(x->data_type());
+    *from = (uintptr_t)x->data();
+    *to = *from + x->size() * es;
+    if (x->pitch() != 0 && x->size() > 0) *to = *from + ((x->shape()[0] - 1) * x->pitch() + x->shape()[1]) * es;
+  };
+  uintptr_t a0, a1, b0, b1;
+  range(a, &a0, &a1);
+  range(b, &b0, &b1);
+  return a0 < b1 && b0 < a1;
+}
+}  // namespace
+
 // Outputs that were read after the last Forward are copied to the host behind this one, under the same wait: a copy asked
 // for by Output alone is another launch and another wait, 16 us of a 58 us request.  Small ones only, by a kernel that
 // writes the pinned copy over the link (the copy engine's hand-over would cost more than it moves); larger ones are
-// copied by Output.  Into a second buffer: the one Output handed out stays as it is until the next Output.
+// copied by Output.  Into a second buffer: the one Output handed out stays as it is until the next Output.  Not where the
+// caller holds the device address of that memory: what it writes there after the pass is the output, too.
 void Predictor::QueueOutputs() {
   constexpr size_t kMax = 64 << 10;
   hipStream_t st = (hipStream_t)net_->WaitedStream();
@@ -396,6 +413,7 @@ void Predictor::QueueOutputs() {
     const size_t bytes = blob->size() * DataTypeSize(blob->data_type());
     if (!wanted || st == nullptr || blob->device_type() != kHIP || blob->pitch() != 0 || blob->data() == nullptr || bytes == 0 || bytes > kMax)
       continue;
+    if (std::any_of(handed_out_.begin(), handed_out_.end(), [&](Blob* b) { return Overlap(b, blob); })) continue;
     Blob* next = output_next_[i].get();
     next->set_data_type((DataType)blob->data_type());
     next->Reshape(blob->shape());
@@ -533,11 +551,16 @@ void* Predictor::InputDevicePtr(const char* name) {
     blob->Reshape(shape);
   }
   // (a strided input -- one that lives inside a Concat's output -- has no plain buffer to hand out)
-  return idx < 0 || external_input_blob_[idx]->pitch() != 0 ? nullptr : external_input_blob_[idx]->data();
+  return idx < 0 || external_input_blob_[idx]->pitch() != 0 ? nullptr : HandOut(external_input_blob_[idx]);
 }
 void* Predictor::OutputDevicePtr(const char* name) {
   const int idx = OutputName2Idx(name);
-  return idx < 0 ? nullptr : external_output_blob_[idx]->data();
+  return idx < 0 ? nullptr : HandOut(external_output_blob_[idx]);
+}
+void* Predictor::HandOut(Blob* blob) {
+  output_ahead_.assign(output_ahead_.size(), false);
+  if (std::find(handed_out_.begin(), handed_out_.end(), blob) == handed_out_.end()) handed_out_.push_back(blob);
+  return blob->data();
 }
 
 std::string& last_error_for_thread() {

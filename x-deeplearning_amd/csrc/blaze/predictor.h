@@ -88,6 +88,8 @@ class Predictor {
   std::vector<std::shared_ptr<Blob>> output_next_;  // what Forward copied ahead of Output (QueueOutputs)
   std::vector<bool> output_wanted_;                 // read since the last Forward
   std::vector<bool> output_ahead_;                  // output_next_ holds the last Forward's result
+  std::vector<Blob*> handed_out_;                   // whose device address the caller has
+  void* HandOut(Blob* blob);
   void QueueOutputs();
   // pinned staging of fed inputs: Feed copies the caller's bytes here and queues the transfer on the thread's
   // stream; Forward runs behind it on the same stream.  feed_pending_[i]: input i's staging is still being read.
