@@ -936,3 +936,46 @@ def test_output_sees_what_was_written_through_a_device_address(pb, through, when
             np.testing.assert_allclose(p.output_asnumpy(out), _sigmoid(x), rtol=1e-5)
         elif through == "in-place input":
             np.testing.assert_allclose(p.output_asnumpy(out), _sigmoid(np.full_like(x, step)), rtol=1e-5)
+
+
+def test_outputs_copied_ahead_of_output(pb):
+    """Ten outputs (one launch copies eight ahead) at batches whose outputs are below and above what is copied ahead
+    (64 KB): read once, twice or not at all after a pass, in either order, after growing and shrinking.  Every read is the
+    pass's own result, and from the second pass of a shape on neither Forward nor Output allocates."""
+    rng = np.random.default_rng(6)
+    nb = pb.NetBuilder("many", device_type=1)
+    nb.external_input("x", 1)
+    cs = [np.float32(0.5 * k - 2.0) for k in range(10)]
+    for k, c in enumerate(cs):
+        nb.constant("c%d" % k, np.full((1, 8), c, np.float32))
+        nb.op("Add", ["x", "c%d" % k], ["y%d" % k])
+        nb.external_output("y%d" % k, 1)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for batch in (3, 2048, 2049, 1, 700):  # 2048 rows of 32 bytes are 64 KB
+        for step, reads in enumerate(((0, 1, 2), range(10), range(9, -1, -1), (9, 9, 8), (), tuple(range(10)) * 2, (4, 4, 4))):
+            x = rng.standard_normal((batch, 8)).astype(np.float32)
+            p.feed("x", x)
+            if step == 2:
+                before = pb.allocation_count()  # every output of this shape has been read once
+            p.forward()
+            for k in reads:
+                np.testing.assert_array_equal(p.output_asnumpy("y%d" % k), x + cs[k], err_msg="batch %d step %d output %d" % (batch, step, k))
+        assert pb.allocation_count() == before
+
+
+def test_the_pass_after_the_first_output_allocates_nothing(pb):
+    """The buffer that Forward copies an output into is made by Output, not between a launch and its wait."""
+    pm = _in_place_net(pb)
+    p = pm.create_predictor(1, 0)
+    x = np.random.default_rng(8).standard_normal((5, 7)).astype(np.float32)
+    p.feed("x", x)
+    p.forward()
+    np.testing.assert_allclose(p.output_asnumpy("x"), _sigmoid(x), rtol=1e-5)
+    before = pb.allocation_count()
+    for _ in range(3):
+        p.feed("x", x)
+        p.forward()
+        np.testing.assert_allclose(p.output_asnumpy("x"), _sigmoid(x), rtol=1e-5)
+    assert pb.allocation_count() == before

@@ -374,6 +374,7 @@ bool Predictor::Forward(const PredictorCallback&& cb) {
     if (cb) cb();
     return true;
   } catch (std::exception& e) {
+    output_ahead_.assign(output_ahead_.size(), false);
     LOG_ERROR("failed: %s", e.what());
     last_error_for_thread() = e.what();
     return false;
@@ -400,34 +401,36 @@ bool Overlap(Blob* a, Blob* b) {
 // for by Output alone is another launch and another wait, 16 us of a 58 us request.  Small ones only, by a kernel that
 // writes the pinned copy over the link (the copy engine's hand-over would cost more than it moves); larger ones are
 // copied by Output.  Into a second buffer: the one Output handed out stays as it is until the next Output.  Not where the
-// caller holds the device address of that memory: what it writes there after the pass is the output, too.
+// caller holds the device address of that memory: what it writes there after the pass is the output, too.  Output makes
+// the second buffer as large as the one it fills (allocating between a launch and its wait would hold the pass up), so an
+// output that has grown since is copied by Output once more.
+constexpr size_t kCopiedAheadMax = 64 << 10;
+
 void Predictor::QueueOutputs() {
-  constexpr size_t kMax = 64 << 10;
   hipStream_t st = (hipStream_t)net_->WaitedStream();
   bz_feed_rows rows[BZ_FEED_MAX_ROWS];
+  size_t which[BZ_FEED_MAX_ROWS];
   int n = 0;
-  for (size_t i = 0; i < external_output_blob_.size() && n < BZ_FEED_MAX_ROWS; ++i) {
-    const bool wanted = output_wanted_[i];
+  for (size_t i = 0; i < external_output_blob_.size(); ++i) {
+    const bool wanted = output_wanted_[i] && n < BZ_FEED_MAX_ROWS;
     output_wanted_[i] = false;
     Blob* blob = external_output_blob_[i];
     const size_t bytes = blob->size() * DataTypeSize(blob->data_type());
-    if (!wanted || st == nullptr || blob->device_type() != kHIP || blob->pitch() != 0 || blob->data() == nullptr || bytes == 0 || bytes > kMax)
+    if (!wanted || st == nullptr || blob->device_type() != kHIP || blob->pitch() != 0 || blob->data() == nullptr || bytes == 0 || bytes > kCopiedAheadMax)
       continue;
     if (std::any_of(handed_out_.begin(), handed_out_.end(), [&](Blob* b) { return Overlap(b, blob); })) continue;
     Blob* next = output_next_[i].get();
-    next->set_data_type((DataType)blob->data_type());
+    if (next->data() == nullptr || next->data_type() != blob->data_type() || next->capacity() < blob->size() || !IsPinnedHost(next->data()))
+      continue;
     next->Reshape(blob->shape());
-    if (!IsPinnedHost(next->data())) continue;
     rows[n].src = blob->data();
     rows[n].dst = next->data();
     rows[n].rows = 1;
     rows[n].row_bytes = rows[n].src_pitch = rows[n].dst_pitch = (int64_t)bytes;
-    ++n;
-    output_ahead_[i] = true;
+    which[n++] = i;
   }
-  if (n == 0) return;
-  const int rc = bz_feed(nullptr, nullptr, 0, rows, n, st);
-  if (rc != 0) output_ahead_.assign(output_ahead_.size(), false);  // Output copies by itself
+  if (n == 0 || bz_feed(nullptr, nullptr, 0, rows, n, st) != 0) return;  // (not launched: Output copies by itself)
+  for (int k = 0; k < n; ++k) output_ahead_[which[k]] = true;
 }
 
 bool Predictor::Output(const char* name, void** data, size_t* len) {
@@ -464,6 +467,10 @@ bool Predictor::Output(size_t idx, void** data, size_t* len) {
         HIPContext ctx(blob->device_option());
         ctx.Activate();
         CopyBytes(cpu->data(), kCPU, blob->data(), kHIP, bytes, ctx.hip_stream());
+        if (bytes <= kCopiedAheadMax) {
+          output_next_[idx]->set_data_type((DataType)blob->data_type());
+          output_next_[idx]->Reshape(blob->shape());
+        }
       }
       *data = cpu->data();
     }
