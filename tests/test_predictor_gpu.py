@@ -979,3 +979,33 @@ def test_the_pass_after_the_first_output_allocates_nothing(pb):
         p.forward()
         np.testing.assert_allclose(p.output_asnumpy("x"), _sigmoid(x), rtol=1e-5)
     assert pb.allocation_count() == before
+
+
+@pytest.mark.parametrize("n_in", [1, 8, 9, 17])
+def test_feed_many_of_strided_inputs(pb, n_in):
+    """Inputs that live side by side inside a Concat's output: one launch takes eight of them.  Odd widths, a plain input
+    beside them, an input named twice (the last one counts), a batch that grows and shrinks."""
+    rng = np.random.default_rng(n_in)
+    nb = pb.NetBuilder("strided", device_type=1)
+    widths = [1 + (5 * k) % 7 for k in range(n_in)]
+    for k in range(n_in):
+        nb.external_input("x%d" % k, 1)
+    nb.external_input("plain", 1)
+    nb.op("Concat", ["x%d" % k for k in range(n_in)], ["z"], axis=1)
+    nb.op("Sigmoid", ["plain"], ["s"])
+    nb.external_output("z", 1)
+    nb.external_output("s", 1)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for batch in (4, 301, 2):
+        for _ in range(2):
+            xs = [rng.standard_normal((batch, w)).astype(np.float32) for w in widths]
+            plain = rng.standard_normal((batch, 3)).astype(np.float32)
+            items = [("x%d" % k, a) for k, a in enumerate(xs)] + [("plain", plain)]
+            for name, a in items:
+                p.reshape_input(name, a.shape)
+            p.feed_many(p.feed_batch([("x0", xs[0] + 1)] + items))
+            p.forward()
+            np.testing.assert_array_equal(p.output_asnumpy("z"), np.concatenate(xs, 1))
+            np.testing.assert_allclose(p.output_asnumpy("s"), _sigmoid(plain), rtol=1e-5)
