@@ -161,6 +161,8 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     (2049, 513, 80, "prelu", {}), (4100, 200, 33, "none", {"full_bias": True}),   # 64x64, fp32: two groups of waves on each K tile
     (3000, 700, 72, "dice", {}), (2100, 1000, 65, "relu", {}), (4100, 500, 136, "sigmoid", {}),  # 2-byte: 128x128 and 64x128 from their first sizes
     (4100, 1000, 73, "prelu", {}), (8200, 1000, 201, "dice", {}), (33000, 80, 215, "dice", {}),  # 64x128, 128x128, 128x96
+    (2100, 300, 256 + 5, "prelu", {}), (3000, 200, 255, "dice", {}), (4100, 200, 769, "relu", {}),  # off 16 bytes: K tiles one and two in flight
+    (2049, 4097, 513, "none", {}),                                # fp32 off 16 bytes: 128x128 once K is deep
 ])
 def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, act, kw):
     print("case any %s M=%d N=%d K=%d act=%s %r" % (in_name, M, N, K, act, kw), flush=True)

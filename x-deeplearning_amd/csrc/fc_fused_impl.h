@@ -1233,23 +1233,34 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
     if (d.n > 64 && wg128 >= 140) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
     if (d.n > 64 && wg64x128 >= 256) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
   } else {
-    if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
-    if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+    if (d.n > 64 && wg128 >= 512 && (ALIGNED || d.k > 512)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
+    if constexpr (ALIGNED)
+      if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
   }
-  // fp32: eight waves, two to a SIMD, that share each K tile.  Its MFMAs are long, and with one wave a SIMD nothing runs
-  // while that wave reads fragments or waits at the barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way (at 8192 rows the
-  // matrix cores set the time, 64 us, either way).
-  if constexpr (DT == BZ_F32) {
-    if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
-  }
-  if (wg64 >= 256) {
+  // Rows that start anywhere: K is seldom a whole number of tiles, and a tile that is loaded only to be dropped costs as
+  // much as any other, so few are in flight: one while K is at most four tiles of 2-byte operands, else two.  64x64
+  // however many there are (us alone / with eight streams of the same; 32x64 or 64x64 with four in flight: fp16
+  // 3000 x 162 -> 200 8.1 / 3.7, now 6.0 / 2.8, 10000 x 50 -> 64 8.8 / 3.6 and 4.5 / 2.1, 2000 x 901 -> 400 14.9 / 9.2 and
+  // 10.3 / 5.8, fp32 3000 x 162 -> 200 16.5 / 7.5 and 9.0 / 5.0; 64x128: fp32 20000 x 162 -> 256 42.1 / 29.7 and
+  // 26.5 / 21.9; 128x128: fp32 16384 x 301 -> 512 65.5 / 58.9 and 55.9 / 52.3, but 16384 x 901 -> 512 140 / 130 and 149 / 146).
+  if constexpr (!ALIGNED) {
+    if constexpr (In<DT>::kSize == 2)
+      if (d.k <= 4 * BK) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, ALIGNED>(d, ep, st);
+    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
+  } else {
+    // fp32: eight waves, two to a SIMD, that share each K tile.  Its MFMAs are long, and with one wave a SIMD nothing runs
+    // while that wave reads fragments or waits at the barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way (at 8192 rows the
+    // matrix cores set the time, 64 us, either way).
+    if constexpr (DT == BZ_F32) {
+      if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
+    }
     // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
     // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
     // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
     // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
-    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+    if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
   }
-  return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
 }
 
 template <int DT, typename OutT>
