@@ -1259,6 +1259,10 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
     // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
     // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
     if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+    // Below a workgroup per CU the same tile with two in flight (1024 x 896 -> 512 7.4 us alone / 3.5 with eight streams of
+    // the same, 32x64 with four 8.4 / 4.1; 1500 x 896 -> 512 7.9 / 4.0 and 10.8 / 5.8, 5000 x 128 -> 100 5.8 / 2.6 and
+    // 7.2 / 3.2)
+    if constexpr (In<DT>::kSize == 2) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
   }
 }
@@ -1268,11 +1272,20 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   // rows 16-byte aligned and K a whole number of chunks
   const bool aligned = vec_a && vec_w && d.k % In<DT>::kChunk == 0;
-  // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Up to 512 32x32 tiles
-  // (fp32 1024 x 896 -> 512 15.4 us against the staged tile's 23.2, fp16 1024 x 1000 -> 512 7.5 and 8.4; with 1024 tiles
-  // fp32 2048 x 896 -> 512 29 and 24, fp16 9.5 and 8.8).
+  // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Its workgroups are large for
+  // what they do, so beyond a line they cost other streams more than they save a lone launch.
+  //  fp32: 512 32x32 tiles (us alone / with eight streams of the same, against 64x64 with two K tiles in flight:
+  //   1024 x 896 -> 512, 512 tiles, 15.1 / 11.4 and 22.3 / 13.0, 2000 x 144 -> 200, 441, 7.1 / 4.9 and 7.6 / 4.2;
+  //   2048 x 896 -> 512, 1024, 27.0 / 22.2 and 22.6 / 16.6).
+  //  2-byte: 256 (512 x 896 -> 512, 256 tiles, 4.4 / 2.6 and 7.3 / 3.3; 800 x 896 -> 512, 400, 6.7 / 4.1 and 7.9 / 3.7).
+  //   Among the other kernels of a CTR model's passes, on eight serving threads, 1024 x 896 -> 512 took 11.2 us a pass
+  //   this way and 8.7 on the tile, though 35.1 and 36.7 alone.
+  //  2-byte rows that start anywhere, K at most 256: 128 (512 x 162 -> 200, 112 tiles, 4.3 / 2.0 and 5.0 / 2.1;
+  //   1024 x 162 -> 200, 224, 4.4 / 2.2 and 5.1 / 2.2, but in the attention model of that layer at batch 1024, eight
+  //   serving threads, 41.1 M samples/s this way and 43.1 on the tile, 63.2 and 63.7 us a lone pass).
   const int64_t wg32 = (int64_t)((d.m + 31) / 32) * ((d.n + 31) / 32);
-  if (d.k < In<DT>::kChunk || wg32 <= 512) return launch_split<DT, OutT>(d, ep, st);
+  const int64_t few = DT == BZ_F32 ? 512 : (aligned || d.k > 256) ? 256 : 128;
+  if (d.k < In<DT>::kChunk || wg32 <= few) return launch_split<DT, OutT>(d, ep, st);
   if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
   // Largest first, and never a tile much wider than N.  128x256 with eight waves and three K tiles in flight fills the
   // chip once it has a workgroup per CU (its fp32 output tile would not fit the operand buffers it is staged in, so
