@@ -165,6 +165,7 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     (2100, 300, 256 + 5, "prelu", {}), (3000, 200, 255, "dice", {}), (4100, 200, 769, "relu", {}),  # off 16 bytes: K tiles one and two in flight
     (512, 512, 80, "dice", {}), (513, 512, 80, "dice", {}), (1024, 512, 264, "prelu", {}),  # 2-byte: 256 tiles, one row more; two K tiles in flight
     (512, 256, 77, "relu", {}), (513, 256, 77, "relu", {}), (512, 512, 257, "none", {}), (520, 512, 257, "none", {}),  # the same off 16 bytes
+    (1025, 512, 80, "relu", {}), (2049, 513, 520, "dice", {}), (2049, 513, 508, "none", {}), (4097, 512, 520, "prelu", {}),  # fp32: 64x64, shared by eight waves from K 512 and up to 511 tiles
     (2049, 4097, 513, "none", {}),                                # fp32 off 16 bytes: 128x128 once K is deep
 ])
 def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, act, kw):

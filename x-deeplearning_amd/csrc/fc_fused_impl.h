@@ -1248,11 +1248,17 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
       if (d.k <= 4 * BK) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, ALIGNED>(d, ep, st);
     return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
   } else {
-    // fp32: eight waves, two to a SIMD, that share each K tile.  Its MFMAs are long, and with one wave a SIMD nothing runs
-    // while that wave reads fragments or waits at the barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way (at 8192 rows the
-    // matrix cores set the time, 64 us, either way).
     if constexpr (DT == BZ_F32) {
-      if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
+      // fp32, K of 512 and more, tiles for at most two rounds of the CUs: eight waves, two to a SIMD, that share each K
+      // tile.  Its MFMAs are long, and with one wave a SIMD nothing runs while that wave reads fragments or waits at the
+      // barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way, 2048 x 512 -> 512 14.8 and 13.4.  With more tiles the matrix
+      // cores set the time either way (8192 rows 64 us), and next to other kernels the smaller workgroup wins (the tower
+      // of that layer at 4096 rows, eight serving threads, 57.8 us a pass this way and 56.8 the other).
+      if (d.k >= 512 && wg64 >= 256 && wg64 < 512) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
+      // Else four waves and two K tiles in flight (us alone / with eight streams of the same; the eight waves:
+      // 10000 x 64 -> 200 14.5 / 9.4 and now 9.6 / 5.8, 4096 x 192 -> 512 14.4 / 11.3 and 12.4 / 8.8, 1500 x 400 -> 700
+      // 21.9 / 11.6 and 19.5 / 10.8; 32x64 with four in flight: 1500 x 896 -> 512 37.0 / 19.0 and 22.3 / 15.2).
+      return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     }
     // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
     // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
@@ -1262,8 +1268,7 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
     // Below a workgroup per CU the same tile with two in flight (1024 x 896 -> 512 7.4 us alone / 3.5 with eight streams of
     // the same, 32x64 with four 8.4 / 4.1; 1500 x 896 -> 512 7.9 / 4.0 and 10.8 / 5.8, 5000 x 128 -> 100 5.8 / 2.6 and
     // 7.2 / 3.2)
-    if constexpr (In<DT>::kSize == 2) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
-    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, ALIGNED>(d, ep, st);
+    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
   }
 }
 
