@@ -173,6 +173,24 @@ def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, 
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + 5 * N + K, **kw)
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 512, 192), (10000, 200, 64), (1500, 700, 400), (2048, 512, 500), (2048, 512, 512), (4096, 512, 896),
+                                   (3000, 200, 301), (20000, 256, 162)])
+def test_fc_fp32_error_against_64_bits(bz, M, N, K):
+    """Four partial sums an output.  A running sum of n terms of one magnitude grows like sqrt(i), each step rounds it by
+    u / sqrt(3) of itself (u = 2^-24), so relative to the result the error is u * sqrt(n / 6); an MFMA step adds two products,
+    so n = K / 8 for a partial sum of four.  Adding the four and the bias rounds some more: 0.8 u^2.  20 % on top: with two
+    partial sums it is 41 % more."""
+    import torch
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    bias = torch.randn(N, device="cuda") * 0.1
+    y = bz.fc_fused(x, w, K, bias=bias)
+    want = x.double() @ w[:, :K].double().t().contiguous() + bias.double()
+    err = float((y.double() - want).norm() / want.norm())
+    assert err <= 1.2 * 2.0**-24 * (K / 8 / 6 + 0.8)**0.5, err
+
+
 # Large 2-byte layers go to the streaming kernel (256x128 tiles, loader waves, operands straight into LDS) once
 # ceil(M/256) * ceil(N/128) >= 200, K is a multiple of 64 and at least 512, and the output takes 16-byte stores.
 @pytest.mark.parametrize("in_name", ["f16", "bf16"])

@@ -294,8 +294,9 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   }
 
   // with a single 32x32 block per wave, back-to-back MFMAs into one accumulator would each wait for the
-  // previous result; alternate K steps between two accumulators and add them at the end
-  constexpr int KACC = (TM * TN == 1 && BK / T::kStepK / WK >= 2) ? 2 : 1;
+  // previous result; alternate K steps between accumulators and add them at the end.  fp32: one for each step of a K
+  // tile, which also makes the sums shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two)
+  constexpr int KACC = TM * TN > 1 ? 1 : DT == BZ_F32 ? BK / T::kStepK / WK : BK / T::kStepK / WK >= 2 ? 2 : 1;
   floatx16 acc[KACC][TM][TN];
 #pragma unroll
   for (int a = 0; a < KACC; ++a)
@@ -407,14 +408,14 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   }
   }
 
-  if (KACC == 2) {
+#pragma unroll
+  for (int a = 1; a < KACC; ++a)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][i][j][r] += acc[KACC - 1][i][j][r];
-  }
+        for (int r = 0; r < 16; ++r) acc[0][i][j][r] += acc[a][i][j][r];
   // the other groups' partial tiles, through LDS behind the output tile's place: group 0 goes on with the sum
   if constexpr (WK > 1) {
     static_assert(WK == 2 && !HEAD && BM * (BN * (int)sizeof(OutT) + 16) + BM * (BN + 1) * 4 <= (int)sizeof(lds), "room for the partial tile");
@@ -1259,16 +1260,17 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
       // 10000 x 64 -> 200 14.5 / 9.4 and now 9.6 / 5.8, 4096 x 192 -> 512 14.4 / 11.3 and 12.4 / 8.8, 1500 x 400 -> 700
       // 21.9 / 11.6 and 19.5 / 10.8; 32x64 with four in flight: 1500 x 896 -> 512 37.0 / 19.0 and 22.3 / 15.2).
       return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
+    } else {
+      // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
+      // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
+      // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
+      // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
+      if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+      // Below a workgroup per CU the same tile with two in flight (1024 x 896 -> 512 7.4 us alone / 3.5 with eight streams of
+      // the same, 32x64 with four 8.4 / 4.1; 1500 x 896 -> 512 7.9 / 4.0 and 10.8 / 5.8, 5000 x 128 -> 100 5.8 / 2.6 and
+      // 7.2 / 3.2)
+      return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     }
-    // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
-    // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
-    // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
-    // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
-    if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
-    // Below a workgroup per CU the same tile with two in flight (1024 x 896 -> 512 7.4 us alone / 3.5 with eight streams of
-    // the same, 32x64 with four 8.4 / 4.1; 1500 x 896 -> 512 7.9 / 4.0 and 10.8 / 5.8, 5000 x 128 -> 100 5.8 / 2.6 and
-    // 7.2 / 3.2)
-    return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
   }
 }
 
