@@ -173,13 +173,19 @@ def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, 
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + 5 * N + K, **kw)
 
 
+def _fp32_sum_error(n):
+    """Error of an output relative to it, the root mean square over outputs, where every partial sum has n products.  The sum
+    grows like sqrt(i) and each step rounds it; rounding is evenly spread over half a unit in the last place either way, which is
+    0.425 u of the value in the mean over mantissas (u = 2^-24: u / sqrt(3) times the mean of 1 / m^2, 0.541, to the half).
+    So u * 0.425 * sqrt(n / 2); adding a few partial sums and the bias rounds some more: 0.8 u^2.  20 % on top: with half as
+    many partial sums it is 41 % more."""
+    return 1.2 * 2.0**-24 * (0.425**2 * n / 2 + 0.8)**0.5
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 512, 192), (10000, 200, 64), (1500, 700, 400), (2048, 512, 500), (2048, 512, 512), (4096, 512, 896),
                                    (3000, 200, 301), (20000, 256, 162)])
 def test_fc_fp32_error_against_64_bits(bz, M, N, K):
-    """Four partial sums an output.  A running sum of n terms of one magnitude grows like sqrt(i), each step rounds it by
-    u / sqrt(3) of itself (u = 2^-24), so relative to the result the error is u * sqrt(n / 6); an MFMA step adds two products,
-    so n = K / 8 for a partial sum of four.  Adding the four and the bias rounds some more: 0.8 u^2.  20 % on top: with two
-    partial sums it is 41 % more."""
+    """the staged tiles of one block a wave: four partial sums an output"""
     import torch
     torch.manual_seed(M + K)
     x = torch.randn(M, K, device="cuda")
@@ -188,7 +194,23 @@ def test_fc_fp32_error_against_64_bits(bz, M, N, K):
     y = bz.fc_fused(x, w, K, bias=bias)
     want = x.double() @ w[:, :K].double().t().contiguous() + bias.double()
     err = float((y.double() - want).norm() / want.norm())
-    assert err <= 1.2 * 2.0**-24 * (K / 8 / 6 + 0.8)**0.5, err
+    assert err <= _fp32_sum_error(K / 4), err
+
+
+@pytest.mark.parametrize("M,N,K,parts", [(2048, 256, 512, 2), (2048, 128, 1024, 4), (2000, 80, 200, 5), (2049, 256, 512, 2), (4096, 128, 512, 4)])
+def test_fc_fp32_error_of_a_layer_with_a_head(bz, M, N, K, parts):
+    """up to 2048 rows the 32-column blocks of a row share sixteen waves; beyond, two sums of the 256-wide tile, four of the others"""
+    import torch
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    w2 = bz.pack_weight(torch.randn(N, 2, device="cuda"), False, bz.F32)
+    bias = torch.randn(N, device="cuda") * 0.1
+    z = torch.empty((M, 2), device="cuda")
+    y, _ = bz.fc_fused(x, w, K, bias=bias, head=dict(w=w2, act=bz.ACT_NONE, out=z))
+    want = x.double() @ w[:, :K].double().t().contiguous() + bias.double()
+    err = float((y.double() - want).norm() / want.norm())
+    assert err <= _fp32_sum_error(K / parts), err
 
 
 # Large 2-byte layers go to the streaming kernel (256x128 tiles, loader waves, operands straight into LDS) once
@@ -216,8 +238,11 @@ def test_fc_streaming_kernel(bz, oracle, in_name, M, N, K, act, kw):
     (17000, 80, 40, 1, "dice", "none"),        # the same with enough rows for the 64x64 tile
     (513, 128, 128, 8, "relu", "sigmoid"),     # widest head
     (100, 64, 16, 3, "none", "softmax"),
-    (4096, 96, 256, 2, "relu", "sigmoid"),     # fp32: the last size of sixteen rows a workgroup, and the first beyond
+    (4096, 96, 256, 2, "relu", "sigmoid"),
     (4097, 96, 256, 2, "relu", "sigmoid"),
+    (2048, 104, 256, 2, "dice", "softmax"),    # fp32: the last size of sixteen rows a workgroup, and the first beyond
+    (2049, 104, 256, 2, "dice", "softmax"),
+    (2049, 200, 80, 1, "prelu", "sigmoid"),
     (17, 8, 224, 5, "none", "none"),           # a part of one unit of K, seven column blocks on sixteen waves, a single row left
     (1, 1104, 72, 1, "prelu", "sigmoid"),      # units shared by five parts, K ending inside one
 ])

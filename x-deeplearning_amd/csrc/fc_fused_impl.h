@@ -186,8 +186,17 @@ __device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const f
 // ---------------------------------------------------------------------------------------------
 // tiled MFMA kernel
 // ---------------------------------------------------------------------------------------------
+// Sums an output is added up in where a wave owns one 32x32 block.  fp32: one for each step of a K tile, which also makes
+// them shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two).  Two otherwise, and in the tiles with
+// a head, whose other registers are many: with four the 64x64 one takes 10.7 us for 17000 x 80 -> 40 instead of 10.3.
+template <int DT, int BM, int BN, int BK, int WM, int WN, bool HEAD, int WK>
+constexpr int default_sums() {
+  constexpr int steps = BK / In<DT>::kStepK / WK;
+  return BM / WM / 32 * (BN / WN / 32) > 1 ? 1 : DT == BZ_F32 && !HEAD ? steps : steps >= 2 ? 2 : 1;
+}
+
 // WK: groups of WM x WN waves that share each K tile between them and add up at the end
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD, int WK>
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD, int WK, int KACC>
 __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                   OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                   int64_t ldw, int64_t ldy, bool vec_y, int tiles_m, Epilogue ep,
@@ -294,9 +303,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   }
 
   // with a single 32x32 block per wave, back-to-back MFMAs into one accumulator would each wait for the
-  // previous result; alternate K steps between accumulators and add them at the end.  fp32: one for each step of a K
-  // tile, which also makes the sums shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two)
-  constexpr int KACC = TM * TN > 1 ? 1 : DT == BZ_F32 ? BK / T::kStepK / WK : BK / T::kStepK / WK >= 2 ? 2 : 1;
+  // previous result; alternate K steps between KACC accumulators and add them at the end
   floatx16 acc[KACC][TM][TN];
 #pragma unroll
   for (int a = 0; a < KACC; ++a)
@@ -1139,7 +1146,8 @@ inline HeadArgs head_args(const bz_fc_desc& d) {
   return head;
 }
 
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false, int WK = 1>
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false, int WK = 1,
+          int KACC = default_sums<DT, BM, BN, BK, WM, WN, HEAD, WK>()>
 int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
   // output rows 16-byte aligned and N a whole number of 16-byte chunks: coalesced stores through LDS
@@ -1148,7 +1156,7 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
   const HeadArgs head = HEAD ? head_args(d) : HeadArgs{};
-  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
+  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK, KACC>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
   return BZ_OK;
@@ -1193,16 +1201,24 @@ int launch_stream(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 template <int DT, typename OutT>
 int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
-  // fp32 is bound by the matrix cores of the CUs that work: 16 rows a workgroup up to 4096 rows (2048 x 512 -> 256 19.2 us
-  // against 25.2, 4096 x 1024 -> 128 19.4 and 30.7, 201 x 200 -> 80 7.8 and 10.3; 8192 rows 35.7 and 26.4).  2-byte layers
-  // are not (2048 x 512 -> 256 fp16 10.2 and 9.0).
+  // fp32 is bound by the matrix cores of the CUs that work, so the staged tile's 32 rows waste time while they are few: 16
+  // rows a workgroup up to 2048 rows (us alone / with eight streams of the same, the tile's behind: 1024 x 512 -> 256
+  // 18.9 / 7.5 and 25.4 / 9.8, 2048 x 512 -> 256 19.2 / 10.1 and 25.5 / 9.9, 2000 x 512 -> 128 12.4 / 6.4 and 17.7 / 9.0,
+  // 201 x 200 -> 80 7.9 / 3.2 and 10.6 / 4.1; 4096 x 512 -> 256 19.4 / 17.5 and 25.6 / 14.0).  A row's operands cost more
+  // this way, which shows where other kernels fill the chip: of a tower on eight serving threads a pass of 1024 rows takes
+  // 20.4 us and 21.7 with the tile, of 2048 32.1 and 30.7 (64.0 and 69.1 alone), of 4096 63.6 and 57.0 (84.8 and 89.8).
+  // 2-byte layers are not bound by the matrix cores (2048 x 512 -> 256 fp16 10.2, the tile 9.0; measured at that size alone).
   if constexpr (DT == BZ_F32) {
-    if (d.m <= 4096) {
+    if (d.m <= 2048) {
       hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
                          (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d));
       BZ_LAUNCH_OK("bz_fc_split_head_kernel");
       return BZ_OK;
     }
+    // Up to 4096 rows four sums an output, as short as that kernel's (3000 x 512 -> 128 17.9 / 8.3, with two 17.8 / 9.3;
+    // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6)
+    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true, 1, 4>(d, ep, st);
+    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, true, 1, 4>(d, ep, st);
   }
   if (d.n <= 64) {
     if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, true>(d, ep, st);
