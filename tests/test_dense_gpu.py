@@ -160,7 +160,7 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     (1024, 512, 77, "dice", {}), (1025, 512, 77, "dice", {}),                     # 512 tiles, and one row of tiles more
     (3000, 200, 5, "relu", {}), (2100, 300, 9, "none", {"full_bias": True}),      # staged: K about a chunk
     (2049, 513, 80, "prelu", {}), (4100, 200, 33, "none", {"full_bias": True}),   # 64x64, fp32: two groups of waves on each K tile
-    (3000, 700, 72, "dice", {}), (2100, 1000, 65, "relu", {}), (4100, 500, 136, "sigmoid", {}),  # 2-byte: 128x128 and 64x128 from their first sizes
+    (3000, 700, 72, "dice", {}), (2100, 1000, 65, "relu", {}), (4100, 500, 136, "sigmoid", {}), (2048, 1000, 72, "none", {}),  # 2-byte: 128x128 and, one round of tiles, 64x128
     (4100, 1000, 73, "prelu", {}), (8200, 1000, 201, "dice", {}), (33000, 80, 215, "dice", {}),  # 64x128, 128x128, 128x96
     (2100, 300, 256 + 5, "prelu", {}), (3000, 200, 255, "dice", {}), (4100, 200, 769, "relu", {}),  # off 16 bytes: K tiles one and two in flight
     (512, 512, 80, "dice", {}), (513, 512, 80, "dice", {}), (1024, 512, 264, "prelu", {}),  # 2-byte: 256 tiles, one row more; two K tiles in flight

@@ -801,14 +801,14 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 #undef BZ_PIN_PHASE
 
 // ---------------------------------------------------------------------------------------------
-// split kernel: few tiles, or rows that start on no 16 bytes
+// split kernel: few tiles
 // ---------------------------------------------------------------------------------------------
 // A workgroup owns a 32 x 32 tile of C and its eight waves share the K range: unit u (128 bytes of every row) is
 // wave u % 8's.  A wave works for itself: it loads a unit with eight lanes on a row, turns it in LDS of its own into MFMA
 // fragments, the next unit's loads in flight meanwhile, and meets the others only when the partial tiles are added up.
 //  - Few tiles leave the chip idle and the chain of K tiles sets the time: eight waves walk it in an eighth of the steps.
 //  - A lane's 16 bytes may start anywhere (a row pitch of 445 fp16 elements): the memory system takes such loads, and
-//    the lines they share are L1 hits.
+//    the lines they share are L1 hits.  So rows that start on no 16 bytes need no path of their own here.
 // Loaded straight into fragments a group of 16 lanes touches 16 lines, and the path into the CU takes a line a clock:
 // 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile); 32 x 2075 -> 768 fp32 17.0, 14.4 (51.7).
 constexpr int kSplitWaves = 8, kSplitUnit = 128, kSplitPitch = kSplitUnit + 16;
@@ -1242,12 +1242,15 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   // tall and narrow (the attention MLP over batch x history rows): one 96-wide tile reads A once
   if (d.n > 64 && d.n <= 96 && (d.m + 127) / 128 >= 256)
     return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, ALIGNED>(d, ep, st);
-  // 2-byte operands: eight waves on a 128- or 64-row tile of 128 columns with two K tiles in flight, once they give half
-  // the CUs a workgroup of the former or all of them one of the latter (fp16, against four waves on 64x128 or 64x64:
-  // 8192 x 1024 -> 512 17.2 us and 20.2, 4096 x 896 -> 1024 13.4 and 17.9, 3000 x 1024 -> 768, 144 tiles, 12.9 and 17.2;
-  // 4096 x 2048 -> 512, 128 tiles, 22.8 and 20.7, on 64 rows 17.9)
+  // 2-byte operands: eight waves on tiles of 128 columns with two K tiles in flight.  64 rows while that is one round of the
+  // CUs, 256 tiles; with more, 128 rows, where a second round of smaller tiles would cost as much as the first (us alone /
+  // with eight streams of the same, 64 rows, 128 rows, four waves on 64x64: 2048 x 896 -> 1024, 256 tiles of 64 rows,
+  // 10.1 / 7.2, 12.8 / 6.7, 11.1 / 7.6; 2176 rows, 272 tiles, 14.1 / 8.5, 13.3 / 8.0, 13.5 / 8.8; 2048 x 2048 -> 1024
+  // 17.9 / 14.3, 22.5 / 13.2, 20.5 / 15.9; 2176 rows 26.2 / 17.4, 23.1 / 16.3, 24.9 / 21.1).  Where K is shallow the second
+  // round is short and the line lies a little higher (2176 x 128 -> 1024 5.7 / 3.1 and 6.5 / 3.1, 2304 rows, 288 tiles,
+  // 5.7 / 3.1 and 6.0 / 3.1).
   if constexpr (In<DT>::kSize == 2) {
-    if (d.n > 64 && wg128 >= 140) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
+    if (d.n > 64 && wg128 >= (d.k > 256 ? 129 : 140)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
     if (d.n > 64 && wg64x128 >= 256) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
   } else {
     if (d.n > 64 && wg128 >= 512 && (ALIGNED || d.k > 512)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
@@ -1312,8 +1315,7 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
   // Largest first, and never a tile much wider than N.  128x256 with eight waves and three K tiles in flight fills the
   // chip once it has a workgroup per CU (its fp32 output tile would not fit the operand buffers it is staged in, so
-  // 2-byte outputs only); below that, 128x128; then 64x128 while that still gives two workgroups per CU; then the
-  // latency-bound small tiles.
+  // 2-byte outputs only); below that the tiles of dispatch_mid.
   const int64_t wg128x256 = (int64_t)((d.m + 127) / 128) * ((d.n + 255) / 256);
   if constexpr (sizeof(OutT) == 2 && In<DT>::kSize == 2) {
     // the streaming kernel once its 256x128 tiles keep most CUs busy and K is deep enough to pay for filling its ring
