@@ -350,8 +350,11 @@ struct ServePool {
       {
         // a job that follows the previous one at once (a warm-up run, then the timed one) should not pay a futex
         // wake-up per thread: poll for a short while before going to sleep -- but not while another pool of the process
-        // has a job: two idle pools of eight polling threads occupied all 16 CPUs of the box, and the third pool's
-        // threads waited for them to stop (three pools taking turns with 64 passes each: 1880 us a job, 950 us of work)
+        // has a job.  On 16 CPUs, us of wall a job, polling always / by this rule: three pools of eight threads taking turns
+        // with 64 passes each 1940 / 980 (950 us of work); two pools of eight at once, a caller each, 64 passes
+        // 1030-1170 / 914, 8 passes 150-240 / 127; two of four 64 passes 868 / 870, 4 passes 50.2 / 52.8, the one case
+        // where there are CPUs enough and the wake-ups show.  (Polling on as long as the threads that are awake are
+        // fewer than 10 to 16 gives that case its 50 back and the others 1890, 980-1240 and 150-290.)
         const auto spin_until = std::chrono::steady_clock::now() + std::chrono::microseconds(2000);
         while (generation_hint.load(std::memory_order_acquire) == seen &&
                g_jobs_running.load(std::memory_order_relaxed) <= job_running.load(std::memory_order_relaxed) &&
