@@ -17,10 +17,11 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
     cpu.set_device_type(kCPU);
     output_cpu_.push_back(std::make_shared<Blob>(cpu));
     output_cpu_.back()->set_data_type((DataType)b->data_type());
-    output_next_.push_back(std::make_shared<Blob>(cpu));
   }
   output_wanted_.assign(output_cpu_.size(), false);
   output_ahead_.assign(output_cpu_.size(), false);
+  output_half_.assign(output_cpu_.size(), 0);
+  output_read_.assign(output_cpu_.size(), 0);
   for (const auto& name : net_->external_input()) {
     Blob* b = net_->external_input_blob(name);
     BLAZE_CONDITION_THROW(b != nullptr, "external_input: ", name, " is not in external_input_blob");
@@ -400,11 +401,17 @@ bool Overlap(Blob* a, Blob* b) {
 // Outputs that were read after the last Forward are copied to the host behind this one, under the same wait: a copy asked
 // for by Output alone is another launch and another wait, 16 us of a 58 us request.  Small ones only, by a kernel that
 // writes the pinned copy over the link (the copy engine's hand-over would cost more than it moves); larger ones are
-// copied by Output.  Into a second buffer: the one Output handed out stays as it is until the next Output.  Not where the
-// caller holds the device address of that memory: what it writes there after the pass is the output, too.  Output makes
-// the second buffer as large as the one it fills (allocating between a launch and its wait would hold the pass up), so an
-// output that has grown since is copied by Output once more.
+// copied by Output.  Into the other half of the host buffer: the half Output handed out stays as it is until the next Output.
+// Not where the caller holds the device address of that memory: what it writes there after the pass is the output, too.
+// Output makes both halves in one allocation (one between a launch and its wait would hold the pass up), so an output that
+// has grown since is copied by Output once more.
 constexpr size_t kCopiedAheadMax = 64 << 10;
+constexpr TIndex kHalfAlign = 64;  // elements
+
+size_t Predictor::HostHalf(size_t i) const {
+  const Blob& b = *output_cpu_[i];
+  return b.capacity() / (2 * kHalfAlign) * kHalfAlign * DataTypeSize(b.data_type());
+}
 
 void Predictor::QueueOutputs() {
   hipStream_t st = (hipStream_t)net_->WaitedStream();
@@ -419,12 +426,10 @@ void Predictor::QueueOutputs() {
     if (!wanted || st == nullptr || blob->device_type() != kHIP || blob->pitch() != 0 || blob->data() == nullptr || bytes == 0 || bytes > kCopiedAheadMax)
       continue;
     if (std::any_of(handed_out_.begin(), handed_out_.end(), [&](Blob* b) { return Overlap(b, blob); })) continue;
-    Blob* next = output_next_[i].get();
-    if (next->data() == nullptr || next->data_type() != blob->data_type() || next->capacity() < blob->size() || !IsPinnedHost(next->data()))
-      continue;
-    next->Reshape(blob->shape());
+    const size_t half = HostHalf(i);
+    if (output_cpu_[i]->data_type() != blob->data_type() || half < bytes || half < output_read_[i] || !IsPinnedHost(output_cpu_[i]->data())) continue;
     rows[n].src = blob->data();
-    rows[n].dst = next->data();
+    rows[n].dst = (char*)output_cpu_[i]->data() + (1 - output_half_[i]) * half;
     rows[n].rows = 1;
     rows[n].row_bytes = rows[n].src_pitch = rows[n].dst_pitch = (int64_t)bytes;
     which[n++] = i;
@@ -456,23 +461,22 @@ bool Predictor::Output(size_t idx, void** data, size_t* len) {
     if (blob->device_type() == kCPU) {
       *data = blob->data();
     } else {
-      std::shared_ptr<Blob>& cpu = output_cpu_[idx];
+      Blob* cpu = output_cpu_[idx].get();
       output_wanted_[idx] = true;
       if (output_ahead_[idx]) {  // (a second Output of the same pass copies again)
-        cpu.swap(output_next_[idx]);
+        output_half_[idx] = 1 - output_half_[idx];
         output_ahead_[idx] = false;
       } else {
         cpu->set_data_type((DataType)blob->data_type());
-        cpu->Reshape(blob->shape());
+        const bool two = bytes <= kCopiedAheadMax;
+        cpu->Reshape({two ? 2 * ((blob->size() + kHalfAlign - 1) / kHalfAlign * kHalfAlign) : blob->size()});
+        if (HostHalf(idx) < bytes) output_half_[idx] = 0;
         HIPContext ctx(blob->device_option());
         ctx.Activate();
-        CopyBytes(cpu->data(), kCPU, blob->data(), kHIP, bytes, ctx.hip_stream());
-        if (bytes <= kCopiedAheadMax) {
-          output_next_[idx]->set_data_type((DataType)blob->data_type());
-          output_next_[idx]->Reshape(blob->shape());
-        }
+        CopyBytes((char*)cpu->data() + output_half_[idx] * HostHalf(idx), kCPU, blob->data(), kHIP, bytes, ctx.hip_stream());
       }
-      *data = cpu->data();
+      output_read_[idx] = bytes;
+      *data = (char*)cpu->data() + output_half_[idx] * HostHalf(idx);
     }
   } catch (std::exception& e) {
     LOG_ERROR("output failed: %s", e.what());

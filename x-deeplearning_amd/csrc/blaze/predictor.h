@@ -84,11 +84,15 @@ class Predictor {
   std::shared_ptr<Net> net_;
   std::vector<Blob*> external_input_blob_, external_output_blob_;
   std::unordered_map<std::string, int> input_index_, output_index_;
+  // host copies of the outputs, in two halves where they are small: one that Output handed out, one that Forward copies
+  // into ahead of the next Output (QueueOutputs)
   std::vector<std::shared_ptr<Blob>> output_cpu_;
-  std::vector<std::shared_ptr<Blob>> output_next_;  // what Forward copied ahead of Output (QueueOutputs)
-  std::vector<bool> output_wanted_;                 // read since the last Forward
-  std::vector<bool> output_ahead_;                  // output_next_ holds the last Forward's result
-  std::vector<Blob*> handed_out_;                   // whose device address the caller has
+  std::vector<int> output_half_;     // the half handed out last
+  std::vector<size_t> output_read_;  // bytes handed out last: may reach beyond a half when the output was larger then
+  std::vector<bool> output_wanted_;  // read since the last Forward
+  std::vector<bool> output_ahead_;   // the other half holds the last Forward's result
+  std::vector<Blob*> handed_out_;    // whose device address the caller has
+  size_t HostHalf(size_t i) const;   // bytes of a half of output_cpu_[i]
   void* HandOut(Blob* blob);
   void QueueOutputs();
   // pinned staging of fed inputs: Feed copies the caller's bytes here and queues the transfer on the thread's
