@@ -128,13 +128,16 @@ BLAZE_API int Blaze_PredictorManagerLoadModelFromString(PredictorManagerHandle h
  */
 BLAZE_API int Blaze_ConvertNetDef(const char* in, size_t len, int in_is_text, int out_is_text, char* out, size_t cap, size_t* out_len);
 
-/* device address of an input / output blob after ReshapeInput / Forward, for callers that keep inputs on the device */
+/* device address of an input / output blob after ReshapeInput / Forward, for callers that keep inputs on the device.  Output
+ * returns what such a caller wrote there; in turn, memory whose address was handed out is not copied to the host before
+ * Output asks for it. */
 BLAZE_API int Blaze_PredictorInputDevicePtr(PredictorHandle handle, const char* name, void** ptr);
 BLAZE_API int Blaze_PredictorOutputDevicePtr(PredictorHandle handle, const char* name, void** ptr);
 
 /* Blaze_PredictorFeed for `count` inputs in one call (a sparse model has three inputs per feature group).  The shapes
- * must have been set (ReshapeInput).  Inputs that are plain device tensors are staged side by side and travel in one
- * transfer; the predictor's input tensors then view slices of that one device buffer. */
+ * must have been set (ReshapeInput).  Device inputs are staged side by side and cross together, in one launch or, from two
+ * megabytes on, in several as they are staged: plain ones into one device buffer, whose slices the predictor's input
+ * tensors then view, those that live inside a Concat's output into their rows of it. */
 BLAZE_API int Blaze_PredictorFeedMany(PredictorHandle handle, int count, const char* const* names, const void* const* data,
                                       const size_t* lens);
 
