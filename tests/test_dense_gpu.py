@@ -148,9 +148,9 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + N * 3 + K)
 
 
-# Up to 512 32x32 tiles (2-byte operands 256, or 128 where rows start on no 16 bytes and K is at most 256) go to the
-# kernel whose eight waves share K in units of 128 bytes; beyond that, rows that start on no 16 bytes go to the staged
-# tiles with loads at any element.
+# Up to 512 32x32 tiles (2-byte operands 256, or 192 where rows start on no 16 bytes and K is at most 256) go to the
+# kernel whose eight waves share K in units of 128 bytes, 2-byte ones of K above 256 up to 512 tiles to the same with four;
+# beyond that, rows that start on no 16 bytes go to the staged tiles with loads at any element.
 @pytest.mark.parametrize("in_name,out_name", [("f32", "f32"), ("f16", "f16"), ("bf16", "f32")])
 @pytest.mark.parametrize("M,N,K,act,kw", [
     (1, 9, 1, "none", {}), (33, 40, 3, "prelu", {}), (31, 64, 31, "dice", {}),   # a partial unit only
@@ -164,7 +164,8 @@ def test_fc_half(bz, oracle, in_name, out_name, M, N, K, act):
     (4100, 1000, 73, "prelu", {}), (8200, 1000, 201, "dice", {}), (33000, 80, 215, "dice", {}),  # 64x128, 128x128, 128x96
     (2100, 300, 256 + 5, "prelu", {}), (3000, 200, 255, "dice", {}), (4100, 200, 769, "relu", {}),  # off 16 bytes: K tiles one and two in flight
     (512, 512, 80, "dice", {}), (513, 512, 80, "dice", {}), (1024, 512, 264, "prelu", {}),  # 2-byte: 256 tiles, one row more; two K tiles in flight
-    (512, 256, 77, "relu", {}), (513, 256, 77, "relu", {}), (512, 512, 257, "none", {}), (520, 512, 257, "none", {}),  # the same off 16 bytes
+    (384, 512, 77, "relu", {}), (385, 512, 77, "relu", {}), (512, 512, 257, "none", {}), (520, 512, 257, "none", {}),  # the same off 16 bytes
+    (1000, 500, 600, "dice", {"full_bias": True}), (1024, 512, 1001, "sigmoid", {}), (730, 512, 64, "relu", {}),  # four waves; one K tile
     (1025, 512, 80, "relu", {}), (2049, 513, 520, "dice", {}), (2049, 513, 508, "none", {}), (4097, 512, 520, "prelu", {}),  # fp32: 64x64, shared by eight waves from K 512 and up to 511 tiles
     (2049, 4097, 513, "none", {}),                                # fp32 off 16 bytes: 128x128 once K is deep
 ])

@@ -803,15 +803,15 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 // ---------------------------------------------------------------------------------------------
 // split kernel: few tiles
 // ---------------------------------------------------------------------------------------------
-// A workgroup owns a 32 x 32 tile of C and its eight waves share the K range: unit u (128 bytes of every row) is
-// wave u % 8's.  A wave works for itself: it loads a unit with eight lanes on a row, turns it in LDS of its own into MFMA
+// A workgroup owns a 32 x 32 tile of C and its eight or four waves (NW) share the K range: unit u (128 bytes of every row)
+// is wave u % NW's.  A wave works for itself: it loads a unit with eight lanes on a row, turns it in LDS of its own into MFMA
 // fragments, the next unit's loads in flight meanwhile, and meets the others only when the partial tiles are added up.
 //  - Few tiles leave the chip idle and the chain of K tiles sets the time: eight waves walk it in an eighth of the steps.
 //  - A lane's 16 bytes may start anywhere (a row pitch of 445 fp16 elements): the memory system takes such loads, and
 //    the lines they share are L1 hits.  So rows that start on no 16 bytes need no path of their own here.
 // Loaded straight into fragments a group of 16 lanes touches 16 lines, and the path into the CU takes a line a clock:
 // 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile); 32 x 2075 -> 768 fp32 17.0, 14.4 (51.7).
-constexpr int kSplitWaves = 8, kSplitUnit = 128, kSplitPitch = kSplitUnit + 16;
+constexpr int kSplitUnit = 128, kSplitPitch = kSplitUnit + 16;
 
 // One wave's 8 * P rows of an operand, a unit of K at a time: global memory -> registers (lane: row l / 8 of each pass,
 // chunk l % 8) -> LDS rows kSplitPitch apart.
@@ -846,12 +846,12 @@ struct SplitRows {
   }
 };
 
-template <int DT, typename OutT>
-__global__ __launch_bounds__(kSplitWaves * 64, 4) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
-                                                                          OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
-                                                                          int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
+template <int DT, typename OutT, int NW>
+__global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
+                                                                 OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
+                                                                 int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
   using T = In<DT>;
-  constexpr int NW = kSplitWaves, STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
+  constexpr int STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
   constexpr int PITCH = 33;
   __shared__ __attribute__((aligned(16))) char lds[NW][64 * kSplitPitch];
   static_assert(32 * PITCH * 4 <= 64 * kSplitPitch, "a partial tile fits where its wave's operands were");
@@ -891,8 +891,8 @@ __global__ __launch_bounds__(kSplitWaves * 64, 4) void bz_fc_split_kernel(const 
              *(const uint4*)(lw + frow * kSplitPitch + fhalf * 16 + ks * 32), acc);
     __builtin_amdgcn_wave_barrier();
   }
-  // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper four waves leave theirs where
-  // their operands were, the lower four add their own
+  // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper half of the waves leave theirs
+  // where their operands were, the lower half add their own
   float* mine = (float*)lds[wave] + 4 * fhalf * PITCH + frow;
   if (wave >= NW / 2) {
 #pragma unroll
@@ -1163,10 +1163,10 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 }
 
 
-template <int DT, typename OutT>
+template <int DT, typename OutT, int NW>
 int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 31) / 32, tiles_n = (d.n + 31) / 32;
-  hipLaunchKernelGGL((bz_fc_split_kernel<DT, OutT>), dim3(tiles_m * tiles_n), dim3(kSplitWaves * 64), 0, st, (const char*)d.a,
+  hipLaunchKernelGGL((bz_fc_split_kernel<DT, OutT, NW>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a,
                      (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, tiles_m, ep);
   BZ_LAUNCH_OK("bz_fc_split_kernel");
   return BZ_OK;
@@ -1285,9 +1285,10 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
       // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
       // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
       if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
-      // Below a workgroup per CU the same tile with two in flight (1024 x 896 -> 512 7.4 us alone / 3.5 with eight streams of
-      // the same, 32x64 with four 8.4 / 4.1; 1500 x 896 -> 512 7.9 / 4.0 and 10.8 / 5.8, 5000 x 128 -> 100 5.8 / 2.6 and
-      // 7.2 / 3.2)
+      // Below a workgroup per CU the same tile with two in flight (1500 x 896 -> 512 7.9 us alone / 4.0 with eight streams of
+      // the same, 32x64 with four 10.8 / 5.8; 5000 x 128 -> 100 5.8 / 2.6 and 7.2 / 3.2), or the one that there is
+      // (730 x 64 -> 512 3.7 / 1.7, with two 4.0 / 1.8)
+      if (d.k <= BK) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, ALIGNED>(d, ep, st);
       return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     }
   }
@@ -1303,15 +1304,20 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   //  fp32: 512 32x32 tiles (us alone / with eight streams of the same, against 64x64 with two K tiles in flight:
   //   1024 x 896 -> 512, 512 tiles, 15.1 / 11.4 and 22.3 / 13.0, 2000 x 144 -> 200, 441, 7.1 / 4.9 and 7.6 / 4.2;
   //   2048 x 896 -> 512, 1024, 27.0 / 22.2 and 22.6 / 16.6).
-  //  2-byte: 256 (512 x 896 -> 512, 256 tiles, 4.4 / 2.6 and 7.3 / 3.3; 800 x 896 -> 512, 400, 6.7 / 4.1 and 7.9 / 3.7).
-  //   Among the other kernels of a CTR model's passes, on eight serving threads, 1024 x 896 -> 512 took 11.2 us a pass
-  //   this way and 8.7 on the tile, though 35.1 and 36.7 alone.
-  //  2-byte rows that start anywhere, K at most 256: 128 (512 x 162 -> 200, 112 tiles, 4.3 / 2.0 and 5.0 / 2.1;
-  //   1024 x 162 -> 200, 224, 4.4 / 2.2 and 5.1 / 2.2, but in the attention model of that layer at batch 1024, eight
-  //   serving threads, 41.1 M samples/s this way and 43.1 on the tile, 63.2 and 63.7 us a lone pass).
+  //  2-byte: 256 (512 x 896 -> 512, 256 tiles, 4.4 / 2.6 and 7.3 / 3.3; 1024 x 256 -> 512, 512, 4.1 / 2.9 and 4.7 / 2.1);
+  //   K above 256 up to 512 with four waves, half the LDS (1024 x 896 -> 512, 512 tiles, eight waves, four, the 64x64 tile:
+  //   6.2 / 4.3, 6.0 / 3.7, 7.4 / 3.5; 742 x 2179 -> 512, 384, 12.2 / 8.1, 12.9 / 7.9, 16.5 / 8.7).  Models on eight serving
+  //   threads, us a pass, a lone pass in brackets, in the same order: that first layer at batch 1024 11.2 (35.3),
+  //   9.8 (35.2), 8.7 (36.8), 1984 -> 512 at 700 10.2 (40.2), 9.9 (39.7), 11.1 (45.3), at 1000 12.3 (38.8), 11.1 (38.3),
+  //   10.8 (42.9).
+  //  2-byte rows that start anywhere, K at most 256: 192 (850 x 162 -> 200, 189 tiles, 4.3 / 2.2 and 5.1 / 2.2 with one K
+  //   tile in flight; 1024 x 162 -> 200, 224, 4.4 / 2.2 and 5.1 / 2.2, but the attention model of that layer, batch 1024, on
+  //   eight serving threads 41.1 M samples/s this way and 43.1 on the tile, 63.2 and 63.7 us a lone pass).
   const int64_t wg32 = (int64_t)((d.m + 31) / 32) * ((d.n + 31) / 32);
-  const int64_t few = DT == BZ_F32 ? 512 : (aligned || d.k > 256) ? 256 : 128;
-  if (d.k < In<DT>::kChunk || wg32 <= few) return launch_split<DT, OutT>(d, ep, st);
+  const int64_t few = DT == BZ_F32 ? 512 : (aligned || d.k > 256) ? 256 : 192;
+  if (d.k < In<DT>::kChunk || wg32 <= few) return launch_split<DT, OutT, 8>(d, ep, st);
+  if constexpr (In<DT>::kSize == 2)
+    if (wg32 <= 512 && d.k > 256) return launch_split<DT, OutT, 4>(d, ep, st);
   if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
   // Largest first, and never a tile much wider than N.  128x256 with eight waves and three K tiles in flight fills the
   // chip once it has a workgroup per CU (its fp32 output tile would not fit the operand buffers it is staged in, so
