@@ -242,6 +242,8 @@ __device__ __forceinline__ void accum_chunk(float (&acc)[RowTraits<DT>::kElems],
   }
 }
 
+typedef unsigned long long u64x2a8 __attribute__((ext_vector_type(2), aligned(8)));
+
 // key / id -> table row, or -1 when absent.  Hash path = HashTable::Lookup
 // (hashtable.cc:45-64): bucket record {offset:40, size:24}, (key,row) pairs.
 __device__ __forceinline__ int64_t resolve_row(const bz_embed_slot& s, int64_t id) {
@@ -251,13 +253,17 @@ __device__ __forceinline__ int64_t resolve_row(const bz_embed_slot& s, int64_t i
     const uint64_t rec = s.hash_buckets[h % s.hash_bucket_size];
     const uint32_t cnt = (uint32_t)(rec >> 40);
     const uint64_t* p = s.hash_pairs + ((rec & 0xffffffffffull) >> 3);
+    // (a pair in one load: the row number is there with the key, not a trip after it.  1000 x 24 lists of 6 keys, 400-byte
+    // rows 21.0 -> 19.5 us, 8000 x 24 lists of 48-byte rows 34.5 -> 30.4)
+    uint64_t row = ~0ull;
     for (uint32_t i = 0; i < cnt; ++i) {
-      if (p[2 * i] == key) {
-        const uint64_t row = p[2 * i + 1];
-        return row < (uint64_t)s.rows ? (int64_t)row : -1;
+      const u64x2a8 pair = *(const u64x2a8*)(p + 2 * i);
+      if (pair.x == key) {
+        row = pair.y;
+        break;
       }
     }
-    return -1;
+    return row < (uint64_t)s.rows ? (int64_t)row : -1;
   }
   return (id >= 0 && id < s.rows) ? id : -1;
 }
