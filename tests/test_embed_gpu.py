@@ -526,3 +526,27 @@ def test_table_of_more_than_2_to_24_rows_takes_the_plain_load_path(bz, oracle):
     assert variant != 0  # one row shape, ksum / kavg: the specialised kernel
     want = _run_oracle(oracle, [big, small], specs, inputs, batch, (col, cols))
     assert np.array_equal(_bits(got), _bits(want))
+
+
+@pytest.mark.parametrize("batch", [1, 2047, 2048, 2049, 4100, 16385, 20000])
+def test_scan_of_slots_at_the_edges_of_its_tiles(bz, batch):
+    """bz_segments_to_offsets_slots: one slot's scan is split into tiles of 2048 counts over up to 8 workgroups, the last of
+    which walks on; negative counts are zero, offsets stop at nnz, counts start at any element (no 16-byte alignment)."""
+    import torch
+    rng = np.random.default_rng(batch)
+    table = bz.DeviceTable(torch.ones((5, 4), device="cuda"))
+    items, want = [], []
+    for i, cap in enumerate((1.0, 0.6, 0.0)):
+        seg = rng.integers(-2, 9, batch).astype(np.int32)
+        total = int(np.maximum(seg, 0).sum())
+        nnz = int(total * cap)
+        held = _dev(np.concatenate([np.zeros(1 + i, np.int32), seg]))[1 + i:]
+        items.append(dict(table=table, ids=torch.zeros(max(nnz, 1), dtype=torch.int64, device="cuda"), nnz=nnz,
+                          values=torch.ones(max(nnz, 1), device="cuda"), segments=held, out=torch.zeros((batch, 4), device="cuda")))
+        want.append(np.minimum(np.concatenate([[0], np.cumsum(np.maximum(seg, 0).astype(np.int64))]), nnz))
+    print("case batch=%d" % batch, flush=True)
+    plan = bz.EmbeddingPlan(items, fused_scan=False)
+    plan.scan()
+    torch.cuda.synchronize()
+    for off, w in zip(plan.offsets, want):
+        assert np.array_equal(off.cpu().numpy(), w)

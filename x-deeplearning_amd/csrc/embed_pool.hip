@@ -53,11 +53,14 @@ constexpr int kUnroll = 4;  // rows in flight per lane group in the generic kern
 // ---------------------------------------------------------------------------------------------
 // segments -> offsets (exclusive scan), one workgroup per array
 // ---------------------------------------------------------------------------------------------
-constexpr int kScanItems = 8;  // counts per thread per tile -> 4096 per workgroup tile
-constexpr int kScanTile = kThreads * kScanItems;
-// a thread's kScanItems consecutive entries sit kScanItems + 1 apart from the next thread's: its walk over them does
-// not hit its neighbours' LDS banks
-__device__ __forceinline__ int scan_slot(int i) { return i + i / kScanItems; }
+// A wave holds kScanRows rows of 64 consecutive counts, one count a lane, so that every load and store is one coalesced
+// access and the scan runs within the registers: DPP scans of the rows, the rows' totals added up on the way, one barrier
+// for the waves' totals.  (Before, every thread owned a run of 8 counts and the layout was turned in 55 KB of LDS, five
+// barriers a tile of 4096 and a scan of six dependent trips to LDS: 200 slots x 8192 counts 9.0 us, 7.4-8.0 now.)
+constexpr int kScanThreads = 256;
+constexpr int kScanRows = 8;
+constexpr int kScanWaves = kScanThreads / bz::kWave;
+constexpr int kScanTile = kScanThreads * kScanRows;
 
 __device__ __forceinline__ int64_t wave_incl_scan(int64_t v, int lane) {
 #pragma unroll
@@ -68,93 +71,142 @@ __device__ __forceinline__ int64_t wave_incl_scan(int64_t v, int lane) {
   return v;
 }
 
-// Counts below zero are taken as zero and the running offset stops at `limit` (the length of the ids / values arrays),
+// All sums saturate at cap (< 2^31): every term is >= 0 and <= cap, so min(a + b, cap) is associative and gives the
+// clamped offsets whatever the order of the additions, in 32 bits.
+__device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b, uint32_t cap) {
+  const uint32_t t = a + b;  // a, b <= cap < 2^31: no wrap
+  return t < cap ? t : cap;
+}
+
+// Inclusive scan over the 64 lanes with data-parallel primitives (row_shr within rows of 16 lanes, then lane 15 and
+// lane 31 handed on to the following rows): a dozen VALU instructions, where the same scan through ds_bpermute
+// (__shfl_up) is six dependent trips to LDS per 32 bits.
+__device__ __forceinline__ uint32_t wave_scan_sat(uint32_t v, uint32_t cap) {
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false), cap);  // row_shr:1
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false), cap);  // row_shr:2
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false), cap);  // row_shr:4
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false), cap);  // row_shr:8
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false), cap);  // row_bcast:15 -> rows 1, 3
+  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false), cap);  // row_bcast:31 -> rows 2, 3
+  return v;
+}
+
+// the sums of a scan: 32 bits that saturate where the limit allows it, 64 bits without a limit else
+struct ScanSat {
+  typedef uint32_t T;
+  uint32_t cap;
+  __device__ T take(int32_t c) const { return (uint32_t)min(max(c, 0), (int)cap); }
+  __device__ T add(T a, T b) const { return sat_add(a, b, cap); }
+  __device__ T scan(T v, int) const { return wave_scan_sat(v, cap); }
+  __device__ T last(T v) const { return (uint32_t)__builtin_amdgcn_readlane((int)v, bz::kWave - 1); }
+  __device__ int64_t offset(T v) const { return (int64_t)v; }
+};
+struct ScanWide {
+  typedef int64_t T;
+  int64_t limit;
+  __device__ T take(int32_t c) const { return max(c, 0); }
+  __device__ T add(T a, T b) const { return a + b; }
+  __device__ T scan(T v, int lane) const { return wave_incl_scan(v, lane); }
+  __device__ T last(T v) const { return __shfl(v, bz::kWave - 1, bz::kWave); }
+  __device__ int64_t offset(T v) const { return v < limit ? v : limit; }
+};
+
+// Counts below zero are taken as zero and the running offset stops at the limit (the length of the ids / values arrays),
 // so no offset this scan produces points outside them.
-// Global memory is read and written one element per lane, consecutive lanes consecutive elements; the thread-owns-a-run
-// layout the scan wants exists only in LDS.  (With every thread loading and storing its own run directly, a wave's
-// access touched 64 lines for 256 or 512 bytes: 200 slots x 8192 counts took 19.5 us.)
 // Tiles [first_tile, first_tile + n_tiles) of the array (n_tiles < 0: all of them from first_tile on).  A workgroup that
 // does not start at tile 0 first adds up the counts before its first tile - all those loads are independent, so a slot's
 // scan split over several workgroups takes one tile's time, not the array's.
-__device__ void scan_segments(const int32_t* __restrict__ seg, int64_t* __restrict__ off, int64_t n, int64_t limit,
-                              int64_t first_tile = 0, int64_t n_tiles = -1) {
-  __shared__ int64_t wave_tot[kThreads / bz::kWave];
-  __shared__ int64_t carry_s;
-  __shared__ int32_t cnt_s[kScanTile + kThreads];
-  __shared__ int64_t off_s[kScanTile + kThreads];
+template <typename S>
+__device__ __forceinline__ void scan_tiles(const S sums, const int32_t* __restrict__ seg, int64_t* __restrict__ off, int64_t n,
+                                           int64_t first_tile, int64_t n_tiles, int64_t* lds) {
+  typedef typename S::T T;
+  T* tot = (T*)lds;  // [2][kScanWaves]: tiles take turns, so that one barrier a tile is enough
   const int tid = threadIdx.x;
-  const int lane = tid & (bz::kWave - 1);
-  const int wave = tid / bz::kWave;
+  const int lane = tid & (bz::kWave - 1), wave = tid / bz::kWave;
   const int64_t begin = first_tile * kScanTile;
   const int64_t end = (n_tiles < 0 || begin + n_tiles * kScanTile > n) ? n : begin + n_tiles * kScanTile;
   if (begin > n || (begin == n && n != 0)) return;  // nothing here; whoever scans the last tile writes off[n]
-  {
-    int64_t part = 0;
-    for (int64_t i = tid; i < begin; i += kThreads) part += max(seg[i], 0);
-    part = wave_incl_scan(part, lane);
-    if (lane == bz::kWave - 1) wave_tot[wave] = part;
-    __syncthreads();
-    if (tid == 0) {
-      int64_t c = 0;
-      for (int w = 0; w < kThreads / bz::kWave; ++w) c += wave_tot[w];
-      carry_s = c;
+  T carry = 0;
+  if (begin > 0) {
+    T part = 0;
+    for (int64_t i = 0; i < begin; i += kScanTile) {  // (begin is a whole number of tiles)
+      int32_t c[kScanRows];
+#pragma unroll
+      for (int k = 0; k < kScanRows; ++k) c[k] = seg[i + k * kScanThreads + tid];
+#pragma unroll
+      for (int k = 0; k < kScanRows; ++k) part = sums.add(part, sums.take(c[k]));
     }
+    part = sums.last(sums.scan(part, lane));
+    if (lane == 0) tot[kScanWaves + wave] = part;
     __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kScanWaves; ++w) carry = sums.add(carry, tot[kScanWaves + w]);
   }
-  for (int64_t base = begin; base < end; base += kScanTile) {
+  int turn = 0;
+  for (int64_t base = begin; base < end; base += kScanTile, turn ^= kScanWaves) {
+    const int64_t at = base + wave * (kScanRows * bz::kWave) + lane;
+    int32_t c[kScanRows];
+    T excl[kScanRows], run = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      const int j = k * kThreads + tid;
-      cnt_s[scan_slot(j)] = (base + j < n) ? max(seg[base + j], 0) : 0;
+    for (int k = 0; k < kScanRows; ++k) c[k] = at + k * bz::kWave < n ? seg[at + k * bz::kWave] : 0;
+#pragma unroll
+    for (int k = 0; k < kScanRows; ++k) {
+      const T v = sums.take(c[k]);
+      const T incl = sums.scan(v, lane);
+      // (saturated sums have no inverse: the sum before this lane is the scan's value one lane back)
+      T before = __shfl_up(incl, 1, bz::kWave);
+      if (lane == 0) before = 0;
+      excl[k] = sums.add(run, before);
+      run = sums.add(run, sums.last(incl));
     }
+    if (lane == 0) tot[turn + wave] = run;
     __syncthreads();
-    int32_t v[kScanItems];
+    T before = carry;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) v[k] = cnt_s[tid * (kScanItems + 1) + k];
-    int64_t local = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) local += v[k];
-    int64_t incl = wave_incl_scan(local, lane);
-    if (lane == bz::kWave - 1) wave_tot[wave] = incl;
-    __syncthreads();
-    int64_t before = carry_s;
-    for (int w = 0; w < wave; ++w) before += wave_tot[w];
-    int64_t run = before + incl - local;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      off_s[tid * (kScanItems + 1) + k] = run < limit ? run : limit;
-      run += v[k];
+    for (int w = 0; w < kScanWaves; ++w) {
+      const T t = tot[turn + w];
+      if (w < wave) before = sums.add(before, t);
+      carry = sums.add(carry, t);
     }
-    __syncthreads();
-    if (tid == kThreads - 1) carry_s = run;  // last thread's running total = total so far
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      const int j = k * kThreads + tid;
-      if (base + j < n) off[base + j] = off_s[scan_slot(j)];
-    }
-    __syncthreads();
+    for (int k = 0; k < kScanRows; ++k)
+      if (at + k * bz::kWave < n) off[at + k * bz::kWave] = sums.offset(sums.add(before, excl[k]));
   }
-  if (tid == 0 && end == n) off[n] = carry_s < limit ? carry_s : limit;
+  if (tid == 0 && end == n) off[n] = sums.offset(carry);
 }
 
-__global__ __launch_bounds__(kThreads) void bz_scan_segments_kernel(const int32_t* __restrict__ seg,
-                                                                    int64_t* __restrict__ off, int64_t n) {
-  scan_segments(seg, off, n, INT64_MAX);
+__device__ __forceinline__ void scan_segments(const int32_t* __restrict__ seg, int64_t* __restrict__ off, int64_t n, int64_t limit,
+                                              int64_t first_tile, int64_t n_tiles) {
+  __shared__ int64_t lds[2 * kScanWaves];
+  if (limit < (1ll << 31))
+    scan_tiles(ScanSat{(uint32_t)limit}, seg, off, n, first_tile, n_tiles, lds);
+  else
+    scan_tiles(ScanWide{limit}, seg, off, n, first_tile, n_tiles, lds);
+}
+
+// Grid (parts): part p scans tile p, the last part every tile from its own on.
+__global__ __launch_bounds__(kScanThreads) void bz_scan_segments_kernel(const int32_t* __restrict__ seg,
+                                                                        int64_t* __restrict__ off, int64_t n) {
+  scan_segments(seg, off, n, INT64_MAX, blockIdx.x, blockIdx.x + 1 == gridDim.x ? -1 : 1);
 }
 
 // ext_off != nullptr: slot i's offsets go to ext_off + i * ext_stride instead of slot.offsets (at most ext_stride - 1
 // samples of a slot are scanned, so a record whose batch disagrees with the plan cannot write past its share)
-// Grid (slots, parts): part p of a slot scans tiles p, or, for the last part, every tile from p on.
-__global__ __launch_bounds__(kThreads) void bz_scan_segments_slots_kernel(const bz_embed_slot* __restrict__ slots,
-                                                                          int64_t* __restrict__ ext_off, int64_t ext_stride) {
+// Grid (slots, parts): parts as above.
+__global__ __launch_bounds__(kScanThreads) void bz_scan_segments_slots_kernel(const bz_embed_slot* __restrict__ slots,
+                                                                              int64_t* __restrict__ ext_off, int64_t ext_stride) {
   const bz_embed_slot* s = &slots[blockIdx.x];
   const int64_t first = blockIdx.y, count = blockIdx.y + 1 == gridDim.y ? -1 : 1;
+  // (all of the record in one trip to memory)
+  const int32_t* seg = s->segments;
+  int64_t* off = s->offsets;
+  int64_t n = s->batch;
+  const int64_t nnz = s->nnz;
   if (ext_off != nullptr) {
-    const int64_t n = s->batch < ext_stride - 1 ? s->batch : ext_stride - 1;
-    scan_segments(s->segments, ext_off + (int64_t)blockIdx.x * ext_stride, n, s->nnz, first, count);
-  } else {
-    scan_segments(s->segments, s->offsets, s->batch, s->nnz, first, count);
+    off = ext_off + (int64_t)blockIdx.x * ext_stride;
+    n = n < ext_stride - 1 ? n : ext_stride - 1;
   }
+  scan_segments(seg, off, n, nnz, first, count);
 }
 
 // parts a slot's scan is split into: one per tile of the largest batch, at most 8 (a part re-reads the counts before it)
@@ -524,62 +576,52 @@ __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int6
 // the same for the specialised kernel, where lane group g of the workgroup owns sample b0 + g: every lane ends up with
 // its own segment [start, end) in registers
 // ---------------------------------------------------------------------------------------------
-// All sums saturate at cap = nnz (< 2^31 here; larger arrays take stage_offsets): every term is >= 0, so
-// min(a + b, cap) is associative and gives the clamped offsets whatever the order of the additions, in 32 bits.
-__device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b, uint32_t cap) {
-  const uint32_t t = a + b;  // a, b <= cap < 2^31: no wrap
-  return t < cap ? t : cap;
-}
+typedef int i32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // four counts, from any count on
 
-// Inclusive scan over the 64 lanes with data-parallel primitives (row_shr within rows of 16 lanes, then lane 15 and
-// lane 31 handed on to the following rows): a dozen VALU instructions, where the same scan through ds_bpermute
-// (__shfl_up) is six dependent trips to LDS per 32 bits.
-__device__ __forceinline__ uint32_t wave_scan_sat(uint32_t v, uint32_t cap) {
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false), cap);  // row_shr:1
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false), cap);  // row_shr:2
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false), cap);  // row_shr:4
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false), cap);  // row_shr:8
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false), cap);  // row_bcast:15 -> rows 1, 3
-  v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false), cap);  // row_bcast:31 -> rows 2, 3
-  return v;
-}
-
+// (sums saturate at cap = nnz, below 2^31 here; larger arrays take stage_offsets.  The counts before b0 in loads of four:
+// 26 slots x 16384 samples 66.6 -> 57.9 us with single loads, eight in flight, before)
 // start / end of sample b = b0 + g for every lane of lane group g (LPR lanes, g = tid / LPR); lanes of samples beyond
 // the batch get an empty segment.  Every thread of the workgroup calls it; one barrier.
 template <int LPR>
 __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, uint32_t* s_tot, int64_t* start, int64_t* end) {
-  constexpr int WAVES = kThreads / bz::kWave;
+  constexpr int THREADS = kThreads;
+  constexpr int WAVES = THREADS / bz::kWave;
+  static_assert(THREADS / LPR % 4 == 0, "the counts before a workgroup's first sample come in fours");
   const int tid = threadIdx.x;
   const int lane = tid & (bz::kWave - 1), wave = tid / bz::kWave;
   const int g = tid / LPR, l = tid % LPR;
   const int64_t b = b0 + g;
   const uint32_t cap = (uint32_t)s.nnz;
-  // this group's own count first (all its lanes ask for the same word), then the counts before b0, 8 loads in flight a
-  // thread: everything is requested before anything is used
+  // this group's own count first (all its lanes ask for the same word), then the counts before b0, four loads of four
+  // in flight a thread: everything is requested before anything is used
   const int32_t own = b < s.batch ? s.segments[b] : 0;
   // (b0 is below 2^31: batch is an int32.  A workgroup near the head of its slot has few counts before it: the rounds
-  // of 8 loads stop, for the whole workgroup, where b0 ends)
-  const uint32_t nb = (uint32_t)b0;
-  uint64_t part = 0;
-  for (uint32_t i0 = 0; i0 < nb; i0 += 8 * kThreads) {
-    int32_t c[8];
+  // stop, for the whole workgroup, where b0 ends)
+  const uint32_t quads = (uint32_t)b0 / 4;
+  const i32x4a4* before_b0 = (const i32x4a4*)s.segments;
+  uint32_t part = 0;
+  for (uint32_t i0 = 0; i0 < quads; i0 += 4 * THREADS) {
+    i32x4a4 c[4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t i = i0 + k * kThreads + tid;
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t i = i0 + k * THREADS + tid;
       c[k] = 0;
-      if (i0 + k * kThreads < nb) c[k] = s.segments[i < nb ? i : nb - 1];  // (uniform test; a lane past b0 reads the last count, masked below)
-      if (i >= nb) c[k] = 0;
+      if (i0 + k * THREADS < quads) c[k] = before_b0[i < quads ? i : quads - 1];  // (uniform test; a lane past b0 reads the last counts, dropped below)
+      if (i >= quads) c[k] = 0;
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) part += (uint32_t)max(c[k], 0);
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part = sat_add(part, (uint32_t)min(max(c[k][j], 0), (int)cap), cap);
+    }
   }
   const uint32_t mine = min((uint32_t)max(own, 0), cap);
   // the group's count sits in its last lane: after the scan that lane holds the inclusive sum and the group's other
   // lanes the exclusive one (they add nothing)
   const uint32_t scan = wave_scan_sat(l == LPR - 1 ? mine : 0u, cap);
-  const uint32_t before_b0 = wave_scan_sat((uint32_t)(part < cap ? part : cap), cap);
+  const uint32_t earlier = wave_scan_sat(part, cap);
   if (lane == bz::kWave - 1) {
-    s_tot[wave] = before_b0;
+    s_tot[wave] = earlier;
     s_tot[WAVES + wave] = scan;
   }
   __syncthreads();
@@ -1016,7 +1058,7 @@ int bz_embed_plan(bz_embed_slot* slots, int n_slots, bz_embed_launch* launch) {
 int bz_segments_to_offsets(const int32_t* segments, int64_t* offsets, int64_t n, bz_stream_t stream) {
   BZ_REQUIRE(offsets != nullptr && n >= 0 && (n == 0 || segments != nullptr), "bz_segments_to_offsets: null argument");
   BZ_REQUIRE(n <= (1ll << 24), "bz_segments_to_offsets: n=%lld exceeds 2^24", (long long)n);
-  hipLaunchKernelGGL(bz_scan_segments_kernel, dim3(1), dim3(kThreads), 0, bz::as_stream(stream), segments, offsets, n);
+  hipLaunchKernelGGL(bz_scan_segments_kernel, dim3(scan_parts(n)), dim3(kScanThreads), 0, bz::as_stream(stream), segments, offsets, n);
   BZ_LAUNCH_OK("bz_scan_segments_kernel");
   return BZ_OK;
 }
@@ -1024,7 +1066,7 @@ int bz_segments_to_offsets(const int32_t* segments, int64_t* offsets, int64_t n,
 int bz_segments_to_offsets_slots(const bz_embed_slot* slots_dev, int n_slots, bz_stream_t stream) {
   BZ_REQUIRE(slots_dev != nullptr && n_slots > 0, "bz_segments_to_offsets_slots: null argument or n_slots=%d", n_slots);
   // the batch sizes are in device memory: always 8 parts a slot; a part beyond its slot's batch returns at once
-  hipLaunchKernelGGL(bz_scan_segments_slots_kernel, dim3(n_slots, 8), dim3(kThreads), 0, bz::as_stream(stream), slots_dev,
+  hipLaunchKernelGGL(bz_scan_segments_slots_kernel, dim3(n_slots, 8), dim3(kScanThreads), 0, bz::as_stream(stream), slots_dev,
                      (int64_t*)nullptr, (int64_t)0);
   BZ_LAUNCH_OK("bz_scan_segments_slots_kernel");
   return BZ_OK;
@@ -1145,7 +1187,7 @@ int bz_embed_pool_static_scratch(const bz_embed_slot* slots_dev, const bz_embed_
   if (rc != BZ_OK) return rc;
   hipStream_t st = bz::as_stream(stream);
   // nothing to clear: the scan writes entries [0, batch] of every slot's share, the only ones the pooling kernel reads
-  hipLaunchKernelGGL(bz_scan_segments_slots_kernel, dim3(L.n_slots, scan_parts(L.max_batch)), dim3(kThreads), 0, st, slots_dev, off,
+  hipLaunchKernelGGL(bz_scan_segments_slots_kernel, dim3(L.n_slots, scan_parts(L.max_batch)), dim3(kScanThreads), 0, st, slots_dev, off,
                      stride);
   BZ_LAUNCH_OK("bz_scan_segments_slots_kernel");
   return launch_pool(slots_dev, L, off, stride, st);
