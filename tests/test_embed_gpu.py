@@ -550,3 +550,51 @@ def test_scan_of_slots_at_the_edges_of_its_tiles(bz, batch):
     torch.cuda.synchronize()
     for off, w in zip(plan.offsets, want):
         assert np.array_equal(off.cpu().numpy(), w)
+
+
+@pytest.mark.parametrize("kind,dim", [("f32", 4), ("f32", 100), ("f16", 14), ("f16", 64), ("i8", 16), ("i8", 30), ("i8", 64)])
+@pytest.mark.parametrize("keyed", [False, True])
+def test_pooling_walk_over_every_short_length(bz, oracle, kind, dim, keyed):
+    """Segments of 0 to 13 ids next to each other (the walk takes four a step, two steps in flight, and a wave goes as far as
+    its longest segment), steps whose values are all 1 between steps whose are not, counts that start on no 16 bytes, samples
+    before a workgroup's first in every number; offsets scanned, made in the launch, and made by the caller in no order."""
+    import torch
+    rng = np.random.default_rng(dim * 7 + len(kind))
+    batch, rows = 1031, 211
+    t = _make_table(rng, kind, rows, dim, keyed)
+    seg = ((np.arange(batch) * 5 + np.arange(batch) // 14) % 14).astype(np.int32)
+    nnz = int(seg.sum())
+    ids = rng.choice(np.concatenate([t["keys"], [-7, 12345]]), nnz) if keyed else rng.integers(-2, rows + 2, nnz)
+    vals = np.where(rng.random(nnz) < 0.02, 0.5, 1.0).astype(np.float32)
+    want = np.zeros((batch, dim), np.float32)
+    oracle.embed_get(oracle.Table(t["data"], scale=t.get("scale"), keys=t.get("keys")), ids.astype(np.int64), vals, seg, [(0, 0, 0, want, 0)])
+    table = bz.DeviceTable(t["data"], scale=t.get("scale"), keys=t.get("keys"))
+    held = _dev(np.concatenate([[0], seg]).astype(np.int32))[1:]
+    start = np.concatenate([[0], np.cumsum(seg)])
+    print("case kind=%s dim=%d keyed=%s" % (kind, dim, keyed), flush=True)
+    for form in ("fused", "scanned", "caller"):
+        out = torch.full((batch, dim), float("nan"), device="cuda")
+        plan = bz.EmbeddingPlan([dict(table=table, ids=_dev(ids.astype(np.int64)), values=_dev(vals), segments=held, out=out, udf=0)],
+                                fused_scan=form == "fused")
+        if form == "caller":  # offsets that go down from sample to sample here and there: every such pair is an empty segment
+            off = start.copy()
+            off[5:batch:97] = 0
+            plan.offsets[0].copy_(_dev(off))
+            plan.pool()
+            full = np.zeros((batch, dim), np.float32)
+            seg2 = np.maximum(off[1:] - off[:-1], 0).astype(np.int32)
+            for b in range(batch):
+                if off[b] >= off[b + 1]:
+                    continue
+                if off[b] == start[b] and off[b + 1] == start[b + 1]:
+                    full[b] = want[b]
+                else:
+                    one = np.zeros((1, dim), np.float32)
+                    oracle.embed_get(oracle.Table(t["data"], scale=t.get("scale"), keys=t.get("keys")), ids[off[b]:off[b + 1]].astype(np.int64),
+                                     vals[off[b]:off[b + 1]], seg2[b:b + 1], [(0, 0, 0, one, 0)])
+                    full[b] = one[0]
+        else:
+            plan.run()
+            full = want
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(out.cpu().numpy()), _bits(full)), form

@@ -23,9 +23,10 @@
 //   * with equal work per slot the slot index is a division, not a search;
 //   * the specialised ksum/kavg kernel walks a segment kBlockIds ids at a time: the lanes
 //     of a group load disjoint ids/values (one coalesced read), resolve them to rows,
-//     pass rows and values around with ds_bpermute, then issue the row loads before
-//     the first add.  The block is short on purpose: the memory-level parallelism
-//     comes from eight resident waves per SIMD, not from a deep unroll in each.
+//     pass the rows around as DPP operands, and the rows of a step are requested before
+//     those of the step before are added (walk).  The block is short on purpose: the
+//     memory-level parallelism comes from eight resident waves per SIMD, not from a deep
+//     unroll in each.
 // A generic kernel covers kassign, mixed slot shapes, rows wider than 64 chunks and
 // precomputed offsets.
 //
@@ -39,6 +40,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "bz_common.h"
 
@@ -48,6 +50,11 @@ namespace {
 
 constexpr int kThreads = 512;  // measured at 128 / 256 / 512 / 1024 on config 2: 14.7 / 13.5 / 13.3 / 13.4 us per launch,
                                // 127 / 131 / 135 / 129 M samples/s with eight serving threads
+// Workgroups of the specialised kernel when the offsets are given: they share nothing then, and smaller ones fill the chip
+// more evenly (200 slots x 8192 samples, 64 threads 166.5, 128 167.2, 256 168.2, 512 176 us; 1000 x 24 and 1024 x 26 shortest
+// lists 18.2 / 5.4 us at 256 against 17.5 / 6.6 at 64).
+constexpr int kOffsetThreads = 256;
+constexpr int kOffsetSplit = kThreads / kOffsetThreads;
 constexpr int kUnroll = 4;  // rows in flight per lane group in the generic kernel (8 held 118 VGPRs and was no faster)
 
 // ---------------------------------------------------------------------------------------------
@@ -290,6 +297,7 @@ __device__ __forceinline__ void accum_chunk(float (&acc)[RowTraits<DT>::kElems],
     for (int i = 0; i < 16; ++i) {
       const float w = __fmul_rn(scale, (float)(int)(int8_t)((r[i / 4] >> (8 * (i & 3))) & 0xffu));
       acc[i] = __fadd_rn(acc[i], UNIT ? w : __fmul_rn(value, w));
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -523,12 +531,13 @@ __device__ __forceinline__ void pool_zero(const bz_embed_slot& s, int64_t b, int
 // s_off[0..groups] <- exclusive offsets of samples b0 .. b0+groups (clipped to batch).
 // Every thread of the workgroup calls it; ends with a barrier.
 // `offsets`: the slot's precomputed offsets (slot.offsets, or its share of a buffer the launch brings), or nullptr.
+template <int THREADS = kThreads>
 __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int64_t* __restrict__ offsets, int64_t b0,
                                               int groups, int64_t* s_off, int64_t* s_part) {
   const int tid = threadIdx.x;
   const int lane = tid & (bz::kWave - 1), wave = tid / bz::kWave;
   if (offsets != nullptr) {
-    for (int t = tid; t <= groups; t += kThreads)
+    for (int t = tid; t <= groups; t += THREADS)
       if (b0 + t <= s.batch) {
         const int64_t o = offsets[b0 + t];
         s_off[t] = o < 0 ? 0 : (o < s.nnz ? o : s.nnz);  // caller-made offsets get the same bounds as the scan's
@@ -542,11 +551,11 @@ __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int6
   // (a negative count is taken as 0 and the offsets below stop at nnz: see bz_embed_slot.nnz)
   const int64_t mine = (tid < groups && b0 + tid < s.batch) ? (int64_t)max(s.segments[b0 + tid], 0) : 0;
   int64_t part = 0;
-  for (int64_t i0 = 0; i0 < b0; i0 += 8 * kThreads) {
+  for (int64_t i0 = 0; i0 < b0; i0 += 8 * THREADS) {
     int32_t c[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const int64_t i = i0 + k * kThreads + tid;
+      const int64_t i = i0 + k * THREADS + tid;
       c[k] = i < b0 ? max(s.segments[i], 0) : 0;
     }
 #pragma unroll
@@ -558,14 +567,14 @@ __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int6
   const int64_t incl = wave_incl_scan(mine, lane);
   if (lane == bz::kWave - 1) {
     s_part[wave] = base;
-    s_part[kThreads / bz::kWave + wave] = incl;
+    s_part[THREADS / bz::kWave + wave] = incl;
   }
   __syncthreads();
   int64_t before = 0;
 #pragma unroll
-  for (int w = 0; w < kThreads / bz::kWave; ++w) {
+  for (int w = 0; w < THREADS / bz::kWave; ++w) {
     before += s_part[w];
-    if (w < wave) before += s_part[kThreads / bz::kWave + w];
+    if (w < wave) before += s_part[THREADS / bz::kWave + w];
   }
   if (tid < groups) s_off[tid + 1] = (before + incl) < s.nnz ? (before + incl) : s.nnz;
   if (tid == 0) s_off[0] = before < s.nnz ? before : s.nnz;
@@ -582,9 +591,8 @@ typedef int i32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // four co
 // 26 slots x 16384 samples 66.6 -> 57.9 us with single loads, eight in flight, before)
 // start / end of sample b = b0 + g for every lane of lane group g (LPR lanes, g = tid / LPR); lanes of samples beyond
 // the batch get an empty segment.  Every thread of the workgroup calls it; one barrier.
-template <int LPR>
+template <int LPR, int THREADS>
 __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, uint32_t* s_tot, int64_t* start, int64_t* end) {
-  constexpr int THREADS = kThreads;
   constexpr int WAVES = THREADS / bz::kWave;
   static_assert(THREADS / LPR % 4 == 0, "the counts before a workgroup's first sample come in fours");
   const int tid = threadIdx.x;
@@ -651,9 +659,13 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
 // specialised ksum / kavg kernel: every slot has table dtype DT and LPR lanes per row
 // ---------------------------------------------------------------------------------------------
 constexpr int kBlockIds = 4;  // ids walked per step (measured at 2, 4, 8, 16: 4 is best or equal on segments of 1-4, 8 and 20 ids)
-// Above this many bytes of repeated count reads a separate scan launch (about 15 us with its gap) is cheaper than the
-// fused one: config 5 (200 slots x 256 workgroups x batch 8192: 840 MB) pools in 155 + 16 us with offsets against
-// 261 us fused; config 4 (26 MB) and config 2 (3 MB) stay fused.
+// When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
+// preamble a workgroup and, with long batches, the counts read again and again: above this many workgroups of 512 threads
+// of the specialised kernel, or above this many bytes of repeated reads.  Fused / scan + pool in us, by workgroups: 1600 (int8, 20 ids) 80 / 84, 1664
+// (26 slots x 8192 of 64-byte rows) 23 / 27, 3328 (16384) 57 / 59.5, 3840 (60 slots x 16384, 32-byte rows) 76 / 81, 5040 40 /
+// 41.7 and 75 / 70, 5120 38.5 / 34, 7560 (120 slots x 1000, 400-byte rows) 60.5 / 57, 15360 117 / 96, 25600 (200 slots x 8192)
+// 219 / 180.  A plan whose records may travel as kernel arguments needs no upload of them when fused: twice as many there.
+constexpr int64_t kScanFirstGroups = 5000;
 constexpr int64_t kScanFirstBytes = 128ll << 20;
 
 // Slot records handed over as kernel arguments: a workgroup then has its record after the one scalar load every
@@ -665,21 +677,262 @@ struct SlotPack {
 static_assert(sizeof(SlotPack) + 4 * 16 + 32 <= 4096, "the records and the other arguments fit the 4 KB kernel-argument segment");
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-constexpr uint32_t kBeyondTable = 0xF0000000u;  // a byte offset no table read through a buffer resource reaches
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t kBeyondTable = 0xF0000000u;  // a byte offset that nothing read through a buffer resource reaches
+constexpr int64_t kWalkIds = 1ll << 28;         // ids of one wave's segments: their byte offsets and twice kBeyondTable stay apart
+
+// Which lane of a row's group holds what of a step of kBlockIds ids: id u of the step is held by lane u % kSrc of every
+// quad of the group (u / kSrc: which of the lane's kPerLane ids), so that handing it to the group's lanes is one DPP
+// operand of the instruction that uses it.
+template <int LPR>
+struct StepShape {
+  static constexpr int kSrc = LPR < kBlockIds ? LPR : kBlockIds;
+  static constexpr int kPerLane = kBlockIds / kSrc;
+};
+
+// what the lane that holds id U of the step has in v
+template <int LPR, int U>
+__device__ __forceinline__ uint32_t of_id(uint32_t v) {
+  if constexpr (LPR == 1) return v;
+  constexpr int w = U % StepShape<LPR>::kSrc;
+  constexpr int ctrl = LPR >= 4 ? w * 0x55 : (w | w << 2 | (2 + w) << 4 | (2 + w) << 6);  // quad_perm
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
+}
+
+template <typename F>
+__device__ __forceinline__ void each_id(const F& f) {
+  static_assert(kBlockIds == 4, "");
+  f(std::integral_constant<int, 0>{});
+  f(std::integral_constant<int, 1>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{});
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000);
+}
+
+// ids of one step that a lane holds, on their way
+template <int LPR>
+struct StepIds {
+  u32x2 id[StepShape<LPR>::kPerLane];
+  float val[StepShape<LPR>::kPerLane];
+};
+
+// rows of one step, on their way
+template <int DT, int LPR>
+struct StepRows {
+  u32x4 raw[kBlockIds];
+  float val[StepShape<LPR>::kPerLane];    // of the ids the lane holds
+  uint32_t scale[StepShape<LPR>::kPerLane];  // int8 tables: of the same ids, a float's bits
+  uint64_t weighted;                      // the wave's lanes that hold a value other than 1 (uniform)
+};
 
 template <int DT, int LPR>
+__device__ __forceinline__ void add_rows(float (&acc)[RowTraits<DT>::kElems], const StepRows<DT, LPR>& st, float one) {
+  using S = StepShape<LPR>;
+  auto add = [&](auto u, auto unit) {
+    constexpr int U = decltype(u)::value, K = U / S::kSrc;
+    constexpr bool kUnit = decltype(unit)::value;
+    uint4 raw = make_uint4(st.raw[U].x, st.raw[U].y, st.raw[U].z, st.raw[U].w);
+    // (opaque, or the compiler moves the conversions that both forms begin with in front of them: 64 registers more)
+    if (!kUnit) asm volatile("" : "+v"(raw.x), "+v"(raw.y), "+v"(raw.z), "+v"(raw.w));
+    const float scale = DT == BZ_I8 ? __uint_as_float(of_id<LPR, U>(st.scale[K])) : 1.f;
+    accum_chunk<DT, kUnit>(acc, raw, scale, kUnit ? one : __uint_as_float(of_id<LPR, U>(__float_as_uint(st.val[K]))));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // two conditions that the compiler cannot tell to exclude each other: as two branches of one condition the forms' sums
+  // would live in registers of their own
+  uint64_t weighted = st.weighted;
+  asm volatile("" : "+s"(weighted));
+  if (st.weighted == 0) each_id([&](auto u) { add(u, std::true_type{}); });
+  if (weighted != 0) each_id([&](auto u) { add(u, std::false_type{}); });
+}
+
+// The walk over a segment: every operand comes through a buffer resource (the hardware checks every access and returns
+// zeros beyond the end), so that what a lane does not need is asked for beyond the end and no load sits under a branch:
+// the loop is straight-line code that the whole wave runs as often as its longest segment takes, and the rows of a step
+// are under way while those of the step before are added up.  (Waits count outstanding loads in order: after a join of
+// a path with loads and one without, the compiler waits for all of them.)
+// Measured with this walk, before / after: 26 slots x 2048 of 8 ids, 64-byte rows 9.0 /
+// 8.8 us, half the vector instructions; with offsets given 16384 samples 48.4 / 45.9, 200 slots x 8192 of 2.5 ids, 128-byte
+// rows 181 / 157 to 168; int8 rows of 64, 20 ids, 83 / 80; eight serving threads 15.2 / 14.9 us a pass of 2048.  Rows that
+// are found in the caches are bound by the lanes' idle turns (a wave walks as far as its longest segment) and, int8, by the
+// three instructions an element takes (90 % of the vector units' time); rows that are not by memory, 4.7 TB/s of lines.
+// Positions are relative to `first`, the wave's first id; n ids from position `from` on.
+template <int DT, int LPR, bool HASH>
+__device__ __forceinline__ void walk(const bz_embed_slot& s, int64_t first, uint32_t from, int n, int l, float (&acc)[RowTraits<DT>::kElems]) {
+  using S = StepShape<LPR>;
+  constexpr int CE = RowTraits<DT>::kElems;
+  const int q = l % S::kSrc;
+  const int lane = threadIdx.x & (bz::kWave - 1);
+  const int nchunks = (s.dim + CE - 1) / CE;
+  const uint32_t at = l < nchunks ? (uint32_t)l * 16u : 0u;  // (a lane without a chunk reads the group's first and drops it)
+  const int64_t left = s.nnz - first;
+  const uint32_t avail = left < kWalkIds ? (uint32_t)left : (uint32_t)kWalkIds;
+  const __amdgpu_buffer_rsrc_t ids = buffer_of(s.ids + first, avail * 8u), values = buffer_of(s.values + first, avail * 4u);
+  const __amdgpu_buffer_rsrc_t table = buffer_of(s.table, (uint32_t)(s.rows * (int64_t)s.pitch));
+  const uint32_t scale_pitch = s.scale_pitch != 0 ? (uint32_t)s.scale_pitch : 4u;
+  const __amdgpu_buffer_rsrc_t scales = buffer_of(s.row_scale, DT == BZ_I8 ? (uint32_t)(s.rows - 1) * scale_pitch + 4u : 0u);
+  float one = 1.f;  // (opaque: see accum_chunk)
+  asm volatile("" : "+v"(one));
+  // with a hash index only the group's first quad holds ids: a probe is a request of its own
+  const bool holds = !HASH || LPR <= 4 || l < S::kSrc;
+  uint32_t pos = (from + (uint32_t)q) * 4u;
+  int rest = holds ? n - q : 0;  // ids from this lane's first one of the step on
+  StepIds<LPR> next;
+  auto fetch = [&]() {
+#pragma unroll
+    for (int k = 0; k < S::kPerLane; ++k) {
+      const uint32_t o = k * S::kSrc < rest ? pos + 4u * k * S::kSrc : kBeyondTable;
+      next.id[k] = __builtin_amdgcn_raw_buffer_load_b64(ids, (int)(o << 1), 0, 0);
+      next.val[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(values, (int)o, 0, 0));
+    }
+    pos += 4u * kBlockIds;
+  };
+  auto request = [&](StepRows<DT, LPR>& st) {
+    uint32_t off[S::kPerLane], soff[S::kPerLane];
+    bool unit = true;
+#pragma unroll
+    for (int k = 0; k < S::kPerLane; ++k) {
+      const uint64_t id = (uint64_t)next.id[k].y << 32 | next.id[k].x;
+      bool ok = k * S::kSrc < rest;
+      uint32_t row = (uint32_t)id;
+      if constexpr (HASH) {
+        const int64_t r = ok ? resolve_row(s, (int64_t)id) : -1;
+        ok = r >= 0;
+        row = (uint32_t)r;
+      } else {
+        ok = ok && id < (uint64_t)s.rows;
+      }
+      uint32_t at_row = __umul24(row, (uint32_t)s.pitch), at_scale = DT == BZ_I8 ? __umul24(row, scale_pitch) : 0u;
+      float val = next.val[k];
+      // (opaque, or the selects below become a divergent branch, and every uniform branch of the loop with them a pair
+      // of masked blocks with sums of their own)
+      asm volatile("" : "+v"(at_row), "+v"(at_scale), "+v"(val));
+      off[k] = ok ? at_row : kBeyondTable;
+      if (DT == BZ_I8) soff[k] = ok ? at_scale : kBeyondTable;
+      // an id without a row contributes a zero row (times the value 1): adding +0 leaves the running sum as it is (the
+      // sum starts at +0 and so is never -0)
+      st.val[k] = ok ? val : 1.f;
+      unit &= st.val[k] == 1.f;
+    }
+    st.weighted = __builtin_amdgcn_ballot_w64(!unit);
+    if constexpr (HASH && LPR > 4) {
+#pragma unroll
+      for (int k = 0; k < S::kPerLane; ++k) {
+        off[k] = (uint32_t)__shfl((int)off[k], lane - l + q, bz::kWave);
+        if (DT == BZ_I8) soff[k] = (uint32_t)__shfl((int)soff[k], lane - l + q, bz::kWave);
+        st.val[k] = __shfl(st.val[k], lane - l + q, bz::kWave);
+      }
+    }
+    rest -= kBlockIds;
+    fetch();
+    each_id([&](auto u) {
+      constexpr int U = decltype(u)::value, K = U / S::kSrc;
+      st.raw[U] = __builtin_amdgcn_raw_buffer_load_b128(table, (int)(of_id<LPR, U>(off[K]) + at), 0, 0);
+    });
+    if (DT == BZ_I8) {
+#pragma unroll
+      for (int k = 0; k < S::kPerLane; ++k) st.scale[k] = __builtin_amdgcn_raw_buffer_load_b32(scales, (int)soff[k], 0, 0);
+    }
+    asm volatile("" ::: "memory");  // (the loads stay in this order on every path, or the loop's waits count too many)
+  };
+  int steps = n;
+#pragma unroll
+  for (int d = bz::kWave / 2; d >= LPR; d >>= 1) steps = max(steps, __shfl_xor(steps, d, bz::kWave));
+  steps = (__builtin_amdgcn_readfirstlane(steps) + kBlockIds - 1) / kBlockIds;
+  if (steps <= 0) return;
+  StepRows<DT, LPR> a, b;
+  fetch();
+  request(a);
+  if constexpr (HASH) {  // (a probe's own waits are for everything before it: nothing to overlap)
+    for (;;) {
+      add_rows<DT, LPR>(acc, a, one);
+      if (--steps == 0) return;
+      request(a);
+    }
+  }
+  for (; steps > 2; steps -= 2) {
+    request(b);
+    add_rows<DT, LPR>(acc, a, one);
+    request(a);
+    add_rows<DT, LPR>(acc, b, one);
+  }
+  if (steps == 2) {
+    request(b);
+    add_rows<DT, LPR>(acc, a, one);
+    a = b;
+  }
+  add_rows<DT, LPR>(acc, a, one);
+}
+
+// the same for tables and segments beyond what buffer resources address: plain loads under branches
+template <int DT, int LPR>
+__device__ __forceinline__ void walk_plain(const bz_embed_slot& s, int64_t start, int64_t end, int l, float (&acc)[RowTraits<DT>::kElems]) {
+  using S = StepShape<LPR>;
+  constexpr int CE = RowTraits<DT>::kElems;
+  const int gbase = (threadIdx.x & (bz::kWave - 1)) - l;  // first lane of this group within the wave
+  const bool has_chunk = l < (s.dim + CE - 1) / CE;
+  const char* table = (const char*)s.table + (int64_t)l * 16;
+  // the next step's ids are requested before this step's rows, so the two round trips overlap
+  int64_t id_next[S::kPerLane];  // raw ids: resolved to rows only when consumed, so the wait lands after the row loads
+  float val_next[S::kPerLane];
+  auto fetch_ids = [&](int64_t j) {
+#pragma unroll
+    for (int k = 0; k < S::kPerLane; ++k) {
+      const int idx = k * S::kSrc + l;
+      id_next[k] = -1;
+      val_next[k] = 0.f;
+      if (l < S::kSrc && idx < end - j) {
+        id_next[k] = s.ids[j + idx];
+        val_next[k] = s.values[j + idx];
+      }
+    }
+  };
+  if (start < end) fetch_ids(start);
+  for (int64_t j = start; j < end; j += kBlockIds) {
+    int row_own[S::kPerLane];
+    float val_own[S::kPerLane];
+#pragma unroll
+    for (int k = 0; k < S::kPerLane; ++k) {
+      row_own[k] = (l < S::kSrc && k * S::kSrc + l < end - j) ? (int)resolve_row(s, id_next[k]) : -1;
+      val_own[k] = row_own[k] >= 0 ? val_next[k] : 1.f;
+    }
+    if (j + kBlockIds < end) fetch_ids(j + kBlockIds);
+    float val[kBlockIds];
+    uint4 raw[kBlockIds];
+    float sc[kBlockIds];
+#pragma unroll
+    for (int u = 0; u < kBlockIds; ++u) {
+      const int row = __shfl(row_own[u / S::kSrc], gbase + (u % S::kSrc), bz::kWave);
+      val[u] = __shfl(val_own[u / S::kSrc], gbase + (u % S::kSrc), bz::kWave);
+      raw[u] = make_uint4(0, 0, 0, 0);
+      sc[u] = 1.f;
+      if (has_chunk && row >= 0) {
+        raw[u] = *(const uint4*)(table + (int64_t)row * s.pitch);
+        if (DT == BZ_I8) sc[u] = load_scale(s, row);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kBlockIds; ++u) {
+      accum_chunk<DT, false>(acc, raw[u], sc[u], val[u]);
+      __builtin_amdgcn_sched_barrier(0);  // (all conversions of a step's int8 rows at once would hold 64 more registers)
+    }
+  }
+}
+
+template <int DT, int LPR, int THREADS>
 __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0, const int64_t* __restrict__ offsets) {
   constexpr int CE = RowTraits<DT>::kElems;
-  constexpr int GROUPS = kThreads / LPR;
-  constexpr int SRC = LPR < kBlockIds ? LPR : kBlockIds;  // lanes of a group that fetch ids
-  constexpr int KPL = kBlockIds / SRC;                    // ids fetched per such lane
+  constexpr int GROUPS = THREADS / LPR;
   __shared__ int64_t s_off[GROUPS + 1];
-  __shared__ int64_t s_part[2 * kThreads / bz::kWave];
+  __shared__ int64_t s_part[2 * THREADS / bz::kWave];
   const int tid = threadIdx.x;
   const int g = tid / LPR, l = tid % LPR;
   int64_t start, end;
   if (offsets == nullptr && s.nnz < (1ll << 31)) {
-    own_segment<LPR>(s, b0, (uint32_t*)s_part, &start, &end);
+    own_segment<LPR, THREADS>(s, b0, (uint32_t*)s_part, &start, &end);
   } else if (offsets != nullptr) {
     // every lane of a group asks for its sample's two offsets itself (one address a group): nothing goes through LDS
     // and no wave waits for another's.  Caller-made offsets get the same bounds as the scan's.
@@ -688,103 +941,30 @@ __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0,
     start = o0 < 0 ? 0 : (o0 < s.nnz ? o0 : s.nnz);
     end = o1 < 0 ? 0 : (o1 < s.nnz ? o1 : s.nnz);
   } else {
-    stage_offsets(s, offsets, b0, GROUPS, s_off, s_part);
+    stage_offsets<THREADS>(s, offsets, b0, GROUPS, s_off, s_part);
     start = s_off[g];
     end = s_off[g + 1];
   }
   const int64_t b = b0 + g;
   if (b >= s.batch) return;
-  const int nchunks = (s.dim + CE - 1) / CE;
-  const bool has_chunk = l < nchunks;
-  const int gbase = (tid & (bz::kWave - 1)) - l;  // first lane of this group within the wave
-  const char* table = (const char*)s.table + (int64_t)l * 16;
   float acc[CE];
 #pragma unroll
   for (int i = 0; i < CE; ++i) acc[i] = 0.f;
-  float one = 1.f;  // (opaque: see accum_chunk)
-  asm volatile("" : "+v"(one));
-  // fp32 / fp16 tables of up to 2^24 rows and 3.75 GB are read through a buffer resource: the hardware checks every
-  // access against the table's size and returns zeros beyond it, which is what a missing row contributes.  (Measured:
-  // config 2's launch 11.9 -> 11.7 us.  Not for int8 tables: with the rows and their scales through buffer resources
-  // config 4's launch took 97-110 us against 90-92 with plain loads under a branch.)
-  const bool by_buffer = DT != BZ_I8 && s.rows <= (1ll << 24) && (uint64_t)s.rows * (uint64_t)s.pitch <= (uint64_t)kBeyondTable &&
-                         s.pitch < (1 << 24);
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)s.table, 0, by_buffer ? (int)(uint32_t)(s.rows * (int64_t)s.pitch) : 0, 0x00020000);
-  // each fetching lane takes ids j + k*SRC + l: one coalesced read per k for the whole group.  The
-  // next step's ids are requested before this step's rows, so the two round trips overlap.
-  int64_t id_next[KPL];  // raw ids: resolved to rows only when consumed, so the wait lands after the row loads
-  float val_next[KPL];
-  auto fetch_ids = [&](int64_t j) {
-    const int cnt = (int)((end - j) < kBlockIds ? (end - j) : kBlockIds);
-#pragma unroll
-    for (int k = 0; k < KPL; ++k) {
-      const int idx = k * SRC + l;
-      id_next[k] = -1;  // resolves to "absent" on both the direct and (as a never-stored key) the hash path
-      val_next[k] = 0.f;
-      if (l < SRC && idx < cnt) {
-        id_next[k] = s.ids[j + idx];
-        val_next[k] = s.values[j + idx];
-      }
-    }
-  };
-  if (start < end) fetch_ids(start);
-  for (int64_t j = start; j < end; j += kBlockIds) {
-    const int cnt = (int)((end - j) < kBlockIds ? (end - j) : kBlockIds);
-    int row_own[KPL];
-    float val_own[KPL];
-#pragma unroll
-    for (int k = 0; k < KPL; ++k) {
-      row_own[k] = (l < SRC && k * SRC + l < cnt) ? (int)resolve_row(s, id_next[k]) : -1;
-      // an id without a row contributes a zero row (times the value 1): adding +0 leaves the running sum as it is
-      // (the sum starts at +0 and so is never -0), which lets the accumulation below run without the row numbers
-      val_own[k] = row_own[k] >= 0 ? val_next[k] : 1.f;
-    }
-    if (j + kBlockIds < end) fetch_ids(j + kBlockIds);
-    // ids that carry no weight (value 1, the usual case) take the one-rounding form, when that holds for every lane of
-    // the wave: decided on the lanes' own values, before anything is handed round, so that the values need not be
-    bool unit_own = true;
-#pragma unroll
-    for (int k = 0; k < KPL; ++k) unit_own &= val_own[k] == 1.f;
-    const bool unit = __all(unit_own);
-    int row[kBlockIds];
-    float val[kBlockIds];
-    uint4 raw[kBlockIds];
-    float sc[kBlockIds];
-#pragma unroll
-    for (int u = 0; u < kBlockIds; ++u) row[u] = __shfl(row_own[u / SRC], gbase + (u % SRC), bz::kWave);
-    if (!unit) {
-#pragma unroll
-      for (int u = 0; u < kBlockIds; ++u) val[u] = __shfl(val_own[u / SRC], gbase + (u % SRC), bz::kWave);
-    }
-    if (by_buffer) {
-      // no branch round a load, no zero fill, one multiply-add per address: a row that is not there (row[u] is -1 beyond
-      // cnt and for ids without a row) is asked for beyond the table's end and comes back as zeros
-#pragma unroll
-      for (int u = 0; u < kBlockIds; ++u) {
-        const uint32_t off = (has_chunk && row[u] >= 0) ? __umul24((uint32_t)row[u], (uint32_t)s.pitch) + (uint32_t)l * 16u : kBeyondTable;
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
-        raw[u] = make_uint4(v.x, v.y, v.z, v.w);
-        sc[u] = 1.f;
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < kBlockIds; ++u) {
-        raw[u] = make_uint4(0, 0, 0, 0);
-        sc[u] = 1.f;
-        if (has_chunk && row[u] >= 0) {
-          raw[u] = *(const uint4*)(table + (int64_t)row[u] * s.pitch);
-          if (DT == BZ_I8) sc[u] = load_scale(s, row[u]);
-        }
-      }
-    }
-    if (unit) {
-#pragma unroll
-      for (int u = 0; u < kBlockIds; ++u) accum_chunk<DT, true>(acc, raw[u], sc[u], one);
-    } else {
-#pragma unroll
-      for (int u = 0; u < kBlockIds; ++u) accum_chunk<DT, false>(acc, raw[u], sc[u], val[u]);
-    }
+  // the wave's first id: offsets never decrease when the scan makes them (caller-made ones may, and take the other walk)
+  const int64_t first = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)start) |
+                        (int64_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)start >> 32)) << 32;
+  const bool near = __all(start >= first && end - first < kWalkIds);
+  const bool fits = s.rows <= (1ll << 24) && s.pitch < (1 << 24) && (uint64_t)s.rows * (uint64_t)s.pitch <= (uint64_t)kBeyondTable &&
+                    (DT != BZ_I8 || (s.scale_pitch < (1 << 24) && (uint64_t)s.rows * (uint64_t)(uint32_t)s.scale_pitch <= (uint64_t)kBeyondTable));
+  if (near && fits) {
+    const uint32_t from = (uint32_t)(start - first);
+    const int n = (int)(end - start);
+    if (s.hash_buckets != nullptr)
+      walk<DT, LPR, true>(s, first, from, n, l, acc);
+    else
+      walk<DT, LPR, false>(s, first, from, n, l, acc);
+  } else {
+    walk_plain<DT, LPR>(s, start, end, l, acc);
   }
   if (s.udf == BZ_AVG) {
     const int64_t num = end - start;
@@ -794,24 +974,24 @@ __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0,
       for (int i = 0; i < CE; ++i) acc[i] = __fmul_rn(acc[i], inv);
     }
   }
-  if (has_chunk) {
-    const int e0 = l * CE;
+  const int e0 = l * CE;
+  if (e0 < s.dim) {
     const int nvalid = (s.dim - e0) < CE ? (s.dim - e0) : CE;
     store_elems<CE>(s.out, b * s.out_stride + e0, acc, nvalid, s.out_dtype);
   }
 }
 
-template <int DT, int LPR>
-__global__ __launch_bounds__(kThreads) void bz_embed_pool_kernel(const bz_embed_slot* __restrict__ slots, int n_slots,
+template <int DT, int LPR, int THREADS>
+__global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_slot* __restrict__ slots, int n_slots,
                                                                  int total_wg, int wg_per_xcd, int wg_per_slot,
                                                                  const int64_t* __restrict__ ext_off, int64_t ext_stride) {
-  constexpr int GROUPS = kThreads / LPR;
+  constexpr int GROUPS = THREADS / LPR;
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = slots[si];
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
-  pool_samples<DT, LPR>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
+  pool_samples<DT, LPR, THREADS>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
 }
 
 template <int DT, int LPR>
@@ -823,7 +1003,7 @@ __global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(const Slot
   const int si = v / wg_per_slot;
   const bz_embed_slot s = pack.s[si];
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
-  pool_samples<DT, LPR>(s, b0, s.offsets);
+  pool_samples<DT, LPR, kThreads>(s, b0, s.offsets);
 }
 
 __device__ __forceinline__ int chunk_elems(int dt) { return dt == BZ_F32 ? 4 : (dt == BZ_F16 ? 8 : 16); }
@@ -1047,7 +1227,8 @@ int bz_embed_plan(bz_embed_slot* slots, int n_slots, bz_embed_launch* launch) {
   // the fused scan reads, per workgroup, the counts before its first sample: on average batch/2 counts of 4 bytes
   int64_t prefix_bytes = 0;
   for (int i = 0; i < n_slots; ++i) prefix_bytes += (int64_t)slots[i].wg_count * slots[i].batch * 2;
-  launch->scan_first = (launch->fused_scan && prefix_bytes > kScanFirstBytes) ? 1 : 0;
+  const int64_t most = n_slots <= BZ_EMBED_ARG_SLOTS ? 2 * kScanFirstGroups : kScanFirstGroups;
+  launch->scan_first = (launch->fused_scan && ((launch->variant != 0 && total > most) || prefix_bytes > kScanFirstBytes)) ? 1 : 0;
   int32_t max_batch = 0;
   for (int i = 0; i < n_slots; ++i) max_batch = slots[i].batch > max_batch ? slots[i].batch : max_batch;
   launch->max_batch = max_batch;
@@ -1089,9 +1270,16 @@ static int launch_pool(const bz_embed_slot* slots_dev, const bz_embed_launch& L,
   BZ_REQUIRE(L.wg_per_slot > 0 && (int64_t)L.wg_per_slot * L.n_slots == L.total_wg,
              "bz_embed_pool: variant %#x needs equal work per slot", L.variant);
   const int dt = L.variant >> 8, lpr = L.variant & 0xff;
-#define BZ_POOL(DT, LPR)                                                                                             \
-  hipLaunchKernelGGL((bz_embed_pool_kernel<DT, LPR>), grid, block, 0, st, slots_dev, L.n_slots, L.total_wg, per_xcd, \
-                     L.wg_per_slot, ext_off, ext_stride)
+  // with offsets given: smaller workgroups, each with its share of a planned workgroup's samples
+  const bool scanned = ext_off != nullptr || !L.fused_scan;
+  const int per_xcd_scanned = (kOffsetSplit * L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
+#define BZ_POOL(DT, LPR)                                                                                                        \
+  if (scanned)                                                                                                                  \
+    hipLaunchKernelGGL((bz_embed_pool_kernel<DT, LPR, kOffsetThreads>), dim3(per_xcd_scanned * bz::kNumXcd), dim3(kOffsetThreads), 0,  \
+                       st, slots_dev, L.n_slots, kOffsetSplit * L.total_wg, per_xcd_scanned, kOffsetSplit * L.wg_per_slot, ext_off, ext_stride);             \
+  else                                                                                                                          \
+    hipLaunchKernelGGL((bz_embed_pool_kernel<DT, LPR, kThreads>), grid, block, 0, st, slots_dev, L.n_slots, L.total_wg, per_xcd, \
+                       L.wg_per_slot, ext_off, ext_stride)
 #define BZ_POOL_LPR(DT)                                                                      \
   switch (lpr) {                                                                             \
     case 1: BZ_POOL(DT, 1); break;                                                           \
