@@ -598,3 +598,49 @@ def test_pooling_walk_over_every_short_length(bz, oracle, kind, dim, keyed):
             full = want
         torch.cuda.synchronize()
         assert np.array_equal(_bits(out.cpu().numpy()), _bits(full)), form
+
+
+@pytest.mark.parametrize("kind,dims", [("f32", (16, 14, 13)), ("f32", (100, 67, 80)), ("f16", (18, 32, 31)), ("f16", (8, 3, 7)), ("f16", (13, 16, 15)),
+                                       ("f16", (200, 130, 256)), ("i8", (100, 66, 128)), ("i8", (64, 40, 33)), ("i8", (9, 16, 1)), ("i8", (30, 17, 32))])
+@pytest.mark.parametrize("keyed", [False, True])
+@pytest.mark.parametrize("out_dtype", [np.float32, np.float16])
+def test_kassign_beside_sums_of_one_row_shape(bz, oracle, kind, dims, keyed, out_dtype):
+    """kAssign items from either end and sums in one launch, slots of one table type and lane count: rows whose last chunk is
+    partial or whose lane group has lanes without a chunk, columns on every alignment, runs of four positions cut by the
+    truncation and by samples shorter than it, empty samples, values of 1 and others, different batches a slot."""
+    import torch
+    rng = np.random.default_rng(sum(dims) + len(kind) + keyed)
+    out_t = torch.float32 if out_dtype == np.float32 else torch.float16
+    tables = [_make_table(rng, kind, 150 + 10 * i, d, keyed) for i, d in enumerate(dims)]
+    dts = [bz.DeviceTable(t["data"], scale=t.get("scale"), keys=t.get("keys")) for t in tables]
+    items, checks = [], []
+    for i, (ti, udf, tdir, trunc, batch) in enumerate([(0, 2, 0, 7, 301), (1, 2, 1, 5, 301), (2, 0, 0, 0, 301), (1, 2, 0, 1, 64), (0, 1, 0, 0, 1030),
+                                                       (2, 2, 1, 50, 37)]):
+        t, dim = tables[ti], dims[ti]
+        seg = rng.integers(0, 11, batch).astype(np.int32)
+        seg[rng.integers(0, batch, batch // 5)] = 0
+        nnz = int(seg.sum())
+        ids = (rng.choice(np.concatenate([t["keys"], [-7, 12345]]), nnz) if keyed else rng.integers(-2, t["data"].shape[0] + 2, nnz)).astype(np.int64)
+        vals = np.ones(nnz, np.float32) if i % 2 == 0 else np.where(rng.random(nnz) < 0.3, -0.75, 1.0).astype(np.float32)
+        width = dim * trunc if udf == 2 else dim
+        col = i % 4
+        out = torch.full((batch, width + 5), float("nan"), dtype=out_t, device="cuda")
+        items.append(dict(table=dts[ti], ids=_dev(ids), values=_dev(vals), segments=_dev(seg), out=out, col=col, udf=udf, trunc_dir=tdir, trunc_num=trunc))
+        want = np.full((batch, width + 5), np.nan, np.float32)
+        want[:, col:col + width] = 0
+        oracle.embed_get(oracle.Table(t["data"], scale=t.get("scale"), keys=t.get("keys")), ids, vals, seg, [(udf, tdir, trunc, want, col)])
+        checks.append((out, want))
+    print("case kind=%s dims=%s keyed=%s out=%s" % (kind, dims, keyed, out_dtype.__name__), flush=True)
+    for fused, args in ((True, False), (False, False), (True, True)):
+        for out, _ in checks:
+            out.fill_(float("nan"))
+        plan = bz.EmbeddingPlan(items, fused_scan=fused)
+        assert plan.launch.variant == 0 and plan.launch.shape != 0
+        plan.pool_args() if args else plan.run()
+        torch.cuda.synchronize()
+        for i, (out, want) in enumerate(checks):
+            got = out.cpu().numpy()
+            ref = want.astype(out_dtype)
+            assert np.array_equal(np.isnan(got), np.isnan(ref)), (fused, args, i)
+            ok = ~np.isnan(ref)
+            assert np.array_equal(_bits(got[ok]), _bits(ref[ok])), (fused, args, i)

@@ -47,7 +47,7 @@ class FeedRows(C.Structure):
 
 class EmbedLaunch(C.Structure):
     _fields_ = [("n_slots", C.c_int32), ("total_wg", C.c_int32), ("wg_per_slot", C.c_int32), ("variant", C.c_int32),
-                ("fused_scan", C.c_int32), ("scan_first", C.c_int32), ("max_batch", C.c_int32), ("reserved_", C.c_int32)]
+                ("fused_scan", C.c_int32), ("scan_first", C.c_int32), ("max_batch", C.c_int32), ("shape", C.c_int32)]
 
 
 class FcDesc(C.Structure):
