@@ -537,3 +537,64 @@ def test_sibling_embedding_operators_share_one_launch():
         assert g1["q"].any() and g1["his"].any()
         for k in g1:
             np.testing.assert_array_equal(g1[k], g0[k], err_msg=k)
+
+
+@pytest.mark.parametrize("batch,T,dim,n1,n2", [(1, 1, 8, 80, 40), (31, 1, 16, 80, 40), (11, 3, 7, 17, 16), (16, 2, 18, 80, 40), (400, 30, 12, 50, 24),
+                                               (9, 23, 16, 96, 48), (300, 29, 5, 9, 64), (64, 5, 18, 96, 64)])
+def test_fp32_attention_mlp_in_one_launch_equals_layer_by_layer(batch, T, dim, n1, n2):
+    """fp32: the attention input, its two layers and the score in one launch against the operators one by one
+    (fuse_concat_into_fc: 0) and a 64-bit product.  Rows that fill no whole tile of 32, odd widths of x and y, columns that
+    fill no block of 16, more tiles than CUs, and weights that do not fit the launch's LDS (the last: layer by layer again)."""
+    import json
+    import torch
+    import din_model
+    rng = np.random.default_rng(batch + T + dim)
+    cfg = din_model.Config3(batch=batch, rows=3000, T=T)
+    cfg.dim, d3 = dim, 3 * dim
+    weights = {}
+    for tag, layers in (("att", (4 * d3, n1, n2, 1)), ("main", (3 * d3, 200, 80, 2))):
+        weights[tag] = [dict(w=rng.standard_normal((k, n)).astype(np.float32) / np.float32(np.sqrt(k)), b=rng.standard_normal(n).astype(np.float32) * np.float32(0.1),
+                             gamma=rng.standard_normal(n).astype(np.float32) * np.float32(0.1), mean=rng.standard_normal(n).astype(np.float32) * np.float32(0.1),
+                             var=rng.uniform(0.5, 1.5, n).astype(np.float32)) for k, n in zip(layers, layers[1:])]
+    tables = [torch.from_numpy(rng.standard_normal((3000, dim)).astype(np.float32)).cuda() for _ in din_model.KINDS]
+    seg = rng.integers(1, T + 1, batch).astype(np.int32)
+    nnz = int(seg.sum())
+    feed = {"mask": (np.arange(T)[None, :] < seg[:, None]).astype(np.float32).reshape(batch, T, 1)}
+    for kind in din_model.KINDS:
+        for fg, s, n in ((kind, np.ones(batch, np.int32), batch), (kind + "_his", seg, nnz)):
+            feed[fg + ".ids"], feed[fg + ".values"], feed[fg + ".segments"] = rng.integers(0, 3000, n), np.ones(n, np.float32), s
+    got = {}
+    for fuse in (1, 0):
+        pm, inputs = din_model.build_manager(cfg, tables, weights, np.float32, expose=("score", ), net_args={"fuse_concat_into_fc": fuse})
+        p = pm.create_predictor(1, 0)
+        p.register_observers(["profile"])
+        din_model.feed(p, inputs, feed, np.float32)
+        p.forward()
+        got[fuse] = p.output_asnumpy("score").astype(np.float64).reshape(batch, T), p.output_asnumpy("prob").copy()
+        ev = [e for e in json.loads(p.dump_observers()["profile"])["traceEvents"] if e["dur"] > 0]
+        one = fuse == 1 and not (n1 == 96 and n2 == 64)
+        assert ("Gemm:gemm_att1_g" in [e["name"] for e in ev]) == (fuse == 0), ev
+        assert not one or [e["args"]["launches"] for e in ev if e["name"] == "Gemm:gemm_att0_g"] == [1]
+    # 64 bits
+    tb = [t.cpu().numpy().astype(np.float64) for t in tables]
+    q = np.concatenate([tb[i][feed[k + ".ids"]] for i, k in enumerate(din_model.KINDS)], 1)
+    his, off = np.zeros((batch, T, d3)), np.concatenate([[0], np.cumsum(seg)])
+    for i, k in enumerate(din_model.KINDS):
+        rows = tb[i][feed[k + "_his.ids"]]
+        for b in range(batch):
+            his[b, :seg[b], i * dim:(i + 1) * dim] = rows[off[b]:off[b + 1]]
+    x = np.broadcast_to(q[:, None, :], his.shape)
+    x = np.concatenate([x, his, x - his, x * his], 2)
+    for i, l in enumerate(weights["att"]):
+        size = np.abs(x) @ np.abs(l["w"].astype(np.float64)) + np.abs(l["b"])  # of the terms that are added up
+        x = x @ l["w"].astype(np.float64) + l["b"]
+        if i < 2:
+            t = 1 / (1 + np.exp(-(x - l["mean"]) / np.sqrt(l["var"].astype(np.float64) + 1e-8)))
+            x = (1 - t) * l["gamma"] * x + t * x
+    want = x.reshape(batch, T)
+    # A sum of k terms in four parts errs by at most (k / 4 + 3) * 2^-24 of its terms' magnitudes: 57, 27 and 19 * 2^-24 for the
+    # three layers, 6e-6 together, a third of that where roundings go both ways; bounded by the last layer's terms, which may
+    # cancel (a single score can be a hundredth of them)
+    for s, _ in got.values():
+        assert np.linalg.norm(s - want) <= 2e-6 * np.linalg.norm(size)
+    np.testing.assert_allclose(got[1][1], got[0][1], rtol=1e-5, atol=1e-6)

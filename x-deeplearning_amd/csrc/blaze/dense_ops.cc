@@ -11,6 +11,7 @@
 #include "blaze/graph.h"
 #include "blaze/operator.h"
 #include "blaze_hip.h"
+#include "bz_common.h"
 
 namespace blaze {
 
@@ -182,7 +183,7 @@ bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st
     d.a_pieces = c.a_pieces;
     d.next = c.next;
     d.a = nullptr;
-    const int rc = bz_fc_fused(&d, st);
+    const int rc = c.dtype == kFloat ? bz::fc_attention_f32(d, st) : bz_fc_fused(&d, st);
     if (rc == BZ_ENOTSUP) return false;
     BZ_CHECK(rc);
     return true;
@@ -292,11 +293,12 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
 
   // ---- the Concat that makes this layer's input, computed while it is loaded
-  // (the static part of what bz_fc_desc.a_pieces takes: a 2-byte layer of 9..96 columns and at most 224 inputs)
+  // (the static part of what bz_fc_desc.a_pieces takes: a layer of 9..96 columns and at most 224 inputs; an fp32 one only
+  // with the layers behind it, bz::fc_attention_f32)
   bool CanAdoptConcat() override {
     Blob* b = this->Input(1);
     if (!b_constant_ || transa_ || b->shape().size() != 2) return false;
-    if (b->data_type() != kFloat16) return false;
+    if (b->data_type() != kFloat16 && b->data_type() != kFloat) return false;
     const TIndex K = transb_ ? b->shape()[1] : b->shape()[0], N = transb_ ? b->shape()[0] : b->shape()[1];
     if (this->InputSize() > 2 && (!c_constant_ || (TIndex)this->Input(2)->size() != N)) return false;
     return N > 8 && N <= 96 && K <= 224 && !(fused_ && fused_act_ == BZ_ACT_SOFTMAX);

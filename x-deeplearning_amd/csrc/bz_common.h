@@ -46,4 +46,8 @@ inline int dtype_size(int dt) {
 constexpr int kWave = 64;       // CDNA wavefront
 constexpr int kNumXcd = 8;      // MI355X: 8 accelerator complex dies, workgroups are dealt to them round robin
 
+// fc_attention_f32.hip, for the host layer: bz_fc_fused of an fp32 layer on pieces [x, y, x - y, x * y] with a second and a
+// skinny third layer, of whose outputs only the last is stored.  BZ_ENOTSUP, with nothing launched, for anything else.
+int fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream);
+
 }  // namespace bz

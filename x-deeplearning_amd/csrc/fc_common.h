@@ -191,14 +191,78 @@ struct In<BZ_F32> {
   }
 };
 
-
 constexpr int kSkinnyMaxN = 8;
+
+// the optional skinny second layer computed from the first layer's output tile while it is still in LDS
+struct HeadArgs {
+  const char* w;      // [n, ldw], K contiguous, the dtype of the first layer's operands
+  const float* bias;  // [n] or null
+  void* y;            // [M, ldy]
+  int64_t ldw, ldy;
+  int n, act, out_dtype;
+};
+
+// the head's outputs of row m from its dot products: bias, activation, store
+__device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const float (&dot)[kSkinnyMaxN]) {
+  float v[kSkinnyMaxN];
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < head.n) ? dot[j] + (head.bias ? head.bias[j] : 0.f) : 0.f;
+  if (head.act == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
+    float mx = v[0];
+#pragma unroll
+    for (int j = 1; j < kSkinnyMaxN; ++j)
+      if (j < head.n) mx = v[j] > mx ? v[j] : mx;
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j)
+      if (j < head.n) {
+        v[j] = expf(v[j] - mx);
+        sum += v[j];
+      }
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j)
+      if (j < head.n) v[j] = v[j] / sum;
+  } else if (head.act == BZ_ACT_SIGMOID) {
+#pragma unroll
+    for (int j = 0; j < kSkinnyMaxN; ++j) {
+      const float t = expf(v[j]);
+      v[j] = t / (1.f + t);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kSkinnyMaxN; ++j) {
+    if (j < head.n) {
+      const int64_t at = (int64_t)m * head.ldy + j;
+      if (head.out_dtype == BZ_F32)
+        store_out<float>((float*)head.y + at, v[j]);
+      else if (head.out_dtype == BZ_F16)
+        store_out<__half>((__half*)head.y + at, v[j]);
+      else
+        store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
+    }
+  }
+}
+
+inline HeadArgs head_args(const bz_fc_desc& d) {
+  HeadArgs head;
+  head.w = (const char*)d.head_w;
+  head.bias = d.head_bias;
+  head.y = d.head_y;
+  head.ldw = d.head_ldw;
+  head.ldy = d.head_ldy;
+  head.n = d.head_n;
+  head.act = d.head_act;
+  head.out_dtype = d.head_out_dtype;
+  return head;
+}
 
 }  // namespace fc
 
 // fc_pieces.hip: the layer whose A operand is given as pieces (bz_fc_desc.a_pieces); called by bz_fc_fused after its
 // argument checks
 int fc_pieces_launch(const bz_fc_desc& d, const fc::Epilogue& ep, hipStream_t st);
+// the epilogue of a checked descriptor's (first) layer
+fc::Epilogue fc_epilogue(const bz_fc_desc& d);
 // The layer on a stored A, one function per operand type (fc_fused_f16.hip, fc_fused_bf16.hip, fc_fused_f32.hip): with a
 // head when d.head_n != 0, else the skinny, tile or streaming kernel.  bz_fc_fused has checked the descriptor.
 int fc_run_f16(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st);

@@ -30,6 +30,24 @@ __global__ void bz_pack_weight_kernel(const SrcT* __restrict__ src, DstT* __rest
 
 }  // namespace
 
+bz::fc::Epilogue bz::fc_epilogue(const bz_fc_desc& d) {
+  bz::fc::Epilogue ep;
+  ep.bias = (const float*)d.bias;
+  ep.p0 = d.act_p0;
+  ep.p1 = d.act_p1;
+  ep.p2 = d.act_p2;
+  ep.bias_rows = d.bias_rows;
+  ep.act = d.act;
+  ep.act_size = d.act_size;
+  ep.dice_nosqrt = d.dice_nosqrt;
+  ep.alpha = d.alpha;
+  ep.beta = d.beta;
+  ep.act_alpha = d.act_alpha;
+  ep.split_n = d.n_split;
+  ep.split_stride = d.y_split_stride;
+  return ep;
+}
+
 extern "C" {
 
 int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
@@ -68,20 +86,7 @@ int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
       return bz::fail(BZ_EINVAL, "bz_fc_fused: unknown activation %d", d.act);
   }
   if (d.m == 0) return BZ_OK;
-  Epilogue ep;
-  ep.bias = (const float*)d.bias;
-  ep.p0 = d.act_p0;
-  ep.p1 = d.act_p1;
-  ep.p2 = d.act_p2;
-  ep.bias_rows = d.bias_rows;
-  ep.act = d.act;
-  ep.act_size = d.act_size;
-  ep.dice_nosqrt = d.dice_nosqrt;
-  ep.alpha = d.alpha;
-  ep.beta = d.beta;
-  ep.act_alpha = d.act_alpha;
-  ep.split_n = d.n_split;
-  ep.split_stride = d.y_split_stride;
+  const Epilogue ep = bz::fc_epilogue(d);
   const int es = bz::dtype_size(d.in_dtype);
   const bool vec_a = ((uintptr_t)d.a % 16 == 0) && ((d.lda * es) % 16 == 0);
   const bool vec_w = ((uintptr_t)d.w % 16 == 0) && ((d.ldw * es) % 16 == 0);

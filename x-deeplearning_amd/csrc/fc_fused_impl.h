@@ -133,56 +133,6 @@ __device__ __forceinline__ void chunk_to_float(const uint4& c, float (&f)[In<DT>
   }
 }
 
-// the optional skinny second layer computed from the first layer's output tile while it is still in LDS
-struct HeadArgs {
-  const char* w;      // [n, ldw], K contiguous, the dtype of the first layer's operands
-  const float* bias;  // [n] or null
-  void* y;            // [M, ldy]
-  int64_t ldw, ldy;
-  int n, act, out_dtype;
-};
-
-// the head's outputs of row m from its dot products: bias, activation, store
-__device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const float (&dot)[kSkinnyMaxN]) {
-  float v[kSkinnyMaxN];
-#pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < head.n) ? dot[j] + (head.bias ? head.bias[j] : 0.f) : 0.f;
-  if (head.act == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
-    float mx = v[0];
-#pragma unroll
-    for (int j = 1; j < kSkinnyMaxN; ++j)
-      if (j < head.n) mx = v[j] > mx ? v[j] : mx;
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j)
-      if (j < head.n) {
-        v[j] = expf(v[j] - mx);
-        sum += v[j];
-      }
-#pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j)
-      if (j < head.n) v[j] = v[j] / sum;
-  } else if (head.act == BZ_ACT_SIGMOID) {
-#pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j) {
-      const float t = expf(v[j]);
-      v[j] = t / (1.f + t);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j) {
-    if (j < head.n) {
-      const int64_t at = (int64_t)m * head.ldy + j;
-      if (head.out_dtype == BZ_F32)
-        store_out<float>((float*)head.y + at, v[j]);
-      else if (head.out_dtype == BZ_F16)
-        store_out<__half>((__half*)head.y + at, v[j]);
-      else
-        store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
 // tiled MFMA kernel
 // ---------------------------------------------------------------------------------------------
@@ -1130,20 +1080,6 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
         if (n < N) store_out<OutT>(Y + out_index(ep, m, n, ldy), v[n]);
     }
   }
-}
-
-
-inline HeadArgs head_args(const bz_fc_desc& d) {
-  HeadArgs head;
-  head.w = (const char*)d.head_w;
-  head.bias = d.head_bias;
-  head.y = d.head_y;
-  head.ldw = d.head_ldw;
-  head.ldy = d.head_ldy;
-  head.n = d.head_n;
-  head.act = d.head_act;
-  head.out_dtype = d.head_out_dtype;
-  return head;
 }
 
 template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false, int WK = 1,
