@@ -293,6 +293,32 @@ def test_fc_with_skinny_head_in_one_launch(bz, oracle, in_name, M, K, N, N2, act
     assert np.all(np.abs(z1.cpu().numpy() - want) <= 1e-5 * scale + 1e-6)  # fp32 head from the stored tile: fp32 accuracy
 
 
+@pytest.mark.parametrize("in_name", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("M,K,N", [(2049, 512, 256), (33, 64, 136), (1000, 200, 80), (16400, 80, 40), (17, 72, 16), (1, 8, 256), (1, 64, 24)])
+def test_fc_head_of_two_outputs_equals_the_same_two_of_more(bz, in_name, M, K, N):
+    """the code of a head is unrolled for two outputs or for eight: the same sums in the same order, so the same bits"""
+    import torch
+    torch.manual_seed(M + K + N)
+    tdt, bt = _tdtype(in_name), {"f32": bz.F32, "f16": bz.F16, "bf16": bz.BF16}[in_name]
+    a = torch.randn(M, K, device="cuda").to(tdt)
+    w1 = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bt)
+    W2 = torch.randn(N, 8, device="cuda") / N**0.5
+    b2 = torch.randn(8, device="cuda")
+    got = {}
+    for n in (1, 2, 3, 8):
+        z = torch.full((M, n), -7.0, device="cuda")
+        head = dict(w=bz.pack_weight(W2[:, :n].contiguous(), False, bt), bias=b2[:n].contiguous(), act=bz.ACT_SIGMOID, out=z)
+        bz.fc_fused(a, w1, K, out_dtype=bt, store_out=False, head=head)
+        got[n] = z.cpu().numpy()
+    for n in (1, 2, 3):
+        np.testing.assert_array_equal(got[n], got[8][:, :n])
+    y = (a.double() @ w1[:, :K].double().t().contiguous()).cpu().numpy()
+    z = y @ W2.to(tdt).double().cpu().numpy() + b2.double().cpu().numpy()
+    # the rounding of N stored outputs of O(1), times weights of 1 / sqrt(N), times a slope of at most 1 / 4; fp32: of the sums
+    tol = 8 * {"f32": 2.0**-20, "f16": 2.0**-11, "bf16": 2.0**-8}[in_name]
+    np.testing.assert_allclose(got[8], 1 / (1 + np.exp(-z)), rtol=0, atol=tol)
+
+
 def test_fc_head_limits_are_refused(bz):
     import torch
     a = torch.zeros((64, 512), dtype=torch.float16, device="cuda")
@@ -801,3 +827,9 @@ def test_attention_mlp_as_one_launch(bz, oracle, in_name, r0, r1, w, N, N2, N3, 
     np.testing.assert_allclose(y1_one.float().cpu().numpy(), y1.float().cpu().numpy(), rtol=0,
                                atol=4 * eps * max(1.0, float(y1.float().abs().max())))
     np.testing.assert_allclose((z if N3 else y2).float().cpu().numpy(), got, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("in_name", ["f16", "bf16"])
+@pytest.mark.parametrize("N3,head_act", [(1, "sigmoid"), (2, "none"), (3, "sigmoid"), (8, "softmax")])
+def test_attention_mlp_with_heads_of_either_unrolling(bz, oracle, in_name, N3, head_act):
+    test_attention_mlp_as_one_launch(bz, oracle, in_name, 37, 5, 24, 96, 64, N3, "prelu", head_act)

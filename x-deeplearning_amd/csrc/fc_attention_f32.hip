@@ -141,8 +141,8 @@ struct StagedParams {
   }
 };
 
-// VEC: columns of x and y a lane loads at once
-template <int VEC>
+// VEC: columns of x and y a lane loads at once; HN: outputs of the third layer the code is unrolled for
+template <int VEC, int HN>
 __global__ __launch_bounds__(kThreads, 2) void bz_fc_attention_f32_kernel(const Attention a) {
   using Pack = bz::CewPack<float, VEC>;
   constexpr int kLoads = (kRows * 56 / VEC + kThreads - 1) / kThreads;  // w is at most 56
@@ -173,6 +173,7 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_attention_f32_kernel(const 
     }
   };
   load(blockIdx.x);
+  const HeadBias<HN> hbias(a.head);
 
   // both weights, zero beyond their rows and columns, the third layer's, the parameters
   Staged<(96 * 56 + kThreads - 1) / kThreads> s1;
@@ -223,25 +224,23 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_attention_f32_kernel(const 
     __syncthreads();
     // the third layer: sixteen lanes a row, four columns each
     const int r = tid >> 4, c = (tid & 15) * 4, m = tile * kRows + r;
-    float dot[kSkinnyMaxN];
+    float dot[HN];
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (c < l.nb2 * 16) v = *(const float4*)(h2 + r * l.p2 + c);
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j) {
+    for (int j = 0; j < HN; ++j) {
       dot[j] = 0.f;
       if (j < a.head.n) {
         float4 u = make_float4(0.f, 0.f, 0.f, 0.f);
         if (c < l.nb2 * 16) u = *(const float4*)(w3 + j * l.nb2 * 16 + c);
-        dot[j] = fmaf(v.w, u.w, fmaf(v.z, u.z, fmaf(v.y, u.y, v.x * u.x)));
-#pragma unroll
-        for (int d = 8; d > 0; d >>= 1) dot[j] += __shfl_xor(dot[j], d, 64);
+        dot[j] = group_sum<16>(fmaf(v.w, u.w, fmaf(v.z, u.z, fmaf(v.y, u.y, v.x * u.x))));
       }
     }
-    if ((tid & 15) == 0 && m < a.m) head_finish(a.head, m, dot);
+    if ((tid & 15) == 0 && m < a.m) head_finish(a.head, hbias, m, dot);
   }
 }
 
-template <int VEC>
+template <int VEC, int HN>
 int launch(const Attention& a, int lds, hipStream_t st) {
   static std::mutex mu;
   static bool raised[64] = {};
@@ -250,12 +249,12 @@ int launch(const Attention& a, int lds, hipStream_t st) {
   {
     std::lock_guard<std::mutex> lock(mu);
     if (dev >= 0 && dev < 64 && !raised[dev]) {
-      BZ_HIP_OK(hipFuncSetAttribute((const void*)bz_fc_attention_f32_kernel<VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+      BZ_HIP_OK(hipFuncSetAttribute((const void*)bz_fc_attention_f32_kernel<VEC, HN>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
       raised[dev] = true;
     }
   }
   const int tiles = (a.m + kRows - 1) / kRows;
-  hipLaunchKernelGGL((bz_fc_attention_f32_kernel<VEC>), dim3(tiles < 256 ? tiles : 256), dim3(kThreads), lds, st, a);
+  hipLaunchKernelGGL((bz_fc_attention_f32_kernel<VEC, HN>), dim3(tiles < 256 ? tiles : 256), dim3(kThreads), lds, st, a);
   BZ_LAUNCH_OK("bz_fc_attention_f32_kernel");
   return BZ_OK;
 }
@@ -325,7 +324,8 @@ int bz::fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream) {
   a.ep2.act_alpha = x.act_alpha;
   a.head = head_args(d);
   hipStream_t st = bz::as_stream(stream);
-  if (vec >= 4) return launch<4>(a, lds, st);
-  if (vec == 2) return launch<2>(a, lds, st);
-  return launch<1>(a, lds, st);
+  const bool two = head_unroll(d.head_n) == 2;
+  if (vec >= 4) return two ? launch<4, 2>(a, lds, st) : launch<4, kSkinnyMaxN>(a, lds, st);
+  if (vec == 2) return two ? launch<2, 2>(a, lds, st) : launch<2, kSkinnyMaxN>(a, lds, st);
+  return two ? launch<1, 2>(a, lds, st) : launch<1, kSkinnyMaxN>(a, lds, st);
 }

@@ -202,35 +202,54 @@ struct HeadArgs {
   int n, act, out_dtype;
 };
 
-// the head's outputs of row m from its dot products: bias, activation, store
-__device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const float (&dot)[kSkinnyMaxN]) {
-  float v[kSkinnyMaxN];
+// The code that is unrolled over a head's outputs exists for two (the usual heads) and for kSkinnyMaxN: a short kernel
+// runs through code that no CU has at hand, and unrolled for eight with two used most of what it fetches is skipped.
+inline int head_unroll(int n) { return n <= 2 ? 2 : kSkinnyMaxN; }
+
+// the head's bias, asked for where a kernel starts: loaded at its end the whole of a small launch waits for it
+template <int HN>
+struct HeadBias {
+  float b[HN];
+  __device__ __forceinline__ explicit HeadBias(const HeadArgs& head) {
 #pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < head.n) ? dot[j] + (head.bias ? head.bias[j] : 0.f) : 0.f;
+    for (int j = 0; j < HN; ++j) b[j] = 0.f;
+    if (head.bias != nullptr) {
+#pragma unroll
+      for (int j = 0; j < HN; ++j) b[j] = head.bias[j < head.n ? j : head.n - 1];
+    }
+  }
+};
+
+// the head's outputs of row m from its dot products: bias, activation, store
+template <int HN>
+__device__ __forceinline__ void head_finish(const HeadArgs& head, const HeadBias<HN>& bias, int m, const float (&dot)[HN]) {
+  float v[HN];
+#pragma unroll
+  for (int j = 0; j < HN; ++j) v[j] = (j < head.n) ? dot[j] + bias.b[j] : 0.f;
   if (head.act == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
     float mx = v[0];
 #pragma unroll
-    for (int j = 1; j < kSkinnyMaxN; ++j)
+    for (int j = 1; j < HN; ++j)
       if (j < head.n) mx = v[j] > mx ? v[j] : mx;
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j)
+    for (int j = 0; j < HN; ++j)
       if (j < head.n) {
         v[j] = expf(v[j] - mx);
         sum += v[j];
       }
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j)
+    for (int j = 0; j < HN; ++j)
       if (j < head.n) v[j] = v[j] / sum;
   } else if (head.act == BZ_ACT_SIGMOID) {
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j) {
+    for (int j = 0; j < HN; ++j) {
       const float t = expf(v[j]);
       v[j] = t / (1.f + t);
     }
   }
 #pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j) {
+  for (int j = 0; j < HN; ++j) {
     if (j < head.n) {
       const int64_t at = (int64_t)m * head.ldy + j;
       if (head.out_dtype == BZ_F32)
@@ -241,6 +260,28 @@ __device__ __forceinline__ void head_finish(const HeadArgs& head, int m, const f
         store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
     }
   }
+}
+
+// The sum over each aligned group of W lanes, in the group's first lane (the others hold parts): the halves added to each
+// other down to one, as a butterfly of __shfl_xor adds them up for that lane.  Those go through the LDS unit, some 100
+// clocks each; these are plain vector instructions.  All lanes of the wave have to be there.
+template <int N>
+__device__ __forceinline__ float row_shl(float v) {  // lane i of a row of 16: lane i + N's
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x100 + N, 0xf, 0xf, true));
+}
+template <int W>
+__device__ __forceinline__ float group_sum(float v) {
+  static_assert(W == 2 || W == 4 || W == 8 || W == 16 || W == 64, "a power of two within a row, or the wave");
+  if constexpr (W == 64) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  }
+  if constexpr (W >= 16) v += row_shl<8>(v);
+  if constexpr (W >= 8) v += row_shl<4>(v);
+  if constexpr (W >= 4) v += row_shl<2>(v);
+  return v + row_shl<1>(v);
 }
 
 inline HeadArgs head_args(const bz_fc_desc& d) {

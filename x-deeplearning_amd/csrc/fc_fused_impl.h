@@ -139,14 +139,15 @@ __device__ __forceinline__ void chunk_to_float(const uint4& c, float (&f)[In<DT>
 // Sums an output is added up in where a wave owns one 32x32 block.  fp32: one for each step of a K tile, which also makes
 // them shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two).  Two otherwise, and in the tiles with
 // a head, whose other registers are many: with four the 64x64 one takes 10.7 us for 17000 x 80 -> 40 instead of 10.3.
-template <int DT, int BM, int BN, int BK, int WM, int WN, bool HEAD, int WK>
+template <int DT, int BM, int BN, int BK, int WM, int WN, int HEAD, int WK>
 constexpr int default_sums() {
   constexpr int steps = BK / In<DT>::kStepK / WK;
   return BM / WM / 32 * (BN / WN / 32) > 1 ? 1 : DT == BZ_F32 && !HEAD ? steps : steps >= 2 ? 2 : 1;
 }
 
+// HEAD: outputs the code of the skinny second layer is unrolled for, 0 without one
 // WK: groups of WM x WN waves that share each K tile between them and add up at the end
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD, int WK, int KACC>
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD, int WK, int KACC>
 __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                   OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                   int64_t ldw, int64_t ldy, bool vec_y, int tiles_m, Epilogue ep,
@@ -164,11 +165,11 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BK % T::kStepK == 0, "tile shape");
 
   __shared__ __attribute__((aligned(16))) char lds[2][(BM + BN) * PITCH];
-  // HEAD: the second layer's weight [kSkinnyMaxN, BN], requested now into registers, parked in LDS after the K loop
+  // HEAD: the second layer's weight [HEAD, BN], requested now into registers, parked in LDS after the K loop
   constexpr int HW_ROW = BN * ES;  // bytes
-  constexpr int HW_CHUNKS = HEAD ? kSkinnyMaxN * HW_ROW / 16 : 1;
+  constexpr int HW_CHUNKS = HEAD ? HEAD * HW_ROW / 16 : 1;
   constexpr int HW_PER = (HW_CHUNKS + NT - 1) / NT;
-  __shared__ __attribute__((aligned(16))) char lds_hw[HEAD ? kSkinnyMaxN * HW_ROW : 16];
+  __shared__ __attribute__((aligned(16))) char lds_hw[HEAD ? HEAD * HW_ROW : 16];
   uint4 rhw[HW_PER];
 
   const int tid = threadIdx.x;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   // number of exposed round trips, ceil(KT / D), is what sets its duration.
   // which aligned loader: the head tile (see load_chunk_clamped) and the 256x256 tile, whose 256 registers have no room
   // for the zero-chunk select's addresses (it spilled 75 of them)
-  constexpr bool CLAMPED = HEAD || BM * BN >= 256 * 256;
+  constexpr bool CLAMPED = HEAD != 0 || BM * BN >= 256 * 256;
   uint4 ra[D][A_PER], rw[D][W_PER];
   auto gload = [&](int set, int k0) {
 #pragma unroll
@@ -241,7 +242,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
     }
   };
 
-  if constexpr (HEAD) {
+  const HeadBias<HEAD == 0 ? 1 : HEAD> hbias(head);  // (without a head its bias is null)
+  if constexpr (HEAD != 0) {
     const int present = N * ES / 16;  // chunks of a weight row that exist (N is a whole number of chunks)
 #pragma unroll
     for (int i = 0; i < HW_PER; ++i) {
@@ -466,7 +468,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
       epilogue(std::integral_constant<int, BZ_ACT_NONE>());
       break;
   }
-  if constexpr (HEAD) {
+  if constexpr (HEAD != 0) {
 #pragma unroll
     for (int i = 0; i < HW_PER; ++i) {
       const int q = tid + i * NT;
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
       if (m0 + ml < M && n0 + nl < N) Y[out_index(ep, m0 + ml, n0 + nl, ldy)] = ((const OutT*)(lout + ml * OPITCH))[nl];
     }
   }
-  if constexpr (HEAD) {
+  if constexpr (HEAD != 0) {
     // z[m, j] = head_act(sum_n y[m, n] * w2[j, n] + b2[j]) from the rounded tile, as the separate skinny launch
     // computes it from the stored tensor.  NT / BM lanes share a row; this workgroup owns whole rows (n0 == 0).
     static_assert(OS == ES, "the head reads the tile with the operand type");
@@ -496,14 +498,14 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
     const int r = tid / LPRH, hl = tid % LPRH;
     const int m = m0 + r;
     const int nch = N / CH;
-    float hacc[kSkinnyMaxN];
+    float hacc[HEAD];
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j) hacc[j] = 0.f;
+    for (int j = 0; j < HEAD; ++j) hacc[j] = 0.f;
     for (int ch = hl; ch < nch; ch += LPRH) {
       float a[CH];
       chunk_to_float<DT>(*(const uint4*)(lout + r * OPITCH + ch * 16), a);
 #pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) {
+      for (int j = 0; j < HEAD; ++j) {
         if (j < head.n) {
           float w[CH];
           chunk_to_float<DT>(*(const uint4*)(lds_hw + j * HW_ROW + ch * 16), w);
@@ -513,11 +515,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
       }
     }
 #pragma unroll
-    for (int d = LPRH >> 1; d > 0; d >>= 1) {
-#pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) hacc[j] += __shfl_xor(hacc[j], d, 64);
-    }
-    if (hl == 0 && m < M) head_finish(head, m, hacc);
+    for (int j = 0; j < HEAD; ++j) hacc[j] = group_sum<LPRH>(hacc[j]);
+    if (hl == 0 && m < M) head_finish(head, hbias, m, hacc);
   }
 }
 
@@ -877,11 +876,11 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
 // ---------------------------------------------------------------------------------------------
 // A layer with a head keeps whole rows in one workgroup, so M sets how many CUs work: 16 rows a workgroup where the staged
 // tile takes 32, and sixteen waves that share its columns (32 each) and, for N below 256, K, each working for itself as in
-// the split kernel above.  After the partial blocks are added up, wave r
-// owns row r: its lanes hold the row's outputs in registers, and the head is a dot product within the wave.
+// the split kernel above.  After the partial blocks are added up, wave r owns
+// row r: its lanes hold the row's outputs in registers, and the head is a dot product within the wave.
 constexpr int kHeadWaves = 16;
 
-template <int DT, typename OutT>
+template <int DT, typename OutT, int HN>
 __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                            OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                            int64_t ldw, int64_t ldy, Epilogue ep, HeadArgs head) {
@@ -896,7 +895,8 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
   const int m0 = blockIdx.x * 16;
   // the row's columns of this lane: their parameters and the head's weights, asked for first
   float cb[COLS], q0[COLS], q1[COLS], q2[COLS];
-  OutT hw[kSkinnyMaxN][COLS];
+  OutT hw[HN][COLS];
+  const HeadBias<HN> hbias(head);
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const int n = min(lane + 64 * c, N - 1);
@@ -910,8 +910,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
       q2[c] = ep.p2[n];
     }
 #pragma unroll
-    for (int j = 0; j < kSkinnyMaxN; ++j)
-      if (j < head.n) hw[j][c] = w2[j * head.ldw];
+    for (int j = 0; j < HN; ++j) hw[j][c] = w2[(j < head.n ? j : head.n - 1) * head.ldw];
   }
   const int nb = (N + 31) / 32, parts = kHeadWaves / nb, pitch = nb * 32 + 1;
   const int part = wave / nb, block = wave - part * nb;
@@ -966,30 +965,32 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
   __syncthreads();
   const int m = m0 + wave;
   if (m >= M) return;
-  float dot[kSkinnyMaxN];
+  // (read for all columns at once, and beyond N as well: nothing waits in turn)
+  float sum[COLS];
 #pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j) dot[j] = 0.f;
+  for (int c = 0; c < COLS; ++c) sum[c] = 0.f;
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) {
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) sum[c] += red[(p * 16 + wave) * pitch + min(lane + 64 * c, N - 1)];
+  }
+  float dot[HN];
+#pragma unroll
+  for (int j = 0; j < HN; ++j) dot[j] = 0.f;
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const int n = lane + 64 * c;
     if (n < N) {
-      float v = 0.f;
-      for (int p = 0; p < parts; ++p) v += red[(p * 16 + wave) * pitch + n];
       OutT y;
-      store_out<OutT>(&y, apply_act_regs(fmaf(ep.alpha, v, ep.beta * cb[c]), ep, q0[c], q1[c], q2[c]));
+      store_out<OutT>(&y, apply_act_regs(fmaf(ep.alpha, sum[c], ep.beta * cb[c]), ep, q0[c], q1[c], q2[c]));
       if (Y != nullptr) Y[(int64_t)m * ldy + n] = y;
 #pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j)
-        if (j < head.n) dot[j] = fmaf((float)y, (float)hw[j][c], dot[j]);
+      for (int j = 0; j < HN; ++j) dot[j] = fmaf((float)y, (float)hw[j][c], dot[j]);
     }
   }
 #pragma unroll
-  for (int j = 0; j < kSkinnyMaxN; ++j)
-    if (j < head.n) {
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) dot[j] += __shfl_xor(dot[j], d, 64);
-    }
-  if (lane == 0) head_finish(head, m, dot);
+  for (int j = 0; j < HN; ++j) dot[j] = group_sum<64>(dot[j]);
+  if (lane == 0) head_finish(head, hbias, m, dot);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1082,7 +1083,7 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
   }
 }
 
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, bool HEAD = false, int WK = 1,
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD = 0, int WK = 1,
           int KACC = default_sums<DT, BM, BN, BK, WM, WN, HEAD, WK>()>
 int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
@@ -1091,7 +1092,7 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const bool vec_y = d.y != nullptr && ((uintptr_t)d.y % 16 == 0) && ((d.ldy * (int64_t)sizeof(OutT)) % 16 == 0) &&
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
-  const HeadArgs head = HEAD ? head_args(d) : HeadArgs{};
+  const HeadArgs head = HEAD != 0 ? head_args(d) : HeadArgs{};
   hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK, KACC>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
@@ -1134,37 +1135,42 @@ int launch_stream(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 
 
 // Layer + skinny head in one launch: a workgroup owns whole rows of the first layer's output (N <= 256).
-template <int DT, typename OutT>
+template <int DT, typename OutT, int HN>
 int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   // fp32 is bound by the matrix cores of the CUs that work, so the staged tile's 32 rows waste time while they are few: 16
   // rows a workgroup up to 2048 rows (us alone / with eight streams of the same, the tile's behind: 1024 x 512 -> 256
-  // 18.9 / 7.5 and 25.4 / 9.8, 2048 x 512 -> 256 19.2 / 10.1 and 25.5 / 9.9, 2000 x 512 -> 128 12.4 / 6.4 and 17.7 / 9.0,
-  // 201 x 200 -> 80 7.9 / 3.2 and 10.6 / 4.1; 4096 x 512 -> 256 19.4 / 17.5 and 25.6 / 14.0).  A row's operands cost more
-  // this way, which shows where other kernels fill the chip: of a tower on eight serving threads a pass of 1024 rows takes
+  // 17.9 / 4.6 and 24.6 / 6.3, 2048 x 512 -> 256 18.0 / 8.1 and 24.6 / 6.3, 2000 x 512 -> 128 11.5 / 4.9 and 16.7 / 5.9,
+  // 201 x 200 -> 80 7.2 / 2.0 and 10.4 / 2.8; 4096 x 512 -> 256 18.2 / 16.5 and 24.6 / 15.2).  A row's operands cost more
+  // this way, which shows where other kernels fill the chip: of a tower on eight serving threads a pass of 1024 rows took
   // 20.4 us and 21.7 with the tile, of 2048 32.1 and 30.7 (64.0 and 69.1 alone), of 4096 63.6 and 57.0 (84.8 and 89.8).
-  // 2-byte layers are not bound by the matrix cores (2048 x 512 -> 256 fp16 10.2, the tile 9.0; measured at that size alone).
+  // 2-byte layers are not bound by the matrix cores (2048 x 512 -> 256 fp16 8.3 / 3.6, the tile 8.2 / 2.2; 201 x 200 -> 80
+  // 5.8 / 2.1 and 5.8 / 2.3).
+  //
+  // HN: outputs the head's code is unrolled for.  Two instead of eight, its bias asked for at the start and its sums taken
+  // by vector instructions, and each launch ends 1.5 to 2 us earlier: 2048 x 512 -> 256 fp16 9.7 -> 8.1 us alone, 2.5 -> 2.2
+  // with eight streams, fp32 19.9 -> 18.0 / 9.0 -> 8.1; one row of 200 -> 80 fp32 7.9 -> 6.2.
   if constexpr (DT == BZ_F32) {
     if (d.m <= 2048) {
-      hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
+      hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
                          (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d));
       BZ_LAUNCH_OK("bz_fc_split_head_kernel");
       return BZ_OK;
     }
     // Up to 4096 rows four sums an output, as short as that kernel's (3000 x 512 -> 128 17.9 / 8.3, with two 17.8 / 9.3;
-    // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6)
-    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true, 1, 4>(d, ep, st);
-    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, true, 1, 4>(d, ep, st);
+    // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6; measured with the head's code unrolled for eight)
+    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 1, 4>(d, ep, st);
+    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 1, 4>(d, ep, st);
   }
   if (d.n <= 64) {
-    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, true>(d, ep, st);
-    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, true>(d, ep, st);
+    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, HN>(d, ep, st);
+    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN>(d, ep, st);
   }
-  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, true>(d, ep, st);
+  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN>(d, ep, st);
   // eight waves: with one workgroup per 32 rows only M / 32 CUs work, and each has 288 KB of operands to pull in
-  // (two K tiles in flight: with eight waves taking turns that hides the loads, and it is faster than four both alone,
+  // (two K tiles in flight: with eight waves taking turns that hides the loads, and it was faster than four both alone,
   // 10.5 against 11.3 us on config 2's 512 -> 256 -> 2, and next to other kernels)
-  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, true>(d, ep, st);
+  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, HN>(d, ep, st);
 }
 
 // The tiles of the staged kernel that both kinds of rows take (ALIGNED: every row starts on 16 bytes and K is a whole
@@ -1210,7 +1216,7 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
       // barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way, 2048 x 512 -> 512 14.8 and 13.4.  With more tiles the matrix
       // cores set the time either way (8192 rows 64 us), and next to other kernels the smaller workgroup wins (the tower
       // of that layer at 4096 rows, eight serving threads, 57.8 us a pass this way and 56.8 the other).
-      if (d.k >= 512 && wg64 >= 256 && wg64 < 512) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, false, 2>(d, ep, st);
+      if (d.k >= 512 && wg64 >= 256 && wg64 < 512) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, 0, 2>(d, ep, st);
       // Else four waves and two K tiles in flight (us alone / with eight streams of the same; the eight waves:
       // 10000 x 64 -> 200 14.5 / 9.4 and now 9.6 / 5.8, 4096 x 192 -> 512 14.4 / 11.3 and 12.4 / 8.8, 1500 x 400 -> 700
       // 21.9 / 11.6 and 19.5 / 10.8; 32x64 with four in flight: 1500 x 896 -> 512 37.0 / 19.0 and 22.3 / 15.2).
@@ -1322,7 +1328,7 @@ int dispatch_out(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w
 // one operand type's entry: the layer with a head, or the plain layer (skinny / tile / streaming kernel)
 template <int DT, typename T>
 int run_typed(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
-  if (d.head_n != 0) return dispatch_head<DT, T>(d, ep, st);
+  if (d.head_n != 0) return bz::fc::head_unroll(d.head_n) == 2 ? dispatch_head<DT, T, 2>(d, ep, st) : dispatch_head<DT, T, kSkinnyMaxN>(d, ep, st);
   return dispatch_out<DT>(d, ep, vec_a, vec_w, st);
 }
 

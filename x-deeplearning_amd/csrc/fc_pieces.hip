@@ -42,11 +42,7 @@ struct ChainArgs {
   int64_t ldw2, ldy2;
   int n2;              // 9..64
   Epilogue ep2;
-  const char* w3;      // [n3, ldw3] or null
-  const float* bias3;
-  void* y3;            // [M, ldy3]
-  int64_t ldw3, ldy3;
-  int n3, act3, y3_dtype;  // n3 = 0: no third layer
+  HeadArgs head;       // n = 0: no third layer
 };
 constexpr int kChainKS = kPiecesMaxN / 16;  // K steps of the second layer (its K is the first layer's N)
 constexpr int kChainPitch = kPiecesMaxN * 2 + 16;  // bytes between the rows of the second layer's weight in LDS
@@ -160,14 +156,15 @@ __global__ __launch_bounds__(256, 2) void bz_fc_pieces_kernel(bz::CewP p, const 
     const int n = q - which1[h] * kPiecesMaxN;
     pv1[h] = param_load(ep, which1[h], n < N ? n : N - 1);
   }
+  const HeadBias<2> hbias2(ch.head);
   if constexpr (CHAIN) {
     const int n2 = tid & 63;
     pv2 = param_load(ch.ep2, tid >> 6, n2 < ch.n2 ? n2 : ch.n2 - 1);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int q = tid + h * NT, j = q >> 6, c = q & 63;
-      w3use[h] = j < ch.n3 && c < ch.n2;
-      w3v[h] = bz::ldv<ET>(w3use[h] ? (const ET*)ch.w3 + (int64_t)j * ch.ldw3 + c : (const ET*)W);
+      w3use[h] = j < ch.head.n && c < ch.n2;
+      w3v[h] = bz::ldv<ET>(w3use[h] ? (const ET*)ch.head.w + (int64_t)j * ch.head.ldw + c : (const ET*)W);
     }
   }
   // into LDS: the first layer's weight into the A tile's own rows (it is gone from there before the tile is written)
@@ -443,12 +440,13 @@ __global__ __launch_bounds__(256, 2) void bz_fc_pieces_kernel(bz::CewP p, const 
       }
     }
     // ---- skinny third layer: two lanes a row, 32 columns each, from the rounded staged tile
-    if (ch.n3 > 0) {
+    auto third = [&](const auto& hbias, auto hn) {
+      constexpr int HN = decltype(hn)::value;
       const int ml = lane >> 1, hx = lane & 1;
       const int m = m0 + wave * 32 + ml;
-      float hacc[kSkinnyMaxN];
+      float hacc[HN];
 #pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) hacc[j] = 0.f;
+      for (int j = 0; j < HN; ++j) hacc[j] = 0.f;
       // the lane's 32 columns of its row in four 16-byte reads (columns from n2 up are zero, in the tile and in w3s);
       // the weights come from LDS, where the workgroup put them at the start: a load from memory per column here made
       // every wave wait 32 times
@@ -470,8 +468,8 @@ __global__ __launch_bounds__(256, 2) void bz_fc_pieces_kernel(bz::CewP p, const 
         }
       }
 #pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) {
-        if (j < ch.n3) {
+      for (int j = 0; j < HN; ++j) {
+        if (j < ch.head.n) {
           const float4* wj = (const float4*)(w3s + j * 64 + hx * 32);
 #pragma unroll
           for (int q = 0; q < 8; ++q) {
@@ -484,47 +482,13 @@ __global__ __launch_bounds__(256, 2) void bz_fc_pieces_kernel(bz::CewP p, const 
         }
       }
 #pragma unroll
-      for (int j = 0; j < kSkinnyMaxN; ++j) hacc[j] += __shfl_xor(hacc[j], 1, 64);
-      if (hx == 0 && m < M) {
-        float v[kSkinnyMaxN];
-#pragma unroll
-        for (int j = 0; j < kSkinnyMaxN; ++j) v[j] = (j < ch.n3) ? hacc[j] + (ch.bias3 ? ch.bias3[j] : 0.f) : 0.f;
-        if (ch.act3 == BZ_ACT_SOFTMAX) {  // softmax_op.cc:21-78: subtract max, exp, sum in order, divide
-          float mx = v[0];
-#pragma unroll
-          for (int j = 1; j < kSkinnyMaxN; ++j)
-            if (j < ch.n3) mx = v[j] > mx ? v[j] : mx;
-          float sum = 0.f;
-#pragma unroll
-          for (int j = 0; j < kSkinnyMaxN; ++j)
-            if (j < ch.n3) {
-              v[j] = expf(v[j] - mx);
-              sum += v[j];
-            }
-#pragma unroll
-          for (int j = 0; j < kSkinnyMaxN; ++j)
-            if (j < ch.n3) v[j] = v[j] / sum;
-        } else if (ch.act3 == BZ_ACT_SIGMOID) {
-#pragma unroll
-          for (int j = 0; j < kSkinnyMaxN; ++j) {
-            const float t = expf(v[j]);
-            v[j] = t / (1.f + t);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < kSkinnyMaxN; ++j) {
-          if (j < ch.n3) {
-            const int64_t at = (int64_t)m * ch.ldy3 + j;
-            if (ch.y3_dtype == BZ_F32)
-              store_out<float>((float*)ch.y3 + at, v[j]);
-            else if (ch.y3_dtype == BZ_F16)
-              store_out<__half>((__half*)ch.y3 + at, v[j]);
-            else
-              store_out<__hip_bfloat16>((__hip_bfloat16*)ch.y3 + at, v[j]);
-          }
-        }
-      }
-    }
+      for (int j = 0; j < HN; ++j) hacc[j] = group_sum<2>(hacc[j]);
+      if (hx == 0 && m < M) head_finish(ch.head, hbias, m, hacc);
+    };
+    if (ch.head.n > 2)
+      third(HeadBias<kSkinnyMaxN>(ch.head), std::integral_constant<int, kSkinnyMaxN>());
+    else if (ch.head.n > 0)
+      third(hbias2, std::integral_constant<int, 2>());
   }
 }
 
@@ -619,14 +583,7 @@ int launch_pieces(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
                  "bz_fc_fused: head of %d outputs (1..%d), null head_w / head_y, or a leading dimension below its row", d.head_n, kSkinnyMaxN);
       BZ_REQUIRE(d.head_act == BZ_ACT_NONE || d.head_act == BZ_ACT_SIGMOID || d.head_act == BZ_ACT_SOFTMAX, "bz_fc_fused: head activation %d", d.head_act);
       BZ_REQUIRE(d.head_out_dtype == BZ_F32 || d.head_out_dtype == BZ_F16 || d.head_out_dtype == BZ_BF16, "bz_fc_fused: head out dtype %d", d.head_out_dtype);
-      ch.w3 = (const char*)d.head_w;
-      ch.bias3 = d.head_bias;
-      ch.y3 = d.head_y;
-      ch.ldw3 = d.head_ldw;
-      ch.ldy3 = d.head_ldy;
-      ch.n3 = d.head_n;
-      ch.act3 = d.head_act;
-      ch.y3_dtype = d.head_out_dtype;
+      ch.head = head_args(d);
     }
   } else if (d.y == nullptr) {
     return bz::fail(BZ_EINVAL, "bz_fc_fused: null y");
