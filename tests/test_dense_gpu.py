@@ -833,3 +833,21 @@ def test_attention_mlp_as_one_launch(bz, oracle, in_name, r0, r1, w, N, N2, N3, 
 @pytest.mark.parametrize("N3,head_act", [(1, "sigmoid"), (2, "none"), (3, "sigmoid"), (8, "softmax")])
 def test_attention_mlp_with_heads_of_either_unrolling(bz, oracle, in_name, N3, head_act):
     test_attention_mlp_as_one_launch(bz, oracle, in_name, 37, 5, 24, 96, 64, N3, "prelu", head_act)
+
+
+@pytest.mark.parametrize("in_name", ["f16", "bf16"])
+@pytest.mark.parametrize("r0,r1,w,N,N2,N3,act2,head_act", [
+    (1, 1, 8, 16, 16, 1, "dice", "none"),          # the narrowest, one row
+    (3, 5, 10, 16, 16, 2, "relu", "softmax"),      # one row short of a tile, a chunk of which six are the one before's
+    (16, 1, 30, 24, 40, 3, "prelu", "sigmoid"),    # one tile, half a block
+    (17, 1, 32, 40, 64, 8, "dice", "softmax"),     # one row over, a whole step
+    (5, 13, 34, 80, 40, 1, "relu", "none"),        # two columns into the next step
+    (11, 6, 56, 96, 64, 0, "dice", "none"),        # the widest; no third layer
+    (7, 50, 40, 45, 17, 0, "prelu", "none"),
+    (9, 7, 48, 33, 9, 0, "dice", "none"),
+    (2100, 8, 18, 80, 40, 1, "dice", "none"),      # eight waves a workgroup
+    (1500, 50, 24, 80, 40, 2, "dice", "softmax"),  # several tiles a wave, the last ones fewer
+    (40, 3, 6, 24, 16, 1, "dice", "none"),         # narrower than a chunk: the general form
+])
+def test_attention_mlp_at_the_edges_of_its_tiles(bz, oracle, in_name, r0, r1, w, N, N2, N3, act2, head_act):
+    test_attention_mlp_as_one_launch(bz, oracle, in_name, r0, r1, w, N, N2, N3, act2, head_act)

@@ -9,6 +9,7 @@
 #include "bz_common.h"
 
 namespace bz {
+struct CewP;  // bz_pieces.h
 namespace fc {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -269,15 +270,16 @@ template <int N>
 __device__ __forceinline__ float row_shl(float v) {  // lane i of a row of 16: lane i + N's
   return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x100 + N, 0xf, 0xf, true));
 }
+__device__ __forceinline__ float row_quarters_sum(float v) {  // of lanes l, l ^ 16, l ^ 32, l ^ 48, in all four
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
 template <int W>
 __device__ __forceinline__ float group_sum(float v) {
   static_assert(W == 2 || W == 4 || W == 8 || W == 16 || W == 64, "a power of two within a row, or the wave");
-  if constexpr (W == 64) {
-    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
-  }
+  if constexpr (W == 64) v = row_quarters_sum(v);
   if constexpr (W >= 16) v += row_shl<8>(v);
   if constexpr (W >= 8) v += row_shl<4>(v);
   if constexpr (W >= 4) v += row_shl<2>(v);
@@ -302,6 +304,9 @@ inline HeadArgs head_args(const bz_fc_desc& d) {
 // fc_pieces.hip: the layer whose A operand is given as pieces (bz_fc_desc.a_pieces); called by bz_fc_fused after its
 // argument checks
 int fc_pieces_launch(const bz_fc_desc& d, const fc::Epilogue& ep, hipStream_t st);
+// fc_attention.hip: the layer on pieces [x, y, x - y, x * y] with a second and a skinny third one, all 2-byte; called by
+// fc_pieces.hip, which has checked the descriptor.  BZ_ENOTSUP, with nothing launched, for a width it does not take.
+int fc_attention(const bz_fc_desc& d, const CewP& p, const fc::Epilogue& ep1, const fc::Epilogue& ep2, hipStream_t st);
 // the epilogue of a checked descriptor's (first) layer
 fc::Epilogue fc_epilogue(const bz_fc_desc& d);
 // The layer on a stored A, one function per operand type (fc_fused_f16.hip, fc_fused_bf16.hip, fc_fused_f32.hip): with a

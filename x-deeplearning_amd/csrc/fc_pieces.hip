@@ -63,7 +63,7 @@ __host__ __device__ inline int pieces_lds(int k, int tn, int out_size, bool chai
 }
 
 // XY4: the pieces are exactly [x, y, x - y, x * y] of two operands (the attention input): a lane loads x and y once and
-// makes all four from them, instead of addressing and loading eight operands.
+// makes all four from them, instead of addressing and loading eight operands.  (Not with CHAIN: fc_attention.hip's.)
 // CHAIN: a wave goes on with its 32 rows through a second layer of at most 64 columns and a skinny third one; what the
 // layers hand each other is rounded to the tensor type and staged in the wave's rows of LDS, where the separate launches
 // would have stored it and read it back.
@@ -597,12 +597,14 @@ int launch_pieces(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   };
   const bool xy4 = p.n == 4 && p.op[0] == BZ_EW_ASSIGN && p.op[1] == BZ_EW_ASSIGN && p.op[2] == BZ_EW_SUB && p.op[3] == BZ_EW_MUL &&
                    same(2, false, 0) && same(2, true, 1) && same(3, false, 0) && same(3, true, 1);
+  if (chain && xy4) {
+    const int rc2 = bz::fc_attention(d, p, ep, ch.ep2, st);
+    if (rc2 != BZ_ENOTSUP) return rc2;
+  }
 #define BZ_PIECES_V(V)                                                                                         \
   do {                                                                                                         \
     if constexpr (sizeof(OutT) == 2) {                                                                         \
-      if (chain)                                                                                               \
-        return xy4 ? launch_pieces_tn<DT, OutT, V, 4, true, true>(d, p, ep, stage_y, smem, ch, st)             \
-                   : launch_pieces_tn<DT, OutT, V, 4, false, true>(d, p, ep, stage_y, smem, ch, st);           \
+      if (chain) return launch_pieces_tn<DT, OutT, V, 4, false, true>(d, p, ep, stage_y, smem, ch, st);        \
     }                                                                                                          \
     return xy4 ? launch_pieces_tn<DT, OutT, V, 4, true, false>(d, p, ep, stage_y, smem, ch, st)                \
                : launch_pieces_tn<DT, OutT, V, 4, false, false>(d, p, ep, stage_y, smem, ch, st);              \
