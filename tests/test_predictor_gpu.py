@@ -965,6 +965,48 @@ def test_outputs_copied_ahead_of_output(pb):
         assert pb.allocation_count() == before
 
 
+@pytest.mark.parametrize("touched", ["by nothing else", "read by an operator", "written in place"])
+def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
+    """A skinny layer (s) and a layer's skinny head (p) write the host's copy of their outputs themselves, up to 64 KB: read
+    after every pass, some passes or twice, at growing and shrinking batches; and where another operator of the net reads or
+    overwrites the output, which is then copied as it is in the end."""
+    rng = np.random.default_rng(16)
+    w1, w2, w3 = (rng.standard_normal(s).astype(np.float32) * 0.3 for s in ((40, 16), (16, 2), (40, 3)))
+    nb = pb.NetBuilder("copies", device_type=1)
+    nb.external_input("x", 1)
+    for k, w in (("w1", w1), ("w2", w2), ("w3", w3)):
+        nb.constant(k, w)
+    nb.op("Gemm", ["x", "w1"], ["h"], transB=0)
+    nb.op("Sigmoid", ["h"], ["hs"])
+    nb.op("Gemm", ["hs", "w2"], ["z"], transB=0)
+    nb.op("Softmax", ["z"], ["p"], axis=1)
+    nb.op("Gemm", ["x", "w3"], ["s"], transB=0)
+    outs = ["p", "s"]
+    if touched == "read by an operator":
+        nb.op("Sigmoid", ["s"], ["s2"])
+        nb.op("Sigmoid", ["p"], ["p2"])
+        outs += ["p2", "s2"]
+    elif touched == "written in place":
+        nb.constant("one", np.ones((1, 3), np.float32))
+        nb.op("Add", ["s", "one"], ["s"])
+    for o in outs:
+        nb.external_output(o, 1)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for batch in (1, 300, 5461, 5462, 8192, 8193, 7):  # 64 KB are 8192 rows of p, 5461 of s
+        for step in range(5):
+            x = rng.standard_normal((batch, 40)).astype(np.float32)
+            p.feed("x", x)
+            p.forward()
+            d = x.astype(np.float64)
+            e = np.exp(_sigmoid(d @ w1) @ w2)
+            want = {"p": e / e.sum(1, keepdims=True), "s": d @ w3 + (touched == "written in place")}
+            want.update(p2=_sigmoid(want["p"]), s2=_sigmoid(want["s"]))
+            for o in (outs if step != 2 else outs[:1]) + (outs[:1] if step == 3 else []):
+                np.testing.assert_allclose(p.output_asnumpy(o), want[o], rtol=1e-5, atol=1e-5, err_msg="batch %d step %d %s" % (batch, step, o))
+
+
 def test_the_pass_after_the_first_output_allocates_nothing(pb):
     """The buffer that Forward copies an output into is made by Output, not between a launch and its wait."""
     pm = _in_place_net(pb)

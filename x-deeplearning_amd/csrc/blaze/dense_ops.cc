@@ -100,6 +100,7 @@ struct FcCall {
   const float* head_bias = nullptr;
   void* head_y = nullptr;
   int head_n = 0, head_act = BZ_ACT_NONE, head_y_dtype = kFloat;
+  void* copy = nullptr;  // bz::fc_fused's
 };
 
 // false only with a_pieces, when the kernel does not take them (nothing has been launched then)
@@ -188,7 +189,7 @@ bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st
     BZ_CHECK(rc);
     return true;
   }
-  BZ_CHECK(bz_fc_fused(&d, st));
+  BZ_CHECK(bz::fc_fused(d, c.copy, st));
   return true;
 }
 
@@ -642,7 +643,13 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
         call.act_size = (int)N;
       }
     }
-    return RunFc(call, &packed_b_, &packed_a_, st);
+    // (fused_ or head_: the activation behind the layer is in the launch, so this is the whole output)
+    Blob* out = with_head ? hy : y;
+    const size_t bytes = out->size() * DataTypeSize(out->data_type());
+    if (pieces == nullptr && (with_head || N <= 8)) call.copy = out->host_copy().Take(bytes);
+    if (!RunFc(call, &packed_b_, &packed_a_, st)) return false;
+    if (call.copy != nullptr) out->host_copy().copied = bytes;
+    return true;
   }
 
   void CheckValid() {

@@ -91,10 +91,15 @@ class Predictor {
   std::vector<size_t> output_read_;  // bytes handed out last: may reach beyond a half when the output was larger then
   std::vector<bool> output_wanted_;  // read since the last Forward
   std::vector<bool> output_ahead_;   // the other half holds the last Forward's result
+  std::vector<bool> output_sole_;    // one operator of the net writes it, none reads it
+  std::vector<bool> output_pinned_;  // output_cpu_'s memory, as it was last made, is pinned
   std::vector<Blob*> handed_out_;    // whose device address the caller has
   size_t HostHalf(size_t i) const;   // bytes of a half of output_cpu_[i]
   void* HandOut(Blob* blob);
+  bool CopiedAhead(size_t i) const;
+  void OfferHostCopies();
   void QueueOutputs();
+  void WithdrawHostCopies();
   // pinned staging of fed inputs: Feed copies the caller's bytes here and queues the transfer on the thread's
   // stream; Forward runs behind it on the same stream.  feed_pending_[i]: input i's staging is still being read.
   std::vector<std::shared_ptr<Blob>> input_cpu_;

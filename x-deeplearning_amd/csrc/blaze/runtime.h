@@ -64,6 +64,14 @@ class Blob {
     }
     dims_ = dims;
   }
+  // Memory on the host that takes a copy of the data as well: offered for one pass by the predictor whose output this is,
+  // taken by an operator that writes the whole output in its launch.  `copied`: the bytes that were.
+  struct HostCopy {
+    void* at = nullptr;
+    size_t room = 0, copied = 0;
+    void* Take(size_t bytes) const { return bytes > 0 && bytes <= room ? at : nullptr; }
+  };
+  HostCopy& host_copy() { return host_copy_; }
   // the shape alone, for the output of an operator whose work its consumer has taken over: readers may ask the shape,
   // nobody reads the data (a later Reshape allocates as usual)
   void SetShapeOnly(const std::vector<TIndex>& dims) {
@@ -208,6 +216,7 @@ class Blob {
   bool own_handle_ = true;
   uint64_t version_ = 0;
   TIndex pitch_ = 0;
+  HostCopy host_copy_;
   bool slice_view_ = false;
   bool arena_view_ = false;
   bool unplaced_ = false;

@@ -201,6 +201,7 @@ struct HeadArgs {
   void* y;            // [M, ldy]
   int64_t ldw, ldy;
   int n, act, out_dtype;
+  void* copy;         // the outputs once more, [M, n], or null (fc_fused)
 };
 
 // The code that is unrolled over a head's outputs exists for two (the usual heads) and for kSkinnyMaxN: a short kernel
@@ -249,18 +250,22 @@ __device__ __forceinline__ void head_finish(const HeadArgs& head, const HeadBias
       v[j] = t / (1.f + t);
     }
   }
+  auto store = [&](void* y, int64_t ld) {
 #pragma unroll
-  for (int j = 0; j < HN; ++j) {
-    if (j < head.n) {
-      const int64_t at = (int64_t)m * head.ldy + j;
-      if (head.out_dtype == BZ_F32)
-        store_out<float>((float*)head.y + at, v[j]);
-      else if (head.out_dtype == BZ_F16)
-        store_out<__half>((__half*)head.y + at, v[j]);
-      else
-        store_out<__hip_bfloat16>((__hip_bfloat16*)head.y + at, v[j]);
+    for (int j = 0; j < HN; ++j) {
+      if (j < head.n) {
+        const int64_t at = m * ld + j;
+        if (head.out_dtype == BZ_F32)
+          store_out<float>((float*)y + at, v[j]);
+        else if (head.out_dtype == BZ_F16)
+          store_out<__half>((__half*)y + at, v[j]);
+        else
+          store_out<__hip_bfloat16>((__hip_bfloat16*)y + at, v[j]);
+      }
     }
-  }
+  };
+  store(head.y, head.ldy);
+  if (head.copy != nullptr) store(head.copy, head.n);
 }
 
 // The sum over each aligned group of W lanes, in the group's first lane (the others hold parts): the halves added to each
@@ -286,7 +291,7 @@ __device__ __forceinline__ float group_sum(float v) {
   return v + row_shl<1>(v);
 }
 
-inline HeadArgs head_args(const bz_fc_desc& d) {
+inline HeadArgs head_args(const bz_fc_desc& d, void* copy = nullptr) {
   HeadArgs head;
   head.w = (const char*)d.head_w;
   head.bias = d.head_bias;
@@ -296,6 +301,7 @@ inline HeadArgs head_args(const bz_fc_desc& d) {
   head.n = d.head_n;
   head.act = d.head_act;
   head.out_dtype = d.head_out_dtype;
+  head.copy = copy;
   return head;
 }
 
@@ -311,8 +317,8 @@ int fc_attention(const bz_fc_desc& d, const CewP& p, const fc::Epilogue& ep1, co
 fc::Epilogue fc_epilogue(const bz_fc_desc& d);
 // The layer on a stored A, one function per operand type (fc_fused_f16.hip, fc_fused_bf16.hip, fc_fused_f32.hip): with a
 // head when d.head_n != 0, else the skinny, tile or streaming kernel.  bz_fc_fused has checked the descriptor.
-int fc_run_f16(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st);
-int fc_run_bf16(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st);
-int fc_run_f32(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st);
+int fc_run_f16(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, void* copy, hipStream_t st);
+int fc_run_bf16(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, void* copy, hipStream_t st);
+int fc_run_f32(const bz_fc_desc& d, const fc::Epilogue& ep, bool vec_a, bool vec_w, void* copy, hipStream_t st);
 
 }  // namespace bz

@@ -52,7 +52,12 @@ extern "C" {
 
 int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
   BZ_REQUIRE(desc != nullptr, "bz_fc_fused: null descriptor");
-  const bz_fc_desc& d = *desc;
+  return bz::fc_fused(*desc, nullptr, stream);
+}
+
+}  // extern "C"
+
+int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
   BZ_REQUIRE((d.a || d.a_pieces) && d.w && (d.y || d.head_n > 0 || d.next), "bz_fc_fused: null a/w/y");
   BZ_REQUIRE(d.next == nullptr || d.a_pieces != nullptr, "bz_fc_fused: a second layer (next) only follows a layer on a_pieces");
   BZ_REQUIRE(d.m >= 0 && d.n > 0 && d.k > 0, "bz_fc_fused: bad shape m=%d n=%d k=%d", d.m, d.n, d.k);
@@ -91,6 +96,8 @@ int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
   const bool vec_a = ((uintptr_t)d.a % 16 == 0) && ((d.lda * es) % 16 == 0);
   const bool vec_w = ((uintptr_t)d.w % 16 == 0) && ((d.ldw * es) % 16 == 0);
   hipStream_t st = bz::as_stream(stream);
+  BZ_REQUIRE(copy == nullptr || (d.a_pieces == nullptr && d.n_split == 0 && (d.head_n != 0 || d.n <= kSkinnyMaxN)),
+             "bz_fc_fused: only a head's or a layer's of at most %d columns outputs are copied", kSkinnyMaxN);
   if (d.a_pieces != nullptr) {
     if ((d.head_n != 0 && d.next == nullptr) || d.n_split != 0 || d.bias_rows > 1 || d.act == BZ_ACT_SOFTMAX || es != 2 || !vec_w)
       return bz::fail(BZ_ENOTSUP, "bz_fc_fused: a_pieces take a 2-byte layer with aligned weight rows, no head, no split outputs, no softmax and a per-column bias");
@@ -115,11 +122,13 @@ int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
                d.head_out_dtype);
   }
   switch (d.in_dtype) {
-    case BZ_F16: return bz::fc_run_f16(d, ep, vec_a, vec_w, st);
-    case BZ_BF16: return bz::fc_run_bf16(d, ep, vec_a, vec_w, st);
-    default: return bz::fc_run_f32(d, ep, vec_a, vec_w, st);
+    case BZ_F16: return bz::fc_run_f16(d, ep, vec_a, vec_w, copy, st);
+    case BZ_BF16: return bz::fc_run_bf16(d, ep, vec_a, vec_w, copy, st);
+    default: return bz::fc_run_f32(d, ep, vec_a, vec_w, copy, st);
   }
 }
+
+extern "C" {
 
 int bz_fc_pack_weight(const void* src, int src_dtype, int trans_b, int k, int n, void* dst, int dst_dtype, int64_t ldw,
                       bz_stream_t stream) {

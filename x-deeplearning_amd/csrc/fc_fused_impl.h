@@ -999,7 +999,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
 // NMAX: outputs the code is unrolled for
 template <int DT, typename OutT, int NMAX>
 __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restrict__ A, const char* __restrict__ W,
-                                                           OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
+                                                           OutT* __restrict__ Y, OutT* __restrict__ copy, int M, int N, int K, int64_t lda,
                                                            int64_t ldw, int64_t ldy, int lpr, Epilogue ep) {
   constexpr int CH = In<DT>::kChunk;
   const int tid = threadIdx.x;
@@ -1079,20 +1079,25 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
 #pragma unroll
       for (int n = 0; n < NMAX; ++n)
         if (n < N) store_out<OutT>(Y + out_index(ep, m, n, ldy), v[n]);
+      if (copy != nullptr) {
+#pragma unroll
+        for (int n = 0; n < NMAX; ++n)
+          if (n < N) store_out<OutT>(copy + m * N + n, v[n]);
+      }
     }
   }
 }
 
 template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD = 0, int WK = 1,
           int KACC = default_sums<DT, BM, BN, BK, WM, WN, HEAD, WK>()>
-int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st, void* copy = nullptr) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
   // output rows 16-byte aligned and N a whole number of 16-byte chunks: coalesced stores through LDS
   // (with split outputs every slice must start on a chunk boundary as well)
   const bool vec_y = d.y != nullptr && ((uintptr_t)d.y % 16 == 0) && ((d.ldy * (int64_t)sizeof(OutT)) % 16 == 0) &&
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
-  const HeadArgs head = HEAD != 0 ? head_args(d) : HeadArgs{};
+  const HeadArgs head = HEAD != 0 ? head_args(d, copy) : HeadArgs{};
   hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK, KACC>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
@@ -1136,7 +1141,7 @@ int launch_stream(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 
 // Layer + skinny head in one launch: a workgroup owns whole rows of the first layer's output (N <= 256).
 template <int DT, typename OutT, int HN>
-int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream_t st) {
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   // fp32 is bound by the matrix cores of the CUs that work, so the staged tile's 32 rows waste time while they are few: 16
   // rows a workgroup up to 2048 rows (us alone / with eight streams of the same, the tile's behind: 1024 x 512 -> 256
@@ -1153,24 +1158,24 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   if constexpr (DT == BZ_F32) {
     if (d.m <= 2048) {
       hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
-                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d));
+                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d, copy));
       BZ_LAUNCH_OK("bz_fc_split_head_kernel");
       return BZ_OK;
     }
     // Up to 4096 rows four sums an output, as short as that kernel's (3000 x 512 -> 128 17.9 / 8.3, with two 17.8 / 9.3;
     // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6; measured with the head's code unrolled for eight)
-    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 1, 4>(d, ep, st);
-    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 1, 4>(d, ep, st);
+    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 1, 4>(d, ep, st, copy);
+    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 1, 4>(d, ep, st, copy);
   }
   if (d.n <= 64) {
-    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, HN>(d, ep, st);
-    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN>(d, ep, st);
+    if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, HN>(d, ep, st, copy);
+    return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN>(d, ep, st, copy);
   }
-  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN>(d, ep, st);
+  if (d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN>(d, ep, st, copy);
   // eight waves: with one workgroup per 32 rows only M / 32 CUs work, and each has 288 KB of operands to pull in
   // (two K tiles in flight: with eight waves taking turns that hides the loads, and it was faster than four both alone,
   // 10.5 against 11.3 us on config 2's 512 -> 256 -> 2, and next to other kernels)
-  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, HN>(d, ep, st);
+  return launch_mfma<DT, OutT, 32, 256, BK, 1, 8, 2, true, HN>(d, ep, st, copy);
 }
 
 // The tiles of the staged kernel that both kinds of rows take (ALIGNED: every row starts on 16 bytes and K is a whole
@@ -1287,7 +1292,7 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
 }
 
 template <int DT, typename OutT>
-int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream_t st) {
   const int nchunks = (d.k + In<DT>::kChunk - 1) / In<DT>::kChunk;
   int lpr = 1;
   while (lpr < nchunks && lpr < 64) lpr <<= 1;
@@ -1299,25 +1304,25 @@ int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   // 15.2 and 7.1).
   if (d.n <= 2)
     hipLaunchKernelGGL((bz_fc_skinny_kernel<DT, OutT, 2>), dim3((int)grid), dim3(256), 0, st, (const char*)d.a, (const char*)d.w,
-                       (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
+                       (OutT*)d.y, (OutT*)copy, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
   else
     hipLaunchKernelGGL((bz_fc_skinny_kernel<DT, OutT, kSkinnyMaxN>), dim3((int)grid), dim3(256), 0, st, (const char*)d.a,
-                       (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
+                       (const char*)d.w, (OutT*)d.y, (OutT*)copy, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
   BZ_LAUNCH_OK("bz_fc_skinny_kernel");
   return BZ_OK;
 }
 
 template <int DT>
-int dispatch_out(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
+int dispatch_out(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, void* copy, hipStream_t st) {
   const bool skinny = d.n <= kSkinnyMaxN;
   switch (d.out_dtype) {
     case BZ_F32:
-      return skinny ? dispatch_skinny<DT, float>(d, ep, st) : dispatch_tiles<DT, float>(d, ep, vec_a, vec_w, st);
+      return skinny ? dispatch_skinny<DT, float>(d, ep, copy, st) : dispatch_tiles<DT, float>(d, ep, vec_a, vec_w, st);
     case BZ_F16:
-      return skinny ? dispatch_skinny<DT, __half>(d, ep, st)
+      return skinny ? dispatch_skinny<DT, __half>(d, ep, copy, st)
                     : dispatch_tiles<DT, __half>(d, ep, vec_a, vec_w, st);
     case BZ_BF16:
-      return skinny ? dispatch_skinny<DT, __hip_bfloat16>(d, ep, st)
+      return skinny ? dispatch_skinny<DT, __hip_bfloat16>(d, ep, copy, st)
                     : dispatch_tiles<DT, __hip_bfloat16>(d, ep, vec_a, vec_w, st);
     default:
       return bz::fail(BZ_EINVAL, "bz_fc_fused: unsupported out dtype %d", d.out_dtype);
@@ -1327,9 +1332,9 @@ int dispatch_out(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w
 
 // one operand type's entry: the layer with a head, or the plain layer (skinny / tile / streaming kernel)
 template <int DT, typename T>
-int run_typed(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, hipStream_t st) {
-  if (d.head_n != 0) return bz::fc::head_unroll(d.head_n) == 2 ? dispatch_head<DT, T, 2>(d, ep, st) : dispatch_head<DT, T, kSkinnyMaxN>(d, ep, st);
-  return dispatch_out<DT>(d, ep, vec_a, vec_w, st);
+int run_typed(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec_w, void* copy, hipStream_t st) {
+  if (d.head_n != 0) return bz::fc::head_unroll(d.head_n) == 2 ? dispatch_head<DT, T, 2>(d, ep, copy, st) : dispatch_head<DT, T, kSkinnyMaxN>(d, ep, copy, st);
+  return dispatch_out<DT>(d, ep, vec_a, vec_w, copy, st);
 }
 
 }  // namespace
