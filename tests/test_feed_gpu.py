@@ -42,6 +42,19 @@ def test_feed(range_bytes, pieces):
         assert torch.equal(d.cpu(), want), (n, w, sp, dp)
 
 
+@pytest.mark.parametrize("range_bytes,pieces", [
+    (384 << 10, []),                                           # the most of which a lane asks for one unit at a time
+    ((384 << 10) + 16, []),
+    ((384 << 10) - 7 * 130, [(7, 130, 132, 140)]),             # the same with pieces
+    ((384 << 10) - 7 * 130 + 16, [(7, 130, 132, 140)]),
+    (4096, [(257, 1, 1, 3), (2, 255, 256, 300), (256, 3, 4, 5)]),                       # pieces of a workgroup and one unit
+    (400000, [(513, 1, 1, 3), (2, 511, 512, 600), (1, 512, 512, 512), (3001, 6, 6, 9)]),  # the same at two units a lane
+    (0, [(1, 100000, 100000, 100000), (100000, 1, 2, 1), (40000, 7, 8, 7)]),             # rows longer than a workgroup, and shorter than a lane's stride
+])
+def test_feed_at_the_edges_of_its_two_sizes(range_bytes, pieces):
+    test_feed(range_bytes // 16 * 16, pieces)
+
+
 def test_feed_refuses():
     rows = (bz.FeedRows * 9)()
     buf = torch.zeros(64, dtype=torch.uint8).pin_memory()
