@@ -760,11 +760,22 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 //    the lines they share are L1 hits.  So rows that start on no 16 bytes need no path of their own here.
 // Loaded straight into fragments a group of 16 lanes touches 16 lines, and the path into the CU takes a line a clock:
 // 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile); 32 x 2075 -> 768 fp32 17.0, 14.4 (51.7).
-constexpr int kSplitUnit = 128, kSplitPitch = kSplitUnit + 16;
+constexpr int kSplitUnit = 128;
+// Where chunk `chunk` of row `row` lies.  2-byte operands: rows 16 bytes further apart than they are long, so that a fragment
+// read's sixteen lanes (one chunk of sixteen rows) are on all banks.  fp32, which moves twice the bytes for as many products:
+// rows side by side, their chunks in an order of the row's own, so that a write's (two rows) are as well (1024 x 896 -> 512
+// 14.6 us, 13.5 this way, 2048 x 512 -> 256 with a head 18.1 and 17.2; fp16 1024 x 896 -> 512 5.8 and 5.9).
+template <int DT>
+constexpr int kSplitPitch = DT == BZ_F32 ? kSplitUnit : kSplitUnit + 16;
+template <int DT>
+__device__ __forceinline__ int split_at(int row, int chunk) {
+  return row * kSplitPitch<DT> + (DT == BZ_F32 ? (chunk ^ (row >> 1)) & 7 : chunk) * 16;
+}
 
 // One wave's 8 * P rows of an operand, a unit of K at a time: global memory -> registers (lane: row l / 8 of each pass,
-// chunk l % 8) -> LDS rows kSplitPitch apart.
-template <int DT, int P>
+// chunk l % 8) -> LDS as split_at has it.
+// CHUNKS: K is a whole number of chunks (a layer with a head's is)
+template <int DT, int P, bool CHUNKS = false>
 struct SplitRows {
   static constexpr int ES = In<DT>::kSize, CH = In<DT>::kChunk;
   const char* p[P];
@@ -781,36 +792,44 @@ struct SplitRows {
   // the unit that K ends in: zeros beyond K
   __device__ __forceinline__ void load_last(int u, int K, int lane) {
     const int k = u * (kSplitUnit / ES) + (lane & 7) * CH;
+    if constexpr (CHUNKS) {
+      const uint32_t have = k < K ? 0xffffffffu : 0u;
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-      if (K >= CH)
-        r[i] = shift_chunk<DT>(load_chunk_anywhere<DT>(p[i], 0, 0, k, K), k - min(k, K - CH));
-      else
-        r[i] = load_chunk<DT>(p[i], 0, 0, k, K);
+      for (int i = 0; i < P; ++i) __builtin_memcpy(&r[i], p[i] + (int64_t)min(k, K - CH) * ES, 16);
+#pragma unroll
+      for (int i = 0; i < P; ++i) r[i] = make_uint4(r[i].x & have, r[i].y & have, r[i].z & have, r[i].w & have);
+    } else {
+#pragma unroll
+      for (int i = 0; i < P; ++i) {
+        if (K >= CH)
+          r[i] = shift_chunk<DT>(load_chunk_anywhere<DT>(p[i], 0, 0, k, K), k - min(k, K - CH));
+        else
+          r[i] = load_chunk<DT>(p[i], 0, 0, k, K);
+      }
     }
   }
   __device__ __forceinline__ void store(char* lds, int lane) const {
 #pragma unroll
-    for (int i = 0; i < P; ++i) *(uint4*)(lds + (i * 8 + (lane >> 3)) * kSplitPitch + (lane & 7) * 16) = r[i];
+    for (int i = 0; i < P; ++i) *(uint4*)(lds + split_at<DT>(i * 8 + (lane >> 3), lane & 7)) = r[i];
   }
 };
 
-template <int DT, typename OutT, int NW>
+template <int DT, typename OutT, int NW, bool CHUNKS>
 __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                  OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                  int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
   using T = In<DT>;
   constexpr int STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
   constexpr int PITCH = 33;
-  __shared__ __attribute__((aligned(16))) char lds[NW][64 * kSplitPitch];
-  static_assert(32 * PITCH * 4 <= 64 * kSplitPitch, "a partial tile fits where its wave's operands were");
+  __shared__ __attribute__((aligned(16))) char lds[NW][64 * kSplitPitch<DT>];
+  static_assert(32 * PITCH * 4 <= 64 * kSplitPitch<DT>, "a partial tile fits where its wave's operands were");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = (int)(blockIdx.x % tiles_m) * 32, n0 = (int)(blockIdx.x / tiles_m) * 32;
   const int frow = lane & 31, fhalf = lane >> 5;
   char* la = lds[wave];
-  char* lw = la + 32 * kSplitPitch;
-  SplitRows<DT, 4> ra, rw;
+  char* lw = la + 32 * kSplitPitch<DT>;
+  SplitRows<DT, 4, CHUNKS> ra, rw;
   ra.init(A, lda, m0, M, lane);
   rw.init(W, ldw, n0, N, lane);
   floatx16 acc;
@@ -836,8 +855,7 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < STEPS; ++ks)
-      T::mma(*(const uint4*)(la + frow * kSplitPitch + fhalf * 16 + ks * 32),
-             *(const uint4*)(lw + frow * kSplitPitch + fhalf * 16 + ks * 32), acc);
+      T::mma(*(const uint4*)(la + split_at<DT>(frow, fhalf + ks * 2)), *(const uint4*)(lw + split_at<DT>(frow, fhalf + ks * 2)), acc);
     __builtin_amdgcn_wave_barrier();
   }
   // a lane owns column lane & 31 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: the upper half of the waves leave theirs
@@ -887,7 +905,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
   using T = In<DT>;
   static_assert(sizeof(OutT) == T::kSize, "the head reads the tile with the operand type");
   constexpr int ES = T::kSize, STEPS = kSplitUnit / 64, COLS = 256 / 64;
-  constexpr int kHeadStage = 48 * kSplitPitch;
+  constexpr int kHeadStage = 48 * kSplitPitch<DT>;
   __shared__ __attribute__((aligned(16))) char lds[kHeadWaves * kHeadStage];
   static_assert(16 * 33 * 4 <= kHeadStage, "the partial blocks fit");
   const int tid = threadIdx.x, lane = tid & 63;
@@ -895,12 +913,11 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
   const int m0 = blockIdx.x * 16;
   // the row's columns of this lane: their parameters and the head's weights, asked for first
   float cb[COLS], q0[COLS], q1[COLS], q2[COLS];
-  OutT hw[HN][COLS];
+  OutT hw[HN == 2 ? HN : 1][COLS];  // (eight outputs' beside the operands do not fit the registers: read at the end)
   const HeadBias<HN> hbias(head);
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const int n = min(lane + 64 * c, N - 1);
-    const OutT* w2 = (const OutT*)head.w + n;
     cb[c] = ep.bias_rows == 1 ? ep.bias[n] : 0.f;
     q0[c] = q1[c] = q2[c] = 0.f;
     if (ep.act == BZ_ACT_PRELU) q0[c] = ep.p0[ep.act_size == 1 ? 0 : n];
@@ -909,8 +926,10 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
       q1[c] = ep.p1[n];
       q2[c] = ep.p2[n];
     }
+    if constexpr (HN == 2) {
 #pragma unroll
-    for (int j = 0; j < HN; ++j) hw[j][c] = w2[(j < head.n ? j : head.n - 1) * head.ldw];
+      for (int j = 0; j < HN; ++j) hw[j][c] = ((const OutT*)head.w + n)[(j < head.n ? j : head.n - 1) * head.ldw];
+    }
   }
   const int nb = (N + 31) / 32, parts = kHeadWaves / nb, pitch = nb * 32 + 1;
   const int part = wave / nb, block = wave - part * nb;
@@ -920,9 +939,9 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
   for (int r = 0; r < 4; ++r) acc[0][r] = acc[1][r] = 0.f;
   if (part < parts) {
     char* la = lds + wave * kHeadStage;
-    char* lw = la + 16 * kSplitPitch;
-    SplitRows<DT, 2> ra;
-    SplitRows<DT, 4> rw;
+    char* lw = la + 16 * kSplitPitch<DT>;
+    SplitRows<DT, 2, true> ra;
+    SplitRows<DT, 4, true> rw;
     ra.init(A, lda, m0, M, lane);
     rw.init(W, ldw, block * 32, N, lane);
     const int64_t kbytes = (int64_t)K * ES;
@@ -945,9 +964,9 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < STEPS; ++s) {
-        const uint4 a = *(const uint4*)(la + frow * kSplitPitch + s * 64 + fq * 16);
-        T::mma16(a, *(const uint4*)(lw + frow * kSplitPitch + s * 64 + fq * 16), acc[0]);
-        T::mma16(a, *(const uint4*)(lw + (16 + frow) * kSplitPitch + s * 64 + fq * 16), acc[1]);
+        const uint4 a = *(const uint4*)(la + split_at<DT>(frow, s * 4 + fq));
+        T::mma16(a, *(const uint4*)(lw + split_at<DT>(frow, s * 4 + fq)), acc[0]);
+        T::mma16(a, *(const uint4*)(lw + split_at<DT>(16 + frow, s * 4 + fq)), acc[1]);
       }
       __builtin_amdgcn_wave_barrier();
     }
@@ -985,7 +1004,10 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
       store_out<OutT>(&y, apply_act_regs(fmaf(ep.alpha, sum[c], ep.beta * cb[c]), ep, q0[c], q1[c], q2[c]));
       if (Y != nullptr) Y[(int64_t)m * ldy + n] = y;
 #pragma unroll
-      for (int j = 0; j < HN; ++j) dot[j] = fmaf((float)y, (float)hw[j][c], dot[j]);
+      for (int j = 0; j < HN; ++j) {
+        const OutT w = HN == 2 ? hw[HN == 2 ? j : 0][c] : ((const OutT*)head.w + n)[(j < head.n ? j : head.n - 1) * head.ldw];
+        dot[j] = fmaf((float)y, (float)w, dot[j]);
+      }
     }
   }
 #pragma unroll
@@ -1108,7 +1130,9 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st, void* c
 template <int DT, typename OutT, int NW>
 int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 31) / 32, tiles_n = (d.n + 31) / 32;
-  hipLaunchKernelGGL((bz_fc_split_kernel<DT, OutT, NW>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a,
+  // (K of whole chunks has a tail without shifts and branches: 2000 x 144 -> 200 fp32 6.1 us, 5.6 this way)
+  const auto kernel = d.k % In<DT>::kChunk == 0 ? bz_fc_split_kernel<DT, OutT, NW, true> : bz_fc_split_kernel<DT, OutT, NW, false>;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a,
                      (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, tiles_m, ep);
   BZ_LAUNCH_OK("bz_fc_split_kernel");
   return BZ_OK;
@@ -1145,8 +1169,8 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream
   constexpr int BK = In<DT>::kSize == 2 ? 64 : 32;
   // fp32 is bound by the matrix cores of the CUs that work, so the staged tile's 32 rows waste time while they are few: 16
   // rows a workgroup up to 2048 rows (us alone / with eight streams of the same, the tile's behind: 1024 x 512 -> 256
-  // 17.9 / 4.6 and 24.6 / 6.3, 2048 x 512 -> 256 18.0 / 8.1 and 24.6 / 6.3, 2000 x 512 -> 128 11.5 / 4.9 and 16.7 / 5.9,
-  // 201 x 200 -> 80 7.2 / 2.0 and 10.4 / 2.8; 4096 x 512 -> 256 18.2 / 16.5 and 24.6 / 15.2).  A row's operands cost more
+  // 17.1 / 4.4 and 24.6 / 6.3, 2048 x 512 -> 256 17.3 / 9.1 and 24.6 / 6.3, 2000 x 512 -> 128 10.9 / 4.7 and 16.7 / 5.9,
+  // 201 x 200 -> 80 6.9 / 1.9 and 10.4 / 2.8; before that kernel's chunks had an order of their own, 4096 x 512 -> 256 18.2 / 16.5 and 24.6 / 15.2).  A row's operands cost more
   // this way, which shows where other kernels fill the chip: of a tower on eight serving threads a pass of 1024 rows took
   // 20.4 us and 21.7 with the tile, of 2048 32.1 and 30.7 (64.0 and 69.1 alone), of 4096 63.6 and 57.0 (84.8 and 89.8).
   // 2-byte layers are not bound by the matrix cores (2048 x 512 -> 256 fp16 8.3 / 3.6, the tile 8.2 / 2.2; 201 x 200 -> 80
