@@ -26,7 +26,8 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
   for (Blob* b : external_output_blob_) {
     int writers = 0, readers = 0;
     for (const auto& op : net_->GetOperators()) {
-      for (int i = 0; i < op->OutputSize(); ++i) writers += op->Output(i) == b;
+      // (a constant's blob is every predictor's: nothing of one pass is kept in it)
+      for (int i = 0; i < op->OutputSize(); ++i) writers += op->Output(i) == b && op->type() != "ConstantFill";
       for (int i = 0; i < op->InputSize(); ++i) readers += op->Input(i) == b;
     }
     output_sole_.push_back(writers == 1 && readers == 0);
@@ -440,16 +441,17 @@ bool Predictor::CopiedAhead(size_t i) const {
 // the attention model at 1024 105..114 -> 102.  Only where nothing else in the net touches the output.
 void Predictor::OfferHostCopies() {
   for (size_t i = 0; i < external_output_blob_.size(); ++i) {
-    Blob::HostCopy& c = external_output_blob_[i]->host_copy();
-    c = Blob::HostCopy();
     if (!output_sole_[i] || !CopiedAhead(i)) continue;
+    Blob::HostCopy& c = external_output_blob_[i]->host_copy();
+    c.copied = 0;
     c.room = std::min(HostHalf(i), kCopiedAheadMax);
     c.at = (char*)output_cpu_[i]->data() + (1 - output_half_[i]) * HostHalf(i);
   }
 }
 
 void Predictor::WithdrawHostCopies() {
-  for (Blob* b : external_output_blob_) b->host_copy() = Blob::HostCopy();
+  for (size_t i = 0; i < external_output_blob_.size(); ++i)
+    if (output_sole_[i]) external_output_blob_[i]->host_copy() = Blob::HostCopy();
 }
 
 void Predictor::QueueOutputs() {
@@ -463,7 +465,7 @@ void Predictor::QueueOutputs() {
     const bool ahead = st != nullptr && CopiedAhead(i) && blob->pitch() == 0 && blob->data() != nullptr && bytes > 0 &&
                        bytes <= std::min(kCopiedAheadMax, HostHalf(i));
     output_wanted_[i] = false;
-    if (ahead && blob->host_copy().copied == bytes) {
+    if (ahead && output_sole_[i] && blob->host_copy().copied == bytes) {
       output_ahead_[i] = true;
     } else if (ahead && n < BZ_FEED_MAX_ROWS) {
       rows[n].src = blob->data();
