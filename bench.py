@@ -240,7 +240,7 @@ def bench_config3(np, torch, bz, pb, threads):
         sets.append((mlp, k, w16, mask))
     mlp_us = graph_timed(torch, lambda i: sets[i % 2][0].run(), 2, 16, warm_ms=20.0)
     tail_us = graph_timed(torch, lambda i: bz.weighted_pool(sets[i % 2][1], sets[i % 2][2], sets[i % 2][3]), 2, 16, warm_ms=20.0)
-    res["roofline_attention_mlp"] = mfma_roofline("bz_fc_pieces_kernel (%dx%d: %d->%d->%d->%d)" % (B, T, att[0], att[1], att[2], att[3]),
+    res["roofline_attention_mlp"] = mfma_roofline("bz_fc_attention_kernel (%dx%d: %d->%d->%d->%d)" % (B, T, att[0], att[1], att[2], att[3]),
                                                   sets[0][0].flops, mlp_us)
     res["roofline_attention_tail"] = hbm_roofline("bz_weighted_pool_kernel (history read once; scores and mask in, weighted sum and plain sum out)",
                                                   B * T * D3 * 2 + 2 * B * T * 2 + 2 * B * D3 * 2, tail_us)
