@@ -598,3 +598,8 @@ def test_fp32_attention_mlp_in_one_launch_equals_layer_by_layer(batch, T, dim, n
     for s, _ in got.values():
         assert np.linalg.norm(s - want) <= 2e-6 * np.linalg.norm(size)
     np.testing.assert_allclose(got[1][1], got[0][1], rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("batch,T,dim,n1,n2", [(40, 7, 18, 50, 17), (9, 23, 16, 80, 9)])
+def test_fp32_attention_mlp_whose_second_layer_has_odd_columns(batch, T, dim, n1, n2):
+    test_fp32_attention_mlp_in_one_launch_equals_layer_by_layer(batch, T, dim, n1, n2)

@@ -851,3 +851,44 @@ def test_attention_mlp_with_heads_of_either_unrolling(bz, oracle, in_name, N3, h
 ])
 def test_attention_mlp_at_the_edges_of_its_tiles(bz, oracle, in_name, r0, r1, w, N, N2, N3, act2, head_act):
     test_attention_mlp_as_one_launch(bz, oracle, in_name, r0, r1, w, N, N2, N3, act2, head_act)
+
+
+@pytest.mark.parametrize("in_name", ["f16", "bf16"])
+@pytest.mark.parametrize("w,N,N2", [(54, 80, 17), (24, 50, 9), (8, 33, 63)])
+def test_attention_mlp_of_odd_columns_equals_the_padded_one(bz, in_name, w, N, N2):
+    """a second layer of columns that are no whole number of blocks, with its head: the bits of the same layer with columns of
+    zeros up to the next multiple of sixteen (which add zeros to the head's sums)"""
+    import ctypes as C
+    import torch
+    torch.manual_seed(w + N2)
+    tdt, dt = _tdtype(in_name), {"f16": bz.F16, "bf16": bz.BF16}[in_name]
+    r0, r1, P = 21, 7, (N2 + 15) // 16 * 16
+    M, K = r0 * r1, 4 * w
+    q, his = torch.randn(r0, w, device="cuda").to(tdt), torch.randn(M, w, device="cuda").to(tdt)
+    W1, W2, W3 = torch.randn(K, N, device="cuda") / K**0.5, torch.zeros(N, P, device="cuda"), torch.zeros(P, 2, device="cuda")
+    b2, slope = torch.zeros(P, device="cuda"), torch.full((P, ), 0.25, device="cuda")
+    W2[:, :N2], W3[:N2], b2[:N2] = torch.randn(N, N2, device="cuda") / N**0.5, torch.randn(N2, 2, device="cuda"), torch.randn(N2, device="cuda")
+    wp1 = bz.pack_weight(W1, False, dt)
+    got = []
+    for n2 in (N2, P):
+        wp2, wp3 = bz.pack_weight(W2[:, :n2].contiguous(), False, dt), bz.pack_weight(W3[:n2].contiguous(), False, dt)
+        z = torch.full((M, 2), float("nan"), device="cuda")
+        d, pd, nx = bz.FcDesc(), bz.ConcatEwDesc(), bz.FcNext()
+        pd.dtype, pd.n, pd.r0, pd.r1 = dt, 4, r0, r1
+        for i, (op, x, y) in enumerate(((bz.EW_ASSIGN, q, None), (bz.EW_ASSIGN, his, None), (bz.EW_SUB, q, his), (bz.EW_MUL, q, his))):
+            pd.op[i], pd.width[i], pd.x[i] = op, w, x.data_ptr()
+            pd.x_stride[i][0], pd.x_stride[i][1] = (w, 0) if x is q else (r1 * w, w)
+            if y is not None:
+                pd.y[i], pd.y_stride[i][0], pd.y_stride[i][1] = y.data_ptr(), r1 * w, w
+        nx.w, nx.ldw, nx.n, nx.bias, nx.act, nx.act_size = wp2.data_ptr(), wp2.stride(0), n2, b2.data_ptr(), bz.ACT_PRELU, n2
+        nx.act_p0, nx.alpha, nx.beta = slope.data_ptr(), 1.0, 1.0
+        d.a_pieces, d.next = C.addressof(pd), C.addressof(nx)
+        d.w, d.ldw, d.m, d.n, d.k, d.ldy, d.in_dtype, d.out_dtype, d.alpha = wp1.data_ptr(), wp1.stride(0), M, N, K, N, dt, dt, 1.0
+        d.act = bz.ACT_SIGMOID
+        d.head_w, d.head_ldw, d.head_y, d.head_ldy, d.head_n, d.head_out_dtype = wp3.data_ptr(), wp3.stride(0), z.data_ptr(), 2, 2, bz.F32
+        d.head_act = bz.ACT_NONE
+        bz.check(bz.lib().bz_fc_fused(C.byref(d), None))
+        torch.cuda.synchronize()
+        got.append(z.cpu().numpy())
+    assert not np.isnan(got[0]).any()
+    np.testing.assert_array_equal(got[0], got[1])

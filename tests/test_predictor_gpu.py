@@ -965,6 +965,46 @@ def test_outputs_copied_ahead_of_output(pb):
         assert pb.allocation_count() == before
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("k,n,heads", [(256, 100, 2), (64, 50, 1), (128, 9, 3), (96, 255, 8), (40, 17, 1), (256, 4 * 25, 8)])
+def test_head_behind_a_layer_of_any_number_of_columns(pb, dtype, k, n, heads):
+    """columns that are no multiple of eight: the head in the layer's launch up to a number of rows, two launches beyond it,
+    against 64 bits from the rounded layer and against two launches throughout (fuse_fc_head: 0)"""
+    rng = np.random.default_rng(k + n)
+    w1, b1 = (rng.standard_normal((k, n)) / np.sqrt(k)).astype(dtype), (rng.standard_normal(n) * 0.1).astype(dtype)
+    w2, b2 = (rng.standard_normal((n, heads)) / np.sqrt(n)).astype(dtype), (rng.standard_normal(heads) * 0.1).astype(dtype)
+    got = {}
+    rows = (1, 15, 300, 1025, (200 << 10) // k, 2048, 2049, (512 << 10) // k + 1)
+    xs = [rng.standard_normal((m, k)).astype(dtype) for m in rows]
+    for fuse in (1, 0):
+        nb = pb.NetBuilder("any%d" % fuse, device_type=1)
+        nb.arg("fuse_fc_head", fuse)
+        code = pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT
+        nb.external_input("x", code)
+        for name, v in (("w1", w1), ("b1", b1), ("w2", w2), ("b2", b2)):
+            nb.constant(name, v)
+        nb.op("Gemm", ["x", "w1", "b1"], ["h"], transB=0)
+        nb.op("Sigmoid", ["h"], ["hs"])
+        nb.op("Gemm", ["hs", "w2", "b2"], ["z"], transB=0)
+        nb.op("Softmax", ["z"], ["p"], axis=1)
+        nb.external_output("p", code)
+        pm = pb.PredictorManager()
+        pm.load_model_from_string(nb.text(), True)
+        p = pm.create_predictor(1, 0)
+        got[fuse] = []
+        for x in xs:
+            p.feed("x", x)
+            p.forward()
+            got[fuse].append(p.output_asnumpy("p").astype(np.float64).reshape(len(x), heads))
+    for x, g1, g0 in zip(xs, got[1], got[0]):
+        h = _sigmoid(x.astype(np.float64) @ w1.astype(np.float64) + b1)
+        e = np.exp(h @ w2.astype(np.float64) + b2)
+        # fp16: h is rounded (2^-11 of at most 1, weights of 1 / sqrt(n)), and so is the result; fp32: sums of k and n terms
+        tol = 4 * 2.0**-11 if dtype == np.float16 else 1e-5
+        for g in (g1, g0):
+            np.testing.assert_allclose(g, e / e.sum(1, keepdims=True), rtol=0, atol=tol, err_msg="%d rows" % len(x))
+
+
 @pytest.mark.parametrize("touched", ["by nothing else", "read by an operator", "written in place"])
 def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
     """A skinny layer (s) and a layer's skinny head (p) write the host's copy of their outputs themselves, up to 64 KB: read

@@ -252,7 +252,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     Blob* b = this->Input(1);
     if (!b_constant_ || transa_ || b->shape().size() != 2 || head_ != nullptr) return false;
     const int N = (int)(transb_ ? b->shape()[0] : b->shape()[1]);
-    if (N > 256 || N <= 8 || N % 8 != 0) return false;
+    if (N > 256 || N <= 8) return false;
     if (this->InputSize() > 2 && (!c_constant_ || (int)this->Input(2)->size() != N)) return false;
     if (fused_ && fused_act_ == BZ_ACT_SOFTMAX) return false;
     *n_out = N;
@@ -478,6 +478,8 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
       if (a->data_type() != y->data_type() || a->data_type() != head_->Input(1)->data_type() || (k * es) % 16 != 0 ||
           (uintptr_t)a->data() % 16 != 0 || a->pitch() != 0)
         return false;
+      const TIndex n = transb_ ? b->shape()[0] : b->shape()[1];
+      if (n % 8 != 0 && (k == 0 || !bz::head_behind_any_columns(a->size() / k, k, (int)es))) return false;
     }
     const auto& a_shape = a->shape();
     const auto& b_shape = b->shape();

@@ -52,5 +52,13 @@ int fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream);
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);
+// Whether it takes a head behind a layer of columns that are no whole number of 16-byte chunks (bz_fc_fused does not; the
+// kernel is the one of sixteen rows a workgroup).  A model's forward alone / us a pass on eight serving threads, one launch and
+// two: fp16 ... -> 256 -> 100 -> 2 of 1 sample 22.9 / 5.3 and 25.0 / 5.8, of 300 25.8 / 6.7 and 28.1 / 7.3, of 2048 27.9 / 7.0 and
+// 30.2 / 7.8, but with 512 in place of 256 29.8 / 9.1 and 31.5 / 8.3; fp32, bound by the matrix cores of the CUs that work, 300
+// of 400 -> 100 30.7 / 7.8 and 31.2 / 8.2, 1024 of 200 -> 50 27.6 / 7.3 and 29.5 / 7.8, but 1024 of 512 -> 100 35.6 / 11.1 and 32.3 / 10.2.
+inline bool head_behind_any_columns(int64_t rows, int64_t k, int element_size) {
+  return rows <= 2048 && rows * k <= (element_size == 4 ? 200 << 10 : 512 << 10);
+}
 
 }  // namespace bz

@@ -27,6 +27,7 @@ __global__ void bz_pack_weight_kernel(const SrcT* __restrict__ src, DstT* __rest
   }
 }
 
+int run(const bz_fc_desc& d, void* copy, bool any_columns, bz_stream_t stream);
 
 }  // namespace
 
@@ -52,12 +53,19 @@ extern "C" {
 
 int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
   BZ_REQUIRE(desc != nullptr, "bz_fc_fused: null descriptor");
-  return bz::fc_fused(*desc, nullptr, stream);
+  return run(*desc, nullptr, false, stream);
 }
 
 }  // extern "C"
 
 int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
+  return run(d, copy, bz::head_behind_any_columns(d.m, d.k, bz::dtype_size(d.in_dtype)), stream);
+}
+
+namespace {
+
+// any_columns: a head may follow a layer whose columns are no whole number of chunks
+int run(const bz_fc_desc& d, void* copy, bool any_columns, bz_stream_t stream) {
   BZ_REQUIRE((d.a || d.a_pieces) && d.w && (d.y || d.head_n > 0 || d.next), "bz_fc_fused: null a/w/y");
   BZ_REQUIRE(d.next == nullptr || d.a_pieces != nullptr, "bz_fc_fused: a second layer (next) only follows a layer on a_pieces");
   BZ_REQUIRE(d.m >= 0 && d.n > 0 && d.k > 0, "bz_fc_fused: bad shape m=%d n=%d k=%d", d.m, d.n, d.k);
@@ -107,7 +115,7 @@ int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
     const int chunk = 16 / es;
     BZ_REQUIRE(d.head_n > 0 && d.head_n <= kSkinnyMaxN && d.head_w && d.head_y, "bz_fc_fused: head of %d outputs (1..%d) or null head_w/head_y",
                d.head_n, kSkinnyMaxN);
-    if (d.n > 256 || d.n <= kSkinnyMaxN || d.n % chunk != 0)
+    if (d.n > 256 || d.n <= kSkinnyMaxN || (d.n % chunk != 0 && !any_columns))
       return bz::fail(BZ_ENOTSUP, "bz_fc_fused: a fused head needs %d < n <= 256 and n a multiple of %d (n=%d)", kSkinnyMaxN, chunk, d.n);
     if (!(vec_a && vec_w && d.k % chunk == 0))
       return bz::fail(BZ_ENOTSUP, "bz_fc_fused: a fused head needs 16-byte aligned operand rows and k a multiple of %d", chunk);
@@ -127,6 +135,8 @@ int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
     default: return bz::fc_run_f32(d, ep, vec_a, vec_w, copy, st);
   }
 }
+
+}  // namespace
 
 extern "C" {
 
