@@ -603,3 +603,40 @@ def test_file_parsers_under_address_and_undefined_behaviour_sanitizers(tmp_path,
     r = subprocess.run([exe, "1500", "7", str(tmp_path / "scratch"), os.path.join(golden, "quick_embedding"), str(ec_file)] + nets,
                        capture_output=True, text=True, errors="replace", timeout=500, env=env)
     assert r.returncode == 0 and "sanitize_host_parsers: done" in r.stdout, (r.returncode, r.stderr[-3000:])
+
+
+def test_a_descriptor_without_a_head_hands_the_kernels_none(tmp_path):
+    """head_n of 0 (or below) means no head whatever the other head_* fields hold: a kernel asks for the bias of the head it is given
+    before it looks at the number of outputs, so a bias handed on would be read in front of its beginning."""
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    src = tmp_path / "head_args.hip"
+    src.write_text(r"""
+#include <string.h>
+#include "fc_common.h"
+int main() {
+  float w[8], bias[8], y[8], copy[8];
+  bz_fc_desc d;
+  memset(&d, 0, sizeof(d));
+  d.head_w = w;
+  d.head_bias = bias;
+  d.head_y = y;
+  d.head_ldw = d.head_ldy = 8;
+  d.head_act = BZ_ACT_SOFTMAX;
+  for (int n = 0; n >= -1; --n) {
+    d.head_n = n;
+    const bz::fc::HeadArgs none = bz::fc::head_args(d, copy);
+    if (none.n != 0 || none.bias != nullptr || none.w != nullptr || none.y != nullptr || none.copy != nullptr) return 1;
+  }
+  d.head_n = 2;
+  const bz::fc::HeadArgs two = bz::fc::head_args(d, copy);
+  return two.n == 2 && two.bias == bias && two.w == (const char*)w && two.y == y && two.copy == copy ? 0 : 2;
+}
+""")
+    exe = str(tmp_path / "head_args")
+    subprocess.run([hipcc, "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
+    assert subprocess.run([exe], timeout=60).returncode == 0

@@ -291,8 +291,11 @@ __device__ __forceinline__ float group_sum(float v) {
   return v + row_shl<1>(v);
 }
 
+// The descriptor's head; all zero without one, whatever its other head_* fields hold: kernels that may do without a head
+// ask for its bias before they look at head.n, and bias[head.n - 1] would lie in front of it.
 inline HeadArgs head_args(const bz_fc_desc& d, void* copy = nullptr) {
-  HeadArgs head;
+  HeadArgs head = {};
+  if (d.head_n <= 0) return head;
   head.w = (const char*)d.head_w;
   head.bias = d.head_bias;
   head.y = d.head_y;
