@@ -1005,6 +1005,61 @@ def test_head_behind_a_layer_of_any_number_of_columns(pb, dtype, k, n, heads):
             np.testing.assert_allclose(g, e / e.sum(1, keepdims=True), rtol=0, atol=tol, err_msg="%d rows" % len(x))
 
 
+def _launches(p, op_type):
+    ev = json.loads(p.dump_observers()["profile"])["traceEvents"]
+    return sum(e["args"]["launches"] for e in ev if e["name"].split(":")[0] == op_type and e["dur"] > 0)
+
+
+@pytest.mark.parametrize("w,n", [(54, 36), (24, 9)])
+def test_attention_input_in_front_of_a_layer_with_a_head(pb, w, n):
+    """[q, k, q - k, q * k] -> n columns, no multiple of eight -> 1: beyond the rows that a head is in the layer's launch at, the
+    layer computes its input while it loads it and the Concat's tensor is never made; below, the Concat runs and the head
+    is in the launch.  Against the operators one by one."""
+    import torch
+    rng = np.random.default_rng(w)
+    ws = {"w1": (4 * w, n), "b1": (n, ), "g": (n, ), "m": (n, ), "v": (n, ), "w2": (n, 1), "b2": (1, )}
+    ws = {k: (np.abs(rng.standard_normal(sh)) + 0.5 if k == "v" else rng.standard_normal(sh) / np.sqrt(sh[0])).astype(np.float16) for k, sh in ws.items()}
+    reqs = [(rng.standard_normal((B, 1, w)).astype(np.float16), rng.standard_normal((B, T, w)).astype(np.float16)) for B, T in ((600, 50), (1, 20), (683, 3), (600, 50))]
+    got = {}
+    for fuse in (1, 0):
+        nb = pb.NetBuilder("att%d" % fuse, device_type=1)
+        for switch in ("fuse_fc_head", "fuse_concat_into_fc"):
+            nb.arg(switch, fuse)
+        nb.external_input("q", pb.K_FLOAT16)
+        nb.external_input("k", pb.K_FLOAT16)
+        nb.external_output("s", pb.K_FLOAT16)
+        for k, v in ws.items():
+            nb.constant(k, v)
+        nb.op("Sub", ["q", "k"], ["sub"])
+        nb.op("Mul", ["q", "k"], ["mul"])
+        nb.op("BroadcastTo", ["q", "sub"], ["bq"])
+        nb.op("Concat", ["bq", "k", "sub", "mul"], ["a"], axis=2)
+        nb.op("Gemm", ["a", "w1", "b1"], ["h"])
+        nb.op("Dice", ["h", "g", "m", "v"], ["d"])
+        nb.op("Gemm", ["d", "w2", "b2"], ["s"])
+        pm = pb.PredictorManager()
+        pm.load_model_from_string(nb.text(), True)
+        p = pm.create_predictor(1, 0)
+        p.register_observers(["profile"])
+        got[fuse] = []
+        for i, (q, k) in enumerate(reqs):
+            p.feed("q", q)
+            p.feed("k", k)
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            p.forward()
+            if fuse and i == 0:  # the layer's own output is stored, the Concat's (at least as large) is not
+                assert free - torch.cuda.mem_get_info()[0] < q.shape[0] * k.shape[1] * 4 * w * 2
+            got[fuse].append(p.output_asnumpy("s").astype(np.float64))
+            if fuse:
+                assert _launches(p, "Gemm") == 2
+    for (q, k), s1, s0 in zip(reqs, got[1], got[0]):
+        assert s1.shape == (k.shape[0], k.shape[1], 1) and s1.any()
+        # both round the input pieces and the layer's output alike; the layer's sums come in another order: a rounding of its
+        # output of |h| of a few, times weights of 1 / sqrt(n), here and there, and one of the score
+        np.testing.assert_allclose(s1, s0, rtol=0, atol=4 * 2.0**-11 * max(1.0, np.abs(s0).max()))
+
+
 @pytest.mark.parametrize("touched", ["by nothing else", "read by an operator", "written in place"])
 def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
     """A skinny layer (s) and a layer's skinny head (p) write the host's copy of their outputs themselves, up to 64 KB: read

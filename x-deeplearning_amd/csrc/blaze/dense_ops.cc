@@ -328,12 +328,15 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   bool RunOnDevice() override {
     launches_ = 1;
     if (concat_ != nullptr) {
-      if (siblings_.empty() && head_ == nullptr) {
+      if (siblings_.empty() && (head_ == nullptr || !HeadAtAnyRows())) {
         bz_concat_ew_desc pieces;
         auto* c = dynamic_cast<ConcatForFc*>(concat_);
-        if (c != nullptr && c->DescribeAsPieces(&pieces)) {
+        // (the head in this layer's launch is worth more than the stored Concat costs.  The layer on pieces and its head as
+        // a layer / the Concat and both layers in one, alone and with eight serving threads: fp16 rows of 216 -> 36 -> 1, 20
+        // rows 24.6 and 4.7 / 18.7 and 4.4 us, 2000 26.9 and 5.9 / 20.3 and 4.7, but 51200 32.9 and 11.0 / 50.4 and 24.4)
+        if (c != nullptr && c->DescribeAsPieces(&pieces) && !(head_ != nullptr && HeadAtTheseRows())) {
           if (next_ != nullptr && RunSelf(false, &pieces, true)) return true;  // this layer, the next and its head
-          if (RunSelf(false, &pieces)) return RunNextAlone();
+          if (RunSelf(false, &pieces)) return RunHeadAlone() && RunNextAlone();
         }
       }
       // a shape the one-launch form does not take: the Concat runs after all
@@ -348,6 +351,23 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
 
  protected:
+  // whether the head is in this layer's launch at any number of rows, and at those of the input as it is shaped now
+  bool HeadAtAnyRows() {
+    Blob* b = this->Input(1);
+    return (transb_ ? b->shape()[0] : b->shape()[1]) % 8 == 0;
+  }
+  bool HeadAtTheseRows() {
+    Blob *a = this->Input(0), *b = this->Input(1);
+    const TIndex k = transb_ ? b->shape()[1] : b->shape()[0];
+    const int es = (int)DataTypeSize(a->data_type());
+    return HeadAtAnyRows() || (k > 0 && k * es % 16 == 0 && bz::head_behind_any_columns(a->size() / k, k, es));
+  }
+  // the hosted head as a launch of its own
+  bool RunHeadAlone() {
+    if (head_ == nullptr) return true;
+    ++launches_;
+    return head_->RunSelf(false);
+  }
   // the adopted next layer as launches of its own
   bool RunNextAlone() {
     if (next_ == nullptr) return true;
@@ -366,12 +386,15 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
         if (!g->RunSelf(false)) return false;
       return true;
     }
-    if (head_ != nullptr) {
-      if (RunSelf(true)) return true;
-      // an input the one-launch form does not take (unaligned rows, mixed types): one launch per layer
-      return RunSelf(false) && head_->RunSelf(false);
-    }
-    return RunSelf(false);
+    if (head_ == nullptr) return RunSelf(false);
+    launches_ = 0;
+    return RunWithHead();
+  }
+  bool RunWithHead() {
+    ++launches_;
+    if (RunSelf(true)) return true;
+    // an input the one-launch form does not take (unaligned rows, mixed types): one launch per layer
+    return RunSelf(false) && RunHeadAlone();
   }
 
   // this layer and its absorbed siblings as one launch over the stacked weights; every layer's output blob becomes a
@@ -478,8 +501,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
       if (a->data_type() != y->data_type() || a->data_type() != head_->Input(1)->data_type() || (k * es) % 16 != 0 ||
           (uintptr_t)a->data() % 16 != 0 || a->pitch() != 0)
         return false;
-      const TIndex n = transb_ ? b->shape()[0] : b->shape()[1];
-      if (n % 8 != 0 && (k == 0 || !bz::head_behind_any_columns(a->size() / k, k, (int)es))) return false;
+      if (!HeadAtTheseRows()) return false;
     }
     const auto& a_shape = a->shape();
     const auto& b_shape = b->shape();
