@@ -1010,6 +1010,50 @@ def _launches(p, op_type):
     return sum(e["args"]["launches"] for e in ev if e["name"].split(":")[0] == op_type and e["dur"] > 0)
 
 
+@pytest.mark.parametrize("dtype,P,n", [(np.float16, 2, 100), (np.float16, 3, 9), (np.float16, 5, 50), (np.float32, 2, 100), (np.float32, 4, 33)])
+def test_towers_with_heads_on_one_input(pb, dtype, P, n):
+    """P towers K -> n -> 2 written one after the other, n no multiple of eight: up to three 2-byte ones as long as the rows allow
+    a head in a layer's launch each run as one launch, all others as one launch for the layers and one for each head.  Rows
+    below and beyond the limit in turn, against 64 bits from the rounded layer and against one launch for everything."""
+    rng = np.random.default_rng(P * n)
+    code, K = (pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT), 64
+    ws = [[(rng.standard_normal(sh) / np.sqrt(sh[0])).astype(dtype) for sh in ((K, n), (1, n), (n, 2), (1, 2))] for _ in range(P)]
+    xs = [rng.standard_normal((m, K)).astype(dtype) for m in (300, 4096, 1, 2049, 2048, 300)]
+    got = {}
+    for fuse in (1, 0):
+        nb = pb.NetBuilder("towers%d" % fuse, device_type=1)
+        nb.arg("fuse_fc_head", fuse)
+        nb.arg("pack_sibling_gemms", fuse)
+        nb.external_input("x", code)
+        for t, (w, b, u, c) in enumerate(ws):
+            for name, v in (("w", w), ("b", b[0]), ("u", u), ("c", c[0])):
+                nb.constant("%s%d" % (name, t), v)
+            nb.op("Gemm", ["x", "w%d" % t, "b%d" % t], ["h%d" % t])
+            nb.op("Sigmoid", ["h%d" % t], ["s%d" % t])
+            nb.op("Gemm", ["s%d" % t, "u%d" % t, "c%d" % t], ["z%d" % t])
+            nb.op("Softmax", ["z%d" % t], ["p%d" % t], axis=1)
+            nb.external_output("p%d" % t, code)
+        pm = pb.PredictorManager()
+        pm.load_model_from_string(nb.text(), True)
+        p = pm.create_predictor(1, 0)
+        p.register_observers(["profile"])
+        got[fuse] = []
+        for x in xs:
+            p.feed("x", x)
+            p.forward()
+            got[fuse].append([p.output_asnumpy("p%d" % t).astype(np.float64) for t in range(P)])
+            if fuse:
+                heads_in = dtype == np.float16 and P <= 3 and len(x) <= 2048
+                assert _launches(p, "Gemm") == (P if heads_in else 1 + P), len(x)
+    tol = 4 * 2.0**-11 if dtype == np.float16 else 1e-5  # (as for one tower: the rounded layer, weights of 1 / sqrt(n))
+    for x, g1, g0 in zip(xs, got[1], got[0]):
+        for t, (w, b, u, c) in enumerate(ws):
+            h = _sigmoid(x.astype(np.float64) @ w.astype(np.float64) + b)
+            e = np.exp(h @ u.astype(np.float64) + c)
+            for g in (g1[t], g0[t]):
+                np.testing.assert_allclose(g, e / e.sum(1, keepdims=True), rtol=0, atol=tol, err_msg="%d rows, tower %d" % (len(x), t))
+
+
 @pytest.mark.parametrize("w,n", [(54, 36), (24, 9)])
 def test_attention_input_in_front_of_a_layer_with_a_head(pb, w, n):
     """[q, k, q - k, q * k] -> n columns, no multiple of eight -> 1: beyond the rows that a head is in the layer's launch at, the

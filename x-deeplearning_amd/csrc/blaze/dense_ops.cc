@@ -13,6 +13,8 @@
 #include "blaze_hip.h"
 #include "bz_common.h"
 
+#include <algorithm>
+
 namespace blaze {
 
 namespace {
@@ -273,8 +275,10 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   // ---- sibling layers (same input, same shape of constant weight, same arguments) in one launch
   std::string SiblingKey() override {
     Blob* b = this->Input(1);
-    if (!b_constant_ || transa_ || b->shape().size() != 2 || head_ != nullptr || !siblings_.empty()) return "";
+    if (!b_constant_ || transa_ || b->shape().size() != 2 || !siblings_.empty()) return "";
     const TIndex N = transb_ ? b->shape()[0] : b->shape()[1];
+    // (a head that is in the launch at any number of rows is worth more than a sibling)
+    if (head_ != nullptr && N % 8 == 0) return "";
     // (the stacked parameter vectors take N floats from every sibling: a bias of another length is no sibling's)
     if (this->InputSize() > 2 && (!c_constant_ || this->Input(2)->shape().size() != 1 || (TIndex)this->Input(2)->size() != N)) return "";
     if (fused_ && fused_act_ == BZ_ACT_SOFTMAX) return "";
@@ -288,6 +292,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
        << this->device_option().device_id();
     return ss.str();
   }
+  OperatorBase* HeadOp() override { return head_; }
   void AbsorbSiblings(const std::vector<SiblingFc*>& others) override {
     siblings_.clear();
     for (SiblingFc* o : others) siblings_.push_back(static_cast<GemmOp*>(o));
@@ -378,12 +383,28 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   bool RunRest() {
     launches_ = 1;
     if (!siblings_.empty()) {
-      if (RunSiblings()) return true;
-      // an input the one-launch form does not take (3-D, few columns): one launch per layer
-      launches_ = 1 + (int)siblings_.size();
-      if (!RunSelf(false)) return false;
-      for (GemmOp* g : siblings_)
-        if (!g->RunSelf(false)) return false;
+      if (HeadsBeforeSiblings()) {
+        launches_ = 0;
+        if (!RunWithHead()) return false;
+        for (GemmOp* g : siblings_) {
+          g->launches_ = 0;
+          if (!g->RunWithHead()) return false;
+          launches_ += g->launches_;
+        }
+        return true;
+      }
+      if (!RunSiblings()) {
+        // an input the one-launch form does not take (3-D, few columns): one launch per layer
+        launches_ = 1 + (int)siblings_.size();
+        if (!RunSelf(false)) return false;
+        for (GemmOp* g : siblings_)
+          if (!g->RunSelf(false)) return false;
+      }
+      if (!RunHeadAlone()) return false;
+      for (GemmOp* g : siblings_) {
+        launches_ += g->head_ != nullptr;
+        if (!g->RunHeadAlone()) return false;
+      }
       return true;
     }
     if (head_ == nullptr) return RunSelf(false);
@@ -395,6 +416,16 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     if (RunSelf(true)) return true;
     // an input the one-launch form does not take (unaligned rows, mixed types): one launch per layer
     return RunSelf(false) && RunHeadAlone();
+  }
+  // Layers that share an input and have heads: each with its head, or the layers in one launch and the heads behind it.  P
+  // towers 256 -> 100 -> 2, us a pass alone / on eight serving threads, with heads and packed: fp16 P = 2 of 1 sample 19.5 / 4.4
+  // and 21.3 / 4.9, of 2048 22.4 / 5.6 and 25.9 / 6.8; P = 3 of 1 24.0 / 5.2 and 25.2 / 5.6, of 2048 28.0 / 8.0 and 30.5 / 8.1; P = 4
+  // of 1 28.4 / 6.3 and 28.4 / 6.6, of 300 33.6 / 8.3 and 32.6 / 8.0, of 2048 33.7 / 10.5 and 35.2 / 9.6; with more rows than a head
+  // is in the launch at, P = 2 of 4096 32.1 / 8.7 and 26.3 / 7.0.  fp32 P = 2 of 1 24.0 / 5.1 and 20.6 / 4.7, of 2048 27.4 / 7.7 and
+  // 24.8 / 6.7.
+  bool HeadsBeforeSiblings() {
+    if (head_ == nullptr || siblings_.size() > 2 || DataTypeSize(this->Input(0)->data_type()) != 2 || !HeadAtTheseRows()) return false;
+    return std::all_of(siblings_.begin(), siblings_.end(), [](GemmOp* g) { return g->head_ != nullptr; });
   }
 
   // this layer and its absorbed siblings as one launch over the stacked weights; every layer's output blob becomes a

@@ -473,11 +473,15 @@ void SimpleNet::PackSiblingFcs() {
     for (size_t k = idx.front() + 1; k < idx.back() && clean; ++k)
       for (const auto& out : operators_[k]->operator_def().output()) clean &= (out != in);
     // a later sibling's result appears where the first sibling runs: nothing from there up to the sibling's own place may
-    // read or write that name (or the name of the tensor between the sibling and its folded activation)
+    // read or write that name (or the name of the tensor between the sibling and its folded activation, or its head's)
     for (size_t m = 1; m < idx.size() && clean; ++m) {
-      std::set<std::string> names(operators_[idx[m]]->operator_def().output().begin(), operators_[idx[m]]->operator_def().output().end());
-      if (auto* st = dynamic_cast<StackableFc*>(operators_[idx[m]].get()))
-        names.insert(st->StackOutputOp()->operator_def().output().begin(), st->StackOutputOp()->operator_def().output().end());
+      std::set<std::string> names;
+      for (OperatorBase* op : {operators_[idx[m]].get(), dynamic_cast<SiblingFc*>(operators_[idx[m]].get())->HeadOp()}) {
+        if (op == nullptr) continue;
+        names.insert(op->operator_def().output().begin(), op->operator_def().output().end());
+        if (auto* st = dynamic_cast<StackableFc*>(op))
+          names.insert(st->StackOutputOp()->operator_def().output().begin(), st->StackOutputOp()->operator_def().output().end());
+      }
       for (size_t k = idx.front(); k < idx[m] && clean; ++k) {
         for (const auto& in : operators_[k]->operator_def().input()) clean &= names.count(in) == 0;
         for (const auto& out : operators_[k]->operator_def().output()) clean &= names.count(out) == 0;

@@ -161,6 +161,8 @@ class SiblingFc {
   virtual ~SiblingFc() {}
   // empty: not eligible.  Otherwise everything that must agree between siblings, the input blob included.
   virtual std::string SiblingKey() = 0;
+  // the skinny layer this one hosts (StackableFc::AbsorbHead), or null: it runs where this one does
+  virtual OperatorBase* HeadOp() = 0;
   virtual void AbsorbSiblings(const std::vector<SiblingFc*>& others) = 0;
 };
 
