@@ -603,3 +603,69 @@ def test_fp32_attention_mlp_in_one_launch_equals_layer_by_layer(batch, T, dim, n
 @pytest.mark.parametrize("batch,T,dim,n1,n2", [(40, 7, 18, 50, 17), (9, 23, 16, 80, 9)])
 def test_fp32_attention_mlp_whose_second_layer_has_odd_columns(batch, T, dim, n1, n2):
     test_fp32_attention_mlp_in_one_launch_equals_layer_by_layer(batch, T, dim, n1, n2)
+
+
+@pytest.mark.parametrize("batch,T", [(9, 23), (130, 3)])
+def test_fp32_layers_leave_a_concat_that_they_cannot_compute(batch, T):
+    """An fp32 layer of few columns computes its Concat itself only as the first of an attention MLP.  A main tower that starts
+    with 80 columns leaves its Concat to the attention tail, which writes it in its own launch, and a tower behind
+    [x, x - y] leaves it to the net.  Against the operators one by one."""
+    import json
+    import torch
+    import din_model
+    import pyblaze_hip as pb
+    rng = np.random.default_rng(batch)
+    cfg = din_model.Config3(batch=batch, rows=3000, T=T)
+    cfg.dim, d3 = 16, 48
+    weights = {}
+    for tag, layers in (("att", (4 * d3, 80, 40, 1)), ("main", (3 * d3, 80, 40, 2))):
+        weights[tag] = [dict(w=rng.standard_normal((k, n)).astype(np.float32) / np.float32(np.sqrt(k)), b=rng.standard_normal(n).astype(np.float32) * np.float32(0.1),
+                             gamma=rng.standard_normal(n).astype(np.float32) * np.float32(0.1), mean=rng.standard_normal(n).astype(np.float32) * np.float32(0.1),
+                             var=rng.uniform(0.5, 1.5, n).astype(np.float32)) for k, n in zip(layers, layers[1:])]
+    tables = [torch.from_numpy(rng.standard_normal((3000, 16)).astype(np.float32)).cuda() for _ in din_model.KINDS]
+    feed = cfg.batch_inputs()
+
+    def launches(p):
+        ev = json.loads(p.dump_observers()["profile"])["traceEvents"]
+        count = {}
+        for e in ev:
+            if e["dur"] > 0 and e["name"].split(":")[0] in ("Concat", "Gemm", "MatMul"):
+                count[e["name"].split(":")[0]] = count.get(e["name"].split(":")[0], 0) + e["args"]["launches"]
+        return count
+
+    got = {}
+    for fuse in (1, 0):
+        pm, inputs = din_model.build_manager(cfg, tables, weights, np.float32,
+                                             net_args={"fuse_concat_into_fc": fuse, "fuse_concat_into_weighted_pool": fuse, "fuse_fc_head": fuse})
+        p = pm.create_predictor(1, 0)
+        p.register_observers(["profile"])
+        din_model.feed(p, inputs, feed, np.float32)
+        p.forward()
+        got[fuse] = p.output_asnumpy("prob").copy()
+        if fuse:  # the attention MLP; main tower: the first layer, the second with its head
+            assert launches(p) == {"Gemm": 3, "MatMul": 1}
+    np.testing.assert_allclose(got[1], got[0], rtol=1e-5, atol=1e-6)
+
+    w1, w2 = rng.standard_normal((64, 64)).astype(np.float32) / 8, rng.standard_normal((64, 2)).astype(np.float32) / 8
+    x, y = rng.standard_normal((2, batch, 32)).astype(np.float32)
+    nb = pb.NetBuilder("behind_concat", device_type=1)
+    for name in ("x", "y"):
+        nb.external_input(name, pb.K_FLOAT)
+    nb.external_output("z", pb.K_FLOAT)
+    nb.constant("w1", w1)
+    nb.constant("w2", w2)
+    nb.op("Sub", ["x", "y"], ["d"])
+    nb.op("Concat", ["x", "d"], ["c"], axis=1)
+    nb.op("Gemm", ["c", "w1"], ["h"])
+    nb.op("Sigmoid", ["h"], ["s"])
+    nb.op("Gemm", ["s", "w2"], ["z"])
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    p.register_observers(["profile"])
+    p.feed("x", x)
+    p.feed("y", y)
+    p.forward()
+    assert launches(p) == {"Concat": 1, "Gemm": 1}
+    c = np.concatenate([x, x - y], 1).astype(np.float64)
+    np.testing.assert_allclose(p.output_asnumpy("z"), 1 / (1 + np.exp(-(c @ w1))) @ w2, rtol=0, atol=1e-5)

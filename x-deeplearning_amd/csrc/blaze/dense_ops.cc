@@ -300,7 +300,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
 
   // ---- the Concat that makes this layer's input, computed while it is loaded
   // (the static part of what bz_fc_desc.a_pieces takes: a layer of 9..96 columns and at most 224 inputs; an fp32 one only
-  // with the layers behind it, bz::fc_attention_f32)
+  // with the layers behind it, bz::fc_attention_f32: ReleaseConcat)
   bool CanAdoptConcat() override {
     Blob* b = this->Input(1);
     if (!b_constant_ || transa_ || b->shape().size() != 2) return false;
@@ -311,6 +311,18 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
   void AdoptConcat(OperatorBase* concat) override { concat_ = concat; }
   bool HasAdoptedConcat() const override { return concat_ != nullptr; }
+  OperatorBase* ReleaseConcat() override {
+    if (concat_ == nullptr || this->Input(1)->data_type() != kFloat) return nullptr;
+    const auto& b = this->Input(1)->shape();
+    const TIndex K = transb_ ? b[1] : b[0], N = transb_ ? b[0] : b[1];
+    if (next_ != nullptr && next_->head_ != nullptr && head_ == nullptr && dynamic_cast<ConcatForFc*>(concat_)->IsAttentionInput()) {
+      const auto& b2 = next_->Input(1)->shape();
+      if (bz::fc_attention_f32_takes(K, N, next_->transb_ ? b2[0] : b2[1])) return nullptr;
+    }
+    OperatorBase* concat = concat_;
+    concat_ = nullptr;  // (a chained layer stays: it runs behind this one)
+    return concat;
+  }
   bool CanChainNext(OperatorBase* next_op) override {
     auto* g = dynamic_cast<GemmOp*>(next_op);
     if (g == nullptr || concat_ == nullptr || head_ != nullptr || !siblings_.empty() || next_ != nullptr) return false;
@@ -341,7 +353,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
         // rows 24.6 and 4.7 / 18.7 and 4.4 us, 2000 26.9 and 5.9 / 20.3 and 4.7, but 51200 32.9 and 11.0 / 50.4 and 24.4)
         if (c != nullptr && c->DescribeAsPieces(&pieces) && !(head_ != nullptr && HeadAtTheseRows())) {
           if (next_ != nullptr && RunSelf(false, &pieces, true)) return true;  // this layer, the next and its head
-          if (RunSelf(false, &pieces)) return RunHeadAlone() && RunNextAlone();
+          if (this->Input(1)->data_type() != kFloat && RunSelf(false, &pieces)) return RunHeadAlone() && RunNextAlone();
         }
       }
       // a shape the one-launch form does not take: the Concat runs after all

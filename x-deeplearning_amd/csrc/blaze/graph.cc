@@ -223,6 +223,7 @@ SimpleNet::SimpleNet(const std::shared_ptr<const NetDef>& net_def, Workspace* ws
     FuseWeightedPools();
     FuseConcatsIntoFcs();
     ChainNarrowFcs();
+    ReleaseConcats();
     FuseConcatsIntoWeightedPools();
     MergeSiblingEmbeddings();
   }
@@ -449,6 +450,17 @@ void SimpleNet::ChainNarrowFcs() {
     if (readers != 1 || is_output) continue;
     first->AdoptNext(operators_[j].get());
     skipped_[j] = true;
+  }
+}
+
+// An adopted Concat goes back to the net where its layer turns out to be none that computes it (an fp32 layer without the
+// chain behind it): the attention tail may write it then.
+void SimpleNet::ReleaseConcats() {
+  for (size_t i = 0; i < operators_.size(); ++i) {
+    auto* fc = dynamic_cast<ConcatAdopter*>(operators_[i].get());
+    OperatorBase* concat = fc != nullptr ? fc->ReleaseConcat() : nullptr;
+    for (size_t c = 0; concat != nullptr && c < i; ++c)
+      if (operators_[c].get() == concat) skipped_[c] = false;
   }
 }
 

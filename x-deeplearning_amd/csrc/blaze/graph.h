@@ -107,6 +107,7 @@ class SimpleNet : public Net {
   void FuseConcatsIntoWeightedPools();
   void FuseConcatsIntoFcs();
   void ChainNarrowFcs();
+  void ReleaseConcats();
   int ReadersOf(const std::string& name, const OperatorBase* folded) const;
   void InterleaveAssignBlocks();
   void MergeSiblingEmbeddings();
@@ -200,6 +201,8 @@ class ConcatForFc {  // implemented by Concat
   // Describes Output(0) as pieces without computing it and gives the output blob its shape (no memory).  False: the
   // inputs do not fit the piece model; nothing has been touched.
   virtual bool DescribeAsPieces(bz_concat_ew_desc* desc) = 0;
+  // whether the pieces are x, y, x - y, x * y as far as that is known before the operands are (the operators)
+  virtual bool IsAttentionInput() const = 0;
 };
 class ConcatAdopter {  // implemented by Gemm
  public:
@@ -207,6 +210,9 @@ class ConcatAdopter {  // implemented by Gemm
   virtual bool CanAdoptConcat() = 0;  // static part: constant 2-byte weight of a shape the kernel takes, no transposed A
   virtual void AdoptConcat(OperatorBase* concat) = 0;
   virtual bool HasAdoptedConcat() const = 0;
+  // After the layers are chained: a Concat that no launch of this layer can compute is the net's again.  Null when the layer
+  // keeps it.
+  virtual OperatorBase* ReleaseConcat() = 0;
   // The narrow layer after such a layer (with the skinny layer it may already host) in the same launch
   // (bz_fc_desc.next): the attention MLP 4E -> 80 -> 40 -> 1 as one kernel.  `next` reads only this layer's result, and
   // nothing else does.

@@ -247,6 +247,13 @@ class ConcatOp final : public Operator<Context>, public ConcatPieceHost, public 
     std::sort(producers_.begin(), producers_.end(), [](const Adopted& a, const Adopted& b) { return a.position < b.position; });
   }
   bool DescribeAsPieces(bz_concat_ew_desc* desc) override { return RunWithPieces(desc); }
+  bool IsAttentionInput() const override {
+    if (this->InputSize() != 4) return false;
+    std::string op[4];  // (an input that no operator was taken over for, or a BroadcastTo, is a copy)
+    for (const Adopted& a : producers_)
+      if (a.op->type() != "BroadcastTo") op[a.input_idx] = a.op->type();
+    return op[0].empty() && op[1].empty() && op[2] == "Sub" && op[3] == "Mul";
+  }
   // (0 when every input already lives in the output)
   int LaunchesOfLastRun() const override { return launches_; }
   bool RunOnDevice() override {

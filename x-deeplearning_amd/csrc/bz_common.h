@@ -49,6 +49,8 @@ constexpr int kNumXcd = 8;      // MI355X: 8 accelerator complex dies, workgroup
 // fc_attention_f32.hip, for the host layer: bz_fc_fused of an fp32 layer on pieces [x, y, x - y, x * y] with a second and a
 // skinny third layer, of whose outputs only the last is stored.  BZ_ENOTSUP, with nothing launched, for anything else.
 int fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream);
+// whether it takes layers k -> n -> n2
+bool fc_attention_f32_takes(int64_t k, int64_t n, int64_t n2);
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);

@@ -261,6 +261,10 @@ int launch(const Attention& a, int lds, hipStream_t st) {
 
 }  // namespace
 
+bool bz::fc_attention_f32_takes(int64_t k, int64_t n, int64_t n2) {
+  return k <= 4 * 56 && n <= 96 && n2 <= 64 && layout((int)k, (int)n, (int)n2).all * (int)sizeof(float) <= kMaxLds;
+}
+
 int bz::fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream) {
   if (d.a_pieces == nullptr || d.next == nullptr) return bz::fail(BZ_ENOTSUP, "attention MLP: no pieces or no second layer");
   const bz_fc_next& x = *d.next;
@@ -278,10 +282,8 @@ int bz::fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream) {
   const bool xy = bz::cew_uniform(p) && p.n == 4 && p.op[0] == BZ_EW_ASSIGN && p.op[1] == BZ_EW_ASSIGN && p.op[2] == BZ_EW_SUB &&
                   p.op[3] == BZ_EW_MUL && same(2, false, 0) && same(2, true, 1) && same(3, false, 0) && same(3, true, 1);
   auto plain = [](int act) { return act == BZ_ACT_NONE || act == BZ_ACT_PRELU || act == BZ_ACT_DICE || act == BZ_ACT_LEAKY_RELU || act == BZ_ACT_SIGMOID; };
-  const int lds = layout(d.k, d.n, x.n).all * (int)sizeof(float);
   const bool aligned = (uintptr_t)d.w % 16 == 0 && d.ldw % 4 == 0 && (uintptr_t)x.w % 16 == 0 && x.ldw % 4 == 0;
-  if (d.in_dtype != BZ_F32 || d.out_dtype != BZ_F32 || d.a_pieces->dtype != BZ_F32 || !xy || d.k > 4 * 56 || d.n > 96 || x.n > 64 ||
-      lds > kMaxLds || !aligned || d.y != nullptr || x.y != nullptr || d.head_n < 1 || d.head_n > kSkinnyMaxN || d.n_split != 0 ||
+  if (d.in_dtype != BZ_F32 || d.out_dtype != BZ_F32 || d.a_pieces->dtype != BZ_F32 || !xy || !fc_attention_f32_takes(d.k, d.n, x.n) || !aligned || d.y != nullptr || x.y != nullptr || d.head_n < 1 || d.head_n > kSkinnyMaxN || d.n_split != 0 ||
       d.bias_rows > 1 || !plain(d.act) || !plain(x.act) || p.r1 >= (1ll << 31) || d.m >= (1ll << 31) - 256 * kRows)
     return bz::fail(BZ_ENOTSUP, "attention MLP: a shape or form outside the kernel's");
   BZ_REQUIRE(d.w != nullptr && x.w != nullptr && d.head_w != nullptr && d.head_y != nullptr && d.ldw >= d.k && x.ldw >= d.n &&
@@ -324,6 +326,7 @@ int bz::fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream) {
   a.ep2.act_alpha = x.act_alpha;
   a.head = head_args(d);
   hipStream_t st = bz::as_stream(stream);
+  const int lds = layout(d.k, d.n, x.n).all * (int)sizeof(float);
   const bool two = head_unroll(d.head_n) == 2;
   if (vec >= 4) return two ? launch<4, 2>(a, lds, st) : launch<4, kSkinnyMaxN>(a, lds, st);
   if (vec == 2) return two ? launch<2, 2>(a, lds, st) : launch<2, kSkinnyMaxN>(a, lds, st);
