@@ -528,6 +528,35 @@ def test_table_of_more_than_2_to_24_rows_takes_the_plain_load_path(bz, oracle):
     assert np.array_equal(_bits(got), _bits(want))
 
 
+@pytest.mark.parametrize("dtype,dim", [("f16", 8), ("f16", 12), ("i8", 16), ("i8", 40), ("f32", 6)])
+def test_values_of_one_and_others_on_tables_of_more_than_2_to_24_rows(bz, oracle, dtype, dim):
+    """Lists whose values are all 1, lists that weight some of their ids and waves of both kinds, on tables that are read by
+    plain loads: the form for values of 1 adds the same bits as the general one."""
+    rng = np.random.default_rng(dim)
+    rows, batch = (1 << 24) + 5, 200
+    some = rng.standard_normal((4099, dim)) * 0.1
+    table = {"data": np.resize((np.round(some * 300).clip(-127, 127)).astype(np.int8) if dtype == "i8" else some.astype({"f16": np.float16, "f32": np.float32}[dtype]), (rows, dim))}
+    if dtype == "i8":
+        table["scale"] = np.resize(rng.uniform(0.001, 0.01, 997).astype(np.float32), rows)
+    specs, inputs, cols = [], [], []
+    for item, udf in enumerate((0, 1, 0)):
+        seg = rng.integers(0, 12, batch).astype(np.int32)
+        nnz = int(seg.sum())
+        ids = rng.integers(-2, rows + 2, nnz)
+        vals = np.ones(nnz, np.float32)
+        if item == 1:
+            vals[nnz // 2:] = rng.standard_normal(nnz - nnz // 2)
+        elif item == 2:
+            vals[::7] = rng.standard_normal(vals[::7].size)
+        specs.append((0, udf, 0, 0, dim))
+        inputs.append((ids.astype(np.int64), vals, seg))
+        cols.append(item * dim)
+    print("table of %d rows of %s x %d" % (rows, dtype, dim), flush=True)
+    got, _, variant = _run_gpu(bz, [table], specs, inputs, batch, np.float32, (3 * dim, cols))
+    assert variant != 0
+    assert np.array_equal(_bits(got), _bits(_run_oracle(oracle, [table], specs, inputs, batch, (3 * dim, cols))))
+
+
 @pytest.mark.parametrize("batch", [1, 2047, 2048, 2049, 4100, 16385, 20000])
 def test_scan_of_slots_at_the_edges_of_its_tiles(bz, batch):
     """bz_segments_to_offsets_slots: one slot's scan is split into tiles of 2048 counts over up to 8 workgroups, the last of
