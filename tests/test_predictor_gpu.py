@@ -1010,6 +1010,37 @@ def _launches(p, op_type):
     return sum(e["args"]["launches"] for e in ev if e["name"].split(":")[0] == op_type and e["dur"] > 0)
 
 
+@pytest.mark.parametrize("dtype,k,n,rows,launches", [
+    (np.float16, 256, 250, 300, 1), (np.float16, 384, 250, 2048, 1), (np.float16, 384, 250, 2049, 2), (np.float16, 400, 250, 300, 2),
+    (np.float16, 512, 100, 1536, 1), (np.float16, 512, 100, 1537, 2), (np.float32, 144, 250, 300, 1), (np.float32, 400, 250, 300, 2),
+    (np.float32, 400, 92, 614, 1), (np.float32, 400, 92, 615, 2), (np.float32, 400, 93, 1, 2), (np.float32, 64, 100, 2049, 2)])
+def test_a_head_behind_any_columns_stays_where_it_is_faster(pb, dtype, k, n, rows, launches):
+    """the lines in k * n, rows * k and rows up to which a head rides behind columns that are no multiple of eight"""
+    rng = np.random.default_rng(k + n)
+    w1, w2 = (rng.standard_normal((k, n)) / np.sqrt(k)).astype(dtype), (rng.standard_normal((n, 1)) / np.sqrt(n)).astype(dtype)
+    code = pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT
+    nb = pb.NetBuilder("line", device_type=1)
+    nb.external_input("x", code)
+    nb.external_output("z", code)
+    nb.constant("w1", w1)
+    nb.constant("w2", w2)
+    nb.op("Gemm", ["x", "w1"], ["h"])
+    nb.op("Sigmoid", ["h"], ["s"])
+    nb.op("Gemm", ["s", "w2"], ["z"])
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    p.register_observers(["profile"])
+    x = rng.standard_normal((rows, k)).astype(dtype)
+    p.feed("x", x)
+    p.forward()
+    assert _launches(p, "Gemm") == launches
+    want = _sigmoid(x.astype(np.float64) @ w1.astype(np.float64)) @ w2.astype(np.float64)
+    # fp16: the layer's output is rounded (2^-11 of at most 1, n weights of 1 / sqrt(n) whose errors go both ways), and the result
+    tol = (4 + 2 * np.abs(want).max()) * 2.0**-11 if dtype == np.float16 else 1e-5
+    np.testing.assert_allclose(p.output_asnumpy("z").astype(np.float64), want, rtol=0, atol=tol)
+
+
 @pytest.mark.parametrize("dtype,P,n", [(np.float16, 2, 100), (np.float16, 3, 9), (np.float16, 5, 50), (np.float32, 2, 100), (np.float32, 4, 33)])
 def test_towers_with_heads_on_one_input(pb, dtype, P, n):
     """P towers K -> n -> 2 written one after the other, n no multiple of eight: up to three 2-byte ones as long as the rows allow

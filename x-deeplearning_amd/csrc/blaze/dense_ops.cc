@@ -375,9 +375,9 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
   bool HeadAtTheseRows() {
     Blob *a = this->Input(0), *b = this->Input(1);
-    const TIndex k = transb_ ? b->shape()[1] : b->shape()[0];
+    const TIndex k = transb_ ? b->shape()[1] : b->shape()[0], n = transb_ ? b->shape()[0] : b->shape()[1];
     const int es = (int)DataTypeSize(a->data_type());
-    return HeadAtAnyRows() || (k > 0 && k * es % 16 == 0 && bz::head_behind_any_columns(a->size() / k, k, es));
+    return HeadAtAnyRows() || (k > 0 && k * es % 16 == 0 && bz::head_behind_any_columns(a->size() / k, k, n, es));
   }
   // the hosted head as a launch of its own
   bool RunHeadAlone() {

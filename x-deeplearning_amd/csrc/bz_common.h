@@ -55,12 +55,21 @@ bool fc_attention_f32_takes(int64_t k, int64_t n, int64_t n2);
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);
 // Whether it takes a head behind a layer of columns that are no whole number of 16-byte chunks (bz_fc_fused does not; the
-// kernel is the one of sixteen rows a workgroup).  A model's forward alone / us a pass on eight serving threads, one launch and
-// two: fp16 ... -> 256 -> 100 -> 2 of 1 sample 22.9 / 5.3 and 25.0 / 5.8, of 300 25.8 / 6.7 and 28.1 / 7.3, of 2048 27.9 / 7.0 and
-// 30.2 / 7.8, but with 512 in place of 256 29.8 / 9.1 and 31.5 / 8.3; fp32, bound by the matrix cores of the CUs that work, 300
-// of 400 -> 100 30.7 / 7.8 and 31.2 / 8.2, 1024 of 200 -> 50 27.6 / 7.3 and 29.5 / 7.8, but 1024 of 512 -> 100 35.6 / 11.1 and 32.3 / 10.2.
-inline bool head_behind_any_columns(int64_t rows, int64_t k, int element_size) {
-  return rows <= 2048 && rows * k <= (element_size == 4 ? 200 << 10 : 512 << 10);
+// kernel is the one of sixteen rows a workgroup).  That saves a launch, 2 us alone, and costs the whole weight for every
+// sixteen rows: a lone launch gets longer with k * n, which one workgroup multiplies, and takes more of the chip from others
+// with rows * k.  A model's forward alone / us a pass on eight serving threads, one launch and two, below and beyond each line:
+//  k * n, fp16  300 of 256 -> 250 26.9 / 6.7 and 28.2 / 7.2, 400 -> 250 28.5 / 7.4 and 28.7 / 7.4; the two layers by themselves
+//               768 -> 250 21.2 / 5.1 and 19.9 / 4.9
+//         fp32  1024 of 128 -> 250 28.7 / 7.3 and 29.2 / 7.5, 400 -> 100 32.7 / 9.7 and 32.1 / 9.3, 200 -> 250 31.4 / 7.9 and 30.2 / 8.3;
+//               the two layers by themselves 300 of 400 -> 250 25.5 / 6.2 and 20.9 / 5.6
+//  rows * k, fp16  1500 of 512 -> 100 29.3 / 7.4 and 31.6 / 8.2, 2048 of 400 -> 250 31.1 / 9.3 and 32.0 / 8.7, 512 -> 100 29.9 / 9.3 and
+//                  31.5 / 8.3
+//            fp32  1024 of 200 -> 100 28.7 / 7.0 and 29.2 / 7.8, of 256 -> 50 27.6 / 7.8 and 29.3 / 7.7, 2048 of 128 -> 100 27.7 / 8.2 and
+//                  28.6 / 8.0
+//  rows  fp16  2048 of 256 -> 50 27.4 / 7.0 and 29.7 / 7.6, 2600 28.0 / 8.2 and 30.7 / 8.0; the two layers by themselves, 4096 of
+//              64 -> 50 with others 1.28 times as long in one
+inline bool head_behind_any_columns(int64_t rows, int64_t k, int64_t n, int element_size) {
+  return rows <= 2048 && (element_size == 4 ? rows * k <= 240 << 10 && k * n <= 36 << 10 : rows * k <= 768 << 10 && k * n <= 96 << 10);
 }
 
 }  // namespace bz
