@@ -43,9 +43,13 @@ def test_feed(range_bytes, pieces):
 
 
 @pytest.mark.parametrize("range_bytes,pieces", [
-    (384 << 10, []),                                           # the most of which a lane asks for one unit at a time
+    (320 << 10, []),                                           # the most of which a lane asks for one unit at a time
+    ((320 << 10) + 16, []),
+    ((320 << 10) - 7 * 130, [(7, 130, 132, 140)]),             # the same with pieces
+    ((320 << 10) - 7 * 130 + 16, [(7, 130, 132, 140)]),
+    (384 << 10, []),                                           # two units, whole and partial workgroups
     ((384 << 10) + 16, []),
-    ((384 << 10) - 7 * 130, [(7, 130, 132, 140)]),             # the same with pieces
+    ((384 << 10) - 7 * 130, [(7, 130, 132, 140)]),
     ((384 << 10) - 7 * 130 + 16, [(7, 130, 132, 140)]),
     (4096, [(257, 1, 1, 3), (2, 255, 256, 300), (256, 3, 4, 5)]),                       # pieces of a workgroup and one unit
     (400000, [(513, 1, 1, 3), (2, 511, 512, 600), (1, 512, 512, 512), (3001, 6, 6, 9)]),  # the same at two units a lane

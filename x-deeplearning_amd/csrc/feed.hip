@@ -19,9 +19,10 @@ namespace {
 // Units (16 bytes of the range, or `unit` bytes of a piece) a lane asks for before it stores any: one in a small launch, whose
 // requests then leave from as many CUs as there are 4 KB; two where the link is full anyway and half the workgroups drain
 // sooner.  us from the call to the end of the wait for it, with 1, 2, 4 (an empty kernel 11.6): 4 KB 12.9 15.2 14.9, 64 KB 13.9
-// 16.1 16.0, 256 KB 17.9 18.9 19.1, 1 MB 37.0 32.5 35.4, 2 MB 61.7 53.6 57.8, 2048 rows of 128 bytes 18.6 19.8 19.8.
+// 16.1 16.0, 256 KB 17.9 18.9 19.1, 320 KB 19.6 19.8, 384 KB 21.3 20.9, 512 KB 24.5 23.2, 1 MB 37.4 32.6 35.4, 2 MB 61.7 53.6
+// 57.8, 2048 rows of 128 bytes 18.6 19.8 19.8.
 constexpr int kFeedThreads = 256;
-constexpr int64_t kFeedOneUnit = 384 << 10;  // bytes up to which a lane asks for one
+constexpr int64_t kFeedOneUnit = 320 << 10;  // bytes up to which a lane asks for one
 
 struct FeedArgs {
   const char* src;
