@@ -32,11 +32,15 @@ __device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b, uint32_t cap
 // Inclusive scan over the 64 lanes with data-parallel primitives (row_shr within rows of 16 lanes, then lane 15 and
 // lane 31 handed on to the following rows): a dozen VALU instructions, where the same scan through ds_bpermute
 // (__shfl_up) is six dependent trips to LDS per 32 bits.
-__device__ __forceinline__ uint32_t wave_scan_sat(uint32_t v, uint32_t cap) {
+__device__ __forceinline__ uint32_t row_scan_sat(uint32_t v, uint32_t cap) {  // within each row of 16 lanes
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false), cap);  // row_shr:1
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false), cap);  // row_shr:2
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false), cap);  // row_shr:4
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false), cap);  // row_shr:8
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_sat(uint32_t v, uint32_t cap) {
+  v = row_scan_sat(v, cap);
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false), cap);  // row_bcast:15 -> rows 1, 3
   v = sat_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false), cap);  // row_bcast:31 -> rows 2, 3
   return v;
@@ -289,6 +293,24 @@ __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int6
 }
 
 typedef int i32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // four counts, from any count on
+
+// a count as the scans take it, and a sum with four more of them
+__device__ __forceinline__ uint32_t count_sat(int32_t c, uint32_t cap) { return (uint32_t)min(max(c, 0), (int)cap); }
+__device__ __forceinline__ uint32_t add_counts_sat(uint32_t sum, const i32x4a4& c, uint32_t cap) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum = sat_add(sum, count_sat(c[j], cap), cap);
+  return sum;
+}
+
+// What lies before wave w of a workgroup of WAVES, given in LDS each wave's share of the counts before the workgroup's first
+// sample, then each wave's own sum: entry WAVES - 1 + w of the inclusive scan over the 2 * WAVES values, done in one row of
+// 16 lanes, in lane WAVES - 1 + w of each row.
+template <int WAVES>
+__device__ __forceinline__ uint32_t waves_scan_sat(const uint32_t* tot, uint32_t cap) {
+  static_assert(2 * WAVES <= 16, "the waves' totals are scanned within one row of lanes");
+  const int i = threadIdx.x & 15;
+  return row_scan_sat(i < 2 * WAVES ? tot[i] : 0u, cap);
+}
 
 constexpr int kBlockIds = 4;  // ids walked per step (measured at 2, 4, 8, 16: 4 is best or equal on segments of 1-4, 8 and 20 ids)
 

@@ -288,13 +288,9 @@ __device__ __forceinline__ void segment_of(const bz_embed_slot& s, int64_t b_fir
   const uint32_t quads = (uint32_t)b_first / 4;
   const int32_t odd = tid < (int)(b_first & 3) ? s.segments[4 * quads + tid] : 0;
   uint32_t part = 0;
-  for (uint32_t i0 = tid; i0 < quads; i0 += kThreads) {
-    const i32x4a4 c = ((const i32x4a4*)s.segments)[i0];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) part = sat_add(part, (uint32_t)min(max(c[j], 0), (int)cap), cap);
-  }
-  part = sat_add(part, (uint32_t)min(max(odd, 0), (int)cap), cap);
-  const uint32_t incl = wave_scan_sat((uint32_t)min(max(own, 0), (int)cap), cap);
+  for (uint32_t i0 = tid; i0 < quads; i0 += kThreads) part = add_counts_sat(part, ((const i32x4a4*)s.segments)[i0], cap);
+  part = sat_add(part, count_sat(odd, cap), cap);
+  const uint32_t incl = wave_scan_sat(count_sat(own, cap), cap);
   const uint32_t earlier = wave_scan_sat(part, cap);
   lds.incl[tid] = incl;
   if (lane == bz::kWave - 1) {
@@ -302,12 +298,7 @@ __device__ __forceinline__ void segment_of(const bz_embed_slot& s, int64_t b_fir
     lds.tot[WAVES + wave] = incl;
   }
   __syncthreads();
-  static_assert(2 * WAVES <= 16, "the waves' totals are scanned within one row of lanes");
-  uint32_t t = lds.tot[lane & (2 * WAVES - 1)];
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x111, 0xf, 0xf, false), cap);  // row_shr:1
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x112, 0xf, 0xf, false), cap);  // row_shr:2
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x114, 0xf, 0xf, false), cap);  // row_shr:4
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x118, 0xf, 0xf, false), cap);  // row_shr:8
+  const uint32_t t = waves_scan_sat<WAVES>(lds.tot, cap);
   const uint32_t before = (uint32_t)__shfl((int)t, WAVES - 1 + i / bz::kWave, bz::kWave);
   const uint32_t excl = i % bz::kWave == 0 ? 0u : lds.incl[i - 1];
   *start = (int64_t)sat_add(before, excl, cap);

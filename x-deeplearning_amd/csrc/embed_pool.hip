@@ -219,10 +219,7 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
       if (i >= quads) c[k] = 0;
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) part = sat_add(part, (uint32_t)min(max(c[k][j], 0), (int)cap), cap);
-    }
+    for (int k = 0; k < 4; ++k) part = add_counts_sat(part, c[k], cap);
   }
   const uint32_t mine = min((uint32_t)max(own, 0), cap);
   // the group's count sits in its last lane: after the scan that lane holds the inclusive sum and the group's other
@@ -234,14 +231,7 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
     s_tot[WAVES + wave] = scan;
   }
   __syncthreads();
-  // what lies before this wave: all the waves' sums of earlier counts and the totals of the waves before it -- entry
-  // WAVES - 1 + wave of the inclusive (saturating) scan over the 2 * WAVES values, done in one row of 16 lanes
-  static_assert(2 * WAVES <= 16, "the waves' totals are scanned within one row of lanes");
-  uint32_t t = (lane & 15) < 2 * WAVES ? s_tot[lane & 15] : 0u;
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x111, 0xf, 0xf, false), cap);  // row_shr:1
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x112, 0xf, 0xf, false), cap);  // row_shr:2
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x114, 0xf, 0xf, false), cap);  // row_shr:4
-  t = sat_add(t, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x118, 0xf, 0xf, false), cap);  // row_shr:8
+  const uint32_t t = waves_scan_sat<WAVES>(s_tot, cap);
   const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)t, WAVES - 1 + wave);
   const uint32_t x = sat_add(before, scan, cap);
   if constexpr (LPR == 1) {
@@ -258,7 +248,8 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
 
 // ---------------------------------------------------------------------------------------------
 // specialised ksum / kavg kernel: every slot has table dtype DT and LPR lanes per row
-// ---------------------------------------------------------------------------------------------// When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
+// ---------------------------------------------------------------------------------------------
+// When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
 // preamble a workgroup and, with long batches, the counts read again and again: above this many workgroups of 512 threads
 // of the specialised kernel, or above this many bytes of repeated reads.  Fused / scan + pool in us, by workgroups: 1600 (int8, 20 ids) 80 / 84, 1664
 // (26 slots x 8192 of 64-byte rows) 23 / 27, 3328 (16384) 57 / 59.5, 3840 (60 slots x 16384, 32-byte rows) 76 / 81, 5040 40 /

@@ -72,18 +72,6 @@ __host__ __device__ inline Layout layout(int steps, int n, int n2, int hn) {
   return l;
 }
 
-// f with the layer's activation as a constant
-template <typename F>
-__device__ __forceinline__ void with_act(int act, const F& f) {
-  switch (act) {
-    case BZ_ACT_PRELU: f(std::integral_constant<int, BZ_ACT_PRELU>()); break;
-    case BZ_ACT_DICE: f(std::integral_constant<int, BZ_ACT_DICE>()); break;
-    case BZ_ACT_LEAKY_RELU: f(std::integral_constant<int, BZ_ACT_LEAKY_RELU>()); break;
-    case BZ_ACT_SIGMOID: f(std::integral_constant<int, BZ_ACT_SIGMOID>()); break;
-    default: f(std::integral_constant<int, BZ_ACT_NONE>()); break;
-  }
-}
-
 // x op y of a chunk, each element rounded to the type as bz_concat_ew would store it.  (fp16: the difference or product of
 // two in fp32, rounded to fp16, is the one rounded once.)
 template <int DT, int OP>

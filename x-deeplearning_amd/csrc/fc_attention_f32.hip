@@ -1,7 +1,7 @@
 // fc_attention_f32.hip -- the attention MLP of a DIN model in fp32 as one launch: its input [x, y, x - y, x * y] computed
 // while it is loaded, two layers and a skinny third (the reference's Concat of elementwise results followed by 3-D Gemms and
 // their activations, tools/example_model/din/model/graph_ulf.txt; blaze/operator/op/concat_op.h:46-121, gemm_op.h:52-58,77-91).
-// 2-byte models run the same in fc_pieces.hip.
+// 2-byte models run theirs in fc_attention.hip.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -60,18 +60,6 @@ struct Attention {
   Epilogue ep1, ep2;
   HeadArgs head;
 };
-
-// f with the layer's activation as a constant
-template <typename F>
-__device__ __forceinline__ void with_act(int act, const F& f) {
-  switch (act) {
-    case BZ_ACT_PRELU: f(std::integral_constant<int, BZ_ACT_PRELU>()); break;
-    case BZ_ACT_DICE: f(std::integral_constant<int, BZ_ACT_DICE>()); break;
-    case BZ_ACT_LEAKY_RELU: f(std::integral_constant<int, BZ_ACT_LEAKY_RELU>()); break;
-    case BZ_ACT_SIGMOID: f(std::integral_constant<int, BZ_ACT_SIGMOID>()); break;
-    default: f(std::integral_constant<int, BZ_ACT_NONE>()); break;
-  }
-}
 
 // acc <- 16 rows of a times 16 rows of w over `steps` steps of 16, in kSums sums; a, w: this lane's first chunk
 __device__ __forceinline__ floatx4 block_product(const float* a, const float* w, int steps) {

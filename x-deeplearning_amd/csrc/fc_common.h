@@ -6,6 +6,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "bz_common.h"
 
 namespace bz {
@@ -122,6 +124,18 @@ __device__ __forceinline__ float apply_act_t(float v, const Epilogue& e, float p
     return t / (1.f + t);
   } else {
     return v;
+  }
+}
+
+// f with the layer's activation as a constant
+template <typename F>
+__device__ __forceinline__ void with_act(int act, const F& f) {
+  switch (act) {
+    case BZ_ACT_PRELU: f(std::integral_constant<int, BZ_ACT_PRELU>()); break;
+    case BZ_ACT_DICE: f(std::integral_constant<int, BZ_ACT_DICE>()); break;
+    case BZ_ACT_LEAKY_RELU: f(std::integral_constant<int, BZ_ACT_LEAKY_RELU>()); break;
+    case BZ_ACT_SIGMOID: f(std::integral_constant<int, BZ_ACT_SIGMOID>()); break;
+    default: f(std::integral_constant<int, BZ_ACT_NONE>()); break;
   }
 }
 
