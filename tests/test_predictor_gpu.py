@@ -1137,8 +1137,8 @@ def test_attention_input_in_front_of_a_layer_with_a_head(pb, w, n):
 
 @pytest.mark.parametrize("touched", ["by nothing else", "read by an operator", "written in place"])
 def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
-    """A skinny layer (s) and a layer's skinny head (p) write the host's copy of their outputs themselves, up to 64 KB: read
-    after every pass, some passes or twice, at growing and shrinking batches; and where another operator of the net reads or
+    """A skinny layer (s) and a layer's skinny head (p) write the host's copy of their outputs themselves, up to 64 KB, as the
+    observers' dump says: read after every pass, some passes or twice, at growing and shrinking batches; and where another operator of the net reads or
     overwrites the output, which is then copied as it is in the end."""
     rng = np.random.default_rng(16)
     w1, w2, w3 = (rng.standard_normal(s).astype(np.float32) * 0.3 for s in ((40, 16), (16, 2), (40, 3)))
@@ -1161,6 +1161,7 @@ def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
         nb.op("Add", ["s", "one"], ["s"])
     for o in outs:
         nb.external_output(o, 1)
+    shared = {"by nothing else": "", "read by an operator": "ps", "written in place": "s"}[touched]
     pm = pb.PredictorManager()
     pm.load_model_from_string(nb.text(), True)
     p = pm.create_predictor(1, 0)
@@ -1169,6 +1170,12 @@ def test_outputs_that_a_layer_copies_in_its_own_launch(pb, touched):
             x = rng.standard_normal((batch, 40)).astype(np.float32)
             p.feed("x", x)
             p.forward()
+            where = json.loads(p.dump_observers()["outputs"])
+            # (step 0: what Output made for another batch; step 3: s was not read after the pass before)
+            for o, cols in (("p", 2), ("s", 3)) if step else ():
+                by = "operator" if o not in shared else "copied"
+                expect = "device" if batch * cols * 4 > 64 << 10 or (step == 3 and o == "s") else by
+                assert where[o] == expect, "batch %d step %d %s" % (batch, step, o)
             d = x.astype(np.float64)
             e = np.exp(_sigmoid(d @ w1) @ w2)
             want = {"p": e / e.sum(1, keepdims=True), "s": d @ w3 + (touched == "written in place")}

@@ -20,6 +20,7 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
   }
   output_wanted_.assign(output_cpu_.size(), false);
   output_ahead_.assign(output_cpu_.size(), false);
+  output_by_operator_.assign(output_cpu_.size(), false);
   output_half_.assign(output_cpu_.size(), 0);
   output_read_.assign(output_cpu_.size(), 0);
   output_pinned_.assign(output_cpu_.size(), false);
@@ -375,6 +376,7 @@ bool Predictor::Forward(const PredictorCallback&& cb) {
       }
     }
     output_ahead_.assign(output_ahead_.size(), false);
+    output_by_operator_.assign(output_by_operator_.size(), false);
     OfferHostCopies();
     const bool launched = net_->Launch();
     if (launched) QueueOutputs();
@@ -466,7 +468,7 @@ void Predictor::QueueOutputs() {
                        bytes <= std::min(kCopiedAheadMax, HostHalf(i));
     output_wanted_[i] = false;
     if (ahead && output_sole_[i] && blob->host_copy().copied == bytes) {
-      output_ahead_[i] = true;
+      output_ahead_[i] = output_by_operator_[i] = true;
     } else if (ahead && n < BZ_FEED_MAX_ROWS) {
       rows[n].src = blob->data();
       rows[n].dst = (char*)output_cpu_[i]->data() + (1 - output_half_[i]) * HostHalf(i);
@@ -593,6 +595,12 @@ void Predictor::RegisterObservers(const std::vector<std::string>& names) {
 }
 void Predictor::DumpObservers(std::unordered_map<std::string, std::string>* dump_map) {
   (*dump_map)["profile"] = net_->DumpProfile();
+  std::stringstream ss;
+  ss << "{";
+  for (size_t i = 0; i < output_ahead_.size(); ++i)
+    ss << (i ? "," : "") << "\"" << net_->external_output()[i] << "\":\"" << (!output_ahead_[i] ? "device" : output_by_operator_[i] ? "operator" : "copied") << "\"";
+  ss << "}";
+  (*dump_map)["outputs"] = ss.str();
 }
 
 void* Predictor::InputDevicePtr(const char* name) {

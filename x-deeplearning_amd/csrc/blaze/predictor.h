@@ -91,6 +91,7 @@ class Predictor {
   std::vector<size_t> output_read_;  // bytes handed out last: may reach beyond a half when the output was larger then
   std::vector<bool> output_wanted_;  // read since the last Forward
   std::vector<bool> output_ahead_;   // the other half holds the last Forward's result
+  std::vector<bool> output_by_operator_;  // put there by the operator that computed it, not by a launch behind the net's
   std::vector<bool> output_sole_;    // one operator of the net writes it, none reads it
   std::vector<bool> output_pinned_;  // output_cpu_'s memory, as it was last made, is pinned
   std::vector<Blob*> handed_out_;    // whose device address the caller has
