@@ -54,7 +54,7 @@ bool fc_attention_f32_takes(int64_t k, int64_t n, int64_t n2);
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);
-// Whether it takes a head behind a layer of columns that are no whole number of 16-byte chunks (bz_fc_fused does not; the
+// Whether it takes a head behind an fp16 or fp32 layer of columns that are no whole number of 16-byte chunks (bz_fc_fused does not; the
 // kernel is the one of sixteen rows a workgroup).  That saves a launch, 2 us alone, and costs the whole weight for every
 // sixteen rows: a lone launch gets longer with k * n, which one workgroup multiplies, and takes more of the chip from others
 // with rows * k.  A model's forward alone / us a pass on eight serving threads, one launch and two, below and beyond each line:

@@ -59,7 +59,7 @@ int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
 }  // extern "C"
 
 int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
-  return run(d, copy, bz::head_behind_any_columns(d.m, d.k, d.n, bz::dtype_size(d.in_dtype)), stream);
+  return run(d, copy, d.in_dtype != BZ_BF16 && bz::head_behind_any_columns(d.m, d.k, d.n, bz::dtype_size(d.in_dtype)), stream);
 }
 
 namespace {

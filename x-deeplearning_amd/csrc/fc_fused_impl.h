@@ -1190,11 +1190,13 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream
     // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6; measured with the head's code unrolled for eight)
     if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 1, 4>(d, ep, st, copy);
     if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 1, 4>(d, ep, st, copy);
-  } else if (d.n % In<DT>::kChunk != 0) {  // (the tiles read a head's weight in whole chunks)
-    hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
-                       (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d, copy));
-    BZ_LAUNCH_OK("bz_fc_split_head_kernel");
-    return BZ_OK;
+  } else if constexpr (DT == BZ_F16) {  // (bz::fc_fused takes such columns, for a net's layers, none of which is bf16)
+    if (d.n % In<DT>::kChunk != 0) {  // (the tiles read a head's weight in whole chunks)
+      hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
+                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d, copy));
+      BZ_LAUNCH_OK("bz_fc_split_head_kernel");
+      return BZ_OK;
+    }
   }
   if (d.n <= 64) {
     if ((d.m + 63) / 64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, true, HN>(d, ep, st, copy);
