@@ -207,7 +207,7 @@ class ConcatForFc {  // implemented by Concat
 class ConcatAdopter {  // implemented by Gemm
  public:
   virtual ~ConcatAdopter() {}
-  virtual bool CanAdoptConcat() = 0;  // static part: constant 2-byte weight of a shape the kernel takes, no transposed A
+  virtual bool CanAdoptConcat() = 0;  // static part: constant 2-byte or fp32 weight of a shape the kernels take, no transposed A
   virtual void AdoptConcat(OperatorBase* concat) = 0;
   virtual bool HasAdoptedConcat() const = 0;
   // After the layers are chained: a Concat that no launch of this layer can compute is the net's again.  Null when the layer

@@ -249,14 +249,6 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
 // ---------------------------------------------------------------------------------------------
 // specialised ksum / kavg kernel: every slot has table dtype DT and LPR lanes per row
 // ---------------------------------------------------------------------------------------------
-// When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
-// preamble a workgroup and, with long batches, the counts read again and again: above this many workgroups of 512 threads
-// of the specialised kernel, or above this many bytes of repeated reads.  Fused / scan + pool in us, by workgroups: 1600 (int8, 20 ids) 80 / 84, 1664
-// (26 slots x 8192 of 64-byte rows) 23 / 27, 3328 (16384) 57 / 59.5, 3840 (60 slots x 16384, 32-byte rows) 76 / 81, 5040 40 /
-// 41.7 and 75 / 70, 5120 38.5 / 34, 7560 (120 slots x 1000, 400-byte rows) 60.5 / 57, 15360 117 / 96, 25600 (200 slots x 8192)
-// 219 / 180.  A plan whose records may travel as kernel arguments needs no upload of them when fused: twice as many there.
-constexpr int64_t kScanFirstGroups = 5000;
-constexpr int64_t kScanFirstBytes = 128ll << 20;
 template <int DT, int LPR, int THREADS>
 __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0, const int64_t* __restrict__ offsets) {
   constexpr int GROUPS = THREADS / LPR;
@@ -310,6 +302,16 @@ __global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(const Slot
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
   pool_samples<DT, LPR, kThreads>(s, b0, s.offsets);
 }
+
+// When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
+// preamble a workgroup and, with long batches, the counts read again and again: above this many workgroups of 512 threads
+// of the specialised kernel, or above this many bytes of repeated reads.  Fused / scan + pool in us, by workgroups: 1600 (int8, 20 ids) 80 / 84, 1664
+// (26 slots x 8192 of 64-byte rows) 23 / 27, 3328 (16384) 57 / 59.5, 3840 (60 slots x 16384, 32-byte rows) 76 / 81, 5040 40 /
+// 41.7 and 75 / 70, 5120 38.5 / 34, 7560 (120 slots x 1000, 400-byte rows) 60.5 / 57, 15360 117 / 96, 25600 (200 slots x 8192)
+// 219 / 180.  A plan whose records may travel as kernel arguments needs no upload of them when fused: twice as many there.
+constexpr int64_t kScanFirstGroups = 5000;
+constexpr int64_t kScanFirstBytes = 128ll << 20;
+
 int groups_per_wg(const bz_embed_slot& s) {
   const int ce = s.table_dtype == BZ_F32 ? 4 : (s.table_dtype == BZ_F16 ? 8 : 16);
   const int nchunks = (s.dim + ce - 1) / ce;
