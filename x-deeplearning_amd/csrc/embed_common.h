@@ -500,7 +500,7 @@ struct RowStream {
 // 8.8 us, half the vector instructions; with offsets given 16384 samples 48.4 / 45.9, 200 slots x 8192 of 2.5 ids, 128-byte
 // rows 181 / 157 to 168; int8 rows of 64, 20 ids, 83 / 80; eight serving threads 15.2 / 14.9 us a pass of 2048.  Rows that
 // are found in the caches are bound by the lanes' idle turns (a wave walks as far as its longest segment) and, int8, by the
-// three instructions an element takes (90 % of the vector units' time); rows that are not by memory, 4.7 TB/s of lines.
+// three instructions an element takes (92 % of the vector units' time); rows that are not by memory, 4.7 TB/s of lines.
 // Positions are relative to `first`, the wave's first id; n ids from position `from` on.
 template <int DT, int LPR, bool HASH>
 __device__ __forceinline__ void walk(const bz_embed_slot& s, int64_t first, uint32_t from, int n, int l, float (&acc)[RowTraits<DT>::kElems]) {
