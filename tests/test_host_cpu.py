@@ -640,3 +640,16 @@ int main() {
     subprocess.run([hipcc, "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-I" + os.path.join(ROOT, "include"),
                     "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
     assert subprocess.run([exe], timeout=60).returncode == 0
+
+
+def test_host_objects_are_built_again_when_the_dispatch_rules_change():
+    """bz_common.h holds rules that host code compiles in: an object built before a change of them would offer the kernels what they
+    refuse by now"""
+    import shutil
+    import subprocess
+    if not shutil.which("make"):
+        pytest.skip("no make")
+    csrc = os.path.join(ROOT, "x-deeplearning_amd", "csrc")
+    out = subprocess.run(["make", "-n", "-C", csrc, "-W", "bz_common.h"], check=True, capture_output=True, text=True, timeout=120).stdout
+    for f in ("dense_ops", "predictor"):
+        assert "-c blaze/%s.cc" % f in out, f
