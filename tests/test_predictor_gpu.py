@@ -1041,13 +1041,16 @@ def test_a_head_behind_any_columns_stays_where_it_is_faster(pb, dtype, k, n, row
     np.testing.assert_allclose(p.output_asnumpy("z").astype(np.float64), want, rtol=0, atol=tol)
 
 
-@pytest.mark.parametrize("dtype,P,n", [(np.float16, 2, 100), (np.float16, 3, 9), (np.float16, 5, 50), (np.float32, 2, 100), (np.float32, 4, 33)])
-def test_towers_with_heads_on_one_input(pb, dtype, P, n):
-    """P towers K -> n -> 2 written one after the other, n no multiple of eight: up to three 2-byte ones as long as the rows allow
-    a head in a layer's launch each run as one launch, all others as one launch for the layers and one for each head.  Rows
-    below and beyond the limit in turn, against 64 bits from the rounded layer and against one launch for everything."""
+@pytest.mark.parametrize("dtype,P,n,K,heads_in", [
+    (np.float16, 2, 100, 64, 2048), (np.float16, 3, 9, 64, 2048), (np.float16, 3, 172, 256, 2048), (np.float16, 3, 220, 256, 0),
+    (np.float16, 4, 100, 64, 2048), (np.float16, 4, 60, 64, 0), (np.float16, 5, 50, 64, 0), (np.float16, 6, 100, 64, 1024),
+    (np.float32, 2, 50, 64, 2048), (np.float32, 2, 100, 64, 0), (np.float32, 2, 250, 48, 0), (np.float32, 3, 50, 64, 0), (np.float32, 4, 33, 64, 0)])
+def test_towers_with_heads_on_one_input(pb, dtype, P, n, K, heads_in):
+    """P towers K -> n -> 2 written one after the other, n no multiple of eight: up to `heads_in` rows each runs with its head as one
+    launch, else the layers are one launch and each head one.  Rows below and beyond the limits in turn, against 64 bits from
+    the rounded layer and against one launch for everything."""
     rng = np.random.default_rng(P * n)
-    code, K = (pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT), 64
+    code = pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT
     ws = [[(rng.standard_normal(sh) / np.sqrt(sh[0])).astype(dtype) for sh in ((K, n), (1, n), (n, 2), (1, 2))] for _ in range(P)]
     xs = [rng.standard_normal((m, K)).astype(dtype) for m in (300, 4096, 1, 2049, 2048, 300)]
     got = {}
@@ -1074,8 +1077,7 @@ def test_towers_with_heads_on_one_input(pb, dtype, P, n):
             p.forward()
             got[fuse].append([p.output_asnumpy("p%d" % t).astype(np.float64) for t in range(P)])
             if fuse:
-                heads_in = dtype == np.float16 and P <= 3 and len(x) <= 2048
-                assert _launches(p, "Gemm") == (P if heads_in else 1 + P), len(x)
+                assert _launches(p, "Gemm") == (P if len(x) <= heads_in else 1 + P), len(x)
     tol = 4 * 2.0**-11 if dtype == np.float16 else 1e-5  # (as for one tower: the rounded layer, weights of 1 / sqrt(n))
     for x, g1, g0 in zip(xs, got[1], got[0]):
         for t, (w, b, u, c) in enumerate(ws):

@@ -429,15 +429,25 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     // an input the one-launch form does not take (unaligned rows, mixed types): one launch per layer
     return RunSelf(false) && RunHeadAlone();
   }
-  // Layers that share an input and have heads: each with its head, or the layers in one launch and the heads behind it.  P
-  // towers 256 -> 100 -> 2, us a pass alone / on eight serving threads, with heads and packed: fp16 P = 2 of 1 sample 19.5 / 4.4
-  // and 21.3 / 4.9, of 2048 22.4 / 5.6 and 25.9 / 6.8; P = 3 of 1 24.0 / 5.2 and 25.2 / 5.6, of 2048 28.0 / 8.0 and 30.5 / 8.1; P = 4
-  // of 1 28.4 / 6.3 and 28.4 / 6.6, of 300 33.6 / 8.3 and 32.6 / 8.0, of 2048 33.7 / 10.5 and 35.2 / 9.6; with more rows than a head
-  // is in the launch at, P = 2 of 4096 32.1 / 8.7 and 26.3 / 7.0.  fp32 P = 2 of 1 24.0 / 5.1 and 20.6 / 4.7, of 2048 27.4 / 7.7 and
-  // 24.8 / 6.7.
+  // Layers that share an input and have heads: each with its head in its launch, or the layers in one launch and the heads
+  // behind it.  That is one launch more, but shorter ones beside each other: what each workgroup multiplies, k * n, counts once
+  // and not P times.  P towers k -> n -> 2, time with heads over time packed, alone / on eight serving threads, from the smallest to the
+  // largest of 1, 300, 1024, 2048 samples:
+  //  fp16 P * k * n  2 of 384 -> 180 (138 K) .91..1.02 / .86..1.00, 3 of 256 -> 172 (132 K) .91..1.03 / .87..1.01; 4 of 384 -> 100 (154 K)
+  //                  .96..1.09 / .97..1.06, 3 of 256 -> 250 (192 K) .98..1.12 / .92..1.10
+  //       P, n       a packed layer of few columns stays in the split kernel's tiles: 3 of 128 -> 50 .90..1.01 / .90..1.05, 4 .94..1.05 /
+  //                  .94..1.09, of 256 -> 68 .90..1.00 / .88..1.00
+  //       rows       5 and more leave less to others: 6 of 128 -> 100, 2048 samples .90 / 1.05, fewer .96..1.02 / .91..1.02
+  //  fp32 2 of 192 -> 50 (10 K) .97..0.99 / .91..0.98, 256 -> 50 (13 K) 1.01..1.02 / .93..0.96; columns that are whole chunks pack better,
+  //       64 -> 100 .98..1.04 / .90..0.96; 3 of 64 -> 100 1.02..1.12 / .99..1.03
   bool HeadsBeforeSiblings() {
-    if (head_ == nullptr || siblings_.size() > 2 || DataTypeSize(this->Input(0)->data_type()) != 2 || !HeadAtTheseRows()) return false;
-    return std::all_of(siblings_.begin(), siblings_.end(), [](GemmOp* g) { return g->head_ != nullptr; });
+    if (head_ == nullptr || !HeadAtTheseRows()) return false;
+    Blob *a = this->Input(0), *b = this->Input(1);
+    const TIndex k = transb_ ? b->shape()[1] : b->shape()[0], n = transb_ ? b->shape()[0] : b->shape()[1];
+    const TIndex P = 1 + (TIndex)siblings_.size(), rows = a->size() / k;
+    const bool few = DataTypeSize(a->data_type()) == 2 ? P * k * n <= 144 << 10 && (P <= 3 || (n > 64 && (P == 4 || rows <= 1024)))
+                                                       : P == 2 && n % 4 != 0 && k * n <= 10 << 10;
+    return few && std::all_of(siblings_.begin(), siblings_.end(), [](GemmOp* g) { return g->head_ != nullptr; });
   }
 
   // this layer and its absorbed siblings as one launch over the stacked weights; every layer's output blob becomes a
