@@ -345,19 +345,25 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   bool RunOnDevice() override {
     launches_ = 1;
     if (concat_ != nullptr) {
+      bool stored = false;
       if (siblings_.empty() && (head_ == nullptr || !HeadAtAnyRows())) {
         bz_concat_ew_desc pieces;
         auto* c = dynamic_cast<ConcatForFc*>(concat_);
         // (the head in this layer's launch is worth more than the stored Concat costs.  The layer on pieces and its head as
         // a layer / the Concat and both layers in one, alone and with eight serving threads: fp16 rows of 216 -> 36 -> 1, 20
         // rows 24.6 and 4.7 / 18.7 and 4.4 us, 2000 26.9 and 5.9 / 20.3 and 4.7, but 51200 32.9 and 11.0 / 50.4 and 24.4)
-        if (c != nullptr && c->DescribeAsPieces(&pieces) && !(head_ != nullptr && HeadAtTheseRows())) {
-          if (next_ != nullptr && RunSelf(false, &pieces, true)) return true;  // this layer, the next and its head
-          if (this->Input(1)->data_type() != kFloat && RunSelf(false, &pieces)) return RunHeadAlone() && RunNextAlone();
+        if (c != nullptr && c->DescribeAsPieces(&pieces)) {
+          stored = head_ != nullptr && HeadAtTheseRows();
+          if (stored) {
+            c->RunDescribed(&pieces, context_.hip_stream());
+          } else {
+            if (next_ != nullptr && RunSelf(false, &pieces, true)) return true;  // this layer, the next and its head
+            if (this->Input(1)->data_type() != kFloat && RunSelf(false, &pieces)) return RunHeadAlone() && RunNextAlone();
+          }
         }
       }
       // a shape the one-launch form does not take: the Concat runs after all
-      if (!concat_->Run(context_.stream_id())) return false;
+      if (!stored && !concat_->Run(context_.stream_id())) return false;
       launches_ = 2;
       // (the paths below count their own launches from 1)
     }

@@ -201,6 +201,8 @@ class ConcatForFc {  // implemented by Concat
   // Describes Output(0) as pieces without computing it and gives the output blob its shape (no memory).  False: the
   // inputs do not fit the piece model; nothing has been touched.
   virtual bool DescribeAsPieces(bz_concat_ew_desc* desc) = 0;
+  // the launch that computes Output(0) after all, from its description of the same pass
+  virtual void RunDescribed(bz_concat_ew_desc* desc, void* stream) = 0;
   // whether the pieces are x, y, x - y, x * y as far as that is known before the operands are (the operators)
   virtual bool IsAttentionInput() const = 0;
 };

@@ -247,6 +247,12 @@ class ConcatOp final : public Operator<Context>, public ConcatPieceHost, public 
     std::sort(producers_.begin(), producers_.end(), [](const Adopted& a, const Adopted& b) { return a.position < b.position; });
   }
   bool DescribeAsPieces(bz_concat_ew_desc* desc) override { return RunWithPieces(desc); }
+  void RunDescribed(bz_concat_ew_desc* desc, void* stream) override {
+    Blob* y = this->Output(0);
+    y->Reshape(std::vector<TIndex>(y->shape()));
+    desc->dst = y->data();
+    BZ_CHECK(bz_concat_ew(desc, (hipStream_t)stream));
+  }
   bool IsAttentionInput() const override {
     if (this->InputSize() != 4) return false;
     std::string op[4];  // (an input that no operator was taken over for, or a BroadcastTo, is a copy)
