@@ -163,7 +163,8 @@ typedef struct bz_embed_launch {
                            before their first sample (batch * workgroups * 2 bytes per slot) that scanning once into
                            slot.offsets (bz_segments_to_offsets_slots) and planning again is the cheaper way */
   int32_t max_batch;    /* largest slot.batch of the planned slots */
-  int32_t shape;        /* with variant 0: (table_dtype << 8) | lanes_per_row when all slots share them, else 0 */
+  int32_t shape;        /* with variant 0: (table_dtype << 8) | lanes_per_row when all slots share them, else 0; plus
+                           1 << 16 in a plan of one row shape in which a slot has a hash index */
 } bz_embed_launch;
 
 /*

@@ -629,6 +629,40 @@ def test_pooling_walk_over_every_short_length(bz, oracle, kind, dim, keyed):
         assert np.array_equal(_bits(out.cpu().numpy()), _bits(full)), form
 
 
+@pytest.mark.parametrize("kind,dim,lpr", [("f32", 4, 1), ("f16", 14, 2), ("f32", 16, 4), ("f16", 64, 8), ("i8", 200, 16), ("f32", 100, 32), ("f16", 300, 64)])
+def test_keyed_walk_at_the_edges_of_its_batches(bz, oracle, kind, dim, lpr):
+    """Lists of keys as long as the batches that the keyed walk resolves at once (8, or one key a lane), one shorter and one
+    longer, and twice that, unknown keys in every place of a batch; beside a slot without an index; and by the kernel for plans
+    in which no slot has one."""
+    import torch
+    rng = np.random.default_rng(lpr)
+    per = max(8, lpr)
+    lens = np.array([0, 1, 4, 5, per - 1, per, per + 1, per + 4, 2 * per - 1, 2 * per, 2 * per + 1, 0], np.int32)
+    seg = np.concatenate([np.tile(lens, 3), rng.permutation(np.tile(lens, 9))]).astype(np.int32)
+    batch, rows, nnz = seg.size, 173, int(seg.sum())
+    tables = [_make_table(rng, kind, rows, dim, True), _make_table(rng, kind, rows, dim, False)]
+    keys = tables[0]["keys"]
+    inputs = []
+    for ids in (np.where(rng.random(nnz) < 0.1, -3 - np.arange(nnz), rng.choice(keys, nnz)), rng.integers(-2, rows + 2, nnz)):
+        inputs.append((ids.astype(np.int64), np.where(rng.random(nnz) < 0.02, 0.5, 1.0).astype(np.float32), seg))
+    specs, cols = [(0, 0, 0, 0, dim), (1, 1, 0, 0, dim)], [0, dim]
+    print("case kind=%s dim=%d" % (kind, dim), flush=True)
+    want = _run_oracle(oracle, tables, specs, inputs, batch, (2 * dim, cols))
+    for fused in (True, False):
+        got, _, variant = _run_gpu(bz, tables, specs, inputs, batch, np.float32, (2 * dim, cols), fused)
+        assert variant & 0xff == lpr
+        assert np.array_equal(_bits(got), _bits(want))
+    dts = [bz.DeviceTable(t["data"], scale=t.get("scale"), keys=t.get("keys")) for t in tables]
+    out = torch.full((batch, 2 * dim), float("nan"), device="cuda")
+    plan = bz.EmbeddingPlan([dict(table=t, ids=_dev(i), values=_dev(v), segments=_dev(s), out=out, col=c, udf=u)
+                             for t, (i, v, s), c, u in zip(dts, inputs, cols, (0, 1))])
+    assert plan.launch.shape == 1 << 16
+    plan.launch.shape = 0
+    plan.run()
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(out.cpu().numpy()), _bits(want)), "plain loads"
+
+
 @pytest.mark.parametrize("kind,dims", [("f32", (16, 14, 13)), ("f32", (100, 67, 80)), ("f16", (18, 32, 31)), ("f16", (8, 3, 7)), ("f16", (13, 16, 15)),
                                        ("f16", (200, 130, 256)), ("i8", (100, 66, 128)), ("i8", (64, 40, 33)), ("i8", (9, 16, 1)), ("i8", (30, 17, 32))])
 @pytest.mark.parametrize("keyed", [False, True])

@@ -312,6 +312,8 @@ __device__ __forceinline__ uint32_t waves_scan_sat(const uint32_t* tot, uint32_t
   return row_scan_sat(i < 2 * WAVES ? tot[i] : 0u, cap);
 }
 
+constexpr int kShapeKeyed = 1 << 16;  // in a plan's `shape`: a slot is looked up by key
+
 constexpr int kBlockIds = 4;  // ids walked per step (measured at 2, 4, 8, 16: 4 is best or equal on segments of 1-4, 8 and 20 ids)
 
 // Slot records handed over as kernel arguments: a workgroup then has its record after the one scalar load every
@@ -493,6 +495,14 @@ struct RowStream {
   }
 };
 
+// steps of the wave's longest segment, n being this lane's
+template <int LPR>
+__device__ __forceinline__ int wave_steps(int n) {
+#pragma unroll
+  for (int d = bz::kWave / 2; d >= LPR; d >>= 1) n = max(n, __shfl_xor(n, d, bz::kWave));
+  return (__builtin_amdgcn_readfirstlane(n) + kBlockIds - 1) / kBlockIds;
+}
+
 // The walk over a segment: straight-line code that the whole wave runs as often as its longest segment takes, the rows of a
 // step under way while those of the step before are added up.  (Waits count outstanding loads in order: after a join of a
 // path with loads and one without, the compiler waits for all of them.)
@@ -502,26 +512,16 @@ struct RowStream {
 // are found in the caches are bound by the lanes' idle turns (a wave walks as far as its longest segment) and, int8, by the
 // three instructions an element takes (92 % of the vector units' time); rows that are not by memory, 4.7 TB/s of lines.
 // Positions are relative to `first`, the wave's first id; n ids from position `from` on.
-template <int DT, int LPR, bool HASH>
+template <int DT, int LPR>
 __device__ __forceinline__ void walk(const bz_embed_slot& s, int64_t first, uint32_t from, int n, int l, float (&acc)[RowTraits<DT>::kElems]) {
-  RowStream<DT, LPR, HASH> rows(s, first, from, n, l);
+  RowStream<DT, LPR, false> rows(s, first, from, n, l);
   float one = 1.f;  // (opaque: see accum_chunk)
   asm volatile("" : "+v"(one));
-  int steps = n;
-#pragma unroll
-  for (int d = bz::kWave / 2; d >= LPR; d >>= 1) steps = max(steps, __shfl_xor(steps, d, bz::kWave));
-  steps = (__builtin_amdgcn_readfirstlane(steps) + kBlockIds - 1) / kBlockIds;
+  int steps = wave_steps<LPR>(n);
   if (steps <= 0) return;
   StepRows<DT, LPR> a, b;
   rows.fetch();
   rows.template request<true>(a, l);
-  if constexpr (HASH) {  // (a probe's own waits are for everything before it: nothing to overlap)
-    for (;;) {
-      add_rows<DT, LPR>(acc, a, one);
-      if (--steps == 0) return;
-      rows.template request<true>(a, l);
-    }
-  }
   for (; steps > 2; steps -= 2) {
     rows.template request<true>(b, l);
     add_rows<DT, LPR>(acc, a, one);
@@ -534,6 +534,103 @@ __device__ __forceinline__ void walk(const bz_embed_slot& s, int64_t first, uint
     a = b;
   }
   add_rows<DT, LPR>(acc, a, one);
+}
+
+// The same for tables looked up by key.  A probe is two dependent trips to memory (bucket, then pair) before the row's own, so
+// keys are resolved kKeyBatch at a time, one or more a lane: every lane of a group probes, where four did a step's four, and a
+// segment of up to kKeyBatch ids makes those two trips once instead of once a step.  Its rows then follow as in the walk above.
+// What bounds it is that chain (counts, ids, bucket, pair, row).  1000 x 24 lists of 6 keys, 400-byte fp32 rows: 19.1 -> 15.1 us.
+template <int DT, int LPR>
+__device__ __forceinline__ void walk_keyed(const bz_embed_slot& s, int64_t first, uint32_t from, int n, int l, float (&acc)[RowTraits<DT>::kElems]) {
+  using S = StepShape<LPR>;
+  constexpr int kKeyBatch = LPR > 8 ? LPR : 8, kPer = kKeyBatch / LPR;  // lane l holds keys k * LPR + l of a batch
+  const RowStream<DT, LPR, true> rows(s, first, from, n, l);           // (its resources and chunk)
+  float one = 1.f;  // (opaque: see accum_chunk)
+  asm volatile("" : "+v"(one));
+  int steps = wave_steps<LPR>(n);
+  if (steps <= 0) return;
+  const int gbase = (threadIdx.x & (bz::kWave - 1)) - l;
+  u32x2 id[kPer];
+  float val[kPer];
+  int at = l;  // this lane's first id of the batch at hand
+  auto fetch = [&]() {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const uint32_t o = at + k * LPR < n ? (from + (uint32_t)(at + k * LPR)) * 4u : kBeyondTable;
+      id[k] = __builtin_amdgcn_raw_buffer_load_b64(rows.ids, (int)(o << 1), 0, 0);
+      val[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows.values, (int)o, 0, 0));
+    }
+  };
+  fetch();
+  for (;; steps -= kKeyBatch / kBlockIds) {
+    uint32_t off[kPer], soff[kPer];
+    float v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int64_t r = at + k * LPR < n ? resolve_row(s, (int64_t)((uint64_t)id[k].y << 32 | id[k].x)) : -1;
+      off[k] = r >= 0 ? __umul24((uint32_t)r, (uint32_t)s.pitch) : kBeyondTable;
+      soff[k] = DT == BZ_I8 && r >= 0 ? __umul24((uint32_t)r, rows.scale_pitch) : kBeyondTable;
+      v[k] = r >= 0 ? val[k] : 1.f;  // (an id without a row adds a zero row: see RowStream::request)
+    }
+    if (steps > kKeyBatch / kBlockIds) {
+      at += kKeyBatch;
+      fetch();
+    }
+    // step s of the batch
+    auto request = [&](StepRows<DT, LPR>& st, int step) {
+      uint32_t so[S::kPerLane], of[S::kPerLane];
+      bool unit = true;
+#pragma unroll
+      for (int k = 0; k < S::kPerLane; ++k) {
+        if constexpr (LPR <= kBlockIds) {  // the lane's own (`step` is a constant here)
+          of[k] = off[step * S::kPerLane + k];
+          so[k] = soff[step * S::kPerLane + k];
+          st.val[k] = v[step * S::kPerLane + k];
+        } else {
+          const int holder = gbase + step * kBlockIds + l % kBlockIds;
+          of[k] = (uint32_t)__shfl((int)off[0], holder, bz::kWave);
+          if (DT == BZ_I8) so[k] = (uint32_t)__shfl((int)soff[0], holder, bz::kWave);
+          st.val[k] = __shfl(v[0], holder, bz::kWave);
+        }
+        unit &= st.val[k] == 1.f;
+      }
+      st.weighted = __builtin_amdgcn_ballot_w64(!unit);
+      each_id([&](auto u) {
+        constexpr int U = decltype(u)::value, K = U / S::kSrc;
+        st.raw[U] = __builtin_amdgcn_raw_buffer_load_b128(rows.table, (int)(of_id<LPR, U>(of[K]) + rows.at), 0, 0);
+      });
+      if (DT == BZ_I8) {
+#pragma unroll
+        for (int k = 0; k < S::kPerLane; ++k) st.scale[k] = __builtin_amdgcn_raw_buffer_load_b32(rows.scales, (int)so[k], 0, 0);
+      }
+      asm volatile("" ::: "memory");
+    };
+    StepRows<DT, LPR> a, b;
+    const int here = min(steps, kKeyBatch / kBlockIds);
+    request(a, 0);
+    if constexpr (LPR <= 8) {
+      if (here > 1) {
+        request(b, 1);
+        add_rows<DT, LPR>(acc, a, one);
+        a = b;
+      }
+    } else {
+      int i = 1;
+      for (; i + 1 < here; i += 2) {
+        request(b, i);
+        add_rows<DT, LPR>(acc, a, one);
+        request(a, i + 1);
+        add_rows<DT, LPR>(acc, b, one);
+      }
+      if (i < here) {
+        request(b, i);
+        add_rows<DT, LPR>(acc, a, one);
+        a = b;
+      }
+    }
+    add_rows<DT, LPR>(acc, a, one);
+    if (steps <= kKeyBatch / kBlockIds) return;
+  }
 }
 
 // The same for tables and segments beyond what buffer resources address: plain loads under branches.  26 slots x 4096 of 20
@@ -635,19 +732,23 @@ __device__ __forceinline__ bool wave_is_near(int64_t start, int64_t end, int64_t
   return __all(start >= *first && end - *first < kWalkIds);
 }
 
-// acc: the sum of the segment [start, end), for one chunk of the row
-template <int DT, int LPR>
+// acc: the sum of the segment [start, end), for one chunk of the row.  KEYED: the kernel is one for slots with a hash index.
+// In the others the keyed walk's code is left out, and with it 7 to 15 registers (200 slots x 8192 of 2.5 ids 184.5 us with
+// both walks in one kernel, 180.3 without; eight serving threads 976 and 949); a slot that is keyed all the same is right there,
+// by plain loads.
+template <int DT, int LPR, bool KEYED>
 __device__ __forceinline__ void sum_segment(const bz_embed_slot& s, int64_t start, int64_t end, int l, float (&acc)[RowTraits<DT>::kElems]) {
 #pragma unroll
   for (int i = 0; i < RowTraits<DT>::kElems; ++i) acc[i] = 0.f;
   int64_t first;
-  if (wave_is_near(start, end, &first) && table_fits<DT>(s)) {
+  const bool hash = s.hash_buckets != nullptr;
+  if (wave_is_near(start, end, &first) && table_fits<DT>(s) && (KEYED || !hash)) {
     const uint32_t from = (uint32_t)(start - first);
     const int n = (int)(end - start);
-    if (s.hash_buckets != nullptr)
-      walk<DT, LPR, true>(s, first, from, n, l, acc);
+    if (KEYED && hash)
+      walk_keyed<DT, LPR>(s, first, from, n, l, acc);
     else
-      walk<DT, LPR, false>(s, first, from, n, l, acc);
+      walk<DT, LPR>(s, first, from, n, l, acc);
   } else {
     walk_plain<DT, LPR>(s, start, end, l, acc);
   }
@@ -665,9 +766,15 @@ __device__ __forceinline__ void finish_sum(const bz_embed_slot& s, int64_t num, 
   if (e0 < s.dim) store_elems<CE>(s.out, b * s.out_stride + e0, acc, s.dim - e0, s.out_dtype);
 }
 
-// f(table dtype, lanes per row), both as constants, for a (dtype << 8) | lanes code of a plan
+// f(table dtype, lanes per row, whether a slot is keyed), all as constants, for a (dtype << 8) | lanes code of a plan
 template <typename F>
-int with_shape(int code, const F& f) {
+int with_shape(int code, bool keyed, const F& with_keyed) {
+  auto f = [&](auto dt, auto lpr) {
+    if (keyed)
+      with_keyed(dt, lpr, std::true_type{});
+    else
+      with_keyed(dt, lpr, std::false_type{});
+  };
   auto lanes = [&](auto dt) -> int {
     switch (code & 0xff) {
       case 1: f(dt, std::integral_constant<int, 1>{}); return BZ_OK;

@@ -306,7 +306,7 @@ __device__ __forceinline__ void segment_of(const bz_embed_slot& s, int64_t b_fir
 }
 
 // one workgroup of such a launch: workgroup v, owned by slot s
-template <int DT, int LPR>
+template <int DT, int LPR, bool KEYED>
 __device__ __forceinline__ void pool_mixed(const bz_embed_slot& s, int v, const int64_t* __restrict__ offsets) {
   constexpr int GROUPS = kThreads / LPR;
   __shared__ union {
@@ -342,16 +342,17 @@ __device__ __forceinline__ void pool_mixed(const bz_embed_slot& s, int v, const 
   if (item > last) return;
   if (s.udf != BZ_ASSIGN) {
     float acc[RowTraits<DT>::kElems];
-    sum_segment<DT, LPR>(s, start, end, l, acc);
+    sum_segment<DT, LPR, KEYED>(s, start, end, l, acc);
     finish_sum<DT>(s, end - start, l, b, acc);
     return;
   }
   const int p0 = (int)(item - b * per) * kAssignRun;
   int64_t first;
-  if (wave_is_near(start, end, &first) && table_fits<DT>(s)) {
+  const bool hash = s.hash_buckets != nullptr;
+  if (wave_is_near(start, end, &first) && table_fits<DT>(s) && (KEYED || !hash)) {
     const uint32_t from = (uint32_t)(start - first);
     const int num = end > start ? (int)(end - start) : 0;
-    if (s.hash_buckets != nullptr)
+    if (KEYED && hash)
       assign_step<DT, LPR, true>(s, first, from, num, l, b, p0);
     else
       assign_step<DT, LPR, false>(s, first, from, num, l, b, p0);
@@ -360,7 +361,7 @@ __device__ __forceinline__ void pool_mixed(const bz_embed_slot& s, int v, const 
   }
 }
 
-template <int DT, int LPR>
+template <int DT, int LPR, bool KEYED>
 __global__ __launch_bounds__(kThreads) void bz_embed_mixed_kernel(const bz_embed_slot* __restrict__ slots, int n_slots, int total_wg,
                                                                   int wg_per_xcd, int wg_per_slot, const int64_t* __restrict__ ext_off,
                                                                   int64_t ext_stride) {
@@ -368,17 +369,17 @@ __global__ __launch_bounds__(kThreads) void bz_embed_mixed_kernel(const bz_embed
   if (v >= total_wg) return;
   const int lo = wg_per_slot > 0 ? v / wg_per_slot : slot_of(slots, n_slots, v);
   const bz_embed_slot s = slots[lo];
-  pool_mixed<DT, LPR>(s, v, ext_off != nullptr ? ext_off + (int64_t)lo * ext_stride : s.offsets);
+  pool_mixed<DT, LPR, KEYED>(s, v, ext_off != nullptr ? ext_off + (int64_t)lo * ext_stride : s.offsets);
 }
 
-template <int DT, int LPR>
+template <int DT, int LPR, bool KEYED>
 __global__ __launch_bounds__(kThreads) void bz_embed_mixed_args_kernel(const SlotPack pack, const SlotBegins begins, int total_wg,
                                                                        int wg_per_xcd, int wg_per_slot) {
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
   const int lo = wg_per_slot > 0 ? v / wg_per_slot : slot_of(begins, v);
   const bz_embed_slot s = pack.s[lo];
-  pool_mixed<DT, LPR>(s, v, s.offsets);
+  pool_mixed<DT, LPR, KEYED>(s, v, s.offsets);
 }
 }  // namespace
 
@@ -389,8 +390,8 @@ int embed_launch_mixed(const bz_embed_slot* slots_dev, const bz_embed_launch& L,
   const dim3 grid(per_xcd * kNumXcd), block(kThreads);
   const int per_slot = ((int64_t)L.wg_per_slot * L.n_slots == L.total_wg) ? L.wg_per_slot : 0;
   if (L.shape != 0) {
-    const int rc = with_shape(L.shape, [&](auto dt, auto lpr) {
-      hipLaunchKernelGGL((bz_embed_mixed_kernel<decltype(dt)::value, decltype(lpr)::value>), grid, block, 0, st, slots_dev, L.n_slots,
+    const int rc = with_shape(L.shape & ~kShapeKeyed, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
+      hipLaunchKernelGGL((bz_embed_mixed_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st, slots_dev, L.n_slots,
                          L.total_wg, per_xcd, per_slot, ext_off, ext_stride);
     });
     if (rc != BZ_OK) return rc;
@@ -416,8 +417,8 @@ int embed_launch_mixed_args(const bz_embed_slot* slots_host, const bz_embed_laun
   for (int i = 0; i < 16; ++i) begins.b[i] = i < L.n_slots ? pack.s[i].wg_begin : INT_MAX;
   const int per_slot = ((int64_t)L.wg_per_slot * L.n_slots == L.total_wg) ? L.wg_per_slot : 0;
   if (L.shape != 0) {
-    const int rc = with_shape(L.shape, [&](auto dt, auto lpr) {
-      hipLaunchKernelGGL((bz_embed_mixed_args_kernel<decltype(dt)::value, decltype(lpr)::value>), grid, block, 0, st, pack, begins,
+    const int rc = with_shape(L.shape & ~kShapeKeyed, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
+      hipLaunchKernelGGL((bz_embed_mixed_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st, pack, begins,
                          L.total_wg, per_xcd, per_slot);
     });
     if (rc != BZ_OK) return rc;

@@ -249,7 +249,7 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
 // ---------------------------------------------------------------------------------------------
 // specialised ksum / kavg kernel: every slot has table dtype DT and LPR lanes per row
 // ---------------------------------------------------------------------------------------------
-template <int DT, int LPR, int THREADS>
+template <int DT, int LPR, int THREADS, bool KEYED>
 __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0, const int64_t* __restrict__ offsets) {
   constexpr int GROUPS = THREADS / LPR;
   __shared__ int64_t s_off[GROUPS + 1];
@@ -274,11 +274,11 @@ __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0,
   const int64_t b = b0 + g;
   if (b >= s.batch) return;
   float acc[RowTraits<DT>::kElems];
-  sum_segment<DT, LPR>(s, start, end, l, acc);
+  sum_segment<DT, LPR, KEYED>(s, start, end, l, acc);
   finish_sum<DT>(s, end - start, l, b, acc);
 }
 
-template <int DT, int LPR, int THREADS>
+template <int DT, int LPR, int THREADS, bool KEYED>
 __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_slot* __restrict__ slots, int n_slots,
                                                                  int total_wg, int wg_per_xcd, int wg_per_slot,
                                                                  const int64_t* __restrict__ ext_off, int64_t ext_stride) {
@@ -288,10 +288,10 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_s
   const int si = v / wg_per_slot;
   const bz_embed_slot s = slots[si];
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
-  pool_samples<DT, LPR, THREADS>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
+  pool_samples<DT, LPR, THREADS, KEYED>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
 }
 
-template <int DT, int LPR>
+template <int DT, int LPR, bool KEYED>
 __global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(const SlotPack pack, int total_wg, int wg_per_xcd,
                                                                       int wg_per_slot) {
   constexpr int GROUPS = kThreads / LPR;
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(const Slot
   const int si = v / wg_per_slot;
   const bz_embed_slot s = pack.s[si];
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
-  pool_samples<DT, LPR, kThreads>(s, b0, s.offsets);
+  pool_samples<DT, LPR, kThreads, KEYED>(s, b0, s.offsets);
 }
 
 // When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
@@ -367,7 +367,7 @@ int32_t bz_table_pitch(int64_t row_bytes, int scale_bytes) {
 int bz_embed_plan(bz_embed_slot* slots, int n_slots, bz_embed_launch* launch) {
   BZ_REQUIRE(slots != nullptr && launch != nullptr && n_slots > 0, "bz_embed_plan: null argument or n_slots=%d", n_slots);
   int64_t total = 0;
-  bool uniform_wg = true, uniform_shape = true, one_shape = true, any_offsets = false, all_offsets = true;
+  bool uniform_wg = true, uniform_shape = true, one_shape = true, any_offsets = false, all_offsets = true, keyed = false;
   int lpr0 = 0;
   for (int i = 0; i < n_slots; ++i) {
     bz_embed_slot& s = slots[i];
@@ -397,6 +397,7 @@ int bz_embed_plan(bz_embed_slot* slots, int n_slots, bz_embed_launch* launch) {
       if (s.hash_buckets != nullptr)
         BZ_REQUIRE(s.hash_pairs != nullptr && s.hash_bucket_size > 0, "slot %d: incomplete hash index", i);
     }
+    keyed |= s.table != nullptr && s.hash_buckets != nullptr;
     any_offsets |= s.offsets != nullptr;
     all_offsets &= s.offsets != nullptr;
     const int g = groups_per_wg(s);
@@ -428,6 +429,7 @@ int bz_embed_plan(bz_embed_slot* slots, int n_slots, bz_embed_launch* launch) {
   for (int i = 0; i < n_slots; ++i) max_batch = slots[i].batch > max_batch ? slots[i].batch : max_batch;
   launch->max_batch = max_batch;
   launch->shape = (launch->variant == 0 && one_shape) ? ((slots[0].table_dtype << 8) | lpr0) : 0;
+  if (keyed && (launch->variant != 0 || launch->shape != 0)) launch->shape |= kShapeKeyed;
   return BZ_OK;
 }
 
@@ -462,14 +464,15 @@ static int launch_pool(const bz_embed_slot* slots_dev, const bz_embed_launch& L,
   // with offsets given: smaller workgroups, each with its share of a planned workgroup's samples
   const bool scanned = ext_off != nullptr || !L.fused_scan;
   const int per_xcd_scanned = (kOffsetSplit * L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
-  const int rc = with_shape(L.variant, [&](auto dt, auto lpr) {
+  const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
     constexpr int kDt = decltype(dt)::value, kLpr = decltype(lpr)::value;
+    constexpr bool kKeyed = decltype(keyed)::value;
     if (scanned)
-      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kOffsetThreads>), dim3(per_xcd_scanned * bz::kNumXcd), dim3(kOffsetThreads), 0,
+      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kOffsetThreads, kKeyed>), dim3(per_xcd_scanned * bz::kNumXcd), dim3(kOffsetThreads), 0,
                          st, slots_dev, L.n_slots, kOffsetSplit * L.total_wg, per_xcd_scanned, kOffsetSplit * L.wg_per_slot, ext_off,
                          ext_stride);
     else
-      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kThreads>), grid, block, 0, st, slots_dev, L.n_slots, L.total_wg, per_xcd,
+      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kThreads, kKeyed>), grid, block, 0, st, slots_dev, L.n_slots, L.total_wg, per_xcd,
                          L.wg_per_slot, ext_off, ext_stride);
   });
   if (rc != BZ_OK) return rc;
@@ -499,9 +502,9 @@ int bz_embed_pool_args(const bz_embed_slot* slots_host, const bz_embed_launch* l
   const int per_xcd = (L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
   const dim3 grid(per_xcd * bz::kNumXcd), block(kThreads);
   hipStream_t st = bz::as_stream(stream);
-  const int rc = with_shape(L.variant, [&](auto dt, auto lpr) {
-    hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value>), grid, block, 0, st, pack, L.total_wg,
-                       per_xcd, L.wg_per_slot);
+  const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
+    hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st,
+                       pack, L.total_wg, per_xcd, L.wg_per_slot);
   });
   if (rc != BZ_OK) return rc;
   BZ_LAUNCH_OK("bz_embed_pool_args_kernel");
