@@ -214,6 +214,62 @@ def test_fc_fp32_error_of_a_layer_with_a_head(bz, M, N, K, parts):
     assert err <= _fp32_sum_error(K / parts), err
 
 
+def _plain_bound(x, w, bias):
+    """what any order of K fp32 products and sums stays within, and a split that drops 2^-24 of a product"""
+    return (x.shape[1] + 8) * 2.0**-24 * (x.double().abs() @ w.double().abs().t().contiguous() + bias.double().abs())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 9, 4), (31, 33, 5), (33, 65, 15), (32, 32, 16), (65, 31, 17), (3, 300, 127), (130, 90, 2075), (257, 257, 33),
+                                   (700, 512, 201), (520, 520, 600), (1000, 500, 257), (2300, 260, 97), (9000, 130, 130), (1100, 500, 600),
+                                   (2111, 321, 203), (3000, 700, 1000)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_fc_fp32_on_bf16_pieces(bz, M, N, K, off):
+    """fp32 layers as products of three bf16s a float: edges of tiles, of a stage of 16 and of its chunks, waves without a stage,
+    rows that start on no 16 bytes"""
+    import torch
+    torch.manual_seed(M + 3 * N + K)
+    held = torch.randn(M * (K + off) + off, device="cuda")
+    x = held[off:].view(M, K + off)[:, :K]
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    bias = torch.randn(N, device="cuda") * 0.1
+    print("case M=%d N=%d K=%d off=%d" % (M, N, K, off), flush=True)
+    full = torch.full((M + 1, N + 3), 7.0, device="cuda")
+    bz.fc_fused(x, w, K, bias=bias, out=full[:M, :N])
+    want = x.double() @ w[:, :K].double().t().contiguous() + bias.double()
+    assert ((full[:M, :N].double() - want).abs() <= _plain_bound(x, w[:, :K], bias)).all()
+    assert (full[M:] == 7.0).all() and (full[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (1200, 400, 160), (1200, 800, 250)])
+def test_fc_fp32_infinities_and_numbers_at_the_ends_of_the_range(bz, M, N, K):
+    """numbers that no bf16 is near to, and such whose pieces lie below the smallest bf16"""
+    import torch
+    torch.manual_seed(K)
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.rand(K, N, device="cuda") + 0.5, False, bz.F32)
+    bias = torch.zeros(N, device="cuda")
+    x[0, 3] = float("inf")
+    x[1, K - 1] = -float("inf")
+    x[2, 7] = float("nan")
+    x[3] = 1e-3
+    x[3, 5] = 3.402e38
+    w[2, :K] *= 2.0**-10  # (a column that takes it without overflow)
+    x[4] *= 1e-37
+    x[5] = 0.0
+    x[6] = -0.0
+    x[M - 1] *= 1e-30
+    print("case M=%d N=%d K=%d" % (M, N, K), flush=True)
+    y = bz.fc_fused(x, w, K, bias=bias)
+    want = x.double() @ w[:, :K].double().t().contiguous()
+    as32 = want.float()
+    assert torch.equal(torch.isnan(y), torch.isnan(as32)) and torch.equal(torch.isposinf(y), torch.isposinf(as32))
+    assert torch.equal(torch.isneginf(y), torch.isneginf(as32)) and torch.isfinite(y[3, 2])
+    fine = torch.isfinite(as32)
+    bound = _plain_bound(x, w[:, :K], bias)
+    assert ((y.double() - want).abs() <= bound)[fine].all()
+    assert (y[5:7] == 0).all()
+
+
 # Large 2-byte layers go to the streaming kernel (256x128 tiles, loader waves, operands straight into LDS) once
 # ceil(M/256) * ceil(N/128) >= 200, K is a multiple of 64 and at least 512, and the output takes 16-byte stores.
 @pytest.mark.parametrize("in_name", ["f16", "bf16"])

@@ -206,6 +206,39 @@ struct In<BZ_F32> {
   }
 };
 
+// A float as the sum of three bf16s: each the nearest to what the ones before leave over, 8 significant bits and a sign a
+// piece, so that nothing is left over (|x| from 2^-110 up; below, what is left over is at most 2^-134).  A product of two
+// such sums, without the three of its nine products that are below 2^-25 of it, comes from the bf16 matrix instructions: six of
+// them multiply 32x32x16 in 192 clocks, the fp32 ones in 512.
+// A float that is no bf16 to be rounded to, an infinity or one within 2^-9 of it, makes infinite or undefined pieces, which
+// make infinite or undefined sums: whoever uses this looks at the sums and computes such ones with fp32 instructions.
+struct Bf16x3 {
+  uint4 hi, mid, lo;  // eight floats: element i in half i % 2 of word i / 2
+};
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t nearest_bf16x2(float x0, float x1) {
+  const bf16x2 h = __builtin_convertvector((floatx2{x0, x1}), bf16x2);  // v_cvt_pk_bf16_f32
+  return *(const uint32_t*)&h;
+}
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = nearest_bf16x2(x0, x1);
+  x0 -= __uint_as_float(hi << 16);
+  x1 -= __uint_as_float(hi & 0xffff0000u);
+  mid = nearest_bf16x2(x0, x1);
+  x0 -= __uint_as_float(mid << 16);
+  x1 -= __uint_as_float(mid & 0xffff0000u);
+  lo = nearest_bf16x2(x0, x1);
+}
+__device__ __forceinline__ Bf16x3 split_floats(const uint4& a, const uint4& b) {
+  Bf16x3 s;
+  split_pair(__uint_as_float(a.x), __uint_as_float(a.y), s.hi.x, s.mid.x, s.lo.x);
+  split_pair(__uint_as_float(a.z), __uint_as_float(a.w), s.hi.y, s.mid.y, s.lo.y);
+  split_pair(__uint_as_float(b.x), __uint_as_float(b.y), s.hi.z, s.mid.z, s.lo.z);
+  split_pair(__uint_as_float(b.z), __uint_as_float(b.w), s.hi.w, s.mid.w, s.lo.w);
+  return s;
+}
+
 constexpr int kSkinnyMaxN = 8;
 
 // the optional skinny second layer computed from the first layer's output tile while it is still in LDS

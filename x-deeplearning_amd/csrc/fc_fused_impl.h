@@ -139,21 +139,20 @@ __device__ __forceinline__ void chunk_to_float(const uint4& c, float (&f)[In<DT>
 // Sums an output is added up in where a wave owns one 32x32 block.  fp32: one for each step of a K tile, which also makes
 // them shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two).  Two otherwise, and in the tiles with
 // a head, whose other registers are many: with four the 64x64 one takes 10.7 us for 17000 x 80 -> 40 instead of 10.3.
-template <int DT, int BM, int BN, int BK, int WM, int WN, int HEAD, int WK>
+template <int DT, int BM, int BN, int BK, int WM, int WN, int HEAD>
 constexpr int default_sums() {
-  constexpr int steps = BK / In<DT>::kStepK / WK;
+  constexpr int steps = BK / In<DT>::kStepK;
   return BM / WM / 32 * (BN / WN / 32) > 1 ? 1 : DT == BZ_F32 && !HEAD ? steps : steps >= 2 ? 2 : 1;
 }
 
 // HEAD: outputs the code of the skinny second layer is unrolled for, 0 without one
-// WK: groups of WM x WN waves that share each K tile between them and add up at the end
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD, int WK, int KACC>
-__global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD, int KACC>
+__global__ __launch_bounds__(WM* WN * 64) void bz_fc_mfma_kernel(const char* __restrict__ A, const char* __restrict__ W,
                                                                   OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
                                                                   int64_t ldw, int64_t ldy, bool vec_y, int tiles_m, Epilogue ep,
                                                                   HeadArgs head) {
   using T = In<DT>;
-  constexpr int NT = WM * WN * WK * 64;
+  constexpr int NT = WM * WN * 64;
   constexpr int ES = T::kSize;
   constexpr int ROWB = BK * ES;        // bytes of one tile row
   constexpr int PITCH = ROWB + 16;     // padded LDS pitch
@@ -175,8 +174,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wk = WK == 1 ? 0 : wave / (WM * WN), wmn = WK == 1 ? wave : wave % (WM * WN);
-  const int wm = wmn / WN, wn = wmn % WN;
+  const int wm = wave / WN, wn = wave % WN;
   // consecutive workgroups walk down M within one N panel: the W panel stays hot in L2
   const int tile_m = blockIdx.x % tiles_m, tile_n = blockIdx.x / tiles_m;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -301,14 +299,13 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
   // (not the 256x256 tile: with 128 accumulator registers a wave has no room for a second set of fragments; measured on
   // the other tiles: 128x256 245 -> 238 us on 8192x12800x1024, 64x64 9.6 -> 9.2 us on config 2's first layer)
   constexpr bool PIPE = !HEAD && BM * BN >= 64 * 64 && BM * BN < 256 * 256;
-  constexpr int KS = BK / T::kStepK / WK;  // sub-steps of a K tile that are this wave's
-  static_assert(WK == 1 || PIPE, "K is shared in the pipelined loop");
+  constexpr int KS = BK / T::kStepK;  // sub-steps of a K tile
   if constexpr (PIPE) {
     static_assert(KS % 2 == 0, "fragment double buffer needs an even number of sub-steps");
     uint4 fa[2][TM], fw[2][TN];
     auto fread = [&](int slot, int buf, int ks) {
-      const char* la = &lds[buf][(wm * WTM + frag_row) * PITCH + frag_half * 16 + wk * (KS * 32)];
-      const char* lw = &lds[buf][(BM + wn * WTN + frag_row) * PITCH + frag_half * 16 + wk * (KS * 32)];
+      const char* la = &lds[buf][(wm * WTM + frag_row) * PITCH + frag_half * 16];
+      const char* lw = &lds[buf][(BM + wn * WTN + frag_row) * PITCH + frag_half * 16];
 #pragma unroll
       for (int i = 0; i < TM; ++i) fa[slot][i] = *(const uint4*)(la + i * 32 * PITCH + ks * 32);
 #pragma unroll
@@ -375,28 +372,6 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[0][i][j][r] += acc[a][i][j][r];
-  // the other groups' partial tiles, through LDS behind the output tile's place: group 0 goes on with the sum
-  if constexpr (WK > 1) {
-    static_assert(WK == 2 && !HEAD && BM * (BN * (int)sizeof(OutT) + 16) + BM * (BN + 1) * 4 <= (int)sizeof(lds), "room for the partial tile");
-    float* part = (float*)(&lds[0][0] + BM * (BN * (int)sizeof(OutT) + 16)) + (wm * WTM + 4 * frag_half) * (BN + 1) + wn * WTN + frag_row;
-    if (wk == 1) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) part[(i * 32 + 8 * (r >> 2) + (r & 3)) * (BN + 1) + j * 32] = acc[0][i][j][r];
-    }
-    __syncthreads();
-    if (wk == 0) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[0][i][j][r] += part[(i * 32 + 8 * (r >> 2) + (r & 3)) * (BN + 1) + j * 32];
-    }
-  }
   // epilogue: lane owns column n, rows 8*(r/4) + 4*(lane/32) + r%4 of each 32x32 block.  The activated tile
   // goes through LDS (free after the K loop) so that global stores are 16 bytes per lane along rows.
   constexpr int OS = (int)sizeof(OutT);
@@ -449,9 +424,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void bz_fc_mfma_kernel(const char*
       }
     }
   };
-  switch (WK > 1 && wk != 0 ? -1 : ep.act) {
-    case -1:
-      break;
+  switch (ep.act) {
     case BZ_ACT_PRELU:
       epilogue(std::integral_constant<int, BZ_ACT_PRELU>());
       break;
@@ -890,6 +863,279 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
 }
 
 // ---------------------------------------------------------------------------------------------
+// fp32 layers on the bf16 matrix cores
+// ---------------------------------------------------------------------------------------------
+// A workgroup owns a tile of 32 * TM x 32 * TN outputs and its NW waves share K, 16 at a time (stage t is wave t % NW's), each
+// working for itself: it loads a stage of the tile's rows straight into LDS of its own, reads fragments from there, splits them
+// into three bf16s a float (Bf16x3) and multiplies those; the partial tiles meet once, at the end.
+//  - The conversion, 11 vector instructions for two floats, is what bounds it, not the products: between 32-clock MFMAs the SIMD
+//    issues a vector instruction every five clocks, where 7.3 come to each MFMA of a 64x64 tile, and it does so only if a wave's
+//    own instructions alternate (beside another wave's MFMAs a wave of vector instructions gets one in 18 clocks).  So a step
+//    multiplies one stage, converts the next and reads the one after, and tells the scheduler to alternate (with all conversions
+//    in front of the products, as they came, 2048 x 896 -> 512 took 17.5 us, with the read in front of them 16.2, this way 14.5).
+//  - That takes two sets of pieces in registers, and none are left for loads in flight: they go to LDS without any.
+//  - 2048 x 896 -> 512 by clocks, eight waves: 4 500 to the first stage, 15 000 for two waves' seven steps a SIMD (11 000 of MFMAs), 1 500
+//    to add up, 3 000 to finish and store.
+constexpr int kF32Stage = 16;                   // of K
+constexpr int kF32RowB = kF32Stage * 4;         // bytes of a row of a stage
+constexpr uint32_t kF32RowsWithin = 0x80000000u;  // bytes that a tile's rows lie within
+inline bool f32_rows_fit(int64_t ld, int k) { return k >= 4 && (64 * ld + k) * 4 < (int64_t)kF32RowsWithin; }
+
+// 16 bytes per lane from base + off to LDS at lds_addr + 16 * lane where `left`, as base and lds_addr the same in all lanes, is
+// above 0.  (The branch stands in the assembler: one that the compiler sees ends the block in which it may alternate products
+// and conversions.)
+__device__ __forceinline__ void load_to_lds_from(const char* base, uint32_t off, uint32_t lds_addr, int left) {
+  asm volatile("s_cmp_lt_i32 %3, 1\n\ts_cbranch_scc1 .Lnone%=\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1\n.Lnone%=:" ::"v"(off),
+               "s"(base), "s"(lds_addr), "s"(left)
+               : "memory", "m0", "scc");
+}
+
+// the dot product of two fp32 rows, in four sums
+__device__ __forceinline__ float plain_dot(const float* a, const float* w, int K) {
+  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+  int k = 0;
+  for (; k + 4 <= K; k += 4) {
+    s0 = fmaf(a[k], w[k], s0);
+    s1 = fmaf(a[k + 1], w[k + 1], s1);
+    s2 = fmaf(a[k + 2], w[k + 2], s2);
+    s3 = fmaf(a[k + 3], w[k + 3], s3);
+  }
+  for (; k < K; ++k) s0 = fmaf(a[k], w[k], s0);
+  return (s0 + s1) + (s2 + s3);
+}
+// whether a sum of split products may be off: it is not finite, or so small that the operands may lie where a split drops bits
+__device__ __forceinline__ bool doubtful(float v) { return !(v == 0.f || (fabsf(v) >= 0x1p-80f && fabsf(v) < __builtin_huge_valf())); }
+
+template <typename OutT, int NW, int TM, int TN>
+__global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, OutT* __restrict__ Y, int M,
+                                                            int N, int K, int64_t lda, int64_t ldw, int64_t ldy, int tiles_m,
+                                                            Epilogue ep) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, NT = NW * 64, ROWS = BM + BN;
+  constexpr int LOADS = ROWS / 16;  // a load instruction brings 16 rows of a stage
+  constexpr int SLOT = ROWS * kF32RowB;
+  static_assert(BM * BN * 4 <= 2 * SLOT, "a partial tile fits where its wave's operands were");
+  __shared__ __attribute__((aligned(16))) char lds[NW][2][SLOT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = (int)(blockIdx.x % tiles_m) * BM, n0 = (int)(blockIdx.x / tiles_m) * BN;
+  const int frow = lane & 31, fhalf = lane >> 5;
+  // Row r of a stage lies at 64 * r, its chunk c at position c ^ ((r >> 2) & 3): sixteen lanes that read one chunk of sixteen rows
+  // are on all banks.  Lane l of a load has position l % 4 of row l / 4 of its sixteen.
+  const int lrow = lane >> 2, lchunk = (lane & 3) ^ (lane >> 4);
+  const char* abase = A + (int64_t)m0 * lda * 4;
+  const char* wbase = W + (int64_t)n0 * ldw * 4;
+  uint32_t off[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    if (i * 16 < BM)
+      off[i] = (uint32_t)min(i * 16 + lrow, M - 1 - m0) * (uint32_t)(lda * 4) + lchunk * 16;
+    else
+      off[i] = (uint32_t)min(i * 16 - BM + lrow, N - 1 - n0) * (uint32_t)(ldw * 4) + lchunk * 16;
+  }
+  const int stages = (K + kF32Stage - 1) / kF32Stage;
+  const int n = wave < stages ? (stages - 1 - wave) / NW + 1 : 0;  // this wave's
+  // The wave's stages in descending order, so that the one that K ends in comes first
+  auto stage_at = [&](int i) { return wave + (n - 1 - i) * NW; };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char*)&lds[0][0][0] + wave * (2 * SLOT);
+  auto issue = [&](int i) {
+    const int64_t k = (int64_t)stage_at(i) * kF32RowB;
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds0 + (i & 1) * SLOT);
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) load_to_lds_from((q * 16 < BM ? abase : wbase) + k, off[q], to + q * 1024, n - i);
+  };
+  // the same through registers, for a stage that reaches beyond K: zeros there
+  auto issue_part = [&](int i) {
+    const int k = stage_at(i) * kF32Stage + lchunk * 4, back = k - min(k, K - 4);
+    uint4 r[LOADS];
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) __builtin_memcpy(&r[q], (q * 16 < BM ? abase : wbase) + (int64_t)(k - back) * 4 + (off[q] - lchunk * 16), 16);
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) *(uint4*)(&lds[wave][i & 1][q * 1024 + lane * 16]) = shift_chunk<BZ_F32>(r[q], back);
+  };
+  const bool part = n > 0 && (stage_at(0) + 1) * kF32Stage > K;
+  if (n > 0) {
+    if (!part) issue(0);
+    issue(1);
+    if (part) issue_part(0);
+  }
+  // the parameters of the column that this thread finishes: asked for now, looked at at the end
+  float cbias = 0.f, cp0 = 0.f, cp1 = 0.f, cp2 = 0.f;
+  {
+    const int c = min(n0 + tid % BN, N - 1);
+    if (ep.bias_rows == 1) cbias = ep.bias[c];
+    if (ep.act == BZ_ACT_PRELU) cp0 = ep.p0[ep.act_size == 1 ? 0 : c];
+    if (ep.act == BZ_ACT_DICE) {
+      cp0 = ep.p0[c];
+      cp1 = ep.p1[c];
+      cp2 = ep.p2[c];
+    }
+  }
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  struct Pieces {
+    Bf16x3 a[TM], w[TN];
+  };
+  struct Raw {
+    uint4 a[TM][2], w[TN][2];
+  };
+  // chunks h and h + 2 of its row are the lane's in half h
+  auto read = [&](int i, Raw& raw) {
+    const char* from = &lds[wave][i & 1][0] + frow * kF32RowB;
+    const int p0 = (fhalf ^ ((frow >> 2) & 3)) * 16, p1 = p0 ^ 32;
+#pragma unroll
+    for (int b = 0; b < TM; ++b) {
+      raw.a[b][0] = *(const uint4*)(from + b * 32 * kF32RowB + p0);
+      raw.a[b][1] = *(const uint4*)(from + b * 32 * kF32RowB + p1);
+    }
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+      raw.w[b][0] = *(const uint4*)(from + (BM + b * 32) * kF32RowB + p0);
+      raw.w[b][1] = *(const uint4*)(from + (BM + b * 32) * kF32RowB + p1);
+    }
+  };
+  auto convert = [&](const Raw& raw, Pieces& p) {
+#pragma unroll
+    for (int b = 0; b < TM; ++b) p.a[b] = split_floats(raw.a[b][0], raw.a[b][1]);
+#pragma unroll
+    for (int b = 0; b < TN; ++b) p.w[b] = split_floats(raw.w[b][0], raw.w[b][1]);
+  };
+  // the smallest products first
+  auto multiply = [&](const Pieces& p) {
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f(p.a[i], p.w[j], acc[i][j]);
+    };
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.lo, y.hi, c); });
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.hi, y.lo, c); });
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.mid, y.mid, c); });
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.mid, y.hi, c); });
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.hi, y.mid, c); });
+    each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.hi, y.hi, c); });
+  };
+  // Stage i has landed where every load but the last stage's is waited for; the waits are written out because only this code
+  // knows how many loads may stay in flight.
+  auto landed = [&](int i) {
+    asm volatile("s_cmp_gt_i32 %0, 1\n\ts_cbranch_scc1 .Lmore%=\n\ts_waitcnt vmcnt(0)\n.Lmore%=:\n\ts_waitcnt vmcnt(%1)" ::"s"(n - i), "n"(LOADS)
+                 : "memory", "scc");
+  };
+  // the stage after next goes where stage i was, once every read of it has returned
+  auto refill = [&](int i) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    issue(i + 2);
+  };
+  // multiplies stage i, converts stage i + 1, reads stage i + 2
+  auto step = [&](const Pieces& now, Pieces& next, const Raw& raw, Raw& raw_next, int i) {
+    landed(i + 2);
+    read(i + 2, raw_next);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(now);
+    convert(raw, next);
+    constexpr int MFMAS = 6 * TM * TN, VALU = 88 * (TM + TN) / 2, EACH = VALU / MFMAS;
+#pragma unroll
+    for (int q = 0; q < MFMAS; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, EACH, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    refill(i + 2);
+  };
+  if (n > 0) {
+    Pieces p0, p1;
+    Raw r0, r1;
+    landed(0);
+    read(0, r0);
+    refill(0);
+    landed(1);
+    read(1, r1);
+    convert(r0, p0);
+    refill(1);
+    int i = 0;
+    for (; i + 2 < n; i += 2) {
+      step(p0, p1, r1, r0, i);
+      step(p1, p0, r0, r1, i + 1);
+    }
+    if (i + 1 < n) {
+      step(p0, p1, r1, r0, i);
+      multiply(p1);
+    } else {
+      multiply(p0);
+    }
+  }
+  // A lane owns column lane & 31 of each block and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: four rows of a column are a chunk.  Every
+  // wave leaves its partial tile where its operands were, column by column, the chunks of a column in an order of its own, so
+  // that writes and reads are on all banks; then a thread adds up and finishes chunks of one column.
+  constexpr int CHUNKS = BM / 4, EACH = (CHUNKS * BN + NT - 1) / NT;  // of a column; of a thread
+  static_assert(NT % BN == 0 && (CHUNKS * BN % NT == 0 || EACH == 1) && (CHUNKS & (CHUNKS - 1)) == 0, "threads share the tile's chunks evenly");
+  auto chunk_at = [&](int col, int chunk) { return (col * CHUNKS + (chunk ^ (col & (CHUNKS - 1)))) * 16; };
+  const int col = tid % BN, nn = n0 + col;
+  float v[EACH][4];
+  auto add_up = [&]() {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(float4*)(&lds[wave][0][0] + chunk_at(j * 32 + frow, i * 8 + q * 2 + fhalf)) =
+              make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < EACH; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[e][c] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int e = 0; e < EACH; ++e) {
+        const float4 p = *(const float4*)(&lds[w][0][0] + chunk_at(col, tid / BN + e * (NT / BN)));
+        v[e][0] += p.x;
+        v[e][1] += p.y;
+        v[e][2] += p.z;
+        v[e][3] += p.w;
+      }
+  };
+  add_up();
+  if (nn >= N || tid / BN >= CHUNKS) return;
+  uint32_t again = 0;
+#pragma unroll
+  for (int e = 0; e < EACH; ++e)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) again |= doubtful(v[e][c]) ? 1u << (e * 4 + c) : 0u;
+  while (again != 0) {  // (rare, and slow)
+    const int which = __builtin_ctz(again);
+    again &= again - 1;
+    const int m = m0 + (tid / BN + which / 4 * (NT / BN)) * 4 + which % 4;
+    const float s = plain_dot((const float*)A + (int64_t)min(m, M - 1) * lda, (const float*)W + (int64_t)nn * ldw, K);
+#pragma unroll
+    for (int e = 0; e < EACH; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[e][c] = which == e * 4 + c ? s : v[e][c];
+  }
+  cbias *= ep.beta;
+  if (ep.act == BZ_ACT_DICE) cp2 = dice_inv_den(ep, cp2);
+  OutT* const y = Y + out_index(ep, m0, nn, ldy);
+  with_act(ep.act, [&](auto act) {
+#pragma unroll
+    for (int e = 0; e < EACH; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int ml = (tid / BN + e * (NT / BN)) * 4 + c;
+        if (m0 + ml >= M) continue;
+        const float b = ep.bias_rows > 1 ? ep.beta * ep.bias[full_bias_index(ep, m0 + ml, nn, M, N)] : cbias;
+        store_out<OutT>(y + ml * ldy, apply_act_t<decltype(act)::value>(fmaf(ep.alpha, v[e][c], b), ep, cp0, cp1, cp2));
+      }
+  });
+}
+
+// ---------------------------------------------------------------------------------------------
 // split kernel with the skinny head
 // ---------------------------------------------------------------------------------------------
 // A layer with a head keeps whole rows in one workgroup, so M sets how many CUs work: 16 rows a workgroup where the staged
@@ -1110,8 +1356,8 @@ __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restric
   }
 }
 
-template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD = 0, int WK = 1,
-          int KACC = default_sums<DT, BM, BN, BK, WM, WN, HEAD, WK>()>
+template <int DT, typename OutT, int BM, int BN, int BK, int WM, int WN, int D, bool ALIGNED, int HEAD = 0,
+          int KACC = default_sums<DT, BM, BN, BK, WM, WN, HEAD>()>
 int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st, void* copy = nullptr) {
   const int tiles_m = (d.m + BM - 1) / BM, tiles_n = (d.n + BN - 1) / BN;
   // output rows 16-byte aligned and N a whole number of 16-byte chunks: coalesced stores through LDS
@@ -1120,7 +1366,7 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st, void* c
                      (d.n % (16 / (int)sizeof(OutT)) == 0) &&
                      (d.n_split == 0 || (d.n_split % (16 / (int)sizeof(OutT)) == 0 && (d.y_split_stride * (int64_t)sizeof(OutT)) % 16 == 0));
   const HeadArgs head = HEAD != 0 ? head_args(d, copy) : HeadArgs{};
-  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, WK, KACC>), dim3(tiles_m * tiles_n), dim3(WM * WN * WK * 64), 0,
+  hipLaunchKernelGGL((bz_fc_mfma_kernel<DT, OutT, BM, BN, BK, WM, WN, D, ALIGNED, HEAD, KACC>), dim3(tiles_m * tiles_n), dim3(WM * WN * 64), 0,
                      st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, vec_y, tiles_m, ep, head);
   BZ_LAUNCH_OK("bz_fc_mfma_kernel");
   return BZ_OK;
@@ -1138,6 +1384,15 @@ int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   return BZ_OK;
 }
 
+
+template <typename OutT, int NW, int TM, int TN>
+int launch_f32(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
+  const int tiles_m = (d.m + 32 * TM - 1) / (32 * TM), tiles_n = (d.n + 32 * TN - 1) / (32 * TN);
+  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
+                     d.ldw, d.ldy, tiles_m, ep);
+  BZ_LAUNCH_OK("bz_fc_f32_kernel");
+  return BZ_OK;
+}
 
 // 2-byte operands and outputs, 16-byte aligned rows on all three, K a whole number of 64-wide tiles
 template <int DT, typename OutT>
@@ -1188,8 +1443,8 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream
     }
     // Up to 4096 rows four sums an output, as short as that kernel's (3000 x 512 -> 128 17.9 / 8.3, with two 17.8 / 9.3;
     // 8000 x 512 -> 128 18.1 / 12.7 and 17.9 / 11.6; measured with the head's code unrolled for eight)
-    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 1, 4>(d, ep, st, copy);
-    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 1, 4>(d, ep, st, copy);
+    if (d.m <= 4096 && d.n <= 64) return launch_mfma<DT, OutT, 32, 64, BK, 1, 2, 4, true, HN, 4>(d, ep, st, copy);
+    if (d.m <= 4096 && d.n <= 128) return launch_mfma<DT, OutT, 32, 128, BK, 1, 4, 4, true, HN, 4>(d, ep, st, copy);
   } else if constexpr (DT == BZ_F16) {  // (bz::fc_fused takes such columns, for a net's layers, none of which is bf16)
     if (d.n % In<DT>::kChunk != 0) {  // (the tiles read a head's weight in whole chunks)
       hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
@@ -1230,32 +1485,22 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   if constexpr (In<DT>::kSize == 2) {
     if (d.n > 64 && wg128 >= (d.k > 256 ? 129 : 140)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
     if (d.n > 64 && wg64x128 >= 256) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
-  } else {
-    if (d.n > 64 && wg128 >= 512 && (ALIGNED || d.k > 512)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
-    if constexpr (ALIGNED)
-      if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
+  } else if constexpr (ALIGNED) {
+    if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
+    if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
   }
   // Rows that start anywhere: K is seldom a whole number of tiles, and a tile that is loaded only to be dropped costs as
   // much as any other, so few are in flight: one while K is at most four tiles of 2-byte operands, else two.  64x64
   // however many there are (us alone / with eight streams of the same; 32x64 or 64x64 with four in flight: fp16
   // 3000 x 162 -> 200 8.1 / 3.7, now 6.0 / 2.8, 10000 x 50 -> 64 8.8 / 3.6 and 4.5 / 2.1, 2000 x 901 -> 400 14.9 / 9.2 and
-  // 10.3 / 5.8, fp32 3000 x 162 -> 200 16.5 / 7.5 and 9.0 / 5.0; 64x128: fp32 20000 x 162 -> 256 42.1 / 29.7 and
-  // 26.5 / 21.9; 128x128: fp32 16384 x 301 -> 512 65.5 / 58.9 and 55.9 / 52.3, but 16384 x 901 -> 512 140 / 130 and 149 / 146).
+  // 10.3 / 5.8).
   if constexpr (!ALIGNED) {
     if constexpr (In<DT>::kSize == 2)
       if (d.k <= 4 * BK) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, ALIGNED>(d, ep, st);
     return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
   } else {
     if constexpr (DT == BZ_F32) {
-      // fp32, K of 512 and more, tiles for at most two rounds of the CUs: eight waves, two to a SIMD, that share each K
-      // tile.  Its MFMAs are long, and with one wave a SIMD nothing runs while that wave reads fragments or waits at the
-      // barrier: 2048 x 896 -> 512 24.2 us, 21.6 this way, 2048 x 512 -> 512 14.8 and 13.4.  With more tiles the matrix
-      // cores set the time either way (8192 rows 64 us), and next to other kernels the smaller workgroup wins (the tower
-      // of that layer at 4096 rows, eight serving threads, 57.8 us a pass this way and 56.8 the other).
-      if (d.k >= 512 && wg64 >= 256 && wg64 < 512) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED, 0, 2>(d, ep, st);
-      // Else four waves and two K tiles in flight (us alone / with eight streams of the same; the eight waves:
-      // 10000 x 64 -> 200 14.5 / 9.4 and now 9.6 / 5.8, 4096 x 192 -> 512 14.4 / 11.3 and 12.4 / 8.8, 1500 x 400 -> 700
-      // 21.9 / 11.6 and 19.5 / 10.8; 32x64 with four in flight: 1500 x 896 -> 512 37.0 / 19.0 and 22.3 / 15.2).
+      // (two K tiles in flight; with four waves sharing each, 10000 x 64 -> 200 14.5 / 9.4 and this way 9.6 / 5.8)
       return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     } else {
       // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
@@ -1279,10 +1524,8 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   const bool aligned = vec_a && vec_w && d.k % In<DT>::kChunk == 0;
   // Few tiles: the split kernel (and K below a chunk, which the other loaders cannot read).  Its workgroups are large for
   // what they do, so beyond a line they cost other streams more than they save a lone launch.
-  //  fp32: 512 32x32 tiles (us alone / with eight streams of the same, against 64x64 with two K tiles in flight:
-  //   1024 x 896 -> 512, 512 tiles, 15.1 / 11.4 and 22.3 / 13.0, 2000 x 144 -> 200, 441, 7.1 / 4.9 and 7.6 / 4.2;
-  //   2048 x 896 -> 512, 1024, 27.0 / 22.2 and 22.6 / 16.6).
-  //  2-byte: 256 (512 x 896 -> 512, 256 tiles, 4.4 / 2.6 and 7.3 / 3.3; 1024 x 256 -> 512, 512, 4.1 / 2.9 and 4.7 / 2.1);
+  //  2-byte: 256 tiles of 32x32 (us alone / with eight streams of the same, against 64x64: 512 x 896 -> 512, 256 tiles,
+  //   4.4 / 2.6 and 7.3 / 3.3; 1024 x 256 -> 512, 512, 4.1 / 2.9 and 4.7 / 2.1);
   //   K above 256 up to 512 with four waves, half the LDS (1024 x 896 -> 512, 512 tiles, eight waves, four, the 64x64 tile:
   //   6.2 / 4.3, 6.0 / 3.7, 7.4 / 3.5; 742 x 2179 -> 512, 384, 12.2 / 8.1, 12.9 / 7.9, 16.5 / 8.7).  Models on eight serving
   //   threads, us a pass, a lone pass in brackets, in the same order: that first layer at batch 1024 11.2 (35.3),
@@ -1292,8 +1535,28 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
   //   tile in flight; 1024 x 162 -> 200, 224, 4.4 / 2.2 and 5.1 / 2.2, but the attention model of that layer, batch 1024, on
   //   eight serving threads 41.1 M samples/s this way and 43.1 on the tile, 63.2 and 63.7 us a lone pass).
   const int64_t wg32 = (int64_t)((d.m + 31) / 32) * ((d.n + 31) / 32);
-  const int64_t few = DT == BZ_F32 ? 512 : (aligned || d.k > 256) ? 256 : 192;
-  if (d.k < In<DT>::kChunk || wg32 <= few) return launch_split<DT, OutT, 8>(d, ep, st);
+  if constexpr (DT == BZ_F32) {
+    // The bf16 matrix cores, but for rows of shallow K in more tiles than CUs.  32x32 tiles of eight waves while there are few,
+    // 32x64 of four up to a 64x64 one for half the CUs, and where K is shallow; else 64x64 (us alone / with eight streams of
+    // the same, in that order; with eight waves a 64x64 tile is a little faster alone, 2048 x 896 -> 512 14.5 / 13.7, and slower beside others):
+    //  500 x 600 -> 500, 256 tiles of 32x32, 6.7 / 4.1, 8.6 / 3.8, 11.2 / 4.3; 520 rows -> 520, 289, 9.0 / 4.5, 8.6 / 4.0, 11.3 / 4.5;
+    //  700 x 200 -> 512, 352, 5.5 / 3.4, 5.9 / 3.2, 8.0 / 3.3; 2000 x 144 -> 200, 441, 5.3 / 4.0, 5.8 / 4.0, 7.3 / 4.1;
+    //  1000 x 600 -> 500, 128 of 64x64, 9.4 / 7.1, 9.4 / 5.8, 11.6 / 5.3; 1100 rows, 144, 12.6 / 8.0, 12.7 / 6.6, 11.8 / 5.9;
+    //  20000 x 162 -> 256 36.9 / 31.5, 24.8 / 20.4, 26.2 / 19.5; 2000 x 200 -> 800 14.5 / 10.8, 12.7 / 8.0, 11.3 / 7.4.
+    // The fp32 tiles / 32x64: 50000 x 80 -> 80 20.8 / 14.4 and 22.0 / 17.1, 20000 x 80 -> 512 37.3 / 24.2 and 32.3 / 27.2,
+    // 50000 x 100 -> 200 68 / 47 and 43 / 38, 20000 x 128 -> 512 53 / 38 and 36 / 33.
+    // Before, the split kernel below and those tiles: 300 x 445 -> 256 6.8 / 4.0 and now 4.9 / 3.1, 32 x 2075 -> 768 14.8 / 6.0 and
+    // 10.2 / 4.0, 1024 x 896 -> 512 13.7 / 10.8 and 11.1 / 7.3, 2048 x 896 -> 512 19.6 / 15.9 and 14.9 / 12.1, 8192 rows 65 / 62 and 49 / 49,
+    // 16384 x 301 -> 512 55 / 52 and 43 / 42, 5000 x 3000 -> 1024 380 / 250 and 213 / 220.  Errors against 64 bits, in the
+    // same order: 1.5e-7 and 1.2e-7, 2.9e-7 and 2.5e-7, 2.0e-7 and 2.3e-7, 2.7e-7 and 2.3e-7, 5.4e-7 and 2.3e-7, 1.6e-7 and 1.3e-7, 9.7e-7 and 4.2e-7.
+    const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
+    if (f32_rows_fit(d.lda, d.k) && f32_rows_fit(d.ldw, d.k) && (d.k > 96 || wg64 <= 128 || wg32 <= 512)) {
+      if (wg32 <= 256 || (wg32 <= 512 && d.k <= 256)) return launch_f32<OutT, 8, 1, 1>(d, ep, st);
+      if (wg64 <= 128 || d.k < 200) return launch_f32<OutT, 4, 1, 2>(d, ep, st);
+      return launch_f32<OutT, 4, 2, 2>(d, ep, st);
+    }
+  }
+  if (d.k < In<DT>::kChunk || (In<DT>::kSize == 2 && wg32 <= (aligned || d.k > 256 ? 256 : 192))) return launch_split<DT, OutT, 8>(d, ep, st);
   if constexpr (In<DT>::kSize == 2)
     if (wg32 <= 512 && d.k > 256) return launch_split<DT, OutT, 4>(d, ep, st);
   if (!aligned) return dispatch_mid<DT, OutT, false>(d, ep, st);
