@@ -300,7 +300,7 @@ typedef struct bz_fc_desc {
   float act_alpha;     /* LEAKY_RELU slope */
   int32_t reserved_;
   /*
-   * Optional second, skinny layer in the same launch (head_n > 0): Z[M, head_n] = head_act(Y * head_w^T + head_bias),
+   * Optional second, skinny layer in the same call (head_n > 0; one launch, but see bz_fc_head_apart): Z[M, head_n] = head_act(Y * head_w^T + head_bias),
    * computed from the rounded tile of Y while it is still on chip -- the Gemm -> activation -> Gemm(N <= 8) ->
    * Softmax | Sigmoid tail of a CTR tower without the second launch.  Needs 8 < n <= 256 (a workgroup owns whole rows
    * of Y), out_dtype == in_dtype, 16-byte aligned operand rows.  y may be NULL then (Y is not stored).
@@ -335,6 +335,10 @@ typedef struct bz_fc_desc {
 } bz_fc_desc;
 
 BZ_API int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream);
+
+/* 1 where bz_fc_fused runs the head of a layer k -> n of that type as a launch behind the layer's, given memory for the layer's
+ * outputs (y): fp32 layers of much work a row.  With y NULL the head is always in the layer's launch. */
+BZ_API int bz_fc_head_apart(int k, int n, int in_dtype);
 
 /*
  * Repack a Blaze weight blob for bz_fc_fused: src is [K,N] (trans_b=0) or [N,K]

@@ -270,6 +270,50 @@ def test_fc_fp32_infinities_and_numbers_at_the_ends_of_the_range(bz, M, N, K):
     assert (y[5:7] == 0).all()
 
 
+@pytest.mark.parametrize("M,K,N,H,act", [(1, 1024, 48, 1, "none"), (17, 516, 100, 8, "softmax"), (300, 256, 196, 2, "softmax"), (2049, 512, 256, 2, "none"),
+                                         (300, 256, 192, 3, "sigmoid"), (2000, 200, 256, 2, "softmax")])
+def test_fc_fp32_head_apart_and_in_the_launch(bz, M, K, N, H, act):
+    """below and above k * n = 48 K: with memory for the layer's output, without (in the launch: another stream's call, a capture),
+    and with the output left out"""
+    import torch
+    torch.manual_seed(M + N)
+    code = dict(none=bz.ACT_NONE, softmax=bz.ACT_SOFTMAX, sigmoid=bz.ACT_SIGMOID)[act]
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    w2 = bz.pack_weight(torch.randn(N, H, device="cuda") / N**0.5, False, bz.F32)
+    bias, bias2 = torch.randn(N, device="cuda") * 0.1, torch.randn(H, device="cuda")
+    slope = torch.full((N, ), 0.25, device="cuda")
+    wide = x.double() @ w[:, :K].double().t().contiguous() + bias.double()
+    wide = torch.where(wide > 0, wide, 0.25 * wide)
+    want = wide @ w2[:, :N].double().t().contiguous() + bias2.double()
+    want = dict(none=lambda v: v, softmax=lambda v: v.softmax(1), sigmoid=torch.sigmoid)[act](want)
+    print("case M=%d K=%d N=%d H=%d %s" % (M, K, N, H, act), flush=True)
+    assert bz.lib().bz_fc_head_apart(K, N, bz.F32) == (K * N > 48 << 10) and bz.lib().bz_fc_head_apart(K, N, bz.F16) == 0
+    # sums of K and of N terms in any order, the second behind values of about 1 and columns of about N**-0.5
+    bound = (K + N + 16) * 2.0**-24 * (1 + wide.abs() @ w2[:, :N].double().abs().t().contiguous())
+
+    def call(store, **kw):
+        z, y = torch.full((M, H + 1), 9.0, device="cuda"), torch.full((M, N), 9.0, device="cuda")
+        got, _ = bz.fc_fused(x, w, K, bias=bias, act=bz.ACT_PRELU, act_params=(slope, ), out=y, store_out=store,
+                             head=dict(w=w2, bias=bias2, act=code, out=z[:, :H]), **kw)
+        return z, y, got
+
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    for store, kw in ((True, {}), (False, {}), (False, dict(stream=other))):
+        z, y, got = call(store, **kw)
+        torch.cuda.synchronize()
+        assert ((z[:, :H].double() - want).abs() <= bound).all() and (z[:, H:] == 9.0).all()
+        assert got is y if store else got is None and (y == 9.0).all()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z, _, _ = call(False)
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((z[:, :H].double() - want).abs() <= bound).all()
+
+
 # Large 2-byte layers go to the streaming kernel (256x128 tiles, loader waves, operands straight into LDS) once
 # ceil(M/256) * ceil(N/128) >= 200, K is a multiple of 64 and at least 512, and the output takes 16-byte stores.
 @pytest.mark.parametrize("in_name", ["f16", "bf16"])

@@ -21,7 +21,7 @@ ACT_NONE, ACT_PRELU, ACT_DICE, ACT_LEAKY_RELU, ACT_SIGMOID, ACT_SOFTMAX = 0, 1, 
 
 EXPORTS = [
     "bz_last_error", "bz_device_check", "bz_table_pitch", "bz_embed_plan", "bz_segments_to_offsets", "bz_segments_to_offsets_slots",
-    "bz_embed_pool", "bz_embed_pool_args", "bz_embed_pool_static_scratch", "bz_embed_pool_kernel_name", "bz_fc_fused", "bz_fc_pack_weight", "bz_gemm_strided_batched", "bz_weighted_pool",
+    "bz_embed_pool", "bz_embed_pool_args", "bz_embed_pool_static_scratch", "bz_embed_pool_kernel_name", "bz_fc_fused", "bz_fc_head_apart", "bz_fc_pack_weight", "bz_gemm_strided_batched", "bz_weighted_pool",
     "bz_activation", "bz_concat_cols", "bz_broadcast_op", "bz_reduce_sum", "bz_batch_norm", "bz_softmax_axis",
     "bz_concat_ew", "bz_gather_rows", "bz_spin", "bz_feed"
 ]
@@ -144,6 +144,7 @@ def lib():
         l.bz_embed_pool_args.argtypes = [C.POINTER(EmbedSlot), C.POINTER(EmbedLaunch), vp]
         l.bz_embed_pool_kernel_name.restype = C.c_char_p
         l.bz_fc_fused.argtypes = [C.POINTER(FcDesc), vp]
+        l.bz_fc_head_apart.argtypes = [C.c_int, C.c_int, C.c_int]
         l.bz_fc_pack_weight.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int, vp, C.c_int, i64, vp]
         l.bz_gemm_strided_batched.argtypes = [C.POINTER(BgemmDesc), vp]
         l.bz_weighted_pool.argtypes = [C.POINTER(WeightedPoolDesc), vp]
@@ -408,7 +409,7 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
              act_alpha=0.0, dice_nosqrt=False, stream=None, head=None, store_out=True):
     """head: dict(w=packed [n2, ldw] weight of a second layer with n2 <= 8 outputs, bias=fp32 [n2] or None, act=ACT_NONE |
     ACT_SIGMOID | ACT_SOFTMAX, out=tensor [m, n2]) computed in the same launch; then returns (out, head out), and
-    store_out=False skips storing the first layer's output (out is returned as None)."""
+    store_out=False leaves the first layer's output out (out is returned as None, a tensor given as `out` as it was)."""
     m, n = a.shape[0], w_packed.shape[0]
     dt = bz_dtype(a.dtype)
     if out is None:
@@ -425,7 +426,7 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
             assert bz_dtype(t.dtype) == F32
             p[i] = t.data_ptr()
     act_size = act_params[0].numel() if act_params and act_params[0] is not None else 0
-    y = out.data_ptr()
+    y, ldy = out.data_ptr(), out.stride(0)
     hw_ptr = hb_ptr = hy_ptr = h_ldw = h_ldy = h_n = h_act = h_dt = 0
     if head is not None:
         hw, hb, hy = head["w"], head.get("bias"), head["out"]
@@ -436,10 +437,16 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
             assert bz_dtype(hb.dtype) == F32
             hb_ptr = hb.data_ptr()
         if not store_out:
-            y = 0
+            y, ldy = 0, n
+            if dt == F32 and stream is None and lib().bz_fc_head_apart(k, n, dt):
+                # the head runs behind the layer, which needs memory for its output: the caller's stream's, but not in a capture
+                import torch
+                if not torch.cuda.is_current_stream_capturing():
+                    between = torch.empty((m, n), dtype=out.dtype, device=a.device)
+                    y = between.data_ptr()
     d = FcDesc()
     _FC_DESC.pack_into(d, 0, a.data_ptr(), w_packed.data_ptr(), bias_ptr, y, p[0], p[1], p[2], a.stride(0), w_packed.stride(0),
-                       out.stride(0), m, n, k, dt, bz_dtype(out.dtype), bias_rows, act, act_size, int(dice_nosqrt), alpha, beta,
+                       ldy, m, n, k, dt, bz_dtype(out.dtype), bias_rows, act, act_size, int(dice_nosqrt), alpha, beta,
                        act_alpha, 0, hw_ptr, hb_ptr, hy_ptr, h_ldw, h_ldy, h_n, h_act, h_dt, 0, 0, 0, 0)
     check(lib().bz_fc_fused(C.byref(d), _stream_ptr(stream)))
     if head is not None:

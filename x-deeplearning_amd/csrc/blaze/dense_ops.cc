@@ -374,7 +374,8 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
 
  protected:
-  // whether the head is in this layer's launch at any number of rows, and at those of the input as it is shaped now
+  // Whether the head is in this layer's launch at any number of rows, and at those of the input as it is shaped now.  (The first
+  // also says yes where the head is better off apart at any number of rows: who asks it has layers too small for that.)
   bool HeadAtAnyRows() {
     Blob* b = this->Input(1);
     return (transb_ ? b->shape()[0] : b->shape()[1]) % 8 == 0;
@@ -383,6 +384,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     Blob *a = this->Input(0), *b = this->Input(1);
     const TIndex k = transb_ ? b->shape()[1] : b->shape()[0], n = transb_ ? b->shape()[0] : b->shape()[1];
     const int es = (int)DataTypeSize(a->data_type());
+    if (bz::head_apart(k, n, es)) return false;
     return HeadAtAnyRows() || (k > 0 && k * es % 16 == 0 && bz::head_behind_any_columns(a->size() / k, k, n, es));
   }
   // the hosted head as a launch of its own

@@ -72,4 +72,11 @@ inline bool head_behind_any_columns(int64_t rows, int64_t k, int64_t n, int elem
   return rows <= 2048 && (element_size == 4 ? rows * k <= 240 << 10 && k * n <= 36 << 10 : rows * k <= 768 << 10 && k * n <= 96 << 10);
 }
 
+// Whether an fp32 layer's head is better off behind it, in a launch of its own.  In the layer's launch a workgroup owns whole rows,
+// multiplies all of k * n for them, and the rows set how many CUs work; by itself the layer is on all of them.  One launch / two,
+// us alone (errors against 64 bits are smaller in two): 300 of 256 -> 100 (25 K) 7.1 / 7.3, 201 of 200 -> 80 6.4 / 7.4, 2048 of
+// 256 -> 64 6.1 / 7.5, 16384 of 200 -> 80 14.9 / 18.5; 1000 and 2000 of 512 -> 128 (64 K) 10.4 / 8.4 and 10.6 / 9.5, 64 of 2000 -> 48
+// 16.1 / 12.5, 1024 of 512 -> 256 16.6 / 8.8, 2048 17.0 / 11.8, 4096 25.3 / 16.4, 8192 26.1 / 25.2, 2000 of 4096 -> 256 102 / 41.
+inline bool head_apart(int64_t k, int64_t n, int element_size) { return element_size == 4 && k * n > 48 << 10; }
+
 }  // namespace bz

@@ -56,6 +56,8 @@ int bz_fc_fused(const bz_fc_desc* desc, bz_stream_t stream) {
   return run(*desc, nullptr, false, stream);
 }
 
+int bz_fc_head_apart(int k, int n, int in_dtype) { return bz::head_apart(k, n, bz::dtype_size(in_dtype)) ? 1 : 0; }
+
 }  // extern "C"
 
 int bz::fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
@@ -128,6 +130,27 @@ int run(const bz_fc_desc& d, void* copy, bool any_columns, bz_stream_t stream) {
                (long long)d.head_ldy);
     BZ_REQUIRE(d.head_out_dtype == BZ_F32 || d.head_out_dtype == BZ_F16 || d.head_out_dtype == BZ_BF16, "bz_fc_fused: head out dtype %d",
                d.head_out_dtype);
+  }
+  if (d.head_n != 0 && d.y != nullptr && bz::head_apart(d.k, d.n, es)) {
+    bz_fc_desc layer = d, head = {};
+    layer.head_n = 0;
+    head.a = d.y;
+    head.lda = d.ldy;
+    head.w = d.head_w;
+    head.ldw = d.head_ldw;
+    head.bias = d.head_bias;
+    head.bias_rows = d.head_bias != nullptr ? 1 : 0;
+    head.y = d.head_y;
+    head.ldy = d.head_ldy;
+    head.m = d.m;
+    head.n = d.head_n;
+    head.k = d.n;
+    head.in_dtype = d.out_dtype;
+    head.out_dtype = d.head_out_dtype;
+    head.act = d.head_act;
+    head.alpha = head.beta = 1.f;
+    const int rc = run(layer, nullptr, false, stream);
+    return rc != BZ_OK ? rc : run(head, copy, false, stream);
   }
   switch (d.in_dtype) {
     case BZ_F16: return bz::fc_run_f16(d, ep, vec_a, vec_w, copy, st);
