@@ -938,6 +938,87 @@ def test_output_sees_what_was_written_through_a_device_address(pb, through, when
             np.testing.assert_allclose(p.output_asnumpy(out), _sigmoid(np.full_like(x, step)), rtol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_outputs_with_every_bit_set_arrive_too(pb, dtype):
+    """A pass ends when its outputs have reached the host, which shows in the value that stood there before (all bits set): an
+    output that holds that value comes out as any other, in the passes before and behind it too."""
+    nb = pb.NetBuilder("bits", device_type=1)
+    code = pb.K_FLOAT16 if dtype == np.float16 else pb.K_FLOAT
+    for name in ("a", "b"):
+        nb.external_input(name, code)
+    nb.op("Concat", ["a", "b"], ["y"], axis=1)
+    nb.external_output("y", code)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    rng = np.random.default_rng(9)
+    bits = np.uint32 if dtype == np.float32 else np.uint16
+    for step in range(80):  # (every 32nd pass waits for the stream)
+        a, b = rng.standard_normal((5, 3)).astype(dtype), rng.standard_normal((5, 4)).astype(dtype)
+        if step in (3, 4, 40):
+            b.view(bits)[step % 5, step % 4] = ~bits(0)
+        p.reshape_input("a", a.shape)
+        p.reshape_input("b", b.shape)
+        p.feed_many(p.feed_batch([("a", a), ("b", b)]))
+        p.forward()
+        got = p.output_asnumpy("y").reshape(5, 7)
+        assert np.array_equal(got.view(bits), np.concatenate([a.view(bits), b.view(bits)], 1)), step
+
+
+def test_feed_forward_and_output_in_threads_of_their_own(pb):
+    """Inputs fed by one thread, the pass run by another, the output read by a third, each of them new or the same as last time,
+    fed twice before a pass, read twice behind it, and through the device address: always the pass's own."""
+    import threading
+    import torch
+    nb = pb.NetBuilder("threads", device_type=1)
+    nb.external_input("x", pb.K_FLOAT)
+    rng = np.random.default_rng(10)
+    w, u = (rng.standard_normal(sh).astype(np.float32) for sh in ((64, 32), (32, 2)))
+    nb.constant("w", w)
+    nb.constant("u", u)
+    nb.op("Gemm", ["x", "w"], ["h"])
+    nb.op("Gemm", ["h", "u"], ["y"])
+    nb.external_output("y", pb.K_FLOAT)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    errors = []
+
+    def run(where, f):
+        def guarded():
+            try:
+                f()
+            except Exception as e:  # noqa: BLE001
+                errors.append(repr(e))
+        if where == "here":
+            return guarded()
+        t = threading.Thread(target=guarded)
+        t.start()
+        t.join()
+
+    for step in range(60):
+        x = rng.standard_normal((300, 64)).astype(np.float32)
+        want = x.astype(np.float64) @ w.astype(np.float64) @ u.astype(np.float64)
+        who = ["here" if rng.random() < 0.6 else "there" for _ in range(3)]
+        p.reshape_input("x", x.shape)
+        if step % 7 == 0:
+            run(who[2], lambda: p.feed_many(p.feed_batch([("x", x + 1)])))
+        if step % 3:
+            run(who[0], lambda: p.feed_many(p.feed_batch([("x", x)])))
+        else:
+            run(who[0], lambda: p.feed("x", x))
+        run(who[1], p.forward)
+        got = []
+        run(who[2], lambda: got.append(p.output_asnumpy("y").copy()))
+        if step % 5 == 0:
+            run(who[0], lambda: got.append(p.output_asnumpy("y").copy()))
+        if step > 50:
+            got.append(torch.as_tensor(_DeviceArray(p.output_device_ptr("y"), (300, 2)), device="cuda").cpu().numpy())
+        assert not errors, errors
+        for g in got:
+            np.testing.assert_allclose(g.reshape(300, 2), want, rtol=0, atol=2e-4, err_msg="step %d %s" % (step, who))
+
+
 def test_outputs_copied_ahead_of_output(pb):
     """Ten outputs (one launch copies eight ahead) at batches whose outputs are below and above what is copied ahead
     (64 KB): read once, twice or not at all after a pass, in either order, after growing and shrinking.  Every read is the

@@ -98,6 +98,7 @@ class Predictor {
   size_t HostHalf(size_t i) const;   // bytes of a half of output_cpu_[i]
   void* HandOut(Blob* blob);
   bool CopiedAhead(size_t i) const;
+  bool Awaitable(size_t i) const;
   void OfferHostCopies();
   void QueueOutputs();
   void WithdrawHostCopies();
@@ -106,8 +107,26 @@ class Predictor {
   std::vector<std::shared_ptr<Blob>> input_cpu_;
   std::vector<bool> feed_pending_;
   bool any_feed_pending_ = false;
-  hipEvent_t feed_done_ = nullptr;  // recorded behind the last queued transfer; Forward's stream waits for it
-                                    // (Feed and Forward may be called from different threads = different streams)
+  // Feed and Forward may be called from different threads = different streams: an event behind the last queued transfer, which
+  // Forward's stream waits for.  Not recorded where the last Forward was on the transfer's stream, as it mostly is: in the
+  // stream the event costs 2.4 us between the transfer and the net.
+  hipEvent_t feed_done_ = nullptr;
+  uint64_t feed_on_ = 0, forward_on_ = 0;  // HIPContext::stream_serial of the last transfer's and the last pass's streams
+  bool feed_recorded_ = false;
+  void FeedQueued(const HIPContext& ctx);
+  void FinishFeeds();
+  void OrderBehindFeeds();
+  // A pass whose outputs all go to the host by itself ends when they are there: see PassIsThere.
+  struct Awaited {
+    void* at;
+    size_t elements, size;
+  };
+  std::vector<Awaited> awaited_;
+  bool await_outputs_ = true;  // false once an output had the value that stands for "not there yet"
+  bool settled_ = true;        // the last pass's stream has been waited for
+  int passes_unsettled_ = 0;
+  bool PassIsThere();
+  void Settle();
   char* arena_host_ = nullptr;         // FeedMany's pinned staging arena and its device twin
   char* arena_dev_ = nullptr;
   size_t arena_cap_ = 0;

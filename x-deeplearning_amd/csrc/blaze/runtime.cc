@@ -77,18 +77,27 @@ void HIPContext::Activate() const {
 }
 
 namespace {
+struct ThreadStream {
+  hipStream_t stream = nullptr;
+  uint64_t serial = 0;
+  void Set(hipStream_t s) {
+    static std::atomic<uint64_t> made{0};
+    stream = s;
+    serial = ++made;
+  }
+};
 struct ThreadStreams {
-  std::vector<std::vector<hipStream_t>> per_device;
+  std::vector<std::vector<ThreadStream>> per_device;
   ~ThreadStreams() {
     for (auto& v : per_device)
-      for (auto s : v)
-        if (s) (void)hipStreamDestroy(s);
+      for (auto& s : v)
+        if (s.stream) (void)hipStreamDestroy(s.stream);
   }
-  hipStream_t& at(int device_id, int stream_id) {
+  ThreadStream& at(int device_id, int stream_id) {
     BLAZE_CONDITION_THROW(device_id >= 0 && stream_id >= 0 && stream_id < kMaxStreamNum, "device_id=", device_id, " stream_id=", stream_id);
     if ((int)per_device.size() <= device_id) per_device.resize(device_id + 1);
     auto& v = per_device[device_id];
-    if (v.empty()) v.resize(kMaxStreamNum, nullptr);
+    if (v.empty()) v.resize(kMaxStreamNum);
     return v[stream_id];
   }
 };
@@ -99,24 +108,32 @@ ThreadStreams& StreamsOfThisThread() {
 }  // namespace
 
 hipStream_t HIPContext::hip_stream(int device_id, int stream_id) {
-  hipStream_t& s = StreamsOfThisThread().at(device_id, stream_id);
-  if (s == nullptr) {
+  ThreadStream& s = StreamsOfThisThread().at(device_id, stream_id);
+  if (s.stream == nullptr) {
     int cur = 0;
     HIP_CHECK(hipGetDevice(&cur));
     if (cur != device_id) HIP_CHECK(hipSetDevice(device_id));
-    HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));  // default priority
+    hipStream_t made = nullptr;
+    HIP_CHECK(hipStreamCreateWithFlags(&made, hipStreamNonBlocking));  // default priority
+    s.Set(made);
     if (cur != device_id) HIP_CHECK(hipSetDevice(cur));
   }
-  return s;
+  return s.stream;
+}
+
+uint64_t HIPContext::stream_serial() const {
+  (void)hip_stream();
+  return StreamsOfThisThread().at(device_id_, stream_id_).serial;
 }
 
 void HIPContext::AdoptThreadStream(int device_id, int stream_id, hipStream_t stream) {
-  hipStream_t& s = StreamsOfThisThread().at(device_id, stream_id);
-  if (s != nullptr && s != stream) {
-    HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipStreamDestroy(s));
+  ThreadStream& s = StreamsOfThisThread().at(device_id, stream_id);
+  if (s.stream == stream) return;
+  if (s.stream != nullptr) {
+    HIP_CHECK(hipStreamSynchronize(s.stream));
+    HIP_CHECK(hipStreamDestroy(s.stream));
   }
-  s = stream;
+  s.Set(stream);
 }
 
 void CopyBytes(void* dst, int dst_device_type, const void* src, int src_device_type, size_t bytes, hipStream_t stream) {

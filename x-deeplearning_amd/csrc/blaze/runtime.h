@@ -250,6 +250,8 @@ class HIPContext {
   hipStream_t hip_stream() const { return hip_stream(device_id_, stream_id_); }
   void* device_stream() const { return (void*)hip_stream(); }
   static hipStream_t hip_stream(int device_id, int stream_id);  // thread-local, created on first use
+  // a number that no other stream of the process has or had (a handle may be given out again once its thread is gone)
+  uint64_t stream_serial() const;
   // makes `stream` (created on device_id, default priority) the calling thread's stream from now on; the thread owns it:
   // it is destroyed when the thread ends, like one created on first use.  A stream the thread already had is
   // waited for and destroyed.
