@@ -214,6 +214,18 @@ def test_fc_fp32_error_of_a_layer_with_a_head(bz, M, N, K, parts):
     assert err <= _fp32_sum_error(K / parts), err
 
 
+# 2-byte layers of more than 256 tiles of 64x64: 64x128 and 128x64 tiles, also for rows that start on no 16 bytes
+@pytest.mark.parametrize("in_name,out_name", [("f16", "f16"), ("bf16", "f32")])
+@pytest.mark.parametrize("M,N,K,act,kw", [(1900, 520, 392, "dice", {}), (6017, 136, 64, "prelu", {"full_bias": True}),   # 64x128, ragged; one K tile
+                                          (16449, 64, 136, "relu", {}), (16448, 33, 72, "dice", {}), (17001, 9, 192, "none", {"full_bias": True}),  # 128x64
+                                          (16449, 40, 65, "prelu", {}), (2049, 513, 255, "dice", {}), (2050, 520, 9, "none", {}),   # off 16 bytes: one K tile in flight
+                                          (16449, 64, 257, "relu", {}), (3000, 390, 301, "sigmoid", {"full_bias": True}), (2049, 520, 523, "prelu", {})])  # two
+def test_fc_two_byte_layers_beyond_one_round_of_tiles(bz, oracle, in_name, out_name, M, N, K, act, kw):
+    print("case round %s M=%d N=%d K=%d act=%s %r" % (in_name, M, N, K, act, kw), flush=True)
+    assert -(-M // 64) * -(-N // 64) > 256
+    _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + N + K, **kw)
+
+
 def _plain_bound(x, w, bias):
     """what any order of K fp32 products and sums stays within, and a split that drops 2^-24 of a product"""
     return (x.shape[1] + 8) * 2.0**-24 * (x.double().abs() @ w.double().abs().t().contiguous() + bias.double().abs())

@@ -1475,23 +1475,40 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   // tall and narrow (the attention MLP over batch x history rows): one 96-wide tile reads A once
   if (d.n > 64 && d.n <= 96 && (d.m + 127) / 128 >= 256)
     return launch_mfma<DT, OutT, 128, 96, BK, 4, 1, 2, ALIGNED>(d, ep, st);
-  // 2-byte operands: eight waves on tiles of 128 columns with two K tiles in flight.  64 rows while that is one round of the
-  // CUs, 256 tiles; with more, 128 rows, where a second round of smaller tiles would cost as much as the first (us alone /
-  // with eight streams of the same, 64 rows, 128 rows, four waves on 64x64: 2048 x 896 -> 1024, 256 tiles of 64 rows,
-  // 10.1 / 7.2, 12.8 / 6.7, 11.1 / 7.6; 2176 rows, 272 tiles, 14.1 / 8.5, 13.3 / 8.0, 13.5 / 8.8; 2048 x 2048 -> 1024
-  // 17.9 / 14.3, 22.5 / 13.2, 20.5 / 15.9; 2176 rows 26.2 / 17.4, 23.1 / 16.3, 24.9 / 21.1).  Where K is shallow the second
-  // round is short and the line lies a little higher (2176 x 128 -> 1024 5.7 / 3.1 and 6.5 / 3.1, 2304 rows, 288 tiles,
-  // 5.7 / 3.1 and 6.0 / 3.1).
+  // 2-byte operands: eight waves with two K tiles in flight as soon as 64x64 tiles make more than one round of the CUs: 64x128
+  // then, 128x64 where that covers the columns, and 128x128 from 129 tiles on, where another round of the smaller ones
+  // would cost as much as the first.  us alone / with eight streams of the same: four waves on 64x64 with two K tiles in flight,
+  // 64x128, 128x64, 128x128:
+  //  2048 x 896 -> 512, 256 tiles of 64x64, 7.6 / 4.9, 8.5 / 4.4, 8.6 / 4.8, 11.3 / 5.4; 1100 x 512 -> 1000, 288, 7.3 / 4.0, 6.5 / 3.9,
+  //  6.6 / 3.8; 1500 x 896 -> 704, 264, 9.6 / 5.1, 8.5 / 5.1, 8.6 / 4.8; 2048 x 896 -> 1024, 128 of 128x128, 10.6 / 7.8, 9.6 / 7.3,
+  //  9.8 / 7.1, 11.9 / 6.8; 2176 rows, 136, 13.3 / 8.9, 13.6 / 8.5, 14.4 / 9.1, 12.7 / 7.5; 2048 x 2048 -> 1024 17.9 / 14.3 (64x128) and 22.5 / 13.2,
+  //  2176 rows 26.2 / 17.4 and 23.1 / 16.3; 20000 x 896 -> 64 10.1 / 6.4, 13.2 / 8.5, 9.2 / 6.2; 17000 x 512 -> 64, 266, 7.2 / 4.4, 9.1 / 5.4,
+  //  6.6 / 4.0; 6000 rows of 2048 -> 64, 94, 11.8 / 6.5, 14.6 / 7.7, 14.6 / 7.3.
+  // Before, four waves on 64x64 with four K tiles in flight up to 256 tiles of 64x128: 1500 x 896 -> 704 10.7 / 5.5, 2500 x 640 -> 400 9.1 / 4.7
+  // and now 7.1 / 4.3, 50000 x 128 -> 64 9.0 / 5.9 and 5.8 / 4.3.
+  // Where K is shallow the second round is short and the line to 128x128 lies a little higher (2176 x 128 -> 1024 5.7 / 3.1 and
+  // 6.5 / 3.1, 2304 rows, 288 tiles of 64x128, 5.7 / 3.1 and 6.0 / 3.1).
+  // Rows that start anywhere: 128x64 (64x64, 64x128, 128x64: 3000 x 901 -> 400 16.5 / 9.7, 13.4 / 8.5, 12.8 / 7.6; 20000 x 901 -> 64 15.7 / 9.4, 20.9 / 13.0,
+  // 12.8 / 8.1; 12000 x 301 -> 100 10.4 / 6.0, 9.0 / 5.1, 9.4 / 5.5), up to four K tiles one in flight, as below (4000 x 61 -> 512 5.5 / 3.7
+  // and 5.2 / 3.3, with two 6.1 / 3.9; 10000 x 162 -> 200 6.9 / 4.3 and 6.9 / 4.2, 8.1 / 4.6).  At 257 to 272 tiles of 64x64 with deep rows
+  // that start anywhere the line is not sharp: 4288 x 1501 -> 200 19.1 / 9.7 (64x64) and 16.6 / 9.1, 4352 rows 15.9 / 9.3 and 16.7 / 9.2.
   if constexpr (In<DT>::kSize == 2) {
     if (d.n > 64 && wg128 >= (d.k > 256 ? 129 : 140)) return launch_mfma<DT, OutT, 128, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
-    if (d.n > 64 && wg64x128 >= 256) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
+    if (wg64 > 256) {
+      if constexpr (ALIGNED) {
+        if (d.n > 64) return launch_mfma<DT, OutT, 64, 128, BK, 2, 4, 2, ALIGNED>(d, ep, st);
+      } else if (d.k <= 4 * BK) {
+        return launch_mfma<DT, OutT, 128, 64, BK, 4, 2, 1, ALIGNED>(d, ep, st);
+      }
+      return launch_mfma<DT, OutT, 128, 64, BK, 4, 2, 2, ALIGNED>(d, ep, st);
+    }
   } else if constexpr (ALIGNED) {
     if (d.n > 64 && wg128 >= 512) return launch_mfma<DT, OutT, 128, 128, BK, 2, 2, 3, ALIGNED>(d, ep, st);
     if (d.n > 64 && wg64x128 >= 512) return launch_mfma<DT, OutT, 64, 128, BK, 2, 2, 4, ALIGNED>(d, ep, st);
   }
   // Rows that start anywhere: K is seldom a whole number of tiles, and a tile that is loaded only to be dropped costs as
-  // much as any other, so few are in flight: one while K is at most four tiles of 2-byte operands, else two.  64x64
-  // however many there are (us alone / with eight streams of the same; 32x64 or 64x64 with four in flight: fp16
+  // much as any other, so few are in flight: one while K is at most four tiles of 2-byte operands, else two.  64x64,
+  // 4-byte rows however many there are (us alone / with eight streams of the same; 32x64 or 64x64 with four in flight: fp16
   // 3000 x 162 -> 200 8.1 / 3.7, now 6.0 / 2.8, 10000 x 50 -> 64 8.8 / 3.6 and 4.5 / 2.1, 2000 x 901 -> 400 14.9 / 9.2 and
   // 10.3 / 5.8).
   if constexpr (!ALIGNED) {
@@ -1503,14 +1520,9 @@ int dispatch_mid(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
       // (two K tiles in flight; with four waves sharing each, 10000 x 64 -> 200 14.5 / 9.4 and this way 9.6 / 5.8)
       return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     } else {
-      // Four K tiles in flight (120 VGPRs, three waves per SIMD).  Seven save a round trip on config 2's 896-deep layer
-      // when the kernel runs alone (9.2 against 9.8 us) but hold 182 VGPRs, and next to the kernels of other serving
-      // threads the leaner one wins: 127.5 against 121 M samples/s at the same forward latency.  (Eight waves on two K
-      // tiles likewise: 7.3 against 8.5 us alone, 2.3 % fewer passes with eight serving threads.)
-      if (wg64 >= 256) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 4, ALIGNED>(d, ep, st);
-      // Below a workgroup per CU the same tile with two in flight (1500 x 896 -> 512 7.9 us alone / 4.0 with eight streams of
-      // the same, 32x64 with four 10.8 / 5.8; 5000 x 128 -> 100 5.8 / 2.6 and 7.2 / 3.2), or the one that there is
-      // (730 x 64 -> 512 3.7 / 1.7, with two 4.0 / 1.8)
+      // Two K tiles in flight, or the one that there is (2048 x 896 -> 512 7.6 us alone / 4.9 with eight streams of the same, with
+      // four in flight 8.4 / 4.9, and the model of that layer on eight serving threads 14.2 us a pass with either; 1500 x 896 -> 512
+      // 7.9 / 4.0, 32x64 with four 10.8 / 5.8; 730 x 64 -> 512 with one 3.7 / 1.7, with two 4.0 / 1.8)
       if (d.k <= BK) return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 1, ALIGNED>(d, ep, st);
       return launch_mfma<DT, OutT, 64, 64, BK, 2, 2, 2, ALIGNED>(d, ep, st);
     }
