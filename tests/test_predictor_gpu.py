@@ -1311,3 +1311,28 @@ def test_feed_many_of_strided_inputs(pb, n_in):
             p.forward()
             np.testing.assert_array_equal(p.output_asnumpy("z"), np.concatenate(xs, 1))
             np.testing.assert_allclose(p.output_asnumpy("s"), _sigmoid(plain), rtol=1e-5)
+
+
+# bytes of the inputs, one behind the other on multiples of 256: parts end after 384, 960, 1824 KB and then every MB, from 4 MB on every
+# MB, unless less than half a part would be left
+@pytest.mark.parametrize("sizes", [[4, 393212], [393216, 196604], [393216, 196608], [393216, 196612], [393000, 300, 300000],   # in the padding; left over: half a part or less
+                                   [393212, 4, 600000], [983040, 4, 430000], [300, 983040 - 512, 900000, 2 << 20], [(4 << 20) - 256, 4],
+                                   [(4 << 20) - 512, 252], [5 << 20, 260], [(1 << 20) - 4, 4, 4 << 20]])
+def test_feed_many_at_the_borders_of_its_parts(pb, sizes):
+    rng = np.random.default_rng(sum(sizes))
+    nb = pb.NetBuilder("parts", device_type=1)
+    for k in range(len(sizes)):
+        nb.external_input("x%d" % k, pb.K_FLOAT)
+        nb.op("Sigmoid", ["x%d" % k], ["y%d" % k])
+        nb.external_output("y%d" % k, pb.K_FLOAT)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for _ in range(2):
+        xs = [rng.standard_normal((s // 4, 1)).astype(np.float32) for s in sizes]
+        for k, x in enumerate(xs):
+            p.reshape_input("x%d" % k, x.shape)
+        p.feed_many(p.feed_batch([("x%d" % k, x) for k, x in enumerate(xs)]))
+        p.forward()
+        for k, x in enumerate(xs):
+            np.testing.assert_allclose(p.output_asnumpy("y%d" % k).reshape(-1), _sigmoid(x).reshape(-1), rtol=1e-5)

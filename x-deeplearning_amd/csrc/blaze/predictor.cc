@@ -170,13 +170,15 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
   return true;
 }
 
-// A request is moved in as many even parts as it has whole megabytes (at least one), each launched as soon as it is
-// staged.  Staging runs at 58 GB/s and the kernel at 47, so the transfer hides under the staging but for the last part and
-// the difference; a launch costs the host 2.9 us, the time of 160 KB, so that 1 MB in four parts was 5 us slower than in
-// one.  (The copy engine moves 57 GB/s, but each copy costs 10 us until what follows it on the stream may start: 5 MB in
-// ten parts arrived 230 us after the first byte was staged, in one part behind the whole staging 210, through five
-// launches of the kernel 162.)
-constexpr size_t kFeedPart = 1 << 20;
+// A request is moved in parts, each launched as soon as it is staged.  Up to 4 MB the link is what bounds it (the kernel moves
+// 47 GB/s and leaves a gap behind each launch, staging runs at 58), so it starts early: 384 KB first, each part half as large
+// again as the one before until 1 MB.  Beyond, staging is (35 GB/s, the copies no longer fit the caches between requests), and a
+// launch costs the host 2.9 us: parts of 1 MB.  The last part takes what would be left of it below half a part.  us to the end of a
+// request among others, even parts of 1 MB or more / these: 0.74 MB 79.3 / 78.5, 1.07 92.8 / 88.5, 1.8 125 / 112, 2.5 115 / 112,
+// 3 135 / 127, 4 162 / 158, 4.6 180..191 / 184..194, 5.1 203 / 217.  (The copy engine moves 57 GB/s, but each copy costs 10 us until
+// what follows it on the stream may start: 5 MB in ten parts arrived 230 us after the first byte was staged, in one part behind
+// the whole staging 210, through five launches of the kernel 162.)
+constexpr size_t kFeedFirst = 384 << 10, kFeedMost = 1 << 20, kFeedLong = 4 << 20;
 
 // a transfer has been queued on the context's stream
 void Predictor::FeedQueued(const HIPContext& ctx) {
@@ -284,15 +286,16 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
     }
     // from the first launch on the arena is being read: whatever happens next, it is waited for before it is written again
     try {
-      const size_t parts = std::max<size_t>(plain / kFeedPart, 1), part = (plain / parts / 256 + 1) * 256;
       bz_feed_rows rows[BZ_FEED_MAX_ROWS];
-      size_t moved = 0;
+      size_t moved = 0, part = plain < kFeedLong ? kFeedFirst : kFeedMost;
       int n = 0;
       auto launch = [&](size_t upto) {
         BZ_CHECK(bz_feed(arena_host_ + moved, arena_dev_ + moved, (int64_t)(upto - moved), rows, n, st));
         moved = upto;
         n = 0;
       };
+      auto end_of_part = [&]() { return plain - moved < part + part / 2 ? plain : moved + part; };
+      size_t end = end_of_part();
       for (const Item& it : strided) {
         if (n == BZ_FEED_MAX_ROWS) launch(moved);
         memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
@@ -301,10 +304,14 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       for (const Item& it : in_arena)
         for (size_t at = 0; at < lens[it.arg];) {
           // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte)
-          const size_t len = std::min(lens[it.arg] - at, moved + part - (it.offset + at));
+          const size_t len = std::min(lens[it.arg] - at, end - (it.offset + at));
           memcpy(arena_host_ + it.offset + at, (const char*)data[it.arg] + at, len);
           at += len;
-          if (it.offset + at == moved + part) launch(it.offset + at);
+          if (it.offset + at == end) {
+            launch(end);
+            part = std::min(part + part / 2, kFeedMost);
+            end = end_of_part();
+          }
         }
       if (plain > moved || n > 0) launch(plain);
       FeedQueued(ctx);
