@@ -438,7 +438,7 @@ def fc_fused(a, w_packed, k, bias=None, act=ACT_NONE, act_params=(), out=None, o
             hb_ptr = hb.data_ptr()
         if not store_out:
             y, ldy = 0, n
-            if dt == F32 and stream is None and lib().bz_fc_head_apart(k, n, dt):
+            if dt == F32 and k * n >= 1 << 15 and stream is None and lib().bz_fc_head_apart(k, n, dt):  # (no smaller one is: spares the call)
                 # the head runs behind the layer, which needs memory for its output: the caller's stream's, but not in a capture
                 import torch
                 if not torch.cuda.is_current_stream_capturing():
