@@ -1336,3 +1336,104 @@ def test_feed_many_at_the_borders_of_its_parts(pb, sizes):
         p.forward()
         for k, x in enumerate(xs):
             np.testing.assert_allclose(p.output_asnumpy("y%d" % k).reshape(-1), _sigmoid(x).reshape(-1), rtol=1e-5)
+
+
+def _tower(pb, ws, bs, acts, chain, heads):
+    nb = pb.NetBuilder("tower%d" % chain, device_type=1)
+    nb.arg("chain_narrow_fcs", chain)
+    nb.external_input("x", pb.K_FLOAT16)
+    h = "x"
+    for i, (w, b) in enumerate(zip(ws, bs)):
+        nb.constant("w%d" % i, w)
+        nb.constant("b%d" % i, b)
+        nb.op("Gemm", [h, "w%d" % i, "b%d" % i], ["g%d" % i], transB=0)
+        h = "g%d" % i
+        if i < 2 and acts[i] is not None:
+            ins = [h]
+            for j, p in enumerate(acts[i][1:]):
+                nb.constant("a%d%d" % (i, j), p)
+                ins.append("a%d%d" % (i, j))
+            h = "h%d" % i
+            nb.op(acts[i][0], ins, [h])
+    if heads > 1:
+        nb.op("Softmax", [h], ["p"], axis=1)
+    else:
+        nb.op("Sigmoid", [h], ["p"])
+    nb.external_output("p", pb.K_FLOAT16)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    return pm.create_predictor(1, 0)
+
+
+def _tower_act(z, act):
+    if act is None:
+        return z
+    if act[0] == "PRelu":
+        return np.where(z > 0, z, z * act[1].astype(np.float64))
+    if act[0] == "Dice":
+        g, m, v = (a.astype(np.float64) for a in act[1:])
+        p = _sigmoid((z - m) / np.sqrt(v + 1e-8))
+        return (1 - p) * g * z + p * z
+    return _sigmoid(z)
+
+
+# k: one input, rows of 16-byte, 4-byte and 2-byte steps, whole and ragged 64s, the longest that is staged at once and the longest taken;
+# n1: one and two blocks a wave; n2, heads: the smallest and the largest; rows: one workgroup's edges and the lines of bz::fc_tower_pays
+@pytest.mark.parametrize("k,n1,n2,heads,rows", [(1, 9, 9, 1, (1, 33)), (64, 32, 33, 2, (31, 32, 33, 4096, 4097)), (65, 33, 64, 8, (5, 300)), (66, 256, 100, 2, (300, 64)),
+                                                (445, 256, 100, 2, (300, 1, 2049)), (448, 257, 256, 3, (40, 4096)), (1024, 192, 96, 1, (70, 2)), (1027, 200, 80, 2, (33, 500)),
+                                                (1280, 160, 40, 2, (100, )), (896, 512, 256, 2, (1399, 1400, 2048, 32)), (128, 512, 250, 8, (77, 1500))])
+@pytest.mark.parametrize("act", ["PRelu", "Dice", "Sigmoid", None])
+def test_tower_in_one_launch(pb, k, n1, n2, heads, rows, act):
+    """fp16 layer -> layer -> skinny layer against 64 bits from the rounded layers and against one launch a layer, the rows growing and
+    shrinking past the lines beyond which it is no launch of its own; and while the operators are timed one by one."""
+    rng = np.random.default_rng(k * n1 + n2)
+    sizes = (k, n1, n2, heads)
+    ws = [(rng.standard_normal(s) / np.sqrt(s[0])).astype(np.float16) for s in zip(sizes, sizes[1:])]
+    bs = [(rng.standard_normal(n) * 0.1).astype(np.float16) for n in sizes[1:]]
+    acts = []
+    for n in (n1, n2):
+        p = [rng.uniform(0.1, 0.4, n).astype(np.float16), (rng.standard_normal(n) * 0.1).astype(np.float16), rng.uniform(0.5, 1.5, n).astype(np.float16)]
+        acts.append({"PRelu": ("PRelu", p[0]), "Dice": ("Dice", *p), "Sigmoid": ("Sigmoid", ), None: None}[act])
+    one, apart = (_tower(pb, ws, bs, acts, chain, heads) for chain in (1, 0))
+    for step, m in enumerate(rows + rows[:1]):
+        print("tower %d x %d -> %d -> %d -> %d %s" % (m, k, n1, n2, heads, act), flush=True)
+        if step == len(rows):
+            one.register_observers(["profile"])
+        x = rng.standard_normal((m, k)).astype(np.float16)
+        got = []
+        for p in (one, apart):
+            p.feed("x", x)
+            p.forward()
+            got.append(p.output_asnumpy("p").astype(np.float64).reshape(m, heads))
+        h = x.astype(np.float64)
+        for w, b, a in zip(ws[:2], bs, acts):
+            h = _tower_act(h @ w.astype(np.float64) + b, a).astype(np.float16).astype(np.float64)
+        z = h @ ws[2].astype(np.float64) + bs[2]
+        e = np.exp(z - z.max(1, keepdims=True)) if heads > 1 else z
+        want = e / e.sum(1, keepdims=True) if heads > 1 else _sigmoid(z)
+        # a hidden value between two fp16s may be rounded to either, 2^-10 of itself apart: of sqrt(sum of squares) about 1 at the next
+        # layer, and the result, at most 1 with a slope of at most 1/4, is rounded to 2^-11
+        for g in got:
+            np.testing.assert_allclose(g, want, rtol=0, atol=4 * 2.0**-11, err_msg="%d rows" % m)
+
+
+@pytest.mark.parametrize("k", [72, 70, 69])
+def test_tower_rows_do_not_reach_into_each_other(pb, k):
+    """infinities and NaNs in some rows, the last one of a workgroup and of the input among them: the others come out as without"""
+    rng = np.random.default_rng(k)
+    ws = [(rng.standard_normal(s) / np.sqrt(s[0])).astype(np.float16) for s in ((k, 100), (100, 50), (50, 2))]
+    bs = [(rng.standard_normal(n) * 0.1).astype(np.float16) for n in (100, 50, 2)]
+    p = _tower(pb, ws, bs, [("PRelu", np.full(100, 0.25, np.float16)), None], 1, 2)
+    x = rng.standard_normal((70, k)).astype(np.float16)
+    bad = [0, 31, 64, 69]
+    got = []
+    for values in (None, (np.inf, np.nan, -np.inf, np.inf)):
+        y = x.copy()
+        if values is not None:
+            y[bad, [0, k - 1, k - 1, k - 1]] = values
+        p.feed("x", y)
+        p.forward()
+        got.append(p.output_asnumpy("p").reshape(70, 2).copy())
+    rest = [i for i in range(70) if i not in bad]
+    np.testing.assert_array_equal(got[0][rest], got[1][rest])
+    assert np.isnan(got[1][31]).all()

@@ -71,7 +71,8 @@ struct FcCall {
   // operands
   const void* a = nullptr;
   const bz_concat_ew_desc* a_pieces = nullptr;  // instead of a: the rows as pieces computed on the fly (bz_fc_desc.a_pieces)
-  const bz_fc_next* next = nullptr;             // with a_pieces: a second layer in the same launch
+  const bz_fc_next* next = nullptr;             // with a_pieces or tower_w: a second layer in the same launch
+  const void* tower_w = nullptr;                // instead of b: the weight as bz::fc_tower takes it
   int a_rows = 0, a_cols = 0;  // as stored
   bool trans_a = false;
   Blob* b_blob = nullptr;
@@ -105,7 +106,7 @@ struct FcCall {
   void* copy = nullptr;  // bz::fc_fused's
 };
 
-// false only with a_pieces, when the kernel does not take them (nothing has been launched then)
+// false only with a_pieces or tower_w, when the kernel does not take them (nothing has been launched then)
 bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st) {
   const int P = c.slices;
   const int M = c.trans_a ? c.a_cols : c.a_rows;
@@ -130,7 +131,10 @@ bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st
   }
   // W: [N,K] with aligned rows is used in place (stacked slices under trans_b are exactly that), anything else is
   // packed (once for constants), slice by slice when the slices are stacked [K,N] matrices
-  if (c.trans_b && (K % chunk == 0) && ((uintptr_t)c.b % 16 == 0)) {
+  if (c.tower_w != nullptr) {
+    d.w = c.tower_w;
+    d.ldw = K;
+  } else if (c.trans_b && (K % chunk == 0) && ((uintptr_t)c.b % 16 == 0)) {
     d.w = c.b;
     d.ldw = K;
   } else {
@@ -181,6 +185,13 @@ bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st
     d.head_n = c.head_n;
     d.head_act = c.head_act;
     d.head_out_dtype = BzType(c.head_y_dtype);
+  }
+  if (c.tower_w != nullptr) {
+    d.next = c.next;
+    const int rc = bz::fc_tower(d, c.copy, st);
+    if (rc == BZ_ENOTSUP) return false;
+    BZ_CHECK(rc);
+    return true;
   }
   if (c.a_pieces != nullptr) {
     d.a_pieces = c.a_pieces;
@@ -325,25 +336,45 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   }
   bool CanChainNext(OperatorBase* next_op) override {
     auto* g = dynamic_cast<GemmOp*>(next_op);
-    if (g == nullptr || concat_ == nullptr || head_ != nullptr || !siblings_.empty() || next_ != nullptr) return false;
+    if (g == nullptr || head_ != nullptr || !siblings_.empty() || next_ != nullptr || tower_ != nullptr) return false;
     Blob* b0 = this->Input(1);
     Blob* b = g->Input(1);
+    // without a Concat of its own this layer takes the next one only with a skinny one behind that, 2-byte ones of some sizes: a tower
+    const bool tower = concat_ == nullptr;
+    if (tower && (!b_constant_ || transa_ || b0->shape().size() != 2 || DataTypeSize(b0->data_type()) != 2 || g->head_ == nullptr || g->next_ != nullptr || g->tower_ != nullptr ||
+                  g->head_->Input(1)->data_type() != b0->data_type() || (fused_ && fused_act_ == BZ_ACT_SOFTMAX)))
+      return false;
+    if (tower && this->InputSize() > 2 && (!c_constant_ || this->Input(2)->size() != (transb_ ? b0->shape()[0] : b0->shape()[1]))) return false;
     if (!g->b_constant_ || g->transa_ || b->shape().size() != 2 || b->data_type() != b0->data_type()) return false;
     if (!g->siblings_.empty() || g->concat_ != nullptr) return false;
     const TIndex N1 = transb_ ? b0->shape()[0] : b0->shape()[1];
     const TIndex K2 = g->transb_ ? b->shape()[1] : b->shape()[0], N2 = g->transb_ ? b->shape()[0] : b->shape()[1];
-    if (K2 != N1 || N2 <= 8 || N2 > 64) return false;
+    if (K2 != N1 || N2 <= 8) return false;
+    if (tower ? !bz::fc_tower_takes(transb_ ? b0->shape()[1] : b0->shape()[0], N1, N2) : N2 > 64) return false;
     if (g->InputSize() > 2 && (!g->c_constant_ || (TIndex)g->Input(2)->size() != N2)) return false;
     if (g->fused_ && g->fused_act_ == BZ_ACT_SOFTMAX) return false;
     if (g->fused_ && g->fused_act_ == BZ_ACT_PRELU && (TIndex)g->fused_->Input(1)->size() != N2 && g->fused_->Input(1)->size() != 1) return false;
     return true;
   }
-  void AdoptNext(OperatorBase* next_op) override { next_ = static_cast<GemmOp*>(next_op); }
+  bool AdoptNext(OperatorBase* next_op) override {
+    (concat_ != nullptr ? next_ : tower_) = static_cast<GemmOp*>(next_op);
+    return concat_ != nullptr;
+  }
+  void RunApart(bool apart) override { apart_ = apart; }
 
   int LaunchesOfLastRun() const override { return launches_; }
 
   bool RunOnDevice() override {
+    if (in_tower_) {  // the layer before this one has computed it
+      in_tower_ = false;
+      launches_ = 0;
+      return true;
+    }
     launches_ = 1;
+    if (tower_ != nullptr) {
+      tower_->in_tower_ = !apart_ && TowerAtTheseRows() && RunSelf(false, nullptr, true);
+      if (tower_->in_tower_) return true;
+    }
     if (concat_ != nullptr) {
       bool stored = false;
       if (siblings_.empty() && (head_ == nullptr || !HeadAtAnyRows())) {
@@ -386,6 +417,13 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     const int es = (int)DataTypeSize(a->data_type());
     if (bz::head_apart(k, n, es)) return false;
     return HeadAtAnyRows() || (k > 0 && k * es % 16 == 0 && bz::head_behind_any_columns(a->size() / k, k, n, es));
+  }
+  // Whether this layer, the next and its head are one launch at the rows of the input as it is shaped now.
+  bool TowerAtTheseRows() {
+    Blob *a = this->Input(0), *b = this->Input(1), *b2 = tower_->Input(1);
+    const TIndex k = transb_ ? b->shape()[1] : b->shape()[0], n = transb_ ? b->shape()[0] : b->shape()[1];
+    const TIndex n2 = tower_->transb_ ? b2->shape()[0] : b2->shape()[1];
+    return a->pitch() == 0 && k > 0 && bz::fc_tower_pays(a->size() / k, k, n, n2);
   }
   // the hosted head as a launch of its own
   bool RunHeadAlone() {
@@ -548,14 +586,15 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   // with_head: also compute head_'s layer in this launch and leave this layer's own output unstored; false when the
   // operands do not allow it (nothing has been launched then)
   // pieces: the input given as pieces computed on the fly (an adopted Concat); false when the kernel does not take them
-  // chain: also run next_ (and the skinny layer it hosts) in this launch; this layer's and next_'s own outputs are then
-  // not stored
+  // chain: also run next_, or without pieces tower_, (and the skinny layer it hosts) in this launch; this layer's and the next
+  // one's own outputs are then not stored.  False when the kernel does not take it (nothing has been launched then)
   bool RunSelf(bool with_head, const bz_concat_ew_desc* pieces = nullptr, bool chain = false) {
     CheckValid();
     Blob* a = this->Input(0);
     Blob* b = this->Input(1);
     Blob* c = this->InputSize() > 2 ? this->Input(2) : nullptr;
     Blob* y = fused_ ? fused_->Output(0) : this->Output(0);
+    const bool tower = chain && pieces == nullptr;
     if (with_head) {
       const size_t es = DataTypeSize(a->data_type());
       const TIndex k = a->shape().back();
@@ -597,23 +636,35 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     }
     hipStream_t st = context_.hip_stream();
     FcCall call;
-    bz_fc_next nx;
+    bz_fc_next nx = {};
     if (chain) {
-      // next_ (with its folded activation) as bz_fc_next, the skinny layer it hosts through the head_* fields
-      GemmOp* g = next_;
+      // the next layer (with its folded activation) as bz_fc_next, the skinny layer it hosts through the head_* fields
+      GemmOp* g = tower ? tower_ : next_;
       Blob* b2 = g->Input(1);
       if (y->data_type() != a->data_type()) return false;
       const int es2 = (int)DataTypeSize(b2->data_type());
       const int n2 = (int)(g->transb_ ? b2->shape()[0] : b2->shape()[1]);
       const int64_t ldw2 = (N + 7) / 8 * 8;
-      if (g->packed_b_.Stale(b2) || g->packed_b_.bytes < (size_t)n2 * ldw2 * es2) {
+      if (tower) {
+        auto laid_out = [&](GemmOp* of, int k_in, int n_out) {
+          Blob* w = of->Input(1);
+          const size_t bytes = bz::fc_tower_weight_bytes(k_in, n_out);
+          if (of->tower_w_.Stale(w) || of->tower_w_.bytes < bytes) {
+            of->tower_w_.Resize(bytes);
+            BZ_CHECK(bz::fc_tower_pack(w->data(), of->transb_, k_in, n_out, of->tower_w_.ptr, st));
+            of->tower_w_.Mark(w);
+          }
+          return of->tower_w_.ptr;
+        };
+        call.tower_w = laid_out(this, (int)K, (int)N);
+        nx.w = laid_out(g, (int)N, n2);
+      } else if (g->packed_b_.Stale(b2) || g->packed_b_.bytes < (size_t)n2 * ldw2 * es2) {
         g->packed_b_.Resize((size_t)n2 * ldw2 * es2);
         BZ_CHECK(bz_fc_pack_weight(b2->data(), BzType(b2->data_type()), g->transb_ ? 1 : 0, (int)N, n2, g->packed_b_.ptr,
                                    BzType(b2->data_type()), ldw2, st));
         g->packed_b_.Mark(b2);
       }
-      memset(&nx, 0, sizeof(nx));
-      nx.w = g->packed_b_.ptr;
+      if (!tower) nx.w = g->packed_b_.ptr;
       nx.ldw = ldw2;
       nx.n = n2;
       nx.alpha = g->alpha_;
@@ -651,6 +702,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
         }
         y2->SetShapeOnly(shape2);
         Blob* hy3 = h->fused_ ? h->fused_->Output(0) : h->Output(0);
+        if (tower) hy = hy3;
         std::vector<TIndex> shape3 = shape2;
         shape3.back() = n3;
         hy3->Reshape(shape3);
@@ -729,9 +781,9 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
       }
     }
     // (fused_ or head_: the activation behind the layer is in the launch, so this is the whole output)
-    Blob* out = with_head ? hy : y;
+    Blob* out = with_head || tower ? hy : y;
     const size_t bytes = out->size() * DataTypeSize(out->data_type());
-    if (pieces == nullptr && (with_head || N <= 8)) call.copy = out->host_copy().Take(bytes);
+    if (pieces == nullptr && (with_head || tower || N <= 8)) call.copy = out->host_copy().Take(bytes);
     if (!RunFc(call, &packed_b_, &packed_a_, st)) return false;
     if (call.copy != nullptr) out->host_copy().copied = bytes;
     return true;
@@ -766,10 +818,13 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   float alpha_, beta_;
   bool transa_, transb_;
   bool b_constant_ = false, c_constant_ = false;
-  Derived packed_b_, packed_a_, bias_f32_, p_f32_[3];
+  Derived packed_b_, packed_a_, bias_f32_, p_f32_[3], tower_w_;
   GemmOp* head_ = nullptr;       // the layer of at most 8 outputs computed in this operator's launch
   OperatorBase* concat_ = nullptr;  // the Concat that makes Input(0), computed by this operator's kernel
   GemmOp* next_ = nullptr;          // the narrow layer after this one, computed in this operator's launch
+  GemmOp* tower_ = nullptr;         // the layer after this one, computed with its head in this operator's launch where that pays
+  bool apart_ = false;              // (but not while the operators are timed one by one)
+  bool in_tower_ = false;           // this pass, the layer before has computed this one
   std::vector<GemmOp*> siblings_;  // layers on the same input computed in this operator's launch
   Derived sib_w_, sib_f32_, sib_y_;  // stacked weights / fp32 parameters / outputs
   const Blob* sib_src_ = nullptr;    // this layer's weight as it was stacked

@@ -160,6 +160,12 @@ void Net::Wait() {
   if (!operators_.empty()) operators_.back()->WaitStream();
 }
 
+void Net::set_profile(bool on) {
+  profile_ = on;
+  for (auto& op : operators_)
+    if (auto* fc = dynamic_cast<ConcatAdopter*>(op.get())) fc->RunApart(on);
+}
+
 std::string Net::DumpProfile() const {
   std::stringstream ss;
   ss << "{\"traceEvents\":[";
@@ -429,14 +435,15 @@ void SimpleNet::FuseConcatsIntoFcs() {
 }
 
 // A Gemm that computes its Concat input itself -> the narrow Gemm that reads only its result: the second (and the skinny
-// layer it may host) runs in the first one's launch (graph.h, ConcatAdopter::CanChainNext).  Switch: chain_narrow_fcs: 0.
+// layer it may host) runs in the first one's launch (graph.h, ConcatAdopter::CanChainNext).  So does the second layer of a tower,
+// Gemm -> Gemm with a skinny layer behind it.  Switch: chain_narrow_fcs: 0.
 void SimpleNet::ChainNarrowFcs() {
   const Argument* arg = ArgumentHelper::Find(net_def_->arg_, "chain_narrow_fcs");
   if (arg && arg->has_i && arg->i == 0) return;
   for (size_t i = 0; i < operators_.size(); ++i) {
     auto* first = skipped_[i] ? nullptr : dynamic_cast<ConcatAdopter*>(operators_[i].get());
     auto* first_fc = first ? dynamic_cast<StackableFc*>(operators_[i].get()) : nullptr;
-    if (!first || !first_fc || !first->HasAdoptedConcat()) continue;
+    if (!first || !first_fc) continue;
     size_t j = i + 1;
     while (j < operators_.size() && skipped_[j]) ++j;  // (the first layer's folded activation)
     if (j >= operators_.size()) break;
@@ -448,8 +455,7 @@ void SimpleNet::ChainNarrowFcs() {
     bool is_output = false;
     for (const auto& eo : external_output_) is_output |= (eo == mid);
     if (readers != 1 || is_output) continue;
-    first->AdoptNext(operators_[j].get());
-    skipped_[j] = true;
+    skipped_[j] = first->AdoptNext(operators_[j].get());
   }
 }
 

@@ -77,8 +77,8 @@ class Net {
   bool has_external_input_info(const std::string& name) const { return workspace_->has_input_info(name); }
   std::vector<std::unique_ptr<OperatorBase>>& GetOperators() { return operators_; }
   Workspace* workspace() { return workspace_; }
-  // "profile" observer: per-operator host wall time of the last Run, as chrome-trace JSON
-  void set_profile(bool on) { profile_ = on; }
+  // "profile" observer: per-operator host wall time of the last Run, as chrome-trace JSON.  (A tower's layers run one by one then.)
+  void set_profile(bool on);
   std::string DumpProfile() const;
   const std::string& name() const { return name_; }
 
@@ -217,9 +217,14 @@ class ConcatAdopter {  // implemented by Gemm
   virtual OperatorBase* ReleaseConcat() = 0;
   // The narrow layer after such a layer (with the skinny layer it may already host) in the same launch
   // (bz_fc_desc.next): the attention MLP 4E -> 80 -> 40 -> 1 as one kernel.  `next` reads only this layer's result, and
-  // nothing else does.
+  // nothing else does.  Without an adopted Concat: a tower, layer -> layer -> skinny layer, in one launch at the numbers of rows
+  // where that is faster (bz::fc_tower_pays).
   virtual bool CanChainNext(OperatorBase* next) = 0;  // static part
-  virtual void AdoptNext(OperatorBase* next) = 0;
+  // true: the next layer is run by this one, in its launch or behind it, and no more by the net.  False for a tower's: the net
+  // runs it, which does nothing in a pass where this layer has computed it.
+  virtual bool AdoptNext(OperatorBase* next) = 0;
+  // no tower in one launch from now on: the operators are timed one by one, and a time has to be one layer's
+  virtual void RunApart(bool apart) = 0;
 };
 
 // Embedding blocks that are each one kAssign item [batch, T * D_i] -> Reshape [batch, T, D_i] (read by nothing else) ->

@@ -51,6 +51,14 @@ constexpr int kNumXcd = 8;      // MI355X: 8 accelerator complex dies, workgroup
 int fc_attention_f32(const bz_fc_desc& d, bz_stream_t stream);
 // whether it takes layers k -> n -> n2
 bool fc_attention_f32_takes(int64_t k, int64_t n, int64_t n2);
+// fc_tower.hip, for the host layer: an fp16 layer on a stored input, a second one (d.next) and a skinny third (the head) in one
+// launch, of whose outputs only the last is stored, once more at `copy` unless that is null.  d.w and d.next->w are weights that
+// fc_tower_pack laid out, fc_tower_weight_bytes each.  BZ_ENOTSUP, with nothing launched, for anything else.
+int fc_tower(const bz_fc_desc& d, void* copy, bz_stream_t stream);
+bool fc_tower_takes(int64_t k, int64_t n1, int64_t n2);  // whether it takes layers k -> n1 -> n2
+bool fc_tower_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2);  // whether that is faster than the first and the others in two
+size_t fc_tower_weight_bytes(int64_t k, int64_t n);
+int fc_tower_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream);  // from [k, n], or [n, k] when transposed
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);
