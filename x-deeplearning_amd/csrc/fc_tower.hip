@@ -7,7 +7,7 @@
 // the matrix cores' registers, laid out once in the order these take them (through LDS they would cross it twice), 128 KB a CU on their
 // way; the rows, which all eight waves read, are in LDS.
 // us alone / a launch on four streams, two launches and this: 1024 of 198 -> 200 -> 80 -> 2 11.7 / 5.5 and 7.5 / 3.0, 300 of 445 -> 256 -> 100
-// 10.9 / 5.2 and 9.2 / 3.0, 2048 of 896 -> 512 -> 256 16.4 / 6.5 and 14.9 / 4.5 (of these 14.9: rows to LDS 2.9, first layer 6.3, its
+// 10.9 / 5.2 and 8.4 / 3.2, 2048 of 896 -> 512 -> 256 16.4 / 6.5 and 14.9 / 4.5 (of these 14.9: rows to LDS 2.9, first layer 6.3, its
 // activation 1.1, second layer and activation 2.1, skinny layer 0.9).  fp16 model of 2048 x 26 lists on eight serving threads, us a pass:
 // 14.9 and 13.8.
 #include <mutex>
@@ -227,50 +227,66 @@ __device__ __forceinline__ void finish(const Epilogue& ep, const float* params, 
 }
 
 // The workgroup's rows of the input to LDS, inputs filled up with zeros to 64.  `meanwhile` runs when the first are asked for, `then`
-// when they are written.  V: bytes that every row can be read in.
-template <int V, typename F, typename G>
+// when they are written.  16-byte loads need addresses that are multiples of 4 only; ODD: rows may start 2 bytes behind one, and every
+// unit is put together from the 16 bytes before its start and the next 4 (300 x 445 -> 256 -> 100: 9.2 us with eight 2-byte loads a
+// unit, 8.4 this way).  Inputs that fill no unit come one by one, the last wave's lanes a row each.
+template <bool ODD, typename F, typename G>
 __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, const F& meanwhile, const G& then) {
-  constexpr int kPer = 16 / V, kAhead = V == 16 ? 8 : 4;
+  constexpr int kAhead = 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
-  const int here = min(a.m - m0, kRows), groups = up(a.k, 64) / 64;
-  const auto x = buffer_of(a.x + (int64_t)m0 * a.lda, (uint32_t)((here - 1) * (int)a.lda + a.k * 2));
+  const int here = min(a.m - m0, kRows), groups = up(a.k, 64) / 64, whole = a.k / 8, rest = a.k % 8;
+  const char* from = a.x + (int64_t)m0 * a.lda;
+  const int start = ODD ? (int)((uintptr_t)from & 2) : 0;
+  const auto x = buffer_of(from - start, (uint32_t)up(start + (here - 1) * (int)a.lda + a.k * 2, 4));
   // A wave has eight of the rows (lane % 8), every other 64 inputs (unit lane / 8): whole lines read, and 128 bytes a quarter wave
   // written
   const int r = wave % 4 * 8 + lane % 8, c0 = wave / 4 * 8 + lane / 8;
+  const bool last = rest != 0 && wave == kWaves - 1 && lane < kRows;
+  uint16_t tail[8];
   auto batch = [&](int g0, const F* meanwhile) {
     uint4 v[kAhead];
+    uint32_t next[kAhead];
+    const int base = start + r * (int)a.lda, odd = ODD ? base & 2 : 0;
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      const int in = (g0 * 8 + c0 + i * 16) * 8, off = r * (int)a.lda + in * 2;
-      uint32_t* w = (uint32_t*)&v[i];
-      if constexpr (V == 16) {
-        const auto u = __builtin_amdgcn_raw_buffer_load_b128(x, r < here && in < a.k ? off : kBeyond, 0, 0);
-        v[i] = *(const uint4*)&u;
-      } else if constexpr (V == 4) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) w[p] = __builtin_amdgcn_raw_buffer_load_b32(x, r < here && in + p * 2 < a.k ? off + p * 4 : kBeyond, 0, 0);
-      } else {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          const uint32_t lo = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x, r < here && in + p * 2 < a.k ? off + p * 4 : kBeyond, 0, 0);
-          const uint32_t hi = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x, r < here && in + p * 2 + 1 < a.k ? off + p * 4 + 2 : kBeyond, 0, 0);
-          w[p] = lo | hi << 16;
-        }
-      }
+      const int c = g0 * 8 + c0 + i * 16;
+      const int at = r < here && c < whole ? base - odd + c * 16 : kBeyond;
+      const auto u = __builtin_amdgcn_raw_buffer_load_b128(x, at, 0, 0);
+      v[i] = *(const uint4*)&u;
+      if constexpr (ODD) next[i] = __builtin_amdgcn_raw_buffer_load_b32(x, odd != 0 ? at : kBeyond, 16, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (meanwhile != nullptr) (*meanwhile)();
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i)
-      if (g0 + wave / 4 + i * 2 < groups) *(uint4*)(rows + ((g0 * 8 + c0 + i * 16) * kRows + r) * 16) = v[i];
+    for (int i = 0; i < kAhead; ++i) {
+      if constexpr (ODD) {
+        v[i].x = __builtin_amdgcn_alignbyte(v[i].y, v[i].x, odd);
+        v[i].y = __builtin_amdgcn_alignbyte(v[i].z, v[i].y, odd);
+        v[i].z = __builtin_amdgcn_alignbyte(v[i].w, v[i].z, odd);
+        v[i].w = __builtin_amdgcn_alignbyte(next[i], v[i].w, odd);
+      }
+      const int g = g0 + wave / 4 + i * 2, c = g0 * 8 + c0 + i * 16;
+      if (g < groups && (rest == 0 || c != whole)) *(uint4*)(rows + (c * kRows + r) * 16) = v[i];
+    }
   };
+  if (last) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      tail[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x, i < rest && lane < here ? start + lane * (int)a.lda + (whole * 8 + i) * 2 : kBeyond, 0, 0);
+  }
   batch(0, &meanwhile);
   then();
+  if (last) {
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = tail[2 * i] | (uint32_t)tail[2 * i + 1] << 16;
+    *(uint4*)(rows + (whole * kRows + lane) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
   for (int g = kAhead * 2; g < groups; g += kAhead * 2) batch(g, nullptr);
 }
 
-// TN: blocks of 32 columns a wave holds of the first layer.  HN: outputs the skinny layer's code is unrolled for.  V: stage_rows'.
-template <int TN, int HN, int V>
+// TN: blocks of 32 columns a wave holds of the first layer.  HN: outputs the skinny layer's code is unrolled for.  ODD: stage_rows'.
+template <int TN, int HN, bool ODD>
 __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a) {
   typedef __half T;
   extern __shared__ __align__(16) char lds[];
@@ -294,7 +310,7 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a)
     const int j = hj + i * (kThreads / kMaxNarrow);
     hw[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from_head, j < a.head.n && hc < a.n2 ? (j * (int)a.head.ldw + hc) * 2 : kBeyond, 0, 0);
   }
-  stage_rows<V>(
+  stage_rows<ODD>(
       a, m0, lds,
       [&]() {
         first.start(w1, wave);
@@ -353,7 +369,7 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a)
   }
 }
 
-template <int TN, int HN, int V>
+template <int TN, int HN, bool ODD>
 int launch(const Tower& a, int lds, hipStream_t st) {
   // more dynamic LDS than the default limit: raised once per kernel and device
   static std::mutex mu;
@@ -363,21 +379,18 @@ int launch(const Tower& a, int lds, hipStream_t st) {
   {
     std::lock_guard<std::mutex> lock(mu);
     if (dev >= 0 && dev < 64 && !raised[dev]) {
-      BZ_HIP_OK(hipFuncSetAttribute((const void*)bz_fc_tower_kernel<TN, HN, V>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+      BZ_HIP_OK(hipFuncSetAttribute((const void*)bz_fc_tower_kernel<TN, HN, ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
       raised[dev] = true;
     }
   }
-  hipLaunchKernelGGL((bz_fc_tower_kernel<TN, HN, V>), dim3((a.m + kRows - 1) / kRows), dim3(kThreads), lds, st, a);
+  hipLaunchKernelGGL((bz_fc_tower_kernel<TN, HN, ODD>), dim3((a.m + kRows - 1) / kRows), dim3(kThreads), lds, st, a);
   BZ_LAUNCH_OK("bz_fc_tower_kernel");
   return BZ_OK;
 }
 
 template <int TN, int HN>
 int with_rows(const Tower& a, int lds, hipStream_t st) {
-  const uintptr_t all = (uintptr_t)a.x | (uintptr_t)a.lda | (uintptr_t)(a.k * 2);
-  if (all % 16 == 0) return launch<TN, HN, 16>(a, lds, st);
-  if (all % 4 == 0) return launch<TN, HN, 4>(a, lds, st);
-  return launch<TN, HN, 2>(a, lds, st);
+  return (((uintptr_t)a.x | (uintptr_t)a.lda) & 3) != 0 ? launch<TN, HN, true>(a, lds, st) : launch<TN, HN, false>(a, lds, st);
 }
 
 }  // namespace
@@ -401,13 +414,14 @@ bool bz::fc_tower_takes(int64_t k, int64_t n1, int64_t n2) {
 // weights, so up to 512 KB it is the better at any number of rows that one round of workgroups takes: 300 of 64 -> 256 -> 104 (82)
 // 6.2 / 3.5 and 8.9 / 5.7, 1024 of 198 -> 200 -> 80 (108) 7.5 / 3.0 and 11.7 / 5.5, one of 200 -> 200 -> 80 6.4 / 3.0 and 8.4 / 5.5,
 // 300 of 896 -> 256 -> 104 (500) 9.8 / 3.8 and 10.4 / 6.9, but 640 -> 400 -> 128 (600) 12.0 / 3.8 and 11.7 / 6.8; with more, where the
-// rows fill the CUs of two launches: 1024, 2048 and 4096 of 896 -> 512 -> 256 (1152) 14.9 / 4.6 and 14.3 / 6.7, 14.9 / 4.5 and 16.4 / 6.5,
+// rows fill the CUs of two launches and from where on a model with it is as fast alone and faster on eight serving threads (1024
+// samples 113 / 10.4 us a pass with two, 115 / 10.4 with one, 1300 131.2 / 11.4 and 130.6 / 10.4): 1024, 2048 and 4096 of 896 -> 512 -> 256 (1152) 14.9 / 4.6 and 14.3 / 6.7, 14.9 / 4.5 and 16.4 / 6.5,
 // 15.0 / 8.0 and 18.7 / 10.7, but 2048 of 1280 -> 512 -> 256 (1536) 18.6 / 6.0 and 18.0 / 7.8.  Rows of more than 1280 inputs are
 // long to stage (300 of 1600 -> 64 -> 32 (204) 10.2 / 3.9 and 10.0 / 6.9), and beyond 4096 rows two launches leave more to others: 6000 of
 // 896 -> 400 -> 128 15.5 / 11.5 and 21.4 / 10.9, 16000 of 640 -> 64 -> 32 10.3 / 7.9 and 13.2 / 6.7.
 bool bz::fc_tower_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2) {
   const int64_t weights = k * n1 + n1 * n2;
-  return rows >= 1 && rows <= 4096 && ((k <= 1280 && weights <= 256 << 10) || (k <= 1024 && weights <= 576 << 10 && rows >= 1400));
+  return rows >= 1 && rows <= 4096 && ((k <= 1280 && weights <= 256 << 10) || (k <= 1024 && weights <= 576 << 10 && rows >= 1100));
 }
 
 int bz::fc_tower(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
