@@ -1313,8 +1313,8 @@ def test_feed_many_of_strided_inputs(pb, n_in):
             np.testing.assert_allclose(p.output_asnumpy("s"), _sigmoid(plain), rtol=1e-5)
 
 
-# bytes of the inputs, one behind the other on multiples of 256: parts end after 384, 960, 1824 KB and then every MB, from 4 MB on every
-# MB, unless less than half a part would be left
+# bytes of the inputs, one behind the other on multiples of 256: parts end after 384, 960, 1824 KB and then every MB, from 4 MB on there
+# are as many even ones as whole MB, unless less than half a part would be left
 @pytest.mark.parametrize("sizes", [[4, 393212], [393216, 196604], [393216, 196608], [393216, 196612], [393000, 300, 300000],   # in the padding; left over: half a part or less
                                    [393212, 4, 600000], [983040, 4, 430000], [300, 983040 - 512, 900000, 2 << 20], [(4 << 20) - 256, 4],
                                    [(4 << 20) - 512, 252], [5 << 20, 260], [(1 << 20) - 4, 4, 4 << 20]])

@@ -173,9 +173,9 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
 // A request is moved in parts, each launched as soon as it is staged.  Up to 4 MB the link is what bounds it (the kernel moves
 // 47 GB/s and leaves a gap behind each launch, staging runs at 58), so it starts early: 384 KB first, each part half as large
 // again as the one before until 1 MB.  Beyond, staging is (35 GB/s, the copies no longer fit the caches between requests), and a
-// launch costs the host 2.9 us: parts of 1 MB.  The last part takes what would be left of it below half a part.  us to the end of a
+// launch costs the host 2.9 us: even parts of 1 MB or more.  The last part takes what would be left of it below half a part.  us to the end of a
 // request among others, even parts of 1 MB or more / these: 0.74 MB 79.3 / 78.5, 1.07 92.8 / 88.5, 1.8 125 / 112, 2.5 115 / 112,
-// 3 135 / 127, 4 162 / 158, 4.6 180..191 / 184..194, 5.1 203 / 217.  (The copy engine moves 57 GB/s, but each copy costs 10 us until
+// 3 135 / 127, 4 162 / 158, 4.6 180..191 / 184..194 (not taken), 5.1 203 / 217 (not taken).  (The copy engine moves 57 GB/s, but each copy costs 10 us until
 // what follows it on the stream may start: 5 MB in ten parts arrived 230 us after the first byte was staged, in one part behind
 // the whole staging 210, through five launches of the kernel 162.)
 constexpr size_t kFeedFirst = 384 << 10, kFeedMost = 1 << 20, kFeedLong = 4 << 20;
@@ -287,7 +287,7 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
     // from the first launch on the arena is being read: whatever happens next, it is waited for before it is written again
     try {
       bz_feed_rows rows[BZ_FEED_MAX_ROWS];
-      size_t moved = 0, part = plain < kFeedLong ? kFeedFirst : kFeedMost;
+      size_t moved = 0, part = plain < kFeedLong ? kFeedFirst : (plain / (plain / kFeedMost) / 256 + 1) * 256;
       int n = 0;
       auto launch = [&](size_t upto) {
         BZ_CHECK(bz_feed(arena_host_ + moved, arena_dev_ + moved, (int64_t)(upto - moved), rows, n, st));
@@ -309,7 +309,7 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
           at += len;
           if (it.offset + at == end) {
             launch(end);
-            part = std::min(part + part / 2, kFeedMost);
+            if (plain < kFeedLong) part = std::min(part + part / 2, kFeedMost);
             end = end_of_part();
           }
         }
