@@ -214,6 +214,21 @@ def test_fc_fp32_error_of_a_layer_with_a_head(bz, M, N, K, parts):
     assert err <= _fp32_sum_error(K / parts), err
 
 
+# 32x64 tiles from 257 of 32x32 on (four waves, two sums each), 32x32 of eight waves for few columns and for few tiles
+@pytest.mark.parametrize("M,N,K", [(1024, 512, 896), (300, 1024, 2048), (700, 400, 2048), (700, 512, 400), (16384, 32, 1024), (9000, 20, 512), (500, 256, 1024)])
+def test_fc_fp32_error_of_eight_sums(bz, M, N, K):
+    """Eight sums an output, K / 8 inputs each in steps of sixteen, each step rounded once or a few times: an error that grows with the
+    root of K / 8, 0.26 * 2^-24 of it as measured here.  Half as many sums, the next lower number, would be 1.41 times that."""
+    import torch
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    y = bz.fc_fused(x, w, K)
+    want = x.double() @ w[:, :K].double().t().contiguous()
+    err = float((y.double() - want).norm() / want.norm())
+    assert err <= 0.26 * 2.0**-24 * (K / 8) ** 0.5 * 1.15, err
+
+
 # 2-byte layers of more than 256 tiles of 64x64: 64x128 and 128x64 tiles, also for rows that start on no 16 bytes
 @pytest.mark.parametrize("in_name,out_name", [("f16", "f16"), ("bf16", "f32")])
 @pytest.mark.parametrize("M,N,K,act,kw", [(1900, 520, 392, "dice", {}), (6017, 136, 64, "prelu", {"full_bias": True}),   # 64x128, ragged; one K tile

@@ -906,7 +906,7 @@ __device__ __forceinline__ float plain_dot(const float* a, const float* w, int K
 // whether a sum of split products may be off: it is not finite, or so small that the operands may lie where a split drops bits
 __device__ __forceinline__ bool doubtful(float v) { return !(v == 0.f || (fabsf(v) >= 0x1p-80f && fabsf(v) < __builtin_huge_valf())); }
 
-template <typename OutT, int NW, int TM, int TN>
+template <typename OutT, int NW, int TM, int TN, int SUMS>
 __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, OutT* __restrict__ Y, int M,
                                                             int N, int K, int64_t lda, int64_t ldw, int64_t ldy, int tiles_m,
                                                             Epilogue ep) {
@@ -970,13 +970,16 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
       cp2 = ep.p2[c];
     }
   }
-  floatx16 acc[TM][TN];
+  // (the sums that an output is added up in, stage by stage in turn)
+  floatx16 acc[SUMS][TM][TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int a = 0; a < SUMS; ++a)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][i][j][r] = 0.f;
 
   struct Pieces {
     Bf16x3 a[TM], w[TN];
@@ -1006,12 +1009,13 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
     for (int b = 0; b < TN; ++b) p.w[b] = split_floats(raw.w[b][0], raw.w[b][1]);
   };
   // the smallest products first
-  auto multiply = [&](const Pieces& p) {
+  auto multiply = [&](const Pieces& p, auto parity) {
+    constexpr int SUM = decltype(parity)::value % SUMS;
     auto each = [&](auto f) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) f(p.a[i], p.w[j], acc[i][j]);
+        for (int j = 0; j < TN; ++j) f(p.a[i], p.w[j], acc[SUM][i][j]);
     };
     each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.lo, y.hi, c); });
     each([](const Bf16x3& x, const Bf16x3& y, floatx16& c) { In<BZ_BF16>::mma(x.hi, y.lo, c); });
@@ -1032,11 +1036,11 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
     issue(i + 2);
   };
   // multiplies stage i, converts stage i + 1, reads stage i + 2
-  auto step = [&](const Pieces& now, Pieces& next, const Raw& raw, Raw& raw_next, int i) {
+  auto step = [&](const Pieces& now, Pieces& next, const Raw& raw, Raw& raw_next, int i, auto parity) {
     landed(i + 2);
     read(i + 2, raw_next);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(now);
+    multiply(now, parity);
     convert(raw, next);
     constexpr int MFMAS = 6 * TM * TN, VALU = 88 * (TM + TN) / 2, EACH = VALU / MFMAS;
 #pragma unroll
@@ -1057,16 +1061,18 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
     read(1, r1);
     convert(r0, p0);
     refill(1);
+    const std::integral_constant<int, 0> even;
+    const std::integral_constant<int, 1> odd;
     int i = 0;
     for (; i + 2 < n; i += 2) {
-      step(p0, p1, r1, r0, i);
-      step(p1, p0, r0, r1, i + 1);
+      step(p0, p1, r1, r0, i, even);
+      step(p1, p0, r0, r1, i + 1, odd);
     }
     if (i + 1 < n) {
-      step(p0, p1, r1, r0, i);
-      multiply(p1);
+      step(p0, p1, r1, r0, i, even);
+      multiply(p1, odd);
     } else {
-      multiply(p0);
+      multiply(p0, even);
     }
   }
   // A lane owns column lane & 31 of each block and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4: four rows of a column are a chunk.  Every
@@ -1079,13 +1085,21 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
   float v[EACH][4];
   auto add_up = [&]() {
 #pragma unroll
+    for (int a = 1; a < SUMS; ++a)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[0][i][j][r] += acc[a][i][j][r];
+#pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *(float4*)(&lds[wave][0][0] + chunk_at(j * 32 + frow, i * 8 + q * 2 + fhalf)) =
-              make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+              make_float4(acc[0][i][j][4 * q], acc[0][i][j][4 * q + 1], acc[0][i][j][4 * q + 2], acc[0][i][j][4 * q + 3]);
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < EACH; ++e)
@@ -1385,10 +1399,10 @@ int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 }
 
 
-template <typename OutT, int NW, int TM, int TN>
+template <typename OutT, int NW, int TM, int TN, int SUMS>
 int launch_f32(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 32 * TM - 1) / (32 * TM), tiles_n = (d.n + 32 * TN - 1) / (32 * TN);
-  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
+  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN, SUMS>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
                      d.ldw, d.ldy, tiles_m, ep);
   BZ_LAUNCH_OK("bz_fc_f32_kernel");
   return BZ_OK;
@@ -1558,14 +1572,19 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
     // The fp32 tiles / 32x64: 50000 x 80 -> 80 20.8 / 14.4 and 22.0 / 17.1, 20000 x 80 -> 512 37.3 / 24.2 and 32.3 / 27.2,
     // 50000 x 100 -> 200 68 / 47 and 43 / 38, 20000 x 128 -> 512 53 / 38 and 36 / 33.
     // Before, the split kernel below and those tiles: 300 x 445 -> 256 6.8 / 4.0 and now 4.9 / 3.1, 32 x 2075 -> 768 14.8 / 6.0 and
-    // 10.2 / 4.0, 1024 x 896 -> 512 13.7 / 10.8 and 11.1 / 7.3, 2048 x 896 -> 512 19.6 / 15.9 and 14.9 / 12.1, 8192 rows 65 / 62 and 49 / 49,
+    // 10.2 / 4.0, 1024 x 896 -> 512 13.7 / 10.8 and 11.9 / 8.2, 2048 x 896 -> 512 19.6 / 15.9 and 14.9 / 12.1, 8192 rows 65 / 62 and 49 / 49,
     // 16384 x 301 -> 512 55 / 52 and 43 / 42, 5000 x 3000 -> 1024 380 / 250 and 213 / 220.  Errors against 64 bits, in the
-    // same order: 1.5e-7 and 1.2e-7, 2.9e-7 and 2.5e-7, 2.0e-7 and 2.3e-7, 2.7e-7 and 2.3e-7, 5.4e-7 and 2.3e-7, 1.6e-7 and 1.3e-7, 9.7e-7 and 4.2e-7.
+    // same order: 1.5e-7 and 1.2e-7, 2.9e-7 and 2.5e-7, 2.0e-7 and 1.6e-7, 2.7e-7 and 2.3e-7, 5.4e-7 and 2.3e-7, 1.6e-7 and 1.3e-7, 9.7e-7 and 4.2e-7.
+    // They grow with what one sum takes in, K over the waves, so beyond 256 inputs the 32x64 tiles, four waves where the split kernel has
+    // eight, add every output up in two sums, stage by stage in turn (1024 x 896 -> 512 with one 11.1 / 7.4 and 2.3e-7, 1024 x 4096 -> 512 35.9 / 33
+    // and 5.0e-7, with two 38.3 / 32 and 3.5e-7, before 49.8 / 45 and 4.1e-7), and up to 32 columns eight waves stay with
+    // 32x32 (12000 x 512 -> 20 9.9 / 6.0, 64x64 11.1 / 6.0, now 8.7 / 5.3; 16384 x 1024 -> 32 17.3 / 13.1, 16.9 / 13.7 and 15.9 / 11.7).
     const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
     if (f32_rows_fit(d.lda, d.k) && f32_rows_fit(d.ldw, d.k) && (d.k > 96 || wg64 <= 128 || wg32 <= 512)) {
-      if (wg32 <= 256 || (wg32 <= 512 && d.k <= 256)) return launch_f32<OutT, 8, 1, 1>(d, ep, st);
-      if (wg64 <= 128 || d.k < 200) return launch_f32<OutT, 4, 1, 2>(d, ep, st);
-      return launch_f32<OutT, 4, 2, 2>(d, ep, st);
+      if (wg32 <= 256 || (wg32 <= 512 && (d.k <= 256 || d.n <= 32))) return launch_f32<OutT, 8, 1, 1, 1>(d, ep, st);
+      if (wg64 <= 128) return launch_f32<OutT, 4, 1, 2, 2>(d, ep, st);
+      if (d.k < 200) return launch_f32<OutT, 4, 1, 2, 1>(d, ep, st);
+      return launch_f32<OutT, 4, 2, 2, 1>(d, ep, st);
     }
   }
   if (d.k < In<DT>::kChunk || (In<DT>::kSize == 2 && wg32 <= (aligned || d.k > 256 ? 256 : 192))) return launch_split<DT, OutT, 8>(d, ep, st);
