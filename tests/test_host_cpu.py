@@ -48,6 +48,21 @@ def test_struct_layouts_match_header():
                      C.sizeof(blaze_hip.ConcatEwDesc), C.sizeof(blaze_hip.WeightedPoolDesc), C.sizeof(blaze_hip.FcNext)]
 
 
+def test_scalar_writes_of_m0_in_inline_assembly_are_a_wait_state_ahead_of_loads_to_lds():
+    """A load whose target is LDS reads M0, which needs a wait state behind a scalar write (s_nop 0); the compiler keeps that
+    between its own instructions and does not look into an asm's text."""
+    import glob
+    seen = 0
+    for path in glob.glob(os.path.join(ROOT, "x-deeplearning_amd", "csrc", "**", "*.h*"), recursive=True):
+        for text in re.findall(r'asm(?:\s+volatile)?\s*\(((?:\s*"(?:[^"\\]|\\.)*")+)', open(path).read()):
+            lines = [x.strip() for x in "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', text)).replace("\\t", "").split("\\n")]
+            for at, line in enumerate(lines):
+                if re.match(r"s_\w+ m0\b", line):
+                    seen += 1
+                    assert lines[at + 1].startswith("s_nop"), (path, lines)
+    assert seen >= 2
+
+
 def _sample_net():
     import pyblaze_hip as pb
     nb = pb.NetBuilder("ctr", device_type=1)

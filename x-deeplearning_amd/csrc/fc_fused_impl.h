@@ -518,9 +518,10 @@ constexpr int kStreamCompute = 256;                                       // thr
 
 typedef __attribute__((address_space(3))) char lds_char;
 
-// 16 bytes per lane from global memory to LDS at lds_addr + 16 * lane (lds_addr is the same in all lanes)
+// 16 bytes per lane from global memory to LDS at lds_addr + 16 * lane (lds_addr is the same in all lanes).  A scalar write of M0
+// needs a wait state before a load to LDS reads it; the compiler puts one between its own instructions, in an asm's text nobody does.
 __device__ __forceinline__ void load_to_lds(const char* g, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr) : "memory", "m0");
 }
 
 // one phase = 6 fragment reads for the phase after next and 8 MFMAs on fragments read a phase ago
@@ -885,7 +886,7 @@ inline bool f32_rows_fit(int64_t ld, int k) { return k >= 4 && (64 * ld + k) * 4
 // above 0.  (The branch stands in the assembler: one that the compiler sees ends the block in which it may alternate products
 // and conversions.)
 __device__ __forceinline__ void load_to_lds_from(const char* base, uint32_t off, uint32_t lds_addr, int left) {
-  asm volatile("s_cmp_lt_i32 %3, 1\n\ts_cbranch_scc1 .Lnone%=\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1\n.Lnone%=:" ::"v"(off),
+  asm volatile("s_cmp_lt_i32 %3, 1\n\ts_cbranch_scc1 .Lnone%=\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n.Lnone%=:" ::"v"(off),
                "s"(base), "s"(lds_addr), "s"(left)
                : "memory", "m0", "scc");
 }
