@@ -80,7 +80,8 @@ BLAZE_API int Blaze_PredictorListOutputNames(PredictorHandle handle, size_t* ndi
 
 /* c_api_predictor.h:101-107 -- observer "profile": per-operator host wall time as chrome-trace JSON.  A dump also holds
  * "outputs", JSON: for every output of the net where Output would find it now: in "device" memory, "copied" to the host by a
- * launch behind the last Forward's, or put there by the launch of the "operator" that computed it */
+ * launch behind the last Forward's, or put there by the launch of the "operator" that computed it; and "pass": whether the last
+ * Forward's stream has been waited for ("ended") or its outputs alone ("arrived") */
 BLAZE_API int Blaze_PredictorRegisterObservers(PredictorHandle handle, size_t ndim, const char** names);
 BLAZE_API int Blaze_PredictorDumpObservers(PredictorHandle handle, size_t* ndim, const char*** key, const char*** value);
 

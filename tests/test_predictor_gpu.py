@@ -965,6 +965,83 @@ def test_outputs_with_every_bit_set_arrive_too(pb, dtype):
         assert np.array_equal(got.view(bits), np.concatenate([a.view(bits), b.view(bits)], 1)), step
 
 
+def _in_another_thread(f):
+    import threading
+    result = []
+    t = threading.Thread(target=lambda: result.append(f()))
+    t.start()
+    t.join()
+    return result[0]
+
+
+@pytest.mark.parametrize("what", ["feed", "feed_many", "launch", "device address"])
+def test_another_threads_work_waits_for_a_pass_that_ended_by_its_outputs(pb, what):
+    """A pass may end when its outputs are on the host, the end of its last launch still running on this thread's stream.  What
+    another thread queues, on a stream of its own, comes behind that."""
+    nb = pb.NetBuilder("arrived", device_type=1)
+    nb.external_input("x", pb.K_FLOAT)
+    nb.op("Sigmoid", ["x"], ["y"])
+    nb.external_output("y", pb.K_FLOAT)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    x = np.random.default_rng(2).standard_normal((4, 16)).astype(np.float32)
+    do = {"feed": lambda: p.feed("x", x), "feed_many": lambda: p.feed_many(p.feed_batch([("x", x)])), "launch": p.forward_launch,
+          "device address": lambda: p.output_device_ptr("y")}[what]
+
+    def state():
+        return p.dump_observers()["pass"]
+
+    def there():
+        do()
+        now = state()
+        if what == "launch":
+            p.forward_wait()
+        return now
+
+    seen = 0
+    for _ in range(16):
+        p.feed("x", x)
+        p.forward()
+        np.testing.assert_allclose(p.output_asnumpy("y").reshape(4, 16), _sigmoid(x), rtol=1e-5)
+        if state() != "arrived":  # (the first pass, and one in which this thread was interrupted)
+            continue
+        seen += 1
+        p.feed("x", x)
+        assert state() == "arrived"  # (the same stream)
+        assert _in_another_thread(there) == "ended"
+        p.forward()
+        np.testing.assert_allclose(p.output_asnumpy("y").reshape(4, 16), _sigmoid(x), rtol=1e-5)
+        if what == "device address":
+            assert state() == "ended"
+            break
+    assert seen > 0
+
+
+@pytest.mark.parametrize("declared", [("y", ), ("y", "z")])
+def test_a_pass_ends_by_its_outputs_only_where_every_operator_feeds_one(pb, declared):
+    """Operators behind the last output, which nothing shows the end of: such a net's stream is waited for."""
+    nb = pb.NetBuilder("tail", device_type=1)
+    nb.external_input("x", pb.K_FLOAT)
+    nb.op("Sigmoid", ["x"], ["y"])
+    nb.op("Sigmoid", ["x"], ["t"])
+    nb.op("Sigmoid", ["t"], ["z"])
+    for o in declared:
+        nb.external_output(o, pb.K_FLOAT)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    x = np.random.default_rng(2).standard_normal((4, 16)).astype(np.float32)
+    states = set()
+    for _ in range(8):
+        p.feed("x", x)
+        p.forward()
+        states.add(p.dump_observers()["pass"])
+        for o in declared:
+            p.output_asnumpy(o)
+    assert ("arrived" in states) == (len(declared) == 2), states
+
+
 def test_feed_forward_and_output_in_threads_of_their_own(pb):
     """Inputs fed by one thread, the pass run by another, the output read by a third, each of them new or the same as last time,
     fed twice before a pass, read twice behind it, and through the device address: always the pass's own."""

@@ -36,6 +36,7 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
     }
     output_sole_.push_back(writers == 1 && readers == 0);
   }
+  await_outputs_ = EveryOperatorFeedsAnOutput();
   for (const auto& name : net_->external_input()) {
     Blob* b = net_->external_input_blob(name);
     BLAZE_CONDITION_THROW(b != nullptr, "external_input: ", name, " is not in external_input_blob");
@@ -144,6 +145,7 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
         blob->DropArenaView();
         blob->Reshape(shape);
       }
+      SettleBefore(ctx);
       // stage in pinned memory and queue the transfer; a second Feed of the same input first waits for the first
       if (feed_done_ == nullptr) HIP_CHECK(hipEventCreateWithFlags(&feed_done_, hipEventDisableTiming));
       if (feed_pending_[idx]) FinishFeeds();
@@ -206,20 +208,22 @@ void Predictor::FinishFeeds() {
   any_feed_pending_ = false;
 }
 
-// what this thread launches from here on runs behind the queued transfers
+// what this thread launches from here on runs behind the queued transfers, and behind the last pass
 void Predictor::OrderBehindFeeds() {
-  for (Blob* b : external_input_blob_) {
-    if (b->device_type() != kHIP) continue;
-    HIPContext ctx(b->device_option());
-    ctx.Activate();
-    forward_on_ = ctx.stream_serial();
-    if (!any_feed_pending_ || forward_on_ == feed_on_) return;
-    if (feed_recorded_)
-      HIP_CHECK(hipStreamWaitEvent(ctx.hip_stream(), feed_done_, 0));
-    else
-      HIP_CHECK(hipDeviceSynchronize());
-    return;
-  }
+  for (const auto* list : {&external_input_blob_, &external_output_blob_})
+    for (Blob* b : *list) {
+      if (b->device_type() != kHIP) continue;
+      HIPContext ctx(b->device_option());
+      ctx.Activate();
+      SettleBefore(ctx);
+      forward_on_ = ctx.stream_serial();
+      if (!any_feed_pending_ || forward_on_ == feed_on_) return;
+      if (feed_recorded_)
+        HIP_CHECK(hipStreamWaitEvent(ctx.hip_stream(), feed_done_, 0));
+      else
+        HIP_CHECK(hipDeviceSynchronize());
+      return;
+    }
 }
 
 bool Predictor::FeedMany(int count, const char* const* names, const void* const* data, const size_t* lens) {
@@ -270,6 +274,7 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
     }
     HIPContext ctx(*dev);
     ctx.Activate();
+    SettleBefore(ctx);
     hipStream_t st = ctx.hip_stream();
     if (feed_done_ == nullptr) HIP_CHECK(hipEventCreateWithFlags(&feed_done_, hipEventDisableTiming));
     if (any_feed_pending_) FinishFeeds();  // the staging arena may still be read by the previous transfer
@@ -498,8 +503,10 @@ bool Predictor::Awaitable(size_t i) const {
 
 // Whether the pass has ended, as far as anybody but a stream can tell: every output is on its way to the host by itself, and
 // all of it has arrived.  The stream behind it need not be waited for, which is a packet on the queue and the runtime's own
-// turn: 4.6 us of a chain of four small launches of 19.1.  What runs on the device still is the end of the last launch: what is
-// queued on this stream is behind it, who goes round the stream waits first (Settle).  Every 32nd pass waits for the stream, so
+// turn: 4.6 us of a chain of four small launches of 19.1.  What runs on the device still is the end of the launches whose results
+// have arrived, since every operator's reach an output (EveryOperatorFeedsAnOutput).  What this thread queues is behind that on the
+// stream; who goes round the stream waits first: a feed or a pass on another one (SettleBefore), a device address, a copy by Output,
+// the destructor (Settle); and memory that is freed waits for the device by itself.  Every 32nd pass waits for the stream, so
 // that the runtime can put away what it keeps for each launch (left alone it does so every thousand or so, in 5 ms).
 // us a request, with the event that is no longer recorded behind the transfer: one sample fp32 35.5 -> 32.0, 300 samples fp16
 // 50.7 -> 45.2, attention models of 201 and 1024 59.2 -> 52.7 and 101.6 -> 93.7, 2048 samples 230 -> 209.
@@ -532,6 +539,25 @@ bool Predictor::PassIsThere() {
   }
   std::atomic_thread_fence(std::memory_order_acquire);
   return true;
+}
+
+// Whether each operator's results reach an output: only then is a pass whose outputs have arrived done with all its memory.
+bool Predictor::EveryOperatorFeedsAnOutput() const {
+  std::vector<Blob*> needed = external_output_blob_;
+  const auto& ops = net_->GetOperators();
+  for (auto it = ops.rbegin(); it != ops.rend(); ++it) {
+    if ((*it)->type() == "ConstantFill") continue;  // (the net's, or nobody's any more where operators were folded)
+    const auto& out = (*it)->Outputs();
+    const bool used = std::any_of(out.begin(), out.end(), [&](Blob* b) { return std::find(needed.begin(), needed.end(), b) != needed.end(); });
+    if (!used) return false;
+    needed.insert(needed.end(), (*it)->Inputs().begin(), (*it)->Inputs().end());
+  }
+  return true;
+}
+
+// what is queued on ctx's stream from here on runs behind the last pass
+void Predictor::SettleBefore(const HIPContext& ctx) {
+  if (!settled_ && ctx.stream_serial() != forward_on_) Settle();
 }
 
 // the last pass has ended on the device as well
@@ -708,6 +734,7 @@ void Predictor::DumpObservers(std::unordered_map<std::string, std::string>* dump
     ss << (i ? "," : "") << "\"" << net_->external_output()[i] << "\":\"" << (!output_ahead_[i] ? "device" : output_by_operator_[i] ? "operator" : "copied") << "\"";
   ss << "}";
   (*dump_map)["outputs"] = ss.str();
+  (*dump_map)["pass"] = settled_ ? "ended" : "arrived";
 }
 
 void* Predictor::InputDevicePtr(const char* name) {

@@ -122,11 +122,13 @@ class Predictor {
     size_t elements, size;
   };
   std::vector<Awaited> awaited_;
-  bool await_outputs_ = true;  // false once an output had the value that stands for "not there yet"
+  bool await_outputs_ = true;  // false once an output had the value that stands for "not there yet", and where outputs do not tell
   bool settled_ = true;        // the last pass's stream has been waited for
   int passes_unsettled_ = 0;
+  bool EveryOperatorFeedsAnOutput() const;
   bool PassIsThere();
   void Settle();
+  void SettleBefore(const HIPContext& ctx);
   char* arena_host_ = nullptr;         // FeedMany's pinned staging arena and its device twin
   char* arena_dev_ = nullptr;
   size_t arena_cap_ = 0;

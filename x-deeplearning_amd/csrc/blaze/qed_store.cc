@@ -524,7 +524,7 @@ Status QedHipSparsePuller::GetOnStream(const std::vector<SparsePullerInput>& inp
       slots.push_back(s);
     }
   }
-  // (the previous call's tables are let go only now: its launch has been waited for before this predictor runs again)
+  // (the previous call's tables are let go only now: what it launched has run, or freeing waits for it)
   sc->tables.swap(held);
   if (slots.empty()) return kOK;
   BZ_CHECK(bz_embed_plan(slots.data(), (int)slots.size(), &sc->launch));
@@ -534,7 +534,7 @@ Status QedHipSparsePuller::GetOnStream(const std::vector<SparsePullerInput>& inp
     size_t need = 0;
     for (const auto& s : slots) need += (size_t)s.batch + 1;
     if (sc->offsets_cap < need) {
-      if (sc->offsets) HIP_CHECK(hipFree(sc->offsets));  // (its last reader finished: a predictor is waited for before its next pass)
+      if (sc->offsets) HIP_CHECK(hipFree(sc->offsets));  // (waits for its last reader, if that still runs)
       ++AllocationCount();
       HIP_CHECK(hipMalloc((void**)&sc->offsets, need * sizeof(int64_t)));
       sc->offsets_cap = need;
@@ -555,7 +555,8 @@ Status QedHipSparsePuller::GetOnStream(const std::vector<SparsePullerInput>& inp
   const bool changed = sc->host.size() != slots.size() || memcmp(sc->host.data(), slots.data(), bytes) != 0;
   if (changed) {
     if (sc->cap < slots.size()) {
-      // the previous launch that read the old buffers has completed: the net waits for its stream after every run
+      // (freeing waits for the launch that read them.  The pinned one may be written again all the same: the transfer from it came
+      // before results that the last pass has waited for)
       if (sc->pinned) HIP_CHECK(hipHostFree(sc->pinned));
       if (sc->dev) HIP_CHECK(hipFree(sc->dev));
       sc->cap = slots.size();
