@@ -63,6 +63,20 @@ def test_scalar_writes_of_m0_in_inline_assembly_are_a_wait_state_ahead_of_loads_
     assert seen >= 2
 
 
+def test_the_host_layer_waits_for_a_device_that_it_has_made_current():
+    """hipDeviceSynchronize waits for the calling thread's current device, which need not be the predictor's (its destructor may
+    run on any thread): it stands only behind a hipSetDevice in the same function."""
+    import glob
+    seen = 0
+    for path in glob.glob(os.path.join(ROOT, "x-deeplearning_amd", "csrc", "blaze", "*.*")):
+        for body in re.split(r"\n}\n", open(path).read()):  # (a function ends in the first column)
+            at = body.find("hipDeviceSynchronize(")
+            if at >= 0:
+                seen += 1
+                assert "hipSetDevice(" in body[:at], (path, body[max(0, at - 300):at + 40])
+    assert seen >= 1
+
+
 def _sample_net():
     import pyblaze_hip as pb
     nb = pb.NetBuilder("ctr", device_type=1)

@@ -52,12 +52,8 @@ Predictor::Predictor(std::shared_ptr<Net> net) : net_(net) {
 Predictor::~Predictor() {
   // Wait only for work that is still queued: an event that was already waited for may belong to a stream that died with
   // its serving thread.  Nothing here may leave an error behind for the caller's next runtime call.
-  if (any_feed_pending_) {
-    if (feed_recorded_)
-      (void)hipEventSynchronize(feed_done_);
-    else
-      (void)hipDeviceSynchronize();
-  }
+  if (any_feed_pending_ && feed_recorded_) (void)hipEventSynchronize(feed_done_);
+  if ((any_feed_pending_ && !feed_recorded_) || !settled_) (void)WaitForDevice();
   if (forward_done_ && forward_in_flight_) (void)hipEventSynchronize(forward_done_);
   if (arena_host_) (void)hipHostFree(arena_host_);
   if (arena_dev_) (void)hipFree(arena_dev_);
@@ -65,6 +61,17 @@ Predictor::~Predictor() {
   if (forward_done_) (void)hipEventDestroy(forward_done_);
   if (feed_done_) (void)hipEventDestroy(feed_done_);
   (void)hipGetLastError();
+}
+
+// All streams of this predictor's device have been waited for, whatever device the calling thread is on.
+hipError_t Predictor::WaitForDevice() const {
+  int before = 0;
+  hipError_t rc = hipGetDevice(&before);
+  const int mine = device_id();
+  if (rc == hipSuccess && mine >= 0) rc = hipSetDevice(mine);
+  if (rc == hipSuccess) rc = hipDeviceSynchronize();
+  if (mine >= 0 && mine != before) (void)hipSetDevice(before);
+  return rc;
 }
 
 int Predictor::InputName2Idx(const char* name) const {
@@ -200,7 +207,7 @@ void Predictor::FinishFeeds() {
       if (b->device_type() != kHIP) continue;
       HIPContext ctx(b->device_option());
       ctx.Activate();
-      HIP_CHECK(ctx.stream_serial() == feed_on_ ? hipStreamSynchronize(ctx.hip_stream()) : hipDeviceSynchronize());
+      HIP_CHECK(ctx.stream_serial() == feed_on_ ? hipStreamSynchronize(ctx.hip_stream()) : WaitForDevice());
       break;
     }
   }
@@ -221,7 +228,7 @@ void Predictor::OrderBehindFeeds() {
       if (feed_recorded_)
         HIP_CHECK(hipStreamWaitEvent(ctx.hip_stream(), feed_done_, 0));
       else
-        HIP_CHECK(hipDeviceSynchronize());
+        HIP_CHECK(WaitForDevice());
       return;
     }
 }
@@ -567,7 +574,7 @@ void Predictor::Settle() {
     if (b->device_type() != kHIP) continue;
     HIPContext ctx(b->device_option());
     ctx.Activate();
-    HIP_CHECK(ctx.stream_serial() == forward_on_ ? hipStreamSynchronize(ctx.hip_stream()) : hipDeviceSynchronize());
+    HIP_CHECK(ctx.stream_serial() == forward_on_ ? hipStreamSynchronize(ctx.hip_stream()) : WaitForDevice());
     break;
   }
   settled_ = true;

@@ -128,6 +128,7 @@ class Predictor {
   bool EveryOperatorFeedsAnOutput() const;
   bool PassIsThere();
   void Settle();
+  hipError_t WaitForDevice() const;
   void SettleBefore(const HIPContext& ctx);
   char* arena_host_ = nullptr;         // FeedMany's pinned staging arena and its device twin
   char* arena_dev_ = nullptr;
