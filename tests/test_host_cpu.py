@@ -634,6 +634,38 @@ def test_file_parsers_under_address_and_undefined_behaviour_sanitizers(tmp_path,
     assert r.returncode == 0 and "sanitize_host_parsers: done" in r.stdout, (r.returncode, r.stderr[-3000:])
 
 
+def test_an_output_prepares_only_its_own_bytes_of_the_hosts_copy(tmp_path):
+    """The host's copy has room for the largest output so far; a pass that writes a few bytes there sets those few and no more."""
+    import shutil
+    import subprocess
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src = tmp_path / "host_copy.cc"
+    src.write_text(r"""
+#include "blaze/runtime.h"
+int main() {
+  unsigned char at[64] = {0};
+  blaze::Blob::HostCopy c;
+  c.at = at;
+  c.room = sizeof(at);
+  if (c.Take(0) != nullptr || c.Take(65) != nullptr || c.Take(64) != at) return 1;
+  for (int i = 0; i < 64; ++i)
+    if (at[i] != 0) return 2;
+  c.fill = 0xff;
+  if (c.Take(0) != nullptr || c.Take(65) != nullptr || c.Take(8) != at) return 3;
+  for (int i = 0; i < 64; ++i)
+    if (at[i] != (i < 8 ? 0xff : 0)) return 4;
+  return 0;
+}
+""")
+    exe = str(tmp_path / "host_copy")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
+    assert subprocess.run([exe]).returncode == 0
+    predictor = open(os.path.join(ROOT, "x-deeplearning_amd", "csrc", "blaze", "predictor.cc")).read()
+    assert re.findall(r"memset\(([^;]*)\);", predictor) == ["rows[n].dst, kNotThereByte, bytes"]  # (an output copied behind the launches)
+
+
 def test_a_descriptor_without_a_head_hands_the_kernels_none(tmp_path):
     """head_n of 0 (or below) means no head whatever the other head_* fields hold: a kernel asks for the bias of the head it is given
     before it looks at the number of outputs, so a bias handed on would be read in front of its beginning."""

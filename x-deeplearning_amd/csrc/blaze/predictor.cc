@@ -499,7 +499,7 @@ void Predictor::OfferHostCopies() {
     c.copied = 0;
     c.room = std::min(HostHalf(i), kCopiedAheadMax);
     c.at = (char*)output_cpu_[i]->data() + (1 - output_half_[i]) * HostHalf(i);
-    if (Awaitable(i)) memset(c.at, kNotThereByte, c.room);
+    c.fill = Awaitable(i) ? kNotThereByte : -1;
   }
 }
 

@@ -7,6 +7,8 @@
 // synchronisation inside operators.
 #pragma once
 
+#include <string.h>
+
 #include <atomic>
 #include <memory>
 #include <vector>
@@ -65,11 +67,17 @@ class Blob {
     dims_ = dims;
   }
   // Memory on the host that takes a copy of the data as well: offered for one pass by the predictor whose output this is,
-  // taken by an operator that writes the whole output in its launch.  `copied`: the bytes that were.
+  // taken by an operator that writes the whole output in its launch.  `copied`: the bytes that were.  `fill`: what every byte is
+  // set to before the launch, -1: as it is.
   struct HostCopy {
     void* at = nullptr;
     size_t room = 0, copied = 0;
-    void* Take(size_t bytes) const { return bytes > 0 && bytes <= room ? at : nullptr; }
+    int fill = -1;
+    void* Take(size_t bytes) const {
+      if (bytes == 0 || bytes > room) return nullptr;
+      if (fill >= 0) memset(at, fill, bytes);
+      return at;
+    }
   };
   HostCopy& host_copy() { return host_copy_; }
   // the shape alone, for the output of an operator whose work its consumer has taken over: readers may ask the shape,
