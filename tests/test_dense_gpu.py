@@ -297,6 +297,43 @@ def test_fc_fp32_infinities_and_numbers_at_the_ends_of_the_range(bz, M, N, K):
     assert (y[5:7] == 0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (1200, 400, 160), (1200, 800, 250), (1024, 512, 300), (3, 9, 1000)])
+def test_fc_fp32_small_numbers_times_large_ones(bz, M, N, K):
+    """Operands whose last bits no three bf16s hold, or none at all, times such of the other side that the sums are ordinary numbers, or
+    small ones that are not 0; whole rows and columns of them, and single ones among zeros.  Ordinary rows beside them, and rows of
+    zeros, come out as without."""
+    import torch
+    torch.manual_seed(K)
+    small = torch.tensor([1.0, 1.2e-38, 1e-40, 1e-41, 1.2e-37, 3.3e-36, 1e-33, 1e14, 1e15], device="cuda", dtype=torch.float64)
+    large = torch.tensor([1.0, 1e3, 1e15, 1e18, 1e20, 1e10, 1e-39, 1e-36, 2e-38], device="cuda", dtype=torch.float64)
+    plain = torch.randn(M, K, device="cuda")
+    x = (plain.double() * small[torch.arange(M, device="cuda") % 9, None]).float()
+    w = torch.zeros(N, (K + 3) // 4 * 4, device="cuda")
+    w[:, :K] = (torch.randn(N, K, device="cuda").double() * large[torch.arange(N, device="cuda") % 9, None]).float()
+    if M > 16:
+        x[9] = 0.0
+        x[9, 3] = 3e-39
+        x[10] = 0.0
+        w[11] = 0.0
+        w[11, 3] = 1e10
+        w[12] = 0.0
+    bias = torch.zeros(N, device="cuda")
+    print("case M=%d N=%d K=%d" % (M, N, K), flush=True)
+    y = bz.fc_fused(x, w, K, bias=bias)
+    want = x.double() @ w[:, :K].double().t().contiguous()
+    bound = _plain_bound(x, w[:, :K], bias) + K * 2.0**-149  # (below 2^-126 numbers are whole multiples of 2^-149)
+    assert (want.abs() < 1e38).all() and (want.abs() > 0).sum() > M * N // 2
+    off = (y.double() - want).abs() - bound
+    assert (off <= 0).all(), (float((off / bound).max()), int(off.argmax()) // N % 9, int(off.argmax()) % N % 9)
+    if M > 16:
+        assert (y[10] == 0).all() and (y[:, 12] == 0).all()
+        # (rows 0, 9, 18 .. and 7, 16 .. beside others of ordinary numbers)
+        ordinary = [r for r in range(M) if r % 9 in (0, 7) and r != 9]
+        x1 = plain.clone()
+        x1[ordinary] = x[ordinary]
+        assert torch.equal(bz.fc_fused(x1, w, K, bias=bias)[ordinary], y[ordinary])
+
+
 @pytest.mark.parametrize("M,K,N,H,act", [(1, 1024, 48, 1, "none"), (17, 516, 100, 8, "softmax"), (300, 256, 196, 2, "softmax"), (2049, 512, 256, 2, "none"),
                                          (300, 256, 192, 3, "sigmoid"), (2000, 200, 256, 2, "softmax")])
 def test_fc_fp32_head_apart_and_in_the_launch(bz, M, K, N, H, act):

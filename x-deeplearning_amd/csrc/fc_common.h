@@ -207,11 +207,12 @@ struct In<BZ_F32> {
 };
 
 // A float as the sum of three bf16s: each the nearest to what the ones before leave over, 8 significant bits and a sign a
-// piece, so that nothing is left over (|x| from 2^-110 up; below, what is left over is at most 2^-134).  A product of two
+// piece, so that nothing is left over (|x| from 2^-110 up; below, what is left over is at most 2^-134, and 2^-126 where the matrix
+// instructions take a piece that small for zero: whoever uses this looks for sums that may be of such products).  A product of two
 // such sums, without the three of its nine products that are below 2^-25 of it, comes from the bf16 matrix instructions: six of
 // them multiply 32x32x16 in 192 clocks, the fp32 ones in 512.
 // A float that is no bf16 to be rounded to, an infinity or one within 2^-9 of it, makes infinite or undefined pieces, which
-// make infinite or undefined sums: whoever uses this looks at the sums and computes such ones with fp32 instructions.
+// make infinite or undefined sums: whoever uses this looks for them, too, and computes them with fp32 instructions.
 struct Bf16x3 {
   uint4 hi, mid, lo;  // eight floats: element i in half i % 2 of word i / 2
 };

@@ -904,8 +904,21 @@ __device__ __forceinline__ float plain_dot(const float* a, const float* w, int K
   for (; k < K; ++k) s0 = fmaf(a[k], w[k], s0);
   return (s0 + s1) + (s2 + s3);
 }
-// whether a sum of split products may be off: it is not finite, or so small that the operands may lie where a split drops bits
-__device__ __forceinline__ bool doubtful(float v) { return !(v == 0.f || (fabsf(v) >= 0x1p-80f && fabsf(v) < __builtin_huge_valf())); }
+// m = the largest of m, |x| and |y|.  (NaNs are passed over, and make their sums NaNs anyway.  In assembly, so that it stands where the
+// products have ended: alternated with them, 2048 x 896 -> 512 took 0.8 us more.)
+__device__ __forceinline__ void largest(float& m, float x, float y) { asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x), "v"(y)); }
+// Whether a sum of K split products may be off, max_a and max_w being the largest |operands| of its two rows: it is not finite, or so
+// small that what a split may drop of operands below 2^-110, at most 2^-126 of each, times the other row's largest counts in it.
+// (What the matrix instructions may flush of the products, 2^-126 of each of the six, is less than that for 1.)
+constexpr float kSplitDrops = 0x1p-98f;
+__device__ __forceinline__ bool doubtful(float v, int K, float max_a, float max_w) {
+  const float least = (float)K * kSplitDrops * fmaxf(1.f, fmaxf(max_a, max_w));
+  const bool off = !(fabsf(v) >= least && fabsf(v) < __builtin_huge_valf());
+  return off && !(v == 0.f && (max_a == 0.f || max_w == 0.f));
+}
+// Where no operand of a tile is beyond this, and no sum of it doubtful for this, nothing is: one look at the tile.  (Each sum by its own
+// rows' largest operands, without it, made 2048 x 896 -> 512 16.9 us, the tile's at once 16.0; without any of this it was 15.8.)
+constexpr float kOrdinary = 0x1p40f;
 
 template <typename OutT, int NW, int TM, int TN, int SUMS>
 __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, OutT* __restrict__ Y, int M,
@@ -916,6 +929,8 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
   constexpr int SLOT = ROWS * kF32RowB;
   static_assert(BM * BN * 4 <= 2 * SLOT, "a partial tile fits where its wave's operands were");
   __shared__ __attribute__((aligned(16))) char lds[NW][2][SLOT];
+  __shared__ float most[NW][2][ROWS];  // the largest |operand| of each row that a half of the wave saw
+  __shared__ __attribute__((aligned(16))) uint32_t beyond[NW];  // whether any of them is beyond kOrdinary
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = (int)(blockIdx.x % tiles_m) * BM, n0 = (int)(blockIdx.x / tiles_m) * BN;
@@ -1003,11 +1018,25 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
       raw.w[b][1] = *(const uint4*)(from + (BM + b * 32) * kF32RowB + p1);
     }
   };
+  // (the largest operands so far of the rows whose fragments the lane has)
+  float max_a[TM], max_w[TN];
+#pragma unroll
+  for (int b = 0; b < TM; ++b) max_a[b] = 0.f;
+#pragma unroll
+  for (int b = 0; b < TN; ++b) max_w[b] = 0.f;
+  auto split = [&](const uint4 (&raw)[2], float& most) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      largest(most, __uint_as_float(raw[c].x), __uint_as_float(raw[c].y));
+      largest(most, __uint_as_float(raw[c].z), __uint_as_float(raw[c].w));
+    }
+    return split_floats(raw[0], raw[1]);
+  };
   auto convert = [&](const Raw& raw, Pieces& p) {
 #pragma unroll
-    for (int b = 0; b < TM; ++b) p.a[b] = split_floats(raw.a[b][0], raw.a[b][1]);
+    for (int b = 0; b < TM; ++b) p.a[b] = split(raw.a[b], max_a[b]);
 #pragma unroll
-    for (int b = 0; b < TN; ++b) p.w[b] = split_floats(raw.w[b][0], raw.w[b][1]);
+    for (int b = 0; b < TN; ++b) p.w[b] = split(raw.w[b], max_w[b]);
   };
   // the smallest products first
   auto multiply = [&](const Pieces& p, auto parity) {
@@ -1117,13 +1146,41 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
         v[e][3] += p.w;
       }
   };
+  {
+    float all = 0.f;
+#pragma unroll
+    for (int b = 0; b < TM + TN; ++b) {
+      const float m = b < TM ? max_a[b < TM ? b : 0] : max_w[b < TM ? 0 : b - TM];
+      most[wave][fhalf][b * 32 + frow] = m;
+      all = fmaxf(all, m);
+    }
+    const uint64_t any = __builtin_amdgcn_ballot_w64(all > kOrdinary);
+    if (lane == 0) beyond[wave] = any != 0;
+  }
   add_up();
   if (nn >= N || tid / BN >= CHUNKS) return;
-  uint32_t again = 0;
+  // |v| from what is doubtful for kOrdinary up to infinity, as bits without the sign's
+  uint32_t again = 0, worst = 0, large = 0;
+  const uint32_t least = __float_as_uint((float)K * (kSplitDrops * kOrdinary)) << 1;
 #pragma unroll
   for (int e = 0; e < EACH; ++e)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) again |= doubtful(v[e][c]) ? 1u << (e * 4 + c) : 0u;
+    for (int c = 0; c < 4; ++c) worst = max(worst, (__float_as_uint(v[e][c]) << 1) - least);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) large |= beyond[w];
+  if (__builtin_expect(large != 0 || worst >= 0xff000000u - least, 0)) {
+    auto row_most = [&](int row) {
+      float m = 0.f;
+      for (int w = 0; w < NW; ++w) m = fmaxf(m, fmaxf(most[w][0][row], most[w][1][row]));
+      return m;
+    };
+    const float max_w = row_most(BM + col);
+#pragma unroll
+    for (int e = 0; e < EACH; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        again |= doubtful(v[e][c], K, row_most((tid / BN + e * (NT / BN)) * 4 + c), max_w) ? 1u << (e * 4 + c) : 0u;
+  }
   while (again != 0) {  // (rare, and slow)
     const int which = __builtin_ctz(again);
     again &= again - 1;
