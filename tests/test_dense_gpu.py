@@ -334,6 +334,40 @@ def test_fc_fp32_small_numbers_times_large_ones(bz, M, N, K):
         assert torch.equal(bz.fc_fused(x1, w, K, bias=bias)[ordinary], y[ordinary])
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (700, 512, 201), (1000, 500, 300), (2048, 512, 899), (33, 9, 4)])
+def test_fc_fp32_tiles_of_sums_that_are_computed_again(bz, M, N, K):
+    """an infinity, a NaN or the largest float in every row: all sums again, in a time that does not explode (3.4 of a plain call's at
+    2048 x 899 -> 512; 30 as a dot product for each sum)"""
+    import torch
+    torch.manual_seed(K)
+    x = torch.rand(M, K, device="cuda") + 0.5
+    plain = x.clone()
+    w = bz.pack_weight(torch.rand(K, N, device="cuda") / (4 * K), False, bz.F32)
+    rows = torch.arange(M, device="cuda")
+    x[rows, rows % K] = torch.tensor([float("inf"), float("nan"), -float("inf"), 3.4028235e38, -3.4e38], device="cuda")[rows % 5]
+    print("case M=%d N=%d K=%d" % (M, N, K), flush=True)
+    bias = torch.zeros(N, device="cuda")
+    y = bz.fc_fused(x, w, K, bias=bias)
+    want = x.double() @ w[:, :K].double().t().contiguous()
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isposinf(y), torch.isposinf(want)) and torch.equal(torch.isneginf(y), torch.isneginf(want))
+    fine = torch.isfinite(want)
+    assert fine.any() and ((y.double() - want).abs() <= _plain_bound(x, w[:, :K], bias))[fine].all()
+
+    def us(a):
+        times = []
+        for _ in range(20):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(5):
+                bz.fc_fused(a, w, K, out=y)
+            e1.record()
+            e1.synchronize()
+            times.append(e0.elapsed_time(e1))
+        return sorted(times)[5]
+    if M >= 2048:
+        assert us(x) < 10 * us(plain)
+
+
 @pytest.mark.parametrize("M,K,N,H,act", [(1, 1024, 48, 1, "none"), (17, 516, 100, 8, "softmax"), (300, 256, 196, 2, "softmax"), (2049, 512, 256, 2, "none"),
                                          (300, 256, 192, 3, "sigmoid"), (2000, 200, 256, 2, "softmax")])
 def test_fc_fp32_head_apart_and_in_the_launch(bz, M, K, N, H, act):

@@ -891,19 +891,6 @@ __device__ __forceinline__ void load_to_lds_from(const char* base, uint32_t off,
                : "memory", "m0", "scc");
 }
 
-// the dot product of two fp32 rows, in four sums
-__device__ __forceinline__ float plain_dot(const float* a, const float* w, int K) {
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  int k = 0;
-  for (; k + 4 <= K; k += 4) {
-    s0 = fmaf(a[k], w[k], s0);
-    s1 = fmaf(a[k + 1], w[k + 1], s1);
-    s2 = fmaf(a[k + 2], w[k + 2], s2);
-    s3 = fmaf(a[k + 3], w[k + 3], s3);
-  }
-  for (; k < K; ++k) s0 = fmaf(a[k], w[k], s0);
-  return (s0 + s1) + (s2 + s3);
-}
 // m = the largest of m, |x| and |y|.  (NaNs are passed over, and make their sums NaNs anyway.  In assembly, so that it stands where the
 // products have ended: alternated with them, 2048 x 896 -> 512 took 0.8 us more.)
 __device__ __forceinline__ void largest(float& m, float x, float y) { asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x), "v"(y)); }
@@ -1109,6 +1096,7 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
   // wave leaves its partial tile where its operands were, column by column, the chunks of a column in an order of its own, so
   // that writes and reads are on all banks; then a thread adds up and finishes chunks of one column.
   constexpr int CHUNKS = BM / 4, EACH = (CHUNKS * BN + NT - 1) / NT;  // of a column; of a thread
+  static_assert((BN == 64 || (BN == 32 && EACH == 1)) && EACH <= 4, "the rows of a wave's threads are sixteen or fewer");
   static_assert(NT % BN == 0 && (CHUNKS * BN % NT == 0 || EACH == 1) && (CHUNKS & (CHUNKS - 1)) == 0, "threads share the tile's chunks evenly");
   auto chunk_at = [&](int col, int chunk) { return (col * CHUNKS + (chunk ^ (col & (CHUNKS - 1)))) * 16; };
   const int col = tid % BN, nn = n0 + col;
@@ -1158,7 +1146,7 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
     if (lane == 0) beyond[wave] = any != 0;
   }
   add_up();
-  if (nn >= N || tid / BN >= CHUNKS) return;
+  if (tid / BN >= CHUNKS) return;  // (whole waves)
   // |v| from what is doubtful for kOrdinary up to infinity, as bits without the sign's
   uint32_t again = 0, worst = 0, large = 0;
   const uint32_t least = __float_as_uint((float)K * (kSplitDrops * kOrdinary)) << 1;
@@ -1181,16 +1169,63 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
       for (int c = 0; c < 4; ++c)
         again |= doubtful(v[e][c], K, row_most((tid / BN + e * (NT / BN)) * 4 + c), max_w) ? 1u << (e * 4 + c) : 0u;
   }
-  while (again != 0) {  // (rare, and slow)
-    const int which = __builtin_ctz(again);
-    again &= again - 1;
-    const int m = m0 + (tid / BN + which / 4 * (NT / BN)) * 4 + which % 4;
-    const float s = plain_dot((const float*)A + (int64_t)min(m, M - 1) * lda, (const float*)W + (int64_t)nn * ldw, K);
+  if (__builtin_expect(__any(again != 0), 0)) {
+    // The wave's rows times all columns once more, with fp32 instructions; of these products the doubtful ones are taken.  A row of sixteen
+    // operands is four rows of chunk i / 4, in the order the wave's threads have them; an instruction's four inputs have a sum of their own.
+    // (It waits for its operands, 64 inputs of all rows at a time.  2048 x 896 -> 512, 16.0 us without: a NaN in one row 42 us, in every 32nd 42,
+    // in all 53; as dot products of the threads, a sum at a time, 42, 65 and 504.)
+    const int i = lane & 15, q = i >> 2;
+    const int chunk = BN == 64 ? wave + min(q, EACH - 1) * (NT / BN) : wave * 2 + (q & 1);
+    const float* const a = (const float*)A + min(m0 + chunk * 4 + (i & 3), M - 1) * lda;
+    const float* w[BN / 16];
+    floatx4 sums[BN / 16][4];
 #pragma unroll
-    for (int e = 0; e < EACH; ++e)
+    for (int b = 0; b < BN / 16; ++b) {
+      w[b] = (const float*)W + min(n0 + b * 16 + i, N - 1) * ldw;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) v[e][c] = which == e * 4 + c ? s : v[e][c];
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[b][t][r] = 0.f;
+    }
+    constexpr int kAhead = 4;  // steps of sixteen inputs asked for together
+    for (int k0 = 0; k0 < K; k0 += 16 * kAhead) {
+      uint4 x[kAhead], y[kAhead][BN / 16];
+      int beyond_k[kAhead];
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) {
+        const int k = k0 + s * 16 + (lane >> 4) * 4, from = min(k, K - 4);
+        beyond_k[s] = k - from;
+        __builtin_memcpy(&x[s], a + from, 16);
+#pragma unroll
+        for (int b = 0; b < BN / 16; ++b) __builtin_memcpy(&y[s][b], w[b] + from, 16);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) {
+        const uint4 xs = shift_chunk<BZ_F32>(x[s], beyond_k[s]);
+#pragma unroll
+        for (int b = 0; b < BN / 16; ++b) {
+          const uint4 ys = shift_chunk<BZ_F32>(y[s][b], beyond_k[s]);
+          sums[b][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(xs.x), __uint_as_float(ys.x), sums[b][0], 0, 0, 0);
+          sums[b][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(xs.y), __uint_as_float(ys.y), sums[b][1], 0, 0, 0);
+          sums[b][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(xs.z), __uint_as_float(ys.z), sums[b][2], 0, 0, 0);
+          sums[b][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(xs.w), __uint_as_float(ys.w), sums[b][3], 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < BN / 16; ++b)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float s = (sums[b][0][c] + sums[b][1][c]) + (sums[b][2][c] + sums[b][3][c]);
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+          const float t = __shfl(s, (col & 15) + 16 * (BN == 64 ? e : lane >> 5), bz::kWave);
+          if ((col >> 4) == b && (again >> (e * 4 + c) & 1) != 0) v[e][c] = t;
+        }
+      }
   }
+  if (nn >= N) return;
   cbias *= ep.beta;
   if (ep.act == BZ_ACT_DICE) cp2 = dice_inv_den(ep, cp2);
   OutT* const y = Y + out_index(ep, m0, nn, ldy);
