@@ -229,6 +229,14 @@ def test_fc_fp32_error_of_eight_sums(bz, M, N, K):
     assert err <= 0.26 * 2.0**-24 * (K / 8) ** 0.5 * 1.15, err
 
 
+# up to 512 tiles of 32x32 that make more than 128 of 64x64, their edges being half empty: 64x64 of eight waves
+@pytest.mark.parametrize("M,N,K", [(5000, 90, 896), (4097, 65, 512), (5425, 96, 300), (3000, 150, 1024), (2200, 200, 896), (1700, 270, 2048), (1409, 321, 401)])
+def test_fc_fp32_error_of_eight_sums_in_ragged_layers(bz, M, N, K):
+    """as above"""
+    assert -(-M // 32) * -(-N // 32) <= 512 and -(-M // 64) * -(-N // 64) > 128
+    test_fc_fp32_error_of_eight_sums(bz, M, N, K)
+
+
 # 2-byte layers of more than 256 tiles of 64x64: 64x128 and 128x64 tiles, also for rows that start on no 16 bytes
 @pytest.mark.parametrize("in_name,out_name", [("f16", "f16"), ("bf16", "f32")])
 @pytest.mark.parametrize("M,N,K,act,kw", [(1900, 520, 392, "dice", {}), (6017, 136, 64, "prelu", {"full_bias": True}),   # 64x128, ragged; one K tile
@@ -297,7 +305,7 @@ def test_fc_fp32_infinities_and_numbers_at_the_ends_of_the_range(bz, M, N, K):
     assert (y[5:7] == 0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (1200, 400, 160), (1200, 800, 250), (1024, 512, 300), (3, 9, 1000)])
+@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (1200, 400, 160), (1200, 800, 250), (1024, 512, 300), (1409, 321, 301), (3, 9, 1000)])
 def test_fc_fp32_small_numbers_times_large_ones(bz, M, N, K):
     """Operands whose last bits no three bf16s hold, or none at all, times such of the other side that the sums are ordinary numbers, or
     small ones that are not 0; whole rows and columns of them, and single ones among zeros.  Ordinary rows beside them, and rows of
@@ -334,7 +342,7 @@ def test_fc_fp32_small_numbers_times_large_ones(bz, M, N, K):
         assert torch.equal(bz.fc_fused(x1, w, K, bias=bias)[ordinary], y[ordinary])
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (700, 512, 201), (1000, 500, 300), (2048, 512, 899), (33, 9, 4)])
+@pytest.mark.parametrize("M,N,K", [(40, 70, 130), (700, 512, 201), (1000, 500, 300), (2048, 512, 899), (1409, 321, 301), (33, 9, 4)])
 def test_fc_fp32_tiles_of_sums_that_are_computed_again(bz, M, N, K):
     """an infinity, a NaN or the largest float in every row: all sums again, in a time that does not explode (3.4 of a plain call's at
     2048 x 899 -> 512; 30 as a dot product for each sum)"""

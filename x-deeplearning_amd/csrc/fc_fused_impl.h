@@ -1672,10 +1672,14 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
     // eight, add every output up in two sums, stage by stage in turn (1024 x 896 -> 512 with one 11.1 / 7.4 and 2.3e-7, 1024 x 4096 -> 512 35.9 / 33
     // and 5.0e-7, with two 38.3 / 32 and 3.5e-7, before 49.8 / 45 and 4.1e-7), and up to 32 columns eight waves stay with
     // 32x32 (12000 x 512 -> 20 9.9 / 6.0, 64x64 11.1 / 6.0, now 8.7 / 5.3; 16384 x 1024 -> 32 17.3 / 13.1, 16.9 / 13.7 and 15.9 / 11.7).
+    // Ragged layers of up to 512 tiles of 32x32 and more than 128 of 64x64, which the split kernel had, too, have eight sums from eight waves
+    // on 64x64 (four waves, four sums / 32x64, two sums each / this: 2200 x 896 -> 200 16.0 / 7.0 and 2.2e-7, 17.9 / 8.8 and 1.6e-7, 15.6 / 8.5
+    // and 1.6e-7; 1700 x 2048 -> 270 26.8 / 14.5, 31.0 / 17.8, 26.0 / 15.7; 4500 x 512 -> 96 11.4 / 5.9, 12.1 / 6.1, 11.4 / 6.2).
     const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
     if (f32_rows_fit(d.lda, d.k) && f32_rows_fit(d.ldw, d.k) && (d.k > 96 || wg64 <= 128 || wg32 <= 512)) {
       if (wg32 <= 256 || (wg32 <= 512 && (d.k <= 256 || d.n <= 32))) return launch_f32<OutT, 8, 1, 1, 1>(d, ep, st);
       if (wg64 <= 128) return launch_f32<OutT, 4, 1, 2, 2>(d, ep, st);
+      if (wg32 <= 512) return launch_f32<OutT, 8, 2, 2, 1>(d, ep, st);
       if (d.k < 200) return launch_f32<OutT, 4, 1, 2, 1>(d, ep, st);
       return launch_f32<OutT, 4, 2, 2, 1>(d, ep, st);
     }
