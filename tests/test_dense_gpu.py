@@ -229,6 +229,22 @@ def test_fc_fp32_error_of_eight_sums(bz, M, N, K):
     assert err <= 0.26 * 2.0**-24 * (K / 8) ** 0.5 * 1.15, err
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 256, 64), (700, 512, 200), (12000, 20, 300), (1024, 512, 300), (2200, 200, 300), (1024, 256, 512)])
+@pytest.mark.parametrize("nosqrt", [False, True])
+def test_fc_fp32_dice_of_small_layers_is_the_activation_kernels(bz, M, N, K, nosqrt):
+    """up to 512 tiles of 32x32 Dice is computed with expf and exact divisions: bit for bit what the standalone kernel makes of the layer"""
+    import torch
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda")
+    w = bz.pack_weight(torch.randn(K, N, device="cuda") / K**0.5, False, bz.F32)
+    bias = torch.randn(N, device="cuda") * 0.1
+    params = (torch.rand(N, device="cuda"), torch.randn(N, device="cuda") * 0.1, torch.rand(N, device="cuda") + 0.2)
+    assert -(-M // 32) * -(-N // 32) <= 512
+    got = bz.fc_fused(x, w, K, bias=bias, act=bz.ACT_DICE, act_params=params, dice_nosqrt=nosqrt)
+    want = bz.activation(bz.fc_fused(x, w, K, bias=bias), bz.ACT_DICE, params, dice_nosqrt=nosqrt)
+    assert torch.equal(got, want), float((got - want).abs().max())
+
+
 # up to 512 tiles of 32x32 that make more than 128 of 64x64, their edges being half empty: 64x64 of eight waves
 @pytest.mark.parametrize("M,N,K", [(5000, 90, 896), (4097, 65, 512), (5425, 96, 300), (3000, 150, 1024), (2200, 200, 896), (1700, 270, 2048), (1409, 321, 401)])
 def test_fc_fp32_error_of_eight_sums_in_ragged_layers(bz, M, N, K):

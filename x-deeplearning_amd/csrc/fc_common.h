@@ -50,19 +50,22 @@ __device__ __forceinline__ int64_t full_bias_index(const Epilogue& ep, int64_t m
   return ((int64_t)p * M + m) * ep.split_n + (n - p * ep.split_n);
 }
 
+// Dice as the standalone kernel computes it: the denominator of a column, and an output
+__device__ __forceinline__ float dice_den(const Epilogue& e, float var) { return e.dice_nosqrt ? var : sqrtf(var + kDiceEps); }
+__device__ __forceinline__ float dice_exact(float v, float gamma, float mean, float den) {
+  const float t = expf(-1.f * (v - mean) / den);
+  const float p = 1.f / (1.f + t);
+  return (1.f - p) * gamma * v + p * v;
+}
+
 __device__ __forceinline__ float apply_act(float v, int n, const Epilogue& e) {
   switch (e.act) {
     case BZ_ACT_PRELU: {
       const float w = e.p0[e.act_size == 1 ? 0 : n];
       return v * ((float)(v > 0.f) + (float)(v < 0.f) * w);  // math/activation.h:37-42
     }
-    case BZ_ACT_DICE: {
-      const float var = e.p2[n];
-      const float den = e.dice_nosqrt ? var : sqrtf(var + kDiceEps);
-      const float t = expf(-1.f * (v - e.p1[n]) / den);
-      const float p = 1.f / (1.f + t);
-      return (1.f - p) * e.p0[n] * v + p * v;
-    }
+    case BZ_ACT_DICE:
+      return dice_exact(v, e.p0[n], e.p1[n], dice_den(e, e.p2[n]));
     case BZ_ACT_LEAKY_RELU:
       return v >= 0.f ? v : e.act_alpha * v;
     case BZ_ACT_SIGMOID: {
@@ -79,12 +82,8 @@ __device__ __forceinline__ float apply_act_regs(float v, const Epilogue& e, floa
   switch (e.act) {
     case BZ_ACT_PRELU:
       return v * ((float)(v > 0.f) + (float)(v < 0.f) * p0);
-    case BZ_ACT_DICE: {
-      const float den = e.dice_nosqrt ? p2 : sqrtf(p2 + kDiceEps);
-      const float t = expf(-1.f * (v - p1) / den);
-      const float p = 1.f / (1.f + t);
-      return (1.f - p) * p0 * v + p * v;
-    }
+    case BZ_ACT_DICE:
+      return dice_exact(v, p0, p1, dice_den(e, p2));
     case BZ_ACT_LEAKY_RELU:
       return v >= 0.f ? v : e.act_alpha * v;
     case BZ_ACT_SIGMOID: {
@@ -98,7 +97,7 @@ __device__ __forceinline__ float apply_act_regs(float v, const Epilogue& e, floa
 
 // log2(e) / (the Dice denominator of a column): computed once per column, before the K loop
 __device__ __forceinline__ float dice_inv_den(const Epilogue& e, float var) {
-  return 1.44269504088896341f / (e.dice_nosqrt ? var : sqrtf(var + kDiceEps));
+  return 1.44269504088896341f / dice_den(e, var);
 }
 
 // The tile kernels' epilogue, activation fixed at compile time.  For Dice p2 is dice_inv_den() of the column, not its

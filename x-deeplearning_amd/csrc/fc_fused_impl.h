@@ -907,7 +907,8 @@ __device__ __forceinline__ bool doubtful(float v, int K, float max_a, float max_
 // rows' largest operands, without it, made 2048 x 896 -> 512 16.9 us, the tile's at once 16.0; without any of this it was 15.8.)
 constexpr float kOrdinary = 0x1p40f;
 
-template <typename OutT, int NW, int TM, int TN, int SUMS>
+// EXACT: Dice as apply_act computes it, not as the tile kernels do
+template <typename OutT, int NW, int TM, int TN, int SUMS, bool EXACT>
 __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, OutT* __restrict__ Y, int M,
                                                             int N, int K, int64_t lda, int64_t ldw, int64_t ldy, int tiles_m,
                                                             Epilogue ep) {
@@ -1227,7 +1228,7 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
   }
   if (nn >= N) return;
   cbias *= ep.beta;
-  if (ep.act == BZ_ACT_DICE) cp2 = dice_inv_den(ep, cp2);
+  if (ep.act == BZ_ACT_DICE) cp2 = EXACT ? dice_den(ep, cp2) : dice_inv_den(ep, cp2);
   OutT* const y = Y + out_index(ep, m0, nn, ldy);
   with_act(ep.act, [&](auto act) {
 #pragma unroll
@@ -1237,7 +1238,12 @@ __global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __res
         const int ml = (tid / BN + e * (NT / BN)) * 4 + c;
         if (m0 + ml >= M) continue;
         const float b = ep.bias_rows > 1 ? ep.beta * ep.bias[full_bias_index(ep, m0 + ml, nn, M, N)] : cbias;
-        store_out<OutT>(y + ml * ldy, apply_act_t<decltype(act)::value>(fmaf(ep.alpha, v[e][c], b), ep, cp0, cp1, cp2));
+        const float z = fmaf(ep.alpha, v[e][c], b);
+        constexpr int ACT = decltype(act)::value;
+        if constexpr (EXACT && ACT == BZ_ACT_DICE)
+          store_out<OutT>(y + ml * ldy, dice_exact(z, cp0, cp1, cp2));
+        else
+          store_out<OutT>(y + ml * ldy, apply_act_t<ACT>(z, ep, cp0, cp1, cp2));
       }
   });
 }
@@ -1492,10 +1498,10 @@ int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 }
 
 
-template <typename OutT, int NW, int TM, int TN, int SUMS>
+template <typename OutT, int NW, int TM, int TN, int SUMS, bool EXACT>
 int launch_f32(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 32 * TM - 1) / (32 * TM), tiles_n = (d.n + 32 * TN - 1) / (32 * TN);
-  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN, SUMS>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
+  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN, SUMS, EXACT>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
                      d.ldw, d.ldy, tiles_m, ep);
   BZ_LAUNCH_OK("bz_fc_f32_kernel");
   return BZ_OK;
@@ -1675,13 +1681,15 @@ int dispatch_tiles(const bz_fc_desc& d, const Epilogue& ep, bool vec_a, bool vec
     // Ragged layers of up to 512 tiles of 32x32 and more than 128 of 64x64, which the split kernel had, too, have eight sums from eight waves
     // on 64x64 (four waves, four sums / 32x64, two sums each / this: 2200 x 896 -> 200 16.0 / 7.0 and 2.2e-7, 17.9 / 8.8 and 1.6e-7, 15.6 / 8.5
     // and 1.6e-7; 1700 x 2048 -> 270 26.8 / 14.5, 31.0 / 17.8, 26.0 / 15.7; 4500 x 512 -> 96 11.4 / 5.9, 12.1 / 6.1, 11.4 / 6.2).
+    // Up to 512 tiles of 32x32 Dice is exact, as it was in the split kernels (the activation's own error 3.6e-8 of the outputs, with v_exp_f32 and
+    // v_rcp_f32 3.9e-8; 1024 x 896 -> 512 with Dice 11.9 us and 11.1, without 10.8); with more, as it was in the tiles.
     const int64_t wg64 = (int64_t)((d.m + 63) / 64) * ((d.n + 63) / 64);
     if (f32_rows_fit(d.lda, d.k) && f32_rows_fit(d.ldw, d.k) && (d.k > 96 || wg64 <= 128 || wg32 <= 512)) {
-      if (wg32 <= 256 || (wg32 <= 512 && (d.k <= 256 || d.n <= 32))) return launch_f32<OutT, 8, 1, 1, 1>(d, ep, st);
-      if (wg64 <= 128) return launch_f32<OutT, 4, 1, 2, 2>(d, ep, st);
-      if (wg32 <= 512) return launch_f32<OutT, 8, 2, 2, 1>(d, ep, st);
-      if (d.k < 200) return launch_f32<OutT, 4, 1, 2, 1>(d, ep, st);
-      return launch_f32<OutT, 4, 2, 2, 1>(d, ep, st);
+      if (wg32 <= 256 || (wg32 <= 512 && (d.k <= 256 || d.n <= 32))) return launch_f32<OutT, 8, 1, 1, 1, true>(d, ep, st);
+      if (wg64 <= 128) return launch_f32<OutT, 4, 1, 2, 2, true>(d, ep, st);
+      if (wg32 <= 512) return launch_f32<OutT, 8, 2, 2, 1, true>(d, ep, st);
+      if (d.k < 200) return launch_f32<OutT, 4, 1, 2, 1, false>(d, ep, st);
+      return launch_f32<OutT, 4, 2, 2, 1, false>(d, ep, st);
     }
   }
   if (d.k < In<DT>::kChunk || (In<DT>::kSize == 2 && wg32 <= (aligned || d.k > 256 ? 256 : 192))) return launch_split<DT, OutT, 8>(d, ep, st);
