@@ -8,8 +8,8 @@
 // way; the rows, which all eight waves read, are in LDS.
 // us alone / a launch on four streams, two launches and this: 1024 of 198 -> 200 -> 80 -> 2 11.7 / 5.5 and 7.5 / 3.0, 300 of 445 -> 256 -> 100
 // 10.9 / 5.2 and 8.4 / 3.2, 2048 of 896 -> 512 -> 256 16.4 / 6.5 and 14.9 / 4.5 (of these 14.9: rows to LDS 2.9, first layer 6.3, its
-// activation 1.1, second layer and activation 2.1, skinny layer 0.9).  fp16 model of 2048 x 26 lists on eight serving threads, us a pass:
-// 14.9 and 13.8.
+// activation 1.1, second layer and activation 2.1, skinny layer 0.9).  fp16 model of 2048 x 26 lists, us a lone pass / of eight serving threads:
+// 43.5 / 13.8 and 41.7 / 11.9.
 #include <mutex>
 
 #include "fc_common.h"
@@ -126,6 +126,27 @@ struct WeightStream {
         w[j][t] = *(const uint4*)&v;
       }
     __builtin_amdgcn_sched_barrier(0);  // (they stay ahead of what the wave multiplies meanwhile)
+  }
+};
+
+// The weights on their way into the XCD's L2: its workgroups ask for a share each, a word of every line, while the rows are staged.  In a
+// pass of a whole model the lookups have been through L2 since the last one, all workgroups walk the weights in step, and each waits for
+// every line as if it were alone: 128 KB under way are too few for the memory's latency.  (A lone pass of 2048 x 26 lists, 896 -> 512 -> 256 -> 2,
+// without this 45.4 us, 43.5 in two launches, 41.7 this way; on eight threads 12.4, 13.8 and 11.9 a pass.)
+struct WarmWeights {
+  static constexpr int kEach = 2;  // of the first layer, a thread's: its 0.9 MB where eight workgroups share an XCD
+  uint32_t w[kEach + 1];
+  __device__ __forceinline__ void ask(const Weights& w1, const Weights& w2) {
+    const uint32_t sharers = (gridDim.x + bz::kNumXcd - 1) / bz::kNumXcd, at = blockIdx.x / bz::kNumXcd * kThreads + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(w1.from, (int)((i * sharers * kThreads + at) * 128u), 0, 0);
+    w[kEach] = __builtin_amdgcn_raw_buffer_load_b32(w2.from, (int)(at * 128u), 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // (they have arrived by now; until here nobody has waited for them)
+  __device__ __forceinline__ void done() const {
+#pragma unroll
+    for (int i = 0; i <= kEach; ++i) asm volatile("" ::"v"(w[i]));
   }
 };
 
@@ -311,10 +332,12 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a)
     const int j = hj + i * (kThreads / kMaxNarrow);
     hw[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from_head, j < a.head.n && hc < a.n2 ? (j * (int)a.head.ldw + hc) * 2 : kBeyond, 0, 0);
   }
+  WarmWeights warm;
   stage_rows<ODD>(
       a, m0, lds,
       [&]() {
         first.start(w1, wave);
+        warm.ask(w1, w2);
       },
       [&]() {
         col1.put(a.ep1, k2, params1);
@@ -327,6 +350,7 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a)
 
   const bool busy1 = wave * 32 < k2, busy2 = wave * 32 < k3;
   if (busy1) first.run(w1, lds, wave);
+  warm.done();
   Layer<1> second;
   second.start(w2, wave);
   __syncthreads();
