@@ -435,18 +435,20 @@ bool bz::fc_tower_takes(int64_t k, int64_t n1, int64_t n2) {
          layout((int)k, (int)n1, (int)n2, kSkinnyMaxN).all <= kMaxLds;
 }
 
-// One launch against two, us alone / a launch on four streams (the weights of both layers in KB).  Each workgroup reads all the
-// weights, so up to 512 KB it is the better at any number of rows that one round of workgroups takes: 300 of 64 -> 256 -> 104 (82)
-// 6.2 / 3.5 and 8.9 / 5.7, 1024 of 198 -> 200 -> 80 (108) 7.5 / 3.0 and 11.7 / 5.5, one of 200 -> 200 -> 80 6.4 / 3.0 and 8.4 / 5.5,
-// 300 of 896 -> 256 -> 104 (500) 9.8 / 3.8 and 10.4 / 6.9, but 640 -> 400 -> 128 (600) 12.0 / 3.8 and 11.7 / 6.8; with more, where the
-// rows fill the CUs of two launches and from where on a model with it is as fast alone and faster on eight serving threads (1024
-// samples 113 / 10.4 us a pass with two, 115 / 10.4 with one, 1300 131.2 / 11.4 and 130.6 / 10.4): 1024, 2048 and 4096 of 896 -> 512 -> 256 (1152) 14.9 / 4.6 and 14.3 / 6.7, 14.9 / 4.5 and 16.4 / 6.5,
-// 15.0 / 8.0 and 18.7 / 10.7, but 2048 of 1280 -> 512 -> 256 (1536) 18.6 / 6.0 and 18.0 / 7.8.  Rows of more than 1280 inputs are
-// long to stage (300 of 1600 -> 64 -> 32 (204) 10.2 / 3.9 and 10.0 / 6.9), and beyond 4096 rows two launches leave more to others: 6000 of
-// 896 -> 400 -> 128 15.5 / 11.5 and 21.4 / 10.9, 16000 of 640 -> 64 -> 32 10.3 / 7.9 and 13.2 / 6.7.
+// One launch against two, in models that look 32-wide rows up for the input, us of a lone pass / of eight serving threads (weights in units
+// of 1024).  From 1200 rows on one launch is as fast alone and faster beside others, with inputs up to 1024:
+//  896 -> 512 -> 256 (576) 1100 rows 37.8 / 9.9 and 37.7 / 9.3, 1300 39.0 / 9.2 and 39.2 / 10.5, 2048 39.4 / 10.3 and 39.6 / 11.9, 4096 47.2 / 18.8
+//  and 50.4 / 21.7; 1024 -> 512 -> 256 (640) 1600 41.1 / 10.5 and 40.8 / 12.1, 3000 45.0 / 16.2 and 47.6 / 18.8; 640 -> 400 -> 128 (300) 1300
+//  32.9 / 8.5 and 34.4 / 8.8; but 2048 of 1152 -> 512 -> 256 47.0 / 13.2 and 45.8 / 14.8, of 1216 -> 200 -> 80 41.9 / 11.6 and 40.4 / 13.2.
+// With fewer rows, and few workgroups to pull all the weights, where these are few:
+//  256 -> 200 -> 80 (65) one row 22.9 / 4.9 and 24.0 / 5.2, 1024 26.1 / 6.2 and 27.8 / 6.5; 448 -> 256 -> 100 (137) one row 24.0 / 5.1 and 23.8 / 5.3,
+//  300 28.0 / 6.2 and 28.7 / 6.9; 640 -> 200 -> 80 (140) 64 rows 27.7 / 5.8 and 26.7 / 6.0, 300 29.9 / 6.6 and 29.5 / 6.7; 1280 -> 100 -> 40 (128) 300
+//  33.5 / 7.8 and 35.3 / 8.3; but 300 of 1152 -> 128 -> 64 (152) 35.3 / 7.5 and 31.3 / 7.5, of 896 -> 200 -> 80 (190) 32.5 / 7.4 and 31.0 / 7.0, of
+//  896 -> 512 -> 256 38.5 / 9.7 and 33.7 / 8.0.  (Alone on hot weights one launch wins far beyond these lines: 300 of 896 -> 256 -> 104 9.8 and 10.4.)
+// Beyond 4096 rows two launches leave more to others (6000 of 896 -> 400 -> 128 on hot weights 15.5 us alone, 11.5 on four streams, and 21.4, 10.9).
 bool bz::fc_tower_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2) {
-  const int64_t weights = k * n1 + n1 * n2;
-  return rows >= 1 && rows <= 4096 && ((k <= 1280 && weights <= 256 << 10) || (k <= 1024 && weights <= 576 << 10 && rows >= 1100));
+  if (rows >= 1200) return rows <= 4096 && (k <= 1024 || (k <= 1280 && k * n1 + n1 * n2 <= 144 << 10));
+  return rows >= (k <= 512 ? 1 : 300) && k <= 1280 && k * n1 + n1 * n2 <= 144 << 10;
 }
 
 int bz::fc_tower(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
