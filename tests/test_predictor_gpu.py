@@ -1419,19 +1419,19 @@ def _tower(pb, ws, bs, acts, chain, heads):
     nb = pb.NetBuilder("tower%d" % chain, device_type=1)
     nb.arg("chain_narrow_fcs", chain)
     nb.external_input("x", pb.K_FLOAT16)
-    h = "x"
-    for i, (w, b) in enumerate(zip(ws, bs)):
+    params = [[] if a is None else a[1:] for a in acts]
+    for i, (w, b) in enumerate(zip(ws, bs)):  # (in front of the layers: operators are joined where they follow each other)
         nb.constant("w%d" % i, w)
         nb.constant("b%d" % i, b)
+        for j, p in enumerate(params[i] if i < 2 else []):
+            nb.constant("a%d%d" % (i, j), p)
+    h = "x"
+    for i in range(3):
         nb.op("Gemm", [h, "w%d" % i, "b%d" % i], ["g%d" % i], transB=0)
         h = "g%d" % i
         if i < 2 and acts[i] is not None:
-            ins = [h]
-            for j, p in enumerate(acts[i][1:]):
-                nb.constant("a%d%d" % (i, j), p)
-                ins.append("a%d%d" % (i, j))
+            nb.op(acts[i][0], [h] + ["a%d%d" % (i, j) for j in range(len(params[i]))], ["h%d" % i])
             h = "h%d" % i
-            nb.op(acts[i][0], ins, [h])
     if heads > 1:
         nb.op("Softmax", [h], ["p"], axis=1)
     else:
@@ -1440,6 +1440,16 @@ def _tower(pb, ws, bs, acts, chain, heads):
     pm = pb.PredictorManager()
     pm.load_model_from_string(nb.text(), True)
     return pm.create_predictor(1, 0)
+
+
+def _tower_pays(rows, k, n1, n2):
+    few = k * n1 + n1 * n2 <= 144 << 10
+    return rows <= 4096 and (k <= 1024 or few and k <= 1280) if rows >= 1200 else rows >= (1 if k <= 512 else 300) and k <= 1280 and few
+
+
+def _tower_launches(p):
+    layers = [e for e in json.loads(p.dump_observers()["profile"])["traceEvents"] if e["name"].startswith("Gemm:")][:2]
+    return sum(e["args"]["launches"] for e in layers), [e["dur"] for e in layers]
 
 
 def _tower_act(z, act):
@@ -1457,8 +1467,8 @@ def _tower_act(z, act):
 # k: one input, rows of 16-byte, 4-byte and 2-byte steps, whole and ragged 64s, the longest that is staged at once and the longest taken;
 # n1: one and two blocks a wave; n2, heads: the smallest and the largest; rows: one workgroup's edges and the lines of bz::fc_tower_pays
 @pytest.mark.parametrize("k,n1,n2,heads,rows", [(1, 9, 9, 1, (1, 33)), (64, 32, 33, 2, (31, 32, 33, 4096, 4097)), (65, 33, 64, 8, (5, 300)), (66, 256, 100, 2, (300, 64)),
-                                                (445, 256, 100, 2, (300, 1, 2049)), (448, 257, 256, 3, (40, 4096)), (1024, 192, 96, 1, (70, 2)), (1027, 200, 80, 2, (33, 500)),
-                                                (1280, 160, 40, 2, (100, )), (896, 512, 256, 2, (1099, 1100, 2048, 32)), (128, 512, 250, 8, (77, 1500))])
+                                                (445, 256, 100, 2, (300, 1, 2049)), (448, 257, 256, 3, (40, 4096)), (1024, 192, 96, 1, (70, 1301)), (1027, 104, 40, 2, (33, 500)),
+                                                (1280, 88, 40, 2, (300, )), (896, 512, 256, 2, (1199, 1200, 2048, 32)), (128, 512, 250, 8, (77, 1500))])
 @pytest.mark.parametrize("act", ["PRelu", "Dice", "Sigmoid", None])
 def test_tower_in_one_launch(pb, k, n1, n2, heads, rows, act):
     """fp16 layer -> layer -> skinny layer against 64 bits from the rounded layers and against one launch a layer, the rows growing and
@@ -1482,6 +1492,9 @@ def test_tower_in_one_launch(pb, k, n1, n2, heads, rows, act):
             p.feed("x", x)
             p.forward()
             got.append(p.output_asnumpy("p").astype(np.float64).reshape(m, heads))
+        # (a head behind columns that are no multiple of eight may be a launch of its own; two layers with nothing between are made one)
+        if act is not None and step < len(rows):
+            assert (_tower_launches(one)[0] == 1) == _tower_pays(m, k, n1, n2) and _tower_launches(apart)[0] >= 2, "%d rows" % m
         h = x.astype(np.float64)
         for w, b, a in zip(ws[:2], bs, acts):
             h = _tower_act(h @ w.astype(np.float64) + b, a).astype(np.float16).astype(np.float64)
@@ -1492,6 +1505,24 @@ def test_tower_in_one_launch(pb, k, n1, n2, heads, rows, act):
         # layer, and the result, at most 1 with a slope of at most 1/4, is rounded to 2^-11
         for g in got:
             np.testing.assert_allclose(g, want, rtol=0, atol=4 * 2.0**-11, err_msg="%d rows" % m)
+
+
+# both sides of each line of bz::fc_tower_pays, and of what the kernel takes
+@pytest.mark.parametrize("k,n1,n2,rows,one", [(512, 200, 80, 1, True), (513, 200, 80, 299, False), (513, 200, 80, 300, True), (896, 200, 80, 300, False),
+                                              (1280, 100, 40, 2048, True), (1280, 200, 80, 2048, False), (1024, 512, 256, 1199, False), (1024, 512, 256, 1200, True),
+                                              (896, 512, 256, 4096, True), (896, 512, 256, 4097, False), (64, 520, 64, 300, False), (64, 64, 264, 300, False)])
+def test_tower_launches(pb, k, n1, n2, rows, one):
+    """the launches of a pass as it runs, with nothing timing its operators: one for a tower where that pays, else two or three"""
+    ws = [np.full(s, 2.0**-10, np.float16) for s in ((k, n1), (n1, n2), (n2, 2))]
+    bs = [np.zeros(n, np.float16) for n in (n1, n2, 2)]
+    for chain in (1, 0):
+        p = _tower(pb, ws, bs, [("Sigmoid", ), ("Sigmoid", )], chain, 2)
+        for m in (rows, 8, rows):
+            p.feed("x", np.ones((m, k), np.float16))
+            p.forward()
+        np.testing.assert_allclose(p.output_asnumpy("p"), 0.5, rtol=1e-3)
+        launches, timed = _tower_launches(p)
+        assert timed == [0, 0] and (launches == 1) == (one and chain == 1)
 
 
 @pytest.mark.parametrize("k", [72, 70, 69])
