@@ -168,7 +168,10 @@ template <int TN>
 struct Layer {
   WeightStream<TN> w[3];
   RowFragments r[3];
-  floatx16 acc[TN];
+  // An output's sums, of every second or fourth step of 16 inputs: two as in the tiles, and four where these were the split kernel's, with
+  // eight (896 -> 512 -> 256 -> 2: the model's error is that of two launches, with one sum 20 % more outputs are rounded to the other side).
+  static constexpr int kSums = TN == 1 ? 4 : 2;
+  floatx16 acc[TN], more[kSums - 1][TN];
   __device__ __forceinline__ void start(const Weights& from, int block) {
     w[0].ask(from, block, 0);
     w[1].ask(from, block, 1);
@@ -177,7 +180,7 @@ struct Layer {
 #pragma unroll
     for (int j = 0; j < kGroup; ++j)
 #pragma unroll
-      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[j][t], r[i].x[j], acc[t]);
+      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[j][t], r[i].x[j], j % kSums == 0 ? acc[t] : more[(j + kSums - 1) % kSums][t]);
     __builtin_amdgcn_sched_barrier(0);
   }
   // acc = the weights' blocks times the rows.  (Behind the last group's fragments lie others: read, and not used.)
@@ -185,7 +188,11 @@ struct Layer {
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+      for (int i = 0; i < 16; ++i) {
+        acc[t][i] = 0.f;
+#pragma unroll
+        for (int s = 0; s < kSums - 1; ++s) more[s][t][i] = 0.f;
+      }
     const int groups = from.steps / kGroup;
     r[0].read(rows, 0);
     int g = 0;
@@ -202,6 +209,11 @@ struct Layer {
       multiply(0);
       if (g + 1 < groups) multiply(1);
     }
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        acc[t][i] = kSums == 2 ? acc[t][i] + more[0][t][i] : (acc[t][i] + more[0][t][i]) + (more[1 % (kSums - 1)][t][i] + more[2 % (kSums - 1)][t][i]);
   }
 };
 
