@@ -137,7 +137,7 @@ __device__ __forceinline__ void chunk_to_float(const uint4& c, float (&f)[In<DT>
 // tiled MFMA kernel
 // ---------------------------------------------------------------------------------------------
 // Sums an output is added up in where a wave owns one 32x32 block.  fp32: one for each step of a K tile, which also makes
-// them shorter (error against 64 bits of 4096 x 896 -> 512 2.7e-7, 3.8e-7 with two).  Two otherwise, and in the tiles with
+// them shorter (error against 64 bits of 4096 x 896 -> 512, when these tiles computed it, 2.7e-7, 3.8e-7 with two).  Two otherwise, and in the tiles with
 // a head, whose other registers are many: with four the 64x64 one takes 10.7 us for 17000 x 80 -> 40 instead of 10.3.
 template <int DT, int BM, int BN, int BK, int WM, int WN, int HEAD>
 constexpr int default_sums() {
@@ -733,12 +733,12 @@ __global__ __launch_bounds__(2 * kStreamCompute, 1) void bz_fc_stream_kernel(con
 //  - A lane's 16 bytes may start anywhere (a row pitch of 445 fp16 elements): the memory system takes such loads, and
 //    the lines they share are L1 hits.  So rows that start on no 16 bytes need no path of their own here.
 // Loaded straight into fragments a group of 16 lanes touches 16 lines, and the path into the CU takes a line a clock:
-// 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile); 32 x 2075 -> 768 fp32 17.0, 14.4 (51.7).
+// 128 x 4096 -> 1024 fp16 18.7 us, 9.1 this way (21.9 on the staged tile).
 constexpr int kSplitUnit = 128;
 // Where chunk `chunk` of row `row` lies.  2-byte operands: rows 16 bytes further apart than they are long, so that a fragment
 // read's sixteen lanes (one chunk of sixteen rows) are on all banks.  fp32, which moves twice the bytes for as many products:
-// rows side by side, their chunks in an order of the row's own, so that a write's (two rows) are as well (1024 x 896 -> 512
-// 14.6 us, 13.5 this way, 2048 x 512 -> 256 with a head 18.1 and 17.2; fp16 1024 x 896 -> 512 5.8 and 5.9).
+// rows side by side, their chunks in an order of the row's own, so that a write's (two rows) are as well (2048 x 512 -> 256 with a
+// head in its launch 18.1 us, 17.2 this way; fp16 1024 x 896 -> 512 5.8 and 5.9).
 template <int DT>
 constexpr int kSplitPitch = DT == BZ_F32 ? kSplitUnit : kSplitUnit + 16;
 template <int DT>
@@ -1489,8 +1489,10 @@ int launch_mfma(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st, void* c
 template <int DT, typename OutT, int NW>
 int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 31) / 32, tiles_n = (d.n + 31) / 32;
-  // (K of whole chunks has a tail without shifts and branches: 2000 x 144 -> 200 fp32 6.1 us, 5.6 this way)
-  const auto kernel = d.k % In<DT>::kChunk == 0 ? bz_fc_split_kernel<DT, OutT, NW, true> : bz_fc_split_kernel<DT, OutT, NW, false>;
+  // (K of whole chunks has a tail without shifts and branches.  fp32 layers come here with less than a chunk only.)
+  auto kernel = bz_fc_split_kernel<DT, OutT, NW, false>;
+  if constexpr (DT != BZ_F32)
+    if (d.k % In<DT>::kChunk == 0) kernel = bz_fc_split_kernel<DT, OutT, NW, true>;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a,
                      (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, tiles_m, ep);
   BZ_LAUNCH_OK("bz_fc_split_kernel");
