@@ -137,10 +137,12 @@ struct WarmWeights {
   static constexpr int kEach = 2;  // of the first layer, a thread's: its 0.9 MB where eight workgroups share an XCD
   uint32_t w[kEach + 1];
   __device__ __forceinline__ void ask(const Weights& w1, const Weights& w2) {
-    const uint32_t sharers = (gridDim.x + bz::kNumXcd - 1) / bz::kNumXcd, at = blockIdx.x / bz::kNumXcd * kThreads + threadIdx.x;
+    // (shares of a wave's 64 lines, so that few weights, too, are as many loads for each)
+    const uint32_t sharers = (gridDim.x + bz::kNumXcd - 1) / bz::kNumXcd, mine = blockIdx.x / bz::kNumXcd, wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    auto line = [&](uint32_t i) { return (int)((((i * kWaves + wave) * sharers + mine) * 64 + lane) * 128u); };
 #pragma unroll
-    for (int i = 0; i < kEach; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(w1.from, (int)((i * sharers * kThreads + at) * 128u), 0, 0);
-    w[kEach] = __builtin_amdgcn_raw_buffer_load_b32(w2.from, (int)(at * 128u), 0, 0);
+    for (int i = 0; i < kEach; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(w1.from, line(i), 0, 0);
+    w[kEach] = __builtin_amdgcn_raw_buffer_load_b32(w2.from, line(0), 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   }
   // (they have arrived by now; until here nobody has waited for them)
@@ -150,49 +152,52 @@ struct WarmWeights {
   }
 };
 
-// the rows' side of a group
+// the rows' side of half a group
 struct RowFragments {
-  uint4 x[kGroup];
-  __device__ __forceinline__ void read(const char* rows, int group) {
+  uint4 x[kGroup / 2];
+  __device__ __forceinline__ void read(const char* rows, int half) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j) x[j] = *(const uint4*)(rows + (((group * kGroup + j) * 2 + lane / 32) * kRows + lane % 32) * 16);
+    for (int j = 0; j < kGroup / 2; ++j) x[j] = *(const uint4*)(rows + (((half * (kGroup / 2) + j) * 2 + lane / 32) * kRows + lane % 32) * 16);
     __builtin_amdgcn_sched_barrier(0);
   }
 };
 
 // A layer's weights on their way through three sets of registers: two groups are asked for at its start, and one ahead of each
-// that is multiplied, 128 KB a CU under way; the rows' fragments are read a group ahead.  (2048 x 896 -> 512 -> 256 with two sets 15.1 us
-// alone as with three, 64 passes on eight serving threads 877 and 857; with four and five 16.0 and 15.9.)
+// that is multiplied, 128 KB a CU under way; the rows' fragments are read half a group ahead.  (2048 x 896 -> 512 -> 256 with two sets
+// 15.1 us alone as with three, 64 passes on eight serving threads 877 and 857; with four and five 16.0 and 15.9.)
 template <int TN>
 struct Layer {
   WeightStream<TN> w[3];
-  RowFragments r[3];
-  // An output's sums, of every second or fourth step of 16 inputs: two as in the tiles, and four where these were the split kernel's, with
-  // eight (896 -> 512 -> 256 -> 2: the model's error is that of two launches, with one sum 20 % more outputs are rounded to the other side).
-  static constexpr int kSums = TN == 1 ? 4 : 2;
-  floatx16 acc[TN], more[kSums - 1][TN];
+  RowFragments r[2];
+  // An output's two sums, of every other step of 16 inputs, as in the tiles.  (896 -> 512 -> 256 -> 2: the model's error is that of two
+  // launches; with one sum 20 % more outputs are rounded to the other side.  With fragments read a whole group ahead, or four sums, the
+  // kernel for one block of columns a wave does not fit 128 registers, and the attention model on eight threads, whose 162 -> 200 -> 80 it
+  // is, comes to 62 M samples/s for 66.)
+  floatx16 acc[TN], odd[TN];
   __device__ __forceinline__ void start(const Weights& from, int block) {
     w[0].ask(from, block, 0);
     w[1].ask(from, block, 1);
   }
-  __device__ __forceinline__ void multiply(int i) {
+  __device__ __forceinline__ void multiply(int i, int half) {
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j)
+    for (int j = 0; j < kGroup / 2; ++j)
 #pragma unroll
-      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[j][t], r[i].x[j], j % kSums == 0 ? acc[t] : more[(j + kSums - 1) % kSums][t]);
+      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[half * (kGroup / 2) + j][t], r[half].x[j], j % 2 == 0 ? acc[t] : odd[t]);
     __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void multiply(int i, const char* rows, int group) {
+    r[1].read(rows, group * 2 + 1);
+    multiply(i, 0);
+    r[0].read(rows, group * 2 + 2);
+    multiply(i, 1);
   }
   // acc = the weights' blocks times the rows.  (Behind the last group's fragments lie others: read, and not used.)
   __device__ __forceinline__ void run(const Weights& from, const char* rows, int block) {
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        acc[t][i] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kSums - 1; ++s) more[s][t][i] = 0.f;
-      }
+      for (int i = 0; i < 16; ++i) acc[t][i] = odd[t][i] = 0.f;
     const int groups = from.steps / kGroup;
     r[0].read(rows, 0);
     int g = 0;
@@ -200,20 +205,15 @@ struct Layer {
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         w[(i + 2) % 3].ask(from, block, g + i + 2);
-        r[(i + 1) % 3].read(rows, g + i + 1);
-        multiply(i);
+        multiply(i, rows, g + i);
       }
     }
-    if (g < groups) {
-      r[1].read(rows, g + 1);
-      multiply(0);
-      if (g + 1 < groups) multiply(1);
-    }
+    if (g < groups) multiply(0, rows, g);
+    if (g + 1 < groups) multiply(1, rows, g + 1);
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        acc[t][i] = kSums == 2 ? acc[t][i] + more[0][t][i] : (acc[t][i] + more[0][t][i]) + (more[1 % (kSums - 1)][t][i] + more[2 % (kSums - 1)][t][i]);
+      for (int i = 0; i < 16; ++i) acc[t][i] += odd[t][i];
   }
 };
 
