@@ -152,64 +152,68 @@ struct WarmWeights {
   }
 };
 
-// the rows' side of half a group
+// Not for a layer of one block of columns a wave: the loads of a word a line, and the registers, cost its short workgroups what they spare (eight
+// serving threads, 64 passes of 2595 rows, 104 -> 100 -> 100, 380 us with them and 360 without; a lone pass of 2048 x 26 lists, 896 -> 256 -> 104, 33.2
+// either way).
+struct NoWarming {
+  __device__ __forceinline__ void ask(const Weights&, const Weights&) {}
+  __device__ __forceinline__ void done() const {}
+};
+
+// the rows' side of a group
 struct RowFragments {
-  uint4 x[kGroup / 2];
-  __device__ __forceinline__ void read(const char* rows, int half) {
+  uint4 x[kGroup];
+  __device__ __forceinline__ void read(const char* rows, int group) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int j = 0; j < kGroup / 2; ++j) x[j] = *(const uint4*)(rows + (((half * (kGroup / 2) + j) * 2 + lane / 32) * kRows + lane % 32) * 16);
+    for (int j = 0; j < kGroup; ++j) x[j] = *(const uint4*)(rows + (((group * kGroup + j) * 2 + lane / 32) * kRows + lane % 32) * 16);
     __builtin_amdgcn_sched_barrier(0);
   }
 };
 
 // A layer's weights on their way through three sets of registers: two groups are asked for at its start, and one ahead of each
-// that is multiplied, 128 KB a CU under way; the rows' fragments are read half a group ahead.  (2048 x 896 -> 512 -> 256 with two sets
-// 15.1 us alone as with three, 64 passes on eight serving threads 877 and 857; with four and five 16.0 and 15.9.)
+// that is multiplied, 128 KB a CU under way; the rows' fragments are read a group ahead.  (2048 x 896 -> 512 -> 256 with two sets 15.1 us
+// alone as with three, 64 passes on eight serving threads 877 and 857; with four and five 16.0 and 15.9.)
 template <int TN>
 struct Layer {
   WeightStream<TN> w[3];
-  RowFragments r[2];
+  RowFragments r[3];
   // An output's two sums, of every other step of 16 inputs, as in the tiles.  (896 -> 512 -> 256 -> 2: the model's error is that of two
-  // launches; with one sum 20 % more outputs are rounded to the other side.  With fragments read a whole group ahead, or four sums, the
-  // kernel for one block of columns a wave does not fit 128 registers, and the attention model on eight threads, whose 162 -> 200 -> 80 it
-  // is, comes to 62 M samples/s for 66.)
+  // launches; with one sum 20 % more outputs are rounded to the other side.)
   floatx16 acc[TN], odd[TN];
   __device__ __forceinline__ void start(const Weights& from, int block) {
     w[0].ask(from, block, 0);
     w[1].ask(from, block, 1);
   }
-  __device__ __forceinline__ void multiply(int i, int half) {
+  __device__ __forceinline__ void multiply(int i) {
 #pragma unroll
-    for (int j = 0; j < kGroup / 2; ++j)
+    for (int j = 0; j < kGroup; ++j)
 #pragma unroll
-      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[half * (kGroup / 2) + j][t], r[half].x[j], j % 2 == 0 ? acc[t] : odd[t]);
+      for (int t = 0; t < TN; ++t) In<BZ_F16>::mma(w[i].w[j][t], r[i].x[j], j % 2 == 0 ? acc[t] : odd[t]);
     __builtin_amdgcn_sched_barrier(0);
-  }
-  __device__ __forceinline__ void multiply(int i, const char* rows, int group) {
-    r[1].read(rows, group * 2 + 1);
-    multiply(i, 0);
-    r[0].read(rows, group * 2 + 2);
-    multiply(i, 1);
   }
   // acc = the weights' blocks times the rows.  (Behind the last group's fragments lie others: read, and not used.)
   __device__ __forceinline__ void run(const Weights& from, const char* rows, int block) {
+    const int groups = from.steps / kGroup;
+    r[0].read(rows, 0);
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[t][i] = odd[t][i] = 0.f;
-    const int groups = from.steps / kGroup;
-    r[0].read(rows, 0);
     int g = 0;
     for (; g + 3 <= groups; g += 3) {  // (no branch around an ask: the waits behind it would be for everything)
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         w[(i + 2) % 3].ask(from, block, g + i + 2);
-        multiply(i, rows, g + i);
+        r[(i + 1) % 3].read(rows, g + i + 1);
+        multiply(i);
       }
     }
-    if (g < groups) multiply(0, rows, g);
-    if (g + 1 < groups) multiply(1, rows, g + 1);
+    if (g < groups) {
+      r[1].read(rows, g + 1);
+      multiply(0);
+      if (g + 1 < groups) multiply(1);
+    }
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -319,9 +323,10 @@ __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, c
   for (int g = kAhead * 2; g < groups; g += kAhead * 2) batch(g, nullptr);
 }
 
-// TN: blocks of 32 columns a wave holds of the first layer.  HN: outputs the skinny layer's code is unrolled for.  ODD: stage_rows'.
+// TN: blocks of 32 columns a wave holds of the first layer; with one, two workgroups share a CU (with more registers than that leaves, the
+// attention model on eight serving threads, whose 162 -> 200 -> 80 it is, comes to 62 M samples/s for 66).  HN: outputs the skinny layer's code is unrolled for.  ODD: stage_rows'.
 template <int TN, int HN, bool ODD>
-__global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a) {
+__global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(const Tower a) {
   typedef __half T;
   extern __shared__ __align__(16) char lds[];
   const Layout at = layout(a.k, a.n1, a.n2, HN);
@@ -344,7 +349,7 @@ __global__ __launch_bounds__(kThreads, 2) void bz_fc_tower_kernel(const Tower a)
     const int j = hj + i * (kThreads / kMaxNarrow);
     hw[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from_head, j < a.head.n && hc < a.n2 ? (j * (int)a.head.ldw + hc) * 2 : kBeyond, 0, 0);
   }
-  WarmWeights warm;
+  std::conditional_t<(TN > 1), WarmWeights, NoWarming> warm;
   stage_rows<ODD>(
       a, m0, lds,
       [&]() {
