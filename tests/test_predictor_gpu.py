@@ -1443,8 +1443,8 @@ def _tower(pb, ws, bs, acts, chain, heads):
 
 
 def _tower_pays(rows, k, n1, n2):
-    few = k * n1 + n1 * n2 <= 144 << 10
-    return rows <= 4096 and (k <= 1024 or few and k <= 1280) if rows >= 1200 else rows >= (1 if k <= 512 else 300) and k <= 1280 and few
+    weights = k * n1 + n1 * n2
+    return rows <= 4096 and k <= 1280 and (rows >= 1200 and k <= 1024 or weights <= (256 if k <= 768 or rows >= 600 and k <= 1024 else 144) << 10)
 
 
 def _tower_launches(p):
@@ -1534,8 +1534,9 @@ def test_tower_adds_up_as_finely_as_two_launches(pb):
 
 
 # both sides of each line of bz::fc_tower_pays, and of what the kernel takes
-@pytest.mark.parametrize("k,n1,n2,rows,one", [(512, 200, 80, 1, True), (513, 200, 80, 299, False), (513, 200, 80, 300, True), (896, 200, 80, 300, False),
-                                              (1280, 100, 40, 2048, True), (1280, 200, 80, 2048, False), (1024, 512, 256, 1199, False), (1024, 512, 256, 1200, True),
+@pytest.mark.parametrize("k,n1,n2,rows,one", [(1024, 100, 40, 1, True), (768, 256, 72, 1, True), (768, 320, 64, 1199, False), (776, 256, 72, 599, False),
+                                              (776, 256, 72, 600, True), (1024, 200, 80, 600, True), (1032, 128, 64, 300, True), (1032, 200, 80, 1200, False),
+                                              (1280, 100, 40, 2048, True), (1288, 40, 16, 2048, False), (1024, 512, 256, 1199, False), (1024, 512, 256, 1200, True),
                                               (896, 512, 256, 4096, True), (896, 512, 256, 4097, False), (64, 520, 64, 300, False), (64, 64, 264, 300, False)])
 def test_tower_launches(pb, k, n1, n2, rows, one):
     """the launches of a pass as it runs, with nothing timing its operators: one for a tower where that pays, else two or three"""

@@ -453,19 +453,25 @@ bool bz::fc_tower_takes(int64_t k, int64_t n1, int64_t n2) {
 }
 
 // One launch against two, in models that look 32-wide rows up for the input, us of a lone pass / of eight serving threads (weights in units
-// of 1024).  From 1200 rows on one launch is as fast alone and faster beside others, with inputs up to 1024:
+// of 1024): one where a lone pass is no longer, or by 2 % where the threads gain more.  From 1200 rows on that is with inputs up to 1024:
 //  896 -> 512 -> 256 (576) 1100 rows 37.8 / 9.9 and 37.7 / 9.3, 1300 39.0 / 9.2 and 39.2 / 10.5, 2048 39.4 / 10.3 and 39.6 / 11.9, 4096 47.2 / 18.8
-//  and 50.4 / 21.7; 1024 -> 512 -> 256 (640) 1600 41.1 / 10.5 and 40.8 / 12.1, 3000 45.0 / 16.2 and 47.6 / 18.8; 640 -> 400 -> 128 (300) 1300
-//  32.9 / 8.5 and 34.4 / 8.8; but 2048 of 1152 -> 512 -> 256 47.0 / 13.2 and 45.8 / 14.8, of 1216 -> 200 -> 80 41.9 / 11.6 and 40.4 / 13.2.
+//  and 50.4 / 21.7; 1024 -> 512 -> 256 (640) 1600 41.1 / 10.5 and 40.8 / 12.1, 3000 45.0 / 16.2 and 47.6 / 18.8; 1024 -> 256 -> 128 (288) 1300
+//  34.2 / 8.6 and 36.1 / 10.3; but 2048 of 1152 -> 512 -> 256 47.0 / 13.2 and 45.8 / 14.8, of 1216 -> 200 -> 80 41.9 / 11.6 and 40.4 / 13.2.
 // With fewer rows, and few workgroups to pull all the weights, where these are few:
-//  256 -> 200 -> 80 (65) one row 22.9 / 4.9 and 24.0 / 5.2, 1024 26.1 / 6.2 and 27.8 / 6.5; 448 -> 256 -> 100 (137) one row 24.0 / 5.1 and 23.8 / 5.3,
-//  300 28.0 / 6.2 and 28.7 / 6.9; 640 -> 200 -> 80 (140) 64 rows 27.7 / 5.8 and 26.7 / 6.0, 300 29.9 / 6.6 and 29.5 / 6.7; 1280 -> 100 -> 40 (128) 300
-//  33.5 / 7.8 and 35.3 / 8.3; but 300 of 1152 -> 128 -> 64 (152) 35.3 / 7.5 and 31.3 / 7.5, of 896 -> 200 -> 80 (190) 32.5 / 7.4 and 31.0 / 7.0, of
-//  896 -> 512 -> 256 38.5 / 9.7 and 33.7 / 8.0.  (Alone on hot weights one launch wins far beyond these lines: 300 of 896 -> 256 -> 104 9.8 and 10.4.)
-// Beyond 4096 rows two launches leave more to others (6000 of 896 -> 400 -> 128 on hot weights 15.5 us alone, 11.5 on four streams, and 21.4, 10.9).
+//  (256) with inputs up to 768, or up to 1024 from 600 rows on: 600 rows of 640 -> 256 -> 100 (185) 29.1 / 6.4 and 30.2 / 7.4, 768 -> 256 -> 100
+//   (217) 30.4 / 6.8 and 31.0 / 7.7, 352 -> 512 -> 100 (226) 30.1 / 6.6 and 31.1 / 7.6; 300 of them 29.2 / 6.2 and 29.7 / 6.8, 30.2 / 6.6 and
+//   30.2 / 7.0, 30.5 / 6.9 and 29.6 / 7.1; 64 (longer alone in the model, but not in a whole request: two samples of 730 -> 256 -> 256 looked up by key
+//   36.4 and 38.2) 27.4 / 5.5 and 26.7 / 6.0, 28.7 / 6.0 and 27.5 / 6.4, 29.2 / 5.6 and 26.7 / 6.2; 900 of 896 -> 200 -> 80 (190) 31.9 / 7.4 and
+//   32.5 / 7.9; but 300 of 896 -> 256 -> 104 (250) 32.6 / 7.4 and 31.7 / 7.0, 600 of 640 -> 400 -> 128 (300) 33.5 / 8.5 and 31.9 / 7.6;
+//  (144) any: 256 -> 200 -> 80 (65) 300 rows 24.0 / 5.3 and 26.5 / 6.2; 448 -> 256 -> 100 (137) one row 23.0 / 5.0 and 23.4 / 5.3, 300 26.6 / 5.8
+//   and 28.4 / 6.9; 640 -> 100 -> 256 (87) 203 27.3 / 5.8 and 31.6 / 7.3; 640 -> 200 -> 80 (140) 64 27.7 / 5.5 and 27.0 / 6.1; 1024 -> 128 -> 100 (140) 64
+//   28.7 / 6.0 and 28.2 / 6.2; 1280 -> 100 -> 40 (128) 300 33.2 / 7.1 and 35.3 / 7.8; but 64 of 1152 -> 128 -> 64 (152) 30.6 / 6.1 and 28.8 / 6.7.
+// (Alone on hot weights one launch wins far beyond these lines: 300 of 896 -> 256 -> 104 9.8 and 10.4.)  Beyond 4096 rows two launches leave
+// more to others (6000 of 896 -> 400 -> 128 on hot weights 15.5 us alone, 11.5 on four streams, and 21.4, 10.9).
 bool bz::fc_tower_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2) {
-  if (rows >= 1200) return rows <= 4096 && (k <= 1024 || (k <= 1280 && k * n1 + n1 * n2 <= 144 << 10));
-  return rows >= (k <= 512 ? 1 : 300) && k <= 1280 && k * n1 + n1 * n2 <= 144 << 10;
+  if (rows < 1 || rows > 4096 || k > 1280) return false;
+  const bool more = k <= 768 || (k <= 1024 && rows >= 600);
+  return (rows >= 1200 && k <= 1024) || k * n1 + n1 * n2 <= (more ? 256 << 10 : 144 << 10);
 }
 
 int bz::fc_tower(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
