@@ -869,9 +869,9 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
 // A workgroup owns a tile of 32 * TM x 32 * TN outputs and its NW waves share K, 16 at a time (stage t is wave t % NW's), each
 // working for itself: it loads a stage of the tile's rows straight into LDS of its own, reads fragments from there, splits them
 // into three bf16s a float (Bf16x3) and multiplies those; the partial tiles meet once, at the end.
-//  - The conversion, 11 vector instructions for two floats, is what bounds it, not the products: between 32-clock MFMAs the SIMD
-//    issues a vector instruction every five clocks, where 7.3 come to each MFMA of a 64x64 tile, and it does so only if a wave's
-//    own instructions alternate (beside another wave's MFMAs a wave of vector instructions gets one in 18 clocks).  So a step
+//  - The conversion, 11 vector instructions for two floats and one that keeps the largest of them, is what bounds it, not the products:
+//    between 32-clock MFMAs the SIMD issues a vector instruction every five clocks, where 8 come to each MFMA of a 64x64 tile, and it does
+//    so only if a wave's own instructions alternate (beside another wave's MFMAs a wave of vector instructions gets one in 18 clocks).  So a step
 //    multiplies one stage, converts the next and reads the one after, and tells the scheduler to alternate (with all conversions
 //    in front of the products, as they came, 2048 x 896 -> 512 took 17.5 us, with the read in front of them 16.2, this way 14.5).
 //  - That takes two sets of pieces in registers, and none are left for loads in flight: they go to LDS without any.

@@ -8,8 +8,9 @@
 // way; the rows, which all eight waves read, are in LDS.
 // us alone / a launch on four streams, two launches and this: 1024 of 198 -> 200 -> 80 -> 2 11.7 / 5.5 and 7.5 / 3.0, 300 of 445 -> 256 -> 100
 // 10.9 / 5.2 and 8.4 / 3.2, 2048 of 896 -> 512 -> 256 16.4 / 6.5 and 14.9 / 4.5 (of these 14.9: rows to LDS 2.9, first layer 6.3, its
-// activation 1.1, second layer and activation 2.1, skinny layer 0.9).  fp16 model of 2048 x 26 lists, us a lone pass / of eight serving threads:
-// 43.5 / 13.8 and 41.7 / 11.9.
+// activation 1.1, second layer and activation 2.1, skinny layer 0.9; since then 0.7 more with weights hot in L2, for a second sum an output and for
+// what WarmWeights takes, which gives 3.5 where they are not).  fp16 model of 2048 x 26 lists, us a lone pass / of eight serving threads: 43.6 / 13.9
+// and 41.8 / 11.9.
 #include <mutex>
 
 #include "fc_common.h"
