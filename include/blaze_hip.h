@@ -80,6 +80,26 @@ typedef struct bz_feed_rows {
 } bz_feed_rows;
 BZ_API int bz_feed(const void* src, void* dst, int64_t bytes, const bz_feed_rows* rows, int n_rows, bz_stream_t stream);
 
+/*
+ * bz_feed with a list of ranges (none of which overlap at dst), each of which may lie at its source in fewer bytes than it has
+ * at dst.  Every src that is read and every dst is 16-byte aligned, bytes is a multiple of 16, and where a source has no
+ * multiple of 16 bytes the rest of its last 16 are readable.
+ */
+#define BZ_FEED_MAX_PIECES 64
+enum bz_feed_form {
+  BZ_FEED_RAW = 0,   /* as it is */
+  BZ_FEED_LOW32 = 1, /* 64-bit words whose upper halves are zero: the lower halves side by side, bytes / 2 of them */
+  BZ_FEED_SAME32 = 2 /* one 32-bit word throughout: `word`; src is not read */
+};
+typedef struct bz_feed_piece {
+  const void* src;
+  void* dst;
+  int64_t bytes;
+  int32_t form;
+  uint32_t word;
+} bz_feed_piece;
+BZ_API int bz_feed_pieces(const bz_feed_piece* pieces, int n_pieces, const bz_feed_rows* rows, int n_rows, bz_stream_t stream);
+
 /* ------------------------------------------------------------------------- */
 /* Embedding                                                                  */
 /* ------------------------------------------------------------------------- */

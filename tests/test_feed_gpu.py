@@ -70,3 +70,66 @@ def test_feed_refuses():
     rows[0] = bz.FeedRows(p, p, 2, 8, 4, 8)                # rows that overlap
     assert call(None, None, 0, rows, 1, None) == bz.EINVAL
     assert C.sizeof(bz.FeedRows) == 48
+
+
+def _pieces(spec, gen):
+    """[(form, bytes)] -> (pieces, what lies at each destination before, what has to lie there after, what must stay alive)"""
+    pieces, dsts, wants, keep = (bz.FeedPiece * max(len(spec), 1))(), [], [], []
+    for i, (form, n) in enumerate(spec):
+        dst = torch.full((n + 16, ), 7, dtype=torch.uint8, device="cuda")
+        want = torch.full((n + 16, ), 7, dtype=torch.uint8)
+        word = int(torch.randint(1 << 31, (1, ), generator=gen)) * 2 + 1
+        if form == bz.FEED_SAME32:
+            want[:n] = torch.tensor([word - (1 << 32) if word >> 31 else word] * (n // 4), dtype=torch.int32).view(torch.uint8)
+            src = None
+        else:
+            src = torch.randint(256, ((n if form == bz.FEED_RAW else n // 2 + 15) // 16 * 16, ), generator=gen, dtype=torch.uint8).pin_memory()
+            if form == bz.FEED_RAW:
+                want[:n] = src
+            else:
+                want[:n].view(torch.int32).view(-1, 2).copy_(torch.stack([src[:n // 2].view(torch.int32), torch.zeros(n // 8, dtype=torch.int32)], 1))
+        pieces[i] = bz.FeedPiece(src.data_ptr() if src is not None and n else None, dst.data_ptr(), n, form, word)
+        dsts.append(dst)
+        wants.append(want)
+        keep.append(src)
+    return pieces, dsts, wants, keep
+
+
+RAW, LOW, SAME = 0, 1, 2
+
+
+@pytest.mark.parametrize("spec", [
+    [(LOW, 16)], [(SAME, 16)], [(RAW, 16)], [(RAW, 0), (LOW, 0), (SAME, 0), (LOW, 48)],  # the smallest, empty ones, an odd number of chunks
+    [(LOW, 8192 - 16), (LOW, 8192), (LOW, 8192 + 16)],         # a workgroup's worth at one unit a lane, and either side of it
+    [(SAME, 16384 - 16), (SAME, 16384), (SAME, 16384 + 16), (RAW, 4096), (RAW, 4112)],
+    [(LOW, (640 << 10) + 16), (RAW, 48), (SAME, 1 << 20)],     # two units a lane
+    [(LOW, 16384 - 16), (LOW, 16384 + 16), (RAW, 320 << 10)],
+    [((RAW, LOW, SAME)[k % 3], 16 * (1 + 37 * k)) for k in range(64)],  # as many as a launch takes
+])
+@pytest.mark.parametrize("rows", [False, True])
+def test_feed_pieces(spec, rows):
+    gen = torch.Generator().manual_seed(len(spec) + 1000 * spec[0][1])
+    pieces, dsts, wants, keep = _pieces(spec, gen)
+    strided = (bz.FeedRows * 2)()
+    src = torch.randint(256, (2, 9 * 26), generator=gen, dtype=torch.uint8).pin_memory()
+    dst = torch.full((2, 9 * 890), 9, dtype=torch.uint8, device="cuda")
+    for i in range(2):
+        strided[i] = bz.FeedRows(src[i].data_ptr(), dst[i].data_ptr(), 9, 26, 26, 890)
+    bz.check(bz.lib().bz_feed_pieces(pieces, len(spec), strided, 2 if rows else 0, bz._stream_ptr()))
+    for got, want, piece in zip(dsts, wants, spec):
+        assert torch.equal(got.cpu(), want), piece
+    want = torch.full((2, 9, 890), 9, dtype=torch.uint8)
+    if rows:
+        want[:, :, :26] = src.view(2, 9, 26)
+    assert torch.equal(dst.cpu().view(2, 9, 890), want)
+
+
+def test_feed_pieces_refuses():
+    buf = torch.zeros(64, dtype=torch.uint8).pin_memory()
+    p, call = buf.data_ptr(), bz.lib().bz_feed_pieces
+    many = (bz.FeedPiece * 65)()
+    assert call(many, 65, None, 0, None) == bz.EINVAL
+    for bad in ((p, p, 24, RAW), (p + 4, p, 16, LOW), (p, p + 8, 16, LOW), (None, p, 16, RAW), (None, p, 16, LOW), (p, None, 16, SAME), (p, p, 16, 3),
+                (p, p, -16, SAME)):
+        many[0] = bz.FeedPiece(*bad, 0)
+        assert call(many, 1, None, 0, None) == bz.EINVAL, bad

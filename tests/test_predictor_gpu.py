@@ -1415,6 +1415,44 @@ def test_feed_many_at_the_borders_of_its_parts(pb, sizes):
             np.testing.assert_allclose(p.output_asnumpy("y%d" % k).reshape(-1), _sigmoid(x).reshape(-1), rtol=1e-5)
 
 
+# 64-bit ids cross as their lower halves and equal 32-bit words as one, in blocks of 1024 words: the word that does not fit stands at
+# the edges of blocks and parts, at the end, or nowhere
+@pytest.mark.parametrize("n,odd", [(1, []), (255, []), (256, []), (1023, [1022]), (1024, []), (1025, [1024]), (5000, [7]), (5000, [8]), (5000, [1023]),
+                                   (5000, [1024]), (5000, [4999]), (5000, [2048, 3000]), (49152, [49151]), (49153, [49152]), (200001, [131072]), (700000, [])])
+def test_feed_many_of_words_that_are_packed(pb, n, odd):
+    import torch
+    rng = np.random.default_rng(n)
+    nb = pb.NetBuilder("packed", device_type=1)
+    kinds = {"ids": pb.K_INT64, "before": pb.K_FLOAT, "values": pb.K_FLOAT, "counts": pb.K_INT32, "more": pb.K_INT64}
+    nb.constant("flat", np.array([-1], np.int32))
+    for name, code in kinds.items():
+        nb.external_input(name, code)
+        nb.op("Reshape", [name, "flat"], ["flat_" + name])
+        nb.external_output("flat_" + name, code)
+    nb.external_input("x", pb.K_FLOAT)
+    nb.op("Sigmoid", ["x"], ["y"])
+    nb.external_output("y", pb.K_FLOAT)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for turn in range(3):
+        ids = rng.integers(0, 1 << 32, n, dtype=np.int64)
+        more = rng.integers(-1 << 62, 1 << 62, n // 3 + 1, dtype=np.int64)
+        values, counts = np.full(n, -0.0 if turn else np.nan, np.float32), np.full(n, 255, np.int32)
+        for k in odd if turn < 2 else []:
+            ids[k] = -1 - k if turn else ids[k] + (1 << 32)
+            values[k], counts[k] = 0.0 if turn else 1.0, -255
+        feed = {"ids": ids, "before": rng.standard_normal(67).astype(np.float32), "values": values, "counts": counts, "more": more, "x": values[:3].copy()}
+        for name, a in feed.items():
+            p.reshape_input(name, a.shape)
+        p.feed_many(p.feed_batch(list(feed.items())))
+        p.forward()
+        for name in kinds:
+            there = dict(shape=feed[name].shape, typestr=feed[name].dtype.str, data=(p.input_device_ptr(name), False), version=3, strides=None)
+            got = torch.as_tensor(type("View", (), dict(__cuda_array_interface__=there))(), device="cuda").cpu().numpy()
+            assert got.tobytes() == feed[name].tobytes(), (turn, name)
+
+
 def _tower(pb, ws, bs, acts, chain, heads):
     nb = pb.NetBuilder("tower%d" % chain, device_type=1)
     nb.arg("chain_narrow_fcs", chain)

@@ -23,7 +23,7 @@ EXPORTS = [
     "bz_last_error", "bz_device_check", "bz_table_pitch", "bz_embed_plan", "bz_segments_to_offsets", "bz_segments_to_offsets_slots",
     "bz_embed_pool", "bz_embed_pool_args", "bz_embed_pool_static_scratch", "bz_embed_pool_kernel_name", "bz_fc_fused", "bz_fc_head_apart", "bz_fc_pack_weight", "bz_gemm_strided_batched", "bz_weighted_pool",
     "bz_activation", "bz_concat_cols", "bz_broadcast_op", "bz_reduce_sum", "bz_batch_norm", "bz_softmax_axis",
-    "bz_concat_ew", "bz_gather_rows", "bz_spin", "bz_feed"
+    "bz_concat_ew", "bz_gather_rows", "bz_spin", "bz_feed", "bz_feed_pieces"
 ]
 EW_ADD, EW_SUB, EW_MUL, EW_DIV, EW_ASSIGN, EW_WHERE = 0, 1, 2, 3, 4, 5
 OK, EINVAL, ENOTSUP, EHIP = 0, -22, -95, -5  # bz_status
@@ -43,6 +43,13 @@ class EmbedSlot(C.Structure):
 class FeedRows(C.Structure):
     _fields_ = [("src", C.c_void_p), ("dst", C.c_void_p), ("rows", C.c_int64), ("row_bytes", C.c_int64), ("src_pitch", C.c_int64),
                 ("dst_pitch", C.c_int64)]
+
+
+FEED_RAW, FEED_LOW32, FEED_SAME32 = 0, 1, 2  # enum bz_feed_form
+
+
+class FeedPiece(C.Structure):
+    _fields_ = [("src", C.c_void_p), ("dst", C.c_void_p), ("bytes", C.c_int64), ("form", C.c_int32), ("word", C.c_uint32)]
 
 
 class EmbedLaunch(C.Structure):
@@ -137,6 +144,7 @@ def lib():
         l.bz_embed_plan.argtypes = [C.POINTER(EmbedSlot), C.c_int, C.POINTER(EmbedLaunch)]
         l.bz_spin.argtypes = [i64, vp]
         l.bz_feed.argtypes = [vp, vp, i64, C.POINTER(FeedRows), C.c_int, vp]
+        l.bz_feed_pieces.argtypes = [C.POINTER(FeedPiece), C.c_int, C.POINTER(FeedRows), C.c_int, vp]
         l.bz_segments_to_offsets.argtypes = [vp, vp, i64, vp]
         l.bz_segments_to_offsets_slots.argtypes = [vp, C.c_int, vp]
         l.bz_embed_pool.argtypes = [vp, C.POINTER(EmbedLaunch), vp]

@@ -5,6 +5,7 @@
 #include <chrono>
 #include <type_traits>
 
+#include "blaze/feed_pack.h"
 #include "blaze/qed_store.h"
 #include "blaze_hip.h"
 
@@ -188,6 +189,11 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
 // what follows it on the stream may start: 5 MB in ten parts arrived 230 us after the first byte was staged, in one part behind
 // the whole staging 210, through five launches of the kernel 162.)
 constexpr size_t kFeedFirst = 384 << 10, kFeedMost = 1 << 20, kFeedLong = 4 << 20;
+// Inputs of this many bytes are staged in the form that crosses in fewest (feed_pack.h), if one fits; smaller ones would make
+// more ranges than they save.  us a request, as they are / packed: 5.1 MB of ids below 2^32 and values of 1 199 / 134..160, with keys of 62
+// bits for ids 205 / 182, 10 MB 450 / 360, 1.07 MB 86.6 / 72, 0.7 MB 64.5 / 51 (keys: 72 / 65); of any values and keys, where nothing fits,
+// 220 / 215.
+constexpr size_t kPackFrom = 2 << 10;
 
 // a transfer has been queued on the context's stream
 void Predictor::FeedQueued(const HIPContext& ctx) {
@@ -299,12 +305,14 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
     // from the first launch on the arena is being read: whatever happens next, it is waited for before it is written again
     try {
       bz_feed_rows rows[BZ_FEED_MAX_ROWS];
-      size_t moved = 0, part = plain < kFeedLong ? kFeedFirst : (plain / (plain / kFeedMost) / 256 + 1) * 256;
-      int n = 0;
+      bz_feed_piece pieces[BZ_FEED_MAX_PIECES];
+      int n = 0, n_pieces = 0;
+      size_t moved = 0, staged = 0;  // bytes of the device arena whose transfer has been launched; of the staging arena in use
+      size_t part = plain < kFeedLong ? kFeedFirst : (plain / (plain / kFeedMost) / 256 + 1) * 256;
       auto launch = [&](size_t upto) {
-        BZ_CHECK(bz_feed(arena_host_ + moved, arena_dev_ + moved, (int64_t)(upto - moved), rows, n, st));
+        BZ_CHECK(bz_feed_pieces(pieces, n_pieces, rows, n, st));
         moved = upto;
-        n = 0;
+        n = n_pieces = 0;
       };
       auto end_of_part = [&]() { return plain - moved < part + part / 2 ? plain : moved + part; };
       size_t end = end_of_part();
@@ -313,19 +321,49 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
         memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
         rows[n++] = StridedRows(external_input_blob_[it.idx], arena_host_ + it.offset);
       }
-      for (const Item& it : in_arena)
-        for (size_t at = 0; at < lens[it.arg];) {
-          // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte)
-          const size_t len = std::min(lens[it.arg] - at, end - (it.offset + at));
-          memcpy(arena_host_ + it.offset + at, (const char*)data[it.arg] + at, len);
-          at += len;
+      // `bytes` of the device arena from `at` on, of which `source` bytes have been staged
+      auto add = [&](size_t at, size_t bytes, int form, uint32_t word, size_t source) {
+        char *from = arena_host_ + staged, *to = arena_dev_ + at;
+        staged += source;
+        bz_feed_piece* last = n_pieces > 0 ? &pieces[n_pieces - 1] : nullptr;
+        if (last && form == BZ_FEED_RAW && last->form == BZ_FEED_RAW && (const char*)last->src + last->bytes == from && (char*)last->dst + last->bytes == to) {
+          last->bytes += bytes;
+          return;
+        }
+        if (n_pieces == BZ_FEED_MAX_PIECES) launch(at);
+        pieces[n_pieces++] = {from, to, (int64_t)bytes, form, word};
+      };
+      auto up = [](size_t bytes, size_t to) { return (bytes + to - 1) / to * to; };
+      for (const Item& it : in_arena) {
+        const size_t len = lens[it.arg];
+        const size_t word = len >= kPackFrom ? DataTypeSize(external_input_blob_[it.idx]->data_type()) : 0;
+        bool packs = word == 8 || word == 4;
+        uint32_t first = 0;
+        if (packs) memcpy(&first, data[it.arg], 4);
+        for (size_t at = 0; at < len;) {
+          // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte; and staged <= it.offset + at)
+          const char* from = (const char*)data[it.arg] + at;
+          const size_t left = std::min(len - at, end - (it.offset + at));
+          size_t now = 0;
+          if (packs) {
+            now = word * (word == 8 ? PackLow32((uint32_t*)(arena_host_ + staged), (const uint64_t*)from, left / 8) : CountSame32(from, left / 4, first));
+            packs = now == left;
+            if (now > 0) add(it.offset + at, up(now, 16), word == 8 ? BZ_FEED_LOW32 : BZ_FEED_SAME32, first, word == 8 ? up(now / 2, 256) : 0);
+          }
+          if (now == 0) {
+            now = left;
+            memcpy(arena_host_ + staged, from, now);
+            add(it.offset + at, up(now, 256), BZ_FEED_RAW, 0, up(now, 256));
+          }
+          at += now;
           if (it.offset + at == end) {
             launch(end);
             if (plain < kFeedLong) part = std::min(part + part / 2, kFeedMost);
             end = end_of_part();
           }
         }
-      if (plain > moved || n > 0) launch(plain);
+      }
+      if (n_pieces > 0 || n > 0) launch(plain);
       FeedQueued(ctx);
     } catch (...) {
       (void)hipStreamSynchronize(st);  // no event stands behind what was launched

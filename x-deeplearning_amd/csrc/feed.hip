@@ -24,15 +24,32 @@ namespace {
 constexpr int kFeedThreads = 256;
 constexpr int64_t kFeedOneUnit = 320 << 10;  // bytes up to which a lane asks for one
 
-struct FeedArgs {
+// 16-byte stores of a lane in a range of one repeated word, which reads nothing
+constexpr int kSameUnits = 4;
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (arrays of HIP's uint4 ended up in LDS, one load waited for at a time)
+
+struct FeedRange {
   const char* src;
   char* dst;
-  int64_t chunks;  // 16-byte chunks of the contiguous range
-  int range_wg;    // workgroups that copy it
+  int64_t chunks;  // 16-byte chunks at dst
+  int32_t form;
+  uint32_t word;
+  int32_t wg_begin;  // workgroups of the ranges before it
+};
+
+// N: ranges that the launch has room for
+template <int N>
+struct FeedArgs {
+  FeedRange r[N];
+  int wg_end[N];  // workgroups of the ranges up to and including this one
+  int n_ranges;
+  int range_wg;  // of all of them
   int n;
   bz_feed_rows p[BZ_FEED_MAX_ROWS];
-  int unit[BZ_FEED_MAX_ROWS];    // widest power of two (<= 16) that divides addresses, pitches and row length
-  int wg_end[BZ_FEED_MAX_ROWS];  // workgroups of the range and of the pieces up to and including this one
+  int unit[BZ_FEED_MAX_ROWS];     // widest power of two (<= 16) that divides addresses, pitches and row length
+  int row_end[BZ_FEED_MAX_ROWS];  // workgroups of the ranges and of the strided pieces up to and including this one
 };
 
 template <typename U, int UNITS>
@@ -59,58 +76,102 @@ __device__ __forceinline__ void feed_rows(const bz_feed_rows& p, int64_t first) 
 }
 
 template <int UNITS>
-__global__ __launch_bounds__(kFeedThreads) void bz_feed_kernel(const FeedArgs a) {
+__device__ __forceinline__ void feed_raw(const FeedRange& r, int wg) {
+  const u32x4* src = (const u32x4*)r.src;
+  u32x4* dst = (u32x4*)r.dst;
+  const int64_t i0 = (int64_t)wg * (kFeedThreads * UNITS) + (int)threadIdx.x;
+  u32x4 v[UNITS];
+#pragma unroll
+  for (int k = 0; k < UNITS; ++k) v[k] = src[min(i0 + k * kFeedThreads, r.chunks - 1)];
+#pragma unroll
+  for (int k = 0; k < UNITS; ++k)
+    if (i0 + k * kFeedThreads < r.chunks) dst[i0 + k * kFeedThreads] = v[k];
+}
+
+template <int UNITS>
+__device__ __forceinline__ void feed_low32(const FeedRange& r, int wg) {
+  const u32x4* src = (const u32x4*)r.src;
+  u32x4* dst = (u32x4*)r.dst;
+  const int64_t units = (r.chunks + 1) >> 1;  // 16 bytes at the source are 32 here
+  const int64_t i0 = (int64_t)wg * (kFeedThreads * UNITS) + (int)threadIdx.x;
+  u32x4 v[UNITS];
+#pragma unroll
+  for (int k = 0; k < UNITS; ++k) v[k] = src[min(i0 + k * kFeedThreads, units - 1)];
+#pragma unroll
+  for (int k = 0; k < UNITS; ++k) {
+    const int64_t i = i0 + k * kFeedThreads;
+    if (i < units) dst[2 * i] = u32x4{v[k].x, 0, v[k].y, 0};
+    if (2 * i + 1 < r.chunks) dst[2 * i + 1] = u32x4{v[k].z, 0, v[k].w, 0};
+  }
+}
+
+__device__ __forceinline__ void feed_same32(const FeedRange& r, int wg) {
+  u32x4* dst = (u32x4*)r.dst;
+  const int64_t i0 = (int64_t)wg * (kFeedThreads * kSameUnits) + (int)threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kSameUnits; ++k)
+    if (i0 + k * kFeedThreads < r.chunks) dst[i0 + k * kFeedThreads] = u32x4{r.word, r.word, r.word, r.word};
+}
+
+template <int UNITS, int N>
+__global__ __launch_bounds__(kFeedThreads) void bz_feed_kernel(const FeedArgs<N> a) {
   const int wg = (int)blockIdx.x;
   if (wg < a.range_wg) {
-    const uint4* src = (const uint4*)a.src;
-    uint4* dst = (uint4*)a.dst;
-    const int64_t i0 = (int64_t)wg * (kFeedThreads * UNITS) + threadIdx.x;
-    uint4 v[UNITS];
-#pragma unroll
-    for (int k = 0; k < UNITS; ++k) {
-      const int64_t i = i0 + k * kFeedThreads;
-      v[k] = src[i < a.chunks ? i : a.chunks - 1];
+    if (N == 1) {
+      feed_raw<UNITS>(a.r[0], wg);
+      return;
     }
-#pragma unroll
-    for (int k = 0; k < UNITS; ++k) {
-      const int64_t i = i0 + k * kFeedThreads;
-      if (i < a.chunks) dst[i] = v[k];
-    }
+    // which range: every lane looks at one, in one trip to the arguments
+    const int lane = (int)threadIdx.x & (bz::kWave - 1);
+    const int q = __popcll(__ballot(lane < a.n_ranges && wg >= a.wg_end[min(lane, N - 1)]));
+    const FeedRange r = a.r[__builtin_amdgcn_readfirstlane(q)];
+    if (r.form == BZ_FEED_RAW)
+      feed_raw<UNITS>(r, wg - r.wg_begin);
+    else if (r.form == BZ_FEED_LOW32)
+      feed_low32<UNITS>(r, wg - r.wg_begin);
+    else
+      feed_same32(r, wg - r.wg_begin);
     return;
   }
   int q = 0;
-  while (q < a.n - 1 && wg >= a.wg_end[q]) ++q;  // (uniform; at most BZ_FEED_MAX_ROWS steps)
+  while (q < a.n - 1 && wg >= a.row_end[q]) ++q;  // (uniform; at most BZ_FEED_MAX_ROWS steps)
   const bz_feed_rows p = a.p[q];
-  const int64_t first = (int64_t)(wg - (q == 0 ? a.range_wg : a.wg_end[q - 1])) * (kFeedThreads * UNITS);
+  const int64_t first = (int64_t)(wg - (q == 0 ? a.range_wg : a.row_end[q - 1])) * (kFeedThreads * UNITS);
   switch (a.unit[q]) {
-    case 16: feed_rows<uint4, UNITS>(p, first); break;
-    case 8: feed_rows<uint2, UNITS>(p, first); break;
+    case 16: feed_rows<u32x4, UNITS>(p, first); break;
+    case 8: feed_rows<u32x2, UNITS>(p, first); break;
     case 4: feed_rows<uint32_t, UNITS>(p, first); break;
     case 2: feed_rows<uint16_t, UNITS>(p, first); break;
     default: feed_rows<uint8_t, UNITS>(p, first); break;
   }
 }
 
-}  // namespace
-
-extern "C" int bz_feed(const void* src, void* dst, int64_t bytes, const bz_feed_rows* rows, int n_rows, bz_stream_t stream) {
-  BZ_REQUIRE(bytes >= 0 && n_rows >= 0 && n_rows <= BZ_FEED_MAX_ROWS && (n_rows == 0 || rows != nullptr),
-             "bz_feed: bytes=%lld n_rows=%d (at most %d)", (long long)bytes, n_rows, BZ_FEED_MAX_ROWS);
-  BZ_REQUIRE(bytes == 0 || (src != nullptr && dst != nullptr && bytes % 16 == 0 && (((uintptr_t)src | (uintptr_t)dst) & 15) == 0),
-             "bz_feed: the contiguous range needs 16-byte aligned addresses and a multiple of 16 bytes (%lld)", (long long)bytes);
-  FeedArgs a = {};
-  a.src = (const char*)src;
-  a.dst = (char*)dst;
-  a.chunks = bytes / 16;
-  int64_t all = bytes;
+// the arguments from checked pieces, and the launch
+template <int N>
+int launch_feed(const bz_feed_piece* pieces, int n_pieces, const bz_feed_rows* rows, int n_rows, bz_stream_t stream) {
+  FeedArgs<N> a = {};
+  int64_t all = 0;  // what is read
+  for (int i = 0; i < n_pieces; ++i) all += pieces[i].form == BZ_FEED_RAW ? pieces[i].bytes : pieces[i].form == BZ_FEED_LOW32 ? pieces[i].bytes / 2 : 0;
   for (int i = 0; i < n_rows; ++i) {
     const bz_feed_rows& p = rows[i];
     if (p.rows > 0 && p.row_bytes > 0) all += p.rows < (1ll << 40) / p.row_bytes ? p.rows * p.row_bytes : 1ll << 40;
   }
   const int units = all <= kFeedOneUnit ? 1 : all <= (1ll << 30) ? 2 : 4;  // (four for the sake of the grid's size)
   const int64_t span = kFeedThreads * units;
-  int64_t wg = (a.chunks + span - 1) / span;
-  BZ_REQUIRE(wg < (1ll << 30), "bz_feed: %lld bytes make too many workgroups", (long long)bytes);
+  int64_t wg = 0;
+  for (int i = 0; i < n_pieces; ++i) {
+    const bz_feed_piece& p = pieces[i];
+    if (p.bytes == 0) continue;
+    const int64_t chunks = p.bytes / 16;
+    FeedRange& r = a.r[a.n_ranges];
+    r = {(const char*)p.src, (char*)p.dst, chunks, p.form, p.word, (int32_t)wg};
+    if (p.form == BZ_FEED_SAME32)
+      wg += (chunks + kFeedThreads * kSameUnits - 1) / (kFeedThreads * kSameUnits);
+    else
+      wg += ((p.form == BZ_FEED_LOW32 ? (chunks + 1) / 2 : chunks) + span - 1) / span;
+    BZ_REQUIRE(wg < (1ll << 30), "bz_feed: %lld bytes make too many workgroups", (long long)p.bytes);
+    a.wg_end[a.n_ranges++] = (int)wg;
+  }
   a.range_wg = (int)wg;
   for (int i = 0; i < n_rows; ++i) {
     const bz_feed_rows& p = rows[i];
@@ -127,11 +188,39 @@ extern "C" int bz_feed(const void* src, void* dst, int64_t bytes, const bz_feed_
     BZ_REQUIRE(wg < (1ll << 30), "bz_feed: piece %d makes too many workgroups", i);
     a.p[a.n] = p;
     a.unit[a.n] = unit;
-    a.wg_end[a.n] = (int)wg;
+    a.row_end[a.n] = (int)wg;
     ++a.n;
   }
   if (wg == 0) return BZ_OK;
-  hipLaunchKernelGGL(units == 1 ? bz_feed_kernel<1> : units == 2 ? bz_feed_kernel<2> : bz_feed_kernel<4>, dim3((int)wg), dim3(kFeedThreads), 0, bz::as_stream(stream), a);
+  hipLaunchKernelGGL((units == 1 ? bz_feed_kernel<1, N> : units == 2 ? bz_feed_kernel<2, N> : bz_feed_kernel<4, N>), dim3((int)wg),
+                     dim3(kFeedThreads), 0, bz::as_stream(stream), a);
   BZ_LAUNCH_OK("bz_feed_kernel");
   return BZ_OK;
+}
+
+}  // namespace
+
+extern "C" int bz_feed(const void* src, void* dst, int64_t bytes, const bz_feed_rows* rows, int n_rows, bz_stream_t stream) {
+  const bz_feed_piece range = {src, dst, bytes, BZ_FEED_RAW, 0};
+  return bz_feed_pieces(&range, 1, rows, n_rows, stream);
+}
+
+extern "C" int bz_feed_pieces(const bz_feed_piece* pieces, int n_pieces, const bz_feed_rows* rows, int n_rows, bz_stream_t stream) {
+  BZ_REQUIRE(n_rows >= 0 && n_rows <= BZ_FEED_MAX_ROWS && (n_rows == 0 || rows != nullptr), "bz_feed: n_rows=%d (at most %d)", n_rows,
+             BZ_FEED_MAX_ROWS);
+  BZ_REQUIRE(n_pieces >= 0 && n_pieces <= BZ_FEED_MAX_PIECES && (n_pieces == 0 || pieces != nullptr), "bz_feed: n_pieces=%d (at most %d)", n_pieces,
+             BZ_FEED_MAX_PIECES);
+  bool one = true;
+  for (int i = 0; i < n_pieces; ++i) {
+    const bz_feed_piece& p = pieces[i];
+    BZ_REQUIRE(p.form == BZ_FEED_RAW || p.form == BZ_FEED_LOW32 || p.form == BZ_FEED_SAME32, "bz_feed: form %d", p.form);
+    BZ_REQUIRE(p.bytes >= 0 && p.bytes < (1ll << 44), "bz_feed: %lld bytes make too many workgroups", (long long)p.bytes);
+    const bool read = p.form != BZ_FEED_SAME32;
+    BZ_REQUIRE(p.bytes == 0 || (p.dst != nullptr && (!read || p.src != nullptr) && p.bytes % 16 == 0 && ((uintptr_t)p.dst & 15) == 0 &&
+                                (!read || ((uintptr_t)p.src & 15) == 0)),
+               "bz_feed: a contiguous range needs 16-byte aligned addresses and a multiple of 16 bytes (%lld)", (long long)p.bytes);
+    one = one && p.form == BZ_FEED_RAW;
+  }
+  return n_pieces <= 1 && one ? launch_feed<1>(pieces, n_pieces, rows, n_rows, stream)
+                              : launch_feed<BZ_FEED_MAX_PIECES>(pieces, n_pieces, rows, n_rows, stream);
 }
