@@ -707,3 +707,26 @@ def test_kassign_beside_sums_of_one_row_shape(bz, oracle, kind, dims, keyed, out
             assert np.array_equal(np.isnan(got), np.isnan(ref)), (fused, args, i)
             ok = ~np.isnan(ref)
             assert np.array_equal(_bits(got[ok]), _bits(ref[ok])), (fused, args, i)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("dim", [4, 8, 16, 32, 64, 128, 256])  # 1 to 64 lanes a row
+def test_the_longest_segment_of_a_wave_wherever_it_lies(bz, oracle, dim, fused, mixed):
+    """A wave walks as many steps as its longest segment takes: in each lane group of a wave in turn, the last wave of a batch whole
+    and with one group only (the lanes behind it have no sample).  mixed: beside a kassign item, in the kernel for both."""
+    rng = np.random.default_rng(dim)
+    lpr = dim // 4
+    groups = 64 // lpr  # samples a wave
+    t = _make_table(rng, "f32", 50, dim, False)
+    for batch in (groups, groups + 1, 2 * groups):
+        for long_at in {0, groups // 2, groups - 1, batch - 1}:
+            seg = rng.integers(0, 3, batch).astype(np.int32)
+            seg[long_at] = 23
+            ids = rng.integers(0, 50, int(seg.sum())).astype(np.int64)
+            inputs = [(ids, rng.standard_normal(ids.size).astype(np.float32), seg)] * (1 + mixed)
+            specs = [(0, 0, 0, 0, dim)] + [(0, 2, 0, 2, dim)] * mixed
+            cols = (dim * (1 + 2 * mixed), [0, dim][:1 + mixed])
+            got, _, _ = _run_gpu(bz, [t], specs, inputs, batch, np.float32, cols, fused_scan=fused)
+            want = _run_oracle(oracle, [t], specs, inputs, batch, cols)
+            assert np.array_equal(_bits(got), _bits(want)), (batch, long_at)

@@ -185,10 +185,9 @@ struct Stage {
 };
 
 template <int DT, bool TA, bool TB, int G>
-__global__ __launch_bounds__(256) void bz_bgemm_mfma_kernel(const char* __restrict__ A, const char* __restrict__ B,
-                                                            typename Elem<DT>::T* __restrict__ C, int64_t sa, int64_t sb, int64_t sc,
-                                                            int M, int N, int K, int batch, int tiles_m, int tiles_n, int total_wg,
-                                                            int wg_per_xcd, float alpha, float beta) {
+__global__ __launch_bounds__(256) void bz_bgemm_mfma_kernel(const char* __restrict__ A, const char* __restrict__ B, int64_t sa, int64_t sb,
+                                                            int M, int N, int K, int tiles, int total_wg, int wg_per_xcd, int batch,
+                                                            typename Elem<DT>::T* __restrict__ C, int64_t sc, float alpha, float beta) {
   typedef typename Elem<DT>::T T;
   typedef bz::fc::In<DT> IN;
   constexpr int ES = IN::kSize;
@@ -199,9 +198,10 @@ __global__ __launch_bounds__(256) void bz_bgemm_mfma_kernel(const char* __restri
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tile = v % (tiles_m * tiles_n);
-  const int mine = v / (tiles_m * tiles_n) * G + (G == 1 ? 0 : wave);
-  const bool live = mine < batch;
+  const int tiles_n = (N + TILE - 1) / TILE;
+  const int tile = v % tiles;
+  const int mine = v / tiles * G + (G == 1 ? 0 : wave);
+  const bool live = G == 1 || mine < batch;
   const int64_t item = live ? mine : batch - 1;  // (a wave without an item of its own meets the barriers and stores nothing)
   const int t = G == 1 ? threadIdx.x : lane;
   const int m0 = tile / tiles_n * TILE, n0 = tile % tiles_n * TILE;
@@ -271,8 +271,8 @@ int launch_bgemm(const bz_bgemm_desc& d, hipStream_t s) {
   const int per_xcd = (int)((total + bz::kNumXcd - 1) / bz::kNumXcd);
 #define BZ_BGEMM(TA, TB, G)                                                                                                        \
   hipLaunchKernelGGL((bz_bgemm_mfma_kernel<DT, TA, TB, G>), dim3(per_xcd * bz::kNumXcd), dim3(256), 0, s, (const char*)d.a,        \
-                     (const char*)d.b, (T*)d.c, d.stride_a, d.stride_b, d.stride_c, d.m, d.n, d.k, d.batch, (int)tiles_m,          \
-                     (int)tiles_n, (int)total, per_xcd, d.alpha, d.beta)
+                     (const char*)d.b, d.stride_a, d.stride_b, d.m, d.n, d.k, (int)(tiles_m * tiles_n), (int)total, per_xcd,        \
+                     d.batch, (T*)d.c, d.stride_c, d.alpha, d.beta)
 #define BZ_BGEMM_G(TA, TB) \
   if (small)               \
     BZ_BGEMM(TA, TB, 4);   \

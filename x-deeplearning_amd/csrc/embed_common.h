@@ -495,12 +495,19 @@ struct RowStream {
   }
 };
 
-// steps of the wave's longest segment, n being this lane's
+// Steps of the wave's longest segment, n being this lane's (the same in the LPR lanes of a group; every lane of the wave takes
+// part).  The maximum ends up in lane 63, by DPP operands as in wave_scan_sat: through LDS it was up to six dependent trips of 120
+// clocks in front of every walk.
 template <int LPR>
 __device__ __forceinline__ int wave_steps(int n) {
-#pragma unroll
-  for (int d = bz::kWave / 2; d >= LPR; d >>= 1) n = max(n, __shfl_xor(n, d, bz::kWave));
-  return (__builtin_amdgcn_readfirstlane(n) + kBlockIds - 1) / kBlockIds;
+  n = max(n, 0);
+  if (LPR < 2) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x111, 0xf, 0xf, false));   // row_shr:1
+  if (LPR < 4) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x112, 0xf, 0xf, false));   // row_shr:2
+  if (LPR < 8) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x114, 0xf, 0xf, false));   // row_shr:4
+  if (LPR < 16) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x118, 0xf, 0xf, false));  // row_shr:8
+  if (LPR < 32) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x142, 0xa, 0xf, false));  // row_bcast:15 -> rows 1, 3
+  if (LPR < 64) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x143, 0xc, 0xf, false));  // row_bcast:31 -> rows 2, 3
+  return (__builtin_amdgcn_readlane(n, bz::kWave - 1) + kBlockIds - 1) / kBlockIds;
 }
 
 // The walk over a segment: straight-line code that the whole wave runs as often as its longest segment takes, the rows of a
@@ -764,6 +771,16 @@ __device__ __forceinline__ void finish_sum(const bz_embed_slot& s, int64_t num, 
   }
   const int e0 = l * CE;
   if (e0 < s.dim) store_elems<CE>(s.out, b * s.out_stride + e0, acc, s.dim - e0, s.out_dtype);
+}
+
+// The sum of sample b, `inside`: whether there is such a sample.  All lanes of a wave with one come along (wave_steps).
+template <int DT, int LPR, bool KEYED>
+__device__ __forceinline__ void sum_samples(const bz_embed_slot& s, int64_t start, int64_t end, int l, int64_t b, bool inside) {
+  if (__builtin_amdgcn_ballot_w64(inside) == 0) return;
+  if (!inside) end = start;
+  float acc[RowTraits<DT>::kElems];
+  sum_segment<DT, LPR, KEYED>(s, start, end, l, acc);
+  if (inside) finish_sum<DT>(s, end - start, l, b, acc);
 }
 
 // f(table dtype, lanes per row, whether a slot is keyed), all as constants, for a (dtype << 8) | lanes code of a plan

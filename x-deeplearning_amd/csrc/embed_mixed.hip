@@ -219,8 +219,8 @@ __global__ __launch_bounds__(kThreads) void bz_embed_pool_generic_kernel(const b
   pool_generic(s, v, ext_off != nullptr ? ext_off + (int64_t)lo * ext_stride : s.offsets, s_off, s_part);
 }
 
-__global__ __launch_bounds__(kThreads) void bz_embed_pool_generic_args_kernel(const SlotPack pack, const SlotBegins begins,
-                                                                              int total_wg, int wg_per_xcd, int wg_per_slot) {
+__global__ __launch_bounds__(kThreads) void bz_embed_pool_generic_args_kernel(int total_wg, int wg_per_xcd, int wg_per_slot,
+                                                                              const SlotPack pack, const SlotBegins begins) {
   __shared__ int64_t s_off[kThreads + 1];
   __shared__ int64_t s_part[2 * kThreads / bz::kWave];
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
@@ -339,13 +339,11 @@ __device__ __forceinline__ void pool_mixed(const bz_embed_slot& s, int v, const 
     start = sh.wide.off[b - b_first];
     end = sh.wide.off[b - b_first + 1];
   }
-  if (item > last) return;
   if (s.udf != BZ_ASSIGN) {
-    float acc[RowTraits<DT>::kElems];
-    sum_segment<DT, LPR, KEYED>(s, start, end, l, acc);
-    finish_sum<DT>(s, end - start, l, b, acc);
+    sum_samples<DT, LPR, KEYED>(s, start, end, l, b, item <= last);
     return;
   }
+  if (item > last) return;
   const int p0 = (int)(item - b * per) * kAssignRun;
   int64_t first;
   const bool hash = s.hash_buckets != nullptr;
@@ -373,8 +371,8 @@ __global__ __launch_bounds__(kThreads) void bz_embed_mixed_kernel(const bz_embed
 }
 
 template <int DT, int LPR, bool KEYED>
-__global__ __launch_bounds__(kThreads) void bz_embed_mixed_args_kernel(const SlotPack pack, const SlotBegins begins, int total_wg,
-                                                                       int wg_per_xcd, int wg_per_slot) {
+__global__ __launch_bounds__(kThreads) void bz_embed_mixed_args_kernel(int total_wg, int wg_per_xcd, int wg_per_slot,
+                                                                       const SlotPack pack, const SlotBegins begins) {
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
   const int lo = wg_per_slot > 0 ? v / wg_per_slot : slot_of(begins, v);
@@ -418,14 +416,14 @@ int embed_launch_mixed_args(const bz_embed_slot* slots_host, const bz_embed_laun
   const int per_slot = ((int64_t)L.wg_per_slot * L.n_slots == L.total_wg) ? L.wg_per_slot : 0;
   if (L.shape != 0) {
     const int rc = with_shape(L.shape & ~kShapeKeyed, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
-      hipLaunchKernelGGL((bz_embed_mixed_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st, pack, begins,
-                         L.total_wg, per_xcd, per_slot);
+      hipLaunchKernelGGL((bz_embed_mixed_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st, L.total_wg, per_xcd, per_slot, pack,
+                         begins);
     });
     if (rc != BZ_OK) return rc;
     BZ_LAUNCH_OK("bz_embed_mixed_args_kernel");
     return BZ_OK;
   }
-  hipLaunchKernelGGL(bz_embed_pool_generic_args_kernel, grid, block, 0, st, pack, begins, L.total_wg, per_xcd, per_slot);
+  hipLaunchKernelGGL(bz_embed_pool_generic_args_kernel, grid, block, 0, st, L.total_wg, per_xcd, per_slot, pack, begins);
   BZ_LAUNCH_OK("bz_embed_pool_generic_args_kernel");
   return BZ_OK;
 }

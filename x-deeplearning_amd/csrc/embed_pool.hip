@@ -239,6 +239,9 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
     if (lane == 0) excl = 0;
     *start = (int64_t)sat_add(before, excl, cap);
     *end = (int64_t)x;
+  } else if constexpr (LPR == 2 || LPR == 4) {  // (an operand, where a shuffle is a trip to LDS)
+    *start = (int64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, LPR == 4 ? 0x00 : 0xa0, 0xf, 0xf, true);  // quad_perm
+    *end = (int64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, LPR == 4 ? 0xff : 0xf5, 0xf, 0xf, true);
   } else {
     const int gbase = lane - l;
     *start = (int64_t)(uint32_t)__shfl((int)x, gbase, bz::kWave);
@@ -262,7 +265,7 @@ __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0,
   } else if (offsets != nullptr) {
     // every lane of a group asks for its sample's two offsets itself (one address a group): nothing goes through LDS
     // and no wave waits for another's.  Caller-made offsets get the same bounds as the scan's.
-    const int64_t bb = b0 + g < s.batch ? b0 + g : s.batch - 1;  // (lanes past the batch return below)
+    const int64_t bb = b0 + g < s.batch ? b0 + g : s.batch - 1;  // (lanes past the batch: any)
     const int64_t o0 = offsets[bb], o1 = offsets[bb + 1];
     start = o0 < 0 ? 0 : (o0 < s.nnz ? o0 : s.nnz);
     end = o1 < 0 ? 0 : (o1 < s.nnz ? o1 : s.nnz);
@@ -272,10 +275,7 @@ __device__ __forceinline__ void pool_samples(const bz_embed_slot& s, int64_t b0,
     end = s_off[g + 1];
   }
   const int64_t b = b0 + g;
-  if (b >= s.batch) return;
-  float acc[RowTraits<DT>::kElems];
-  sum_segment<DT, LPR, KEYED>(s, start, end, l, acc);
-  finish_sum<DT>(s, end - start, l, b, acc);
+  sum_samples<DT, LPR, KEYED>(s, start, end, l, b, b < s.batch);
 }
 
 template <int DT, int LPR, int THREADS, bool KEYED>
@@ -292,8 +292,8 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_s
 }
 
 template <int DT, int LPR, bool KEYED>
-__global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(const SlotPack pack, int total_wg, int wg_per_xcd,
-                                                                      int wg_per_slot) {
+__global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(int total_wg, int wg_per_xcd, int wg_per_slot,
+                                                                      const SlotPack pack) {
   constexpr int GROUPS = kThreads / LPR;
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
@@ -504,7 +504,7 @@ int bz_embed_pool_args(const bz_embed_slot* slots_host, const bz_embed_launch* l
   hipStream_t st = bz::as_stream(stream);
   const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
     hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st,
-                       pack, L.total_wg, per_xcd, L.wg_per_slot);
+                       L.total_wg, per_xcd, L.wg_per_slot, pack);
   });
   if (rc != BZ_OK) return rc;
   BZ_LAUNCH_OK("bz_embed_pool_args_kernel");

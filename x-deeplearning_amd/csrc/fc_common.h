@@ -259,7 +259,9 @@ inline int head_unroll(int n) { return n <= 2 ? 2 : kSkinnyMaxN; }
 template <int HN>
 struct HeadBias {
   float b[HN];
-  __device__ __forceinline__ explicit HeadBias(const HeadArgs& head) {
+  HeadBias() = default;
+  __device__ __forceinline__ explicit HeadBias(const HeadArgs& head) { ask(head); }
+  __device__ __forceinline__ void ask(const HeadArgs& head) {
 #pragma unroll
     for (int j = 0; j < HN; ++j) b[j] = 0.f;
     if (head.bias != nullptr) {

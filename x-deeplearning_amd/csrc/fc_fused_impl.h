@@ -790,8 +790,8 @@ struct SplitRows {
 
 template <int DT, typename OutT, int NW, bool CHUNKS>
 __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __restrict__ A, const char* __restrict__ W,
-                                                                 OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
-                                                                 int64_t ldw, int64_t ldy, int tiles_m, Epilogue ep) {
+                                                                 int M, int N, int K, int tiles_m, int64_t lda, int64_t ldw,
+                                                                 OutT* __restrict__ Y, int64_t ldy, Epilogue ep) {
   using T = In<DT>;
   constexpr int STEPS = kSplitUnit / 32;  // a step: 16 bytes of K in each half of the lanes
   constexpr int PITCH = 33;
@@ -909,8 +909,8 @@ constexpr float kOrdinary = 0x1p40f;
 
 // EXACT: Dice as apply_act computes it, not as the tile kernels do
 template <typename OutT, int NW, int TM, int TN, int SUMS, bool EXACT>
-__global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, OutT* __restrict__ Y, int M,
-                                                            int N, int K, int64_t lda, int64_t ldw, int64_t ldy, int tiles_m,
+__global__ __launch_bounds__(NW * 64, 2) void bz_fc_f32_kernel(const char* __restrict__ A, const char* __restrict__ W, int M, int N, int K,
+                                                            int tiles_m, int64_t lda, int64_t ldw, OutT* __restrict__ Y, int64_t ldy,
                                                             Epilogue ep) {
   constexpr int BM = 32 * TM, BN = 32 * TN, NT = NW * 64, ROWS = BM + BN;
   constexpr int LOADS = ROWS / 16;  // a load instruction brings 16 rows of a stage
@@ -1259,8 +1259,8 @@ constexpr int kHeadWaves = 16;
 
 template <int DT, typename OutT, int HN>
 __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const char* __restrict__ A, const char* __restrict__ W,
-                                                                           OutT* __restrict__ Y, int M, int N, int K, int64_t lda,
-                                                                           int64_t ldw, int64_t ldy, Epilogue ep, HeadArgs head) {
+                                                                           int M, int N, int K, int64_t lda, int64_t ldw,
+                                                                           OutT* __restrict__ Y, int64_t ldy, Epilogue ep, HeadArgs head) {
   using T = In<DT>;
   static_assert(sizeof(OutT) == T::kSize, "the head reads the tile with the operand type");
   constexpr int ES = T::kSize, STEPS = kSplitUnit / 64, COLS = 256 / 64;
@@ -1380,8 +1380,8 @@ __global__ __launch_bounds__(kHeadWaves * 64) void bz_fc_split_head_kernel(const
 // NMAX: outputs the code is unrolled for
 template <int DT, typename OutT, int NMAX>
 __global__ __launch_bounds__(256) void bz_fc_skinny_kernel(const char* __restrict__ A, const char* __restrict__ W,
-                                                           OutT* __restrict__ Y, OutT* __restrict__ copy, int M, int N, int K, int64_t lda,
-                                                           int64_t ldw, int64_t ldy, int lpr, Epilogue ep) {
+                                                           int M, int N, int K, int lpr, int64_t lda, int64_t ldw,
+                                                           OutT* __restrict__ Y, OutT* __restrict__ copy, int64_t ldy, Epilogue ep) {
   constexpr int CH = In<DT>::kChunk;
   const int tid = threadIdx.x;
   const int g = tid / lpr, l = tid - g * lpr;
@@ -1494,7 +1494,7 @@ int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   if constexpr (DT != BZ_F32)
     if (d.k % In<DT>::kChunk == 0) kernel = bz_fc_split_kernel<DT, OutT, NW, true>;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a,
-                     (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, tiles_m, ep);
+                     (const char*)d.w, d.m, d.n, d.k, tiles_m, d.lda, d.ldw, (OutT*)d.y, d.ldy, ep);
   BZ_LAUNCH_OK("bz_fc_split_kernel");
   return BZ_OK;
 }
@@ -1503,8 +1503,8 @@ int launch_split(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
 template <typename OutT, int NW, int TM, int TN, int SUMS, bool EXACT>
 int launch_f32(const bz_fc_desc& d, const Epilogue& ep, hipStream_t st) {
   const int tiles_m = (d.m + 32 * TM - 1) / (32 * TM), tiles_n = (d.n + 32 * TN - 1) / (32 * TN);
-  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN, SUMS, EXACT>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda,
-                     d.ldw, d.ldy, tiles_m, ep);
+  hipLaunchKernelGGL((bz_fc_f32_kernel<OutT, NW, TM, TN, SUMS, EXACT>), dim3(tiles_m * tiles_n), dim3(NW * 64), 0, st, (const char*)d.a, (const char*)d.w, d.m, d.n, d.k, tiles_m,
+                     d.lda, d.ldw, (OutT*)d.y, d.ldy, ep);
   BZ_LAUNCH_OK("bz_fc_f32_kernel");
   return BZ_OK;
 }
@@ -1552,7 +1552,7 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream
   if constexpr (DT == BZ_F32) {
     if (d.m <= 2048) {
       hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
-                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d, copy));
+                         (const char*)d.w, d.m, d.n, d.k, d.lda, d.ldw, (OutT*)d.y, d.ldy, ep, head_args(d, copy));
       BZ_LAUNCH_OK("bz_fc_split_head_kernel");
       return BZ_OK;
     }
@@ -1563,7 +1563,7 @@ int dispatch_head(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStream
   } else if constexpr (DT == BZ_F16) {  // (bz::fc_fused takes such columns, for a net's layers, none of which is bf16)
     if (d.n % In<DT>::kChunk != 0) {  // (the tiles read a head's weight in whole chunks)
       hipLaunchKernelGGL((bz_fc_split_head_kernel<DT, OutT, HN>), dim3((d.m + 15) / 16), dim3(kHeadWaves * 64), 0, st, (const char*)d.a,
-                         (const char*)d.w, (OutT*)d.y, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, ep, head_args(d, copy));
+                         (const char*)d.w, d.m, d.n, d.k, d.lda, d.ldw, (OutT*)d.y, d.ldy, ep, head_args(d, copy));
       BZ_LAUNCH_OK("bz_fc_split_head_kernel");
       return BZ_OK;
     }
@@ -1736,10 +1736,10 @@ int dispatch_skinny(const bz_fc_desc& d, const Epilogue& ep, void* copy, hipStre
   // 15.2 and 7.1).
   if (d.n <= 2)
     hipLaunchKernelGGL((bz_fc_skinny_kernel<DT, OutT, 2>), dim3((int)grid), dim3(256), 0, st, (const char*)d.a, (const char*)d.w,
-                       (OutT*)d.y, (OutT*)copy, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
+                       d.m, d.n, d.k, lpr, d.lda, d.ldw, (OutT*)d.y, (OutT*)copy, d.ldy, ep);
   else
     hipLaunchKernelGGL((bz_fc_skinny_kernel<DT, OutT, kSkinnyMaxN>), dim3((int)grid), dim3(256), 0, st, (const char*)d.a,
-                       (const char*)d.w, (OutT*)d.y, (OutT*)copy, d.m, d.n, d.k, d.lda, d.ldw, d.ldy, lpr, ep);
+                       (const char*)d.w, d.m, d.n, d.k, lpr, d.lda, d.ldw, (OutT*)d.y, (OutT*)copy, d.ldy, ep);
   BZ_LAUNCH_OK("bz_fc_skinny_kernel");
   return BZ_OK;
 }

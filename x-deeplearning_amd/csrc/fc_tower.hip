@@ -45,9 +45,12 @@ __global__ __launch_bounds__(256) void bz_fc_tower_pack_kernel(const uint16_t* _
 
 struct Tower {
   const char* x;  // [m, lda]
-  int64_t lda;    // bytes
+  int lda;        // bytes
   int m, k, n1, n2;
   const char *w1, *w2;
+};
+// what is needed later than that
+struct Finish {
   Epilogue ep1, ep2;
   HeadArgs head;
 };
@@ -79,7 +82,7 @@ constexpr int kBeyond = 1 << 30;  // an offset behind any of them
 // apply_act_t takes them; zeros behind the layer's columns.
 struct Column {
   float bias, p0, p1, p2;
-  __device__ __forceinline__ Column(const Epilogue& ep, int n) {
+  __device__ __forceinline__ void ask(const Epilogue& ep, int n) {
     const int at = threadIdx.x * 4;
     auto load = [&](const float* from, int size, int off) {
       return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buffer_of(from, from != nullptr ? size * 4 : 0), off, 0, 0));
@@ -276,7 +279,7 @@ __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, c
   const int here = min(a.m - m0, kRows), groups = up(a.k, 64) / 64, whole = a.k / 8, rest = a.k % 8;
   const char* from = a.x + (int64_t)m0 * a.lda;
   const int start = ODD ? (int)((uintptr_t)from & 2) : 0;
-  const auto x = buffer_of(from - start, (uint32_t)up(start + (here - 1) * (int)a.lda + a.k * 2, 4));
+  const auto x = buffer_of(from - start, (uint32_t)up(start + (here - 1) * a.lda + a.k * 2, 4));
   // A wave has eight of the rows (lane % 8), every other 64 inputs (unit lane / 8): whole lines read, and 128 bytes a quarter wave
   // written
   const int r = wave % 4 * 8 + lane % 8, c0 = wave / 4 * 8 + lane / 8;
@@ -285,7 +288,7 @@ __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, c
   auto batch = [&](int g0, const F* meanwhile) {
     uint4 v[kAhead];
     uint32_t next[kAhead];
-    const int base = start + r * (int)a.lda, odd = ODD ? base & 2 : 0;
+    const int base = start + r * a.lda, odd = ODD ? base & 2 : 0;
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int c = g0 * 8 + c0 + i * 16;
@@ -311,7 +314,7 @@ __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, c
   if (last) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      tail[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x, i < rest && lane < here ? start + lane * (int)a.lda + (whole * 8 + i) * 2 : kBeyond, 0, 0);
+      tail[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x, i < rest && lane < here ? start + lane * a.lda + (whole * 8 + i) * 2 : kBeyond, 0, 0);
   }
   batch(0, &meanwhile);
   then();
@@ -327,8 +330,10 @@ __device__ __forceinline__ void stage_rows(const Tower& a, int m0, char* rows, c
 // TN: blocks of 32 columns a wave holds of the first layer; with one, two workgroups share a CU (with more registers than that leaves, the
 // attention model on eight serving threads, whose 162 -> 200 -> 80 it is, comes to 62 M samples/s for 66).  HN: outputs the skinny layer's code is unrolled for.  ODD: stage_rows'.
 template <int TN, int HN, bool ODD>
-__global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(const Tower a) {
+__global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(const char* x, const char* w1_, const char* w2_, int lda, int m, int k, int n1,
+                                                                                int n2, const Finish f) {
   typedef __half T;
+  const Tower a = {x, lda, m, k, n1, n2, w1_, w2_};
   extern __shared__ __align__(16) char lds[];
   const Layout at = layout(a.k, a.n1, a.n2, HN);
   const int k2 = up(a.n1, 64), k3 = up(a.n2, 64);
@@ -338,28 +343,34 @@ __global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(
   float *params1 = (float*)(lds + at.params), *params2 = params1 + 4 * k2, *dots = (float*)(lds + at.dots);
   T* head_w = (T*)(lds + at.head_w);
 
+  // The rows first, whose addresses come with the wave (the kernel's first arguments are preloaded); then, once the other arguments have
+  // arrived, the parameters, and the weights behind them
   Layer<TN> first;
-  const HeadBias<HN> hbias(a.head);
-  const Column col1(a.ep1, a.n1), col2(a.ep2, a.n2);
+  HeadBias<HN> hbias;
+  Column col1, col2;
   constexpr int kHeadPer = HN * kMaxNarrow / kThreads;  // of the skinny layer's weights, a thread's
   const int hc = threadIdx.x % kMaxNarrow, hj = threadIdx.x / kMaxNarrow;
-  const auto from_head = buffer_of(a.head.w, (uint32_t)(((a.head.n - 1) * (int)a.head.ldw + a.n2) * 2));
   uint16_t hw[kHeadPer];
-#pragma unroll
-  for (int i = 0; i < kHeadPer; ++i) {
-    const int j = hj + i * (kThreads / kMaxNarrow);
-    hw[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from_head, j < a.head.n && hc < a.n2 ? (j * (int)a.head.ldw + hc) * 2 : kBeyond, 0, 0);
-  }
   std::conditional_t<(TN > 1), WarmWeights, NoWarming> warm;
   stage_rows<ODD>(
       a, m0, lds,
       [&]() {
+        hbias.ask(f.head);
+        col1.ask(f.ep1, a.n1);
+        col2.ask(f.ep2, a.n2);
+        const auto from_head = buffer_of(f.head.w, (uint32_t)(((f.head.n - 1) * (int)f.head.ldw + a.n2) * 2));
+#pragma unroll
+        for (int i = 0; i < kHeadPer; ++i) {
+          const int j = hj + i * (kThreads / kMaxNarrow);
+          hw[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from_head, j < f.head.n && hc < a.n2 ? (j * (int)f.head.ldw + hc) * 2 : kBeyond, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         first.start(w1, wave);
         warm.ask(w1, w2);
       },
       [&]() {
-        col1.put(a.ep1, k2, params1);
-        col2.put(a.ep2, k3, params2);
+        col1.put(f.ep1, k2, params1);
+        col2.put(f.ep2, k3, params2);
 #pragma unroll
         for (int i = 0; i < kHeadPer; ++i)
           if (hc < k3) ((uint16_t*)head_w)[(hj + i * (kThreads / kMaxNarrow)) * k3 + hc] = hw[i];
@@ -372,11 +383,11 @@ __global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(
   Layer<1> second;
   second.start(w2, wave);
   __syncthreads();
-  if (busy1) finish<TN>(a.ep1, params1, a.n1, k2, wave, first.acc, lds);
+  if (busy1) finish<TN>(f.ep1, params1, a.n1, k2, wave, first.acc, lds);
   __syncthreads();
   if (busy2) {
     second.run(w2, lds, wave);
-    finish<1>(a.ep2, params2, a.n2, k3, wave, second.acc, rows2);
+    finish<1>(f.ep2, params2, a.n2, k3, wave, second.acc, rows2);
   }
   __syncthreads();
 
@@ -408,12 +419,12 @@ __global__ __launch_bounds__(kThreads, TN == 1 ? 4 : 2) void bz_fc_tower_kernel(
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) dot[j] += dots[(w * HN + j) * kRows + r];
     }
-    head_finish(a.head, hbias, m0 + r, dot);
+    head_finish(f.head, hbias, m0 + r, dot);
   }
 }
 
 template <int TN, int HN, bool ODD>
-int launch(const Tower& a, int lds, hipStream_t st) {
+int launch(const Tower& a, const Finish& f, int lds, hipStream_t st) {
   // more dynamic LDS than the default limit: raised once per kernel and device
   static std::mutex mu;
   static bool raised[64] = {};
@@ -426,14 +437,15 @@ int launch(const Tower& a, int lds, hipStream_t st) {
       raised[dev] = true;
     }
   }
-  hipLaunchKernelGGL((bz_fc_tower_kernel<TN, HN, ODD>), dim3((a.m + kRows - 1) / kRows), dim3(kThreads), lds, st, a);
+  hipLaunchKernelGGL((bz_fc_tower_kernel<TN, HN, ODD>), dim3((a.m + kRows - 1) / kRows), dim3(kThreads), lds, st, a.x, a.w1, a.w2, a.lda, a.m, a.k, a.n1, a.n2,
+                     f);
   BZ_LAUNCH_OK("bz_fc_tower_kernel");
   return BZ_OK;
 }
 
 template <int TN, int HN>
-int with_rows(const Tower& a, int lds, hipStream_t st) {
-  return (((uintptr_t)a.x | (uintptr_t)a.lda) & 3) != 0 ? launch<TN, HN, true>(a, lds, st) : launch<TN, HN, false>(a, lds, st);
+int with_rows(const Tower& a, const Finish& f, int lds, hipStream_t st) {
+  return (((uintptr_t)a.x | (uintptr_t)a.lda) & 3) != 0 ? launch<TN, HN, true>(a, f, lds, st) : launch<TN, HN, false>(a, f, lds, st);
 }
 
 }  // namespace
@@ -494,35 +506,36 @@ int bz::fc_tower(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
   BZ_REQUIRE(d.m >= 0 && d.m < (1ll << 31) - kRows, "tower: %lld rows", (long long)d.m);
   if (d.m == 0) return BZ_OK;
   Tower a = {};
+  Finish f = {};
   a.x = (const char*)d.a;
-  a.lda = d.lda * 2;
+  a.lda = (int)d.lda * 2;
   a.m = d.m;
   a.k = d.k;
   a.n1 = d.n;
   a.n2 = x.n;
   a.w1 = (const char*)d.w;
   a.w2 = (const char*)x.w;
-  a.ep1 = fc_epilogue(d);
-  a.ep2.bias = x.bias;
-  a.ep2.bias_rows = x.bias != nullptr ? 1 : 0;
-  a.ep2.p0 = x.act_p0;
-  a.ep2.p1 = x.act_p1;
-  a.ep2.p2 = x.act_p2;
-  a.ep2.act = x.act;
-  a.ep2.act_size = x.act_size;
-  a.ep2.dice_nosqrt = x.dice_nosqrt;
-  a.ep2.alpha = x.alpha;
-  a.ep2.beta = x.beta;
-  a.ep2.act_alpha = x.act_alpha;
+  f.ep1 = fc_epilogue(d);
+  f.ep2.bias = x.bias;
+  f.ep2.bias_rows = x.bias != nullptr ? 1 : 0;
+  f.ep2.p0 = x.act_p0;
+  f.ep2.p1 = x.act_p1;
+  f.ep2.p2 = x.act_p2;
+  f.ep2.act = x.act;
+  f.ep2.act_size = x.act_size;
+  f.ep2.dice_nosqrt = x.dice_nosqrt;
+  f.ep2.alpha = x.alpha;
+  f.ep2.beta = x.beta;
+  f.ep2.act_alpha = x.act_alpha;
   // (a layer without these activations may have their pointers set all the same)
-  for (Epilogue* e : {&a.ep1, &a.ep2}) {
+  for (Epilogue* e : {&f.ep1, &f.ep2}) {
     if (e->act != BZ_ACT_PRELU && e->act != BZ_ACT_DICE) e->p0 = nullptr;
     if (e->act != BZ_ACT_DICE) e->p1 = e->p2 = nullptr;
   }
-  a.head = head_args(d, copy);
+  f.head = head_args(d, copy);
   hipStream_t st = bz::as_stream(stream);
   const int lds = layout(d.k, d.n, x.n, head_unroll(d.head_n)).all;
   const bool two = head_unroll(d.head_n) == 2;
-  if (a.n1 <= kWaves * 32) return two ? with_rows<1, 2>(a, lds, st) : with_rows<1, kSkinnyMaxN>(a, lds, st);
-  return two ? with_rows<2, 2>(a, lds, st) : with_rows<2, kSkinnyMaxN>(a, lds, st);
+  if (a.n1 <= kWaves * 32) return two ? with_rows<1, 2>(a, f, lds, st) : with_rows<1, kSkinnyMaxN>(a, f, lds, st);
+  return two ? with_rows<2, 2>(a, f, lds, st) : with_rows<2, kSkinnyMaxN>(a, f, lds, st);
 }

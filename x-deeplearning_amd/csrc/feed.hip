@@ -44,8 +44,6 @@ template <int N>
 struct FeedArgs {
   FeedRange r[N];
   int wg_end[N];  // workgroups of the ranges up to and including this one
-  int n_ranges;
-  int range_wg;  // of all of them
   int n;
   bz_feed_rows p[BZ_FEED_MAX_ROWS];
   int unit[BZ_FEED_MAX_ROWS];     // widest power of two (<= 16) that divides addresses, pitches and row length
@@ -113,18 +111,23 @@ __device__ __forceinline__ void feed_same32(const FeedRange& r, int wg) {
     if (i0 + k * kFeedThreads < r.chunks) dst[i0 + k * kFeedThreads] = u32x4{r.word, r.word, r.word, r.word};
 }
 
+// (the first four arguments are there when a wave starts: N == 1 reads over the link at once)
 template <int UNITS, int N>
-__global__ __launch_bounds__(kFeedThreads) void bz_feed_kernel(const FeedArgs<N> a) {
+__global__ __launch_bounds__(kFeedThreads) void bz_feed_kernel(int range_wg, const char* src, char* dst, int64_t chunks, const FeedArgs<N> a) {
   const int wg = (int)blockIdx.x;
-  if (wg < a.range_wg) {
+  if (wg < range_wg) {
     if (N == 1) {
-      feed_raw<UNITS>(a.r[0], wg);
+      feed_raw<UNITS>({src, dst, chunks, BZ_FEED_RAW, 0, 0}, wg);
       return;
     }
-    // which range: every lane looks at one, in one trip to the arguments
-    const int lane = (int)threadIdx.x & (bz::kWave - 1);
-    const int q = __popcll(__ballot(lane < a.n_ranges && wg >= a.wg_end[min(lane, N - 1)]));
-    const FeedRange r = a.r[__builtin_amdgcn_readfirstlane(q)];
+    // which range: every lane brings one, and where it ends, in one trip to the arguments (ranges that are not there end with the last)
+    const int lane = min((int)threadIdx.x & (bz::kWave - 1), N - 1);
+    const FeedRange mine = a.r[lane];
+    const int q = __popcll(__ballot(wg >= a.wg_end[lane]));
+    auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, q); };
+    auto of64 = [&](uint64_t v) { return (uint64_t)of((uint32_t)(v >> 32)) << 32 | of((uint32_t)v); };
+    const FeedRange r = {(const char*)of64((uint64_t)mine.src), (char*)of64((uint64_t)mine.dst), (int64_t)of64((uint64_t)mine.chunks),
+                         (int32_t)of((uint32_t)mine.form), of(mine.word), (int32_t)of((uint32_t)mine.wg_begin)};
     if (r.form == BZ_FEED_RAW)
       feed_raw<UNITS>(r, wg - r.wg_begin);
     else if (r.form == BZ_FEED_LOW32)
@@ -136,7 +139,7 @@ __global__ __launch_bounds__(kFeedThreads) void bz_feed_kernel(const FeedArgs<N>
   int q = 0;
   while (q < a.n - 1 && wg >= a.row_end[q]) ++q;  // (uniform; at most BZ_FEED_MAX_ROWS steps)
   const bz_feed_rows p = a.p[q];
-  const int64_t first = (int64_t)(wg - (q == 0 ? a.range_wg : a.row_end[q - 1])) * (kFeedThreads * UNITS);
+  const int64_t first = (int64_t)(wg - (q == 0 ? range_wg : a.row_end[q - 1])) * (kFeedThreads * UNITS);
   switch (a.unit[q]) {
     case 16: feed_rows<u32x4, UNITS>(p, first); break;
     case 8: feed_rows<u32x2, UNITS>(p, first); break;
@@ -159,20 +162,22 @@ int launch_feed(const bz_feed_piece* pieces, int n_pieces, const bz_feed_rows* r
   const int units = all <= kFeedOneUnit ? 1 : all <= (1ll << 30) ? 2 : 4;  // (four for the sake of the grid's size)
   const int64_t span = kFeedThreads * units;
   int64_t wg = 0;
+  int n_ranges = 0;
   for (int i = 0; i < n_pieces; ++i) {
     const bz_feed_piece& p = pieces[i];
     if (p.bytes == 0) continue;
     const int64_t chunks = p.bytes / 16;
-    FeedRange& r = a.r[a.n_ranges];
+    FeedRange& r = a.r[n_ranges];
     r = {(const char*)p.src, (char*)p.dst, chunks, p.form, p.word, (int32_t)wg};
     if (p.form == BZ_FEED_SAME32)
       wg += (chunks + kFeedThreads * kSameUnits - 1) / (kFeedThreads * kSameUnits);
     else
       wg += ((p.form == BZ_FEED_LOW32 ? (chunks + 1) / 2 : chunks) + span - 1) / span;
     BZ_REQUIRE(wg < (1ll << 30), "bz_feed: %lld bytes make too many workgroups", (long long)p.bytes);
-    a.wg_end[a.n_ranges++] = (int)wg;
+    a.wg_end[n_ranges++] = (int)wg;
   }
-  a.range_wg = (int)wg;
+  const int range_wg = (int)wg;
+  for (int i = n_ranges; i < N; ++i) a.wg_end[i] = range_wg;
   for (int i = 0; i < n_rows; ++i) {
     const bz_feed_rows& p = rows[i];
     BZ_REQUIRE(p.rows >= 0 && p.row_bytes >= 0 && p.src_pitch >= p.row_bytes && p.dst_pitch >= p.row_bytes,
@@ -193,7 +198,7 @@ int launch_feed(const bz_feed_piece* pieces, int n_pieces, const bz_feed_rows* r
   }
   if (wg == 0) return BZ_OK;
   hipLaunchKernelGGL((units == 1 ? bz_feed_kernel<1, N> : units == 2 ? bz_feed_kernel<2, N> : bz_feed_kernel<4, N>), dim3((int)wg),
-                     dim3(kFeedThreads), 0, bz::as_stream(stream), a);
+                     dim3(kFeedThreads), 0, bz::as_stream(stream), range_wg, a.r[0].src, a.r[0].dst, a.r[0].chunks, a);
   BZ_LAUNCH_OK("bz_feed_kernel");
   return BZ_OK;
 }
