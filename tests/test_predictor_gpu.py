@@ -1454,9 +1454,10 @@ def test_feed_many_of_words_that_are_packed(pb, n, odd):
 
 
 def _tower(pb, ws, bs, acts, chain, heads):
+    kind = pb.K_FLOAT if ws[0].dtype == np.float32 else pb.K_FLOAT16
     nb = pb.NetBuilder("tower%d" % chain, device_type=1)
     nb.arg("chain_narrow_fcs", chain)
-    nb.external_input("x", pb.K_FLOAT16)
+    nb.external_input("x", kind)
     params = [[] if a is None else a[1:] for a in acts]
     for i, (w, b) in enumerate(zip(ws, bs)):  # (in front of the layers: operators are joined where they follow each other)
         nb.constant("w%d" % i, w)
@@ -1474,7 +1475,7 @@ def _tower(pb, ws, bs, acts, chain, heads):
         nb.op("Softmax", [h], ["p"], axis=1)
     else:
         nb.op("Sigmoid", [h], ["p"])
-    nb.external_output("p", pb.K_FLOAT16)
+    nb.external_output("p", kind)
     pm = pb.PredictorManager()
     pm.load_model_from_string(nb.text(), True)
     return pm.create_predictor(1, 0)
@@ -1610,3 +1611,92 @@ def test_tower_rows_do_not_reach_into_each_other(pb, k):
     rest = [i for i in range(70) if i not in bad]
     np.testing.assert_array_equal(got[0][rest], got[1][rest])
     assert np.isnan(got[1][31]).all()
+
+
+# k: one input, ragged and whole chunks of four and groups of sixteen, more than one ring of groups a wave, the longest taken; n1, n2: a lane, one
+# block of 64 and two, ragged and whole, the most; rows: one to four a workgroup, and the line of bz::fc_rows_pays
+@pytest.mark.parametrize("k,n1,n2,heads,rows", [(1, 9, 9, 1, (1, 5)), (4, 64, 63, 2, (3, 128, 129)), (5, 65, 64, 8, (4, 257)), (192, 200, 80, 2, (1, 201, 385)),
+                                                (468, 256, 100, 2, (2, 1024, 1025)), (445, 250, 256, 3, (300, 7)), (1280, 130, 40, 1, (130, 514)),
+                                                (771, 129, 65, 2, (127, 512))])
+@pytest.mark.parametrize("act", ["PRelu", "Dice", "Sigmoid", None])
+def test_few_rows_in_one_launch(pb, k, n1, n2, heads, rows, act):
+    """fp32 layer -> layer -> skinny layer against 64 bits and against one launch a layer, the rows growing and shrinking past the line
+    beyond which it is no launch of its own; and while the operators are timed one by one."""
+    rng = np.random.default_rng(k * n1 + n2)
+    sizes = (k, n1, n2, heads)
+    ws = [(rng.standard_normal(s) / np.sqrt(s[0])).astype(np.float32) for s in zip(sizes, sizes[1:])]
+    bs = [(rng.standard_normal(n) * 0.1).astype(np.float32) for n in sizes[1:]]
+    acts = []
+    for n in (n1, n2):
+        p = [rng.uniform(0.1, 0.4, n).astype(np.float32), (rng.standard_normal(n) * 0.1).astype(np.float32), rng.uniform(0.5, 1.5, n).astype(np.float32)]
+        acts.append({"PRelu": ("PRelu", p[0]), "Dice": ("Dice", *p), "Sigmoid": ("Sigmoid", ), None: None}[act])
+    one, apart = (_tower(pb, ws, bs, acts, chain, heads) for chain in (1, 0))
+    for step, m in enumerate(rows + rows[:1]):
+        print("few rows %d x %d -> %d -> %d -> %d %s" % (m, k, n1, n2, heads, act), flush=True)
+        if step == len(rows):
+            one.register_observers(["profile"])
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        got = []
+        for p in (one, apart):
+            p.feed("x", x)
+            p.forward()
+            got.append(p.output_asnumpy("p").astype(np.float64).reshape(m, heads))
+        if act is not None and step < len(rows):
+            assert (_tower_launches(one)[0] == 1) == (m <= 1024) and _tower_launches(apart)[0] >= 2, "%d rows" % m
+        h = x.astype(np.float64)
+        for w, b, a in zip(ws[:2], bs, acts):
+            h = _tower_act(h @ w.astype(np.float64) + b, a)
+        z = h @ ws[2].astype(np.float64) + bs[2]
+        e = np.exp(z - z.max(1, keepdims=True)) if heads > 1 else z
+        want = e / e.sum(1, keepdims=True) if heads > 1 else _sigmoid(z)
+        # a layer's sums, of terms whose squares add up to about 1, are off by at most 0.5 * 2^-24 * sqrt(K / 8) each, three layers' to about
+        # 1e-6 together; the result has a slope of at most 1/4
+        errors = [np.sqrt(np.mean((g - want)**2)) for g in got]
+        for g in got:
+            np.testing.assert_allclose(g, want, rtol=0, atol=2e-6, err_msg="%d rows" % m)
+        # and no further off than the launches that it stands for, by the mean of many (a single one is off by up to half its last bit, 2^-25,
+        # either way; the mean of n such by a part of 1 / sqrt(2 n) more or less)
+        if m * heads >= 200:
+            assert errors[0] <= 1.1 * errors[1], errors
+
+
+# both sides of each line of bz::fc_rows_pays, and of what the kernel takes
+@pytest.mark.parametrize("k,n1,n2,rows,one", [(192, 200, 80, 1024, True), (192, 200, 80, 1025, False), (732, 256, 100, 1, True), (733, 256, 100, 1, False), (64, 256, 64, 9, True),
+                                              (64, 257, 64, 9, False), (1280, 16, 16, 9, True), (1281, 16, 16, 9, False), (64, 64, 256, 9, True), (64, 64, 257, 9, False)])
+def test_few_rows_launches(pb, k, n1, n2, rows, one):
+    """the launches of a pass as it runs, with nothing timing its operators: one for a tower of few rows where that pays, else two or three"""
+    ws = [np.full(s, 2.0**-10, np.float32) for s in ((k, n1), (n1, n2), (n2, 2))]
+    bs = [np.zeros(n, np.float32) for n in (n1, n2, 2)]
+    for chain in (1, 0):
+        p = _tower(pb, ws, bs, [("Sigmoid", ), ("Sigmoid", )], chain, 2)
+        for m in (rows, 8, rows):
+            p.feed("x", np.ones((m, k), np.float32))
+            p.forward()
+        np.testing.assert_allclose(p.output_asnumpy("p"), 0.5, rtol=1e-6)
+        launches, timed = _tower_launches(p)
+        assert timed == [0, 0] and (launches == 1) == (one and chain == 1)
+
+
+@pytest.mark.parametrize("k", [72, 71, 69])
+def test_few_rows_do_not_reach_into_each_other(pb, k):
+    """infinities and NaNs in some rows, a workgroup's first and last and the input's last among them: the others come out as without, and an
+    infinite sum stays infinite"""
+    rng = np.random.default_rng(k)
+    ws = [(rng.standard_normal(s) / np.sqrt(s[0])).astype(np.float32) for s in ((k, 100), (100, 50), (50, 2))]
+    bs = [(rng.standard_normal(n) * 0.1).astype(np.float32) for n in (100, 50, 2)]
+    p = _tower(pb, ws, bs, [("Sigmoid", ), ("Sigmoid", )], 1, 2)
+    x = rng.standard_normal((390, k)).astype(np.float32)
+    bad, last = [0, 2, 200, 389], [0, k - 1, k - 1, k - 1]
+    got = []
+    for values in (None, (np.inf, np.nan, -np.inf, np.inf)):
+        y = x.copy()
+        if values is not None:
+            y[bad, last] = values
+        p.feed("x", y)
+        p.forward()
+        got.append(p.output_asnumpy("p").reshape(390, 2).copy())
+    rest = [i for i in range(390) if i not in bad]
+    np.testing.assert_array_equal(got[0][rest], got[1][rest])
+    assert np.isnan(got[1][2]).all()
+    for i, c, sign in ((0, 0, 1), (200, k - 1, -1), (389, k - 1, 1)):  # Sigmoid(e^x / (1 + e^x)) of +inf is NaN, of -inf 0: NaN where any output is +inf
+        assert np.isnan(got[1][i]).all() == (sign * ws[0][c] > 0).any(), i

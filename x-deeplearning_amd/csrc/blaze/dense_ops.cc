@@ -72,7 +72,8 @@ struct FcCall {
   const void* a = nullptr;
   const bz_concat_ew_desc* a_pieces = nullptr;  // instead of a: the rows as pieces computed on the fly (bz_fc_desc.a_pieces)
   const bz_fc_next* next = nullptr;             // with a_pieces or tower_w: a second layer in the same launch
-  const void* tower_w = nullptr;                // instead of b: the weight as bz::fc_tower takes it
+  const void* tower_w = nullptr;                // instead of b: the weight as bz::fc_tower takes it, or
+  bool few_rows = false;                        // as bz::fc_rows does
   int a_rows = 0, a_cols = 0;  // as stored
   bool trans_a = false;
   Blob* b_blob = nullptr;
@@ -188,7 +189,7 @@ bool RunFc(const FcCall& c, Derived* packed_b, Derived* packed_a, hipStream_t st
   }
   if (c.tower_w != nullptr) {
     d.next = c.next;
-    const int rc = bz::fc_tower(d, c.copy, st);
+    const int rc = c.few_rows ? bz::fc_rows(d, c.copy, st) : bz::fc_tower(d, c.copy, st);
     if (rc == BZ_ENOTSUP) return false;
     BZ_CHECK(rc);
     return true;
@@ -339,9 +340,9 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     if (g == nullptr || head_ != nullptr || !siblings_.empty() || next_ != nullptr || tower_ != nullptr) return false;
     Blob* b0 = this->Input(1);
     Blob* b = g->Input(1);
-    // without a Concat of its own this layer takes the next one only with a skinny one behind that, 2-byte ones of some sizes: a tower
+    // without a Concat of its own this layer takes the next one only with a skinny one behind that, of some sizes: a tower
     const bool tower = concat_ == nullptr;
-    if (tower && (!b_constant_ || transa_ || b0->shape().size() != 2 || DataTypeSize(b0->data_type()) != 2 || g->head_ == nullptr || g->next_ != nullptr || g->tower_ != nullptr ||
+    if (tower && (!b_constant_ || transa_ || b0->shape().size() != 2 || (b0->data_type() != kFloat16 && b0->data_type() != kFloat) || g->head_ == nullptr || g->next_ != nullptr || g->tower_ != nullptr ||
                   g->head_->Input(1)->data_type() != b0->data_type() || (fused_ && fused_act_ == BZ_ACT_SOFTMAX)))
       return false;
     if (tower && this->InputSize() > 2 && (!c_constant_ || this->Input(2)->size() != (transb_ ? b0->shape()[0] : b0->shape()[1]))) return false;
@@ -350,7 +351,8 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     const TIndex N1 = transb_ ? b0->shape()[0] : b0->shape()[1];
     const TIndex K2 = g->transb_ ? b->shape()[1] : b->shape()[0], N2 = g->transb_ ? b->shape()[0] : b->shape()[1];
     if (K2 != N1 || N2 <= 8) return false;
-    if (tower ? !bz::fc_tower_takes(transb_ ? b0->shape()[1] : b0->shape()[0], N1, N2) : N2 > 64) return false;
+    const TIndex K1 = transb_ ? b0->shape()[1] : b0->shape()[0];
+    if (tower ? !(b0->data_type() == kFloat ? bz::fc_rows_takes(K1, N1, N2) : bz::fc_tower_takes(K1, N1, N2)) : N2 > 64) return false;
     if (g->InputSize() > 2 && (!g->c_constant_ || (TIndex)g->Input(2)->size() != N2)) return false;
     if (g->fused_ && g->fused_act_ == BZ_ACT_SOFTMAX) return false;
     if (g->fused_ && g->fused_act_ == BZ_ACT_PRELU && (TIndex)g->fused_->Input(1)->size() != N2 && g->fused_->Input(1)->size() != 1) return false;
@@ -423,7 +425,9 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
     Blob *a = this->Input(0), *b = this->Input(1), *b2 = tower_->Input(1);
     const TIndex k = transb_ ? b->shape()[1] : b->shape()[0], n = transb_ ? b->shape()[0] : b->shape()[1];
     const TIndex n2 = tower_->transb_ ? b2->shape()[0] : b2->shape()[1];
-    return a->pitch() == 0 && k > 0 && bz::fc_tower_pays(a->size() / k, k, n, n2);
+    if (a->pitch() != 0 || k <= 0) return false;
+    const TIndex rows = a->size() / k;
+    return b->data_type() == kFloat ? bz::fc_rows_pays(rows, k, n, n2) : bz::fc_tower_pays(rows, k, n, n2);
   }
   // the hosted head as a launch of its own
   bool RunHeadAlone() {
@@ -645,16 +649,19 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
       const int es2 = (int)DataTypeSize(b2->data_type());
       const int n2 = (int)(g->transb_ ? b2->shape()[0] : b2->shape()[1]);
       const int64_t ldw2 = (N + 7) / 8 * 8;
+      call.few_rows = tower && a->data_type() == kFloat;
       if (tower) {
         auto laid_out = [&](GemmOp* of, int k_in, int n_out) {
           Blob* w = of->Input(1);
-          const size_t bytes = bz::fc_tower_weight_bytes(k_in, n_out);
-          if (of->tower_w_.Stale(w) || of->tower_w_.bytes < bytes) {
-            of->tower_w_.Resize(bytes);
-            BZ_CHECK(bz::fc_tower_pack(w->data(), of->transb_, k_in, n_out, of->tower_w_.ptr, st));
-            of->tower_w_.Mark(w);
+          Derived& to = call.few_rows ? of->rows_w_ : of->tower_w_;
+          const size_t bytes = call.few_rows ? bz::fc_rows_weight_bytes(k_in, n_out, es2) : bz::fc_tower_weight_bytes(k_in, n_out);
+          if (to.Stale(w) || to.bytes < bytes) {
+            to.Resize(bytes);
+            BZ_CHECK(call.few_rows ? bz::fc_rows_pack(w->data(), of->transb_, k_in, n_out, es2, to.ptr, st)
+                                   : bz::fc_tower_pack(w->data(), of->transb_, k_in, n_out, to.ptr, st));
+            to.Mark(w);
           }
-          return of->tower_w_.ptr;
+          return to.ptr;
         };
         call.tower_w = laid_out(this, (int)K, (int)N);
         nx.w = laid_out(g, (int)N, n2);
@@ -818,7 +825,7 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
   float alpha_, beta_;
   bool transa_, transb_;
   bool b_constant_ = false, c_constant_ = false;
-  Derived packed_b_, packed_a_, bias_f32_, p_f32_[3], tower_w_;
+  Derived packed_b_, packed_a_, bias_f32_, p_f32_[3], tower_w_, rows_w_;
   GemmOp* head_ = nullptr;       // the layer of at most 8 outputs computed in this operator's launch
   OperatorBase* concat_ = nullptr;  // the Concat that makes Input(0), computed by this operator's kernel
   GemmOp* next_ = nullptr;          // the narrow layer after this one, computed in this operator's launch
