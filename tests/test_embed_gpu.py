@@ -730,3 +730,29 @@ def test_the_longest_segment_of_a_wave_wherever_it_lies(bz, oracle, dim, fused, 
             got, _, _ = _run_gpu(bz, [t], specs, inputs, batch, np.float32, cols, fused_scan=fused)
             want = _run_oracle(oracle, [t], specs, inputs, batch, cols)
             assert np.array_equal(_bits(got), _bits(want)), (batch, long_at)
+
+
+@pytest.mark.parametrize("rows", [97, 2**24 + 7])  # through buffer resources and by plain loads
+@pytest.mark.parametrize("weighted", [False, True])
+def test_int8_scales_of_any_size(bz, oracle, rows, weighted):
+    """Ids of value 1 have q * scale from q + 128 and -128 * scale, which is no longer finite from 2^121 on: scales around that, infinities, NaN,
+    zeros of both signs and subnormal ones, beside ordinary ones in the same wave and in waves of their own."""
+    rng = np.random.default_rng(rows)
+    dim = 20
+    odd = np.array([2.0**120, -(2.0**120), np.nextafter(np.float32(2.0**120), np.float32(0)), 2.0**121, -3e38, 2.0**127, np.inf, -np.inf, np.nan, 0.0, -0.0,
+                    1e-40, -1e-45, 2.0**-126], np.float32)
+    some = np.concatenate([odd, rng.uniform(1e-3, 1e-2, 97 - odd.size).astype(np.float32)])
+    t = dict(data=np.resize(rng.integers(-128, 128, (97, dim)).astype(np.int8), (rows, dim)), scale=np.resize(some, rows))
+    for first, many in ((0, 97), (odd.size, 97)):  # with them, and ordinary ones alone
+        batch = 70
+        seg = rng.integers(0, 9, batch).astype(np.int32)
+        ids = rng.integers(first, many, int(seg.sum())).astype(np.int64)
+        ids[rng.random(ids.size) < 0.05] = -1
+        vals = rng.standard_normal(ids.size).astype(np.float32) if weighted else np.ones(ids.size, np.float32)
+        specs, cols = [(0, 0, 0, 0, dim)], (dim, [0])
+        got, _, _ = _run_gpu(bz, [t], specs, [(ids, vals, seg)], batch, np.float32, cols)
+        want = _run_oracle(oracle, [t], specs, [(ids, vals, seg)], batch, cols)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert first != 0 or np.isinf(want).any()
+        ok = ~np.isnan(want)
+        assert np.array_equal(_bits(got[ok]), _bits(want[ok]))
