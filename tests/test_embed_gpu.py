@@ -756,3 +756,23 @@ def test_int8_scales_of_any_size(bz, oracle, rows, weighted):
         assert first != 0 or np.isinf(want).any()
         ok = ~np.isnan(want)
         assert np.array_equal(_bits(got[ok]), _bits(want[ok]))
+
+
+@pytest.mark.parametrize("kind,keyed,slots,batch,dim", [("f16", False, 63, 513, 32), ("f16", False, 64, 512, 32), ("f16", False, 51, 520, 32), ("f32", False, 255, 3, 256), ("f32", False, 256, 3, 256),
+                                                        ("f32", False, 5, 131, 4), ("i8", False, 64, 512, 64), ("i8", False, 3, 24000, 64), ("i8", False, 5, 33000, 64),
+                                                        ("f32", True, 24, 300, 100), ("f16", True, 4, 20000, 64)])
+def test_workgroups_of_either_size(bz, oracle, kind, keyed, slots, batch, dim):
+    """sums of workgroups of 256 and of 512 threads on both sides of the lines between them (less than 256 of the larger ones; int8 rows, or keys, and at most
+    32 MB of counts read in front of the workgroups), whole and ragged ones, fused scan with and without the records as arguments"""
+    rng = np.random.default_rng(slots * batch)
+    t = _make_table(rng, kind, 50, dim, keyed)
+    keys = t.get("keys")
+    inputs = []
+    for _ in range(slots):
+        seg = rng.integers(0, 4, batch).astype(np.int32)
+        ids = rng.integers(0, 50, int(seg.sum())).astype(np.int64)
+        inputs.append((ids if keys is None else np.asarray(keys)[ids].astype(np.int64), np.ones(ids.size, np.float32), seg))
+    specs, cols = [(0, i % 2, 0, 0, dim) for i in range(slots)], (dim * slots, [dim * i for i in range(slots)])
+    got, _, variant = _run_gpu(bz, [t], specs, inputs, batch, np.float32, cols)
+    assert variant != 0
+    assert np.array_equal(_bits(got), _bits(_run_oracle(oracle, [t], specs, inputs, batch, cols)))

@@ -291,16 +291,32 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_s
   pool_samples<DT, LPR, THREADS, KEYED>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
 }
 
-template <int DT, int LPR, bool KEYED>
-__global__ __launch_bounds__(kThreads) void bz_embed_pool_args_kernel(int total_wg, int wg_per_xcd, int wg_per_slot,
+template <int DT, int LPR, int THREADS, bool KEYED>
+__global__ __launch_bounds__(THREADS) void bz_embed_pool_args_kernel(int total_wg, int wg_per_xcd, int wg_per_slot,
                                                                       const SlotPack pack) {
-  constexpr int GROUPS = kThreads / LPR;
+  constexpr int GROUPS = THREADS / LPR;
   const int v = (int)(blockIdx.x % bz::kNumXcd) * wg_per_xcd + (int)(blockIdx.x / bz::kNumXcd);
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = pack.s[si];
   const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
-  pool_samples<DT, LPR, kThreads, KEYED>(s, b0, s.offsets);
+  pool_samples<DT, LPR, THREADS, KEYED>(s, b0, s.offsets);
+}
+
+// When workgroups that find their offsets themselves have 256 threads instead of 512: where the larger ones would leave CUs without any, and
+// for the forms whose walk takes more than 64 registers (int8 rows, slots looked up by key), of which three of the larger ones share a CU
+// and not four; unless the counts in front of each workgroup, which twice as many then read, are more than 32 MB.
+// us with 512 / 256 threads, by workgroups of 512: 6 (223 x 3 lists of 9 ids, fp16) 4.7 / 4.4, 10 (108 x 10 of 22, int8) 9.7 / 7.5, 72 (380 x 3 of 22,
+// fp32 rows of 128) 5.4 / 4.5, 95 (1058 x 19 of 12, fp16) 6.3 / 5.0, 119 (1050 x 7 of 21) 5.9 / 4.8, 208 (1024 x 26 of 8) 5.0 / 4.9; but 400 (100 x 200
+// of 10) 6.4 / 6.8, 416 (2048 x 26 of 8) 7.0 / 7.0 and on eight serving threads 12.1 / 12.2 a pass.  int8: 580 (7193 x 20 of 17) 42.0 / 36.7, 1600 (4096
+// x 50 of 20) 52.6 / 49.8, 3486 (10539 x 83 of 21, 146 MB of counts) 295 / 297.  By key: 1512 (1000 x 24 of 6, fp32 rows of 100) 14.7 / 13.8, 54
+// (300 x 18 of 3, fp16) 5.6 / 5.2, a request with them 39.4 / 38.8; 1011 (10782 x 6 of 20, 43 MB of counts) 29.3 / 30.3.
+constexpr int kSmallThreads = 256;
+constexpr int kSmallGroups = 256;
+constexpr int64_t kSmallBytes = 32ll << 20;
+inline bool small_groups(const bz_embed_launch& L, int dtype, bool keyed) {
+  const int64_t groups = (int64_t)L.total_wg * (kThreads / kSmallThreads);
+  return (L.total_wg < kSmallGroups || dtype == BZ_I8 || keyed) && groups * L.max_batch * 2 <= kSmallBytes;
 }
 
 // When a separate scan launch (4.2-8 us, and 3-4 between the launches) is cheaper than the fused scan, whose cost is one
@@ -467,7 +483,8 @@ static int launch_pool(const bz_embed_slot* slots_dev, const bz_embed_launch& L,
   const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
     constexpr int kDt = decltype(dt)::value, kLpr = decltype(lpr)::value;
     constexpr bool kKeyed = decltype(keyed)::value;
-    if (scanned)
+    static_assert(kOffsetThreads == kSmallThreads, "one kernel for both");
+    if (scanned || small_groups(L, kDt, kKeyed))
       hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kOffsetThreads, kKeyed>), dim3(per_xcd_scanned * bz::kNumXcd), dim3(kOffsetThreads), 0,
                          st, slots_dev, L.n_slots, kOffsetSplit * L.total_wg, per_xcd_scanned, kOffsetSplit * L.wg_per_slot, ext_off,
                          ext_stride);
@@ -499,12 +516,18 @@ int bz_embed_pool_args(const bz_embed_slot* slots_host, const bz_embed_launch* l
   SlotPack pack;
   memcpy(pack.s, slots_host, (size_t)L.n_slots * sizeof(bz_embed_slot));
   memset(pack.s + L.n_slots, 0, (size_t)(BZ_EMBED_ARG_SLOTS - L.n_slots) * sizeof(bz_embed_slot));
-  const int per_xcd = (L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
-  const dim3 grid(per_xcd * bz::kNumXcd), block(kThreads);
   hipStream_t st = bz::as_stream(stream);
   const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
-    hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, decltype(keyed)::value>), grid, block, 0, st,
-                       L.total_wg, per_xcd, L.wg_per_slot, pack);
+    auto launch = [&](auto threads) {
+      constexpr int kEach = decltype(threads)::value, kSplit = kThreads / kEach;
+      const int per_xcd = (kSplit * L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
+      hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, kEach, decltype(keyed)::value>), dim3(per_xcd * bz::kNumXcd),
+                         dim3(kEach), 0, st, kSplit * L.total_wg, per_xcd, kSplit * L.wg_per_slot, pack);
+    };
+    if (small_groups(L, decltype(dt)::value, decltype(keyed)::value))
+      launch(std::integral_constant<int, kSmallThreads>{});
+    else
+      launch(std::integral_constant<int, kThreads>{});
   });
   if (rc != BZ_OK) return rc;
   BZ_LAUNCH_OK("bz_embed_pool_args_kernel");
