@@ -174,6 +174,32 @@ def test_fc_few_tiles_and_any_row_start(bz, oracle, in_name, out_name, M, N, K, 
     _fc_case(bz, oracle, M, N, K, in_name, out_name, act, seed=M + 5 * N + K, **kw)
 
 
+@pytest.mark.parametrize("in_name", ["f16", "bf16"])
+@pytest.mark.parametrize("K", [8, 9, 15, 63, 65, 71, 445, 513])  # a chunk, its remainders, the unit of 64 and one more, more than one unit a wave
+def test_fc_split_reads_nothing_of_a_ragged_row_but_its_own(bz, K, in_name):
+    """The unit that K ends in is read from in front of its start and shifted: the numbers behind K of a wider row, NaNs here, and those in front
+    of it, count in nothing: every output is the same as without them."""
+    import torch
+    tdt, dt = {"f16": (torch.float16, bz.F16), "bf16": (torch.bfloat16, bz.BF16)}[in_name]
+    g = torch.Generator(device="cuda").manual_seed(K)
+    M, N = 33, 65
+    wide = torch.full((M, K + 11), float("nan"), device="cuda", dtype=tdt)
+    wide[:, :K] = torch.randn((M, K), generator=g, device="cuda").to(tdt)
+    w = bz.pack_weight(torch.randn((K, N), generator=g, device="cuda") / K**0.5, False, dt)
+    w[:, K:] = float("nan")
+    bias = torch.randn(N, generator=g, device="cuda")
+    outs = []
+    for a in (wide[:, :K], wide[:, :K].contiguous()):
+        y = torch.zeros((M, N), device="cuda", dtype=tdt)
+        bz.fc_fused(a, w, K, bias=bias, out=y, act=bz.ACT_LEAKY_RELU, act_alpha=0.25)
+        outs.append(y)
+    want = wide[:, :K].double() @ w[:, :K].double().t() + bias.double()
+    want = torch.where(want >= 0, want, 0.25 * want)
+    assert torch.equal(outs[0], outs[1])
+    # (sums of about 1 in fp32, rounded once to 2^-11 or 2^-8 of themselves)
+    torch.testing.assert_close(outs[0].double(), want, rtol=2.0**-10 if in_name == "f16" else 2.0**-7, atol=1e-5)
+
+
 def _fp32_sum_error(n):
     """Error of an output relative to it, the root mean square over outputs, where every partial sum has n products.  The sum
     grows like sqrt(i) and each step rounds it; rounding is evenly spread over half a unit in the last place either way, which is

@@ -754,16 +754,20 @@ struct SplitRows {
   static constexpr int ES = In<DT>::kSize, CH = In<DT>::kChunk;
   const char* p[P];
   uint4 r[P];
+  bool part = false;  // the unit is the one that K ends in: `back` elements in front of what is wanted were loaded with it (as in shift_chunk)
+  int back = 0;
   __device__ __forceinline__ void init(const char* base, int64_t ld, int row0, int rows, int lane) {
 #pragma unroll
     for (int i = 0; i < P; ++i) p[i] = base + (int64_t)min(row0 + i * 8 + (lane >> 3), rows - 1) * ld * ES;
   }
   // a whole unit
   __device__ __forceinline__ void load(int u, int lane) {
+    part = false;
 #pragma unroll
     for (int i = 0; i < P; ++i) __builtin_memcpy(&r[i], p[i] + (int64_t)u * kSplitUnit + (lane & 7) * 16, 16);
   }
-  // the unit that K ends in: zeros beyond K
+  // The unit that K ends in, zeros beyond K.  (Ragged rows are shifted when they are stored: where they are loaded, each was a trip of its
+  // own, eight for the wave whose unit it is.  300 x 445 -> 256 fp16 4.9 -> 4.3 us, one row 4.2 -> 3.6, 2000 x 901 -> 128 7.2 -> 6.4.)
   __device__ __forceinline__ void load_last(int u, int K, int lane) {
     const int k = u * (kSplitUnit / ES) + (lane & 7) * CH;
     if constexpr (CHUNKS) {
@@ -772,19 +776,29 @@ struct SplitRows {
       for (int i = 0; i < P; ++i) __builtin_memcpy(&r[i], p[i] + (int64_t)min(k, K - CH) * ES, 16);
 #pragma unroll
       for (int i = 0; i < P; ++i) r[i] = make_uint4(r[i].x & have, r[i].y & have, r[i].z & have, r[i].w & have);
+      return;
+    }
+    part = K >= CH;
+    if (part) {
+      const int at = min(k, K - CH);
+      back = k - at;
+#pragma unroll
+      for (int i = 0; i < P; ++i) __builtin_memcpy(&r[i], p[i] + (int64_t)at * ES, 16);
     } else {
 #pragma unroll
-      for (int i = 0; i < P; ++i) {
-        if (K >= CH)
-          r[i] = shift_chunk<DT>(load_chunk_anywhere<DT>(p[i], 0, 0, k, K), k - min(k, K - CH));
-        else
-          r[i] = load_chunk<DT>(p[i], 0, 0, k, K);
-      }
+      for (int i = 0; i < P; ++i) r[i] = load_chunk<DT>(p[i], 0, 0, k, K);
     }
   }
   __device__ __forceinline__ void store(char* lds, int lane) const {
+    uint4 v[P];
 #pragma unroll
-    for (int i = 0; i < P; ++i) *(uint4*)(lds + split_at<DT>(i * 8 + (lane >> 3), lane & 7)) = r[i];
+    for (int i = 0; i < P; ++i) v[i] = r[i];
+    if (!CHUNKS && part) {
+#pragma unroll
+      for (int i = 0; i < P; ++i) v[i] = shift_chunk<DT>(r[i], back);
+    }
+#pragma unroll
+    for (int i = 0; i < P; ++i) *(uint4*)(lds + split_at<DT>(i * 8 + (lane >> 3), lane & 7)) = v[i];
   }
 };
 
@@ -820,6 +834,19 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
     }
   };
   load(wave);
+  // the parameters of the column that this thread finishes: asked for now, looked at at the end.  (Behind the operands, whose addresses come
+  // with the wave: the parameters' are still on their way.)
+  float cbias = 0.f, cp0 = 0.f, cp1 = 0.f, cp2 = 0.f;
+  {
+    const int c = min(n0 + tid % 32, N - 1);
+    if (ep.bias_rows == 1) cbias = ep.bias[c];
+    if (ep.act == BZ_ACT_PRELU) cp0 = ep.p0[ep.act_size == 1 ? 0 : c];
+    if (ep.act == BZ_ACT_DICE) {
+      cp0 = ep.p0[c];
+      cp1 = ep.p1[c];
+      cp2 = ep.p2[c];
+    }
+  }
   for (int u = wave; u < units; u += NW) {
     // (a wave's own LDS operations keep their order: nobody to wait for)
     ra.store(la, lane);
@@ -857,8 +884,8 @@ __global__ __launch_bounds__(NW * 64, 4) void bz_fc_split_kernel(const char* __r
 #pragma unroll
     for (int w = 0; w < NW / 2; ++w) v += ((const float*)lds[w])[ml * PITCH + nl];
     if (m < M && n < N) {
-      const float b = ep.bias_rows == 0 ? 0.f : ep.bias[ep.bias_rows == 1 ? n : full_bias_index(ep, m, n, M, N)];
-      store_out<OutT>(Y + out_index(ep, m, n, ldy), apply_act(fmaf(ep.alpha, v, ep.beta * b), n, ep));
+      const float b = ep.bias_rows <= 1 ? cbias : ep.bias[full_bias_index(ep, m, n, M, N)];
+      store_out<OutT>(Y + out_index(ep, m, n, ldy), apply_act_regs(fmaf(ep.alpha, v, ep.beta * b), ep, cp0, cp1, cp2));
     }
   }
 }
