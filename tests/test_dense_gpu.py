@@ -582,6 +582,14 @@ def test_fc_head_limits_are_refused(bz):
 
 
 @pytest.mark.parametrize("in_name", ["f32", "f16", "bf16"])
+# lanes a row: 1 (less than a chunk, one), 2 to 64, more chunks than lanes; ragged ends; whole and ragged last workgroups, rows beyond the grid's first pass
+@pytest.mark.parametrize("M,N,K,act", [(1, 1, 1, "none"), (257, 2, 3, "softmax"), (33, 2, 7, "prelu"), (300, 2, 9, "dice"), (129, 1, 17, "sigmoid"), (65, 5, 33, "softmax"),
+                                       (31, 2, 101, "softmax"), (5, 2, 127, "none"), (9, 8, 250, "dice"), (3, 2, 513, "sigmoid"), (6, 1, 2061, "none"), (33000, 2, 259, "softmax")])
+def test_fc_skinny_of_any_depth(bz, oracle, in_name, M, N, K, act):
+    _fc_case(bz, oracle, M, N, K, in_name, in_name, act, seed=M + N + K)
+
+
+@pytest.mark.parametrize("in_name", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("M,N,K,act", [(2048, 2, 256, "softmax"), (128, 2, 80, "softmax"), (5000, 1, 40, "none"),
                                        (8192, 1, 256, "sigmoid"), (7, 8, 1000, "prelu"), (3, 3, 12, "dice")])
 def test_fc_skinny(bz, oracle, in_name, M, N, K, act):
