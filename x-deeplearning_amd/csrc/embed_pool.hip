@@ -96,15 +96,33 @@ __device__ __forceinline__ void scan_tiles(const S sums, const int32_t* __restri
   const int64_t begin = first_tile * kScanTile;
   const int64_t end = (n_tiles < 0 || begin + n_tiles * kScanTile > n) ? n : begin + n_tiles * kScanTile;
   if (begin > n || (begin == n && n != 0)) return;  // nothing here; whoever scans the last tile writes off[n]
+  // The first tile's counts and those before it, eight times four of these a thread, are all on their way before any is added up.  (One count a
+  // load, a trip for every 2048 of them, and the tile's own behind those: 200 slots x 8192 counts in front of their lookups 13.1 us, 8.4 this way.)
+  int32_t c[kScanRows];
+  auto ask = [&](int64_t base) {
+    const int64_t at = base + wave * (kScanRows * bz::kWave) + lane;
+#pragma unroll
+    for (int k = 0; k < kScanRows; ++k) c[k] = at + k * bz::kWave < n ? seg[at + k * bz::kWave] : 0;
+  };
+  ask(begin);
   T carry = 0;
   if (begin > 0) {
     T part = 0;
-    for (int64_t i = 0; i < begin; i += kScanTile) {  // (begin is a whole number of tiles)
-      int32_t c[kScanRows];
+    const i32x4a4* before = (const i32x4a4*)seg;
+    const int64_t quads = begin / 4;  // (begin is a whole number of tiles)
+    constexpr int kQuads = 8;
+    static_assert(kScanTile / 4 % kScanThreads == 0, "a row of quads is there or not for the whole workgroup");
+    for (int64_t i = 0; i < quads; i += kQuads * kScanThreads) {
+      i32x4a4 q[kQuads];
 #pragma unroll
-      for (int k = 0; k < kScanRows; ++k) c[k] = seg[i + k * kScanThreads + tid];
+      for (int k = 0; k < kQuads; ++k) {
+        q[k] = 0;
+        if (i + k * kScanThreads < quads) q[k] = before[i + k * kScanThreads + tid];
+      }
 #pragma unroll
-      for (int k = 0; k < kScanRows; ++k) part = sums.add(part, sums.take(c[k]));
+      for (int k = 0; k < kQuads; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part = sums.add(part, sums.take(q[k][j]));
     }
     part = sums.last(sums.scan(part, lane));
     if (lane == 0) tot[kScanWaves + wave] = part;
@@ -115,10 +133,7 @@ __device__ __forceinline__ void scan_tiles(const S sums, const int32_t* __restri
   int turn = 0;
   for (int64_t base = begin; base < end; base += kScanTile, turn ^= kScanWaves) {
     const int64_t at = base + wave * (kScanRows * bz::kWave) + lane;
-    int32_t c[kScanRows];
     T excl[kScanRows], run = 0;
-#pragma unroll
-    for (int k = 0; k < kScanRows; ++k) c[k] = at + k * bz::kWave < n ? seg[at + k * bz::kWave] : 0;
 #pragma unroll
     for (int k = 0; k < kScanRows; ++k) {
       const T v = sums.take(c[k]);
@@ -129,6 +144,7 @@ __device__ __forceinline__ void scan_tiles(const S sums, const int32_t* __restri
       excl[k] = sums.add(run, before);
       run = sums.add(run, sums.last(incl));
     }
+    if (base + kScanTile < end) ask(base + kScanTile);
     if (lane == 0) tot[turn + wave] = run;
     __syncthreads();
     T before = carry;
