@@ -654,10 +654,10 @@ class GemmOp : public Operator<Context>, public FusableProducer, public Stackabl
         auto laid_out = [&](GemmOp* of, int k_in, int n_out) {
           Blob* w = of->Input(1);
           Derived& to = call.few_rows ? of->rows_w_ : of->tower_w_;
-          const size_t bytes = call.few_rows ? bz::fc_rows_weight_bytes(k_in, n_out, es2) : bz::fc_tower_weight_bytes(k_in, n_out);
+          const size_t bytes = call.few_rows ? bz::fc_rows_weight_bytes(k_in, n_out) : bz::fc_tower_weight_bytes(k_in, n_out);
           if (to.Stale(w) || to.bytes < bytes) {
             to.Resize(bytes);
-            BZ_CHECK(call.few_rows ? bz::fc_rows_pack(w->data(), of->transb_, k_in, n_out, es2, to.ptr, st)
+            BZ_CHECK(call.few_rows ? bz::fc_rows_pack(w->data(), of->transb_, k_in, n_out, to.ptr, st)
                                    : bz::fc_tower_pack(w->data(), of->transb_, k_in, n_out, to.ptr, st));
             to.Mark(w);
           }

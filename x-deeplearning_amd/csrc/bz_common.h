@@ -59,12 +59,12 @@ bool fc_tower_takes(int64_t k, int64_t n1, int64_t n2);  // whether it takes lay
 bool fc_tower_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2);  // whether that is faster than the first and the others in two
 size_t fc_tower_weight_bytes(int64_t k, int64_t n);
 int fc_tower_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream);  // from [k, n], or [n, k] when transposed
-// fc_rows.hip, for the host layer: the same for few rows, fp32 or fp16; d.w and d.next->w as fc_rows_pack laid them out
+// fc_rows.hip, for the host layer: the same for few rows, fp32; d.w and d.next->w as fc_rows_pack laid them out
 int fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream);
 bool fc_rows_takes(int64_t k, int64_t n1, int64_t n2);
 bool fc_rows_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2);
-size_t fc_rows_weight_bytes(int64_t k, int64_t n, int element_size);
-int fc_rows_pack(const void* w, bool transposed, int k, int n, int element_size, void* out, bz_stream_t stream);
+size_t fc_rows_weight_bytes(int64_t k, int64_t n);
+int fc_rows_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream);
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
 // once more at `copy`, [m, columns] without gaps (pinned host memory: results that are there when the launch has ended)
 int fc_fused(const bz_fc_desc& d, void* copy, bz_stream_t stream);

@@ -5,7 +5,7 @@
 // what bounds it is how fast all the weights reach a CU, 64 bytes a clock.  So weights are laid out once as the lanes take them and asked
 // for as early as there are registers for them (256 KB a CU under way; the second layer's follow the first's, ahead of the first's
 // outputs), and no instruction is spent on them but the load and the products: a lane has one output's 16 bytes, and
-// v_mfma_*_4x4x* (sixteen blocks of four outputs and four rows) multiplies four rows at a time by them; waves share K.
+// v_mfma_f32_4x4x1 (sixteen blocks of four outputs and four rows) multiplies four rows at a time by them; waves share K.
 //
 // us of the kernels, before (layer, and layer with head; 1.5 to 2 between the two) and now: one row of 192 -> 200 -> 80 -> 2 4.5 + 6.1 and 7.0, 201 of 144
 // -> 200 -> 80 -> 2 4.8 + 8.5 and 8.5; a request with them 30.9 -> 28.6 and 54.3 -> 48.9.  Of one row's 14,600 clocks the first loads are under way
@@ -26,36 +26,28 @@ constexpr int kBeyond = 1 << 30;  // an offset behind any operand
 
 __host__ __device__ constexpr int up(int v, int to) { return (v + to - 1) / to * to; }
 
-typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-
 // How a layer's waves share it: blocks of 64 outputs, and of each block's K slices of whole groups.  (Made on the host: a kernel this
 // short would spend as long on the divisions as on a layer.)
 struct Split {
   int chunks, blocks, slices, groups;  // groups: of a slice
   int per_block;                       // 2^16 / blocks, rounded up: wave / blocks is wave * per_block / 2^16
   Split() = default;
-  Split(int k, int n, int chunk)
-      : chunks((k + chunk - 1) / chunk), blocks((n + 63) / 64), slices(kWaves / blocks), groups(((chunks + slices - 1) / slices + kGroup - 1) / kGroup),
+  Split(int k, int n)
+      : chunks((k + 3) / 4), blocks((n + 63) / 64), slices(kWaves / blocks), groups(((chunks + slices - 1) / slices + kGroup - 1) / kGroup),
         per_block(65535 / blocks + 1) {}
 };
 
 // Weights as the lanes take them: block by block of 64 outputs (the last of what is left), chunk by chunk of 16 bytes of inputs, an output's
 // 16 bytes after the other's; zeros behind K.
-__global__ __launch_bounds__(256) void bz_fc_rows_pack_kernel(const char* __restrict__ w, uint4* __restrict__ out, int k, int n, int64_t sk, int64_t sn, int es,
-                                                              int units) {
+__global__ __launch_bounds__(256) void bz_fc_rows_pack_kernel(const float* __restrict__ w, float4* __restrict__ out, int k, int n, int64_t sk, int64_t sn, int units) {
   const int u = blockIdx.x * 256 + threadIdx.x;
   if (u >= units) return;
-  const int ce = 16 / es, chunks = (k + ce - 1) / ce, block = u / (64 * chunks), width = min(64, n - block * 64);
+  const int chunks = (k + 3) / 4, block = u / (64 * chunks), width = min(64, n - block * 64);
   const int c = (u - block * 64 * chunks) / width, o = block * 64 + (u - block * 64 * chunks) % width;
-  uint4 v = make_uint4(0, 0, 0, 0);
-  for (int i = 0; i < ce && c * ce + i < k; ++i) {
-    const char* from = w + ((c * ce + i) * sk + o * sn) * es;
-    if (es == 4)
-      ((uint32_t*)&v)[i] = *(const uint32_t*)from;
-    else
-      ((uint16_t*)&v)[i] = *(const uint16_t*)from;
-  }
-  out[u] = v;
+  float v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = c * 4 + i < k ? w[(c * 4 + i) * sk + o * sn] : 0.f;
+  out[u] = make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // LDS, in bytes: rows of operands, 16 bytes further apart than whole groups, so that four rows' reads of one chunk are on different
@@ -63,9 +55,9 @@ __global__ __launch_bounds__(256) void bz_fc_rows_pack_kernel(const char* __rest
 struct Layout {
   int pitch1, pitch2, x2, sums, params1, params2, head_w, all;
   Layout() = default;
-  Layout(int k, int n1, int n2, int hn, int chunk) {
-    pitch1 = up((k + chunk - 1) / chunk, kGroup) * 16 + 16;
-    pitch2 = up((n1 + chunk - 1) / chunk, kGroup) * 16 + 16;
+  Layout(int k, int n1, int n2, int hn) {
+    pitch1 = up((k + 3) / 4, kGroup) * 16 + 16;
+    pitch2 = up((n1 + 3) / 4, kGroup) * 16 + 16;
     x2 = kRows * pitch1;
     sums = x2 + kRows * pitch2;
     params1 = sums + kThreads * 16;
@@ -103,9 +95,8 @@ struct Column {
   }
 };
 
-// output `col` of row `row` from the waves' sums, rounded as it would be stored
-template <typename T>
-__device__ __forceinline__ T finished(const Epilogue& ep, const float* params, const Split& by, int row, int col, const float* sums) {
+// output `col` of row `row` from the waves' sums
+__device__ __forceinline__ float finished(const Epilogue& ep, const float* params, const Split& by, int row, int col, const float* sums) {
   const float* of = sums + (col / 4 * 4 + row) * 4 + col % 4;  // (block by block of 64 lanes, a lane's four outputs of row lane % 4)
   const int next = by.blocks * 256;
   const float4 p = *(const float4*)(params + col * 4);
@@ -118,13 +109,10 @@ __device__ __forceinline__ T finished(const Epilogue& ep, const float* params, c
     sum = of[0] + of[next];
   else
     sum = of[0];
-  T t;
-  store_out<T>(&t, apply_act_regs(fmaf(ep.alpha, sum, p.x), ep, p.y, p.z, p.w));
-  return t;
+  return apply_act_regs(fmaf(ep.alpha, sum, p.x), ep, p.y, p.z, p.w);
 }
 
 // A wave's share of a layer's weights
-template <int DT>
 struct Share {
   __amdgpu_buffer_rsrc_t from;  // the share
   int lane, step;               // the lane's bytes of the first chunk (or beyond), from one chunk to the next
@@ -152,24 +140,16 @@ struct Share {
 };
 
 // sixteen blocks of 4 outputs x 4 rows: lane l has 16 bytes of output l in w and of row l % 4 in x; a block's sums of row l % 4 are in lane l
-template <int DT>
-__device__ __forceinline__ void mma4(const uint4& w, const uint4& x, floatx4 (&acc)[4], int i) {
-  if constexpr (DT == BZ_F32) {
-    acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.x), __uint_as_float(x.x), acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.y), __uint_as_float(x.y), acc[1], 0, 0, 0);
-    acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.z), __uint_as_float(x.z), acc[2], 0, 0, 0);
-    acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.w), __uint_as_float(x.w), acc[3], 0, 0, 0);
-  } else {
-    const uint2 w0 = make_uint2(w.x, w.y), w1 = make_uint2(w.z, w.w), x0 = make_uint2(x.x, x.y), x1 = make_uint2(x.z, x.w);
-    floatx4 &even = acc[i % 2 * 2], &odd = acc[i % 2 * 2 + 1];
-    even = __builtin_amdgcn_mfma_f32_4x4x4f16(*(const half4v*)&w0, *(const half4v*)&x0, even, 0, 0, 0);
-    odd = __builtin_amdgcn_mfma_f32_4x4x4f16(*(const half4v*)&w1, *(const half4v*)&x1, odd, 0, 0, 0);
-  }
+__device__ __forceinline__ void mma4(const uint4& w, const uint4& x, floatx4 (&acc)[4]) {
+  acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.x), __uint_as_float(x.x), acc[0], 0, 0, 0);
+  acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.y), __uint_as_float(x.y), acc[1], 0, 0, 0);
+  acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.z), __uint_as_float(x.z), acc[2], 0, 0, 0);
+  acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w.w), __uint_as_float(x.w), acc[3], 0, 0, 0);
 }
 
 // The wave's sums of a layer, whose first kRing groups are on their way; `then` asks for others behind the layer's own
-template <int DT, typename Then>
-__device__ __forceinline__ void multiply(uint4 (&w)[kRing][kGroup], const Share<DT>& of, const char* x, int pitch, floatx4* sums, const Then& then) {
+template <typename Then>
+__device__ __forceinline__ void multiply(uint4 (&w)[kRing][kGroup], const Share& of, const char* x, int pitch, floatx4* sums, const Then& then) {
   const char* row = x + (threadIdx.x % kRows) * pitch + of.first * 16;
   // A group has sums of its own, four an output, which are added to the output's: sums over all of K that one float takes up one
   // product after the other were up to 1.4 times as far off 64 bits as the launches that this one stands for (771 -> 129 -> 65 -> 2).
@@ -183,7 +163,7 @@ __device__ __forceinline__ void multiply(uint4 (&w)[kRing][kGroup], const Share<
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < kGroup; ++i) mma4<DT>(w[slot][i], f[i], acc, i);
+    for (int i = 0; i < kGroup; ++i) mma4(w[slot][i], f[i], acc);
     all += (acc[0] + acc[1]) + (acc[2] + acc[3]);
   };
   int g = 0;
@@ -204,23 +184,16 @@ __device__ __forceinline__ void multiply(uint4 (&w)[kRing][kGroup], const Share<
 }
 
 // a workgroup's rows to LDS, a quarter of the threads each, at any alignment of their elements; zeros behind K and for rows that are not there
-template <int DT>
 struct Input {
-  static constexpr int ES = In<DT>::kSize;
-  static constexpr int kEach = up(ES == 4 ? kMaxIn / 4 : kMaxIn, kPerRow) / kPerRow;
-  uint4 q[ES == 4 ? kEach : 1];
-  uint16_t h[ES == 4 ? 1 : kEach];
-  __device__ __forceinline__ void ask(const char* x, int64_t row, bool there, int k) {
-    const auto from = buffer_of(x + (there ? row : 0), there ? (uint32_t)(k * ES) : 0u);
+  static constexpr int kEach = up(kMaxIn / 4, kPerRow) / kPerRow;
+  uint4 q[kEach];
+  __device__ __forceinline__ void ask(const float* x, int64_t row, bool there, int k) {
+    const auto from = buffer_of(x + (there ? row : 0), there ? (uint32_t)k * 4u : 0u);
     const int c = threadIdx.x % kPerRow;
 #pragma unroll
     for (int i = 0; i < kEach; ++i) {
-      if constexpr (ES == 4) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(from, (c + i * kPerRow) * 16, 0, 0);
-        q[i] = *(const uint4*)&v;
-      } else {
-        h[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from, (c + i * kPerRow) * 2, 0, 0);
-      }
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(from, (c + i * kPerRow) * 16, 0, 0);
+      q[i] = *(const uint4*)&v;
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -228,39 +201,33 @@ struct Input {
     const int c = threadIdx.x % kPerRow;
 #pragma unroll
     for (int i = 0; i < kEach; ++i) {
-      if constexpr (ES == 4) {
-        const int at = c + i * kPerRow;
-        if (at * 4 < k && at * 4 + 4 > k) {  // (the chunk that K ends in)
-          if (at * 4 + 1 >= k) q[i].y = 0;
-          if (at * 4 + 2 >= k) q[i].z = 0;
-          q[i].w = 0;
-        }
-        if (at * 16 < bytes) *(uint4*)(to + at * 16) = q[i];
-      } else {
-        const int at = (c + i * kPerRow) * 2;
-        if (at < bytes) *(uint16_t*)(to + at) = h[i];
+      const int at = c + i * kPerRow;
+      if (at * 4 < k && at * 4 + 4 > k) {  // (the chunk that K ends in)
+        if (at * 4 + 1 >= k) q[i].y = 0;
+        if (at * 4 + 2 >= k) q[i].z = 0;
+        q[i].w = 0;
       }
+      if (at * 16 < bytes) *(uint4*)(to + at * 16) = q[i];
     }
   }
 };
 
 // HN: outputs the skinny layer's code is unrolled for.  rows: of a workgroup.  by1: the first layer's.
-template <int DT, typename T, int HN>
-__global__ __launch_bounds__(kThreads) void bz_fc_rows_kernel(const char* x, const char* w1_, int lda, int m, int k, int n1, int rows, int chunks, int blocks,
+template <int HN>
+__global__ __launch_bounds__(kThreads) void bz_fc_rows_kernel(const float* x, const char* w1_, int lda, int m, int k, int n1, int rows, int chunks, int blocks,
                                                               int slices, int groups, int per_block, const char* w2_, int n2, const Finish f) {
   extern __shared__ __align__(16) char lds[];
-  constexpr int ES = In<DT>::kSize;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x & 63;
   const int m0 = blockIdx.x * rows, here = min(rows, m - m0), r = wave / (kWaves / kRows), c = threadIdx.x % kPerRow;
-  Input<DT> in;
-  in.ask(x, (int64_t)(m0 + r) * lda * ES, r < here, k);
+  Input in;
+  in.ask(x, (int64_t)(m0 + r) * lda, r < here, k);
   Split by1;
   by1.chunks = chunks;
   by1.blocks = blocks;
   by1.slices = slices;
   by1.groups = groups;
   by1.per_block = per_block;
-  const Share<DT> of1(w1_, by1, n1, wave);
+  const Share of1(w1_, by1, n1, wave);
   uint4 w[kRing][kGroup];
 #pragma unroll
   for (int i = 0; i < kRing; ++i) of1.ask(w[i], i);
@@ -273,27 +240,27 @@ __global__ __launch_bounds__(kThreads) void bz_fc_rows_kernel(const char* x, con
   col1.ask(f.ep1, n1, (const float*)w1_);
   col2.ask(f.ep2, n2, (const float*)w1_);
   constexpr int kHeadPer = HN * kMaxLast / kThreads;
-  T hw[kHeadPer];
+  float hw[kHeadPer];
 #pragma unroll
   for (int i = 0; i < kHeadPer; ++i) {
     const int j = (threadIdx.x + i * kThreads) / kMaxLast, hc = threadIdx.x % kMaxLast;
-    hw[i] = ((const T*)f.head.w)[min(j, f.head.n - 1) * (int)f.head.ldw + min(hc, n2 - 1)];
+    hw[i] = ((const float*)f.head.w)[min(j, f.head.n - 1) * (int)f.head.ldw + min(hc, n2 - 1)];
   }
   __builtin_amdgcn_sched_barrier(0);
   in.put(lds + r * at.pitch1, at.pitch1 - 16, k);
   __syncthreads();
-  const Share<DT> of2(w2_, f.by2, n2, wave);
-  multiply<DT>(w, of1, lds, at.pitch1, (floatx4*)sums, [&](uint4 (&slot)[kGroup], int group) { of2.ask(slot, group); });
+  const Share of2(w2_, f.by2, n2, wave);
+  multiply(w, of1, lds, at.pitch1, (floatx4*)sums, [&](uint4 (&slot)[kGroup], int group) { of2.ask(slot, group); });
   col1.put(f.ep1, n1, params1);
   col2.put(f.ep2, n2, params2);
 #pragma unroll
-  for (int i = 0; i < kHeadPer; ++i) head_w[threadIdx.x + i * kThreads] = (float)hw[i];
+  for (int i = 0; i < kHeadPer; ++i) head_w[threadIdx.x + i * kThreads] = hw[i];
   __syncthreads();
   if (r < rows)
-    for (int o = c; o * ES < at.pitch2 - 16; o += kPerRow)
-      ((T*)(lds + at.x2 + r * at.pitch2))[o] = o < n1 ? finished<T>(f.ep1, params1, by1, r, o, sums) : (T)0.f;
+    for (int o = c; o * 4 < at.pitch2 - 16; o += kPerRow)
+      ((float*)(lds + at.x2 + r * at.pitch2))[o] = o < n1 ? finished(f.ep1, params1, by1, r, o, sums) : 0.f;
   __syncthreads();
-  multiply<DT>(w, of2, lds + at.x2, at.pitch2, (floatx4*)sums, [](uint4 (&)[kGroup], int) {});
+  multiply(w, of2, lds + at.x2, at.pitch2, (floatx4*)sums, [](uint4 (&)[kGroup], int) {});
   __syncthreads();
   // a wave a row: the second layer's activation and the skinny layer
   if (wave < here) {
@@ -301,7 +268,7 @@ __global__ __launch_bounds__(kThreads) void bz_fc_rows_kernel(const char* x, con
 #pragma unroll
     for (int j = 0; j < HN; ++j) dot[j] = 0.f;
     for (int o = lane; o < n2; o += 64) {
-      const float v = (float)finished<T>(f.ep2, params2, f.by2, wave, o, sums);
+      const float v = finished(f.ep2, params2, f.by2, wave, o, sums);
 #pragma unroll
       for (int j = 0; j < HN; ++j) dot[j] = fmaf(v, head_w[j * kMaxLast + o], dot[j]);
     }
@@ -312,41 +279,37 @@ __global__ __launch_bounds__(kThreads) void bz_fc_rows_kernel(const char* x, con
 }
 
 struct Rows {
-  const char *x, *w1, *w2;
+  const float* x;
+  const char *w1, *w2;
   int lda, m, k, n1, n2, rows;
 };
 
-template <int DT, typename T, int HN>
+template <int HN>
 int launch(const Rows& a, Finish& f, hipStream_t st) {
-  const Split by1(a.k, a.n1, In<DT>::kChunk);
-  f.by2 = Split(a.n1, a.n2, In<DT>::kChunk);
-  f.at = Layout(a.k, a.n1, a.n2, HN, In<DT>::kChunk);
-  hipLaunchKernelGGL((bz_fc_rows_kernel<DT, T, HN>), dim3((a.m + a.rows - 1) / a.rows), dim3(kThreads), f.at.all, st, a.x, a.w1, a.lda, a.m, a.k, a.n1, a.rows,
+  const Split by1(a.k, a.n1);
+  f.by2 = Split(a.n1, a.n2);
+  f.at = Layout(a.k, a.n1, a.n2, HN);
+  hipLaunchKernelGGL((bz_fc_rows_kernel<HN>), dim3((a.m + a.rows - 1) / a.rows), dim3(kThreads), f.at.all, st, a.x, a.w1, a.lda, a.m, a.k, a.n1, a.rows,
                      by1.chunks, by1.blocks, by1.slices, by1.groups, by1.per_block, a.w2, a.n2, f);
   BZ_LAUNCH_OK("bz_fc_rows_kernel");
   return BZ_OK;
 }
 
-template <int DT, typename T>
-int with_head(const Rows& a, Finish& f, hipStream_t st) {
-  return head_unroll(f.head.n) == 2 ? launch<DT, T, 2>(a, f, st) : launch<DT, T, kSkinnyMaxN>(a, f, st);
-}
-
 }  // namespace
 
-size_t bz::fc_rows_weight_bytes(int64_t k, int64_t n, int element_size) { return (size_t)n * ((k * element_size + 15) / 16) * 16; }
+size_t bz::fc_rows_weight_bytes(int64_t k, int64_t n) { return (size_t)n * ((k + 3) / 4) * 16; }
 
-int bz::fc_rows_pack(const void* w, bool transposed, int k, int n, int element_size, void* out, bz_stream_t stream) {
-  const int units = (int)(fc_rows_weight_bytes(k, n, element_size) / 16);
-  hipLaunchKernelGGL(bz_fc_rows_pack_kernel, dim3((units + 255) / 256), dim3(256), 0, bz::as_stream(stream), (const char*)w, (uint4*)out, k, n,
-                     transposed ? (int64_t)1 : (int64_t)n, transposed ? (int64_t)k : (int64_t)1, element_size, units);
+int bz::fc_rows_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream) {
+  const int units = (int)(fc_rows_weight_bytes(k, n) / 16);
+  hipLaunchKernelGGL(bz_fc_rows_pack_kernel, dim3((units + 255) / 256), dim3(256), 0, bz::as_stream(stream), (const float*)w, (float4*)out, k, n,
+                     transposed ? (int64_t)1 : (int64_t)n, transposed ? (int64_t)k : (int64_t)1, units);
   BZ_LAUNCH_OK("bz_fc_rows_pack_kernel");
   return BZ_OK;
 }
 
 bool bz::fc_rows_takes(int64_t k, int64_t n1, int64_t n2) {
   return k >= 1 && k <= kMaxIn && n1 > kSkinnyMaxN && n1 <= kMaxWide && n2 > kSkinnyMaxN && n2 <= kMaxLast &&
-         Layout((int)k, (int)n1, (int)n2, kSkinnyMaxN, 4).all <= 64 * 1024;
+         Layout((int)k, (int)n1, (int)n2, kSkinnyMaxN).all <= 64 * 1024;
 }
 
 // One launch against two or three, in fp32 models that look rows up for the input, us of a lone request / a pass on eight serving threads
@@ -381,7 +344,7 @@ int bz::fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
   BZ_REQUIRE(d.m >= 0, "rows: %lld rows", (long long)d.m);
   if (d.m == 0) return BZ_OK;
   Rows a = {};
-  a.x = (const char*)d.a;
+  a.x = (const float*)d.a;
   a.w1 = (const char*)d.w;
   a.w2 = (const char*)x.w;
   a.lda = (int)d.lda;
@@ -413,5 +376,5 @@ int bz::fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
   }
   f.head = head_args(d, copy);
   hipStream_t st = bz::as_stream(stream);
-  return d.in_dtype == BZ_F32 ? with_head<BZ_F32, float>(a, f, st) : with_head<BZ_F16, __half>(a, f, st);
+  return head_unroll(d.head_n) == 2 ? launch<2>(a, f, st) : launch<kSkinnyMaxN>(a, f, st);
 }
