@@ -218,7 +218,7 @@ class ConcatAdopter {  // implemented by Gemm
   // The narrow layer after such a layer (with the skinny layer it may already host) in the same launch
   // (bz_fc_desc.next): the attention MLP 4E -> 80 -> 40 -> 1 as one kernel.  `next` reads only this layer's result, and
   // nothing else does.  Without an adopted Concat: a tower, layer -> layer -> skinny layer, in one launch at the numbers of rows
-  // where that is faster (bz::fc_tower_pays).
+  // where that is faster (bz::fc_tower_pays, fp32 bz::fc_rows_pays).
   virtual bool CanChainNext(OperatorBase* next) = 0;  // static part
   // true: the next layer is run by this one, in its launch or behind it, and no more by the net.  False for a tower's: the net
   // runs it, which does nothing in a pass where this layer has computed it.

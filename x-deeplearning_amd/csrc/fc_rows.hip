@@ -1,16 +1,16 @@
 // fc_rows.hip -- two layers and the skinny one behind them in one launch, for few rows: a workgroup takes one to four rows through all of
 // them, and nothing but the last layer's outputs goes to memory.
 //
-// With few rows a layer is a chain and not work: each launch starts, waits for operands, adds up, ends.  Here there is one chain, and
-// what bounds it is how fast all the weights reach a CU, 64 bytes a clock.  So weights are laid out once as the lanes take them and asked
-// for as early as there are registers for them (256 KB a CU under way; the second layer's follow the first's, ahead of the first's
+// With few rows a layer is a chain and not work: each launch starts, waits for operands, adds up, ends.  Here there is one chain; what bounds
+// it is the instructions in front of the first products and, with more weights, how fast these reach a CU, 64 bytes a clock.  So weights are laid out once as the lanes take them and asked
+// for as early as there are registers for them (128 KB a CU under way; the second layer's follow the first's, ahead of the first's
 // outputs), and no instruction is spent on them but the load and the products: a lane has one output's 16 bytes, and
 // v_mfma_f32_4x4x1 (sixteen blocks of four outputs and four rows) multiplies four rows at a time by them; waves share K.
 //
 // us of the kernels, before (layer, and layer with head; 1.5 to 2 between the two) and now: one row of 192 -> 200 -> 80 -> 2 4.5 + 6.1 and 7.0, 201 of 144
 // -> 200 -> 80 -> 2 4.8 + 8.5 and 8.5; a request with them 30.9 -> 28.6 and 54.3 -> 48.9.  Of one row's 14,600 clocks the first loads are under way
 // at 2,200, the rows are in LDS at 4,600, the first layer's sums are there at 9,500, its activation at 10,600, the second's sums at 12,400.  What
-// is short in it is the code, which every CU has to fetch: with the splits worked out in the kernel and sixteen waves it took 9.3, with outputs
+// is kept short is the code, which every CU has to fetch: with the splits worked out in the kernel and sixteen waves it took 9.3, with outputs
 // beside each other in a lane's block, each load's bounds checked and a reduction every 64 outputs 14.7.
 #include "fc_common.h"
 
