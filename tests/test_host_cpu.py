@@ -315,6 +315,84 @@ def test_embedding_planner_geometry_and_scan_advice():
     assert launch.variant == 0 and [s.wg_count for s in slots] == [1024 * 13 // 128] * 3
 
 
+def test_no_pooling_workgroup_begins_behind_its_slots_samples(tmp_path):
+    """A workgroup finds its offsets by adding up the counts in front of its first sample, so one that began behind the last sample would
+    read counts beyond the caller's array, which its dropped sums would not show: of a plan's workgroups, whole and halved, those that
+    go on have each sample once and begin in front of the last one's end, at batches around every multiple of either size."""
+    import shutil
+    import subprocess
+    import blaze_hip
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    src = tmp_path / "groups.hip"
+    src.write_text(r"""
+#include <stdio.h>
+#include <string.h>
+#include <vector>
+#include "blaze_hip.h"
+#include "embed_groups.h"
+int main() {
+  int idle = 0;
+  for (int lanes = 1; lanes <= 64; lanes *= 2) {
+    std::vector<int> batches = {1, 2, 3, 4};
+    for (int at = 256 / lanes; at <= 8 * 256 / lanes; at += 256 / lanes)
+      for (int b = at - 1; b <= at + 1; ++b)
+        if (b > 0) batches.push_back(b);
+    for (int batch : batches)
+      for (int n_slots : {1, 3, 26}) {
+        std::vector<bz_embed_slot> slots(n_slots);
+        for (bz_embed_slot& s : slots) {
+          memset((void*)&s, 0, sizeof(s));
+          s.table = s.out = (void*)0x10000;  // (a plan follows no pointer)
+          s.ids = (const int64_t*)0x20000;
+          s.values = (const float*)0x30000;
+          s.segments = (const int32_t*)0x40000;
+          s.table_dtype = s.out_dtype = BZ_F32;
+          s.dim = s.out_stride = 4 * lanes;
+          s.pitch = 16 * lanes;
+          s.rows = s.nnz = 1000;
+          s.batch = batch;
+          s.udf = BZ_SUM;
+        }
+        bz_embed_launch L;
+        if (bz_embed_plan(slots.data(), n_slots, &L) != BZ_OK || L.variant != (BZ_F32 << 8 | lanes)) return 1;
+        for (int split = 1; split <= 2; ++split) {
+          const bz::PoolGrid grid(L.total_wg, L.wg_per_slot, split);
+          const int groups = 512 / split / lanes;
+          std::vector<int> seen((size_t)n_slots * batch);
+          for (int block = 0; block < grid.blocks; ++block) {
+            const int v = block % bz::kNumXcd * grid.wg_per_xcd + block / bz::kNumXcd;
+            if (v >= grid.total_wg) continue;
+            const int slot = v / grid.wg_per_slot, wg = v - slot * grid.wg_per_slot;
+            const int64_t first = bz::first_sample(wg, groups, slots[slot].batch);
+            idle += first < 0;
+            if (first >= batch) {
+              printf("batch %d, %d lanes, %d samples a workgroup: one reads counts 0 to %d\n", batch, lanes, groups, (int)first);
+              return 2;
+            }
+            for (int g = 0; first >= 0 && g < groups && first + g < batch; ++g) ++seen[(size_t)slot * batch + first + g];
+          }
+          for (int n : seen)
+            if (n != 1) return 3;
+        }
+      }
+  }
+  return idle > 0 ? 0 : 4;
+}
+""")
+    exe, lib = str(tmp_path / "groups"), os.path.dirname(blaze_hip.LIB_PATH)
+    subprocess.run([hipcc, "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"),
+                    str(src), "-L" + lib, "-lblaze_hip", "-Wl,-rpath," + lib, "-o", exe], check=True, capture_output=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout)
+    # and every workgroup of the kernel asks, before anything is read
+    kernels = re.findall(r"__global__[^;{]*bz_embed_pool(?:_args)?_kernel\(.*?\n}\n", open(os.path.join(ROOT, "x-deeplearning_amd", "csrc", "embed_pool.hip")).read(), flags=re.S)
+    assert len(kernels) == 2
+    for text in kernels:
+        assert re.search(r"const int64_t b0 = bz::first_sample\(v - si \* wg_per_slot, GROUPS, s\.batch\);\s*if \(b0 < 0\) return;\s*pool_samples<", text), text
+
+
 def test_baseline_forward_with_library_sgemm_agrees_with_the_pinned_sums(oracle):
     """bench.py times the oracle with the products handed to the BLAS numpy links (as the reference hands them to
     MKL, math/gemm.cc:13-27).  That variant must be the same computation: on a scaled-down config 2 it agrees with

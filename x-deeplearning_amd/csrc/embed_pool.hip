@@ -41,6 +41,7 @@
 #include <mutex>
 
 #include "embed_common.h"
+#include "embed_groups.h"
 
 namespace {
 
@@ -48,7 +49,6 @@ namespace {
 // more evenly (200 slots x 8192 samples, 64 threads 166.5, 128 167.2, 256 168.2, 512 176 us; 1000 x 24 and 1024 x 26 shortest
 // lists 18.2 / 5.4 us at 256 against 17.5 / 6.6 at 64).
 constexpr int kOffsetThreads = 256;
-constexpr int kOffsetSplit = kThreads / kOffsetThreads;
 
 // ---------------------------------------------------------------------------------------------
 // segments -> offsets (exclusive scan), one workgroup per array
@@ -303,7 +303,8 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_s
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = slots[si];
-  const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
+  const int64_t b0 = bz::first_sample(v - si * wg_per_slot, GROUPS, s.batch);
+  if (b0 < 0) return;
   pool_samples<DT, LPR, THREADS, KEYED>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
 }
 
@@ -315,7 +316,8 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_args_kernel(int total_w
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = pack.s[si];
-  const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
+  const int64_t b0 = bz::first_sample(v - si * wg_per_slot, GROUPS, s.batch);
+  if (b0 < 0) return;
   pool_samples<DT, LPR, THREADS, KEYED>(s, b0, s.offsets);
 }
 
@@ -488,25 +490,23 @@ static int launch_pool(const bz_embed_slot* slots_dev, const bz_embed_launch& L,
   BZ_REQUIRE(L.n_slots > 0 && L.total_wg >= 0 && L.wg_per_slot >= 0, "bz_embed_pool: bad launch record (n_slots=%d total_wg=%d)",
              L.n_slots, L.total_wg);
   if (L.total_wg == 0) return BZ_OK;
-  const int per_xcd = (L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
-  const dim3 grid(per_xcd * bz::kNumXcd), block(kThreads);
   if (L.variant == 0) return bz::embed_launch_mixed(slots_dev, L, ext_off, ext_stride, st);
   BZ_REQUIRE(L.wg_per_slot > 0 && (int64_t)L.wg_per_slot * L.n_slots == L.total_wg,
              "bz_embed_pool: variant %#x needs equal work per slot", L.variant);
   // with offsets given: smaller workgroups, each with its share of a planned workgroup's samples
   const bool scanned = ext_off != nullptr || !L.fused_scan;
-  const int per_xcd_scanned = (kOffsetSplit * L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
   const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
-    constexpr int kDt = decltype(dt)::value, kLpr = decltype(lpr)::value;
-    constexpr bool kKeyed = decltype(keyed)::value;
+    auto launch = [&](auto threads) {
+      constexpr int kEach = decltype(threads)::value;
+      const bz::PoolGrid grid(L.total_wg, L.wg_per_slot, kThreads / kEach);
+      hipLaunchKernelGGL((bz_embed_pool_kernel<decltype(dt)::value, decltype(lpr)::value, kEach, decltype(keyed)::value>), dim3(grid.blocks), dim3(kEach),
+                         0, st, slots_dev, L.n_slots, grid.total_wg, grid.wg_per_xcd, grid.wg_per_slot, ext_off, ext_stride);
+    };
     static_assert(kOffsetThreads == kSmallThreads, "one kernel for both");
-    if (scanned || small_groups(L, kDt, kKeyed))
-      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kOffsetThreads, kKeyed>), dim3(per_xcd_scanned * bz::kNumXcd), dim3(kOffsetThreads), 0,
-                         st, slots_dev, L.n_slots, kOffsetSplit * L.total_wg, per_xcd_scanned, kOffsetSplit * L.wg_per_slot, ext_off,
-                         ext_stride);
+    if (scanned || small_groups(L, decltype(dt)::value, decltype(keyed)::value))
+      launch(std::integral_constant<int, kSmallThreads>{});
     else
-      hipLaunchKernelGGL((bz_embed_pool_kernel<kDt, kLpr, kThreads, kKeyed>), grid, block, 0, st, slots_dev, L.n_slots, L.total_wg, per_xcd,
-                         L.wg_per_slot, ext_off, ext_stride);
+      launch(std::integral_constant<int, kThreads>{});
   });
   if (rc != BZ_OK) return rc;
   BZ_LAUNCH_OK("bz_embed_pool_kernel");
@@ -535,10 +535,10 @@ int bz_embed_pool_args(const bz_embed_slot* slots_host, const bz_embed_launch* l
   hipStream_t st = bz::as_stream(stream);
   const int rc = with_shape(L.variant, (L.shape & kShapeKeyed) != 0, [&](auto dt, auto lpr, auto keyed) {
     auto launch = [&](auto threads) {
-      constexpr int kEach = decltype(threads)::value, kSplit = kThreads / kEach;
-      const int per_xcd = (kSplit * L.total_wg + bz::kNumXcd - 1) / bz::kNumXcd;
-      hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, kEach, decltype(keyed)::value>), dim3(per_xcd * bz::kNumXcd),
-                         dim3(kEach), 0, st, kSplit * L.total_wg, per_xcd, kSplit * L.wg_per_slot, pack);
+      constexpr int kEach = decltype(threads)::value;
+      const bz::PoolGrid grid(L.total_wg, L.wg_per_slot, kThreads / kEach);
+      hipLaunchKernelGGL((bz_embed_pool_args_kernel<decltype(dt)::value, decltype(lpr)::value, kEach, decltype(keyed)::value>), dim3(grid.blocks),
+                         dim3(kEach), 0, st, grid.total_wg, grid.wg_per_xcd, grid.wg_per_slot, pack);
     };
     if (small_groups(L, decltype(dt)::value, decltype(keyed)::value))
       launch(std::integral_constant<int, kSmallThreads>{});
