@@ -792,3 +792,34 @@ def test_host_objects_are_built_again_when_the_dispatch_rules_change():
     out = subprocess.run(["make", "-n", "-C", csrc, "-W", "bz_common.h"], check=True, capture_output=True, text=True, timeout=120).stdout
     for f in ("dense_ops", "predictor"):
         assert "-c blaze/%s.cc" % f in out, f
+
+
+def test_few_row_towers_are_one_launch_where_serving_does_not_lose(tmp_path):
+    """both sides of the lines of the rule: rows, weights, columns, and rows times weights, beyond which a pass on serving threads takes longer in
+    one launch (592 -> 256 -> 100 at 1024 rows 10.4 us for 9.4, 732 -> 256 -> 100 11.6 for 10.4)"""
+    import shutil
+    import subprocess
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src = tmp_path / "rows.cc"
+    src.write_text(r"""
+#include <stdio.h>
+#include "bz_common.h"
+int main() {
+  const int at[][5] = {  // k, n1, n2, most rows
+      {48, 64, 32, 1024}, {192, 200, 80, 1024}, {468, 256, 100, 1024}, {592, 256, 100, 852}, {732, 256, 100, 708}, {733, 256, 100, 0}, {64, 257, 64, 0}};
+  int wrong = 0;
+  for (const auto& c : at) {
+    const int last = c[3];
+    if ((last > 0 && !(bz::fc_rows_pays(1, c[0], c[1], c[2]) && bz::fc_rows_pays(last, c[0], c[1], c[2]))) || bz::fc_rows_pays(last + 1, c[0], c[1], c[2]))
+      wrong += printf("%d -> %d -> %d\n", c[0], c[1], c[2]);
+    if (bz::fc_rows_pays(0, c[0], c[1], c[2])) wrong += printf("no rows\n");
+  }
+  return wrong > 0;
+}
+""")
+    exe = str(tmp_path / "rows")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout

@@ -312,18 +312,6 @@ bool bz::fc_rows_takes(int64_t k, int64_t n1, int64_t n2) {
          Layout((int)k, (int)n1, (int)n2, kSkinnyMaxN).all <= 64 * 1024;
 }
 
-// One launch against two or three, in fp32 models that look rows up for the input, us of a lone request / a pass on eight serving threads
-// (weights in units of 1024):
-//  48 -> 64 -> 32 (5) 201 rows 29.4 / 5.4 and 33.2 / 5.3, 1000 36.5 / 5.9 and 37.3 / 6.0; 192 -> 200 -> 80 (53) one row 28.5 / 4.7 and 30.9 / 5.3,
-//  201 31.1 / 5.6 and 34.2 / 6.2, 1000 42.7 / 6.2 and 46.0 / 6.6, 2000 56.8 / 9.3 and 59.9 / 9.2; 429 -> 128 -> 64 (61) 201 42.9 / 5.7 and 48.7 / 6.3,
-//  2000 82.4 / 10.9 and 89.0 / 10.1; 468 -> 256 -> 100 (142) one 29.9 / 5.1 and 35.5 / 5.7, 201 37.6 / 6.9 and 40.3 / 6.6, 1000 56.8 / 8.7 and 58.6 /
-//  8.7, 2000 78.9 / 15.4 and 85.2 / 13.5.  With more weights it takes more from others: 1032 -> 256 -> 256 (322) one 38.1 / 6.8 and 40.8 / 6.5, 1000
-//  80.1 / 15.1 and 80.6 / 13.1; and with more than four blocks of outputs the waves are too few to share K: 896 -> 400 -> 128 (400) one 43.0 / 7.5
-//  and 41.0 / 6.3.
-bool bz::fc_rows_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2) {
-  return rows >= 1 && rows <= 1024 && n1 <= 256 && k * n1 + n1 * n2 <= 208 << 10;
-}
-
 int bz::fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
   BZ_REQUIRE(d.next != nullptr, "rows: no second layer");
   const bz_fc_next& x = *d.next;
