@@ -811,9 +811,9 @@ int main() {
   int wrong = 0;
   for (const auto& c : at) {
     const int last = c[3];
-    if ((last > 0 && !(bz::fc_rows_pays(1, c[0], c[1], c[2]) && bz::fc_rows_pays(last, c[0], c[1], c[2]))) || bz::fc_rows_pays(last + 1, c[0], c[1], c[2]))
-      wrong += printf("%d -> %d -> %d\n", c[0], c[1], c[2]);
-    if (bz::fc_rows_pays(0, c[0], c[1], c[2])) wrong += printf("no rows\n");
+    auto one = [&](int rows) { return bz::fc_rows_takes(c[0], c[1], c[2]) && bz::fc_rows_pays(rows, c[0], c[1], c[2]); };
+    if ((last > 0 && !(one(1) && one(last))) || one(last + 1)) wrong += printf("%d -> %d -> %d\n", c[0], c[1], c[2]);
+    if (one(0)) wrong += printf("no rows\n");
   }
   return wrong > 0;
 }
@@ -823,3 +823,39 @@ int main() {
                     "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+def test_few_row_towers_that_are_taken_are_run(tmp_path):
+    """What the kernel for few rows takes, a net lays out for it and asks about at every pass: nothing that it would run at no number of rows.
+    And the kernel's code is for what is taken: eight waves share K in at least two slices of at most four blocks of 64 columns."""
+    import shutil
+    import subprocess
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src = tmp_path / "takes.cc"
+    src.write_text(r"""
+#include <stdio.h>
+#include "bz_common.h"
+int main() {
+  int taken = 0;
+  for (int k : {0, 1, 48, 64, 192, 445, 468, 732, 733, 896, 1032, 1280, 1281})
+    for (int n1 : {8, 9, 64, 65, 128, 192, 200, 256, 257, 320, 400, 512, 513})
+      for (int n2 : {8, 9, 64, 80, 128, 256, 257}) {
+        if (!bz::fc_rows_takes(k, n1, n2)) continue;
+        ++taken;
+        if (!bz::fc_rows_pays(1, k, n1, n2) || !bz::fc_rows_pays(64, k, n1, n2) || (n1 + 63) / 64 > 4 || (n2 + 63) / 64 > 4) {
+          printf("%d -> %d -> %d\n", k, n1, n2);
+          return 1;
+        }
+      }
+  const int lines[][3] = {{1, 9, 9}, {1280, 130, 40}, {64, 256, 256}, {732, 256, 100}};
+  for (const auto& c : lines)
+    if (!bz::fc_rows_takes(c[0], c[1], c[2])) return 2;
+  return taken > 100 ? 0 : 3;
+}
+""")
+    exe = str(tmp_path / "takes")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout)

@@ -61,7 +61,6 @@ size_t fc_tower_weight_bytes(int64_t k, int64_t n);
 int fc_tower_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream);  // from [k, n], or [n, k] when transposed
 // fc_rows.hip, for the host layer: the same for few rows, fp32; d.w and d.next->w as fc_rows_pack laid them out
 int fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream);
-bool fc_rows_takes(int64_t k, int64_t n1, int64_t n2);
 size_t fc_rows_weight_bytes(int64_t k, int64_t n);
 int fc_rows_pack(const void* w, bool transposed, int k, int n, void* out, bz_stream_t stream);
 // fc_fused.hip, for the host layer: bz_fc_fused that stores the outputs of a head, or of a layer of at most eight columns,
@@ -92,7 +91,15 @@ inline bool head_behind_any_columns(int64_t rows, int64_t k, int64_t n, int elem
 // 16.1 / 12.5, 1024 of 512 -> 256 16.6 / 8.8, 2048 17.0 / 11.8, 4096 25.3 / 16.4, 8192 26.1 / 25.2, 2000 of 4096 -> 256 102 / 41.
 inline bool head_apart(int64_t k, int64_t n, int element_size) { return element_size == 4 && k * n > 48 << 10; }
 
-// Whether few rows of a fp32 tower k -> n1 -> n2 -> skinny are better off in one launch (fc_rows.hip: one row a workgroup up to 128 rows, two to
+// What fc_rows takes: no more columns than four blocks of 64, so that at least two waves share K (with one each, 896 -> 400 -> 128, us of one lone row /
+// a pass on eight serving threads, apart and in one launch 41.0 / 6.3 and 43.0 / 7.5), and weights that it does not lose with at any number of rows
+// (322 K, 1032 -> 256 -> 256, 40.8 / 6.5 and 38.1 / 6.8).
+constexpr int kRowsMaxIn = 1280, kRowsMaxColumns = 256;
+inline bool fc_rows_takes(int64_t k, int64_t n1, int64_t n2) {
+  return k >= 1 && k <= kRowsMaxIn && n1 > 8 && n1 <= kRowsMaxColumns && n2 > 8 && n2 <= kRowsMaxColumns && k * n1 + n1 * n2 <= 208 << 10;
+}
+
+// Whether few rows of a fp32 tower that it takes, k -> n1 -> n2 -> skinny, are better off in one launch (fc_rows.hip: one row a workgroup up to 128 rows, two to
 // 256, three to 384, then four) than in two or three.  Models that look rows up for the input, us of a lone request / a pass on eight serving
 // threads, apart and in one launch, by weights in units of 1024 and by rows:
 //    5 (48 -> 64 -> 32)    1: 31.2 / 5.0 and 30.8 / 5.0, 300: 34.6 / 6.0 and 34.4 / 6.0, 600: 35.3 / 6.1 and 35.1 / 6.1, 1024: 37.2 / 6.2 and 37.1 / 6.2:
@@ -106,12 +113,9 @@ inline bool head_apart(int64_t k, int64_t n, int element_size) { return element_
 //  208 (732 -> 256 -> 100) 1: 38.9 / 6.2 and 37.6 / 6.1, 300: 56.0 / 7.7 and 51.0 / 7.4, 640: 62.8 / 8.7 and 58.0 / 8.5, 700: 67.6 / 9.0 and 62.4 / 9.1,
 //      768: 69.1 / 9.5 and 65.3 / 9.7, 896: 73.6 / 9.9 and 68.4 / 10.6, 1024: 74.4 / 10.4 and 71.5 / 11.6
 // A lone request is no slower in one; what it takes from others grows with rows times weights, and the line is where serving has begun
-// to lose: 3 % at 142 x 1024, level at 173 x 832 and 208 x 700.  Beyond the rows and weights (with one row a workgroup at 201 rows, four at 1000 and 2000):
-// 53 x 2000 59.9 / 9.2 and 56.8 / 9.3, 61 x 2000 89.0 / 10.1 and 82.4 / 10.9; 322 (1032 -> 256 -> 256) 1: 40.8 / 6.5 and 38.1 / 6.8; with more than four
-// blocks of 64 columns the waves are too few to share K: 400 (896 -> 400 -> 128) 1: 41.0 / 6.3 and 43.0 / 7.5.
+// to lose: 3 % at 142 x 1024, level at 173 x 832 and 208 x 700.  Beyond 1024 rows (with four a workgroup): 53 x 2000 59.9 / 9.2 and 59.6 / 9.1, 61 x 2000 89.0 / 10.1 and 86.3 / 11.1, 142 x 2000 85.2 / 13.5 and 79.5 / 15.4.
 inline bool fc_rows_pays(int64_t rows, int64_t k, int64_t n1, int64_t n2) {
-  const int64_t weights = k * n1 + n1 * n2;
-  return rows >= 1 && rows <= 1024 && n1 <= 256 && weights <= 208 << 10 && rows * weights <= 144 << 20;
+  return rows >= 1 && rows <= 1024 && rows * (k * n1 + n1 * n2) <= 144 << 20;
 }
 
 }  // namespace bz

@@ -21,7 +21,7 @@ namespace {
 constexpr int kWaves = 8, kThreads = kWaves * 64, kRows = 4, kPerRow = kThreads / kRows;
 constexpr int kGroup = 4;  // chunks of 16 bytes (a lane's, of its output) asked for together
 constexpr int kRing = 4;   // such groups under way
-constexpr int kMaxIn = 1280, kMaxWide = 512, kMaxLast = 256;
+constexpr int kMaxIn = bz::kRowsMaxIn, kMaxWide = bz::kRowsMaxColumns, kMaxLast = bz::kRowsMaxColumns;
 constexpr int kBeyond = 1 << 30;  // an offset behind any operand
 
 __host__ __device__ constexpr int up(int v, int to) { return (v + to - 1) / to * to; }
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void bz_fc_rows_pack_kernel(const float* __res
 struct Layout {
   int pitch1, pitch2, x2, sums, params1, params2, head_w, all;
   Layout() = default;
-  Layout(int k, int n1, int n2, int hn) {
+  constexpr Layout(int k, int n1, int n2, int hn) : pitch1(), pitch2(), x2(), sums(), params1(), params2(), head_w(), all() {
     pitch1 = up((k + 3) / 4, kGroup) * 16 + 16;
     pitch2 = up((n1 + 3) / 4, kGroup) * 16 + 16;
     x2 = kRows * pitch1;
@@ -66,6 +66,9 @@ struct Layout {
     all = head_w + hn * kMaxLast * 4;
   }
 };
+
+static_assert(Layout(kMaxIn, kMaxWide, kMaxLast, kSkinnyMaxN).all <= 64 * 1024, "what a launch gets without asking for more");
+static_assert(kMaxWide <= kWaves / 2 * 64 && kMaxLast <= kWaves / 2 * 64, "eight, four or two slices of K");
 
 // what the kernel's first loads need comes first, as plain arguments (they are in registers when a wave starts); the rest
 struct Finish {
@@ -105,10 +108,8 @@ __device__ __forceinline__ float finished(const Epilogue& ep, const float* param
     sum = ((of[0] + of[next]) + (of[2 * next] + of[3 * next])) + ((of[4 * next] + of[5 * next]) + (of[6 * next] + of[7 * next]));
   else if (by.slices == 4)
     sum = (of[0] + of[next]) + (of[2 * next] + of[3 * next]);
-  else if (by.slices == 2)
-    sum = of[0] + of[next];
   else
-    sum = of[0];
+    sum = of[0] + of[next];
   return apply_act_regs(fmaf(ep.alpha, sum, p.x), ep, p.y, p.z, p.w);
 }
 
@@ -305,11 +306,6 @@ int bz::fc_rows_pack(const void* w, bool transposed, int k, int n, void* out, bz
                      transposed ? (int64_t)1 : (int64_t)n, transposed ? (int64_t)k : (int64_t)1, units);
   BZ_LAUNCH_OK("bz_fc_rows_pack_kernel");
   return BZ_OK;
-}
-
-bool bz::fc_rows_takes(int64_t k, int64_t n1, int64_t n2) {
-  return k >= 1 && k <= kMaxIn && n1 > kSkinnyMaxN && n1 <= kMaxWide && n2 > kSkinnyMaxN && n2 <= kMaxLast &&
-         Layout((int)k, (int)n1, (int)n2, kSkinnyMaxN).all <= 64 * 1024;
 }
 
 int bz::fc_rows(const bz_fc_desc& d, void* copy, bz_stream_t stream) {
