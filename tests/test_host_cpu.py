@@ -859,3 +859,113 @@ int main() {
                     "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout)
+
+
+def test_requests_staged_in_fewer_bytes_take_no_more_launches(tmp_path):
+    """The parts that a request is staged in, applied as the device would: every input arrives, nothing that a launch reads is written again or lies
+    outside the staging memory, and a request whose inputs are packed has no more launches than one that crosses as it is (26 lists of 100
+    samples made 78 ranges where a launch takes 64, and a second launch where there had been one).  Lists of the sizes on either side of
+    the lines, words that stop fitting anywhere, odd lengths and addresses."""
+    import shutil
+    import subprocess
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src = tmp_path / "stage.cc"
+    src.write_text(r"""
+#include <stdio.h>
+#include <stdlib.h>
+#include <memory>
+#include <random>
+#include "blaze/feed_pack.h"
+using blaze::FeedInput;
+struct Sent { const char* at; std::vector<char> was; };
+// launches of a request; below zero: what is wrong with it
+static int Send(const std::vector<FeedInput>& in, size_t plain) {
+  std::unique_ptr<char, void (*)(void*)> staging((char*)aligned_alloc(256, plain + 256), free), arena((char*)aligned_alloc(256, plain + 256), free);
+  memset(staging.get(), 0x5a, plain);
+  memset(arena.get(), 0x5a, plain);
+  std::vector<Sent> sent;
+  std::vector<bool> there(plain / 16);
+  int launches = 0, wrong = 0;
+  blaze::StageInputs(in, plain, staging.get(), arena.get(), [&](const bz_feed_piece* p, int n) {
+    ++launches;
+    if (n < 1 || n > BZ_FEED_MAX_PIECES) wrong = -1;
+    for (int i = 0; i < n; ++i) {
+      const char* src = (const char*)p[i].src;
+      char* dst = (char*)p[i].dst;
+      const size_t bytes = p[i].bytes, read = p[i].form == BZ_FEED_RAW ? bytes : p[i].form == BZ_FEED_LOW32 ? (bytes / 2 + 15) / 16 * 16 : 0;
+      if (bytes == 0 || bytes % 16 || (dst - arena.get()) % 16 || dst < arena.get() || dst + bytes > arena.get() + plain) { wrong = -2; return; }
+      if (read > 0 && ((src - staging.get()) % 16 || src < staging.get() || src + read > staging.get() + plain)) { wrong = -3; return; }
+      for (size_t k = 0; k < bytes / 16; ++k) {
+        if (there[(dst - arena.get()) / 16 + k]) wrong = -4;
+        there[(dst - arena.get()) / 16 + k] = true;
+      }
+      if (read > 0) sent.push_back({src, std::vector<char>(src, src + read)});
+      for (size_t k = 0; k < bytes; k += 4) {
+        const uint32_t low = p[i].form == BZ_FEED_LOW32 && k % 8 == 0 ? *(const uint32_t*)(src + k / 2) : 0;
+        if (p[i].form == BZ_FEED_RAW) memcpy(dst + k, src + k, 4);
+        if (p[i].form == BZ_FEED_LOW32) memcpy(dst + k, &low, 4);
+        if (p[i].form == BZ_FEED_SAME32) memcpy(dst + k, &p[i].word, 4);
+      }
+    }
+  });
+  for (const Sent& s : sent)
+    if (memcmp(s.at, s.was.data(), s.was.size()) != 0) wrong = -5;
+  for (const FeedInput& f : in)
+    if (f.len > 0 && memcmp(arena.get() + f.offset, f.data, f.len) != 0) wrong = -6;
+  return wrong != 0 ? wrong : launches;
+}
+int main() {
+  std::mt19937_64 rng(7);
+  auto request = [&](const std::vector<std::pair<size_t, size_t>>& inputs, int odd) {  // (words, bytes of one); odd: of how many inputs one has words that do not fit
+    std::vector<std::vector<char>> keep;
+    std::vector<FeedInput> in, raw;
+    size_t plain = 0;
+    for (const auto& i : inputs) {
+      const size_t len = i.first * i.second, skew = rng() % 2;
+      keep.emplace_back(len + skew);
+      char* at = keep.back().data() + skew;
+      const uint32_t same = (uint32_t)rng();
+      for (size_t k = 0; k < i.first; ++k) {
+        const uint64_t v = i.second == 8 ? rng() & 0xffffffffu : i.second == 4 ? same : rng();
+        memcpy(at + k * i.second, &v, i.second);
+      }
+      if (odd > 0 && rng() % odd == 0 && i.first > 0)
+        for (int k = 0; k < 3; ++k) {
+          const size_t w = k == 0 && rng() % 2 ? i.first - 1 : rng() % i.first;
+          memset(at + w * i.second, 0xff, i.second);
+        }
+      in.push_back({at, len, plain, i.second});
+      raw.push_back({at, len, plain, 1});
+      plain += (len + 255) / 256 * 256;
+    }
+    const int one = Send(in, plain), other = Send(raw, plain);
+    if (one >= 0 && one <= other) return 0;
+    printf("%zu inputs, the first of %zu words, %zu bytes: %d for %d launches\n", inputs.size(), inputs[0].first, plain, one, other);
+    return 1;
+  };
+  int bad = 0;
+  for (size_t slots : {3, 18, 26, 32, 40, 64})
+    for (size_t batch : {32, 64, 80, 100, 128, 160, 200, 256, 400}) {
+      std::vector<std::pair<size_t, size_t>> in;
+      for (size_t s = 0; s < slots; ++s) {
+        in.push_back({8 * batch + s, 8});
+        in.push_back({8 * batch + s, 4});
+        in.push_back({batch, 4});
+      }
+      bad += request(in, 0) + request(in, 4);
+    }
+  for (int k = 0; k < 300; ++k) {
+    std::vector<std::pair<size_t, size_t>> in;
+    const size_t n = 1 + rng() % 90, most = (size_t)1 << (1 + rng() % (k % 10 == 0 ? 17 : 12));
+    for (size_t i = 0; i < n; ++i) in.push_back({rng() % 8 == 0 ? 0 : rng() % most + (rng() % 3 == 0 ? 256 - most % 256 : 0), (size_t)1 << rng() % 4});
+    bad += request(in, 1 + rng() % 6);
+  }
+  return bad > 0;
+}
+""")
+    exe = str(tmp_path / "stage")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=undefined", "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "x-deeplearning_amd", "csrc"), str(src), "-o", exe], check=True, capture_output=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-3000:])

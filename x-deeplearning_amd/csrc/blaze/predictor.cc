@@ -180,21 +180,6 @@ bool Predictor::Feed(size_t idx, const void* data, size_t len) {
   return true;
 }
 
-// A request is moved in parts, each launched as soon as it is staged.  Up to 4 MB the link is what bounds it (the kernel moves
-// 47 GB/s and leaves a gap behind each launch, staging runs at 58), so it starts early: 384 KB first, each part half as large
-// again as the one before until 1 MB.  Beyond, staging is (35 GB/s, the copies no longer fit the caches between requests), and a
-// launch costs the host 2.9 us: even parts of 1 MB or more.  The last part takes what would be left of it below half a part.  us to the end of a
-// request among others, even parts of 1 MB or more / these: 0.74 MB 79.3 / 78.5, 1.07 92.8 / 88.5, 1.8 125 / 112, 2.5 115 / 112,
-// 3 135 / 127, 4 162 / 158, 4.6 180..191 / 184..194 (not taken), 5.1 203 / 217 (not taken).  (The copy engine moves 57 GB/s, but each copy costs 10 us until
-// what follows it on the stream may start: 5 MB in ten parts arrived 230 us after the first byte was staged, in one part behind
-// the whole staging 210, through five launches of the kernel 162.)
-constexpr size_t kFeedFirst = 384 << 10, kFeedMost = 1 << 20, kFeedLong = 4 << 20;
-// Inputs of this many bytes are staged in the form that crosses in fewest (feed_pack.h), if one fits; smaller ones would make
-// more ranges than they save.  us a request, as they are / packed: 5.1 MB of ids below 2^32 and values of 1 199 / 134..160, with keys of 62
-// bits for ids 205 / 182, 10 MB 450 / 360, 1.07 MB 86.6 / 72, 0.7 MB 64.5 / 51 (keys: 72 / 65); of any values and keys, where nothing fits,
-// 220 / 215.
-constexpr size_t kPackFrom = 2 << 10;
-
 // a transfer has been queued on the context's stream
 void Predictor::FeedQueued(const HIPContext& ctx) {
   feed_on_ = ctx.stream_serial();
@@ -305,65 +290,21 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
     // from the first launch on the arena is being read: whatever happens next, it is waited for before it is written again
     try {
       bz_feed_rows rows[BZ_FEED_MAX_ROWS];
-      bz_feed_piece pieces[BZ_FEED_MAX_PIECES];
-      int n = 0, n_pieces = 0;
-      size_t moved = 0, staged = 0;  // bytes of the device arena whose transfer has been launched; of the staging arena in use
-      size_t part = plain < kFeedLong ? kFeedFirst : (plain / (plain / kFeedMost) / 256 + 1) * 256;
-      auto launch = [&](size_t upto) {
+      int n = 0;
+      auto launch = [&](const bz_feed_piece* pieces, int n_pieces) {
         BZ_CHECK(bz_feed_pieces(pieces, n_pieces, rows, n, st));
-        moved = upto;
-        n = n_pieces = 0;
+        n = 0;
       };
-      auto end_of_part = [&]() { return plain - moved < part + part / 2 ? plain : moved + part; };
-      size_t end = end_of_part();
       for (const Item& it : strided) {
-        if (n == BZ_FEED_MAX_ROWS) launch(moved);
+        if (n == BZ_FEED_MAX_ROWS) launch(nullptr, 0);
         memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
         rows[n++] = StridedRows(external_input_blob_[it.idx], arena_host_ + it.offset);
       }
-      // `bytes` of the device arena from `at` on, of which `source` bytes have been staged
-      auto add = [&](size_t at, size_t bytes, int form, uint32_t word, size_t source) {
-        char *from = arena_host_ + staged, *to = arena_dev_ + at;
-        staged += source;
-        bz_feed_piece* last = n_pieces > 0 ? &pieces[n_pieces - 1] : nullptr;
-        if (last && form == BZ_FEED_RAW && last->form == BZ_FEED_RAW && (const char*)last->src + last->bytes == from && (char*)last->dst + last->bytes == to) {
-          last->bytes += bytes;
-          return;
-        }
-        if (n_pieces == BZ_FEED_MAX_PIECES) launch(at);
-        pieces[n_pieces++] = {from, to, (int64_t)bytes, form, word};
-      };
-      auto up = [](size_t bytes, size_t to) { return (bytes + to - 1) / to * to; };
-      for (const Item& it : in_arena) {
-        const size_t len = lens[it.arg];
-        const size_t word = len >= kPackFrom ? DataTypeSize(external_input_blob_[it.idx]->data_type()) : 0;
-        bool packs = word == 8 || word == 4;
-        uint32_t first = 0;
-        if (packs) memcpy(&first, data[it.arg], 4);
-        for (size_t at = 0; at < len;) {
-          // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte; and staged <= it.offset + at)
-          const char* from = (const char*)data[it.arg] + at;
-          const size_t left = std::min(len - at, end - (it.offset + at));
-          size_t now = 0;
-          if (packs) {
-            now = word * (word == 8 ? PackLow32((uint32_t*)(arena_host_ + staged), (const uint64_t*)from, left / 8) : CountSame32(from, left / 4, first));
-            packs = now == left;
-            if (now > 0) add(it.offset + at, up(now, 16), word == 8 ? BZ_FEED_LOW32 : BZ_FEED_SAME32, first, word == 8 ? up(now / 2, 256) : 0);
-          }
-          if (now == 0) {
-            now = left;
-            memcpy(arena_host_ + staged, from, now);
-            add(it.offset + at, up(now, 256), BZ_FEED_RAW, 0, up(now, 256));
-          }
-          at += now;
-          if (it.offset + at == end) {
-            launch(end);
-            if (plain < kFeedLong) part = std::min(part + part / 2, kFeedMost);
-            end = end_of_part();
-          }
-        }
-      }
-      if (n_pieces > 0 || n > 0) launch(plain);
+      std::vector<FeedInput> inputs;
+      inputs.reserve(in_arena.size());
+      for (const Item& it : in_arena) inputs.push_back({data[it.arg], lens[it.arg], it.offset, DataTypeSize(external_input_blob_[it.idx]->data_type())});
+      StageInputs(inputs, plain, arena_host_, arena_dev_, launch);
+      if (n > 0) launch(nullptr, 0);
       FeedQueued(ctx);
     } catch (...) {
       (void)hipStreamSynchronize(st);  // no event stands behind what was launched
