@@ -315,10 +315,11 @@ def test_embedding_planner_geometry_and_scan_advice():
     assert launch.variant == 0 and [s.wg_count for s in slots] == [1024 * 13 // 128] * 3
 
 
-def test_no_pooling_workgroup_begins_behind_its_slots_samples(tmp_path):
-    """A workgroup finds its offsets by adding up the counts in front of its first sample, so one that began behind the last sample would
-    read counts beyond the caller's array, which its dropped sums would not show: of a plan's workgroups, whole and halved, those that
-    go on have each sample once and begin in front of the last one's end, at batches around every multiple of either size."""
+def test_no_pooling_workgroup_reads_counts_behind_its_slots_samples(tmp_path):
+    """A workgroup finds its offsets by adding up the counts in front of its first sample, so one that begins behind the last sample would
+    read counts beyond the caller's array, which its dropped sums would not show: of a plan's workgroups, whole and halved, each sample
+    has one, which adds up all counts in front of it, and none adds up more counts than there are, at batches around every multiple of
+    either size."""
     import shutil
     import subprocess
     import blaze_hip
@@ -365,13 +366,13 @@ int main() {
             const int v = block % bz::kNumXcd * grid.wg_per_xcd + block / bz::kNumXcd;
             if (v >= grid.total_wg) continue;
             const int slot = v / grid.wg_per_slot, wg = v - slot * grid.wg_per_slot;
-            const int64_t first = bz::first_sample(wg, groups, slots[slot].batch);
-            idle += first < 0;
-            if (first >= batch) {
-              printf("batch %d, %d lanes, %d samples a workgroup: one reads counts 0 to %d\n", batch, lanes, groups, (int)first);
+            const int64_t first = (int64_t)wg * groups, counts = bz::counts_before(first, slots[slot].batch);
+            idle += first >= batch;
+            if (counts > batch || (first < batch && counts != first)) {
+              printf("batch %d, %d lanes, %d samples a workgroup: the one from %d on reads counts 0 to %d\n", batch, lanes, groups, (int)first, (int)counts - 1);
               return 2;
             }
-            for (int g = 0; first >= 0 && g < groups && first + g < batch; ++g) ++seen[(size_t)slot * batch + first + g];
+            for (int g = 0; g < groups && first + g < batch; ++g) ++seen[(size_t)slot * batch + first + g];
           }
           for (int n : seen)
             if (n != 1) return 3;
@@ -386,11 +387,14 @@ int main() {
                     str(src), "-L" + lib, "-lblaze_hip", "-Wl,-rpath," + lib, "-o", exe], check=True, capture_output=True, timeout=300)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout)
-    # and every workgroup of the kernel asks, before anything is read
-    kernels = re.findall(r"__global__[^;{]*bz_embed_pool(?:_args)?_kernel\(.*?\n}\n", open(os.path.join(ROOT, "x-deeplearning_amd", "csrc", "embed_pool.hip")).read(), flags=re.S)
-    assert len(kernels) == 2
-    for text in kernels:
-        assert re.search(r"const int64_t b0 = bz::first_sample\(v - si \* wg_per_slot, GROUPS, s\.batch\);\s*if \(b0 < 0\) return;\s*pool_samples<", text), text
+    # and what the kernels add up ends there: the scan within registers, and the one for 2^31 ids and more
+    csrc = os.path.join(ROOT, "x-deeplearning_amd", "csrc")
+    own = open(os.path.join(csrc, "embed_pool.hip")).read()
+    own = own[own.index("__device__ __forceinline__ void own_segment("):own.index("__device__ __forceinline__ void pool_samples(")]
+    assert "const uint32_t quads = (uint32_t)bz::counts_before(b0, s.batch) / 4;" in own and "b0 / 4" not in own and own.count("s.segments") == 2
+    wide = open(os.path.join(csrc, "embed_common.h")).read()
+    wide = wide[wide.index("__device__ __forceinline__ void stage_offsets("):wide.index("typedef int i32x4a4")]
+    assert "const int64_t ahead = bz::counts_before(b0, s.batch);" in wide and "i < b0" not in wide and "i0 < b0" not in wide and wide.count("s.segments[") == 2
 
 
 def test_baseline_forward_with_library_sgemm_agrees_with_the_pinned_sums(oracle):

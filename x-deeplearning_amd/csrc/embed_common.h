@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "bz_common.h"
+#include "embed_groups.h"
 
 namespace {
 
@@ -284,12 +285,13 @@ __device__ __forceinline__ void stage_offsets(const bz_embed_slot& s, const int6
   // (a negative count is taken as 0 and the offsets below stop at nnz: see bz_embed_slot.nnz)
   const int64_t mine = (tid < groups && b0 + tid < s.batch) ? (int64_t)max(s.segments[b0 + tid], 0) : 0;
   int64_t part = 0;
-  for (int64_t i0 = 0; i0 < b0; i0 += 8 * THREADS) {
+  const int64_t ahead = bz::counts_before(b0, s.batch);
+  for (int64_t i0 = 0; i0 < ahead; i0 += 8 * THREADS) {
     int32_t c[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int64_t i = i0 + k * THREADS + tid;
-      c[k] = i < b0 ? max(s.segments[i], 0) : 0;
+      c[k] = i < ahead ? max(s.segments[i], 0) : 0;
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) part += c[k];

@@ -1,8 +1,7 @@
 // embed_groups.h -- which samples a workgroup of the specialised pooling kernel has.
 //
 // A plan counts workgroups of one size, just as many a slot as have samples.  A launch whose workgroups are a part of those has that
-// many times as many, the last of which may begin behind the slot's last sample: with nothing to add up, and no counts of
-// their own that may be read, let alone all those in front of their first sample.
+// many times as many, the last of which may begin behind the slot's last sample: the counts in front of theirs are not all there to be read.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,10 +18,8 @@ struct PoolGrid {
       : total_wg(split * planned), wg_per_slot(split * planned_per_slot), wg_per_xcd((total_wg + kNumXcd - 1) / kNumXcd), blocks(wg_per_xcd * kNumXcd) {}
 };
 
-// first sample of a slot's workgroup `wg`, each of which has `groups`; below zero: it has none
-__host__ __device__ inline int64_t first_sample(int wg, int groups, int32_t batch) {
-  const int64_t first = (int64_t)wg * groups;
-  return first < batch ? first : -1;
-}
+// How many of a slot's counts a workgroup whose first sample is `first` adds up for its offsets.  (It goes on where it has no sample, too: told to
+// return, it asked for its record's `batch` alone and for the rest a trip to memory later, keyed 1000 x 24 lists of rows of 100 14.1 -> 14.4 us.)
+__host__ __device__ inline int64_t counts_before(int64_t first, int32_t batch) { return first < batch ? first : 0; }
 
 }  // namespace bz

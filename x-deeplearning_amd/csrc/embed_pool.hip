@@ -41,7 +41,6 @@
 #include <mutex>
 
 #include "embed_common.h"
-#include "embed_groups.h"
 
 namespace {
 
@@ -222,7 +221,7 @@ __device__ __forceinline__ void own_segment(const bz_embed_slot& s, int64_t b0, 
   const int32_t own = b < s.batch ? s.segments[b] : 0;
   // (b0 is below 2^31: batch is an int32.  A workgroup near the head of its slot has few counts before it: the rounds
   // stop, for the whole workgroup, where b0 ends)
-  const uint32_t quads = (uint32_t)b0 / 4;
+  const uint32_t quads = (uint32_t)bz::counts_before(b0, s.batch) / 4;
   const i32x4a4* before_b0 = (const i32x4a4*)s.segments;
   uint32_t part = 0;
   for (uint32_t i0 = 0; i0 < quads; i0 += 4 * THREADS) {
@@ -303,8 +302,7 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_kernel(const bz_embed_s
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = slots[si];
-  const int64_t b0 = bz::first_sample(v - si * wg_per_slot, GROUPS, s.batch);
-  if (b0 < 0) return;
+  const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
   pool_samples<DT, LPR, THREADS, KEYED>(s, b0, ext_off != nullptr ? ext_off + (int64_t)si * ext_stride : s.offsets);
 }
 
@@ -316,8 +314,7 @@ __global__ __launch_bounds__(THREADS) void bz_embed_pool_args_kernel(int total_w
   if (v >= total_wg) return;
   const int si = v / wg_per_slot;
   const bz_embed_slot s = pack.s[si];
-  const int64_t b0 = bz::first_sample(v - si * wg_per_slot, GROUPS, s.batch);
-  if (b0 < 0) return;
+  const int64_t b0 = (int64_t)(v - si * wg_per_slot) * GROUPS;
   pool_samples<DT, LPR, THREADS, KEYED>(s, b0, s.offsets);
 }
 
