@@ -1415,7 +1415,7 @@ def test_feed_many_at_the_borders_of_its_parts(pb, sizes):
             np.testing.assert_allclose(p.output_asnumpy("y%d" % k).reshape(-1), _sigmoid(x).reshape(-1), rtol=1e-5)
 
 
-# 64-bit ids cross as their lower halves and equal 32-bit words as one, in blocks of 1024 words: the word that does not fit stands at
+# 64-bit ids cross as their lower halves and equal 32-bit words as one, in blocks of 256 words: the word that does not fit stands at
 # the edges of blocks and parts, at the end, or nowhere
 @pytest.mark.parametrize("n,odd", [(1, []), (255, []), (256, []), (1023, [1022]), (1024, []), (1025, [1024]), (5000, [7]), (5000, [8]), (5000, [1023]),
                                    (5000, [1024]), (5000, [4999]), (5000, [2048, 3000]), (49152, [49151]), (49153, [49152]), (200001, [131072]), (700000, [])])
@@ -1443,6 +1443,48 @@ def test_feed_many_of_words_that_are_packed(pb, n, odd):
             ids[k] = -1 - k if turn else ids[k] + (1 << 32)
             values[k], counts[k] = 0.0 if turn else 1.0, -255
         feed = {"ids": ids, "before": rng.standard_normal(67).astype(np.float32), "values": values, "counts": counts, "more": more, "x": values[:3].copy()}
+        for name, a in feed.items():
+            p.reshape_input(name, a.shape)
+        p.feed_many(p.feed_batch(list(feed.items())))
+        p.forward()
+        for name in kinds:
+            there = dict(shape=feed[name].shape, typestr=feed[name].dtype.str, data=(p.input_device_ptr(name), False), version=3, strides=None)
+            got = torch.as_tensor(type("View", (), dict(__cuda_array_interface__=there))(), device="cuda").cpu().numpy()
+            assert got.tobytes() == feed[name].tobytes(), (turn, name)
+
+
+# the line from which a request is packed, and the edges of the first blocks
+@pytest.mark.parametrize("n,odd", [(4095, []), (4096, []), (4097, [255]), (5000, [255]), (5000, [256]), (5000, [511]), (5000, [513])])
+def test_feed_many_packed_or_not(pb, n, odd):
+    test_feed_many_of_words_that_are_packed(pb, n, odd)
+
+
+@pytest.mark.parametrize("lists", [21, 22, 30])  # 63 and 66 ranges, where a launch takes 64, and 90
+def test_feed_many_of_more_ranges_than_a_launch_takes(pb, lists):
+    """lists of ids and equal values with short counts between them, every third value differing somewhere: each input arrives as it is"""
+    import torch
+    rng = np.random.default_rng(lists)
+    nb = pb.NetBuilder("ranges", device_type=1)
+    nb.constant("flat", np.array([-1], np.int32))
+    kinds = {}
+    for i in range(lists):
+        kinds.update({"ids%d" % i: pb.K_INT64, "values%d" % i: pb.K_FLOAT, "counts%d" % i: pb.K_INT32})
+    for name, code in kinds.items():
+        nb.external_input(name, code)
+        nb.op("Reshape", [name, "flat"], ["flat_" + name])
+        nb.external_output("flat_" + name, code)
+    pm = pb.PredictorManager()
+    pm.load_model_from_string(nb.text(), True)
+    p = pm.create_predictor(1, 0)
+    for turn in range(2):
+        feed = {}
+        for i in range(lists):
+            n = 1600 + 37 * i  # 12.8 and 6.4 KB on: 22 lists are one part
+            feed["ids%d" % i] = rng.integers(0, 1 << 32, n, dtype=np.int64)
+            feed["values%d" % i] = np.full(n, 1 + i, np.float32)
+            feed["counts%d" % i] = rng.integers(0, 20, 201).astype(np.int32)
+            if turn and i % 3 == 0:
+                feed["values%d" % i][rng.integers(n)] = -1
         for name, a in feed.items():
             p.reshape_input(name, a.shape)
         p.feed_many(p.feed_batch(list(feed.items())))

@@ -9,8 +9,8 @@
 // (36..256 bytes) plus 12 bytes of id/value.  A row is cut into 16-byte chunks
 // (one 128-bit load); a *lane group* of `lpr` = pow2(chunks per row) lanes owns one
 // (sample, slot) segment and walks its ids in order, so every output element is
-// summed in exactly the reference's order (bit-identical fp32).  A 512-thread
-// workgroup holds 512/lpr segments of consecutive samples of one slot.  One launch
+// summed in exactly the reference's order (bit-identical fp32).  A workgroup of 512
+// or 256 threads (small_groups) holds 512/lpr or 256/lpr segments of consecutive samples of one slot.  One launch
 // covers every slot of the operator; the linear workgroup id is remapped so that
 // each of the 8 XCDs (each with its own L2) serves a contiguous range of slots and
 // therefore caches the hot rows of only those tables.
@@ -18,7 +18,7 @@
 // The kernel is latency bound before it is bandwidth bound (a batch-2048 launch moves
 // ~36 MB), so the dependent chain is kept at: slot record -> segments -> ids -> rows.
 //   * segments -> offsets is fused: a workgroup sums the counts before its first
-//     sample and scans its own 512/lpr counts in LDS (no separate scan launch, no
+//     sample and scans its own in registers (no separate scan launch, no
 //     offsets round trip);
 //   * with equal work per slot the slot index is a division, not a search;
 //   * the specialised ksum/kavg kernel walks a segment kBlockIds ids at a time: the lanes
