@@ -111,17 +111,46 @@ struct FeedInput {
   size_t len;
   size_t offset;  // its slice of the arena: they lie side by side, multiples of 256 bytes each
   size_t word;    // bytes of an element
+  // what the link may be spared of it
+  size_t Spares() const { return word == 8 && len >= kPackWide ? len / 2 : word == 4 && len >= kPackFrom ? len : 0; }
 };
 
-// Stages the inputs, whose slices are `plain` bytes, from `staging` on, which has as many, and has launch(pieces, how many) move them to `arena`.
-template <typename Launch>
-void StageInputs(const std::vector<FeedInput>& inputs, size_t plain, char* staging, char* arena, const Launch& launch) {
+// Stages the inputs, which are FeedInputs and whose slices are `plain` bytes, from `staging` on, which has as many, and has
+// launch(pieces, how many) move them to `arena`.
+template <typename Input, typename Launch>
+void StageInputs(const std::vector<Input>& inputs, size_t plain, char* staging, char* arena, const Launch& launch) {
   bz_feed_piece pieces[BZ_FEED_MAX_PIECES];
   int n = 0;
   size_t moved = 0, staged = 0;  // bytes of the arena whose transfer has been launched; of the staging memory in use
   size_t part = plain < kFeedLong ? kFeedFirst : (plain / (plain / kFeedMost) / 256 + 1) * 256;
   auto end_of_part = [&]() { return plain - moved < part + part / 2 ? plain : moved + part; };
   size_t end = end_of_part();
+  auto next_part = [&]() {
+    moved = end;
+    if (plain < kFeedLong) part = std::min(part + part / 2, kFeedMost);
+    end = end_of_part();
+  };
+  size_t least = 0;
+  for (const Input& in : inputs) least += in.Spares();
+  // As it is, a request of few bytes above all, whose many inputs are no more than a copy each here (one sample of 18 lists: 5.95 us
+  // in the call with the loop below, 5.5 with this one).
+  if (least < kPackLeast) {
+    auto launch_part = [&]() {
+      pieces[0] = {staging + moved, arena + moved, (int64_t)(end - moved), BZ_FEED_RAW, 0};
+      launch(pieces, 1);
+      next_part();
+    };
+    for (const Input& in : inputs)
+      for (size_t at = 0; at < in.len;) {
+        // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte)
+        const size_t now = std::min(in.len - at, end - (in.offset + at));
+        memcpy(staging + in.offset + at, (const char*)in.data + at, now);
+        at += now;
+        if (in.offset + at == end) launch_part();
+      }
+    if (plain > moved) launch_part();
+    return;
+  }
   auto up = [](size_t bytes, size_t to) { return (bytes + to - 1) / to * to; };
   // `bytes` of the arena from `at` on, of which `source` bytes have been staged
   auto add = [&](size_t at, size_t bytes, int form, uint32_t word, size_t source) {
@@ -133,16 +162,12 @@ void StageInputs(const std::vector<FeedInput>& inputs, size_t plain, char* stagi
     else
       pieces[n++] = {from, to, (int64_t)bytes, form, word};
   };
-  // what the link may be spared of an input
-  auto spares = [](const FeedInput& in) { return in.word == 8 && in.len >= kPackWide ? in.len / 2 : in.word == 4 && in.len >= kPackFrom ? in.len : 0; };
-  size_t least = 0;
-  for (const FeedInput& in : inputs) least += spares(in);
-  for (const FeedInput& in : inputs) {
-    bool packs = least >= kPackLeast && spares(in) > 0;
+  for (const Input& in : inputs) {
+    bool packs = in.Spares() > 0;
     uint32_t first = 0;
     if (packs) memcpy(&first, in.data, 4);
     for (size_t at = 0; at < in.len;) {
-      // (a part ends on a multiple of 256 bytes, as every slice begins: never before this byte; and staged <= in.offset + at)
+      // (staged <= in.offset + at)
       const char* from = (const char*)in.data + at;
       const size_t left = std::min(in.len - at, end - (in.offset + at));
       size_t now = 0;
@@ -161,9 +186,7 @@ void StageInputs(const std::vector<FeedInput>& inputs, size_t plain, char* stagi
       if (in.offset + at == end) {
         launch(pieces, n);
         n = 0;
-        moved = end;
-        if (plain < kFeedLong) part = std::min(part + part / 2, kFeedMost);
-        end = end_of_part();
+        next_part();
       }
     }
   }

@@ -227,13 +227,18 @@ void Predictor::OrderBehindFeeds() {
 bool Predictor::FeedMany(int count, const char* const* names, const void* const* data, const size_t* lens) {
   output_ahead_.assign(output_ahead_.size(), false);
   try {
-    struct Item {
+    struct Item : FeedInput {
+      int idx;
+    };
+    struct Strided {
       int idx;
       int arg;
       size_t offset;
     };
     // plain inputs first, in one range that lands as it is staged; inputs that live inside a Concat's output behind them
-    std::vector<Item> in_arena, strided;
+    std::vector<Item> in_arena;
+    in_arena.reserve(std::max(count, 0));
+    std::vector<Strided> strided;
     size_t total = 0;
     const DeviceOption* dev = nullptr;
     for (int i = 0; i < count; ++i) {
@@ -243,7 +248,7 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
         return false;
       }
       Blob* blob = external_input_blob_[idx];
-      const size_t need = blob->size() * DataTypeSize(blob->data_type());
+      const size_t word = DataTypeSize(blob->data_type()), need = blob->size() * word;
       if (lens[i] != need) {
         LOG_ERROR("The len=%zu need size=%zu blob->size()=%zu", lens[i], need, (size_t)blob->size());
         return false;
@@ -254,19 +259,19 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       }
       dev = &blob->device_option();
       if (blob->pitch() != 0) {
-        auto same = std::find_if(strided.begin(), strided.end(), [&](const Item& it) { return it.idx == idx; });
+        auto same = std::find_if(strided.begin(), strided.end(), [&](const Strided& it) { return it.idx == idx; });
         if (same != strided.end())
           same->arg = i;  // named twice: the last one counts, and two pieces of one launch must not share a target
         else
           strided.push_back({idx, i, 0});
         continue;
       }
-      in_arena.push_back({idx, i, total});
+      in_arena.push_back({{data[i], need, total, word}, idx});
       total += (need + 255) / 256 * 256;  // every slice 256-byte aligned
     }
     if (dev == nullptr) return true;
     const size_t plain = total;
-    for (Item& it : strided) {
+    for (Strided& it : strided) {
       it.offset = total;
       total += (lens[it.arg] + 255) / 256 * 256;
     }
@@ -295,15 +300,12 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
         BZ_CHECK(bz_feed_pieces(pieces, n_pieces, rows, n, st));
         n = 0;
       };
-      for (const Item& it : strided) {
+      for (const Strided& it : strided) {
         if (n == BZ_FEED_MAX_ROWS) launch(nullptr, 0);
         memcpy(arena_host_ + it.offset, data[it.arg], lens[it.arg]);
         rows[n++] = StridedRows(external_input_blob_[it.idx], arena_host_ + it.offset);
       }
-      std::vector<FeedInput> inputs;
-      inputs.reserve(in_arena.size());
-      for (const Item& it : in_arena) inputs.push_back({data[it.arg], lens[it.arg], it.offset, DataTypeSize(external_input_blob_[it.idx]->data_type())});
-      StageInputs(inputs, plain, arena_host_, arena_dev_, launch);
+      StageInputs(in_arena, plain, arena_host_, arena_dev_, launch);
       if (n > 0) launch(nullptr, 0);
       FeedQueued(ctx);
     } catch (...) {
@@ -311,7 +313,7 @@ bool Predictor::FeedMany(int count, const char* const* names, const void* const*
       any_feed_pending_ = false;
       throw;
     }
-    for (const Item& it : strided) feed_pending_[it.idx] = true;
+    for (const Strided& it : strided) feed_pending_[it.idx] = true;
     for (const Item& it : in_arena) {
       Blob* blob = external_input_blob_[it.idx];
       // (also when the slice did not move: this records the slice's new size and clears "unplaced")
