@@ -20,7 +20,7 @@
 //
 // Skinny kernel (N <= 8: the 256->2 softmax head, the 40->1 attention score, the 256->1
 // sigmoid head): bandwidth bound on A; a lane group of pow2(K/8) lanes owns a row, the
-// weight fragments live in registers, the N dot products are reduced by shuffles.
+// weight fragments live in registers, the N dot products are added up over it by lane swaps and DPP operands.
 //
 // Compiled once per operand type (fc_fused_f16.hip, fc_fused_bf16.hip, fc_fused_f32.hip include this file and define
 // that type's entry, bz::fc_run_*): three translation units that build side by side instead of one that takes three
